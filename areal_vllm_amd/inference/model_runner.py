@@ -423,6 +423,7 @@ class ModelRunner:
         )
         st["nsplit"] = nsplit
         st["ws"] = ws
+        st["items"] = self._decode_items(Bp)
         if self.keep_logits:
             st["logits"] = torch.zeros(Bp, self.V, dtype=torch.float32, device=dev)
         # Pinned host memory, two sets used alternately: uploads of plan n+1 are written while the copies of
@@ -440,9 +441,16 @@ class ModelRunner:
         return st
 
     def _decode_workspace(self, Bp: int):
-        """(key-range splits, split workspace) of the decode attention at this batch bucket."""
-        nsplit = ops.decode_num_splits(Bp, self.hkv, 4096, fp8=ops.attention.is_fp8(self.kv[0][0]))
-        return nsplit, (ops.DecodeWorkspace(Bp, self.hq, self.cfg.head_dim, nsplit, self.device) if nsplit > 1 else None)
+        """(key-range splits, split workspace) of the decode attention at this batch bucket, for attention that does
+        not run on work items."""
+        return 1, None
+
+    def _decode_items(self, Bp: int) -> Optional["ops.DecodeItems"]:
+        """Work items of the decode attention, laid out anew in every step and shared by its layers."""
+        if self.device.type != "cuda":
+            return None
+        return ops.DecodeItems(Bp, self.hq, self.hkv, self.cfg.head_dim, self.device,
+                               max_context=self.max_pages * PAGE_SIZE)
 
     FUSED_MIN_BATCH = 1  # the hand-written layer wins at every batch size (1.8 against 3.5 ms per step at one row)
 
@@ -556,8 +564,7 @@ class ModelRunner:
                                                self.rope, kc, vc, hq, hkv, D, dtype=self.dtype,
                                                q_norm=blk.attn.q_norm if cfg.qk_norm else None,
                                                k_norm=blk.attn.k_norm if cfg.qk_norm else None, norm_eps=eps)
-            attn = ops.paged_attention_decode(q, kc, vc, st["block_tables"], st["context_lens"], nsplit=st["nsplit"],
-                                              workspace=st["ws"])
+            attn = ops.paged_attention_decode(q, kc, vc, st["block_tables"], st["context_lens"], items=st["items"])
             slab = dg.dgemm(attn.view(Bp, hq * D), blk.attn.o, epilogue=dg.EPI_SLAB)
             x, residual = finish(slab, residual, blk.ln2)
             nw = layers[li + 1].ln1 if li + 1 < len(layers) else self.model.norm
@@ -607,6 +614,8 @@ class ModelRunner:
         ops.decode_begin_(st["kill"], st["active"], st["positions"], st["context_lens"], st["slots"],
                           st["block_tables"])
         for s in range(self.decode_steps):
+            if st["items"] is not None:
+                st["items"].fill_(st["context_lens"])
             h = self._embed(st["input_ids"], st["positions"])
             rope_pos = st["positions"] if self.cfg.pos_embed == "rope" else st["zero_pos"]
             if self.is_vl:  # generated tokens of a request with images sit `delta` away from their index
@@ -639,8 +648,7 @@ class ModelRunner:
                 qkv = qkv2d.view(Bp, hq + 2 * hkv, D)
                 ops.rope_and_cache_write_(qkv, rope_pos, st["slots"], self.rope, kc, vc, hq, hkv)
                 return ops.paged_attention_decode(qkv[:, :hq], kc, vc, st["block_tables"], st["context_lens"],
-                                                  nsplit=st["nsplit"], workspace=st["ws"],
-                                                  q_row_stride=qkv_stride)
+                                                  q_row_stride=qkv_stride, items=st["items"])
 
             h, residual = self._layer(blk, h, residual, st["positions"], st["slots"], attn_fn)
         return self._final_logits(h, residual)
@@ -689,7 +697,7 @@ class ModelRunner:
         self.step_counter.copy_(step_saved)
         self.graphs[key] = g
         logger.info(f"captured decode graph: batch bucket {Bp}, {self.decode_steps} step(s), "
-                    f"kv splits {st['nsplit']}, filtered={filtered}, penalized={penalized}")
+                    f"filtered={filtered}, penalized={penalized}")
         return g, st
 
     def _with_defaults(self, plan: Dict[str, Any], B: int) -> Dict[str, Any]:
@@ -1215,6 +1223,9 @@ class HybridModelRunner(ModelRunner):
                 choice[shape] = self._fastest(arms, max(8, len(mlps)), f"decode batch bucket {Bp}: gate|up {shape} ")
             self._gate_up_choice[Bp] = choice
         return self._gate_up_choice[Bp]
+
+    def _decode_items(self, Bp: int):
+        return None  # the mixers split their key ranges themselves
 
     def _decode_workspace(self, Bp: int):
         from ..ops import window_attention as wattn

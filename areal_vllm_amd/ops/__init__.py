@@ -2,6 +2,7 @@
 from ._lib import available as hip_available  # noqa: F401
 from .attention import (  # noqa: F401
     PAGE_SIZE,
+    DecodeItems,
     DecodeWorkspace,
     alloc_kv_cache,
     cache_gather,

@@ -438,10 +438,44 @@ class DecodeWorkspace:
         self.part_ml = torch.empty(max_batch, n_q_heads, max_splits, 2, dtype=torch.float32, device=device)
 
 
+# Work items of a decode attention over all key / value heads, before the at most half an item that a row's length adds:
+# one a CU, so that with the longest ones first most CUs have a second workgroup at work until the end (figures at
+# ``paged_decode_items_kernel``).
+DECODE_ITEMS = 256
+
+
+class DecodeItems:
+    """Work items of one decode step's attention (near-equal page ranges of the rows; ``paged_decode_items_kernel``) and
+    the buffers their partial results meet in; fixed sizes and addresses, so that captured graphs can refill them."""
+
+    def __init__(self, batch, n_q_heads, n_kv_heads, head_dim, device,
+                 max_context: Optional[int] = None):
+        self.batch, self.n_q_heads, self.n_kv_heads, self.head_dim = batch, n_q_heads, n_kv_heads, head_dim
+        self.target = max(1, DECODE_ITEMS // n_kv_heads)
+        self.n_items = self.target + batch
+        if max_context is not None:  # a row of n pages is at most sqrt(3 n) items
+            self.n_items = min(self.n_items, batch * (math.isqrt(3 * -(-int(max_context) // PAGE_SIZE)) + 1))
+        self.items = torch.zeros(self.n_items, 8, dtype=torch.int32, device=device)
+        self.part_o = torch.empty(self.n_items, n_q_heads, head_dim, dtype=torch.float32, device=device)
+        self.part_ml = torch.empty(self.n_items, n_q_heads, 2, dtype=torch.float32, device=device)
+        self.arrived = torch.zeros(batch, n_kv_heads, dtype=torch.int32, device=device)
+
+    def fill_(self, context_lens: torch.Tensor) -> "DecodeItems":
+        """Lay the items out for these context lengths; every layer of the step then uses them."""
+        if L.use_hip(context_lens):
+            assert context_lens.dtype == torch.int32 and context_lens.is_contiguous() and context_lens.numel() == self.batch
+            L.check(L.lib().areal_paged_decode_items(L.ptr(context_lens), L.ptr(self.items), L.c_int(self.batch),
+                                                     L.c_int(self.target), L.c_int(self.n_items), L.stream_ptr()),
+                    "paged_decode_items")
+        return self
+
+
 def paged_attention_decode(q, kcache, vcache, block_tables, context_lens, scale=None, nsplit=1,
-                           workspace: Optional[DecodeWorkspace] = None, out=None, q_row_stride=None):
+                           workspace: Optional[DecodeWorkspace] = None, out=None, q_row_stride=None,
+                           items: Optional[DecodeItems] = None):
     """q [B, Hq, D] (may be the q slice of a fused qkv row, pass q_row_stride in elements).
-    block_tables int32 [B, max_pages]; context_lens int32 [B] (including the current token)."""
+    block_tables int32 [B, max_pages]; context_lens int32 [B] (including the current token). `items`: the work items of
+    these context lengths (`nsplit` and `workspace` are not used then)."""
     B, Hq, D = q.shape
     Hkv = kcache.shape[1]
     if scale is None:
@@ -453,6 +487,18 @@ def paged_attention_decode(q, kcache, vcache, block_tables, context_lens, scale=
         out = torch.empty(B, Hq, D, dtype=q.dtype, device=q.device)
     if q_row_stride is None:
         q_row_stride = q.stride(0)
+    if items is not None:
+        assert (items.batch, items.n_q_heads, items.n_kv_heads, items.head_dim) == (B, Hq, Hkv, D)
+        L.check(
+            L.lib().areal_paged_decode_walk(
+                L.ptr(q), L.ptr(kcache), L.ptr(vcache), L.ptr(block_tables), L.ptr(context_lens), L.ptr(items.items),
+                L.c_int(items.n_items), L.ptr(out), L.ptr(items.part_o), L.ptr(items.part_ml), L.ptr(items.arrived),
+                L.c_int(Hq), L.c_int(Hkv), L.c_int(D), L.c_int(block_tables.shape[1]), L.c_float(scale),
+                L.c_int(q_row_stride), L.c_int(int(is_fp8(kcache))), L.stream_ptr(),
+            ),
+            "paged_decode_walk",
+        )
+        return out
     part_o = part_ml = None
     if nsplit > 1:
         if workspace is None:

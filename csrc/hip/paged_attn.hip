@@ -312,6 +312,364 @@ extern "C" int areal_paged_decode_window(const void* q, const void* kcache, cons
   return (int)hipGetLastError();
 }
 
+// ---------------------------------------------------------------------------------------------------
+// The same attention on a list of work items of near-equal size (one row and a range of its pages each), so that rows
+// of very different length load the chip evenly, and without a second launch for the combination.
+//
+// What bounds it: HBM streaming of the pages. Measured per layer (12 query heads on 2 key heads of 128 unless said), one
+// split count for all rows and a second launch -> items of about 1/256 of the batch and workgroups of 8 waves, two a CU:
+//   1 x 640 10.0 -> 7.0 us (latency), 24 x 200-4096 22.4 -> 15.4, 320 x 128-1152 53.6 -> 42.4 (3.9 -> 4.9 TB/s),
+//   256 x 640 32.3 -> 32.7 (even already), 64 x 128-1152 with 32 on 4 heads 25.8 -> 24.8, 1 x 16000 16.2 -> 16.3,
+//   fp8: 48 x 6000-24000 101 -> 77 (3.6 -> 4.7 TB/s), 24 x 200-4096 17.7 -> 11.0, 128 x 1000 21.4 -> 16.1.
+// More, smaller items cost more in combining than they even out (24 x 200-4096: 15.4 us with 256 items, 18.2 with 384;
+// 320 x 128-1152, every row divided by its length over the item's rounded up: 42 with 256, 46 with 768-1024).
+// The list depends on the context lengths alone: one launch per decode step serves every layer.
+//
+// Item: {row, first page, end page, first partial result of the row, number of the row's items, this item's partial
+// result} in 8 ints; count 0: none. Longest first: a workgroup that ends early takes the next item, and the short ones
+// fill the gaps at the end.
+struct DecodeItem { int b, p_beg, p_end, base, n, part, pad0, pad1; };
+
+// Pages per item of a row of np pages: the row evenly divided into items of about `even` pages (half as much again at
+// most: splitting a row that is a little longer than an item costs more than it evens out), a multiple of STEP; and so
+// many that the workgroup that combines a row's n partial results does not read longer than the others walk:
+// n^2 <= 3 pages (1 x 16000 tokens: 16.3 us, 22.4 us with n^2 <= 5 pages of 4-page items).
+constexpr int STEP = 4;
+DEVINL int pages_per_item(int np, int even) {
+  const int most = max(1, (int)sqrtf(3.f * (float)np));
+  const int n = min(most, max(1, (np + even / 2) / even));
+  const int per = (np + n - 1) / n;
+  return max(STEP, (per + STEP - 1) / STEP * STEP);
+}
+
+// grid 1, block 1024. n_items >= min(target + B, the rows' largest number of items x B). Pages per item: the whole batch over `target` items.
+__global__ __launch_bounds__(1024) void paged_decode_items_kernel(const int* __restrict__ context_lens,
+                                                                  DecodeItem* __restrict__ items, int B, int target,
+                                                                  int n_items) {
+  constexpr int NB = 64;  // size classes of the sort
+  __shared__ int red[16], hist[NB];
+  const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
+  int pages = 0;
+  for (int b = t; b < B; b += 1024) pages += (max(context_lens[b], 0) + PAGE - 1) / PAGE;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) pages += __shfl_xor(pages, o, 64);
+  if (lane == 0) red[wid] = pages;
+  if (t < NB) hist[t] = 0;
+  __syncthreads();
+  int total = 0;
+#pragma unroll
+  for (int w = 0; w < 16; ++w) total += red[w];
+  const int even = max(STEP, (total + target - 1) / target);
+  const int top = even + even / 2 + STEP;  // an item has more pages only if its row may not be divided further
+  auto size_class = [&](int size) { return NB - 1 - min(NB - 1, size * (NB - 1) / top); };
+  for (int b = t; b < B; b += 1024) {  // items per size class
+    const int np = (max(context_lens[b], 0) + PAGE - 1) / PAGE, per = pages_per_item(np, even);
+    const int n = max(1, (np + per - 1) / per);
+    if (n > 1) atomicAdd(&hist[size_class(per)], n - 1);
+    atomicAdd(&hist[size_class(np - (n - 1) * per)], 1);
+  }
+  __syncthreads();
+  if (t < NB) {  // first place of every class (64 lanes: one wave)
+    int incl = hist[t];
+    const int own = incl;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_up(incl, o, 64);
+      if (lane >= o) incl += v;
+    }
+    hist[t] = incl - own;
+  }
+  int at = 0;  // items of the rows before this pass over 1024 rows
+  for (int b0 = 0; b0 < B; b0 += 1024) {
+    const int b = b0 + t;
+    const int np = b < B ? (max(context_lens[b], 0) + PAGE - 1) / PAGE : 0;
+    const int per = pages_per_item(np, even);
+    const int n = b < B ? max(1, (np + per - 1) / per) : 0;
+    int incl = n;  // prefix sum over the block
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_up(incl, o, 64);
+      if (lane >= o) incl += v;
+    }
+    __syncthreads();
+    if (lane == 63) red[wid] = incl;
+    __syncthreads();
+    int before = at;
+    for (int w = 0; w < 16; ++w) {
+      if (w < wid) before += red[w];
+      at += red[w];
+    }
+    const int base = before + incl - n;
+    for (int i = 0; i < n; ++i) {
+      const int lo = i * per, hi = min(np, lo + per);
+      const int place = atomicAdd(&hist[size_class(hi - lo)], 1);
+      if (place < n_items && base + n <= n_items) items[place] = DecodeItem{b, lo, hi, base, n, base + i, 0, 0};
+    }
+  }
+  for (int i = at + t; i < n_items; i += 1024) items[i] = DecodeItem{0, 0, 0, 0, 0, 0, 0, 0};
+}
+
+// Partial results travel between workgroups of any XCD: stores and loads at agent scope go past the XCD's own L2, so a
+// store that has been waited for (vmcnt) is seen by every later load of this kind. Nothing else has to be written back or
+// invalidated: acquire / release at agent scope on the counter would flush the whole L2 for each workgroup (measured:
+// 93 instead of 34 us for 256 rows of 640 tokens in two items each).
+DEVINL void st_agent(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+DEVINL float ld_agent(const float* p) {
+  return __hip_atomic_load(const_cast<float*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// grid: n_items x Hkv, the heads of an item beside each other and the empty items last (workgroups that exit at once, spread
+// among the others, leave some CUs with two and some with none: 120 instead of 96 us for 64 rows of 4000 tokens, 4 heads);
+// block: NW waves, page by page in turn. part_o: [n_items, Hq, D], part_ml: [n_items, Hq, 2],
+// arrived: [B, Hkv] zeros, zeros again afterwards. The last workgroup of a row to arrive combines its partial results
+// in the order of the items: the result does not depend on the order of arrival.
+// LDS holds the G real query rows only: 8 workgroups of a GQA group of 6 fit a CU (the padded 16 rows: 4).
+template <int D, bool FP8, int NW>
+__global__ __launch_bounds__(64 * NW, (D > 128 ? 1 : 2)) void paged_decode_walk_kernel(
+    const bf16_t* __restrict__ q, const void* __restrict__ kcache, const void* __restrict__ vcache,
+    const int* __restrict__ block_tables, const int* __restrict__ context_lens, const DecodeItem* __restrict__ items,
+    bf16_t* __restrict__ out, float* __restrict__ part_o, float* __restrict__ part_ml, int* __restrict__ arrived, int Hq,
+    int Hkv, int max_pages, float scale_log2, int q_stride) {
+  constexpr int KS = D / 32, DB = D / 16, DP = D + 4;
+  extern __shared__ __attribute__((aligned(16))) float smem[];
+  __shared__ int last;
+  const DecodeItem it = items[blockIdx.x / Hkv];
+  if (it.n == 0) return;
+  const int b = it.b, h = blockIdx.x % Hkv;
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const int G = Hq / Hkv;
+  const int col = lane & 15, c = lane >> 4;
+  const int* bt = block_tables + (size_t)b * max_pages;
+  // this wave's pages: p_beg + wid + NW i; 64 page ids are fetched at once, one a lane
+  const int mine = it.p_end - it.p_beg > wid ? (it.p_end - it.p_beg - wid + NW - 1) / NW : 0;
+  int ids = lane < mine ? bt[it.p_beg + wid + NW * lane] : 0;
+  const int ctx = context_lens[b];
+  // Q as the B operand of S^T = K.Q^T. fp8: a lane's 16 loaded bytes of K are the operand of two k-steps, so lane c
+  // holds Q[64 (ks / 2) + 16 c + 8 (ks % 2) + j] there and Q[32 ks + 8 c + j] otherwise
+  bf16x8 qf[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    const int k0 = FP8 ? (ks >> 1) * 64 + c * 16 + (ks & 1) * 8 : ks * 32 + c * 8;
+    if (col < G) qf[ks] = ld8(q + (size_t)b * q_stride + (size_t)(h * G + col) * D + k0);
+    else
+#pragma unroll
+      for (int j = 0; j < 8; ++j) qf[ks][j] = (bf16_t)0.f;
+  }
+  f32x4 o[DB];
+#pragma unroll
+  for (int i = 0; i < DB; ++i) o[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  float m = -INFINITY, l = 0.f;  // running max (log2 units) is shared by the 4 lanes of a q
+  const int key_a = 8 * (col >> 2) + (col & 3);  // row `col` of tile a; tile b: 4 rows further
+
+  for (int i = 0; i < mine; ++i) {
+    if (i > 0 && (i & 63) == 0) ids = lane + i < mine ? bt[it.p_beg + wid + NW * (lane + i)] : 0;
+    const int p = it.p_beg + wid + NW * i;
+    const int page = __builtin_amdgcn_readlane(ids, i & 63);
+    const size_t kp = ((size_t)page * Hkv + h) * PAGE * D;  // element offset of this page's K / V block
+    // all loads of the page up front (16 KiB, fp8: 8 KiB a wave in flight)
+    bf16x8 ka[KS], kb[KS], vt[DB];
+    if (FP8) {
+      const fp8_t* kc = reinterpret_cast<const fp8_t*>(kcache) + kp + key_a * D + c * 16;
+      const fp8_t* vc = reinterpret_cast<const fp8_t*>(vcache) + kp + col * PAGE + c * 8;
+      u32x4 ra[KS / 2], rb[KS / 2];
+      u32x2 rv[DB];
+#pragma unroll
+      for (int k2 = 0; k2 < KS / 2; ++k2) {
+        ra[k2] = *reinterpret_cast<const u32x4*>(kc + k2 * 64);
+        rb[k2] = *reinterpret_cast<const u32x4*>(kc + 4 * D + k2 * 64);
+      }
+#pragma unroll
+      for (int j = 0; j < DB; ++j) rv[j] = *reinterpret_cast<const u32x2*>(vc + j * 16 * PAGE);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int k2 = 0; k2 < KS / 2; ++k2) {
+        ka[2 * k2] = fp8x8_to_bf16((u32x2){ra[k2][0], ra[k2][1]});
+        ka[2 * k2 + 1] = fp8x8_to_bf16((u32x2){ra[k2][2], ra[k2][3]});
+        kb[2 * k2] = fp8x8_to_bf16((u32x2){rb[k2][0], rb[k2][1]});
+        kb[2 * k2 + 1] = fp8x8_to_bf16((u32x2){rb[k2][2], rb[k2][3]});
+      }
+#pragma unroll
+      for (int j = 0; j < DB; ++j) vt[j] = fp8x8_to_bf16(rv[j]);
+    } else {
+      const bf16_t* kc = reinterpret_cast<const bf16_t*>(kcache) + kp + key_a * D + c * 8;
+      const bf16_t* vc = reinterpret_cast<const bf16_t*>(vcache) + kp + col * PAGE + c * 8;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        ka[ks] = ld8(kc + ks * 32);
+        kb[ks] = ld8(kc + 4 * D + ks * 32);
+      }
+#pragma unroll
+      for (int j = 0; j < DB; ++j) vt[j] = ld8(vc + j * 16 * PAGE);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    f32x4 sa = {0.f, 0.f, 0.f, 0.f}, sb = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      sa = mfma16(ka[ks], qf[ks], sa);
+      sb = mfma16(kb[ks], qf[ks], sb);
+    }
+    // lane (q = col, c): sa[r] = S[key 8c + r], sb[r] = S[key 8c + 4 + r]
+    float s[8];
+    const int key0 = p * PAGE + 8 * c;
+    float mx = -INFINITY;
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      const float v = (r < 4 ? sa[r] : sb[r - 4]) * scale_log2;
+      s[r] = key0 + r < ctx ? v : -INFINITY;
+      mx = fmaxf(mx, s[r]);
+    }
+    mx = max_xor16(mx);
+    mx = max_xor32(mx);
+    const float mn = fmaxf(m, mx);
+    if (__any(mn > m)) {
+      const float alpha = (m == -INFINITY) ? 0.f : fast_exp2(m - mn);
+      l *= alpha;
+#pragma unroll
+      for (int j = 0; j < DB; ++j) o[j] *= alpha;
+      m = mn;
+    }
+    bf16x8 pf;
+    float ls = 0.f;
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      const float pr = (m == -INFINITY) ? 0.f : fast_exp2(s[r] - m);
+      ls += pr;
+      pf[r] = f2bf(pr);
+    }
+    l += ls;
+    // O^T[d, q] += V^T[d, keys] . P^T[keys, q]
+#pragma unroll
+    for (int j = 0; j < DB; ++j) o[j] = mfma16(vt[j], pf, o[j]);
+  }
+  l = sum_xor16(l);  // l is a per-lane partial over this lane's keys: sum the 4 lanes that share a q
+  l = sum_xor32(l);
+
+  // combine the waves through LDS: rows DP floats apart keep the 16-byte stores of a wave's rows on different banks
+  float* so = smem;                // [NW][G][DP]
+  float* sm = smem + NW * G * DP;  // [NW][16]
+  float* sl = sm + NW * 16;        // [NW][16]
+  if (col < G) {
+#pragma unroll
+    for (int j = 0; j < DB; ++j) *reinterpret_cast<f32x4*>(so + (wid * G + col) * DP + j * 16 + 4 * c) = o[j];
+  }
+  if (c == 0) { sm[wid * 16 + col] = m; sl[wid * 16 + col] = l; }
+  __syncthreads();
+  for (int idx = threadIdx.x; idx < G * D; idx += 64 * NW) {
+    const int qq = idx / D, d = idx % D;
+    float mm = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) mm = fmaxf(mm, sm[w * 16 + qq]);
+    float acc = 0.f, ll = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const float mw = sm[w * 16 + qq];
+      const float f = (mw == -INFINITY) ? 0.f : fast_exp2(mw - mm);
+      acc += so[(w * G + qq) * DP + d] * f;
+      ll += sl[w * 16 + qq] * f;
+    }
+    const int head = h * G + qq;
+    if (it.n == 1) {
+      out[((size_t)b * Hq + head) * D + d] = f2bf(ll > 0.f ? acc / ll : 0.f);
+    } else {
+      const size_t row = (size_t)it.part * Hq + head;
+      st_agent(part_o + row * D + d, acc);
+      if (d == 0) {
+        st_agent(part_ml + row * 2, mm);
+        st_agent(part_ml + row * 2 + 1, ll);
+      }
+    }
+  }
+  if (it.n == 1) return;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // every wave's stores have arrived ...
+  __syncthreads();
+  if (threadIdx.x == 0) {                           // ... before the workgroup is counted
+    const int old = __hip_atomic_fetch_add(arrived + (size_t)b * Hkv + h, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    last = old == it.n - 1;
+    if (last) __hip_atomic_store(arrived + (size_t)b * Hkv + h, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
+  if (!last) return;
+  for (int idx = threadIdx.x; idx < G * D; idx += 64 * NW) {
+    const int head = h * G + idx / D, d = idx % D;
+    const float* ml = part_ml + ((size_t)it.base * Hq + head) * 2;
+    const float* po = part_o + ((size_t)it.base * Hq + head) * D + d;
+    float mm = -INFINITY, acc = 0.f, ll = 0.f;
+    for (int s0 = 0; s0 < it.n; s0 += 8) {  // eight partial results in flight
+      float ms[8], ls[8], os[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const size_t s = min(s0 + j, it.n - 1);
+        ms[j] = s0 + j < it.n ? ld_agent(ml + s * Hq * 2) : -INFINITY;
+        ls[j] = ld_agent(ml + s * Hq * 2 + 1);
+        os[j] = ld_agent(po + s * Hq * D);
+      }
+      float mn = mm;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) mn = fmaxf(mn, ms[j]);
+      const float f0 = mm == -INFINITY ? 0.f : fast_exp2(mm - mn);
+      acc *= f0;
+      ll *= f0;
+      mm = mn;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float f = ms[j] == -INFINITY ? 0.f : fast_exp2(ms[j] - mn);
+        acc += os[j] * f;
+        ll += ls[j] * f;
+      }
+    }
+    out[((size_t)b * Hq + head) * D + d] = f2bf(ll > 0.f ? acc / ll : 0.f);
+  }
+}
+
+// Items of the batch's decode attention; `items`: n_items x 8 ints, at least min(target + B, B x most items of a row).
+extern "C" int areal_paged_decode_items(const int* context_lens, void* items, int B, int target, int n_items,
+                                        hipStream_t st) {
+  if (B < 1 || target < 1 || n_items < B) return -1;
+  hipLaunchKernelGGL(paged_decode_items_kernel, dim3(1), dim3(1024), 0, st, context_lens, (DecodeItem*)items, B, target,
+                     n_items);
+  return (int)hipGetLastError();
+}
+
+template <int D, bool FP8, int NW>
+static int launch_paged_decode_walk(const void* q, const void* kcache, const void* vcache, const int* block_tables,
+                                    const int* context_lens, const void* items, int n_items, void* out, float* part_o,
+                                    float* part_ml, int* arrived, int Hq, int Hkv, int max_pages, float scale_log2,
+                                    int q_stride, hipStream_t st) {
+  const size_t lds = (size_t)(NW * (Hq / Hkv) * (D + 4) + 2 * NW * 16) * sizeof(float);
+  if (lds > 65536) {  // large groups: above the default limit
+    static bool attr_set = false;
+    if (!attr_set) {
+      HIP_RET(hipFuncSetAttribute((const void*)paged_decode_walk_kernel<D, FP8, NW>,
+                                  hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  (int)((NW * 16 * (D + 4) + 2 * NW * 16) * sizeof(float))));
+      attr_set = true;
+    }
+  }
+  hipLaunchKernelGGL((paged_decode_walk_kernel<D, FP8, NW>), dim3(n_items * Hkv), dim3(64 * NW), lds, st, (const bf16_t*)q, kcache,
+                     vcache, block_tables, context_lens, (const DecodeItem*)items, (bf16_t*)out, part_o, part_ml, arrived,
+                     Hq, Hkv, max_pages, scale_log2, q_stride);
+  return (int)hipGetLastError();
+}
+
+// Decode attention over the items that areal_paged_decode_items made of the same context lengths.
+extern "C" int areal_paged_decode_walk(const void* q, const void* kcache, const void* vcache, const int* block_tables,
+                                       const int* context_lens, const void* items, int n_items, void* out, float* part_o,
+                                       float* part_ml, int* arrived, int Hq, int Hkv, int D, int max_pages,
+                                       float softmax_scale, int q_stride, int fp8, hipStream_t st) {
+  if (n_items == 0) return 0;
+  if (Hq % Hkv != 0 || Hq / Hkv > 16) return -1;
+  if (D != 128 && D != 64 && D != 256) return -2;
+  const float scale_log2 = softmax_scale * 1.4426950408889634f;
+#define PD(DD, F8, NW)                                                                                                  \
+  return launch_paged_decode_walk<DD, F8, NW>(q, kcache, vcache, block_tables, context_lens, items, n_items, out, part_o, \
+                                              part_ml, arrived, Hq, Hkv, max_pages, scale_log2, q_stride, st)
+  if (D == 256) { if (fp8) PD(256, true, 4); else PD(256, false, 4); }
+  if (D == 128) { if (fp8) PD(128, true, 8); else PD(128, false, 8); }
+  if (fp8) PD(64, true, 8);
+  PD(64, false, 8);
+#undef PD
+}
+
 // ----------------------------------------------------------------------------------
 // Fused RoPE + KV-cache write. qkv: [T, Hq + 2*Hkv, D] (q heads, k heads, v heads).
 // Rotates q and k in place (half-split layout) and scatters k / v of every token into

@@ -1,0 +1,62 @@
+"""Decode attention on work items: the items cover every row's pages once, and the walk equals attention in fp32."""
+import math
+
+import pytest
+import torch
+
+from areal_vllm_amd import ops
+from areal_vllm_amd.ops import attention as A
+
+DEV = "cuda:0"
+pytestmark = pytest.mark.gpu
+
+
+def _setup(ctx, Hq, Hkv, D, fp8, seed):
+    g = torch.Generator().manual_seed(seed)
+    need = [(c + 31) // 32 for c in ctx]
+    width = max(need + [1]) + 1
+    bt = torch.zeros(len(ctx), width, dtype=torch.int32)
+    perm, at = torch.randperm(sum(need), generator=g) + 1, 0
+    for b, n in enumerate(need):
+        bt[b, :n] = perm[at:at + n].int()
+        at += n
+    kc, vc = ops.alloc_kv_cache(sum(need) + 1, Hkv, D, torch.bfloat16, "cpu")
+    kc.copy_(torch.randn(kc.shape, generator=g))
+    vc.copy_(torch.randn(vc.shape, generator=g))
+    if fp8:
+        kc, vc = kc.to(A.FP8), vc.to(A.FP8)
+    q = torch.randn(len(ctx), Hq + 1, D, generator=g).bfloat16()
+    return q, kc, vc, bt, torch.tensor(ctx, dtype=torch.int32)
+
+
+@pytest.mark.parametrize("Hq,Hkv,D,fp8", [(12, 2, 128, False), (12, 2, 128, True), (32, 4, 128, False), (7, 7, 64, False),
+                                          (16, 2, 64, True), (8, 1, 256, False), (16, 1, 256, True)])
+@pytest.mark.parametrize("ctx", [[1], [640], [0, 1, 31, 32, 33, 127, 128, 129, 4099], [3000] * 3 + [1] * 1100])
+def test_decode_attention_on_items(Hq, Hkv, D, fp8, ctx):
+    if len(ctx) > 100 and Hkv == 7:
+        pytest.skip("one wide batch a head count is enough")
+    q, kc, vc, bt, cl = _setup(ctx, Hq, Hkv, D, fp8, 3)
+    d = [t.to(DEV) for t in (q, kc, vc, bt, cl)]
+    items = ops.DecodeItems(len(ctx), Hq, Hkv, D, torch.device(DEV)).fill_(d[4])
+    tight = ops.DecodeItems(len(ctx), Hq, Hkv, D, torch.device(DEV), max_context=max(ctx)).fill_(d[4])
+    assert tight.n_items <= items.n_items and int((tight.items[:, 4] > 0).sum()) == int((items.items[:, 4] > 0).sum())
+    # rows' pages: contiguous ranges, in order, of at most one multiple of four pages each
+    rows = {}
+    parts = set()
+    for b, lo, hi, base, n, part in items.items[:, :6].tolist():
+        if n:
+            rows.setdefault(b, []).append((part - base, lo, hi, n))
+            parts.add(part)
+    assert sorted(rows) == list(range(len(ctx))) and len(parts) == sum(len(r) for r in rows.values())
+    for b, c in enumerate(ctx):
+        r = sorted(rows[b])
+        assert [x[0] for x in r] == list(range(len(r))) and all(x[3] == len(r) for x in r)
+        edges = [0] + [x[2] for x in r]
+        assert [x[1] for x in r] == edges[:-1] and edges[-1] == (c + 31) // 32 and all(e % 4 == 0 for e in edges[:-1])
+    ref = A.paged_decode_ref(q[:, :Hq], kc, vc, bt, cl, 1 / math.sqrt(D)).float()
+    outs = [ops.paged_attention_decode(d[0][:, :Hq], *d[1:], q_row_stride=(Hq + 1) * D, items=items).float().cpu()
+            for _ in range(3)]
+    # P in bf16 (2^-9 relative per weight) and a bf16 result: errors of a few 2^-9 of values of order one
+    assert (outs[0] - ref).abs().max() < 2e-2
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])  # counters are back at zero, order is fixed
+    assert int(items.arrived.abs().sum()) == 0
