@@ -459,7 +459,7 @@ class ModelRunner:
         instead of at the first decode step of each bucket, when a colocated trainer may be sharing the device."""
         if self.fused_decode and self.device.type == "cuda":
             for b in self.buckets:
-                if b >= self.FUSED_MIN_BATCH:
+                if b >= self.FUSED_MIN_BATCH and not self._skinny(b):
                     self._gate_up_mode(b)
 
     def _gate_up_mode(self, Bp: int) -> str:
@@ -532,6 +532,8 @@ class ModelRunner:
         half and run router and experts through the grouped kernels, then residual + the next norm."""
         from ..ops import decode_gemm as dg
 
+        if self._skinny(h.shape[0]):
+            return self._decode_layers_skinny(st, h, rope_pos)
         cfg = self.cfg
         hq, hkv, D = self.hq, self.hkv, cfg.head_dim
         Bp, H = h.shape
@@ -585,6 +587,41 @@ class ModelRunner:
             slab = dg.dgemm(act, blk.mlp.down, epilogue=dg.EPI_SLAB)
             x, residual = finish(slab, residual, nw)
         return x
+
+    # Rows up to which the five-launch layer is faster than split-K GEMMs with row kernels, for hidden sizes up to 1536 and
+    # above. 28 layers of Qwen2-1.5B at 1 / 2 / 4 / 6 / 8 rows: 1.17 / 1.24 / 1.36 / 1.45 / 1.50 ms a step against 1.44 / 1.44 /
+    # 1.47 / 1.58 / 1.48; 12 layers of Llama-3-8B at 1 / 2 / 4: 1.47 / 1.55 / 1.65 against 1.66 / 1.66 / 1.58 (a row's weights
+    # no longer fit the registers at once, and the matrix-core form does not load ahead there).
+    SKINNY_MAX_ROWS, SKINNY_MAX_ROWS_WIDE = 6, 2
+
+    def _skinny(self, rows: int) -> bool:
+        """Whether a decode step of so many rows runs the five-launch layer of ``ops/decode_skinny.py``."""
+        from ..ops import decode_skinny as sk
+
+        cfg = self.cfg
+        return (rows <= (self.SKINNY_MAX_ROWS if cfg.hidden_size <= 1536 else self.SKINNY_MAX_ROWS_WIDE) and self.fused_decode and not self.tp_comm and not cfg.qk_norm
+                and cfg.n_experts == 0 and self.dtype == torch.bfloat16
+                and sk.serves(cfg.hidden_size, cfg.intermediate_size, self.hq * cfg.head_dim, cfg.head_dim))
+
+    def _decode_layers_skinny(self, st: Dict[str, torch.Tensor], h: torch.Tensor, rope_pos: torch.Tensor):
+        """All decoder layers of a decode step of a few rows -> final-normed hidden states [Bp, H]."""
+        from ..ops import decode_skinny as sk
+
+        cfg = self.cfg
+        hq, hkv, D = self.hq, self.hkv, cfg.head_dim
+        Bp = h.shape[0]
+        eps, gemma = cfg.rms_norm_eps, cfg.gemma_norm
+        act = "silu" if cfg.hidden_act == "silu" else "gelu_tanh"
+        residual = h
+        for li, blk in enumerate(self.model.layers):
+            kc, vc = self.kv[li]
+            q = sk.norm_qkv_rope(residual, blk.ln1, blk.attn.qkv, blk.attn.qkv_bias, rope_pos, st["slots"], self.rope, kc,
+                                 vc, hq, hkv, D, eps=eps, gemma=gemma)
+            attn = ops.paged_attention_decode(q, kc, vc, st["block_tables"], st["context_lens"], items=st["items"])
+            residual = sk.linear_residual(attn.view(Bp, hq * D), blk.attn.o, residual)
+            a = sk.norm_gated(residual, blk.ln2, blk.mlp.gate_up, eps=eps, gemma=gemma, act=act)
+            residual = sk.linear_residual(a, blk.mlp.down, residual)
+        return ops.rmsnorm(residual, self.model.norm, eps, None, gemma)[0]
 
     LM_HEAD_OWN_MAX_ROWS = 96
 

@@ -1,0 +1,92 @@
+"""Projections of a decode step of at most 8 rows with the row work around them in the same launch
+(``csrc/hip/decode_skinny.hip``). One decoder layer is five launches:
+
+    residual --norm_qkv_rope (RMSNorm, q|k|v, bias, RoPE, KV-cache write)--> q --paged attention-->
+    --linear_residual (o)--> residual --norm_gated (RMSNorm, gate|up, activation)--> act --linear_residual (down)--> residual
+
+CPU tensors take PyTorch paths with the same rounding points.
+"""
+from typing import Optional
+
+import torch
+import torch.nn.functional as F
+
+from . import _lib as L
+from .decode_gemm import EPI_GEGLU, EPI_SWIGLU, _gate
+
+MAX_ROWS = 8
+MAX_NORM_WIDTH = 8192  # values of a normalised row: 8 of them fit the LDS of a CU
+
+
+def serves(hidden: int, inner: int, q_width: int, head_dim: int) -> bool:
+    """Whether the kernels take a layer of this hidden size, MLP width, query width and head size."""
+    return (hidden % 64 == 0 and hidden <= MAX_NORM_WIDTH and inner % 64 == 0 and q_width % 64 == 0
+            and head_dim % 16 == 0)
+
+
+def _norm_ref(h, weight, eps, gemma):
+    hf = h.float()
+    return (hf * torch.rsqrt(hf.pow(2).mean(-1, keepdim=True) + eps)
+            * (weight.float() + (1.0 if gemma else 0.0))).to(h.dtype)
+
+
+def _rows(x: torch.Tensor, w: torch.Tensor) -> None:
+    assert x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2 and x.shape[0] <= MAX_ROWS
+    assert x.stride(1) == 1 and w.is_contiguous() and w.shape[1] == x.shape[1]
+
+
+def linear_residual(x: torch.Tensor, w: torch.Tensor, residual: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """``round(x @ w.T) + residual`` rounded again, bf16 [M, N]."""
+    M, K = x.shape
+    N = w.shape[0]
+    if not L.use_hip(x):
+        y = F.linear(x.float(), w.float()).to(x.dtype)
+        return y if residual is None else (y.float() + residual.float()).to(x.dtype)
+    _rows(x, w)
+    assert residual is None or (residual.dtype == x.dtype and residual.shape == (M, N) and residual.is_contiguous())
+    y = torch.empty(M, N, dtype=x.dtype, device=x.device)
+    L.check(L.lib().areal_skinny_residual(L.ptr(x), L.c_int64(x.stride(0)), L.ptr(w), L.ptr(residual), L.ptr(y), L.c_int(M),
+                                          L.c_int(N), L.c_int(K), L.stream_ptr()), "skinny_residual")
+    return y
+
+
+def norm_gated(h: torch.Tensor, norm: torch.Tensor, w_gate_up: torch.Tensor, *, eps: float, gemma: bool = False,
+               act: str = "silu") -> torch.Tensor:
+    """``act(x @ gate.T) * (x @ up.T)`` of ``x = rmsnorm(h) * norm`` with ``w_gate_up = [gate; up]`` -> bf16 [M, F]."""
+    M, K = h.shape
+    Fc = w_gate_up.shape[0] // 2
+    if not L.use_hip(h):
+        y = F.linear(_norm_ref(h, norm, eps, gemma).float(), w_gate_up.float()).to(h.dtype).float()
+        return (_gate(y[:, :Fc], EPI_SWIGLU if act == "silu" else EPI_GEGLU) * y[:, Fc:]).to(h.dtype)
+    _rows(h, w_gate_up)
+    assert norm.dtype == torch.bfloat16 and norm.is_contiguous() and norm.numel() == K
+    y = torch.empty(M, Fc, dtype=h.dtype, device=h.device)
+    L.check(L.lib().areal_skinny_norm_gated(L.ptr(h), L.c_int64(h.stride(0)), L.ptr(norm), L.ptr(w_gate_up), L.ptr(y),
+                                            L.c_int(M), L.c_int(Fc), L.c_int(K), L.c_float(eps), L.c_int(int(gemma)),
+                                            L.c_int(0 if act == "silu" else 1), L.stream_ptr()), "skinny_norm_gated")
+    return y
+
+
+def norm_qkv_rope(h: torch.Tensor, norm: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], positions, slots,
+                  table, kcache, vcache, n_q_heads: int, n_kv_heads: int, head_dim: int, *, eps: float,
+                  gemma: bool = False, do_rope: bool = True) -> torch.Tensor:
+    """The packed q|k|v projection of ``rmsnorm(h) * norm`` with bias; q and k rotated, k and v written into the paged
+    caches at ``slots`` (negative: not written); returns the rotated q ``[M, Hq, D]``."""
+    M, K = h.shape
+    Hq, Hkv, D = n_q_heads, n_kv_heads, head_dim
+    if not L.use_hip(h):
+        from .attention import rope_and_cache_write_
+
+        y = F.linear(_norm_ref(h, norm, eps, gemma).float(), w.float(), None if bias is None else bias.float())
+        qkv = y.to(h.dtype).view(M, Hq + 2 * Hkv, D).contiguous()
+        return rope_and_cache_write_(qkv, positions, slots, table, kcache, vcache, Hq, Hkv, do_rope)[:, :Hq].contiguous()
+    _rows(h, w)
+    assert w.shape[0] == (Hq + 2 * Hkv) * D and norm.dtype == torch.bfloat16 and norm.is_contiguous() and norm.numel() == K
+    assert positions.dtype == torch.int32 and slots.dtype == torch.int64 and positions.numel() >= M and slots.numel() >= M
+    q = torch.empty(M, Hq, D, dtype=h.dtype, device=h.device)
+    L.check(L.lib().areal_skinny_norm_qkv(
+        L.ptr(h), L.c_int64(h.stride(0)), L.ptr(norm), L.ptr(w), L.ptr(bias), L.ptr(positions), L.ptr(slots),
+        L.ptr(table.cos), L.ptr(table.sin), L.ptr(q), L.ptr(kcache), L.ptr(vcache), L.c_int(M), L.c_int(K), L.c_int(Hq),
+        L.c_int(Hkv), L.c_int(D), L.c_int(table.max_pos), L.c_int(int(do_rope)), L.c_float(eps), L.c_int(int(gemma)),
+        L.c_int(int(kcache.dtype == torch.float8_e4m3fn)), L.stream_ptr()), "skinny_norm_qkv")
+    return q

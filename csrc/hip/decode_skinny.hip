@@ -1,0 +1,530 @@
+// The projections of a decoder layer for a decode step of at most 8 rows, on gfx950: Y[M, N] = X[M, K] W[N, K]^T with
+// what surrounds it in the same launch, five launches a layer instead of eight:
+//
+//   qkv      RMSNorm of the residual stream, the projection, bias, rotation, KV-cache write
+//   (paged attention)
+//   o        the projection + residual sum
+//   gate|up  RMSNorm, the projection, gated activation
+//   down     the projection + residual sum
+//
+// What bounds it: streaming the weights (55 MB from 256 workgroups that only load: 9.9 us; 6 TB/s in steady state), and as
+// much the chain of dependent launches: a row kernel that sums split-K slabs and normalises takes 4.4 us for a few KB. So
+// a workgroup owns its columns over ALL of K - no slabs, nothing to hand over - and normalises the rows itself, under the
+// latency of its weight loads. One workgroup a CU: N / 256 columns each (o, down of Qwen2-1.5B: 6, gate|up: 35 + 35, qkv:
+// 4 rotated pairs).
+//
+//   * one and two rows: no matrix cores. A packed dot product (v_dot2_f32_bf16: two products added to an fp32 sum) per
+//     pair of weights and row keeps up with memory, and a wave reads 1 KiB of ONE weight row per load instruction; as
+//     matrix operands (16 rows x 64 bytes a load) the same bytes take 10.8 instead of 9.2 us to load;
+//   * three to eight rows: matrix cores (with three rows the dot products take as long as the loads, with eight twice as
+//     long: 2.3 ms a step); from nine rows on the split-K path is as fast;
+//   * 8 waves: WK along K, 8 / WK along the rows, WK so that a wave's share of K is at most 3 x 64 pieces of 16 bytes
+//     (K = 1536: WK = 1, K = 8960: WK = 8); the wave's share of the activations stays in registers for all its rows;
+//   * two sets of RB weight rows in registers: all loads of gate|up, o and down of Qwen2-1.5B are in flight at once;
+//   * lane sums are folded two values at a time by permlane swaps; the waves' sums meet in LDS and are added in the order
+//     of the waves: results do not depend on timing.
+//
+// Rounding points are those of the split-K path (csrc/hip/decode_gemm.hip): normalised rows, projection and residual
+// sum in bf16, sums in fp32.
+//
+// Measured (Qwen2-1.5B, 640-token contexts, captured decode step of 28 layers), split-K path -> this: 1 row 1.44 -> 1.17 ms,
+// 2 rows 1.44 -> 1.24, 4 rows 1.47 -> 1.36, 6 rows 1.58 -> 1.45, 8 rows level. One row: gate|up 13.1 us, down 8.5, o 3.9,
+// qkv 5.2 (8.0 + 4.4, 4.6 + 4.4, 12.5, 4.6 + 4.4 before).
+#include "common.hpp"
+
+namespace {
+
+enum { SK_RES = 0, SK_GATED = 1, SK_QKV = 2 };
+constexpr int WAVES = 8, THREADS = 64 * WAVES;
+
+struct SKArgs {
+  const bf16_t* X;   // [M, K] rows of stride xs: activations, or the residual stream (NORM)
+  const bf16_t* W;   // [N, K]
+  const bf16_t* nw;  // norm weight [K]
+  const bf16_t* res; // SK_RES: residual rows [M, N] (contiguous) or null
+  bf16_t* Y;         // SK_RES: [M, N]; SK_GATED: [M, N / 2]; SK_QKV: rotated q [M, Hq, D]
+  int64_t xs;
+  int M, N, K, cols; // cols: columns of a workgroup (SK_GATED: of either half; SK_QKV: rotated pairs)
+  int wk;            // waves along K: 1, 2, 4 or 8
+  float eps;
+  int gemma, act;
+  const bf16_t* bias;
+  const int* pos;
+  const int64_t* slots;
+  const float* cos_t;
+  const float* sin_t;
+  void* kcache;
+  void* vcache;
+  int Hq, Hkv, D, max_pos, do_rope, fp8;
+};
+
+DEVINL float sk_gate(float x, int act) {
+  if (act == 0) return x / (1.f + __expf(-x));
+  const float inner = 0.7978845608028654f * (x + 0.044715f * x * x * x);
+  const float e = __expf(-2.f * fabsf(inner));
+  return 0.5f * x * (1.f + copysignf((1.f - e) / (1.f + e), inner));
+}
+
+constexpr int P = 3;  // passes of 64 16-byte pieces that a wave makes over its share of K
+
+// Sum over the 64 lanes of each of V values; value v ends up in the lanes of row (v % 4 -> 0, 2, 1, 3) of out[v / 4].
+template <int V>
+DEVINL void lane_sums(const float (&x)[V], float (&out)[(V + 3) / 4]) {
+#pragma unroll
+  for (int j = 0; j < (V + 3) / 4; ++j) {
+    float y[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const unsigned a = __float_as_uint(4 * j + 2 * h < V ? x[4 * j + 2 * h < V ? 4 * j + 2 * h : 0] : 0.f);
+      const unsigned b = __float_as_uint(4 * j + 2 * h + 1 < V ? x[4 * j + 2 * h + 1 < V ? 4 * j + 2 * h + 1 : 0] : 0.f);
+      const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);  // {a low, b low}, {a high, b high}
+      y[h] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    }
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(y[0]), __float_as_uint(y[1]), false, false);
+    float z = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+#pragma unroll
+    for (int o = 8; o > 0; o >>= 1) z += __shfl_xor(z, o, 64);
+    out[j] = z;
+  }
+}
+
+DEVINL float dot8(bf16x8 a, bf16x8 b, float c) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    c = __builtin_amdgcn_fdot2_f32_bf16((bf16x2){a[2 * i], a[2 * i + 1]}, (bf16x2){b[2 * i], b[2 * i + 1]}, c, false);
+  return c;
+}
+
+// What follows the projection; sum(j, h, m): the fp32 sum of column j (SK_GATED: of half h; SK_QKV: member h of pair j) of
+// row m, read from LDS.
+template <int MODE, typename Sum>
+DEVINL void finish(const SKArgs& a, Sum sum) {
+  if (MODE == SK_RES) {
+    for (int i = threadIdx.x; i < a.cols * a.M; i += THREADS) {
+      const int j = i % a.cols, m = i / a.cols, n = blockIdx.x * a.cols + j;
+      if (n >= a.N) continue;
+      float s = sum(j, 0, m);
+      if (a.res) s = bf2f(f2bf(s)) + bf2f(a.res[(size_t)m * a.N + n]);
+      a.Y[(size_t)m * a.N + n] = f2bf(s);
+    }
+  } else if (MODE == SK_GATED) {
+    const int F = a.N >> 1;
+    for (int i = threadIdx.x; i < a.cols * a.M; i += THREADS) {
+      const int j = i % a.cols, m = i / a.cols, n = blockIdx.x * a.cols + j;
+      if (n >= F) continue;
+      // gate / up rounded to bf16 first: the values an unfused bf16 GEMM output would carry
+      const float g = bf2f(f2bf(sum(j, 0, m))), u = bf2f(f2bf(sum(j, 1, m)));
+      a.Y[(size_t)m * F + n] = f2bf(sk_gate(g, a.act) * u);
+    }
+  } else {
+    const int half = a.D >> 1, per = half / a.cols;
+    const int head = blockIdx.x / per, d0 = (blockIdx.x % per) * a.cols;
+    for (int i = threadIdx.x; i < a.cols * a.M; i += THREADS) {
+      const int j = i % a.cols, m = i / a.cols, d = d0 + j;
+      float lo = sum(j, 0, m), hi = sum(j, 1, m);
+      if (a.bias) {
+        lo += bf2f(a.bias[head * a.D + d]);
+        hi += bf2f(a.bias[head * a.D + d + half]);
+      }
+      lo = bf2f(f2bf(lo));  // the unfused path carries the projection as a bf16 tensor
+      hi = bf2f(f2bf(hi));
+      if (a.do_rope && head < a.Hq + a.Hkv) {
+        int p = a.pos[m];
+        p = p < 0 ? 0 : (p >= a.max_pos ? a.max_pos - 1 : p);
+        const float c = a.cos_t[(size_t)p * half + d], s = a.sin_t[(size_t)p * half + d];
+        const float x = lo;
+        lo = x * c - hi * s;
+        hi = hi * c + x * s;
+      }
+      if (head < a.Hq) {
+        bf16_t* q = a.Y + ((size_t)m * a.Hq + head) * a.D + d;
+        q[0] = f2bf(lo);
+        q[half] = f2bf(hi);
+        continue;
+      }
+      const int64_t slot = a.slots[m];
+      if (slot < 0) continue;
+      const int64_t page = slot / 32;
+      const int off = (int)(slot % 32);
+      if (head < a.Hq + a.Hkv) {
+        const size_t at = (((size_t)page * a.Hkv + head - a.Hq) * 32 + off) * a.D + d;
+        st1_cache(a.kcache, at, bf2f(f2bf(lo)), a.fp8);  // fp8: from the bf16 value, as the other writers
+        st1_cache(a.kcache, at + half, bf2f(f2bf(hi)), a.fp8);
+      } else {
+        const size_t at = (((size_t)page * a.Hkv + head - a.Hq - a.Hkv) * a.D + d) * 32 + off;
+        st1_cache(a.vcache, at, lo, a.fp8);
+        st1_cache(a.vcache, at + (size_t)half * 32, hi, a.fp8);
+      }
+    }
+  }
+}
+
+// One and two rows. MT: rows of X (a.M <= MT); RB: weight rows of a register set; NORM: X is normalised first
+// (K <= WK P 512: one turn)
+template <int MT, int RB, bool NORM, int MODE>
+__global__ __launch_bounds__(THREADS) void skinny_dot_kernel(const SKArgs a) {
+  extern __shared__ __attribute__((aligned(16))) float rf[];  // [WK][rows of the workgroup][MT]
+  __shared__ float sq[WAVES][MT];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wk = wave & (a.wk - 1), wr = wave / a.wk, nwr = WAVES / a.wk;
+  const int pieces = a.K >> 3;                                 // 16-byte pieces of a row
+  const int seg = (pieces + a.wk - 1) / a.wk;                  // of a wave's share
+  const int nrows = MODE == SK_RES ? a.cols : 2 * a.cols;
+
+  // a row of the workgroup -> row of W, or -1
+  auto weight_row = [&](int j) -> int {
+    if (MODE == SK_RES) {
+      const int n = blockIdx.x * a.cols + j;
+      return j < nrows && n < a.N ? n : -1;
+    }
+    const int up = j >= a.cols, i = up ? j - a.cols : j;
+    if (MODE == SK_GATED) {
+      const int F = a.N >> 1, col = blockIdx.x * a.cols + i;
+      return j < nrows && col < F ? col + up * F : -1;
+    }
+    const int half = a.D >> 1, per = half / a.cols;  // workgroups of a head
+    return j < nrows ? (blockIdx.x / per) * a.D + (blockIdx.x % per) * a.cols + i + up * half : -1;
+  };
+
+  for (int s0 = 0; s0 < seg; s0 += 64 * P) {  // one turn unless K is very long
+    int at[P];   // this lane's pieces
+    bool ok[P];
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      const int in = s0 + 64 * p + lane;
+      ok[p] = in < seg && wk * seg + in < pieces;
+      at[p] = (ok[p] ? wk * seg + in : 0) * 8;
+    }
+    bf16x8 xv[MT][P], nv[NORM ? P : 1];
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+      for (int p = 0; p < P; ++p) xv[m][p] = ld8(a.X + (size_t)(m < a.M ? m : 0) * a.xs + at[p]);
+    if (NORM)
+#pragma unroll
+      for (int p = 0; p < P; ++p) nv[p] = ld8(a.nw + at[p]);
+    __builtin_amdgcn_sched_barrier(0);  // ahead of the weights: loads return in order
+
+    bf16x8 wv[2][RB][P];
+    auto load = [&](int set, int first) {
+#pragma unroll
+      for (int i = 0; i < RB; ++i) {
+        const int row = weight_row(wr + nwr * (first + i));  // the same for all lanes
+        if (row >= 0)
+#pragma unroll
+          for (int p = 0; p < P; ++p)
+            wv[set][i][p] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(a.W + (size_t)row * a.K + at[p]));
+      }
+    };
+    load(0, 0);
+    load(1, RB);
+    __builtin_amdgcn_sched_barrier(0);
+
+    // pieces beyond the wave's share count as zeros
+#pragma unroll
+    for (int p = 0; p < P; ++p)
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+        if (!ok[p]) xv[m][p] = bf16x8{};
+    if (NORM) {  // every wave normalises its share for itself; with one wave along K no other is asked
+      float ss[MT], fold[(MT + 3) / 4];
+#pragma unroll
+      for (int m = 0; m < MT; ++m) {
+        ss[m] = 0.f;
+#pragma unroll
+        for (int p = 0; p < P; ++p)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) ss[m] += bf2f(xv[m][p][e]) * bf2f(xv[m][p][e]);
+      }
+      lane_sums<MT>(ss, fold);
+#pragma unroll
+      for (int m = 0; m < MT; ++m) {  // value m sits in the lanes of row {0, 2, 1, 3}[m % 4]
+        constexpr int row_of[4] = {0, 2, 1, 3};
+        ss[m] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(fold[m >> 2]), 16 * row_of[m & 3]));
+      }
+      if (a.wk > 1) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+          if (lane == m) sq[wave][m] = ss[m];
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+          float t = 0.f;
+          for (int w = 0; w < a.wk; ++w) t += sq[wave - wk + w][m];
+          ss[m] = t;
+        }
+      }
+#pragma unroll
+      for (int m = 0; m < MT; ++m) {
+        const float rstd = rsqrtf(ss[m] / (float)a.K + a.eps);
+#pragma unroll
+        for (int p = 0; p < P; ++p)
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            xv[m][p][e] = f2bf(bf2f(xv[m][p][e]) * rstd * (bf2f(nv[p][e]) + (a.gemma ? 1.f : 0.f)));
+      }
+    }
+
+    auto multiply = [&](int set, int first) {
+      float acc[RB * MT], fold[(RB * MT + 3) / 4];
+#pragma unroll
+      for (int i = 0; i < RB; ++i)
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+          acc[i * MT + m] = 0.f;
+#pragma unroll
+          for (int p = 0; p < P; ++p) acc[i * MT + m] = dot8(wv[set][i][p], xv[m][p], acc[i * MT + m]);
+        }
+      lane_sums<RB * MT>(acc, fold);
+      if ((lane & 15) == 0) {
+        const int g = lane >> 4, in4 = g == 1 ? 2 : g == 2 ? 1 : g;  // which of four values this row of lanes holds
+#pragma unroll
+        for (int j = 0; j < (RB * MT + 3) / 4; ++j) {
+          const int v = 4 * j + in4, row = wr + nwr * (first + v / MT);
+          if (v < RB * MT && row < nrows) {
+            float* d = rf + ((size_t)wk * nrows + row) * MT + v % MT;
+            *d = s0 == 0 ? fold[j] : *d + fold[j];
+          }
+        }
+      }
+    };
+    for (int first = 0; wr + nwr * first < nrows; first += 2 * RB) {
+#pragma unroll
+      for (int set = 0; set < 2; ++set) {
+        if (wr + nwr * (first + set * RB) < nrows) {
+          multiply(set, first + set * RB);
+          if (wr + nwr * (first + (set + 2) * RB) < nrows) load(set, first + (set + 2) * RB);
+        }
+      }
+    }
+  }
+  __syncthreads();
+  finish<MODE>(a, [&](int j, int h, int m) {
+    float s = 0.f;
+    for (int w = 0; w < a.wk; ++w) s += rf[((size_t)w * nrows + j + h * a.cols) * MT + m];
+    return s;
+  });
+}
+
+// Three to eight rows, on the matrix cores: CT 16-row weight tiles of a workgroup (SK_GATED: gate tiles, then as many up
+// tiles), U: 64-deep chunks of K a wave has in flight (chunk c belongs to wave c mod 8), PRE: and as many more, in a second
+// set of registers.
+template <int CT, int U, bool PRE, bool NORM, int MODE>
+__global__ __launch_bounds__(THREADS) void skinny_mfma_kernel(const SKArgs a) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  bf16_t* xn = reinterpret_cast<bf16_t*>(smem);  // normalised rows [M][K + 8]
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & 15, kq = lane >> 4;  // operand row (weights: column of Y; activations: row of Y), 8 k's each
+  const int nchunk = a.K >> 6;
+  const int mine = wave < nchunk ? (nchunk - wave + WAVES - 1) / WAVES : 0;
+
+  // wave m normalises row m: its first pieces are loaded ahead of the weights, loads return in order
+  bf16x8 hv[P], gv[P];
+  if (NORM && wave < a.M) {
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      const int c = (lane + 64 * p) * 8;
+      if (c < a.K) {
+        hv[p] = ld8(a.X + (size_t)wave * a.xs + c);
+        gv[p] = ld8(a.nw + c);
+      }
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+
+  const bf16_t* wp[CT];  // this lane's weight rows; lanes without one repeat the workgroup's first: the same cache lines,
+                         // and results that are not stored. Lanes without an activation row likewise
+#pragma unroll
+  for (int ct = 0; ct < CT; ++ct) {
+    int row;
+    if (MODE == SK_GATED) {
+      const int j = 16 * (ct % (CT / 2)) + r, F = a.N >> 1, col = blockIdx.x * a.cols;
+      row = (ct < CT / 2 ? 0 : F) + (j < a.cols && col + j < F ? col + j : col);
+    } else if (MODE == SK_QKV) {
+      const int half = a.D >> 1, per = half / a.cols;  // workgroups of a head
+      row = (blockIdx.x / per) * a.D + (blockIdx.x % per) * a.cols + (r < a.cols ? r : r < 2 * a.cols ? r - a.cols + half : 0);
+    } else {
+      const int j = 16 * ct + r, col = blockIdx.x * a.cols;
+      row = j < a.cols && col + j < a.N ? col + j : col;
+    }
+    wp[ct] = a.W + (size_t)row * a.K + 8 * kq;
+  }
+  const int rm = r < a.M ? r : 0;
+  const bf16_t* xp = a.X + (size_t)rm * a.xs + 8 * kq;
+
+  constexpr int SETS = PRE ? 2 : 1;
+  bf16x8 wf[SETS][U][2][CT], xf[SETS][NORM ? 1 : U][2];
+  auto load = [&](int set, int first) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (first + u < mine) {  // the same for all lanes
+        const int k = (wave + WAVES * (first + u)) * 64;
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+#pragma unroll
+          for (int ct = 0; ct < CT; ++ct) wf[set][u][s][ct] = ld8(wp[ct] + k + 32 * s);
+          if (!NORM) xf[set][NORM ? 0 : u][s] = ld8(xp + k + 32 * s);
+        }
+      }
+    }
+  };
+  load(0, 0);
+  __builtin_amdgcn_sched_barrier(0);
+
+  if (NORM) {
+    if (wave < a.M) {
+      float ss = 0.f;
+      for (int c = lane * 8, p = 0; c < a.K; c += 512, ++p) {
+        const bf16x8 h = p == 0 ? hv[0] : p == 1 ? hv[1] : p == 2 ? hv[2] : ld8(a.X + (size_t)wave * a.xs + c);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) ss += bf2f(h[e]) * bf2f(h[e]);
+      }
+      const float rstd = rsqrtf(wave_sum(ss) / (float)a.K + a.eps);
+      for (int c = lane * 8, p = 0; c < a.K; c += 512, ++p) {
+        const bf16x8 h = p == 0 ? hv[0] : p == 1 ? hv[1] : p == 2 ? hv[2] : ld8(a.X + (size_t)wave * a.xs + c);
+        const bf16x8 g = p == 0 ? gv[0] : p == 1 ? gv[1] : p == 2 ? gv[2] : ld8(a.nw + c);
+        bf16x8 o;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] = f2bf(bf2f(h[e]) * rstd * (bf2f(g[e]) + (a.gemma ? 1.f : 0.f)));
+        st8(xn + (size_t)wave * (a.K + 8) + c, o);
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+  }
+
+  f32x4 acc[CT];
+#pragma unroll
+  for (int ct = 0; ct < CT; ++ct) acc[ct] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto multiply = [&](int set, int first) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (first + u < mine) {
+        const int k = (wave + WAVES * (first + u)) * 64;
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          const bf16x8 b = NORM ? ld8(xn + (size_t)rm * (a.K + 8) + k + 32 * s + 8 * kq) : xf[set][NORM ? 0 : u][s];
+#pragma unroll
+          for (int ct = 0; ct < CT; ++ct)
+            acc[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[set][u][s][ct], b, acc[ct], 0, 0, 0);
+        }
+      }
+    }
+  };
+  for (int first = 0; first < mine; first += SETS * U) {
+#pragma unroll
+    for (int set = 0; set < SETS; ++set) {
+      if (PRE) load(set ^ 1, first + (set + 1) * U);
+      multiply(set, first + set * U);
+      if (!PRE) load(0, first + U);
+    }
+  }
+
+  // the waves' partial sums meet in LDS: [wave][tile][lane] of 4 (weight row 4 kq + i, activation row r)
+  if (NORM) __syncthreads();  // in the place of the normalised rows
+  f32x4* red = reinterpret_cast<f32x4*>(smem);
+#pragma unroll
+  for (int ct = 0; ct < CT; ++ct) red[(wave * CT + ct) * 64 + lane] = acc[ct];
+  __syncthreads();
+  const float* rf = reinterpret_cast<const float*>(red);
+  finish<MODE>(a, [&](int j, int h, int m) {
+    const int row = MODE == SK_QKV ? j + h * a.cols : j & 15;  // of the tile
+    const int ct = MODE == SK_QKV ? 0 : (j >> 4) + h * (CT / 2);
+    const int at = ct * 256 + ((row >> 2) * 16 + m) * 4 + (row & 3);
+    float s = 0.f;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) s += rf[w * CT * 256 + at];
+    return s;
+  });
+}
+
+template <int MT, int RB, bool NORM, int MODE>
+int sk_dot(SKArgs& a, int blocks, hipStream_t st) {
+  a.wk = 1;
+  while (a.wk < WAVES && a.K > a.wk * P * 512) a.wk *= 2;
+  if (NORM && a.K > a.wk * P * 512) return -4;
+  const size_t lds = (size_t)a.wk * (MODE == SK_RES ? a.cols : 2 * a.cols) * MT * sizeof(float);
+  hipLaunchKernelGGL((skinny_dot_kernel<MT, RB, NORM, MODE>), dim3(blocks), dim3(THREADS), lds, st, a);
+  return (int)hipGetLastError();
+}
+
+template <int CT, int U, bool PRE, bool NORM, int MODE>
+int sk_mfma(const SKArgs& a, int blocks, hipStream_t st) {
+  const size_t sums = (size_t)WAVES * CT * 1024, rows = NORM ? (size_t)a.M * (a.K + 8) * sizeof(bf16_t) : 0;
+  const size_t lds = sums > rows ? sums : rows;
+  if (lds > 160 * 1024) return -4;
+  if (lds > 64 * 1024)
+    HIP_RET(hipFuncSetAttribute((const void*)skinny_mfma_kernel<CT, U, PRE, NORM, MODE>,
+                                hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+  hipLaunchKernelGGL((skinny_mfma_kernel<CT, U, PRE, NORM, MODE>), dim3(blocks), dim3(THREADS), lds, st, a);
+  return (int)hipGetLastError();
+}
+
+int sk_check(const void* X, int64_t xs, const void* W, int M, int N, int K) {
+  if (M < 1 || M > 8 || K < 64 || K % 64 != 0 || xs % 8 != 0 || N < 1) return -1;
+  if (((uintptr_t)X | (uintptr_t)W) % 16 != 0) return -2;
+  return 0;
+}
+
+constexpr int CUS = 256;
+
+}  // namespace
+
+// Y [M, N] = bf16(X W^T) + residual (may be null), rounded again. M <= 8, K % 64 == 0.
+extern "C" int areal_skinny_residual(const void* X, int64_t xs, const void* W, const void* res, void* Y, int M, int N, int K,
+                                     hipStream_t st) {
+  if (int rc = sk_check(X, xs, W, M, N, K)) return rc;
+  SKArgs a = {};
+  a.X = (const bf16_t*)X; a.xs = xs; a.W = (const bf16_t*)W; a.res = (const bf16_t*)res; a.Y = (bf16_t*)Y;
+  a.M = M; a.N = N; a.K = K;
+  a.cols = (N + CUS - 1) / CUS < 16 ? (N + CUS - 1) / CUS : 16;
+  const int blocks = (N + a.cols - 1) / a.cols;
+  if (M == 1) return sk_dot<1, 3, false, SK_RES>(a, blocks, st);
+  if (M == 2) return sk_dot<2, 3, false, SK_RES>(a, blocks, st);
+  if (K <= 64 * WAVES * 6) return sk_mfma<1, 6, false, false, SK_RES>(a, blocks, st);
+  return sk_mfma<1, 6, true, false, SK_RES>(a, blocks, st);
+}
+
+// Y [M, F] = gate(h W_gate^T) * (h W_up^T), h = RMSNorm(X) nw, W = [gate; up] [2F, K]. K <= 8192.
+extern "C" int areal_skinny_norm_gated(const void* X, int64_t xs, const void* nw, const void* W, void* Y, int M, int F, int K,
+                                       float eps, int gemma, int act, hipStream_t st) {
+  if (int rc = sk_check(X, xs, W, M, F, K)) return rc;
+  if ((uintptr_t)nw % 16 != 0) return -3;
+  SKArgs a = {};
+  a.X = (const bf16_t*)X; a.xs = xs; a.nw = (const bf16_t*)nw; a.W = (const bf16_t*)W; a.Y = (bf16_t*)Y;
+  a.M = M; a.N = 2 * F; a.K = K; a.eps = eps; a.gemma = gemma; a.act = act;
+  int rounds = 1;
+  while ((F + CUS * rounds - 1) / (CUS * rounds) > 48) ++rounds;
+  a.cols = (F + CUS * rounds - 1) / (CUS * rounds);
+  const int blocks = (F + a.cols - 1) / a.cols;
+  if (M == 1) return sk_dot<1, 5, true, SK_GATED>(a, blocks, st);
+  if (M == 2) return sk_dot<2, 5, true, SK_GATED>(a, blocks, st);
+  if (a.cols <= 16) return sk_mfma<2, 3, true, true, SK_GATED>(a, blocks, st);
+  if (a.cols <= 32) return sk_mfma<4, 3, false, true, SK_GATED>(a, blocks, st);
+  return sk_mfma<6, 3, false, true, SK_GATED>(a, blocks, st);
+}
+
+// The packed q|k|v projection of RMSNorm(X) nw with bias, rotation and KV-cache write; returns the rotated q in Y
+// [M, Hq, D]. D a multiple of 16, K <= 8192.
+extern "C" int areal_skinny_norm_qkv(const void* X, int64_t xs, const void* nw, const void* W, const void* bias,
+                                     const int* pos, const int64_t* slots, const float* cos_t, const float* sin_t, void* Y,
+                                     void* kcache, void* vcache, int M, int K, int Hq, int Hkv, int D, int max_pos,
+                                     int do_rope, float eps, int gemma, int fp8, hipStream_t st) {
+  const int N = (Hq + 2 * Hkv) * D;
+  if (int rc = sk_check(X, xs, W, M, N, K)) return rc;
+  if (D % 16 != 0 || (uintptr_t)nw % 16 != 0) return -3;
+  SKArgs a = {};
+  a.X = (const bf16_t*)X; a.xs = xs; a.nw = (const bf16_t*)nw; a.W = (const bf16_t*)W; a.bias = (const bf16_t*)bias;
+  a.Y = (bf16_t*)Y; a.M = M; a.N = N; a.K = K; a.eps = eps; a.gemma = gemma; a.pos = pos; a.slots = slots; a.cos_t = cos_t;
+  a.sin_t = sin_t; a.kcache = kcache; a.vcache = vcache; a.Hq = Hq; a.Hkv = Hkv; a.D = D; a.max_pos = max_pos;
+  a.do_rope = do_rope; a.fp8 = fp8;
+  a.cols = N / 8 <= CUS ? 4 : 8;  // rotated pairs of a workgroup
+  const int blocks = N / (2 * a.cols);
+  if (M == 1) return sk_dot<1, 1, true, SK_QKV>(a, blocks, st);
+  if (M == 2) return sk_dot<2, 1, true, SK_QKV>(a, blocks, st);
+  return sk_mfma<1, 3, true, true, SK_QKV>(a, blocks, st);
+}
