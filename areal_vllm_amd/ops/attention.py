@@ -127,7 +127,7 @@ class _FlashVarlenFn(torch.autograd.Function):
         dk = dqkv[:, Hq:Hq + Hkv]
         dv = dqkv[:, Hq + Hkv:]
         if L.use_hip(qkv):
-            _flash_bwd_hip(q, k, v, out, dout, lse, dq, dk, dv, cu, cu, max_seqlen, scale, causal)
+            _flash_bwd_hip(q, k, v, out, dout, lse, dq, dk, dv, cu, cu, max_seqlen, max_seqlen, scale, causal)
         else:
             with torch.enable_grad():
                 q_ = q.detach().float().requires_grad_(True)
@@ -180,21 +180,34 @@ def _flash_fwd_hip(q, k, v, cu_q, cu_k, max_q, scale, causal) -> Tuple[torch.Ten
     return out, lse
 
 
-def _flash_bwd_hip(q, k, v, out, dout, lse, dq, dk, dv, cu_q, cu_k, max_k, scale, causal):
+def flash_bwd_parts(total_k: int, max_k: int, n_q_heads: int, n_kv_heads: int) -> int:
+    """Workgroups that share a block of 128 keys in the dK / dV kernel, each taking some of the key head's G query heads. 512
+    workgroups run at once; under a causal mask a key block's work is half the longest one's on average, so the longest
+    workgroup (all slices of its heads) should be no more than about 0.8 of what a slot gets; 0.6 for long sequences, whose
+    partial sums cost little beside the work. Measured with 1 / 2 / 3 / 6 parts (backward): 24576 tokens, G = 6, 2 key heads:
+    11.2 / 7.2 / 6.4 / 6.2 ms; 25 x 1133: 717 / 621 / 644 / 715 us; 3 x 8192, G = 7, 4 key heads: 5.9 / 5.9 / 5.1 / 6.0 ms;
+    16 x 200-1216, G = 8, 4 key heads: 837 / 704 / 670 / 745 us."""
+    g = n_q_heads // n_kv_heads
+    blocks = -(-total_k // 128) * n_kv_heads
+    return -(-g // max(1, min(g, int((0.8 if max_k <= 2048 else 0.6) * blocks * g / 1024))))
+
+
+def _flash_bwd_hip(q, k, v, out, dout, lse, dq, dk, dv, cu_q, cu_k, max_q, max_k, scale, causal):
     Tq, Hq, D = q.shape
     Hkv = k.shape[1]
     B = cu_q.numel() - 1
-    delta = torch.empty(Hq, Tq, dtype=torch.float32, device=q.device)
-    # the fp32 accumulator of the atomic dQ path; long sequences compute dQ in a kernel of its own and need none
-    split = D == 256 or bool(L.lib().areal_flash_bwd_split(L.c_int(int(max_k))))  # head size 256: always two kernels
-    dq_acc = None if split else torch.zeros(Tq, Hq, D, dtype=torch.float32, device=q.device)
+    if dout.data_ptr() % 16 != 0:  # tiles are staged 16 bytes at a time
+        dout = dout.clone()
+    delta = torch.empty(2, Hq, Tq, dtype=torch.float32, device=q.device)  # row sums of dO * O, log-sum-exp in base 2
+    Tk = k.shape[0]
+    parts = flash_bwd_parts(Tk, int(max_k), Hq, Hkv) if D == 128 else 1
+    part = torch.empty(parts, 2, Tk, Hkv, D, dtype=torch.float32, device=q.device) if parts > 1 else None
     L.check(
         L.lib().areal_flash_bwd(
             L.ptr(q), L.ptr(k), L.ptr(v), L.ptr(out), L.ptr(dout), L.ptr(lse), L.ptr(delta),
-            L.ptr(dq_acc) if dq_acc is not None else None,
-            L.ptr(dq), L.ptr(dk), L.ptr(dv), L.ptr(cu_q), L.ptr(cu_k), L.c_int(B), L.c_int(int(max_k)),
-            L.c_int(Tq), L.c_int(Hq), L.c_int(Hkv), L.c_int(D), L.c_int64(_strides(q)), L.c_int64(_strides(k)),
-            L.c_int64(_strides(v)), L.c_int64(_strides(out)), L.c_int64(_strides(dout)), L.c_int64(_strides(dq)),
+            L.ptr(dq), L.ptr(dk), L.ptr(dv), L.ptr(part), L.c_int(parts), L.ptr(cu_q), L.ptr(cu_k), L.c_int(B),
+            L.c_int(int(max_q)), L.c_int(int(max_k)), L.c_int(Tq), L.c_int64(Tk), L.c_int(Hq), L.c_int(Hkv), L.c_int(D),
+            L.c_int64(_strides(q)), L.c_int64(_strides(k)), L.c_int64(_strides(v)), L.c_int64(_strides(out)), L.c_int64(_strides(dout)), L.c_int64(_strides(dq)),
             L.c_int64(_strides(dk)), L.c_int64(_strides(dv)), L.c_float(scale), L.c_int(int(causal)),
             L.stream_ptr(),
         ),
@@ -214,19 +227,19 @@ class _FlashVarlenSepFn(torch.autograd.Function):
         else:
             out, lse = attention_varlen_ref(q, k, v, cu_q, cu_k, scale, causal)
         ctx.save_for_backward(q, k, v, out, lse, cu_q, cu_k)
-        ctx.meta = (max_k, scale, causal)
+        ctx.meta = (max_q, max_k, scale, causal)
         return out
 
     @staticmethod
     def backward(ctx, dout):
         q, k, v, out, lse, cu_q, cu_k = ctx.saved_tensors
-        max_k, scale, causal = ctx.meta
+        max_q, max_k, scale, causal = ctx.meta
         dout = dout.contiguous()
         if L.use_hip(q):
             dq = torch.empty(q.shape, dtype=q.dtype, device=q.device)
             dk = torch.zeros(k.shape, dtype=k.dtype, device=k.device)  # keys outside every range get 0
             dv = torch.zeros(v.shape, dtype=v.dtype, device=v.device)
-            _flash_bwd_hip(q, k, v, out, dout, lse, dq, dk, dv, cu_q, cu_k, max_k, scale, causal)
+            _flash_bwd_hip(q, k, v, out, dout, lse, dq, dk, dv, cu_q, cu_k, max_q, max_k, scale, causal)
         else:
             with torch.enable_grad():
                 q_ = q.detach().float().requires_grad_(True)

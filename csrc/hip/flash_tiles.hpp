@@ -43,3 +43,84 @@ DEVINL bf16x8 lds_row_read(const char* tile, int row, int ch) {
 DEVINL void lds_row_write(char* tile, int row, int ch, bf16x8 v) {
   *reinterpret_cast<bf16x8*>(tile + swz_off(row, ch)) = v;
 }
+
+// ---- staging of 64-row tiles by LDS-DMA. One wave instruction (16 bytes a lane) fills four consecutive 256-byte rows of a
+// tile linearly; the swizzle sits on the source address: lane -> row (lane >> 4) of the four, physical chunk lane & 15.
+typedef const __attribute__((address_space(1))) void* dma_gptr_t;
+typedef __attribute__((address_space(3))) void* dma_lptr_t;
+DEVINL void dma16(const void* src, void* lds) {
+  __builtin_amdgcn_global_load_lds((dma_gptr_t)src, (dma_lptr_t)lds, 16, 0, 0);
+}
+// Rows 16 w + 4 i + (lane >> 4), i = 0..3, of a tile of 64 rows go through wave w of four. `off`: this lane's byte offsets of
+// the four pieces for rows `stride` elements apart.
+DEVINL void dma_offsets(unsigned (&off)[4], int wave, int lane, int64_t stride) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int row = 16 * wave + 4 * i + (lane >> 4), chunk = (lane & 15) ^ (((lane >> 4) << 2) | i);
+    off[i] = (unsigned)(row * stride + chunk * 8) * 2;
+  }
+}
+// base: row 0 of the tile (uniform); rows from `rows` on repeat row rows - 1. The base is kept in scalar registers (the
+// compiler would otherwise carry one 64-bit pointer a piece and lane through the loop).
+DEVINL void dma_tile(const bf16_t* base, const unsigned (&off)[4], int64_t stride, int rows, char* tile, int wave, int lane) {
+  char* dst = tile + wave * 4096;
+  const char* b = reinterpret_cast<const char*>(base);
+  asm volatile("" : "+s"(b));
+  if (rows >= 64) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) dma16(b + off[i], dst + i * 1024);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int row = 16 * wave + 4 * i + (lane >> 4), over = row < rows ? 0 : row - (rows - 1);
+      // (same chunk order as row `row` would have: the swizzle belongs to the place in the tile)
+      dma16(b + (off[i] - (unsigned)(over * stride) * 2), dst + i * 1024);
+    }
+  }
+}
+// every DMA of this wave has landed; then all waves have said so (and have finished reading the other buffer)
+DEVINL void dma_arrive() {
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// 32-row tiles, two pieces of each wave of four: rows 8 w + 4 i + (lane >> 4), i = 0, 1
+DEVINL void dma_offsets32(unsigned (&off)[2], int wave, int lane, int64_t stride) {
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int row = 8 * wave + 4 * i + (lane >> 4), chunk = (lane & 15) ^ (((lane >> 4) << 2) | ((2 * wave + i) & 3));
+    off[i] = (unsigned)(row * stride + chunk * 8) * 2;
+  }
+}
+DEVINL void dma_tile32(const bf16_t* base, const unsigned (&off)[2], int64_t stride, int rows, char* tile, int wave, int lane) {
+  char* dst = tile + wave * 2048;
+  const char* b = reinterpret_cast<const char*>(base);
+  asm volatile("" : "+s"(b));
+  if (rows >= 32) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) dma16(b + off[i], dst + i * 1024);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int row = 8 * wave + 4 * i + (lane >> 4), over = row < rows ? 0 : row - (rows - 1);
+      dma16(b + (off[i] - (unsigned)(over * stride) * 2), dst + i * 1024);
+    }
+  }
+}
+
+// Byte offsets inside a tile of this lane's fragment reads. row(s): row r = lane & 31 of a 32-row block, chunk 2 s + hf (add
+// 8192 per block); tr0(db), tr1(db): rows 4 hf + .. (second: + 8), 16-column block 2 db + (grp & 1), transposed (add 4096 per
+// 16 rows). The chunk's bits of s and db do not meet the swizzle's carry: one register each and an exclusive or.
+struct FragOffsets {
+  int r0, t0, t1;
+  DEVINL FragOffsets(int lane) {
+    const int hf = lane >> 5, gl = lane & 15, grp = lane >> 4, ch = 2 * (grp & 1) + ((gl & 3) >> 1);
+    r0 = swz_off(lane & 31, hf);
+    t0 = swz_off(4 * hf + (gl >> 2), ch) + 8 * (gl & 1);
+    t1 = swz_off(8 + 4 * hf + (gl >> 2), ch) + 8 * (gl & 1);
+  }
+  DEVINL int row(int s) const { return r0 ^ (s << 5); }
+  DEVINL int tr0(int db) const { return t0 ^ (db << 6); }
+  DEVINL int tr1(int db) const { return t1 ^ (db << 6); }
+};

@@ -1,0 +1,77 @@
+"""Flash attention forward and backward at the edges of their tiles, with the dK / dV work of a key block shared by several
+workgroups, under scales of either sign and rows that see no key."""
+import math
+
+import numpy as np
+import pytest
+import torch
+
+from areal_vllm_amd import ops
+from areal_vllm_amd.ops import attention as A
+
+DEV = "cuda:0"
+pytestmark = pytest.mark.gpu
+
+
+def _ref(q, k, v, lq, lk, scale, causal):
+    """fp64 attention [Tq, Hq, D]; rows without a key give zero."""
+    g, outs, a, b = q.shape[1] // k.shape[1], [], 0, 0
+    for m, n in zip(lq, lk):
+        qq, kk, vv = (x.transpose(0, 1) for x in (q[a:a + m], k[b:b + n].repeat_interleave(g, 1), v[b:b + n].repeat_interleave(g, 1)))
+        s = torch.matmul(qq, kk.transpose(1, 2)) * scale
+        if causal:
+            i, j = torch.arange(m, device=q.device)[:, None], torch.arange(n, device=q.device)[None, :]
+            s = s.masked_fill(j > i + n - m, -math.inf)
+        p = torch.nan_to_num(torch.softmax(s, -1), nan=0.0)
+        outs.append(torch.matmul(p, vv).transpose(0, 1))
+        a, b = a + m, b + n
+    return torch.cat(outs)
+
+
+@pytest.mark.parametrize("Hq,Hkv", [(6, 1), (14, 2), (3, 3)])
+@pytest.mark.parametrize("lq,lk", [([1], [1]), ([31, 32, 33], None), ([127, 128, 129], None), ([64, 63, 65, 300], None),
+                                   ([5, 130], [700, 131]), ([200, 1, 0], [40, 64, 3]), ([1500], None)])
+@pytest.mark.parametrize("scale,causal", [(None, True), (None, False), (-0.11, True)])
+def test_forward_and_gradients(Hq, Hkv, lq, lk, scale, causal):
+    lk = lk or lq
+    g = torch.Generator(device=DEV).manual_seed(sum(lq) + Hq)
+    q, k, v = (torch.randn(sum(l), h, 128, device=DEV, generator=g).bfloat16().requires_grad_() for l, h in
+               ((lq, Hq), (lk, Hkv), (lk, Hkv)))
+    cu = [torch.tensor([0] + np.cumsum(l).tolist(), dtype=torch.int32, device=DEV) for l in (lq, lk)]
+    assert A.flash_bwd_parts(sum(lk), max(lk), Hq, Hkv) == Hq // Hkv  # every query head a workgroup of its own
+    out = ops.flash_attn_varlen_sep(q, k, v, *cu, max(lq), max(lk), scale, causal)
+    d = torch.randn(out.shape, device=DEV, generator=g).bfloat16()
+    grads = torch.autograd.grad(out, (q, k, v), d, retain_graph=True)
+    again = torch.autograd.grad(out, (q, k, v), d)
+    assert all(torch.equal(x, y) for x, y in zip(grads, again))  # no sum depends on the order of arrival
+    r = [x.detach().double().requires_grad_() for x in (q, k, v)]
+    want = _ref(*r, lq, lk, scale or 128 ** -0.5, causal)
+    refs = torch.autograd.grad(want, r, d.double())
+    out, want = out.detach(), want.detach()
+    # P, dS, O and the gradients pass through bf16 once (2^-9 each, relative to a row's largest value)
+    for x, y in zip((out, *grads), (want, *refs)):
+        assert float((x.double() - y).abs().max()) <= 2e-2 * max(1.0, float(y.abs().max())), (x.shape, float(y.abs().max()))
+        # (a row with one key: dP - delta is the difference of two fp32 sums below 64 in size, 1e-5, where zero is exact)
+        assert float((x.double() - y).norm()) <= 8e-3 * float(y.norm()) + 1e-5 * x.numel() ** 0.5
+
+
+def test_parts_cover_the_heads():
+    for g in range(1, 17):
+        for tk in (1, 700, 5000, 24576, 200000):
+            for mk in (min(tk, 1000), tk):
+                p = A.flash_bwd_parts(tk, mk, 2 * g, 2)
+                assert 1 <= p <= g
+
+
+def test_scores_that_keep_growing_are_rescaled():
+    """Keys whose scores grow by a little per tile stay below the rescaling threshold, then pass it."""
+    T = 1024
+    q = torch.ones(T, 2, 128, device=DEV).bfloat16()
+    k = (torch.arange(T, device=DEV)[:, None, None] * 2e-3 * torch.ones(T, 1, 128, device=DEV)).bfloat16()
+    v = torch.randn(T, 1, 128, device=DEV).bfloat16()
+    cu = torch.tensor([0, T], dtype=torch.int32, device=DEV)
+    for scale in (0.02, 1.0, 0.0):
+        out, lse = ops.flash_attn_varlen(q, k, v, cu, cu, T, scale=scale)
+        ref, ref_lse = A.attention_varlen_ref(q.double(), k.double(), v.double(), cu, cu, scale)
+        assert float((out.float() - ref).abs().max()) < 2e-2
+        assert float((lse - ref_lse).abs().max()) < 2e-3 * max(1.0, float(ref_lse.abs().max()))
