@@ -64,16 +64,12 @@ def wgrad_supported(dy: torch.Tensor, x: torch.Tensor, acc: torch.Tensor) -> boo
 
 def tgemm_wgrad_(acc: torch.Tensor, dy: torch.Tensor, x: torch.Tensor, splits: int = 0, stagger: bool = True) -> torch.Tensor:
     """acc[N, K] (fp32) += dy[M, N]^T @ x[M, K]: the weight gradient of ``y = x @ W^T`` summed straight into the
-    fp32 gradient buffer. The kernel reduces whole pairs of 64-token tiles; the last M % 128 tokens are added by a
-    library GEMM on those few rows."""
+    fp32 gradient buffer."""
     assert wgrad_supported(dy, x, acc)
-    M = dy.shape[0]
-    main = M - M % 128
     L.check(L.lib().areal_tgemm_wgrad(L.ptr(dy), L.c_int64(dy.stride(0)), L.ptr(x), L.c_int64(x.stride(0)), L.ptr(acc),
-                                      L.c_int64(acc.stride(0)), L.c_int(main), L.c_int(dy.shape[1]), L.c_int(x.shape[1]),
-                                      L.c_int(int(splits)), L.c_int(int(stagger)), L.stream_ptr()), "tgemm_wgrad")
-    if main < M:
-        torch.addmm(acc, dy[main:].t(), x[main:], out_dtype=torch.float32, out=acc)
+                                      L.c_int64(acc.stride(0)), L.c_int(dy.shape[0]), L.c_int(dy.shape[1]),
+                                      L.c_int(x.shape[1]), L.c_int(int(splits)), L.c_int(int(stagger)), L.stream_ptr()),
+            "tgemm_wgrad")
     return acc
 
 

@@ -367,7 +367,7 @@ struct TWArgs {
   long ldw;
   int M, N, K;
   int tiles_n, tiles_k;
-  int pairs;          // 128-token pairs of K tiles in M
+  int pairs;          // 128-token pairs of K tiles in M, the last one possibly ragged
   int whole;          // the first `whole` tiles are reduced by one workgroup each
   int splits, chunk;  // the others: workgroups per tile, pairs per workgroup (the last one of a tile may get fewer)
 };
@@ -410,14 +410,22 @@ __global__ __launch_bounds__(512) void tgemm_wgrad_kernel(const TWArgs a) {
   // ---- staging: thread -> token row (wave * 4 + lane / 16) of a 32-row issue, physical 16-byte chunk lane & 15
   const int srow = wave * 4 + (lane >> 4);
   const int pc = ((lane & 15) ^ (((lane >> 4) << 2) | (wave & 3))) * 8;  // piece column whose chunk lands here
-  const bf16_t *pA = nullptr, *pB = nullptr;  // set per segment
+  // Rows past the last token are out of the buffer's range: such loads write zeros. One descriptor per piece and K tile
+  // (scalar registers), of no more than 64 rows: byte offsets stay small however large the operand is.
+  const bf16_t *pA = nullptr, *pB = nullptr;  // the segment's first token, column n0 / k0
+  unsigned vA = 0, vB = 0;                    // this lane's byte offset of a piece's first row and column
+  int tokens = 0;                             // of the segment
   auto stage = [&](int buf, int piece, int kt) __attribute__((always_inline)) {
     char* dst = smem + buf * TG_BUF + piece * TG_PIECE + wave * 1024;
     const bool isA = piece < 2;
-    const long ld = isA ? a.ldy : a.ldx;
-    const bf16_t* s0 = (isA ? pA + (piece & 1) * 64 : pB + (piece & 1) * 32) + (size_t)kt * 64 * ld;
-    __builtin_amdgcn_global_load_lds((gptr_t)s0, (lptr_t)dst, 16, 0, 0);
-    __builtin_amdgcn_global_load_lds((gptr_t)(s0 + 32 * ld), (lptr_t)(dst + 8192), 16, 0, 0);
+    const unsigned row = (unsigned)(isA ? a.ldy : a.ldx) * 2;  // bytes
+    const int rows = min(tokens - kt * 64, 64);
+    const unsigned range = rows > 0 ? (rows - 1) * row + min(row, 512u) : 0u;
+    const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>((isA ? pA : pB) + (size_t)kt * 32 * row), 0, range, 0x00020000);
+    // the whole offset in the vector operand, the one that the range check is about
+    const unsigned v = (isA ? vA : vB) + (piece & 1) * (isA ? 128 : 64);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lptr_t)dst, 16, v, 0, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lptr_t)(dst + 8192), 16, v + 32 * row, 0, 0, 0);
   };
 
   // ---- transposed fragment reads: addresses inside a piece (the same for both buffers and every 16-token slab)
@@ -523,11 +531,14 @@ __global__ __launch_bounds__(512) void tgemm_wgrad_kernel(const TWArgs a) {
     tile_origin(tile_id, n0, k0);
     whole = p0 == 0 && p1 == a.pairs;
     const int tok0 = p0 * 128, KT = (p1 - p0) * 2;
+    tokens = a.M - tok0;
     // N may end half way through the last tile row (N % 256 == 128): the second wave row then re-reads the first
     // one's columns and does not write
     const bool half_n = n0 + 128 >= a.N;
-    pA = a.dY + (size_t)(tok0 + srow) * a.ldy + n0 + (half_n ? 0 : (pc >> 6) * 128) + (pc & 63);
-    pB = a.X + (size_t)(tok0 + srow) * a.ldx + k0 + (pc >> 5) * 64 + (pc & 31);
+    pA = a.dY + (size_t)tok0 * a.ldy + n0;
+    pB = a.X + (size_t)tok0 * a.ldx + k0;
+    vA = (unsigned)(srow * a.ldy + (half_n ? 0 : (pc >> 6) * 128) + (pc & 63)) * 2;
+    vB = (unsigned)(srow * a.ldx + (pc >> 5) * 64 + (pc & 31)) * 2;
 #pragma unroll
     for (int mi = 0; mi < 2; ++mi)
 #pragma unroll
@@ -612,14 +623,16 @@ extern "C" int areal_tgemm_swiglu(const void* A, long lda, const void* W, long l
   return tgemm_tn_launch(A, lda, W, ldw, C, ldc, nullptr, M, F, K, 1, max_blocks, 1, st);
 }
 
-// dW[N, K] (fp32, leading dimension ldw) += dY[M, N]^T . X[M, K]. N a multiple of 128, K of 256, M a multiple of 128 (the
-// caller adds the last M % 128 tokens with a library GEMM), rows 16-byte aligned. splits: 0 = stream-K.
+// dW[N, K] (fp32, leading dimension ldw) += dY[M, N]^T . X[M, K]. N a multiple of 128, K of 256, rows 16-byte aligned.
+// splits: 0 = chosen. A ragged last 128-token pair is filled up with zeros: handing its few tokens to a library GEMM
+// instead reads and writes the whole fp32 gradient a second time (60 tokens: 51 us for 17920 x 1536, 507 us for the
+// 151936 x 1536 LM head, 1.4 of the 9.2 ms of a pass over 700 tokens and 7 layers).
 extern "C" int areal_tgemm_wgrad(const void* dY, long ldy, const void* X, long ldx, float* dW, long ldw, int M, int N,
                                  int K, int splits, int stagger, hipStream_t st) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
-  if (M % 128 != 0 || N % 128 != 0 || K % 256 != 0 || ldy % 8 != 0 || ldx % 8 != 0) return -1;
+  if (N % 128 != 0 || K % 256 != 0 || ldy % 8 != 0 || ldx % 8 != 0) return -1;
   if (((uintptr_t)dY | (uintptr_t)X) % 16 != 0 || (uintptr_t)dW % 4 != 0) return -1;
-  const int tiles = ((N + 255) / 256) * (K / 256), pairs = M / 128;
+  const int tiles = ((N + 255) / 256) * (K / 256), pairs = (M + 127) / 128;
   // splits >= 1: that many workgroups per tile (1 = every tile added without atomics). splits <= 0: choose. Blocks run
   // in rounds of 256 (one per CU); a block costs its share of the pairs (~3.1 us each) plus ~8 us of prologue and
   // flush, ~25 us more when the tile is flushed with atomic adds (a CU retires one 256-byte atomic instruction per
