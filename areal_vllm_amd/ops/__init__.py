@@ -24,7 +24,7 @@ from .logprob import (  # noqa: F401
     vocab_shard_range,
 )
 from .norm_act import RotaryTable, apply_rope, qk_norm, rmsnorm, rope_inplace_, swiglu  # noqa: F401
-from .optim import adam_prepare_, adamw_, scale_, sumsq_  # noqa: F401
+from .optim import adam_prepare_, adamw_, fold_grad_, scale_, sumsq_  # noqa: F401
 from .rl import gae_1d_packed, gae_2d, gae_padded, merge_intervals, set_intervals, slice_intervals  # noqa: F401
 from .sampling import TokenCounts, advance_step_, decode_advance_, decode_begin_, sample  # noqa: F401
 from . import train_gemm  # noqa: F401

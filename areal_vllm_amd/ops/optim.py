@@ -23,6 +23,16 @@ def sumsq_(x: torch.Tensor, out: torch.Tensor) -> None:
         out[0] += x.float().pow(2).sum()
 
 
+def fold_grad_(acc: torch.Tensor, grad: torch.Tensor) -> None:
+    """acc += grad (fp32 buffer, gradient of any type)."""
+    if (L.use_hip(acc) and acc.dtype == torch.float32 and grad.dtype == torch.bfloat16 and grad.is_cuda
+            and acc.shape == grad.shape and acc.is_contiguous() and grad.is_contiguous()
+            and acc.data_ptr() % 16 == 0 and grad.data_ptr() % 16 == 0):
+        L.check(L.lib().areal_fold_grad(L.ptr(acc), L.ptr(grad), L.c_int64(acc.numel()), L.stream_ptr()), "fold_grad")
+    else:
+        acc.add_(grad)
+
+
 def scale_(x: torch.Tensor, scale: float, scale_tensor: torch.Tensor = None) -> None:
     if L.use_hip(x):
         L.check(L.lib().areal_scale(L.ptr(x), L.c_int(L.dtype_flag(x)), L.c_int64(x.numel()), L.ptr(scale_tensor),

@@ -66,6 +66,35 @@ __global__ __launch_bounds__(256) void scale_kernel(T* __restrict__ x, int64_t n
   }
 }
 
+// acc (fp32) += g (bf16): gradients of small parameters (norms, biases, routers) into the main-gradient buffer. The
+// framework's own mixed-type addition takes 42 us for 1536 elements (one workgroup of a general element-wise kernel), this
+// 2-3: 22 of them were 0.9 of the 9.2 ms of a training pass over 700 tokens and 7 layers.
+__global__ __launch_bounds__(256) void fold_grad_kernel(float* __restrict__ acc, const bf16_t* __restrict__ g, int64_t n) {
+  for (int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 8; i < n; i += (int64_t)gridDim.x * 256 * 8) {
+    if (i + 8 <= n) {
+      const bf16x8 x = ld8(g + i);
+      f32x4* a = reinterpret_cast<f32x4*>(acc + i);
+      f32x4 lo = a[0], hi = a[1];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) { lo[j] += bf2f(x[j]); hi[j] += bf2f(x[j + 4]); }
+      a[0] = lo;
+      a[1] = hi;
+    } else {
+      for (int64_t k = i; k < n; ++k) acc[k] += bf2f(g[k]);
+    }
+  }
+}
+
+// both contiguous and 16-byte aligned
+extern "C" int areal_fold_grad(float* acc, const void* g, int64_t n, hipStream_t st) {
+  if (n <= 0) return 0;
+  if (((uintptr_t)acc | (uintptr_t)g) % 16 != 0) return -1;
+  const int64_t blocks = (n + 2047) / 2048;
+  hipLaunchKernelGGL(fold_grad_kernel, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256), 0, st, acc,
+                     (const bf16_t*)g, n);
+  return (int)hipGetLastError();
+}
+
 extern "C" int areal_sumsq(const void* x, int dtype, int64_t n, float* out, hipStream_t st) {
   if (n == 0) return 0;
   if (((uintptr_t)x) % 16 != 0) return -1;
