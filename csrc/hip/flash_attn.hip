@@ -394,6 +394,7 @@ __global__ __launch_bounds__(256, 2) void flash_bwd_dq_kernel(
         dsf[j >> 3][j & 7] = f2bf(pr * (pacc[j] - dlt));
       }
       // ---- dQ^T[d, q] += K^T[d, keys] . dS^T[keys, q]
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int s = 0; s < 2; ++s) {
         bf16x4 a0[4], a1[4];
@@ -576,7 +577,9 @@ __global__ __launch_bounds__(256, 2) void flash_bwd_dkv_kernel(
         dsfr[reg >> 3][reg & 7] = f2bf(p * (pacc[reg] - d4[j]));
       }
     }
-    // ---- dV^T += dO^T.P ; dK^T += Q^T.dS   (A operand from transposed reads)
+    // ---- dV^T += dO^T.P ; dK^T += Q^T.dS   (A operand from transposed reads, which the compiler lets wait for the next
+    // slice's DMA: not before this point)
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
 #pragma unroll
