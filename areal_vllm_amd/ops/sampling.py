@@ -1,6 +1,6 @@
 """Fused temperature / top-k / top-p sampling returning (token, logprob).
 
-GPU: ``csrc/hip/sampling.hip`` (Gumbel-max, bisection thresholds, Philox keyed by a device-resident
+GPU: ``csrc/hip/sampling.hip`` (Gumbel-max, histogram thresholds, Philox keyed by a device-resident
 step counter so captured graphs draw fresh noise on replay). CPU: PyTorch reference.
 Counterparts: ``realhf/impl/model/utils/logits_warper.py:52-125,207-225`` and ``genstep`` in
 ``realhf/impl/model/nn/real_llm_generate.py:30-146``.

@@ -9,10 +9,8 @@
 //  * unfiltered (top_k >= V and top_p >= 1): Gumbel-max over z = logit / T, in the same single pass
 //    over the row (16-byte loads) that accumulates the running max / sum-exp for the log-prob.
 //  * filtered: thresholds for top-k (k-th largest z) and top-p (smallest set whose mass
-//    reaches top_p of the top-k mass) are found by bisection on z - over the whole row only until
-//    the bracket holds a few thousand entries, then among those entries in LDS (fixed-point sums:
-//    order-independent) -, then Gumbel-max runs over the surviving entries. No sort, no [B, V]
-//    temporaries.
+//    reaches top_p of the top-k mass) are found by histograms over z (integer sums: order-independent),
+//    then Gumbel-max runs over the surviving entries. No sort, no [B, V] temporaries.
 //  * frequency / presence penalties: a request that asks for them owns a row of a token-count table
 //    (`counts`, int16 [slots, count_ld]); its logits become logit - freq * count - pres * (count > 0)
 //    before the temperature, in every pass, and the kernel bumps the count of the token it draws.
@@ -101,7 +99,7 @@ struct Row {
 
 // f(i, z_i) over one row: vector loads over [0, V8), scalar loads over the tail [V8, V)
 // (a thread's chunks are fetched four at a time: with one load in flight a pass over a 152k-entry row is a chain of
-// ~19 memory round trips per thread, and the filtered path makes dozens of passes)
+// ~19 memory round trips per thread)
 template <typename T, typename F>
 DEVINL void for_each_z(const Row<T>& r, int V, int V8, F f) {
   constexpr int PF = 4;
@@ -124,80 +122,193 @@ DEVINL void for_each_z(const Row<T>& r, int V, int V8, F f) {
 
 DEVINL float gumbel(uint32_t bits) { return -__logf(-__logf(u32_to_unit(bits) * 0.99999994f)); }
 
-DEVINL unsigned long long block_sum_u64(unsigned long long v, unsigned long long* red) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
-  __syncthreads();
-  if (lane == 0) red[wid] = v;
-  __syncthreads();
-  unsigned long long t = lane < nw ? red[lane] : 0ull;
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) t += __shfl_xor(t, o, 64);
-  return t;
+// ---------------------------------------------------------------------------------------------
+// Thresholds of top-k and top-p: the largest entry t of a row with F(t) >= target, F(t) = number (MASS = false) or
+// softmax mass relative to exp(-mx) (MASS = true) of the entries z >= t. A pass over the row sorts the entries of a
+// bracket [lo, hi] into SEL_BINS bins of equal width (LDS atomics) and finds the bin that holds t; its entries are copied
+// into LDS and split the same way until at most SEL_DIRECT are left, whose F are summed directly. What bounds it is
+// vector instructions of the one workgroup that owns a row: a pass over 151936 entries takes 4 to 10 us however few
+// bytes it reads, so the number of passes counts. Halving the bracket instead took five to ten passes over the row and
+// some 25 block-wide sums after them. 24 rows of 151936 bf16 entries, before and now: top-p 0.95 of normal logits 246 and
+// 132 us, of one dominant token 85 and 45; top-k 50 99 and 57, with top-p 0.9 160 and 86; 320 rows of the first 507 and 271.
+// Counts and masses (fixed point, 2^-40) are integers: no result depends on the order in which atomics arrive, so
+// replays and the ranks of a tensor-parallel group agree bit for bit. Entries more than SEL_RANGE below the maximum
+// have no mass at this resolution.
+constexpr int SEL_BINS = 1024;     // one per thread
+constexpr int SEL_CAP = 4096;      // entries of a bin that are copied into LDS (a fuller bin is split again from the row)
+constexpr int SEL_DIRECT = 256;
+constexpr float SEL_FIX = 1099511627776.f;  // 2^40
+constexpr float SEL_RANGE = 28.f;
+
+struct Select {
+  unsigned long long mass[SEL_BINS];
+  unsigned cnt[SEL_BINS];
+  float cand[SEL_CAP], few[SEL_DIRECT];
+  unsigned long long part[16], above;
+  int bin, n;
+  unsigned bin_n;
+};
+
+// monotone in z: the bins are an ordered partition of [lo, hi] (no contraction with the product that made z, so that
+// every pass puts an entry into the same bin)
+DEVINL int sel_bin(float z, float lo, float scale) {
+#pragma clang fp contract(off)
+  const float d = z - lo;
+  return min(SEL_BINS - 1, (int)(d * scale));
 }
 
-constexpr int THR_CAP = 8192;  // candidates kept in LDS once a threshold's bracket holds no more than that
-constexpr float THR_FIX = 1099511627776.f;  // 2^40: fixed-point scale of exp(z - max) in the LDS phase
+DEVINL unsigned long long sel_mass(float z, float mx) {
+#pragma clang fp contract(off)
+  const float d = z - mx;
+  return (unsigned long long)(__expf(d) * SEL_FIX);
+}
 
-// Largest t in [lo, hi] with F(t) >= target, F(t) = number (MASS = false) or softmax mass relative to exp(-mx)
-// (MASS = true) of the entries z >= t, to the resolution of 32 halvings of [lo, hi] - the threshold of top-k
-// (target k) and of top-p (target p x mass of the allowed entries; lo = the top-k threshold, so that only allowed
-// entries count). The halvings run over the whole row only until the bracket [lo, hi) holds at most THR_CAP
-// entries; those are copied into LDS and the remaining halvings run there. Sums of the LDS phase are taken in fixed
-// point: they do not depend on the order in which the candidates were appended, so replays and the ranks of a
-// tensor-parallel group agree bit for bit.
-template <bool MASS, typename T>
-DEVINL float find_threshold(const Row<T>& R, int V, int V8, float lo, float hi, float target, float mx, float* red,
-                            unsigned long long* red64, float* buf, int* buf_n, float n_ge_lo) {
-  // n_ge_lo: number of entries >= lo, or any upper bound of it (V when unknown)
-  float c_lo = n_ge_lo, c_hi = 0.f, F_hi = 0.f;
-  bool hi_moved = false;
-  int it = 0;
-  for (; it < 32 && c_lo - c_hi > (float)THR_CAP; ++it) {
-    const float mid = 0.5f * (lo + hi);
-    float cm = 0.f, fm = 0.f;
-    for_each_z(R, V, V8, [&](int, float z) {
-      if (z >= mid) {
-        cm += 1.f;
-        if (MASS) fm += __expf(z - mx);
-      }
-    });
-    cm = block_sum(cm, red);
-    const float Fm = MASS ? block_sum(fm, red) : cm;
-    if (Fm >= target) {
-      lo = mid;
-      c_lo = cm;
-    } else {
-      hi = mid;
-      c_hi = cm;
-      F_hi = Fm;
-      hi_moved = true;
-    }
-  }
-  if (it == 32) return lo;
-  if (threadIdx.x == 0) *buf_n = 0;
+// The bin of [lo, hi] in which F reaches target (S.bin, -1: none), F above it (S.above; of everything if none) and its
+// number of entries (S.bin_n). each(f) calls f(z) for every entry, over the whole block.
+template <bool MASS, typename E>
+DEVINL void select_bin(Select& S, E each, float lo, float hi, float scale, float mx, unsigned long long above,
+                       unsigned long long target) {
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   __syncthreads();
-  for_each_z(R, V, V8, [&](int, float z) {
-    if (z >= lo && (!hi_moved || z < hi)) {
-      const int pos = atomicAdd(buf_n, 1);
-      if (pos < THR_CAP) buf[pos] = z;
+  S.cnt[tid] = 0u;
+  if (MASS) S.mass[tid] = 0ull;
+  if (tid == 0) S.bin = -1;
+  __syncthreads();
+  each([&](float z) {
+    if (z >= lo && z <= hi) {
+      const int b = sel_bin(z, lo, scale);
+      atomicAdd(&S.cnt[b], 1u);
+      if (MASS) atomicAdd(&S.mass[b], sel_mass(z, mx));
     }
   });
   __syncthreads();
-  const int n = min(*buf_n, THR_CAP);
-  for (; it < 32; ++it) {
-    const float mid = 0.5f * (lo + hi);
-    unsigned long long q = 0ull;
-    for (int j = threadIdx.x; j < n; j += blockDim.x) {
-      const float z = buf[j];
-      if (z >= mid) q += MASS ? (unsigned long long)(__expf(z - mx) * THR_FIX) : 1ull;
-    }
-    q = block_sum_u64(q, red64);
-    const float Fm = F_hi + (MASS ? (float)q * (1.f / THR_FIX) : (float)q);
-    if (Fm >= target) lo = mid; else hi = mid;
+  const int b = SEL_BINS - 1 - tid;  // from the top bin down
+  const unsigned c = S.cnt[b];
+  const unsigned long long w = MASS ? S.mass[b] : (unsigned long long)c;
+  unsigned long long run = w;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const unsigned long long y = __shfl_up(run, o, 64);
+    if (lane >= o) run += y;
   }
-  return lo;
+  if (lane == 63) S.part[wid] = run;
+  __syncthreads();
+  run += above;
+  for (int i = 0; i < wid; ++i) run += S.part[i];
+  if (run >= target && run - w < target) {  // at most one bin
+    S.bin = b;
+    S.above = run - w;
+    S.bin_n = c;
+  }
+  __syncthreads();
+  if (S.bin < 0 && tid == SEL_BINS - 1) S.above = run;
+  __syncthreads();
+}
+
+// floor: entries below it do not count (the top-k threshold, or -inf); mn, mx: smallest and largest finite entry.
+// Returns floor where even all entries fall short of the target.
+template <bool MASS, typename T>
+DEVINL float select_threshold(Select& S, const Row<T>& R, int V, int V8, float floor, float mn, float mx, float target_f,
+                              float* red) {
+  if (!(mx < INFINITY) || !(mx > -INFINITY) || target_f != target_f) return floor;
+  const int tid = threadIdx.x;
+  const float bottom = fmaxf(floor, mn);
+  const double tf = MASS ? ceil((double)target_f * (double)SEL_FIX) : (double)target_f;
+  const unsigned long long target = tf < 1. ? 1ull : (unsigned long long)tf;
+  unsigned long long above = 0ull;
+  float lo = fmaxf(bottom, mx - SEL_RANGE), hi = mx, scale = 0.f;
+  auto row = [&](auto f) __attribute__((always_inline)) { for_each_z(R, V, V8, [&](int, float z) { f(z); }); };
+  int n = 0;
+  for (int round = 0;; ++round) {
+    if (round == 8) return lo;
+    scale = hi > lo ? (float)SEL_BINS / (hi - lo) : 0.f;
+    if (!(scale < INFINITY)) scale = 0.f;  // a bracket of denormal width: one bin
+    select_bin<MASS>(S, row, lo, hi, scale, mx, above, target);
+    above = S.above;
+    const int bin = S.bin;
+    if (bin < 0) {
+      if (lo <= bottom) return floor;
+      hi = nextafterf(lo, -INFINITY);
+      lo = bottom;
+      continue;
+    }
+    if (scale == 0.f) return lo;
+    n = (int)S.bin_n;
+    if (n <= SEL_CAP) {
+      __syncthreads();
+      if (tid == 0) S.n = 0;
+      __syncthreads();
+      row([&](float z) {
+        if (z >= lo && z <= hi && sel_bin(z, lo, scale) == bin) {
+          const int pos = atomicAdd(&S.n, 1);
+          if (pos < SEL_CAP) S.cand[pos] = z;
+        }
+      });
+      __syncthreads();
+      break;
+    }
+    float l = INFINITY, h = -INFINITY;
+    row([&](float z) {
+      if (z >= lo && z <= hi && sel_bin(z, lo, scale) == bin) {
+        l = fminf(l, z);
+        h = fmaxf(h, z);
+      }
+    });
+    lo = -block_max(-l, red);
+    hi = block_max(h, red);
+  }
+  // ---- the n entries of the bin, in LDS
+  auto list = [&](auto f) __attribute__((always_inline)) { for (int i = tid; i < n; i += SEL_BINS) f(S.cand[i]); };
+  const float* last = S.cand;
+  int m = n;
+  if (n > SEL_DIRECT) {
+    float l = INFINITY, h = -INFINITY;
+    list([&](float z) { l = fminf(l, z); h = fmaxf(h, z); });
+    lo = -block_max(-l, red);
+    hi = block_max(h, red);
+    for (int round = 0;; ++round) {
+      scale = hi > lo ? (float)SEL_BINS / (hi - lo) : 0.f;
+      if (round == 8 || scale == 0.f || !(scale < INFINITY)) return lo;
+      select_bin<MASS>(S, list, lo, hi, scale, mx, above, target);
+      above = S.above;
+      const int bin = S.bin;
+      m = (int)S.bin_n;
+      if (m <= SEL_DIRECT) {
+        __syncthreads();
+        if (tid == 0) S.n = 0;
+        __syncthreads();
+        list([&](float z) {
+          if (z >= lo && z <= hi && sel_bin(z, lo, scale) == bin) {
+            const int pos = atomicAdd(&S.n, 1);
+            if (pos < SEL_DIRECT) S.few[pos] = z;
+          }
+        });
+        __syncthreads();
+        last = S.few;
+        break;
+      }
+      l = INFINITY, h = -INFINITY;
+      list([&](float z) {
+        if (z >= lo && z <= hi && sel_bin(z, lo, scale) == bin) {
+          l = fminf(l, z);
+          h = fmaxf(h, z);
+        }
+      });
+      lo = -block_max(-l, red);
+      hi = block_max(h, red);
+    }
+  }
+  float t = -INFINITY;
+  if (tid < m) S.mass[tid] = MASS ? sel_mass(last[tid], mx) : 1ull;
+  __syncthreads();
+  if (tid < m) {
+    const float z = last[tid];
+    unsigned long long f = above;
+    for (int i = 0; i < m; ++i) f += last[i] >= z ? S.mass[i] : 0ull;
+    if (f >= target) t = z;
+  }
+  t = block_max(t, red);
+  return t > -INFINITY ? t : lo;
 }
 
 template <typename T>
@@ -211,9 +322,7 @@ __global__ __launch_bounds__(1024) void sample_kernel(
   __shared__ float red[16];
   __shared__ float redv[16];
   __shared__ int redi[16];
-  __shared__ unsigned long long red64[16];
-  __shared__ float cand[THR_CAP];
-  __shared__ int cand_n;
+  __shared__ Select sel;
   const int row = blockIdx.x;
   if (active && !active[row]) {  // uniform over the block
     if (threadIdx.x == 0) {
@@ -270,7 +379,7 @@ __global__ __launch_bounds__(1024) void sample_kernel(
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         m8 = fmaxf(m8, z[j]);
-        mn = fminf(mn, z[j]);
+        mn = fminf(mn, z[j] > -INFINITY ? z[j] : INFINITY);
       }
       if (m8 > mx) {
         se *= __expf(mx - m8);
@@ -298,7 +407,7 @@ __global__ __launch_bounds__(1024) void sample_kernel(
   }
   for (int i = V8 + threadIdx.x; i < V; i += blockDim.x) {
     const float z = R.z1(i);
-    mn = fminf(mn, z);
+    mn = fminf(mn, z > -INFINITY ? z : INFINITY);
     if (z > mx) {
       se *= __expf(mx - z);
       mx = z;
@@ -321,38 +430,55 @@ __global__ __launch_bounds__(1024) void sample_kernel(
   if (filtered) {
     float thr = -INFINITY;
     float mass_k = se;  // mass (relative to exp(-mx)) of the top-k set
-    float n_allowed = (float)V;  // entries in it (ties at the k-th value included)
     if (k < V && k >= 1) {
-      // largest t with count(z >= t) >= k
-      thr = find_threshold<false>(R, V, V8, mn, mx, (float)k, mx, red, red64, cand, &cand_n, (float)V);
+      thr = select_threshold<false>(sel, R, V, V8, -INFINITY, mn, mx, (float)k, red);
       if (tp < 1.f) {  // the nucleus is taken inside the top-k set: its mass is the reference
-        float mk = 0.f, nk = 0.f;
+        float mk = 0.f;
         for_each_z(R, V, V8, [&](int, float z) {
-          if (z >= thr) {
-            mk += __expf(z - mx);
-            nk += 1.f;
-          }
+          if (z >= thr) mk += __expf(z - mx);
         });
         mass_k = block_sum(mk, red);
-        n_allowed = block_sum(nk, red);
       }
     }
-    if (tp < 1.f) {
-      // largest t >= thr with mass(z >= t) >= tp * mass_k
-      const float t2 = find_threshold<true>(R, V, V8, fmaxf(thr, mn), mx, tp * mass_k, mx, red, red64, cand, &cand_n,
-                                            n_allowed);
-      thr = fmaxf(thr, t2);
+    if (tp < 1.f) thr = select_threshold<true>(sel, R, V, V8, thr, mn, mx, tp * mass_k, red);
+    // arg-max of z + Gumbel noise over the entries that survive the threshold. The noise block of four entries is made
+    // once, and only where one of them survives: with a block per entry a nucleus of 100k entries took 33 us longer.
+    for (int base = threadIdx.x * 8; base < V8; base += blockDim.x * 8 * PF) {
+      float zz[PF][8];
+#pragma unroll
+      for (int u = 0; u < PF; ++u) {
+        const int i8 = base + u * (int)blockDim.x * 8;
+        if (i8 < V8) R.z8(i8, zz[u]);
+      }
+#pragma unroll
+      for (int u = 0; u < PF; ++u) {
+        const int i8 = base + u * (int)blockDim.x * 8;
+        if (i8 >= V8) break;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const float* z = zz[u] + 4 * h;
+          if (fmaxf(fmaxf(z[0], z[1]), fmaxf(z[2], z[3])) >= thr) {
+            const u32x4 r = Philox::gen(seed, (uint64_t)row, ctr0 + (uint64_t)(i8 >> 2) + h);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              ArgMax c;
+              c.v = z[j] >= thr ? z[j] + gumbel(r[j]) : -INFINITY;
+              c.i = z[j] >= thr ? i8 + 4 * h + j : 0x7fffffff;
+              best = amax(best, c);
+            }
+          }
+        }
+      }
     }
-    // arg-max of z + Gumbel noise over the entries that survive the threshold
-    // (few entries survive: the noise block of four entries is generated only where one of them does)
-    for_each_z(R, V, V8, [&](int i, float z) {
+    for (int i = V8 + threadIdx.x; i < V; i += blockDim.x) {
+      const float z = R.z1(i);
       if (z >= thr) {
         ArgMax c;
         c.v = z + gumbel(Philox::gen(seed, (uint64_t)row, ctr0 + (uint64_t)(i >> 2))[i & 3]);
         c.i = i;
         best = amax(best, c);
       }
-    });
+    }
   }
   best = block_argmax(best, redv, redi);
   if (threadIdx.x == 0) {
