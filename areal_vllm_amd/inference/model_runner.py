@@ -292,9 +292,12 @@ class ModelRunner:
             x, _ = add_norm(cfg, h, self.model.norm, getattr(self.model, "norm_bias", None), residual)
         else:
             x, _ = ops.rmsnorm(h, self.model.norm, cfg.rms_norm_eps, residual, cfg.gemma_norm)
-        if fp32:
-            return F.linear(x.float(), self.model.head_weight.float())
-        return F.linear(x, self.model.head_weight)
+        w = self.model.head_weight
+        if not fp32:
+            return self._lm_head(x)
+        if self._lm_head_own(x) and x.shape[1] >= 512:
+            return self._lm_head(x, fp32=True)
+        return F.linear(x.float(), w.float())
 
     # ----------------------------------------------------------------------------- prefill
     @torch.no_grad()
@@ -352,6 +355,8 @@ class ModelRunner:
         hq, hkv, D = self.hq, self.hkv, self.cfg.head_dim
         T = h.shape[0]
         has_prefix = bt is not None
+        if self._prefill_fused(T):
+            return self._prefill_layers_fused(h, pos, slots, rope, cu_q, cu_k, bt, max_q)
         residual = None
         for li, blk in enumerate(self.model.layers):
             kc, vc = self.kv[li]
@@ -368,6 +373,58 @@ class ModelRunner:
 
             h, residual = self._layer(blk, h, residual, pos, slots, attn_fn)
         return h, residual
+
+    # Rows up to which a prefill runs the decode step's kernels (they take no more than 512). Wall time with the library
+    # GEMMs and with these, one row behind 811 tokens of context: 28 layers of Qwen2-1.5B 32 / 93 / 256 / 512 tokens 5.84 /
+    # 6.00 / 5.99 / 6.07 and 3.54 / 3.58 / 3.60 / 4.09 ms; 12 layers of Llama-3-8B 32 / 128 / 512 3.28 / 3.75 / 4.92 and
+    # 2.30 / 2.80 / 4.65; 6 of Qwen2.5-7B 2.21 / 2.37 / 3.54 and 1.43 / 1.69 / 2.97; 4 of Qwen3-30B-A3B 2.08 / 2.27 / 2.55
+    # and 1.97 / 2.17 / 2.49.
+    PREFILL_FUSED_MAX_ROWS = 512
+
+    def _prefill_fused(self, rows: int) -> bool:
+        return (0 < rows <= self.PREFILL_FUSED_MAX_ROWS and self.fused_decode and not self.tp_comm
+                and self.dtype == torch.bfloat16 and (self.hq + 2 * self.hkv) * self.cfg.head_dim % 32 == 0)
+
+    def _prefill_layers_fused(self, h, pos, slots, rope, cu_q, cu_k, bt, max_q):
+        """The layers of a prefill of few tokens on the decode step's GEMMs and row kernels (`_decode_layers_fused`)."""
+        from ..ops import decode_gemm as dg
+
+        cfg = self.cfg
+        hq, hkv, D = self.hq, self.hkv, cfg.head_dim
+        T, H = h.shape
+        eps, gemma = cfg.rms_norm_eps, cfg.gemma_norm
+        act = "silu" if cfg.hidden_act == "silu" else "gelu_tanh"
+        layers = self.model.layers
+        balanced = cfg.n_experts == 0 and dg.swiglu_plan(T, cfg.intermediate_size) is not None
+        x, residual = ops.rmsnorm(h, layers[0].ln1, eps, None, gemma)
+        for li, blk in enumerate(layers):
+            kc, vc = self.kv[li]
+            if bt is not None:  # some row has context in the cache: attention reads the pages directly
+                slab = dg.dgemm(x, blk.attn.qkv, epilogue=dg.EPI_SLAB)
+                q = dg.splitk_rope_cache_write(slab, slab.shape[0], blk.attn.qkv_bias, pos, slots, rope, kc, vc, hq, hkv, D,
+                                               dtype=self.dtype, q_norm=blk.attn.q_norm if cfg.qk_norm else None,
+                                               k_norm=blk.attn.k_norm if cfg.qk_norm else None, norm_eps=eps)
+                attn = ops.flash_attn_paged_prefill(q, kc, vc, bt, cu_q, cu_k, max_q)
+            else:  # (keys and values as they were projected: the cache may hold them in fewer bits)
+                qkv = blk.attn.project_qkv(x).view(T, hq + 2 * hkv, D)
+                ops.rope_and_cache_write_(qkv, pos, slots, rope, kc, vc, hq, hkv)
+                attn, _ = ops.flash_attn_varlen(qkv[:, :hq], qkv[:, hq:hq + hkv], qkv[:, hq + hkv:], cu_q, cu_q, max_q)
+            slab = dg.dgemm(attn.view(T, hq * D), blk.attn.o, epilogue=dg.EPI_SLAB)
+            x, residual = dg.splitk_residual_rmsnorm(slab, slab.shape[0], T, H, residual=residual, weight=blk.ln2, eps=eps,
+                                                     gemma=gemma, dtype=self.dtype)
+            nw = layers[li + 1].ln1 if li + 1 < len(layers) else None
+            if cfg.n_experts > 0:
+                h = blk.mlp(x, None, self.model.ep_group)
+                if nw is None:
+                    return h, residual
+                x, residual = ops.rmsnorm(h, nw, eps, residual, gemma)
+                continue
+            a = (dg.dgemm_swiglu_balanced(x, blk.mlp.gate_up, act=act) if balanced
+                 else ops.swiglu(F.linear(x, blk.mlp.gate_up), blk.mlp.act))
+            slab = dg.dgemm(a, blk.mlp.down, epilogue=dg.EPI_SLAB)
+            x, residual = dg.splitk_residual_rmsnorm(slab, slab.shape[0], T, H, residual=residual, weight=nw, eps=eps,
+                                                     gemma=gemma, dtype=self.dtype)
+        return residual, None  # nothing left to add
 
     # ------------------------------------------------------------------ penalty count table
     def token_counts(self) -> "ops.TokenCounts":
@@ -625,19 +682,30 @@ class ModelRunner:
 
     LM_HEAD_OWN_MAX_ROWS = 96
 
-    def _lm_head(self, x: torch.Tensor) -> torch.Tensor:
+    def _lm_head_own(self, x: torch.Tensor) -> bool:
+        w = self.model.head_weight
+        return (x.is_cuda and x.shape[0] <= self.LM_HEAD_OWN_MAX_ROWS and x.dtype == torch.bfloat16
+                and w.dtype == torch.bfloat16 and w.is_contiguous() and w.shape[0] % 32 == 0 and w.shape[1] % 64 == 0
+                and x.stride(1) == 1)
+
+    def _lm_head(self, x: torch.Tensor, fp32: bool = False) -> torch.Tensor:
         """Final-normed hidden states [Bp, H] -> logits [Bp, V]. Up to ~100 rows the projection is a pure weight
         stream (467 MB for Qwen2's vocabulary) and the decode GEMM on 64-row x 128-column tiles reads it at
         5.4-6.1 TB/s (77 / 86 / 99 us at 8 / 32 / 64 rows against 163 / 106 / 114 us for the library); from 128 rows
         on the two are level and the library stays."""
         w = self.model.head_weight
-        if (x.is_cuda and x.shape[0] <= self.LM_HEAD_OWN_MAX_ROWS and x.dtype == torch.bfloat16
-                and w.dtype == torch.bfloat16 and w.is_contiguous() and w.shape[0] % 32 == 0 and w.shape[1] % 64 == 0
-                and x.stride(1) == 1):
-            from ..ops import decode_gemm as dg
+        if not self._lm_head_own(x):
+            return F.linear(x, w)
+        from ..ops import decode_gemm as dg
 
-            return dg.dgemm(x, w, epilogue=dg.EPI_BF16, cfg=4, stages=3, ksplit=1, loader_waves=4, nt=True)
-        return F.linear(x, w)
+        kw = dict(cfg=4, stages=3, loader_waves=4, nt=True)
+        if not fp32:
+            return dg.dgemm(x, w, epilogue=dg.EPI_BF16, ksplit=1, **kw)
+        # Products of bf16 numbers are exact in fp32: these are the sums of an fp32 product over widened copies of both
+        # operands (530 us at one row, 539 at 24; 78 and 117 here), in four parts so that the rounding error is no larger:
+        # at K = 1536 rms 8.7e-8 to 9.0e-8 against double precision, the fp32 library product 1.1e-7 to 2.5e-7, one sum over
+        # all of K 1.8e-7.
+        return dg.dgemm(x, w, epilogue=dg.EPI_SLAB, ksplit=4, **kw).sum(0)
 
     def _decode_body(self, st: Dict[str, torch.Tensor], filtered: bool, penalized: bool = False):
         """`decode_steps` decode iterations on the static buffers (captured into a graph)."""

@@ -373,6 +373,17 @@ def context_slots(block_tables: torch.Tensor, cu_k: torch.Tensor) -> torch.Tenso
     return block_tables.long()[seq, t // PAGE_SIZE] * PAGE_SIZE + t % PAGE_SIZE
 
 
+# Workgroups that a prefill against the cache should start, and the fewest keys of one of them
+PAGED_PREFILL_WORKGROUPS, PAGED_PREFILL_KEYS = 256, 128
+
+
+def paged_prefill_splits(batch: int, n_q_heads: int, max_q: int, max_k: int) -> int:
+    """Ranges into which the keys of a query tile are split: one workgroup walks 64 keys in 2.5 us, so the few tiles of a
+    short turn behind a long context wait for one another while most of the chip idles."""
+    tiles = max(1, batch * n_q_heads * ((max_q + 127) // 128))
+    return max(1, min(PAGED_PREFILL_WORKGROUPS // tiles, max_k // PAGED_PREFILL_KEYS, 32))
+
+
 def flash_attn_paged_prefill(q, kcache, vcache, block_tables, cu_q, cu_k, max_q: int, scale: Optional[float] = None,
                              causal: bool = True) -> torch.Tensor:
     """Attention of prefill queries ``q [T, Hq, D]`` (request b owns rows cu_q[b]:cu_q[b+1]) over their requests'
@@ -388,11 +399,14 @@ def flash_attn_paged_prefill(q, kcache, vcache, block_tables, cu_q, cu_k, max_q:
         assert block_tables.dtype == torch.int32 and block_tables.is_contiguous()
         assert cu_q.dtype == torch.int32 and cu_k.dtype == torch.int32
         out = torch.empty(T, Hq, D, dtype=q.dtype, device=q.device)
+        splits = paged_prefill_splits(cu_q.numel() - 1, Hq, int(max_q), block_tables.shape[1] * PAGE_SIZE)
+        part = torch.empty(splits * T * Hq * (D + 2), dtype=torch.float32, device=q.device) if splits > 1 else None
         L.check(L.lib().areal_flash_fwd_paged(
             L.ptr(q), L.ptr(kcache), L.ptr(vcache), L.ptr(block_tables), L.c_int(block_tables.shape[1]), L.ptr(out),
             None, L.ptr(cu_q), L.ptr(cu_k), L.c_int(cu_q.numel() - 1), L.c_int(int(max_q)), L.c_int(T), L.c_int(Hq),
             L.c_int(Hkv), L.c_int(D), L.c_int64(q.stride(0)), L.c_int64(out.stride(0)), L.c_float(scale),
-            L.c_int(int(causal)), L.c_int(int(is_fp8(kcache))), L.stream_ptr()), "flash_fwd_paged")
+            L.c_int(int(causal)), L.c_int(int(is_fp8(kcache))), L.ptr(part), L.c_int(splits), L.stream_ptr()),
+            "flash_fwd_paged")
         return out
     k, v = cache_gather(kcache, vcache, context_slots(block_tables, cu_k))
     out, _ = flash_attn_varlen(q, k, v, cu_q, cu_k, max_q, scale=scale, causal=causal)

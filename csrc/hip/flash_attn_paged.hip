@@ -41,7 +41,7 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_paged_kernel(
     int nbatch, int total_q, float scale_log2, int causal, int window = 0, int keep = 0,
     const bf16_t* __restrict__ r1 = nullptr, const bf16_t* __restrict__ r2 = nullptr,
     const bf16_t* __restrict__ gate = nullptr, int64_t gate_stride = 0, int chunk = 0,
-    const bf16_t* __restrict__ sink = nullptr, const KVStrides str = KVStrides{}) {
+    const bf16_t* __restrict__ sink = nullptr, const KVStrides str = KVStrides{}, float* __restrict__ part = nullptr) {
   constexpr int D = 128;
   __shared__ __attribute__((aligned(16))) char smem[2 * 64 * 256];
   char* ks = smem;             // K tile  [64 keys][256 B], 16-byte chunks swizzled (flash_tiles.hpp)
@@ -115,6 +115,12 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_paged_kernel(
   }
   const int n_iter = n_keep + ntile_k - t_lo;
   auto tile_of = [&](int it) { return it < n_keep ? it : t_lo + it - n_keep; };
+  int it_lo = 0, it_hi = n_iter;
+  if (!WIN && part) {
+    const int per = (n_iter + (int)gridDim.y - 1) / (int)gridDim.y;
+    it_lo = min((int)blockIdx.y * per, n_iter);
+    it_hi = min(it_lo + per, n_iter);
+  }
 
   // K: thread -> (key row = tid>>4 + 16 i, 16-byte chunk tid&15). V^T: piece id = tid + 256 i ->
   // (page half = id>>9, channel = (id>>2)&127, 8-token chunk = id&3): a wave reads 1 KiB of contiguous cache.
@@ -157,17 +163,17 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_paged_kernel(
       *reinterpret_cast<bf16x4*>(row + (((c8 + 1) ^ sw) << 3)) = hi;
     }
   };
-  if (n_iter > 0) {
-    load_tile(tile_of(0));
-    store_tile(tile_of(0));
+  if (it_lo < it_hi) {
+    load_tile(tile_of(it_lo));
+    store_tile(tile_of(it_lo));
   }
   __syncthreads();
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): see flash_fwd_kernel
 
   const int vsw = (r >> 1) & 15;  // swizzle key of this lane's V^T rows (32 db + r)
-  for (int it = 0; it < n_iter; ++it) {
+  for (int it = it_lo; it < it_hi; ++it) {
     const int t = tile_of(it);
-    if (it + 1 < n_iter) load_tile(tile_of(it + 1));
+    if (it + 1 < it_hi) load_tile(tile_of(it + 1));
     f32x16 sacc[2];
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb) {
@@ -245,10 +251,28 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_paged_kernel(
       }
     }
     __syncthreads();
-    if (it + 1 < n_iter) store_tile(tile_of(it + 1));
+    if (it + 1 < it_hi) store_tile(tile_of(it + 1));
     __syncthreads();
   }
   l = sum_xor32(l);
+  if (!WIN && part) {  // this range of keys: O not divided by l, then (m, l) behind the O of all ranges
+    if (my_q < q_len) {
+      const size_t rows = (size_t)total_q * Hq, row = (size_t)(q_beg + my_q) * Hq + head;
+      float* op = part + (blockIdx.y * rows + row) * D + 4 * hf;
+#pragma unroll
+      for (int db = 0; db < 4; ++db)
+#pragma unroll
+        for (int gq = 0; gq < 4; ++gq)
+          *reinterpret_cast<f32x4*>(op + 32 * db + 8 * gq) =
+              f32x4{oacc[db][4 * gq], oacc[db][4 * gq + 1], oacc[db][4 * gq + 2], oacc[db][4 * gq + 3]};
+      if (hf == 0) {
+        float* ml = part + gridDim.y * rows * D + (blockIdx.y * rows + row) * 2;
+        ml[0] = m;
+        ml[1] = l;
+      }
+    }
+    return;
+  }
   const float inv_l = l > 0.f ? 1.f / l : 0.f;
   if (my_q < q_len) {
     bf16_t* op = o + (size_t)(q_beg + my_q) * o_stride + (size_t)head * D;
@@ -273,28 +297,66 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_paged_kernel(
   }
 }
 
+// The ranges' results -> o. One wave per query row and head, a lane per pair of channels.
+__global__ __launch_bounds__(256) void flash_paged_combine_kernel(const float* __restrict__ part, int splits,
+                                                                  bf16_t* __restrict__ o, int64_t o_stride, int Hq, int total_q) {
+  const size_t rows = (size_t)total_q * Hq, row = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= rows) return;
+  const int lane = threadIdx.x & 63;
+  const float* ml = part + splits * rows * 128;
+  float m = -INFINITY, l = 0.f;
+  if (lane < splits) {
+    m = ml[(lane * rows + row) * 2];
+    l = ml[(lane * rows + row) * 2 + 1];
+  }
+  const float mx = wave_max(m);
+  const float w = m > -INFINITY ? fast_exp2(m - mx) : 0.f;
+  const float sum = wave_sum(w * l);
+  float x = 0.f, y = 0.f;
+#pragma unroll 4
+  for (int s = 0; s < splits; ++s) {
+    const float ws = __shfl(w, s, 64);
+    const float* p = part + (s * rows + row) * 128 + lane * 2;
+    x += ws * p[0];
+    y += ws * p[1];
+  }
+  const float inv = sum > 0.f ? 1.f / sum : 0.f;
+  bf16x2 r = {f2bf(x * inv), f2bf(y * inv)};
+  *reinterpret_cast<bf16x2*>(o + row / Hq * o_stride + row % Hq * 128 + lane * 2) = r;
+}
+
 // q [total_q, Hq, 128] (row stride q_stride), K cache [P, Hkv, 32, 128], V cache [P, Hkv, 128, 32], block_tables
 // [B, max_pages] int32 (page of tokens 32 i .. 32 i + 31 of request b), cu_q / cu_k [B + 1]: query rows and context
 // lengths (the context of request b INCLUDES its query rows: they are in the cache already). Every request needs
 // q_len >= 1 and k_len >= q_len. lse may be null.
+// splits > 1 (at most 64): the key tiles of a query tile are dealt to so many workgroups, part holds splits x total_q x Hq x
+// 130 floats (and lse has to be null).
 extern "C" int areal_flash_fwd_paged(const void* q, const void* kcache, const void* vcache, const int* block_tables,
                                      int max_pages, void* o, float* lse, const int* cu_q, const int* cu_k, int B,
                                      int max_q, int total_q, int Hq, int Hkv, int D, int64_t q_stride,
-                                     int64_t o_stride, float softmax_scale, int causal, int fp8, hipStream_t st) {
+                                     int64_t o_stride, float softmax_scale, int causal, int fp8, float* part, int splits,
+                                     hipStream_t st) {
   if (B == 0 || max_q == 0) return 0;
   if (D != 128) return -1;
+  if (splits < 1 || splits > 64 || (splits > 1 && (!part || lse || (uintptr_t)part % 16 != 0 || o_stride % 2 != 0))) return -5;
+  if (splits == 1) part = nullptr;
   if (Hq % Hkv != 0) return -2;
   if ((q_stride | o_stride) % 8 != 0) return -3;
   if (((uintptr_t)q | (uintptr_t)kcache | (uintptr_t)vcache | (uintptr_t)o) % 16 != 0) return -4;
   const float scale_log2 = softmax_scale * 1.4426950408889634f;
   const int n_g_pad = (Hkv * B + 7) & ~7;
   dim3 grid((unsigned)(((max_q + 127) / 128) * (Hq / Hkv) * n_g_pad)), block(256);
-  if (fp8)
-    hipLaunchKernelGGL(flash_fwd_paged_kernel<true>, grid, block, 0, st, (const bf16_t*)q, kcache, vcache, block_tables,
-                       max_pages, (bf16_t*)o, lse, cu_q, cu_k, q_stride, o_stride, Hq, Hkv, B, total_q, scale_log2, causal);
-  else
-    hipLaunchKernelGGL(flash_fwd_paged_kernel<false>, grid, block, 0, st, (const bf16_t*)q, kcache, vcache, block_tables,
-                       max_pages, (bf16_t*)o, lse, cu_q, cu_k, q_stride, o_stride, Hq, Hkv, B, total_q, scale_log2, causal);
+  grid.y = (unsigned)splits;
+#define AREAL_PAGED_LAUNCH(FP8_)                                                                                            \
+  hipLaunchKernelGGL(flash_fwd_paged_kernel<FP8_>, grid, block, 0, st, (const bf16_t*)q, kcache, vcache, block_tables,      \
+                     max_pages, (bf16_t*)o, lse, cu_q, cu_k, q_stride, o_stride, Hq, Hkv, B, total_q, scale_log2, causal,   \
+                     0, 0, (const bf16_t*)nullptr, (const bf16_t*)nullptr, (const bf16_t*)nullptr, (int64_t)0, 0,           \
+                     (const bf16_t*)nullptr, KVStrides{}, part)
+  if (fp8) AREAL_PAGED_LAUNCH(true); else AREAL_PAGED_LAUNCH(false);
+#undef AREAL_PAGED_LAUNCH
+  if (splits > 1)
+    hipLaunchKernelGGL(flash_paged_combine_kernel, dim3((unsigned)(((int64_t)total_q * Hq + 3) / 4)), block, 0, st, part,
+                       splits, (bf16_t*)o, o_stride, Hq, total_q);
   return (int)hipGetLastError();
 }
 
