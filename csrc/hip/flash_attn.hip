@@ -638,14 +638,15 @@ __global__ __launch_bounds__(256, 2) void flash_bwd_dkv_kernel(
   }
 }
 
-// dK, dV (bf16, strided) of the keys of the sequences = sum over the parts; grid (key blocks of 64, sequences)
+// dK, dV (bf16, strided) of the keys of the sequences = sum over the parts; grid (key blocks of 8, sequences): with
+// blocks of 64 keys 700 tokens kept 11 workgroups busy for 31 us (two key heads)
 __global__ __launch_bounds__(256) void flash_bwd_sum_kernel(const float* __restrict__ part, bf16_t* __restrict__ dk,
                                                             bf16_t* __restrict__ dv, const int* __restrict__ cu_k, int Hkv,
                                                             int64_t total_k, int parts, int64_t dk_stride,
                                                             int64_t dv_stride, float softmax_scale) {
   constexpr int D = 128;
   const int k_beg = cu_k[blockIdx.y], k_len = cu_k[blockIdx.y + 1] - k_beg;
-  const int row0 = blockIdx.x * 64, rows = min(64, k_len - row0);
+  const int row0 = blockIdx.x * 8, rows = min(8, k_len - row0);
   const size_t all = (size_t)total_k * Hkv * D;
   for (int i = threadIdx.x; i < rows * Hkv * (D / 8); i += 256) {
     const int ch = i % (D / 8), rest = i / (D / 8), h = rest % Hkv;
@@ -654,6 +655,7 @@ __global__ __launch_bounds__(256) void flash_bwd_sum_kernel(const float* __restr
 #pragma unroll
     for (int w = 0; w < 2; ++w) {
       f32x4 x = {}, y = {};
+#pragma unroll 4
       for (int p = 0; p < parts; ++p) {
         const f32x4* s = reinterpret_cast<const f32x4*>(part + (2 * p + w) * all + at);
         x += s[0];
@@ -701,7 +703,7 @@ extern "C" int areal_flash_bwd(const void* q, const void* k, const void* v, cons
                      cu_k, q_stride, k_stride, v_stride, do_stride, dk_stride, dv_stride, Hq, Hkv, B, total_q, total_k,
                      parts, hs, softmax_scale, causal);
   if (parts > 1)
-    hipLaunchKernelGGL(flash_bwd_sum_kernel, dim3((max_k + 63) / 64, B), dim3(256), 0, st, part, (bf16_t*)dk, (bf16_t*)dv, cu_k,
+    hipLaunchKernelGGL(flash_bwd_sum_kernel, dim3((max_k + 7) / 8, B), dim3(256), 0, st, part, (bf16_t*)dk, (bf16_t*)dv, cu_k,
                        Hkv, total_k, parts, dk_stride, dv_stride, softmax_scale);
   const int n_g_pad = (Hkv * B + 7) & ~7;
   dim3 qgrid((unsigned)(((max_q + 127) / 128) * (Hq / Hkv) * n_g_pad));
