@@ -43,7 +43,7 @@ class _LinearMainGrad(torch.autograd.Function):
         dy2 = dy.reshape(-1, dy.shape[-1])
         dx, work = None, None
         if ctx.needs_input_grad[0]:
-            dx = torch.mm(dy2, weight).view(x.shape)
+            dx = train_gemm.dgrad(dy2, weight).view(x.shape)
             if ctx.group is not None:
                 # column-parallel layer: the input gradient is a partial sum over the tensor-parallel
                 # ranks. Its all-reduce is started here and runs on the communicator's stream while the

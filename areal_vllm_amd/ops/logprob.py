@@ -258,7 +258,7 @@ class _LMHeadLogprobFn(torch.autograd.Function):
             _bwd_inplace(lg, labels[s:e], temperature, lse[s:e], ez[s:e],
                          dlogp[s:e] if dlogp is not None else None, dent[s:e] if dent is not None else None,
                          vocab_start)
-            torch.matmul(lg, weight, out=dh[s:e])
+            train_gemm.dgrad(lg, weight, out=dh[s:e])
             if direct:
                 if train_gemm.wgrad_supported(lg, hidden[s:e], mg):
                     train_gemm.tgemm_wgrad_(mg, lg, hidden[s:e])

@@ -73,6 +73,60 @@ def tgemm_wgrad_(acc: torch.Tensor, dy: torch.Tensor, x: torch.Tensor, splits: i
     return acc
 
 
+def dgrad_splits(M: int, R: int, C: int) -> int:
+    """Parts of the reduction: about one workgroup a CU (256) over the 256 x 256 tiles, none of them empty."""
+    pairs = R // 128
+    tiles = -(-M // 256) * (C // 256)
+    splits = max(1, min(256 // tiles, pairs))
+    return -(-pairs // -(-pairs // splits))
+
+
+def dgrad_supported(dy: torch.Tensor, w: torch.Tensor) -> bool:
+    if not (dy.is_cuda and dy.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and dy.dim() == 2 and w.dim() == 2):
+        return False
+    M, R = dy.shape
+    if w.shape[0] != R or M == 0 or R == 0 or R % 128 or w.shape[1] % 256 or w.shape[1] == 0:
+        return False
+    if dy.stride(1) != 1 or w.stride(1) != 1 or dy.stride(0) % 8 or w.stride(0) % 8:
+        return False
+    if not (R <= dy.stride(0) <= 1 << 22 and w.shape[1] <= w.stride(0) <= 1 << 24):
+        return False
+    return dy.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+
+
+def tgemm_nn(dy: torch.Tensor, w: torch.Tensor, splits: int = 0, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """dy[M, R] @ w[R, C] in bf16 with fp32 accumulation: the input gradient of ``y = x @ W^T`` from the weight as it lies."""
+    assert dgrad_supported(dy, w)
+    (M, R), C = dy.shape, w.shape[1]
+    splits = splits or dgrad_splits(M, R, C)
+    if out is None:
+        out = torch.empty(M, C, dtype=torch.bfloat16, device=dy.device)
+    assert out.shape == (M, C) and out.dtype == torch.bfloat16 and out.is_contiguous()
+    part = torch.empty(splits * M * C, dtype=torch.float32, device=dy.device) if splits > 1 else None
+    L.check(L.lib().areal_tgemm_nn(L.ptr(dy), L.c_int64(dy.stride(0)), L.ptr(w), L.c_int64(w.stride(0)), L.ptr(out),
+                                   L.c_int64(C), L.ptr(part), L.c_int(splits), L.c_int(M), L.c_int(R), L.c_int(C),
+                                   L.stream_ptr()), "tgemm_nn")
+    return out
+
+
+# Few rows and a deep reduction: the library then runs a few dozen workgroups. Its kernel and this one, us (parts): 17920 deep
+# to 1536 columns, 256 / 700 / 2048 / 3072 rows 102 / 130 / 204 / 218 and 36 (35) / 56 (14) / 109 (5) / 152 (3); 151936 to
+# 1536, 64 / 700 / 3072 rows 447 / 600 / 1938 and 105 / 291 / 1201; 28672 to 4096, 700 / 1536 rows 279 / 308 and 154 (5) /
+# 339 (2). From 4096 rows on or below three parts the two are level, and so they are (or the library is ahead: 1536 deep to
+# 8960 columns, 700 rows 26 and 39) where the reduction is short: 9728 deep 52 and 35, 5120 deep 34 and 35.
+DGRAD_MIN_DEPTH, DGRAD_MAX_ROWS, DGRAD_MIN_PARTS = 8192, 3072, 3
+
+
+def dgrad(dy: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """dy @ w inside a backward pass (a library product where that pass is itself recorded)."""
+    if (not torch.is_grad_enabled() and dgrad_supported(dy, w) and (out is None or out.is_contiguous() and out.data_ptr() % 8 == 0
+                                                                    and out.dtype == torch.bfloat16)):
+        (M, R), C = dy.shape, w.shape[1]
+        if R >= DGRAD_MIN_DEPTH and M <= DGRAD_MAX_ROWS and dgrad_splits(M, R, C) >= DGRAD_MIN_PARTS:
+            return tgemm_nn(dy, w, out=out)
+    return torch.mm(dy, w) if out is None else torch.mm(dy, w, out=out)
+
+
 # rows from which the fused gate|up + SwiGLU kernel replaces library GEMM + activation kernel in no-grad forwards
 GATED_MIN_ROWS = int(os.environ.get("AREAL_FUSED_MLP_MIN_ROWS", "4096"))
 

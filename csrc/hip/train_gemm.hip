@@ -575,6 +575,200 @@ __global__ __launch_bounds__(512) void tgemm_wgrad_kernel(const TWArgs a) {
   }
 }
 
+// =====================================================================================
+// Input gradient:  dX[M, C] = dY[M, R] . W[R, C]     (bf16 operands; W as it lies, no transposed copy)
+//
+// The phases of the two kernels above: dY is staged and read as the forward kernel's A operand (reduction contiguous), W as
+// the weight gradient's X (reduction slow, transposed reads). For few rows and a deep reduction: a pass over 700 tokens has 18
+// tiles of 256 x 256 for the gate|up projection's 17920 and the vocabulary's 151936 weight rows, so the reduction is split
+// until the chip is full; the parts are written as fp32 and summed by a kernel of their own (they stay in the L2 and the
+// memory-side cache).
+// =====================================================================================
+struct TNArgs {
+  const bf16_t* dY;
+  long ldy;
+  const bf16_t* W;
+  long ldw;
+  bf16_t* dX;
+  long ldx;
+  float* part;  // [splits][M][C], null for one part
+  int M, R, C;
+  int tiles_m, tiles;
+  int pairs, chunk;  // 128-deep pairs of the reduction: of all of it, of one workgroup
+};
+
+template <bool STAGGER>
+__global__ __launch_bounds__(512) void tgemm_nn_kernel(const TNArgs a) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wr = wave >> 2, wc = wave & 3;
+  // ids are dealt round-robin to the 8 XCDs: one XCD takes neighbouring tiles of one part, which share panels in its L2
+  const int nb = gridDim.x, xq = nb >> 3, xr = nb & 7, xx = blockIdx.x & 7;
+  const int b = (xx < xr ? xx * (xq + 1) : xr * (xq + 1) + (xx - xr) * xq) + ((int)blockIdx.x >> 3);
+  const int split = b / a.tiles, tile_id = b - split * a.tiles;
+  const int m0 = (tile_id % a.tiles_m) * 256, c0 = (tile_id / a.tiles_m) * 256;
+  const int p0 = split * a.chunk, p1 = min(a.pairs, p0 + a.chunk);
+  const int KT = (p1 - p0) * 2;
+  if (KT <= 0) return;
+
+  // ---- staging. dY piece: row (wave * 8 + lane / 8) of a 64-row issue, 16-byte chunk lane & 7. W piece: reduction row
+  // (wave * 4 + lane / 16) of a 32-row issue, chunk lane & 15. Rows of dY past M are out of the buffer's range (zeros).
+  const int arow = wave * 8 + (lane >> 3), ach = (lane & 7) ^ ((arow >> 1) & 7);
+  const int wrow = wave * 4 + (lane >> 4);
+  const int pc = ((lane & 15) ^ (((lane >> 4) << 2) | (wave & 3))) * 8;
+  const unsigned rowA = (unsigned)a.ldy * 2, rowB = (unsigned)a.ldw * 2;
+  const unsigned vA = arow * rowA + ach * 16;
+  const unsigned vB = wrow * rowB + ((pc >> 5) * 64 + (pc & 31)) * 2;
+  const unsigned rangeA = (unsigned)(min(a.M - m0, 256) - 1) * rowA + 128, rangeB = 63 * rowB + 512;
+  const bf16_t* pA = a.dY + (size_t)m0 * a.ldy + (size_t)p0 * 128;
+  const bf16_t* pB = a.W + (size_t)p0 * 128 * a.ldw + c0;
+  auto stage = [&](int buf, int piece, int kt) __attribute__((always_inline)) {
+    char* dst = smem + buf * TG_BUF + piece * TG_PIECE + wave * 1024;
+    const bool isA = piece < 2;
+    const bf16_t* base = isA ? pA + (size_t)kt * 64 : pB + (size_t)kt * 64 * a.ldw;
+    const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(base), 0, isA ? rangeA : rangeB, 0x00020000);
+    const unsigned v = isA ? vA + (piece & 1) * 64 * rowA : vB + (piece & 1) * 64;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lptr_t)dst, 16, v, 0, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lptr_t)(dst + 8192), 16, v + (isA ? 128 * rowA : 32 * rowB), 0, 0, 0);
+  };
+
+  // ---- fragments: element j of lane half hf is reduction row 16 s + 8 hf + j in both operands
+  const int gl = lane & 15, grp = lane >> 4, hf = lane >> 5, r32 = lane & 31;
+  const int sw = (r32 >> 1) & 7;
+  int b_adr[2];
+#pragma unroll
+  for (int h2 = 0; h2 < 2; ++h2)
+    b_adr[h2] = (int)(tr_addr((const char*)0, 8 * hf + 4 * h2, wc * 32 + 16 * (grp & 1), gl) - (const char*)0);
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(lptr_t)smem;
+  auto trl = [&](uint32_t adr, int imm) __attribute__((always_inline)) {  // see the weight gradient
+    bf16x4 v;
+    asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(v) : "v"(adr), "i"(imm));
+    return v;
+  };
+  bf16x8 af[2][4], bf0[4], bf1[4];  // [32-row tile][16-deep slab]
+  auto read_a = [&](int buf, int h) __attribute__((always_inline)) {
+    const char* p = smem + buf * TG_BUF + h * TG_PIECE + (wr * 64 + r32) * 128;
+#pragma unroll
+    for (int mi = 0; mi < 2; ++mi)
+#pragma unroll
+      for (int s = 0; s < 4; ++s) af[mi][s] = *reinterpret_cast<const bf16x8*>(p + mi * 4096 + (((2 * s + hf) ^ sw) << 4));
+  };
+  auto read_b = [&](int buf, int h, bf16x8 (&bf)[4]) __attribute__((always_inline)) {
+    const uint32_t p = lds0 + buf * TG_BUF;
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+      bf[s] = cat4(trl(p + b_adr[0], (2 + h) * TG_PIECE + s * 4096), trl(p + b_adr[1], (2 + h) * TG_PIECE + s * 4096));
+  };
+  tw_acc acc00, acc01, acc10, acc11;  // [row half][column half]
+  auto mma = [&](tw_acc& acc, bf16x8 (&bf)[4]) __attribute__((always_inline)) {
+    tg_barrier();
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int mi = 0; mi < 2; ++mi) acc[mi] = mfma32(bf[s], af[mi][s], acc[mi]);
+    __builtin_amdgcn_s_setprio(0);
+    __builtin_amdgcn_sched_barrier(0);
+    tg_barrier();
+  };
+  // TAIL 0: tiles t+1 and t+2 exist; 1: only t+1 exists; 2: last tile
+  auto tile = [&](auto buf_c, int t, auto tail_c) __attribute__((always_inline)) {
+    constexpr int buf = decltype(buf_c)::value, TAIL = decltype(tail_c)::value;
+    read_b(buf, 0, bf0);
+    __builtin_amdgcn_sched_barrier(0);
+    read_a(buf, 0);
+    if (TAIL < 2) stage(buf ^ 1, PA1, t + 1);
+    asm volatile("s_waitcnt lgkmcnt(8)" ::: "memory");  // the eight B0 reads, issued first of 16, have returned
+    mma(acc00, bf0);
+    read_b(buf, 1, bf1);
+    if (TAIL < 1) stage(buf, PB0, t + 2);
+    mma(acc01, bf1);
+    read_a(buf, 1);
+    if (TAIL < 1) stage(buf, PA0, t + 2);
+    mma(acc11, bf1);
+    if (TAIL < 1) stage(buf, PB1, t + 2);
+    if (TAIL == 0) tg_vmcnt<6>();
+    if (TAIL == 1) tg_vmcnt<0>();
+    mma(acc10, bf0);
+  };
+  using B0 = std::integral_constant<int, 0>;
+  using B1 = std::integral_constant<int, 1>;
+  using T0 = std::integral_constant<int, 0>;
+  using T1 = std::integral_constant<int, 1>;
+  using T2 = std::integral_constant<int, 2>;
+#pragma unroll
+  for (int mi = 0; mi < 2; ++mi)
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      acc00[mi][j] = 0.f;
+      acc01[mi][j] = 0.f;
+      acc10[mi][j] = 0.f;
+      acc11[mi][j] = 0.f;
+    }
+  stage(0, PB0, 0);
+  stage(0, PA0, 0);
+  stage(0, PB1, 0);
+  stage(0, PA1, 0);
+  stage(1, PB0, 1);
+  stage(1, PA0, 1);
+  stage(1, PB1, 1);
+  tg_vmcnt<6>();
+  tg_barrier();
+  if (STAGGER && wr == 1) tg_barrier();
+  int t = 0;
+  for (; t + 2 < KT; t += 2) {
+    tile(B0{}, t, T0{});
+    tile(B1{}, t + 1, T0{});
+  }
+  tile(B0{}, t, T1{});
+  tile(B1{}, t + 1, T2{});
+  if (STAGGER && wr == 0) tg_barrier();
+
+  // ---- lane (row r32, hf) holds columns (reg & 3) + 8 (reg >> 2) + 4 hf of each 32 x 32 tile
+  auto put = [&](tw_acc& acc, int mh, int nh) __attribute__((always_inline)) {
+#pragma unroll
+    for (int mi = 0; mi < 2; ++mi) {
+      const int m = m0 + wr * 128 + mh * 64 + mi * 32 + r32, c = c0 + wc * 64 + nh * 32 + 4 * hf;
+      if (m >= a.M) continue;
+      if (a.part) {
+        float* op = a.part + ((size_t)split * a.M + m) * a.C + c;
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          *reinterpret_cast<f32x4*>(op + 8 * g) =
+              f32x4{acc[mi][4 * g], acc[mi][4 * g + 1], acc[mi][4 * g + 2], acc[mi][4 * g + 3]};
+      } else {
+        bf16_t* op = a.dX + (size_t)m * a.ldx + c;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          bf16x4 v;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) v[j] = f2bf(acc[mi][4 * g + j]);
+          *reinterpret_cast<bf16x4*>(op + 8 * g) = v;
+        }
+      }
+    }
+  };
+  put(acc00, 0, 0);
+  put(acc01, 0, 1);
+  put(acc10, 1, 0);
+  put(acc11, 1, 1);
+}
+
+// dX (rows of C numbers, C a multiple of 256) = sum of the parts, in order
+__global__ __launch_bounds__(256) void tgemm_nn_sum_kernel(const float* __restrict__ part, int splits, bf16_t* __restrict__ dX,
+                                                           long ldx, int M, int C) {
+  const size_t n = (size_t)M * C, i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
+  if (i >= n) return;
+  f32x4 v = *reinterpret_cast<const f32x4*>(part + i);
+#pragma unroll 4
+  for (int s = 1; s < splits; ++s) v += *reinterpret_cast<const f32x4*>(part + s * n + i);
+  const bf16x4 o = {f2bf(v[0]), f2bf(v[1]), f2bf(v[2]), f2bf(v[3])};
+  *reinterpret_cast<bf16x4*>(dX + i / C * ldx + i % C) = o;
+}
+
 }  // namespace
 
 // C[M, N] = A[M, K] . B[N, K]^T (+ bias). Leading dimensions in elements (multiples of 8: 16-byte rows), K a multiple
@@ -685,5 +879,33 @@ extern "C" int areal_tgemm_wgrad(const void* dY, long ldy, const void* X, long l
     hipLaunchKernelGGL(tgemm_wgrad_kernel<true>, grid, block, TG_LDS, st, a);
   else
     hipLaunchKernelGGL(tgemm_wgrad_kernel<false>, grid, block, TG_LDS, st, a);
+  return (int)hipGetLastError();
+}
+
+// dX[M, C] = dY[M, R] . W[R, C]; R a multiple of 128, C of 256, rows 16-byte aligned. part: splits x M x C floats, unused for
+// one part. Every part has work as long as splits <= R / 128 and is the number areal_tgemm_nn_splits returns.
+extern "C" int areal_tgemm_nn(const void* dY, long ldy, const void* W, long ldw, void* dX, long ldx, float* part, int splits,
+                              int M, int R, int C, hipStream_t st) {
+  if (M <= 0 || R <= 0 || C <= 0) return R <= 0 && M > 0 && C > 0 ? -1 : 0;
+  if (R % 128 != 0 || C % 256 != 0 || ldy % 8 != 0 || ldw % 8 != 0 || ldx % 4 != 0) return -1;
+  if (((uintptr_t)dY | (uintptr_t)W) % 16 != 0 || (uintptr_t)dX % 8 != 0 || (uintptr_t)part % 16 != 0) return -1;
+  if (ldy < R || ldw < C || ldx < C || ldy > (1l << 22) || ldw > (1l << 24)) return -1;  // byte offsets of 256 / 64 rows: 32 bits
+  const int tiles_m = (M + 255) / 256, pairs = R / 128;
+  if (splits < 1 || splits > pairs || (splits > 1 && !part)) return -1;
+  const int chunk = (pairs + splits - 1) / splits;
+  if ((pairs + chunk - 1) / chunk != splits) return -1;  // a part without work would leave its sums unwritten
+  const long tiles = (long)tiles_m * (C / 256);
+  if (tiles * splits > 0x7fffffffl) return -1;
+  TNArgs a{(const bf16_t*)dY, ldy, (const bf16_t*)W, ldw, (bf16_t*)dX, ldx, splits > 1 ? part : nullptr, M, R, C, tiles_m,
+           (int)tiles, pairs, chunk};
+  static bool attr_set = false;
+  if (!attr_set) {
+    HIP_RET(hipFuncSetAttribute((const void*)tgemm_nn_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, TG_LDS));
+    attr_set = true;
+  }
+  hipLaunchKernelGGL((tgemm_nn_kernel<true>), dim3((unsigned)(tiles * splits)), dim3(512), TG_LDS, st, a);
+  if (splits > 1)
+    hipLaunchKernelGGL(tgemm_nn_sum_kernel, dim3((unsigned)(((size_t)M * C / 4 + 255) / 256)), dim3(256), 0, st, part, splits,
+                       (bf16_t*)dX, ldx, M, C);
   return (int)hipGetLastError();
 }

@@ -1,0 +1,37 @@
+"""Input-gradient GEMM dX = dY . W from the weight as it lies: ragged row counts, one and several parts of the reduction."""
+import pytest
+import torch
+
+from areal_vllm_amd.ops import train_gemm as tg
+
+DEV = "cuda:0"
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("M", [1, 63, 64, 129, 255, 256, 257, 700, 1024])
+@pytest.mark.parametrize("R,C", [(128, 256), (384, 512), (1536, 1280), (17920, 256)])
+@pytest.mark.parametrize("splits", [0, 1, 2])
+def test_dgrad(M, R, C, splits):
+    g = torch.Generator(device=DEV).manual_seed(M + R)
+    # rows past the last one, and what lies beside the operands, must not be read
+    dy = torch.full((M + 256, R + 8), float("nan"), device=DEV).bfloat16()
+    w = torch.full((R + 64, C + 16), float("nan"), device=DEV).bfloat16()
+    dy[:M, :R] = torch.randn(M, R, device=DEV, generator=g).bfloat16()
+    w[:R, :C] = (torch.randn(R, C, device=DEV, generator=g) / R ** 0.5).bfloat16()
+    dy, w = dy[:M, :R], w[:R, :C]
+    assert tg.dgrad_supported(dy, w)
+    if splits == 2 and R == 128:
+        pytest.skip("one pair of the reduction cannot be split")
+    got = tg.tgemm_nn(dy, w, splits=splits)
+    want = dy.double() @ w.double()
+    # outputs of size one (up to 6), rounded to bf16 once: 2^-9 relative; the fp32 sums are far more accurate
+    assert bool(((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4).all())
+
+
+def test_parts_have_work():
+    for M in (1, 256, 700, 4096, 30000):
+        for R in (128, 256, 1536, 17920, 151936):
+            for C in (256, 1536, 8960):
+                s = tg.dgrad_splits(M, R, C)
+                pairs = R // 128
+                assert 1 <= s <= pairs and -(-pairs // -(-pairs // s)) == s
