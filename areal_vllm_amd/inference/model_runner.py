@@ -382,8 +382,8 @@ class ModelRunner:
     PREFILL_FUSED_MAX_ROWS = 512
 
     def _prefill_fused(self, rows: int) -> bool:
-        return (0 < rows <= self.PREFILL_FUSED_MAX_ROWS and self.fused_decode and not self.tp_comm
-                and self.dtype == torch.bfloat16 and (self.hq + 2 * self.hkv) * self.cfg.head_dim % 32 == 0)
+        return (0 < rows <= self.PREFILL_FUSED_MAX_ROWS and self.fused_decode and self.dtype == torch.bfloat16
+                and (self.hq + 2 * self.hkv) * self.cfg.head_dim % 32 == 0)
 
     def _prefill_layers_fused(self, h, pos, slots, rope, cu_q, cu_k, bt, max_q):
         """The layers of a prefill of few tokens on the decode step's GEMMs and row kernels (`_decode_layers_fused`)."""
@@ -395,7 +395,22 @@ class ModelRunner:
         eps, gemma = cfg.rms_norm_eps, cfg.gemma_norm
         act = "silu" if cfg.hidden_act == "silu" else "gelu_tanh"
         layers = self.model.layers
-        balanced = cfg.n_experts == 0 and dg.swiglu_plan(T, cfg.intermediate_size) is not None
+        balanced = cfg.n_experts == 0 and dg.swiglu_plan(T, layers[0].mlp.gate_up.shape[0] // 2) is not None
+        tp = self.tp_comm
+
+        def finish(slab, residual, weight):
+            """Split-K slabs of a projection -> (normalised input of the next GEMM, new residual stream); without a norm
+            behind it (last output, residual stream or None where it is in the output already)."""
+            if tp:  # (the sums over the group then take the same row kernel: a group of one gives the same bits as none)
+                part, _ = dg.splitk_residual_rmsnorm(slab, slab.shape[0], T, H, dtype=self.dtype)
+                self._tp_all_reduce(part)
+                if weight is None:
+                    return part, residual
+                slab = part.float()[None]
+            x, s = dg.splitk_residual_rmsnorm(slab, slab.shape[0], T, H, residual=residual, weight=weight, eps=eps,
+                                              gemma=gemma, dtype=self.dtype)
+            return (x, s) if weight is not None else (s, None)
+
         x, residual = ops.rmsnorm(h, layers[0].ln1, eps, None, gemma)
         for li, blk in enumerate(layers):
             kc, vc = self.kv[li]
@@ -410,11 +425,12 @@ class ModelRunner:
                 ops.rope_and_cache_write_(qkv, pos, slots, rope, kc, vc, hq, hkv)
                 attn, _ = ops.flash_attn_varlen(qkv[:, :hq], qkv[:, hq:hq + hkv], qkv[:, hq + hkv:], cu_q, cu_q, max_q)
             slab = dg.dgemm(attn.view(T, hq * D), blk.attn.o, epilogue=dg.EPI_SLAB)
-            x, residual = dg.splitk_residual_rmsnorm(slab, slab.shape[0], T, H, residual=residual, weight=blk.ln2, eps=eps,
-                                                     gemma=gemma, dtype=self.dtype)
+            x, residual = finish(slab, residual, blk.ln2)
             nw = layers[li + 1].ln1 if li + 1 < len(layers) else None
             if cfg.n_experts > 0:
                 h = blk.mlp(x, None, self.model.ep_group)
+                if tp:
+                    self._tp_all_reduce(h)
                 if nw is None:
                     return h, residual
                 x, residual = ops.rmsnorm(h, nw, eps, residual, gemma)
@@ -422,9 +438,8 @@ class ModelRunner:
             a = (dg.dgemm_swiglu_balanced(x, blk.mlp.gate_up, act=act) if balanced
                  else ops.swiglu(F.linear(x, blk.mlp.gate_up), blk.mlp.act))
             slab = dg.dgemm(a, blk.mlp.down, epilogue=dg.EPI_SLAB)
-            x, residual = dg.splitk_residual_rmsnorm(slab, slab.shape[0], T, H, residual=residual, weight=nw, eps=eps,
-                                                     gemma=gemma, dtype=self.dtype)
-        return residual, None  # nothing left to add
+            x, residual = finish(slab, residual, nw)
+        return x, residual
 
     # ------------------------------------------------------------------ penalty count table
     def token_counts(self) -> "ops.TokenCounts":

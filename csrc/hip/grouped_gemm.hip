@@ -19,7 +19,8 @@
 
 // Tile `id` (tiles of TM rows, numbered expert by expert) -> its expert, the tile's number there and the expert's rows;
 // false behind the last tile. A lane per expert: walking 128 experts one after the other is a chain of scalar loads ahead of
-// a workgroup's first tile (one decode row, 8 of 128 experts used: 42 us a launch, now 13).
+// a workgroup's first tile (8 rows on 8 of 128 experts, 1536 columns,
+// 2048 deep: 34 us a launch, now 22).
 template <int TM>
 DEVINL bool gg_find_tile(const int* __restrict__ offsets, int E, int id, int& e, int& tile, int& row_lo, int& row_hi) {
   const int lane = threadIdx.x & 63;
