@@ -107,10 +107,10 @@ __global__ __launch_bounds__(64 * (WM * WN + LW)) void dgemm_kernel(const DGArgs
   const int wm = wave % WM, wn = wave / WM;
   int split = blockIdx.x, ct = blockIdx.y, mb = blockIdx.z;
   if (a.inv_z != 0) {
-    // Three row blocks or more. Ids are dealt round-robin to the 8 XCDs: each XCD takes a contiguous range, row blocks first, then
-    // column tiles, so that a weight tile's row blocks meet in one L2 and a K slice of X is fetched by one or two L2s
-    // (320 rows x 1536 columns, 8960 deep: 23.2 -> 19.5 us). With one or two row blocks the launch order is as good or
-    // better (93 rows, 2048 columns, 1536 deep: 6.0 us, dealt this way 6.7).
+    // Three row blocks or more, of 128 rows at least. Ids are dealt round-robin to the 8 XCDs: each XCD takes a contiguous
+    // range, row blocks first, then column tiles, so that a weight tile's row blocks meet in one L2 and a K slice of X is
+    // fetched by one or two L2s (320 rows x 1536 columns, 8960 deep: 23.2 -> 19.5 us). With fewer or smaller row blocks the
+    // launch order is as good or better (93 rows in 64-row blocks, 2048 columns, 1536 deep: 6.0 us, dealt this way 6.7).
     const int nb = gridDim.x * gridDim.y * gridDim.z, q = nb >> 3, r = nb & 7;
     const int id = split + gridDim.x * (ct + gridDim.y * mb), x = id & 7;
     const int pos = (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + (id >> 3);
@@ -369,7 +369,7 @@ int launch_cfg(const DGArgs& a, int ksplit, hipStream_t st) {
   constexpr int cols_per_tile = (EPI == DG_SWIGLU || EPI == DG_ROPE) ? BN / 2 : BN;
   dim3 grid(ksplit, (ncols + cols_per_tile - 1) / cols_per_tile, (a.M + BM - 1) / BM);
   DGArgs b = a;
-  if (grid.z > 2 && grid.y > 1 && (uint64_t)grid.x * grid.y * grid.z < 65536) {
+  if (BM >= 128 && grid.z > 2 && grid.y > 1 && (uint64_t)grid.x * grid.y * grid.z < 65536) {
     b.inv_y = (unsigned)(((1ull << 32) + grid.y - 1) / grid.y);
     b.inv_z = (unsigned)(((1ull << 32) + grid.z - 1) / grid.z);
   }
