@@ -479,9 +479,12 @@ class DecodeItems:
                  max_context: Optional[int] = None):
         self.batch, self.n_q_heads, self.n_kv_heads, self.head_dim = batch, n_q_heads, n_kv_heads, head_dim
         self.target = max(1, DECODE_ITEMS // n_kv_heads)
-        self.n_items = self.target + batch
-        if max_context is not None:  # a row of n pages is at most sqrt(3 n) items
-            self.n_items = min(self.n_items, batch * (math.isqrt(3 * -(-int(max_context) // PAGE_SIZE)) + 1))
+        pages = None if max_context is None else -(-int(max_context) // PAGE_SIZE)
+        # twice the items where shares of 32 pages and items 1.4 times as long can occur
+        self.finer = pages is None or (pages > 44 and batch * pages > 31 * self.target)
+        self.n_items = self.target * (2 if self.finer else 1) + batch
+        if pages is not None:  # a row of n pages is at most sqrt(3 n) items
+            self.n_items = min(self.n_items, batch * (math.isqrt(3 * pages) + 1))
         self.items = torch.zeros(self.n_items, 8, dtype=torch.int32, device=device)
         self.part_o = torch.empty(self.n_items, n_q_heads, head_dim, dtype=torch.float32, device=device)
         self.part_ml = torch.empty(self.n_items, n_q_heads, 2, dtype=torch.float32, device=device)
@@ -492,7 +495,8 @@ class DecodeItems:
         if L.use_hip(context_lens):
             assert context_lens.dtype == torch.int32 and context_lens.is_contiguous() and context_lens.numel() == self.batch
             L.check(L.lib().areal_paged_decode_items(L.ptr(context_lens), L.ptr(self.items), L.c_int(self.batch),
-                                                     L.c_int(self.target), L.c_int(self.n_items), L.stream_ptr()),
+                                                     L.c_int(self.target), L.c_int(self.n_items), L.c_int(int(self.finer)),
+                                                     L.stream_ptr()),
                     "paged_decode_items")
         return self
 

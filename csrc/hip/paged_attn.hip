@@ -335,6 +335,11 @@ struct DecodeItem { int b, p_beg, p_end, base, n, part, pad0, pad1; };
 // many that the workgroup that combines a row's n partial results does not read longer than the others walk:
 // n^2 <= 3 pages (1 x 16000 tokens: 16.3 us, 22.4 us with n^2 <= 5 pages of 4-page items).
 constexpr int STEP = 4;
+// Even share from which the number of items may double (paged_decode_items_kernel). 8 steps of 14 layers, two key heads:
+// 60 rows of 3000-9000 tokens 17.8 -> 15.7 ms, 90 of 2000-7000 21.3 -> 18.3; equal
+// rows, whose items are level, lose by it (100 rows of 6000: 21.0 -> 22.5), and so do short items (5 rows of 4000-16000:
+// 7.9 -> 8.4).
+constexpr int FINER_EVEN = 32;
 DEVINL int pages_per_item(int np, int even) {
   const int most = max(1, (int)sqrtf(3.f * (float)np));
   const int n = min(most, max(1, (np + even / 2) / even));
@@ -342,10 +347,11 @@ DEVINL int pages_per_item(int np, int even) {
   return max(STEP, (per + STEP - 1) / STEP * STEP);
 }
 
-// grid 1, block 1024. n_items >= min(target + B, the rows' largest number of items x B). Pages per item: the whole batch over `target` items.
+// grid 1, block 1024. n_items >= min(target + B, the rows' largest number of items x B),
+// with `finer` 2 target + B. Pages per item: the whole batch over `target` items.
 __global__ __launch_bounds__(1024) void paged_decode_items_kernel(const int* __restrict__ context_lens,
                                                                   DecodeItem* __restrict__ items, int B, int target,
-                                                                  int n_items) {
+                                                                  int n_items, int finer) {
   constexpr int NB = 64;  // size classes of the sort
   __shared__ int red[16], hist[NB];
   const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
@@ -359,7 +365,21 @@ __global__ __launch_bounds__(1024) void paged_decode_items_kernel(const int* __r
   int total = 0;
 #pragma unroll
   for (int w = 0; w < 16; ++w) total += red[w];
-  const int even = max(STEP, (total + target - 1) / target);
+  int even = max(STEP, (total + target - 1) / target);
+  if (finer && even >= FINER_EVEN) {  // long items: where a row's rounding makes one of them 1.4 times the even share, twice as many
+    int longest = 0;
+    for (int b = t; b < B; b += 1024)
+      longest = max(longest, pages_per_item((max(context_lens[b], 0) + PAGE - 1) / PAGE, even));
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) longest = max(longest, __shfl_xor(longest, o, 64));
+    __syncthreads();
+    if (lane == 0) red[wid] = longest;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < 16; ++w) longest = max(longest, red[w]);
+    if (5 * longest > 7 * even) even = max(STEP, (total + 2 * target - 1) / (2 * target));
+    __syncthreads();
+  }
   const int top = even + even / 2 + STEP;  // an item has more pages only if its row may not be divided further
   auto size_class = [&](int size) { return NB - 1 - min(NB - 1, size * (NB - 1) / top); };
   for (int b = t; b < B; b += 1024) {  // items per size class
@@ -621,12 +641,12 @@ __global__ __launch_bounds__(64 * NW, (D > 128 ? 1 : 2)) void paged_decode_walk_
   }
 }
 
-// Items of the batch's decode attention; `items`: n_items x 8 ints, at least min(target + B, B x most items of a row).
-extern "C" int areal_paged_decode_items(const int* context_lens, void* items, int B, int target, int n_items,
+// Items of the batch's decode attention; `items`: n_items x 8 ints, at least min(target + B, B x most items of a row); with finer 2 target + B.
+extern "C" int areal_paged_decode_items(const int* context_lens, void* items, int B, int target, int n_items, int finer,
                                         hipStream_t st) {
   if (B < 1 || target < 1 || n_items < B) return -1;
   hipLaunchKernelGGL(paged_decode_items_kernel, dim3(1), dim3(1024), 0, st, context_lens, (DecodeItem*)items, B, target,
-                     n_items);
+                     n_items, finer);
   return (int)hipGetLastError();
 }
 

@@ -31,7 +31,7 @@ def _setup(ctx, Hq, Hkv, D, fp8, seed):
 
 @pytest.mark.parametrize("Hq,Hkv,D,fp8", [(12, 2, 128, False), (12, 2, 128, True), (32, 4, 128, False), (7, 7, 64, False),
                                           (16, 2, 64, True), (8, 1, 256, False), (16, 1, 256, True)])
-@pytest.mark.parametrize("ctx", [[1], [640], [0, 1, 31, 32, 33, 127, 128, 129, 4099], [3000] * 3 + [1] * 1100])
+@pytest.mark.parametrize("ctx", [[1], [640], list(range(3000, 9000, 100)), [0, 1, 31, 32, 33, 127, 128, 129, 4099], [3000] * 3 + [1] * 1100])
 def test_decode_attention_on_items(Hq, Hkv, D, fp8, ctx):
     if len(ctx) > 100 and Hkv == 7:
         pytest.skip("one wide batch a head count is enough")
