@@ -25,16 +25,18 @@
 // KV tile = 64 keys. D = 128.
 //
 // What bounds it: a wave's 32 x 64 scores take 1024 cycles of matrix pipe per tile and about as much of the vector pipe
-// (32 exponentials and seven more operations each per lane), so the two have to overlap: two workgroups a CU (two waves a
-// SIMD, 250 registers each) that run apart, and as few vector operations as the softmax allows:
-//   * the scale is folded into the exponential's argument, exp2(s c - m c): one fused multiply-add an element; m is the
-//     maximum of the raw scores (a negative scale flips the sign of Q first);
-//   * O and l are rescaled only when some row's maximum has grown by more than 8 (in log2 units) since they last were: a
-//     probability is then at most 2^8, in bf16 as exact as below 1;
+// (32 exponentials and eight more operations each per lane), so the two have to overlap: two workgroups a CU (two waves a
+// SIMD, 228 registers each) that run apart:
 //   * tiles that no query of the wave may miss a key of run without mask code, tiles it sees no key of are skipped;
 //   * K and V tiles come by LDS-DMA into two buffers: no staging registers, one barrier a tile.
-// Measured (12 query heads on 2 key heads), register-staged tiles with one rescale a tile -> this: 25 sequences of ~1133 tokens
-// 216 -> 162 us, 24576 tokens 2.15 -> 1.75 ms (862 -> 1060 TFLOP/s); 3 x 8192 (28 on 4 heads) 2.02 -> 1.57 ms.
+// A row's scores are scaled (rounded once), its maximum follows every tile and the exponential takes the difference: what
+// comes out of a row depends on that row alone, bit for bit, whatever else is packed beside it. (Folding the scale into the
+// exponential's argument and rescaling only when some row of the wave has grown by more than 2^8 takes 5-7 % less time, but
+// then the rows of a wave decide on each other's rounding, and a training pass over 32768 tokens and 7 layers moves the final
+// norm's gradient, elements of some 300 times the overall rms, by 0.7 %.)
+// Measured (12 query heads on 2 key heads), register-staged tiles, one workgroup's waves in step -> this: 25 sequences of 1133
+// tokens 177 -> 151 us, 2 of 300 15.0 -> 11.5 us, 24576 tokens 2.13 -> 1.86 ms (873 -> 998 TFLOP/s); 3 x 8192 (28 on 4
+// heads) 1.94 -> 1.62 ms.
 // =====================================================================================
 __global__ __launch_bounds__(256, 2) void flash_fwd_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf16_t* __restrict__ v,
@@ -81,19 +83,12 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_kernel(
 #pragma unroll
     for (int s = 0; s < 8; ++s) qf[s] = ld8(qp + s * 16);
   }
-  if (scale_log2 < 0.f) {
-#pragma unroll
-    for (int s = 0; s < 8; ++s)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) qf[s][j] = -qf[s][j];
-  }
-  const float c = fmaxf(fabsf(scale_log2), 1e-30f);  // a scale of zero: every score counts as (almost) zero
   f32x16 oacc[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
     for (int j = 0; j < 16; ++j) oacc[i][j] = 0.f;
-  float m = -INFINITY, mc = 0.f, l = 0.f;  // reference maximum of the raw scores, times c; sum of this lane's keys
+  float m = -INFINITY, l = 0.f;  // maximum of the scaled scores; sum of this lane's keys
 
   // number of kv tiles this block needs (the whole block walks the same range)
   int k_hi = k_len;
@@ -135,40 +130,48 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_kernel(
       }
     }
     // ---- online softmax; lane holds q row `my_q`, keys (reg&3)+8(reg>>2)+4hf of each block
-    float mx = -INFINITY;
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        if (decltype(masked)::value) {
-          const int key = kbase + 32 * kb + (j & 3) + 8 * (j >> 2) + 4 * hf;
-          sacc[kb][j] = key >= k_len || (causal && key > my_q + shift) ? -INFINITY : sacc[kb][j];
-        }
-        mx = fmaxf(mx, sacc[kb][j]);
-      }
-    mx = max_xor32(mx);
-    if (__any(mx * c - mc > 8.f || m == -INFINITY)) {
-      const float mn = fmaxf(m, mx), mnc = mn == -INFINITY ? 0.f : mn * c;
-      const float alpha = m == -INFINITY ? 0.f : fast_exp2(mc - mnc);
-      m = mn;
-      mc = mnc;
-      l *= alpha;
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 16; ++j) oacc[i][j] *= alpha;
-    }
-    float ls = 0.f;
+    float mx = -INFINITY, ls = 0.f;
     bf16x8 pf[4];
+    {
+#pragma clang fp contract(off)
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
+      for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        const float pr = fast_exp2(__builtin_fmaf(sacc[kb][j], c, -mc));
-        ls += pr;
-        pf[2 * kb + (j >> 3)][j & 7] = f2bf(pr);
+        for (int j = 0; j < 16; ++j) {
+          sacc[kb][j] *= scale_log2;
+          if (decltype(masked)::value) {
+            const int key = kbase + 32 * kb + (j & 3) + 8 * (j >> 2) + 4 * hf;
+            sacc[kb][j] = key >= k_len || (causal && key > my_q + shift) ? -INFINITY : sacc[kb][j];
+          }
+          mx = fmaxf(mx, sacc[kb][j]);
+        }
+      mx = max_xor32(mx);
+      const float mn = fmaxf(m, mx);
+      const float alpha = mn == -INFINITY ? 1.f : fast_exp2(m - mn);  // m = -inf -> 0
+      m = mn;
+      if (__any(m == -INFINITY)) {  // rows that have seen no key yet: probabilities of zero
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+          for (int j = 0; j < 16; ++j) sacc[kb][j] = m == -INFINITY ? -INFINITY : sacc[kb][j];
       }
-    l += ls;
+      const float ms = m == -INFINITY ? 0.f : m;
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+          const float pr = fast_exp2(sacc[kb][j] - ms);
+          ls += pr;
+          pf[2 * kb + (j >> 3)][j & 7] = f2bf(pr);
+        }
+      l = __builtin_fmaf(l, alpha, ls);
+      if (__any(alpha != 1.f)) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int j = 0; j < 16; ++j) oacc[i][j] *= alpha;
+      }
+    }
     // ---- O^T[d, q] += V^T[d, keys] . P^T[keys, q]
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
@@ -216,9 +219,11 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_kernel(
         for (int j = 0; j < 4; ++j) w[j] = f2bf(oacc[db][4 * g + j] * inv_l);
         *reinterpret_cast<bf16x4*>(op + 32 * db + 8 * g + 4 * hf) = w;
       }
-    if (hf == 0 && lse)
+    if (hf == 0 && lse) {
+#pragma clang fp contract(off)
       lse[(size_t)head * total_q + q_beg + my_q] =
-          (l > 0.f) ? (mc * 0.6931471805599453f + __logf(l)) : -INFINITY;
+          (l > 0.f) ? (m * 0.6931471805599453f + __logf(l)) : -INFINITY;
+    }
   }
 }
 

@@ -75,3 +75,20 @@ def test_scores_that_keep_growing_are_rescaled():
         ref, ref_lse = A.attention_varlen_ref(q.double(), k.double(), v.double(), cu, cu, scale)
         assert float((out.float() - ref).abs().max()) < 2e-2
         assert float((lse - ref_lse).abs().max()) < 2e-3 * max(1.0, float(ref_lse.abs().max()))
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("T,row", [(64, 40), (130, 3), (700, 333), (1200, 1199)])
+def test_a_row_depends_on_its_own_query_only(T, row, causal):
+    """Bit for bit the same output and log-sum-exp whatever the other queries of its tile are."""
+    g = torch.Generator(device=DEV).manual_seed(T)
+    q, k, v = (torch.randn(T, h, 128, device=DEV, generator=g).bfloat16() for h in (4, 2, 2))
+    cu = torch.tensor([0, T], dtype=torch.int32, device=DEV)
+    got = []
+    for size in (0.0, 1.0, 12.0):  # neighbours whose maxima stand still, drift, and jump from tile to tile
+        other = (torch.randn(T, 4, 128, device=DEV, generator=g) * size).bfloat16()
+        other[row] = q[row]
+        out, lse = ops.flash_attn_varlen(other, k, v, cu, cu, T, causal=causal)
+        got.append((out[row], lse[:, row]))
+    for out, lse in got[1:]:
+        assert torch.equal(out, got[0][0]) and torch.equal(lse, got[0][1])
