@@ -424,7 +424,8 @@ class ModelRunner:
                 qkv = blk.attn.project_qkv(x).view(T, hq + 2 * hkv, D)
                 ops.rope_and_cache_write_(qkv, pos, slots, rope, kc, vc, hq, hkv)
                 attn, _ = ops.flash_attn_varlen(qkv[:, :hq], qkv[:, hq:hq + hkv], qkv[:, hq + hkv:], cu_q, cu_q, max_q)
-            slab = dg.dgemm(attn.view(T, hq * D), blk.attn.o, epilogue=dg.EPI_SLAB)
+            # (padded heads come back as a slice of wider rows)
+            slab = dg.dgemm(attn.reshape(T, hq * D), blk.attn.o, epilogue=dg.EPI_SLAB)
             x, residual = finish(slab, residual, blk.ln2)
             nw = layers[li + 1].ln1 if li + 1 < len(layers) else None
             if cfg.n_experts > 0:

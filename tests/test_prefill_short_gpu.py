@@ -63,6 +63,20 @@ def test_split_keys(q_lens, k_lens, hq, hkv, fp8, monkeypatch):
 @pytest.mark.parametrize("new,prefix,kv", [([1], [0], None), ([1], [37], None), ([93], [200], None), ([40, 7, 130], [0, 64, 9], None),
                                            ([512], [0], None), ([93], [200], "fp8"), ([50], [0], "fp8")])
 def test_layers(model, new, prefix, kv):
+    _both_paths(model, new, prefix, kv)
+
+
+# heads that attention pads to 128 or 256 and hands back as a slice, and heads of 256
+@pytest.mark.parametrize("model,heads,fused", [
+    ("dense", dict(n_q_heads=14, n_kv_heads=2, head_dim=64), True), ("qk_norm", dict(n_q_heads=4, n_kv_heads=2, head_dim=64), True),
+    ("dense", dict(n_q_heads=2, n_kv_heads=1, head_dim=96), True), ("dense", dict(n_q_heads=2, n_kv_heads=1, head_dim=256), True)])
+@pytest.mark.parametrize("new,prefix,kv", [([93], [200], None), ([40, 7, 130], [0, 64, 9], None), ([50, 3], [0, 0], None),
+                                           ([93], [200], "fp8")])
+def test_layers_of_other_heads(model, heads, fused, new, prefix, kv):
+    _both_paths(model, new, prefix, kv, fused, **heads)
+
+
+def _both_paths(model, new, prefix, kv, fused=True, **heads):
     from areal_vllm_amd.inference.model_runner import ModelRunner
     from areal_vllm_amd.models.config import ModelConfig
     from areal_vllm_amd.models.transformer import Transformer
@@ -73,7 +87,7 @@ def test_layers(model, new, prefix, kv):
     extra = {"dense": dict(family="qwen2", qkv_bias=True),
              "qk_norm": dict(family="qwen3", qk_norm=True),
              "experts": dict(family="qwen3_moe", qk_norm=True, n_experts=8, n_experts_per_tok=2, moe_intermediate_size=128)}
-    cfg = ModelConfig(**base, **extra[model])
+    cfg = ModelConfig(**{**base, **heads}, **extra[model])
     m = Transformer(cfg, dtype=torch.bfloat16, device=torch.device(DEV))
     m.requires_grad_(False)
     m.eval()
@@ -87,6 +101,7 @@ def test_layers(model, new, prefix, kv):
         r = ModelRunner(m, num_pages=64, max_context=1024, max_batch=4,
                         kv_dtype=torch.float8_e4m3fn if kv else torch.bfloat16)
         r.PREFILL_FUSED_MAX_ROWS = limit
+        assert r._prefill_fused(sum(new)) == (limit > 0 and fused)
         g = torch.Generator(device=DEV).manual_seed(1)
         for pair in r.kv:
             for t in pair:
