@@ -382,8 +382,12 @@ class ModelRunner:
     PREFILL_FUSED_MAX_ROWS = 512
 
     def _prefill_fused(self, rows: int) -> bool:
+        from ..ops import decode_gemm as dg
+
+        D = self.cfg.head_dim
         return (0 < rows <= self.PREFILL_FUSED_MAX_ROWS and self.fused_decode and self.dtype == torch.bfloat16
-                and (self.hq + 2 * self.hkv) * self.cfg.head_dim % 32 == 0)
+                and (self.hq + 2 * self.hkv) * D % 32 == 0
+                and dg.rope_row_supported(self.hq, self.hkv, D, self.cfg.qk_norm))
 
     def _prefill_layers_fused(self, h, pos, slots, rope, cu_q, cu_k, bt, max_q):
         """The layers of a prefill of few tokens on the decode step's GEMMs and row kernels (`_decode_layers_fused`)."""

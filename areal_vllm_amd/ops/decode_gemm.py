@@ -245,6 +245,14 @@ def splitk_residual_rmsnorm(slab: torch.Tensor, n_split: int, M: int, N: int, *,
     return out, res_out
 
 
+def rope_row_supported(n_q_heads: int, n_kv_heads: int, head_dim: int, qk_norm: bool) -> bool:
+    """Whether :func:`splitk_rope_cache_write` takes such rows: a row's fp32 sums in 64 KB of LDS; with norms, the lanes of
+    a head (16 values each) a power of two within a wave."""
+    lanes = head_dim // 16
+    return (head_dim % 16 == 0 and (n_q_heads + 2 * n_kv_heads) * head_dim <= 16384
+            and (not qk_norm or (lanes <= 64 and lanes & (lanes - 1) == 0)))
+
+
 def splitk_rope_cache_write(slab: torch.Tensor, n_split: int, bias: Optional[torch.Tensor], positions, slots, table,
                             kcache, vcache, n_q_heads: int, n_kv_heads: int, head_dim: int,
                             q_out: Optional[torch.Tensor] = None, do_rope: bool = True, dtype=torch.bfloat16,

@@ -66,10 +66,13 @@ def test_layers(model, new, prefix, kv):
     _both_paths(model, new, prefix, kv)
 
 
-# heads that attention pads to 128 or 256 and hands back as a slice, and heads of 256
+# heads that attention pads to 128 or 256 and hands back as a slice, heads of 256, and rows and norms that the decode step's
+# row kernels do not take
 @pytest.mark.parametrize("model,heads,fused", [
     ("dense", dict(n_q_heads=14, n_kv_heads=2, head_dim=64), True), ("qk_norm", dict(n_q_heads=4, n_kv_heads=2, head_dim=64), True),
-    ("dense", dict(n_q_heads=2, n_kv_heads=1, head_dim=96), True), ("dense", dict(n_q_heads=2, n_kv_heads=1, head_dim=256), True)])
+    ("dense", dict(n_q_heads=2, n_kv_heads=1, head_dim=96), True), ("dense", dict(n_q_heads=2, n_kv_heads=1, head_dim=256), True),
+    ("qk_norm", dict(n_q_heads=2, n_kv_heads=1, head_dim=96), False),
+    ("dense", dict(n_q_heads=120, n_kv_heads=8, head_dim=128), False)])
 @pytest.mark.parametrize("new,prefix,kv", [([93], [200], None), ([40, 7, 130], [0, 64, 9], None), ([50, 3], [0, 0], None),
                                            ([93], [200], "fp8")])
 def test_layers_of_other_heads(model, heads, fused, new, prefix, kv):
