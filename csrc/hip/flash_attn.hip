@@ -234,8 +234,8 @@ extern "C" int areal_flash_fwd_d256(const void* q, const void* k, const void* v,
                                     float softmax_scale, int causal, hipStream_t st);
 extern "C" int areal_flash_bwd_d256(const void* q, const void* k, const void* v, const void* o, const void* d_o,
                                     const float* lse, float* delta, void* dq, void* dk, void* dv, const int* cu_q,
-                                    const int* cu_k, int B, int max_k, int total_q, int Hq, int Hkv, int64_t q_stride,
-                                    int64_t k_stride, int64_t v_stride, int64_t o_stride, int64_t do_stride,
+                                    const int* cu_k, int B, int max_k, int total_q, int64_t total_k, int Hq, int Hkv,
+                                    int64_t q_stride, int64_t k_stride, int64_t v_stride, int64_t o_stride, int64_t do_stride,
                                     int64_t dq_stride, int64_t dk_stride, int64_t dv_stride, float softmax_scale,
                                     int causal, hipStream_t st);
 
@@ -262,7 +262,7 @@ extern "C" int areal_flash_fwd(const void* q, const void* k, const void* v, void
 
 // =====================================================================================
 // Backward.
-//  pre : delta[h, t] = sum_d dO[t, h, d] * O[t, h, d], and the log-sum-exp in base 2
+//  pre : delta[h, t] = sum_d dO[t, h, d] * O[t, h, d], and the log-sum-exp in base 2; gradients of rows of no sequence
 //  dkv : workgroups of 128 keys sweep the query slices that see them
 //  dq  : workgroups of 128 queries walk their keys
 // Seven products instead of the five that one kernel needs, but nothing is handed over: with dQ added up by fp32 atomics
@@ -274,14 +274,15 @@ extern "C" int areal_flash_fwd(const void* q, const void* k, const void* v, void
 // =====================================================================================
 __global__ __launch_bounds__(256) void flash_bwd_delta_kernel(
     const bf16_t* __restrict__ o, const bf16_t* __restrict__ d_o, const float* __restrict__ lse,
-    float* __restrict__ delta, int64_t o_stride, int64_t do_stride, int Hq, int total_q) {
+    float* __restrict__ delta, int64_t o_stride, int64_t do_stride, int Hq, int total_q, const FlashGrads grads) {
   constexpr int D = 128;
   // 16 lanes per (token, head)
   const int64_t idx = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 4;
   const int sub = threadIdx.x & 15;
-  if (idx >= (int64_t)total_q * Hq) return;
   const int64_t t = idx / Hq;
   const int h = (int)(idx % Hq);
+  flash_zero_uncovered(grads, t, h, D, sub * 8);
+  if (t >= total_q) return;
   bf16x8 a = ld8(o + t * o_stride + (size_t)h * D + sub * 8);
   bf16x8 bb = ld8(d_o + t * do_stride + (size_t)h * D + sub * 8);
   float s = 0.f;
@@ -685,23 +686,25 @@ extern "C" int areal_flash_bwd(const void* q, const void* k, const void* v, cons
                                int64_t o_stride, int64_t do_stride, int64_t dq_stride,
                                int64_t dk_stride, int64_t dv_stride, float softmax_scale, int causal,
                                hipStream_t st) {
-  if (B == 0 || total_q == 0) return 0;
+  if (total_q == 0) return 0;
   if (D != 128 && D != 256) return -1;
   if (Hq % Hkv != 0) return -2;
   if ((q_stride | k_stride | v_stride | o_stride | do_stride | dq_stride | dk_stride | dv_stride) % 8)
     return -3;
   if (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)d_o) % 16 != 0) return -4;
   if (D == 256)
-    return areal_flash_bwd_d256(q, k, v, o, d_o, lse, delta, dq, dk, dv, cu_q, cu_k, B, max_k, total_q, Hq, Hkv,
+    return areal_flash_bwd_d256(q, k, v, o, d_o, lse, delta, dq, dk, dv, cu_q, cu_k, B, max_k, total_q, total_k, Hq, Hkv,
                                 q_stride, k_stride, v_stride, o_stride, do_stride, dq_stride, dk_stride, dv_stride,
                                 softmax_scale, causal, st);
   {
-    const int64_t n = (int64_t)total_q * Hq * 16;
+    const FlashGrads grads{(bf16_t*)dq, (bf16_t*)dk, (bf16_t*)dv, dq_stride, dk_stride, dv_stride, total_q, total_k, cu_q, cu_k, B, Hkv};
+    const int64_t n = (total_q > total_k ? total_q : total_k) * Hq * 16;
     hipLaunchKernelGGL(flash_bwd_delta_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st,
-                       (const bf16_t*)o, (const bf16_t*)d_o, lse, delta, o_stride, do_stride, Hq, total_q);
+                       (const bf16_t*)o, (const bf16_t*)d_o, lse, delta, o_stride, do_stride, Hq, total_q, grads);
   }
   const int G = Hq / Hkv, hs = (G + parts - 1) / parts;
   if (parts < 1 || parts > G || (parts > 1 && part == nullptr)) return -6;
+  if (B == 0 || max_q == 0 || max_k == 0) return (int)hipGetLastError();  // no sequences, or none with rows
   const unsigned kblocks = (unsigned)((max_k + 127) / 128);
   hipLaunchKernelGGL(flash_bwd_dkv_kernel, dim3(kblocks * Hkv * B * parts), dim3(256), 0, st, (const bf16_t*)q,
                      (const bf16_t*)k, (const bf16_t*)v, (const bf16_t*)d_o, delta, (bf16_t*)dk, (bf16_t*)dv, part, cu_q,

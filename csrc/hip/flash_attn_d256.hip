@@ -204,16 +204,17 @@ __global__ __launch_bounds__(256, 1) void flash_fwd_d256_kernel(
 
 // =====================================================================================
 // Backward.
-//  pre : delta[h, t] = sum_d dO[t, h, d] * O[t, h, d], 32 lanes per (token, head)
+//  pre : delta[h, t] = sum_d dO[t, h, d] * O[t, h, d], 32 lanes per (token, head); gradients of rows of no sequence
 // =====================================================================================
 __global__ __launch_bounds__(256) void flash_bwd_delta_d256_kernel(
     const bf16_t* __restrict__ o, const bf16_t* __restrict__ d_o, float* __restrict__ delta,
-    int64_t o_stride, int64_t do_stride, int Hq, int total_q) {
+    int64_t o_stride, int64_t do_stride, int Hq, int total_q, const FlashGrads grads) {
   const int64_t idx = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 5;
   const int sub = threadIdx.x & 31;
-  if (idx >= (int64_t)total_q * Hq) return;
   const int64_t t = idx / Hq;
   const int h = (int)(idx % Hq);
+  flash_zero_uncovered(grads, t, h, D, sub * 8);
+  if (t >= total_q) return;
   bf16x8 a = ld8(o + t * o_stride + (size_t)h * D + sub * 8);
   bf16x8 bb = ld8(d_o + t * do_stride + (size_t)h * D + sub * 8);
   float s = 0.f;
@@ -553,8 +554,8 @@ extern "C" int areal_flash_fwd_d256(const void* q, const void* k, const void* v,
 
 extern "C" int areal_flash_bwd_d256(const void* q, const void* k, const void* v, const void* o, const void* d_o,
                                     const float* lse, float* delta, void* dq, void* dk, void* dv, const int* cu_q,
-                                    const int* cu_k, int B, int max_k, int total_q, int Hq, int Hkv, int64_t q_stride,
-                                    int64_t k_stride, int64_t v_stride, int64_t o_stride, int64_t do_stride,
+                                    const int* cu_k, int B, int max_k, int total_q, int64_t total_k, int Hq, int Hkv,
+                                    int64_t q_stride, int64_t k_stride, int64_t v_stride, int64_t o_stride, int64_t do_stride,
                                     int64_t dq_stride, int64_t dk_stride, int64_t dv_stride, float softmax_scale,
                                     int causal, hipStream_t st) {
   static bool attr_set = false;
@@ -563,10 +564,12 @@ extern "C" int areal_flash_bwd_d256(const void* q, const void* k, const void* v,
     attr_set = true;
   }
   {
-    const int64_t n = (int64_t)total_q * Hq * 32;
+    const FlashGrads grads{(bf16_t*)dq, (bf16_t*)dk, (bf16_t*)dv, dq_stride, dk_stride, dv_stride, total_q, total_k, cu_q, cu_k, B, Hkv};
+    const int64_t n = (total_q > total_k ? total_q : total_k) * Hq * 32;
     hipLaunchKernelGGL(flash_bwd_delta_d256_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st,
-                       (const bf16_t*)o, (const bf16_t*)d_o, delta, o_stride, do_stride, Hq, total_q);
+                       (const bf16_t*)o, (const bf16_t*)d_o, delta, o_stride, do_stride, Hq, total_q, grads);
   }
+  if (B == 0 || max_k == 0) return (int)hipGetLastError();  // no sequences, or none with rows
   dim3 block(256);
   dim3 kgrid((unsigned)(((max_k + 127) / 128) * Hkv * B * 2));
   hipLaunchKernelGGL(flash_bwd_dkdv_d256_kernel, kgrid, block, 0, st, (const bf16_t*)q, (const bf16_t*)k,

@@ -44,6 +44,24 @@ DEVINL void lds_row_write(char* tile, int row, int ch, bf16x8 v) {
   *reinterpret_cast<bf16x8*>(tile + swz_off(row, ch)) = v;
 }
 
+// ---- gradients of rows that belong to no sequence: zero. A backward's first kernel visits every (token t, head h), `at`: the
+// 8 values of a head that this lane is responsible for.
+struct FlashGrads {
+  bf16_t *dq, *dk, *dv;
+  int64_t dq_stride, dk_stride, dv_stride, total_q, total_k;
+  const int *cu_q, *cu_k;
+  int nbatch, Hkv;
+};
+DEVINL void flash_zero_uncovered(const FlashGrads& g, int64_t t, int h, int D, int at) {
+  const bf16x8 zero = {};
+  const size_t col = (size_t)h * D + at;
+  if (t < g.total_q && (t < g.cu_q[0] || t >= g.cu_q[g.nbatch])) st8(g.dq + t * g.dq_stride + col, zero);
+  if (h < g.Hkv && t < g.total_k && (t < g.cu_k[0] || t >= g.cu_k[g.nbatch])) {
+    st8(g.dk + t * g.dk_stride + col, zero);
+    st8(g.dv + t * g.dv_stride + col, zero);
+  }
+}
+
 // ---- staging of 64-row tiles by LDS-DMA. One wave instruction (16 bytes a lane) fills four consecutive 256-byte rows of a
 // tile linearly; the swizzle sits on the source address: lane -> row (lane >> 4) of the four, physical chunk lane & 15.
 typedef const __attribute__((address_space(1))) void* dma_gptr_t;

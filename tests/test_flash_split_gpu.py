@@ -92,3 +92,37 @@ def test_a_row_depends_on_its_own_query_only(T, row, causal):
         got.append((out[row], lse[:, row]))
     for out, lse in got[1:]:
         assert torch.equal(out, got[0][0]) and torch.equal(lse, got[0][1])
+
+
+@pytest.mark.parametrize("D", [128, 256])
+@pytest.mark.parametrize("n", [300, 3000])
+def test_rows_of_no_sequence_get_zero_gradients(D, n):
+    g = torch.Generator(device=DEV).manual_seed(n)
+    lead, tail, Hq, Hkv = 5, 140, 4, 2
+    T = lead + n + tail
+    qkv = torch.randn(T, Hq + 2 * Hkv, D, device=DEV, generator=g).bfloat16()
+    d = torch.randn(T, Hq, D, device=DEV, generator=g).bfloat16()
+    cu = torch.tensor([lead, lead + n // 3, lead + n], dtype=torch.int32, device=DEV)
+    none = torch.ones(T, dtype=torch.bool, device=DEV)
+    none[lead:lead + n] = False
+
+    def fresh():  # what is allocated next holds NaN
+        for shape in ((T, Hq + 2 * Hkv, D), (T, Hq, D), (T, Hkv, D), (T, Hkv, D)):
+            torch.full(shape, math.nan, dtype=torch.bfloat16, device=DEV)
+
+    grads = []
+    for x in (qkv, qkv[lead:lead + n]):  # with the rows of no sequence, and without them
+        x = x.clone().requires_grad_()
+        o = 0 if x.shape[0] == T else lead
+        y = ops.flash_attn_varlen_qkv(x, cu - o, n, Hq, Hkv)
+        fresh()
+        grads.append(torch.autograd.grad(y, x, d[o:o + y.shape[0]])[0])
+    assert bool((grads[0][none] == 0).all()) and torch.equal(grads[0][~none], grads[1])
+
+    q, k, v = (t.contiguous().requires_grad_() for t in qkv.split([Hq, Hkv, Hkv], 1))
+    more = torch.cat([k.detach(), k.detach()]).requires_grad_()  # more keys than queries, the second half of no sequence
+    y = ops.flash_attn_varlen_sep(q, more, torch.cat([v, v]), cu, cu, n, n)
+    fresh()
+    dq, dk = torch.autograd.grad(y, (q, more), d)
+    assert bool((dq[none] == 0).all()) and bool((dk[:T][none] == 0).all()) and bool((dk[T:] == 0).all())
+    assert torch.equal(dq[~none], grads[1][:, :Hq]) and torch.equal(dk[:T][~none], grads[1][:, Hq:Hq + Hkv])
