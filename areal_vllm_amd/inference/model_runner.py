@@ -520,11 +520,22 @@ class ModelRunner:
     def _decode_workspace(self, Bp: int):
         """(key-range splits, split workspace) of the decode attention at this batch bucket, for attention that does
         not run on work items."""
-        return 1, None
+        D = self.cfg.head_dim
+        if self.device.type != "cuda" or D <= self.ITEMS_MAX_HEAD:
+            return 1, None
+        nsplit = ops.decode_num_splits(Bp, self.hkv, 4096, fp8=ops.attention.is_fp8(self.kv[0][0]))
+        return nsplit, (ops.DecodeWorkspace(Bp, self.hq, D, nsplit, self.device) if nsplit > 1 else None)
+
+    # Largest head size whose decode attention runs on work items. Heads of 256 (one workgroup a CU, and four times the
+    # values for the workgroup that combines a row) gain by them only in ragged batches of many rows; one split count for all
+    # rows and a second launch, and items, 8 query heads on one key head: 4 rows of 8000 tokens 18 and 33 us a layer, 16 of
+    # 4000 20 and 29, 24 of 200-4096 20 and 26, 24 of 20000 94 and 122, 128 of 2000-6000 115 and 120, 200 of 500-5000 144 and
+    # 116. Heads of 128 and 64: ``csrc/hip/paged_attn.hip``.
+    ITEMS_MAX_HEAD = 128
 
     def _decode_items(self, Bp: int) -> Optional["ops.DecodeItems"]:
         """Work items of the decode attention, laid out anew in every step and shared by its layers."""
-        if self.device.type != "cuda":
+        if self.device.type != "cuda" or self.cfg.head_dim > self.ITEMS_MAX_HEAD:
             return None
         return ops.DecodeItems(Bp, self.hq, self.hkv, self.cfg.head_dim, self.device,
                                max_context=self.max_pages * PAGE_SIZE)
@@ -643,7 +654,8 @@ class ModelRunner:
                                                self.rope, kc, vc, hq, hkv, D, dtype=self.dtype,
                                                q_norm=blk.attn.q_norm if cfg.qk_norm else None,
                                                k_norm=blk.attn.k_norm if cfg.qk_norm else None, norm_eps=eps)
-            attn = ops.paged_attention_decode(q, kc, vc, st["block_tables"], st["context_lens"], items=st["items"])
+            attn = ops.paged_attention_decode(q, kc, vc, st["block_tables"], st["context_lens"], nsplit=st["nsplit"],
+                                              workspace=st["ws"], items=st["items"])
             slab = dg.dgemm(attn.view(Bp, hq * D), blk.attn.o, epilogue=dg.EPI_SLAB)
             x, residual = finish(slab, residual, blk.ln2)
             nw = layers[li + 1].ln1 if li + 1 < len(layers) else self.model.norm
@@ -694,7 +706,8 @@ class ModelRunner:
             kc, vc = self.kv[li]
             q = sk.norm_qkv_rope(residual, blk.ln1, blk.attn.qkv, blk.attn.qkv_bias, rope_pos, st["slots"], self.rope, kc,
                                  vc, hq, hkv, D, eps=eps, gemma=gemma)
-            attn = ops.paged_attention_decode(q, kc, vc, st["block_tables"], st["context_lens"], items=st["items"])
+            attn = ops.paged_attention_decode(q, kc, vc, st["block_tables"], st["context_lens"], nsplit=st["nsplit"],
+                                              workspace=st["ws"], items=st["items"])
             residual = sk.linear_residual(attn.view(Bp, hq * D), blk.attn.o, residual)
             a = sk.norm_gated(residual, blk.ln2, blk.mlp.gate_up, eps=eps, gemma=gemma, act=act)
             residual = sk.linear_residual(a, blk.mlp.down, residual)
@@ -773,7 +786,8 @@ class ModelRunner:
                 qkv = qkv2d.view(Bp, hq + 2 * hkv, D)
                 ops.rope_and_cache_write_(qkv, rope_pos, st["slots"], self.rope, kc, vc, hq, hkv)
                 return ops.paged_attention_decode(qkv[:, :hq], kc, vc, st["block_tables"], st["context_lens"],
-                                                  q_row_stride=qkv_stride, items=st["items"])
+                                                  nsplit=st["nsplit"], workspace=st["ws"], q_row_stride=qkv_stride,
+                                                  items=st["items"])
 
             h, residual = self._layer(blk, h, residual, st["positions"], st["slots"], attn_fn)
         return self._final_logits(h, residual)
