@@ -480,8 +480,8 @@ class DecodeItems:
         self.batch, self.n_q_heads, self.n_kv_heads, self.head_dim = batch, n_q_heads, n_kv_heads, head_dim
         self.target = max(1, DECODE_ITEMS // n_kv_heads)
         pages = None if max_context is None else -(-int(max_context) // PAGE_SIZE)
-        # twice the items where shares of 32 pages and items 1.4 times as long can occur
-        self.finer = pages is None or (pages > 44 and batch * pages > 31 * self.target)
+        # twice the items where shares of 32 pages can occur
+        self.finer = pages is None or batch * pages > 31 * self.target
         self.n_items = self.target * (2 if self.finer else 1) + batch
         if pages is not None:  # a row of n pages is at most sqrt(3 n) items
             self.n_items = min(self.n_items, batch * (math.isqrt(3 * pages) + 1))

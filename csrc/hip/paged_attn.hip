@@ -335,11 +335,15 @@ struct DecodeItem { int b, p_beg, p_end, base, n, part, pad0, pad1; };
 // many that the workgroup that combines a row's n partial results does not read longer than the others walk:
 // n^2 <= 3 pages (1 x 16000 tokens: 16.3 us, 22.4 us with n^2 <= 5 pages of 4-page items).
 constexpr int STEP = 4;
-// Even share from which the number of items may double (paged_decode_items_kernel). 8 steps of 14 layers, two key heads:
-// 60 rows of 3000-9000 tokens 17.8 -> 15.7 ms, 90 of 2000-7000 21.3 -> 18.3; equal
-// rows, whose items are level, lose by it (100 rows of 6000: 21.0 -> 22.5), and so do short items (5 rows of 4000-16000:
-// 7.9 -> 8.4).
-constexpr int FINER_EVEN = 32;
+// The number of items doubles (paged_decode_items_kernel) where one of them would be 1.4 times the even share, or where there
+// are more of them than CUs for a key head (`target`) but not twice as many: then some CUs get two items of a whole share each
+// and the others one. Shares below 32, respectively 40 pages never double: the combination costs more than it evens out.
+// Over 335 batches (1 to 384 rows, equal and ragged lengths to 24000, bf16 and fp8, 1 to 8 key heads of 64 and 128) the layout
+// that this picks takes 0.5 % more than the better one, at most 14 %; the first condition alone 2.1 % and 36 %. us a layer,
+// one split count for all rows / items / items doubled, 12 query heads on 2: 48 equal rows of 6000 tokens 62 / 73 / 58 (144 items
+// on 128 CUs), 80 of 6000 106 / 109 / 91, 60 of 3000-9000 87 / 103 / 73, 90 of 2000-7000 116 / 112 / 84; not doubled: 100 of
+// 6000 111 / 105 / 122 (1.28 times the share), 16 of 12000 41 / 40 / 43, 8 of 4000-16000 23 / 20 / 23 (shares of 16).
+constexpr int FINER_EVEN = 32, FINER_COUNT_EVEN = 40;
 DEVINL int pages_per_item(int np, int even) {
   const int most = max(1, (int)sqrtf(3.f * (float)np));
   const int n = min(most, max(1, (np + even / 2) / even));
@@ -353,7 +357,7 @@ __global__ __launch_bounds__(1024) void paged_decode_items_kernel(const int* __r
                                                                   DecodeItem* __restrict__ items, int B, int target,
                                                                   int n_items, int finer) {
   constexpr int NB = 64;  // size classes of the sort
-  __shared__ int red[16], hist[NB];
+  __shared__ int red[16], red_n[16], hist[NB];
   const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
   int pages = 0;
   for (int b = t; b < B; b += 1024) pages += (max(context_lens[b], 0) + PAGE - 1) / PAGE;
@@ -366,18 +370,29 @@ __global__ __launch_bounds__(1024) void paged_decode_items_kernel(const int* __r
 #pragma unroll
   for (int w = 0; w < 16; ++w) total += red[w];
   int even = max(STEP, (total + target - 1) / target);
-  if (finer && even >= FINER_EVEN) {  // long items: where a row's rounding makes one of them 1.4 times the even share, twice as many
-    int longest = 0;
-    for (int b = t; b < B; b += 1024)
-      longest = max(longest, pages_per_item((max(context_lens[b], 0) + PAGE - 1) / PAGE, even));
+  if (finer && even >= FINER_EVEN) {
+    int longest = 0, count = 0;
+    for (int b = t; b < B; b += 1024) {
+      const int np = (max(context_lens[b], 0) + PAGE - 1) / PAGE, per = pages_per_item(np, even);
+      longest = max(longest, per);
+      count += max(1, (np + per - 1) / per);
+    }
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) longest = max(longest, __shfl_xor(longest, o, 64));
+    for (int o = 32; o > 0; o >>= 1) {
+      longest = max(longest, __shfl_xor(longest, o, 64));
+      count += __shfl_xor(count, o, 64);
+    }
     __syncthreads();
-    if (lane == 0) red[wid] = longest;
+    if (lane == 0) { red[wid] = longest; red_n[wid] = count; }
     __syncthreads();
+    count = 0;
 #pragma unroll
-    for (int w = 0; w < 16; ++w) longest = max(longest, red[w]);
-    if (5 * longest > 7 * even) even = max(STEP, (total + 2 * target - 1) / (2 * target));
+    for (int w = 0; w < 16; ++w) {
+      longest = max(longest, red[w]);
+      count += red_n[w];
+    }
+    if (5 * longest > 7 * even || (even >= FINER_COUNT_EVEN && count > target && count <= 2 * target))
+      even = max(STEP, (total + 2 * target - 1) / (2 * target));
     __syncthreads();
   }
   const int top = even + even / 2 + STEP;  // an item has more pages only if its row may not be divided further
