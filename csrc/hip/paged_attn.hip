@@ -15,6 +15,8 @@
 // head (GQA group, zero padded). The two 16-key S^T tiles of a page take the keys
 // {8c+r} and {8c+4+r} (c = lane>>4, r = 0..3) so that each lane ends up holding P for keys
 // 8c..8c+7, which is exactly the B-operand order of the P.V product.
+#include <type_traits>
+
 #include "common.hpp"
 
 #define PAGE 32
@@ -344,8 +346,9 @@ constexpr int STEP = 4;
 // on 128 CUs), 80 of 6000 106 / 109 / 91, 60 of 3000-9000 87 / 103 / 73, 90 of 2000-7000 116 / 112 / 84; not doubled: 100 of
 // 6000 111 / 105 / 122 (1.28 times the share), 16 of 12000 41 / 40 / 43, 8 of 4000-16000 23 / 20 / 23 (shares of 16).
 constexpr int FINER_EVEN = 32, FINER_COUNT_EVEN = 40;
+constexpr int MAX_ROW_ITEMS = 256;  // (reached at 699000 tokens) their (m, l) fit the LDS that the waves' results need, 8 (64 + 4) floats a head
 DEVINL int pages_per_item(int np, int even) {
-  const int most = max(1, (int)sqrtf(3.f * (float)np));
+  const int most = min(MAX_ROW_ITEMS, max(1, (int)sqrtf(3.f * (float)np)));
   const int n = min(most, max(1, (np + even / 2) / even));
   const int per = (np + n - 1) / n;
   return max(STEP, (per + STEP - 1) / STEP * STEP);
@@ -458,9 +461,10 @@ DEVINL float ld_agent(const float* p) {
 // block: NW waves, page by page in turn. part_o: [n_items, Hq, D], part_ml: [n_items, Hq, 2],
 // arrived: [B, Hkv] zeros, zeros again afterwards. The last workgroup of a row to arrive combines its partial results
 // in the order of the items: the result does not depend on the order of arrival.
-// LDS holds the G real query rows only: 8 workgroups of a GQA group of 6 fit a CU (the padded 16 rows: 4).
+// LDS holds the G real query rows only. Two workgroups of 8 waves a CU (128 registers a lane; heads of 64 three, of 256 one
+// of 4 waves): the register file sets that, a GQA group of 6 heads of 128 takes 26 KB of LDS.
 template <int D, bool FP8, int NW>
-__global__ __launch_bounds__(64 * NW, (D > 128 ? 1 : 2)) void paged_decode_walk_kernel(
+__global__ __launch_bounds__(64 * NW, (D > 128 ? 1 : 4)) void paged_decode_walk_kernel(
     const bf16_t* __restrict__ q, const void* __restrict__ kcache, const void* __restrict__ vcache,
     const int* __restrict__ block_tables, const int* __restrict__ context_lens, const DecodeItem* __restrict__ items,
     bf16_t* __restrict__ out, float* __restrict__ part_o, float* __restrict__ part_ml, int* __restrict__ arrived, int Hq,
@@ -624,36 +628,58 @@ __global__ __launch_bounds__(64 * NW, (D > 128 ? 1 : 2)) void paged_decode_walk_
   }
   __syncthreads();
   if (!last) return;
-  for (int idx = threadIdx.x; idx < G * D; idx += 64 * NW) {
-    const int head = h * G + idx / D, d = idx % D;
-    const float* ml = part_ml + ((size_t)it.base * Hq + head) * 2;
-    const float* po = part_o + ((size_t)it.base * Hq + head) * D + d;
-    float mm = -INFINITY, acc = 0.f, ll = 0.f;
-    for (int s0 = 0; s0 < it.n; s0 += 8) {  // eight partial results in flight
-      float ms[8], ls[8], os[8];
+  // (m, l) of the row's items, [n][G][2], in the place of the waves' results; then U values a thread and eight items of
+  // each in flight: ceil(n / 8) round trips past the L2. With one value at a time and its own (m, l) they were ceil(G D / threads)
+  // times as many: 12 heads on 2, 2 rows of 24000 tokens 21.6 us a layer and 19.8 now, 8 of 8000 18.2 and 17.7; 32 on 4, 2 rows
+  // of 1000-24000 20.8 and 18.9; 16 on one, 8 of 4000-16000 27.5 and 23.9.
+  float* mls = smem;
+  const size_t row0 = (size_t)it.base * Hq + h * G;
+  for (int i = threadIdx.x; i < it.n * 2 * G; i += 64 * NW) mls[i] = ld_agent(part_ml + (row0 + (size_t)(i / (2 * G)) * Hq) * 2 + i % (2 * G));
+  __syncthreads();
+  auto combine = [&](auto u_c) {
+    constexpr int U = decltype(u_c)::value;
+    for (int i0 = threadIdx.x; i0 < G * D; i0 += U * 64 * NW) {
+      float mm[U], acc[U], ll[U];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const size_t s = min(s0 + j, it.n - 1);
-        ms[j] = s0 + j < it.n ? ld_agent(ml + s * Hq * 2) : -INFINITY;
-        ls[j] = ld_agent(ml + s * Hq * 2 + 1);
-        os[j] = ld_agent(po + s * Hq * D);
+      for (int u = 0; u < U; ++u) { mm[u] = -INFINITY; acc[u] = 0.f; ll[u] = 0.f; }
+      for (int s0 = 0; s0 < it.n; s0 += 8) {
+        float os[U][8];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+          for (int j = 0; j < 8; ++j)
+            os[u][j] = ld_agent(part_o + (row0 + (size_t)min(s0 + j, it.n - 1) * Hq) * D + min(i0 + u * 64 * NW, G * D - 1));
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const float* ml = mls + min(i0 + u * 64 * NW, G * D - 1) / D * 2;
+          float ms[8], mn = mm[u];
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            ms[j] = s0 + j < it.n ? ml[(s0 + j) * 2 * G] : -INFINITY;
+            mn = fmaxf(mn, ms[j]);
+          }
+          const float f0 = mm[u] == -INFINITY ? 0.f : fast_exp2(mm[u] - mn);
+          acc[u] *= f0;
+          ll[u] *= f0;
+          mm[u] = mn;
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            const float f = ms[j] == -INFINITY ? 0.f : fast_exp2(ms[j] - mn);
+            acc[u] += os[u][j] * f;
+            ll[u] += ml[min(s0 + j, it.n - 1) * 2 * G + 1] * f;
+          }
+        }
       }
-      float mn = mm;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) mn = fmaxf(mn, ms[j]);
-      const float f0 = mm == -INFINITY ? 0.f : fast_exp2(mm - mn);
-      acc *= f0;
-      ll *= f0;
-      mm = mn;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float f = ms[j] == -INFINITY ? 0.f : fast_exp2(ms[j] - mn);
-        acc += os[j] * f;
-        ll += ls[j] * f;
-      }
+      for (int u = 0; u < U; ++u)
+        if (i0 + u * 64 * NW < G * D)
+          out[((size_t)b * Hq + h * G) * D + i0 + u * 64 * NW] = f2bf(ll[u] > 0.f ? acc[u] / ll[u] : 0.f);
     }
-    out[((size_t)b * Hq + head) * D + d] = f2bf(ll > 0.f ? acc / ll : 0.f);
+  };
+  if constexpr (16 * D > 2 * 64 * NW) {
+    if (G * D > 2 * 64 * NW) return combine(std::integral_constant<int, 4>{});
   }
+  combine(std::integral_constant<int, 2>{});
 }
 
 // Items of the batch's decode attention; `items`: n_items x 8 ints, at least min(target + B, B x most items of a row); with finer 2 target + B.
