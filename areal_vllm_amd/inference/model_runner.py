@@ -520,22 +520,25 @@ class ModelRunner:
     def _decode_workspace(self, Bp: int):
         """(key-range splits, split workspace) of the decode attention at this batch bucket, for attention that does
         not run on work items."""
-        D = self.cfg.head_dim
-        if self.device.type != "cuda" or D <= self.ITEMS_MAX_HEAD:
+        if self.device.type != "cuda" or self._on_items(Bp):
             return 1, None
         nsplit = ops.decode_num_splits(Bp, self.hkv, 4096, fp8=ops.attention.is_fp8(self.kv[0][0]))
-        return nsplit, (ops.DecodeWorkspace(Bp, self.hq, D, nsplit, self.device) if nsplit > 1 else None)
+        return nsplit, (ops.DecodeWorkspace(Bp, self.hq, self.cfg.head_dim, nsplit, self.device) if nsplit > 1 else None)
 
-    # Largest head size whose decode attention runs on work items. Heads of 256 (one workgroup a CU, and four times the
-    # values for the workgroup that combines a row) gain by them only in ragged batches of many rows; one split count for all
-    # rows and a second launch, and items, 8 query heads on one key head: 4 rows of 8000 tokens 18 and 33 us a layer, 16 of
-    # 4000 20 and 29, 24 of 200-4096 20 and 26, 24 of 20000 94 and 122, 128 of 2000-6000 115 and 120, 200 of 500-5000 144 and
-    # 116. Heads of 128 and 64: ``csrc/hip/paged_attn.hip``.
-    ITEMS_MAX_HEAD = 128
+    def _on_items(self, Bp: int) -> bool:
+        """Whether the decode attention of so many rows runs on work items. One workgroup combines a row's partial results: with
+        more than 1024 values a key head (two a thread) and few rows it becomes the longest part, and one split count for all
+        rows with a second launch is faster, with heads of 256 (one workgroup a CU) also for equal rows. us a layer, split and
+        items: 16 heads of 128 on one key head, 2 rows of 24000 tokens 20 and 23, 8 of 4000-16000 18 and 24, 16 of 2000-16000
+        26 and 26, 24 of 4000-12000 30 and 26, 64 of 1000-8000 45 and 37; 8 of 256 on one, 4 rows of 8000 18 and 26, 24 of 20000
+        91 and 102, 100 of 6000 110 and 119, 24 of 4000-12000 50 and 50, 200 of 500-5000 141 and 108; 8 of 256 on 4, 4 rows of
+        1000-24000 33 and 25, 32 of 8000 177 and 179. Fewer values: ``csrc/hip/paged_attn.hip``."""
+        D = self.cfg.head_dim
+        return self.hq // self.hkv * D <= 1024 or (D <= 128 and Bp * self.hkv > 16)
 
     def _decode_items(self, Bp: int) -> Optional["ops.DecodeItems"]:
         """Work items of the decode attention, laid out anew in every step and shared by its layers."""
-        if self.device.type != "cuda" or self.cfg.head_dim > self.ITEMS_MAX_HEAD:
+        if self.device.type != "cuda" or not self._on_items(Bp):
             return None
         return ops.DecodeItems(Bp, self.hq, self.hkv, self.cfg.head_dim, self.device,
                                max_context=self.max_pages * PAGE_SIZE)

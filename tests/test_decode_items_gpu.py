@@ -62,26 +62,29 @@ def test_decode_attention_on_items(Hq, Hkv, D, fp8, ctx):
     assert int(items.arrived.abs().sum()) == 0
 
 
-@pytest.mark.parametrize("head_dim,kv", [(64, None), (128, None), (256, None), (256, A.FP8)])
-def test_runner_chooses_items_by_head_size(head_dim, kv):
-    """Heads of 256 decode on key ranges of one count for all rows, smaller ones on items; both equal attention in fp32."""
+@pytest.mark.parametrize("Hq,Hkv,head_dim,kv,rows,on_items", [
+    (4, 1, 64, None, 4, True), (16, 1, 64, None, 4, True), (8, 1, 128, None, 4, True), (16, 1, 128, None, 4, False),
+    (16, 1, 128, None, 17, True), (18, 2, 128, A.FP8, 8, False), (18, 2, 128, None, 9, True), (4, 1, 256, None, 4, True),
+    (8, 1, 256, None, 4, False), (8, 1, 256, A.FP8, 20, False)])
+def test_runner_chooses_items_by_values_a_key_head(Hq, Hkv, head_dim, kv, rows, on_items):
+    """Items, or key ranges of one count for all rows where a row has many values to combine; both equal attention in fp32."""
     from areal_vllm_amd.inference.model_runner import ModelRunner
     from areal_vllm_amd.models.config import ModelConfig
     from areal_vllm_amd.models.transformer import Transformer
 
-    cfg = ModelConfig(family="llama", vocab_size=256, hidden_size=256, n_layers=1, n_q_heads=4, n_kv_heads=1, head_dim=head_dim,
-                      intermediate_size=256, max_position_embeddings=4096)
+    cfg = ModelConfig(family="llama", vocab_size=256, hidden_size=256, n_layers=1, n_q_heads=Hq, n_kv_heads=Hkv,
+                      head_dim=head_dim, intermediate_size=256, max_position_embeddings=4096)
     model = Transformer(cfg, dtype=torch.bfloat16, device=torch.device(DEV))
     model.requires_grad_(False)
     model.flatten()
-    ctx = [1, 33, 700, 2000]
-    q, kc, vc, bt, cl = _setup(ctx, 4, 1, head_dim, kv is not None, 5)
-    r = ModelRunner(model, kc.shape[0], 2048, len(ctx), buckets=[len(ctx)], kv_dtype=kv)
-    st = r._alloc_static(len(ctx))
-    assert (st["items"] is None) == (head_dim == 256) and (st["ws"] is not None) == (head_dim == 256)
-    d = [t.to(DEV) for t in (q[:, :4].contiguous(), kc, vc, bt, cl)]
+    ctx = [(1, 33, 700, 2000)[i % 4] for i in range(rows)]
+    q, kc, vc, bt, cl = _setup(ctx, Hq, Hkv, head_dim, kv is not None, 5)
+    r = ModelRunner(model, kc.shape[0], 2048, rows, buckets=[rows], kv_dtype=kv)
+    st = r._alloc_static(rows)
+    assert (st["items"] is not None) == on_items and (st["ws"] is None) == on_items
+    d = [t.to(DEV) for t in (q[:, :Hq].contiguous(), kc, vc, bt, cl)]
     if st["items"] is not None:
         st["items"].fill_(d[4])
     got = ops.paged_attention_decode(*d, nsplit=st["nsplit"], workspace=st["ws"], items=st["items"]).float().cpu()
-    ref = A.paged_decode_ref(q[:, :4], kc, vc, bt, cl, 1 / math.sqrt(head_dim)).float()
+    ref = A.paged_decode_ref(q[:, :Hq], kc, vc, bt, cl, 1 / math.sqrt(head_dim)).float()
     assert (got - ref).abs().max() < 2e-2
