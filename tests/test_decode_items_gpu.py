@@ -60,6 +60,9 @@ def test_decode_attention_on_items(Hq, Hkv, D, fp8, ctx):
     assert (outs[0] - ref).abs().max() < 2e-2
     assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])  # counters are back at zero, order is fixed
     assert int(items.arrived.abs().sum()) == 0
+    # the form with a bounded context, as a runner allocates it: its own layout is the same, and so is every bit
+    got = ops.paged_attention_decode(d[0][:, :Hq], *d[1:], q_row_stride=(Hq + 1) * D, items=tight).float().cpu()
+    assert torch.equal(got, outs[0])
 
 
 @pytest.mark.parametrize("Hq,Hkv,head_dim,kv,rows,on_items", [
