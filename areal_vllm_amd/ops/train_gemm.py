@@ -59,6 +59,8 @@ def wgrad_supported(dy: torch.Tensor, x: torch.Tensor, acc: torch.Tensor) -> boo
         return False
     if dy.stride(1) != 1 or x.stride(1) != 1 or acc.stride(1) != 1 or dy.stride(0) % 8 or x.stride(0) % 8:
         return False
+    if dy.stride(0) < N or x.stride(0) < K:  # repeated or overlapping rows: the end of the operand is told from a row's place
+        return False
     return dy.data_ptr() % 16 == 0 and x.data_ptr() % 16 == 0
 
 

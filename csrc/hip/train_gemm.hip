@@ -825,6 +825,7 @@ extern "C" int areal_tgemm_wgrad(const void* dY, long ldy, const void* X, long l
                                  int K, int splits, int stagger, hipStream_t st) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   if (N % 128 != 0 || K % 256 != 0 || ldy % 8 != 0 || ldx % 8 != 0) return -1;
+  if (ldy < N || ldx < K) return -1;  // the loads end at the last row's last byte: rows must not overlap
   if (((uintptr_t)dY | (uintptr_t)X) % 16 != 0 || (uintptr_t)dW % 4 != 0) return -1;
   const int tiles = ((N + 255) / 256) * (K / 256), pairs = (M + 127) / 128;
   // splits >= 1: that many workgroups per tile (1 = every tile added without atomics). splits <= 0: choose. Blocks run

@@ -25,3 +25,25 @@ def test_ragged_token_counts(M, N, K, splits):
     want = base.double() + dy.double().t() @ x.double()
     # fp32 sums of M products of size one: 2^-24 sqrt(M) relative per addition, far below 1e-3
     assert float((got.double() - want).abs().max()) < 1e-3 * max(1.0, M ** 0.5 / 16)
+
+
+@pytest.mark.parametrize("M,N,K", [(256, 128, 256), (700, 384, 512)])
+@pytest.mark.parametrize("which", ["dy", "x", "overlapping"])
+def test_rows_that_repeat(M, N, K, which):
+    """An output gradient that is the same for all rows (of a mean over them), an input broadcast over them, rows that overlap."""
+    from areal_vllm_amd.ops.linear import _accumulate_wgrad
+
+    g = torch.Generator(device=DEV).manual_seed(M)
+    dy, x = (torch.randn(M, n, device=DEV, generator=g).bfloat16() for n in (N, K))
+    if which == "dy":
+        dy = dy[:1].expand(M, N)
+    elif which == "x":
+        x = x[:1].expand(M, K)
+    else:
+        dy = torch.randn(M * 64 + N, device=DEV, generator=g).bfloat16().as_strided((M, N), (64, 1))
+    w = torch.nn.Parameter(torch.zeros(N, K, device=DEV).bfloat16())
+    w.main_grad = torch.zeros(N, K, device=DEV)
+    _accumulate_wgrad(w, dy, x)
+    want = dy.double().contiguous().t() @ x.double().contiguous()
+    # fp32 sums of M products of size one, the same M times over where rows repeat
+    assert float((w.main_grad.double() - want).abs().max()) < 1e-5 * M
