@@ -46,6 +46,9 @@ def tgemm_tn(a: torch.Tensor, b: torch.Tensor, bias: Optional[torch.Tensor] = No
     return out
 
 
+MAX_ROW_STRIDE = 1 << 24  # elements: byte offsets inside 64 rows of an operand fit 32 bits
+
+
 def wgrad_supported(dy: torch.Tensor, x: torch.Tensor, acc: torch.Tensor) -> bool:
     if not OWN_WGRAD:
         return False
@@ -60,6 +63,8 @@ def wgrad_supported(dy: torch.Tensor, x: torch.Tensor, acc: torch.Tensor) -> boo
     if dy.stride(1) != 1 or x.stride(1) != 1 or acc.stride(1) != 1 or dy.stride(0) % 8 or x.stride(0) % 8:
         return False
     if dy.stride(0) < N or x.stride(0) < K:  # repeated or overlapping rows: the end of the operand is told from a row's place
+        return False
+    if dy.stride(0) > MAX_ROW_STRIDE or x.stride(0) > MAX_ROW_STRIDE:
         return False
     return dy.data_ptr() % 16 == 0 and x.data_ptr() % 16 == 0
 
@@ -91,7 +96,7 @@ def dgrad_supported(dy: torch.Tensor, w: torch.Tensor) -> bool:
         return False
     if dy.stride(1) != 1 or w.stride(1) != 1 or dy.stride(0) % 8 or w.stride(0) % 8:
         return False
-    if not (R <= dy.stride(0) <= 1 << 22 and w.shape[1] <= w.stride(0) <= 1 << 24):
+    if not (R <= dy.stride(0) <= 1 << 22 and w.shape[1] <= w.stride(0) <= MAX_ROW_STRIDE):  # (256 rows of dy)
         return False
     return dy.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
 

@@ -826,6 +826,7 @@ extern "C" int areal_tgemm_wgrad(const void* dY, long ldy, const void* X, long l
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   if (N % 128 != 0 || K % 256 != 0 || ldy % 8 != 0 || ldx % 8 != 0) return -1;
   if (ldy < N || ldx < K) return -1;  // the loads end at the last row's last byte: rows must not overlap
+  if (ldy > (1l << 24) || ldx > (1l << 24)) return -1;  // byte offsets of 64 rows: 32 bits
   if (((uintptr_t)dY | (uintptr_t)X) % 16 != 0 || (uintptr_t)dW % 4 != 0) return -1;
   const int tiles = ((N + 255) / 256) * (K / 256), pairs = (M + 127) / 128;
   // splits >= 1: that many workgroups per tile (1 = every tile added without atomics). splits <= 0: choose. Blocks run
@@ -884,7 +885,7 @@ extern "C" int areal_tgemm_wgrad(const void* dY, long ldy, const void* X, long l
 }
 
 // dX[M, C] = dY[M, R] . W[R, C]; R a multiple of 128, C of 256, rows 16-byte aligned. part: splits x M x C floats, unused for
-// one part. Every part has work as long as splits <= R / 128 and is the number areal_tgemm_nn_splits returns.
+// one part. Every part has to have work: with P = R / 128, ceil(P / ceil(P / splits)) == splits (12 pairs in 5 parts are 4).
 extern "C" int areal_tgemm_nn(const void* dY, long ldy, const void* W, long ldw, void* dX, long ldx, float* part, int splits,
                               int M, int R, int C, hipStream_t st) {
   if (M <= 0 || R <= 0 || C <= 0) return R <= 0 && M > 0 && C > 0 ? -1 : 0;
