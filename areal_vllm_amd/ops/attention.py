@@ -161,7 +161,13 @@ def _strides(t: torch.Tensor) -> int:
     return t.stride(0)
 
 
+def _near_rows(t: torch.Tensor) -> torch.Tensor:
+    """The kernels take 32-bit byte offsets inside 64 rows: rows further apart than 2^24 elements are copied."""
+    return t if t.stride(0) <= 1 << 24 else t.clone(memory_format=torch.contiguous_format)
+
+
 def _flash_fwd_hip(q, k, v, cu_q, cu_k, max_q, scale, causal) -> Tuple[torch.Tensor, torch.Tensor]:
+    q, k, v = _near_rows(q), _near_rows(k), _near_rows(v)
     Tq, Hq, D = q.shape
     Hkv = k.shape[1]
     assert q.dtype == torch.bfloat16 and cu_q.dtype == torch.int32 and cu_k.dtype == torch.int32
@@ -193,6 +199,7 @@ def flash_bwd_parts(total_k: int, max_k: int, n_q_heads: int, n_kv_heads: int) -
 
 
 def _flash_bwd_hip(q, k, v, out, dout, lse, dq, dk, dv, cu_q, cu_k, max_q, max_k, scale, causal):
+    q, k, v = _near_rows(q), _near_rows(k), _near_rows(v)
     Tq, Hq, D = q.shape
     Hkv = k.shape[1]
     B = cu_q.numel() - 1

@@ -248,6 +248,7 @@ extern "C" int areal_flash_fwd(const void* q, const void* k, const void* v, void
   if (D != 128 && D != 256) return -1;
   if (Hq % Hkv != 0) return -2;
   if ((q_stride | k_stride | v_stride | o_stride) % 8 != 0) return -3;
+  if (k_stride > FLASH_MAX_STRIDE || v_stride > FLASH_MAX_STRIDE) return -5;
   if (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)o) % 16 != 0) return -4;
   if (D == 256)
     return areal_flash_fwd_d256(q, k, v, o, lse, cu_q, cu_k, B, max_q, total_q, Hq, Hkv, q_stride, k_stride, v_stride,
@@ -692,6 +693,7 @@ extern "C" int areal_flash_bwd(const void* q, const void* k, const void* v, cons
   if ((q_stride | k_stride | v_stride | o_stride | do_stride | dq_stride | dk_stride | dv_stride) % 8)
     return -3;
   if (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)d_o) % 16 != 0) return -4;
+  if (q_stride > FLASH_MAX_STRIDE || k_stride > FLASH_MAX_STRIDE || v_stride > FLASH_MAX_STRIDE || do_stride > FLASH_MAX_STRIDE) return -5;
   if (D == 256)
     return areal_flash_bwd_d256(q, k, v, o, d_o, lse, delta, dq, dk, dv, cu_q, cu_k, B, max_k, total_q, total_k, Hq, Hkv,
                                 q_stride, k_stride, v_stride, o_stride, do_stride, dq_stride, dk_stride, dv_stride,

@@ -71,6 +71,7 @@ DEVINL void dma16(const void* src, void* lds) {
 }
 // Rows 16 w + 4 i + (lane >> 4), i = 0..3, of a tile of 64 rows go through wave w of four. `off`: this lane's byte offsets of
 // the four pieces for rows `stride` elements apart.
+constexpr int64_t FLASH_MAX_STRIDE = 1 << 24;  // elements: the byte offsets of 64 rows fit 32 bits
 DEVINL void dma_offsets(unsigned (&off)[4], int wave, int lane, int64_t stride) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {

@@ -1,4 +1,4 @@
-"""Row strides that the weight-gradient GEMM's 32-bit offsets do not reach are refused, on the host, before any launch."""
+"""Row strides that 32-bit offsets do not reach are refused, on the host, before any launch."""
 from types import SimpleNamespace
 
 import pytest
@@ -24,3 +24,25 @@ def test_row_strides(ldy, ldx, taken):
         p = L.c_void_p(1 << 20)  # never read: the entry refuses the strides first
         assert L.lib().areal_tgemm_wgrad(p, L.c_int64(ldy), p, L.c_int64(ldx), p, L.c_int64(256), L.c_int(1024), L.c_int(128),
                                          L.c_int(256), L.c_int(0), L.c_int(1), L.c_void_p(0)) == -1
+
+
+@pytest.mark.parametrize("which", range(4))
+def test_flash_row_strides(which):
+    p, far = L.c_void_p(1 << 20), (1 << 24) + 8
+    st = [L.c_int64(far if i == which else 1536) for i in range(4)]  # q, k, v, dO
+    i, one, scale = L.c_int, L.c_int64(1536), L.c_float(1.0)
+    if which in (1, 2):  # the forward stages keys and values
+        assert L.lib().areal_flash_fwd(p, p, p, p, p, p, p, i(1), i(64), i(64), i(12), i(2), i(128), *st[:3], one, scale, i(1),
+                                       L.c_void_p(0)) == -5
+    assert L.lib().areal_flash_bwd(p, p, p, p, p, p, p, p, p, p, p, i(1), p, p, i(1), i(64), i(64), i(64), L.c_int64(64), i(12),
+                                   i(2), i(128), *st[:3], one, st[3], one, one, one, scale, i(1), L.c_void_p(0)) == -5
+
+
+def test_far_rows_are_copied():
+    from areal_vllm_amd.ops.attention import _near_rows
+
+    t = torch.arange(24.).view(3, 2, 4)
+    assert _near_rows(t) is t
+    far = torch.arange(8.).as_strided((1, 2, 4), ((1 << 24) + 8, 4, 1))
+    near = _near_rows(far)
+    assert near.stride(0) == 8 and torch.equal(near, far)
