@@ -19,8 +19,7 @@
 
 // Tile `id` (tiles of TM rows, numbered expert by expert) -> its expert, the tile's number there and the expert's rows;
 // false behind the last tile. A lane per expert: walking 128 experts one after the other is a chain of scalar loads ahead of
-// a workgroup's first tile (8 rows on 8 of 128 experts, 1536 columns,
-// 2048 deep: 34 us a launch, now 22).
+// a workgroup's first tile (7 rows on 128 experts, 1536 columns, 2048 deep: 30 us a launch, now 18).
 template <int TM>
 DEVINL bool gg_find_tile(const int* __restrict__ offsets, int E, int id, int& e, int& tile, int& row_lo, int& row_hi) {
   const int lane = threadIdx.x & 63;
@@ -77,8 +76,8 @@ __global__ __launch_bounds__(256) void grouped_gemm_nt_kernel(
 
   // cooperative loads: thread -> (row = tid >> 3 (+32 i), chunk = tid & 7). Rows past the expert's last token are not
   // fetched (their results are not stored): a decode step's expert has a handful of rows in a 64-row tile, and what the
-  // launch is bound by, a CU's load path, is then left to the weights. NT: weights that one tile reads once pass the caches
-  // by. 64 rows on 128 experts: gate|up (805 MB) 169 -> 145 us, down (403 MB) 73 -> 66.
+  // launch is bound by, a CU's load path, is then left to the weights. NT: the loads of weights pass the caches by (when: at
+  // the launch below).
   const int lrow = tid >> 3, lch = tid & 7;
   bf16x8 areg[KH * TM / 32] = {}, breg[KH * TN / 32];
   auto load = [&](int k0) {
@@ -184,14 +183,20 @@ extern "C" int areal_grouped_gemm_nt(const void* x, const void* w, void* out, co
     const char* e = getenv("AREAL_GROUPED_GEMM_KSTEP");
     return e && atoi(e) == 128;
   }();
+  // Weights past the caches: where most experts' rows are one tile, so that a weight is read once (up to 48 rows an expert on
+  // average: at 64 half of them are two), and where there is more than a workgroup for each of the 256 CUs: fewer wait for
+  // single loads, which are then slower. us from the caches / past them, cold weights: 128 experts, 1536 columns, 2048 deep,
+  // 7 rows 18 / 24, 32 31 / 31, 64 59 / 52, 512 164 / 149, 48 an expert 193 / 179, 64 212 / 240, 255 465 / 642; 8 experts,
+  // 14336 columns, 4096 deep, 1 row 32 / 48, 2 55 / 55, 4 87 / 77, 64 184 / 167; 16 of 704 columns, 1024 deep, 16 rows 9 / 12.
+  const bool stream = T <= 48l * E && (long)(T < E ? T : E) * (N / tn) > 256;
 #define AREAL_GG_LAUNCH(TM_, TN_, KH_, NT_)                                                                    \
-  hipLaunchKernelGGL((grouped_gemm_nt_kernel<TM_, TN_, KH_, NT_>), grid, block, 0, st, (const bf16_t*)x,      \
+  hipLaunchKernelGGL((grouped_gemm_nt_kernel<TM_, TN_, KH_, NT_>), grid, block, 0, st, (const bf16_t*)x,        \
                      (const bf16_t*)w, (bf16_t*)out, offsets, E, N, K, w_expert_stride)
   if (tm == 128 && tn == 128) {
     if (deep && K % 128 == 0) AREAL_GG_LAUNCH(128, 128, 2, false); else AREAL_GG_LAUNCH(128, 128, 1, false);
   } else if (tm == 128) AREAL_GG_LAUNCH(128, 64, 1, false);
-  else if (tn == 128) AREAL_GG_LAUNCH(64, 128, 1, true);
-  else AREAL_GG_LAUNCH(64, 64, 1, true);
+  else if (tn == 128) { if (stream) AREAL_GG_LAUNCH(64, 128, 1, true); else AREAL_GG_LAUNCH(64, 128, 1, false); }
+  else { if (stream) AREAL_GG_LAUNCH(64, 64, 1, true); else AREAL_GG_LAUNCH(64, 64, 1, false); }
 #undef AREAL_GG_LAUNCH
   return (int)hipGetLastError();
 }
