@@ -59,6 +59,27 @@ def test_split_keys(q_lens, k_lens, hq, hkv, fp8, monkeypatch):
         at += n
 
 
+@pytest.mark.parametrize("q_lens,k_lens", [([1], [1]), ([128], [128]), ([5, 64, 130], [5, 64, 131]), ([200, 3], [400, 33])])
+@pytest.mark.parametrize("splits", [2, 3, 5, 32])
+def test_ranges_without_keys(q_lens, k_lens, splits, monkeypatch):
+    """More ranges than some request has key tiles, whatever the rule would choose: the same as one range."""
+    g = torch.Generator().manual_seed(sum(k_lens))
+    kc, vc, bt, cu_q, cu_k = _paged(q_lens, k_lens, 2, False, g)
+    q = torch.randn(sum(q_lens), 12, 128, generator=g).bfloat16().to(DEV)
+    out = []
+    for n in (1, splits):
+        monkeypatch.setattr(A, "paged_prefill_splits", lambda *a: n)
+        out.append(ops.flash_attn_paged_prefill(q, kc, vc, bt, cu_q, cu_k, max(q_lens)).double())
+    # the same bf16 weights up to a factor, fp32 sums in another order, one rounding to bf16 of values up to 6
+    assert float((out[0] - out[1]).abs().max()) < 0.03
+
+
+def test_ranges_only_where_the_walk_is_long():
+    f = A.paged_prefill_splits
+    assert f(1, 12, 93, 928) > 1 and f(1, 12, 512, 8512) > 1 and f(1, 2, 1, 928) > 1
+    assert f(1, 32, 512, 512) == 1 and f(2, 32, 256, 256) == 1 and f(5, 12, 256, 320) == 1 and f(1, 12, 1, 32) == 1
+
+
 @pytest.mark.parametrize("model", ["dense", "qk_norm", "experts"])
 @pytest.mark.parametrize("new,prefix,kv", [([1], [0], None), ([1], [37], None), ([93], [200], None), ([40, 7, 130], [0, 64, 9], None),
                                            ([512], [0], None), ([93], [200], "fp8"), ([50], [0], "fp8")])
