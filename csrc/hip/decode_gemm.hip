@@ -109,8 +109,10 @@ __global__ __launch_bounds__(64 * (WM * WN + LW)) void dgemm_kernel(const DGArgs
   if (a.inv_z != 0) {
     // Three row blocks or more, of 128 rows at least. Ids are dealt round-robin to the 8 XCDs: each XCD takes a contiguous
     // range, row blocks first, then column tiles, so that a weight tile's row blocks meet in one L2 and a K slice of X is
-    // fetched by one or two L2s (320 rows x 1536 columns, 8960 deep: 23.2 -> 19.5 us). With fewer or smaller row blocks the
-    // launch order is as good or better (93 rows in 64-row blocks, 2048 columns, 1536 deep: 6.0 us, dealt this way 6.7).
+    // fetched by one or two L2s (320 rows x 1536 columns, 8960 deep: 22.4 -> 19.5 us; 17920 columns, 1536 deep 31.9 -> 30.5). With
+    // fewer or smaller row blocks, or reductions of up to 4096 to less than 8192 columns (all of X then fits every L2), the launch
+    // order is as good or better (93 rows in 64-row blocks, 2048 columns, 1536 deep: 6.0 us, dealt this way 6.7; 320 rows 9.4 and
+    // 9.8; 385 rows, 4608 columns, 3584 deep 50.8 and 53.4; 6144 columns, 4096 deep 43.2 and 43.3).
     const int nb = gridDim.x * gridDim.y * gridDim.z, q = nb >> 3, r = nb & 7;
     const int id = split + gridDim.x * (ct + gridDim.y * mb), x = id & 7;
     const int pos = (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + (id >> 3);
@@ -369,7 +371,7 @@ int launch_cfg(const DGArgs& a, int ksplit, hipStream_t st) {
   constexpr int cols_per_tile = (EPI == DG_SWIGLU || EPI == DG_ROPE) ? BN / 2 : BN;
   dim3 grid(ksplit, (ncols + cols_per_tile - 1) / cols_per_tile, (a.M + BM - 1) / BM);
   DGArgs b = a;
-  if (BM >= 128 && grid.z > 2 && grid.y > 1 && (uint64_t)grid.x * grid.y * grid.z < 65536) {
+  if (BM >= 128 && grid.z > 2 && grid.y > 1 && (a.K > 4096 || a.N >= 8192) && (uint64_t)grid.x * grid.y * grid.z < 65536) {
     b.inv_y = (unsigned)(((1ull << 32) + grid.y - 1) / grid.y);
     b.inv_z = (unsigned)(((1ull << 32) + grid.z - 1) / grid.z);
   }
