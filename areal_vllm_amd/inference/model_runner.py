@@ -378,14 +378,19 @@ class ModelRunner:
     # GEMMs and with these, one row behind 811 tokens of context: 28 layers of Qwen2-1.5B 32 / 93 / 256 / 512 tokens 5.84 /
     # 6.00 / 5.99 / 6.07 and 3.54 / 3.58 / 3.60 / 4.09 ms; 12 layers of Llama-3-8B 32 / 128 / 512 3.28 / 3.75 / 4.92 and
     # 2.30 / 2.80 / 4.65; 6 of Qwen2.5-7B 2.21 / 2.37 / 3.54 and 1.43 / 1.69 / 2.97; 4 of Qwen3-30B-A3B 2.08 / 2.27 / 2.55
-    # and 1.97 / 2.17 / 2.49.
-    PREFILL_FUSED_MAX_ROWS = 512
+    # and 1.97 / 2.17 / 2.49. Above a hidden size of 4096 two row blocks are bound by their products and the library's tiles win:
+    # 256 / 320 / 448 tokens behind 300, 2 layers of Llama-3-70B 1.98 / 1.79 / 2.11 and 1.42 / 2.32 / 2.48, 5 of Qwen2.5-14B 2.16 /
+    # 2.02 / 2.29 and 1.52 / 1.85 / 2.44; up to 4096 the worst is 4 % (6 layers of Llama-2-7B, 384: 2.02 and 2.10).
+    PREFILL_FUSED_MAX_ROWS, PREFILL_FUSED_MAX_ROWS_WIDE = 512, 256
 
     def _prefill_fused(self, rows: int) -> bool:
         from ..ops import decode_gemm as dg
 
         D = self.cfg.head_dim
-        return (0 < rows <= self.PREFILL_FUSED_MAX_ROWS and self.fused_decode and self.dtype == torch.bfloat16
+        most = self.PREFILL_FUSED_MAX_ROWS
+        if self.cfg.hidden_size > 4096:
+            most = min(most, self.PREFILL_FUSED_MAX_ROWS_WIDE)
+        return (0 < rows <= most and self.fused_decode and self.dtype == torch.bfloat16
                 and (self.hq + 2 * self.hkv) * D % 32 == 0
                 and dg.rope_row_supported(self.hq, self.hkv, D, self.cfg.qk_norm))
 
@@ -683,7 +688,10 @@ class ModelRunner:
     # Rows up to which the five-launch layer is faster than split-K GEMMs with row kernels, for hidden sizes up to 1536 and
     # above. 28 layers of Qwen2-1.5B at 1 / 2 / 4 / 6 / 8 rows: 1.17 / 1.24 / 1.36 / 1.45 / 1.50 ms a step against 1.44 / 1.44 /
     # 1.47 / 1.58 / 1.48; 12 layers of Llama-3-8B at 1 / 2 / 4: 1.47 / 1.55 / 1.65 against 1.66 / 1.66 / 1.58 (a row's weights
-    # no longer fit the registers at once, and the matrix-core form does not load ahead there).
+    # no longer fit the registers at once, and the matrix-core form does not load ahead there). Other sizes, hidden 896 (24 layers),
+    # 1 / 2 / 3 / 6 rows: 0.70 / 0.76 / 0.79 / 0.83 against 0.94 / 0.97 / 0.97 / 0.99; 2048 (10 layers) 0.58 / 0.61 / 0.67 / 0.71
+    # against 0.67 / 0.68 / 0.68 / 0.69; 1 / 2 rows of 3072 0.52 / 0.55 against 0.62 / 0.63, 3584 0.70 / 0.74 against 0.74 / 0.73, 5120
+    # (13824 inner) 0.70 / 0.74 against 0.76 / 0.73, 8192 0.75 / 0.77 against 0.89 / 0.87.
     SKINNY_MAX_ROWS, SKINNY_MAX_ROWS_WIDE = 6, 2
 
     def _skinny(self, rows: int) -> bool:
