@@ -80,3 +80,67 @@ def test_norm_qkv_rope(M, Hq, Hkv, D, K, fp8, with_bias):
     for a, b in zip(*caches):  # fp8: a value next to a rounding edge of 3 bits of mantissa may take the other one
         _close(a.float(), b.float().double(), bits=2 if fp8 else 5)
         assert torch.equal(a.float() != 0, b.float() != 0) or float(((a.float() != 0) != (b.float() != 0)).sum()) < 3
+
+
+@pytest.mark.parametrize("rows,hidden,inner,heads,extra", [
+    (1, 256, 512, (4, 2, 64), dict(family="qwen2", qkv_bias=True)), (2, 1536, 1024, (12, 2, 128), dict(family="qwen2", qkv_bias=True)),
+    (3, 256, 576, (4, 2, 128), dict(family="llama")), (6, 1536, 1024, (12, 2, 128), dict(family="qwen2", qkv_bias=True)),
+    (6, 256, 512, (2, 1, 256), dict(family="gemma", hidden_act="gelu_tanh", gemma_norm=True)),
+    (1, 2048, 1024, (16, 2, 128), dict(family="llama")), (2, 4096, 512, (8, 8, 128), dict(family="qwen2", qkv_bias=True))])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_layer_inside_the_runner(rows, hidden, inner, heads, extra, fp8):
+    """Captured decode plans of several steps on the five-launch layer and on split-K GEMMs with row kernels: logits, tokens and
+    what is written into the cache."""
+    import numpy as np
+
+    from areal_vllm_amd.inference.model_runner import ModelRunner
+    from areal_vllm_amd.models.config import ModelConfig
+    from areal_vllm_amd.models.transformer import Transformer
+
+    hq, hkv, D = heads
+    cfg = ModelConfig(vocab_size=512, hidden_size=hidden, n_layers=3, n_q_heads=hq, n_kv_heads=hkv, head_dim=D, intermediate_size=inner,
+                      max_position_embeddings=2048, tie_word_embeddings=True, **extra)
+    model = Transformer(cfg, dtype=torch.bfloat16, device=torch.device(DEV))
+    model.requires_grad_(False)
+    model.eval()
+    model.flatten()
+    g = torch.Generator(device=DEV).manual_seed(hidden + rows)
+    with torch.no_grad():
+        for n, p in model.named_parameters():
+            x = torch.randn(p.shape, device=DEV, generator=g)
+            if n == "embed":  # large beside what a layer adds: every row's next token is its own, whatever is rounded how
+                p.copy_(x * 0.5)
+            elif p.dim() > 1:
+                p.copy_(x * 0.5 / p.shape[1] ** 0.5)
+            else:
+                p.copy_(x * 0.1 + (0.0 if "bias" in n or extra.get("gemma_norm") else 1.0))
+    steps, ctx = 4, [5 + 61 * b for b in range(rows)]
+    width = (max(ctx) + steps) // 32 + 1
+    table = (np.random.RandomState(0).permutation(rows * width) + 1).reshape(rows, width).astype(np.int32)
+    pos = np.asarray(ctx, np.int32)
+    plan = dict(req_ids=list(range(rows)), temperature=np.zeros(rows, np.float32), top_p=np.ones(rows, np.float32),
+                top_k=np.full(rows, 1 << 30, np.int64), n_steps=steps, input_ids=np.arange(rows, dtype=np.int32) * 7 + 3, positions=pos,
+                context_lens=pos + 1, block_tables=table, max_pages=width,
+                slot_mapping=table[np.arange(rows), pos // 32].astype(np.int64) * 32 + pos % 32)
+    got = []
+    for five in (False, True):
+        r = ModelRunner(model, rows * width + 1, width * 32, rows, decode_steps=steps, buckets=[rows],
+                        **(dict(kv_dtype=torch.float8_e4m3fn) if fp8 else {}))
+        if not five:
+            r.SKINNY_MAX_ROWS = r.SKINNY_MAX_ROWS_WIDE = 0
+        assert r._skinny(rows) == five
+        gen = torch.Generator(device=DEV).manual_seed(1)
+        for pair in r.kv:
+            for t in pair:
+                t.copy_((torch.randn(t.shape, device=DEV, generator=gen) * 0.5).to(t.dtype))
+        r.keep_logits = True
+        for _ in range(2):  # captured by the first plan, replayed by the second
+            tokens, _ = r.decode(plan)
+        got.append((tokens.copy(), r.static[rows]["logits"].clone(), [t.float().clone() for pair in r.kv for t in pair]))
+    (ta, la, ca), (tb, lb, cb) = got
+    assert np.array_equal(ta, tb) and np.array_equal(ta[:, :rows], np.tile(plan["input_ids"], (steps, 1)))
+    # the same rounding points, sums in another order: three layers of bf16 steps (2^-8), as between the prefill's two layers
+    assert float((la - lb).abs().max()) < 0.06 * max(1.0, float(la.abs().max()))
+    step = 2.0 ** -3 if fp8 else 2.0 ** -6  # a step of the cache's type, a few roundings apart
+    for x, y in zip(ca, cb):
+        assert bool(((x - y).abs() <= 0.05 + step * x.abs()).all())
