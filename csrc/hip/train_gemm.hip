@@ -597,7 +597,6 @@ struct TNArgs {
   int pairs, chunk;  // 128-deep pairs of the reduction: of all of it, of one workgroup
 };
 
-template <bool STAGGER>
 __global__ __launch_bounds__(512) void tgemm_nn_kernel(const TNArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int lane = threadIdx.x & 63;
@@ -717,7 +716,7 @@ __global__ __launch_bounds__(512) void tgemm_nn_kernel(const TNArgs a) {
   stage(1, PB1, 1);
   tg_vmcnt<6>();
   tg_barrier();
-  if (STAGGER && wr == 1) tg_barrier();
+  if (wr == 1) tg_barrier();  // the second wave row runs one barrier behind
   int t = 0;
   for (; t + 2 < KT; t += 2) {
     tile(B0{}, t, T0{});
@@ -725,7 +724,7 @@ __global__ __launch_bounds__(512) void tgemm_nn_kernel(const TNArgs a) {
   }
   tile(B0{}, t, T1{});
   tile(B1{}, t + 1, T2{});
-  if (STAGGER && wr == 0) tg_barrier();
+  if (wr == 0) tg_barrier();
 
   // ---- lane (row r32, hf) holds columns (reg & 3) + 8 (reg >> 2) + 4 hf of each 32 x 32 tile
   auto put = [&](tw_acc& acc, int mh, int nh) __attribute__((always_inline)) {
@@ -902,10 +901,10 @@ extern "C" int areal_tgemm_nn(const void* dY, long ldy, const void* W, long ldw,
            (int)tiles, pairs, chunk};
   static bool attr_set = false;
   if (!attr_set) {
-    HIP_RET(hipFuncSetAttribute((const void*)tgemm_nn_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, TG_LDS));
+    HIP_RET(hipFuncSetAttribute((const void*)tgemm_nn_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, TG_LDS));
     attr_set = true;
   }
-  hipLaunchKernelGGL((tgemm_nn_kernel<true>), dim3((unsigned)(tiles * splits)), dim3(512), TG_LDS, st, a);
+  hipLaunchKernelGGL(tgemm_nn_kernel, dim3((unsigned)(tiles * splits)), dim3(512), TG_LDS, st, a);
   if (splits > 1)
     hipLaunchKernelGGL(tgemm_nn_sum_kernel, dim3((unsigned)(((size_t)M * C / 4 + 255) / 256)), dim3(256), 0, st, part, splits,
                        (bf16_t*)dX, ldx, M, C);
