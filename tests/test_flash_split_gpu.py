@@ -64,7 +64,7 @@ def test_parts_cover_the_heads():
 
 
 def test_scores_that_keep_growing_are_rescaled():
-    """Keys whose scores grow by a little per tile stay below the rescaling threshold, then pass it."""
+    """Keys whose scores grow from tile to tile, by a little and by much: every tile rescales what came before it."""
     T = 1024
     q = torch.ones(T, 2, 128, device=DEV).bfloat16()
     k = (torch.arange(T, device=DEV)[:, None, None] * 2e-3 * torch.ones(T, 1, 128, device=DEV)).bfloat16()
