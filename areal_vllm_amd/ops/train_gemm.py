@@ -4,8 +4,9 @@
 x transposed weight copy). The kernel covers the shapes transformer layers produce (K a multiple of 128, N of 4,
 16-byte aligned rows); `supported()` tells the caller when to keep the library GEMM instead - it is a statement
 about shapes, not a fallback for a missing extension (on a GPU the extension is mandatory)."""
+import functools
 import os
-from typing import Optional
+from typing import Optional, Tuple
 
 import torch
 
@@ -80,12 +81,26 @@ def tgemm_wgrad_(acc: torch.Tensor, dy: torch.Tensor, x: torch.Tensor, splits: i
     return acc
 
 
+@functools.lru_cache(maxsize=1024)
+def dgrad_cost(M: int, R: int, C: int) -> Tuple[float, int, int]:
+    """(time in 128-deep pairs, 3 us each; tiles of 256 x 256 that one workgroup reduces; parts of the reduction of each of the
+    others). A CU runs one workgroup: tiles beyond a multiple of 256 would leave CUs idle in a last round, so they are split
+    until the round is full. A part costs about 4 pairs more (its start, and its 256 KiB of fp32 written and read), the
+    kernel that sums the parts 2."""
+    pairs, tiles = R // 128, -(-M // 256) * (C // 256)
+    rounds, rest = divmod(tiles, 256)
+    best = (float(-(-tiles // 256) * pairs), tiles, 1)
+    if rest:
+        for s in range(2, min(pairs, 64) + 1):
+            chunk = -(-pairs // s)
+            if -(-pairs // chunk) == s:  # (every part has work)
+                cost = rounds * pairs + -(-rest * s // 256) * (chunk + 4) + 2 + 2 * s * rest / 256
+                best = min(best, (cost, rounds * 256, s))
+    return best
+
+
 def dgrad_splits(M: int, R: int, C: int) -> int:
-    """Parts of the reduction: about one workgroup a CU (256) over the 256 x 256 tiles, none of them empty."""
-    pairs = R // 128
-    tiles = -(-M // 256) * (C // 256)
-    splits = max(1, min(256 // tiles, pairs))
-    return -(-pairs // -(-pairs // splits))
+    return dgrad_cost(M, R, C)[2]
 
 
 def dgrad_supported(dy: torch.Tensor, w: torch.Tensor) -> bool:
@@ -105,31 +120,39 @@ def tgemm_nn(dy: torch.Tensor, w: torch.Tensor, splits: int = 0, out: Optional[t
     """dy[M, R] @ w[R, C] in bf16 with fp32 accumulation: the input gradient of ``y = x @ W^T`` from the weight as it lies."""
     assert dgrad_supported(dy, w)
     (M, R), C = dy.shape, w.shape[1]
-    splits = splits or dgrad_splits(M, R, C)
+    tiles = -(-M // 256) * (C // 256)
+    whole, splits = (0 if splits > 1 else tiles, splits) if splits else dgrad_cost(M, R, C)[1:]
     if out is None:
         out = torch.empty(M, C, dtype=torch.bfloat16, device=dy.device)
     assert out.shape == (M, C) and out.dtype == torch.bfloat16 and out.is_contiguous()
-    part = torch.empty(splits * M * C, dtype=torch.float32, device=dy.device) if splits > 1 else None
+    part = torch.empty(splits * (tiles - whole) << 16, dtype=torch.float32, device=dy.device) if splits > 1 else None
     L.check(L.lib().areal_tgemm_nn(L.ptr(dy), L.c_int64(dy.stride(0)), L.ptr(w), L.c_int64(w.stride(0)), L.ptr(out),
-                                   L.c_int64(C), L.ptr(part), L.c_int(splits), L.c_int(M), L.c_int(R), L.c_int(C),
-                                   L.stream_ptr()), "tgemm_nn")
+                                   L.c_int64(C), L.ptr(part), L.c_int(whole), L.c_int(splits), L.c_int(M), L.c_int(R),
+                                   L.c_int(C), L.stream_ptr()), "tgemm_nn")
     return out
 
 
-# Few rows and a deep reduction: the library then runs a few dozen workgroups. Its kernel and this one, us (parts): 17920 deep
-# to 1536 columns, 256 / 700 / 2048 / 3072 rows 102 / 130 / 204 / 218 and 36 (35) / 56 (14) / 109 (5) / 152 (3); 151936 to
-# 1536, 64 / 700 / 3072 rows 447 / 600 / 1938 and 105 / 291 / 1201; 28672 to 4096, 700 / 1536 rows 279 / 308 and 154 (5) /
-# 339 (2). From 4096 rows on or below three parts the two are level, and so they are (or the library is ahead: 1536 deep to
-# 8960 columns, 700 rows 26 and 39) where the reduction is short: 9728 deep 52 and 35, 5120 deep 34 and 35.
-DGRAD_MIN_DEPTH, DGRAD_MAX_ROWS, DGRAD_MIN_PARTS = 8192, 3072, 3
+# Own kernel / library, us (the weight as it lies; the library is 8 to 20 % slower in this layout than with a transposed copy).
+# Deep reductions, at any row count: 17920 deep to 1536 columns, 256 / 700 / 3000 / 12000 / 32768 rows 38 / 109, 55 / 133,
+# 173 / 222, 488 / 912, 1281 / 1324; 151936 to 1536, 256 / 700 / 6000 rows 144 / 466, 281 / 607, 2195 / 4089; 37888 to 3584,
+# 700 / 32768 rows 172 / 341, 6169 / 6466. Short ones: 1536 deep to 8960 columns, 700 / 1500 / 12000 / 32768 rows 38 / 33,
+# 41 / 49, 257 / 290, 682 / 755; 2048 to 4096, 1500 / 3000 / 32768 rows 46 / 33, 48 / 49, 386 / 439; 2048 to 1536, 700 / 6000 /
+# 12000 / 32768 rows 31 / 22, 46 / 42, 78 / 100, 148 / 161. So: a deep reduction, or rounds that are
+# filled to five eighths (384 tiles 16 pairs deep: 92 / 90; 288 tiles 8 deep, two rounds for 1.1: 53 / 49; 1536 deep to 1536, 144 tiles: 35 / 33).
+DGRAD_MIN_DEPTH, DGRAD_MIN_TILES, DGRAD_MAX_LOSS = 8192, 192, 1.6
+
+
+def _dgrad_own(M: int, R: int, C: int) -> bool:
+    tiles = -(-M // 256) * (C // 256)
+    return R >= DGRAD_MIN_DEPTH or (tiles >= DGRAD_MIN_TILES
+                                    and dgrad_cost(M, R, C)[0] <= DGRAD_MAX_LOSS * M * (C // 256) * (R // 128) / 65536)
 
 
 def dgrad(dy: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """dy @ w inside a backward pass (a library product where that pass is itself recorded)."""
     if (not torch.is_grad_enabled() and dgrad_supported(dy, w) and (out is None or out.is_contiguous() and out.data_ptr() % 8 == 0
                                                                     and out.dtype == torch.bfloat16)):
-        (M, R), C = dy.shape, w.shape[1]
-        if R >= DGRAD_MIN_DEPTH and M <= DGRAD_MAX_ROWS and dgrad_splits(M, R, C) >= DGRAD_MIN_PARTS:
+        if _dgrad_own(dy.shape[0], *w.shape):
             return tgemm_nn(dy, w, out=out)
     return torch.mm(dy, w) if out is None else torch.mm(dy, w, out=out)
 

@@ -52,11 +52,16 @@ struct TGArgs {
   const bf16_t* bias;
   int M, N, K;
   int tiles_m, tiles_n;
+  // NN: the tiles from `whole` on are reduced in `splits` parts of `chunk` 128-deep pairs each (the last one may get fewer);
+  // part [splits][tile - whole][256][256] fp32
+  float* part;
+  int whole, splits, chunk;
 };
 
 constexpr int TG_PIECE = 128 * 128;   // bytes of one staged piece
 constexpr int TG_BUF = 4 * TG_PIECE;  // A0 A1 B0 B1 of one K tile
 constexpr int TG_LDS = 2 * TG_BUF;
+constexpr int TG_OUT = 32 * 1024;  // the rest of the CU's 160 KiB: results on their way to whole lines
 enum { PA0 = 0, PA1 = 1, PB0 = 2, PB1 = 3 };
 constexpr int TG_GROUP_M = 4;
 
@@ -70,6 +75,15 @@ DEVINL void tg_barrier() {
   asm volatile("" ::: "memory");
 }
 
+// Transposed LDS read, from inline assembly: behind the builtin, hipcc cannot tell it from the pending LDS-DMA writes and puts
+// s_waitcnt vmcnt(0) in front of every group of reads, draining the pipeline. The results are ordered by the explicit lgkmcnt
+// waits of the phase.
+DEVINL bf16x4 tg_tr(uint32_t adr, int imm) {
+  bf16x4 v;
+  asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(v) : "v"(adr), "i"(imm));
+  return v;
+}
+
 typedef bf16x8 tg_bfrag[2][2];  // [n tile][k step]
 typedef f32x4 tg_acc[4][2];     // [m tile][n tile] of one quadrant
 
@@ -77,8 +91,17 @@ typedef f32x4 tg_acc[4][2];     // [m tile][n tile] of one quadrant
 // of width N each, C[M, N] = silu(A.gate^T) * (A.up^T); an output tile is 256 rows x 128 columns, its B pieces hold
 // the 128 gate rows (read in the phases of the first column half) and the 128 matching up rows (second half), so a
 // lane finds gate and up of the same output element in the same registers of the two accumulator quadrants.
-template <bool STAGGER, int EPI>
-__global__ __launch_bounds__(512) void tgemm_tn_kernel(const TGArgs a) {
+//
+// Result stores of the plain form. A lane of the MFMA result owns 4 consecutive columns of one row; stored from there, a wave
+// instruction touches 16 rows and hands the memory system quarter lines: the 1.17 GB of a 32768 x 17920 result cost 320 of
+// 1510 us (no stores at all: 1190). So a row half passes through the 32 KiB of LDS that the operand tiles leave free, a wave's
+// own 4 KiB at a time, and leaves as whole 128-byte lines: 1510 -> 1346 us, streamed past the caches (nontemporal) 1299;
+// 8192 x 151936 from 1536 deep 3287 -> 2801 us (library: 1294 and 3002). The waits of the stream do not matter: with counts
+// raised by the stores in flight, so that no wait stands behind one, the times are the same.
+// What is left is power: the matrix cores are busy 73 % of the time at a clock of 1.76 GHz (2.4 nominal); bare 16x16x32
+// products of random numbers run at 1.97 PFLOP/s on the whole chip, 32x32x16 ones at 1.75.
+template <bool STAGGER, int EPI, bool NN>
+__global__ __launch_bounds__(512) void tgemm_kernel(const TGArgs a) {
   constexpr int TN = EPI == 1 ? 128 : 256;  // output columns per tile
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int lane = threadIdx.x & 63;
@@ -86,10 +109,23 @@ __global__ __launch_bounds__(512) void tgemm_tn_kernel(const TGArgs a) {
   const int wr = wave >> 2, wc = wave & 3;
 
   // ---- tile sequence number -> output tile
-  const int ntiles = a.tiles_m * a.tiles_n;
-  auto tile_origin = [&](int id, int& m0, int& n0) __attribute__((always_inline)) {
-    const int q = ntiles >> 3, r = ntiles & 7, x = id & 7;
-    const int wg = (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + (id >> 3);
+  const int tiles = a.tiles_m * a.tiles_n, whole = NN ? a.whole : tiles;
+  const int ntiles = NN ? whole + (tiles - whole) * a.splits : tiles;  // work items
+  auto tile_origin = [&](int id, int& m0, int& n0, int& k0, int& kt, float*& part) __attribute__((always_inline)) {
+    const bool in_part = NN && id >= whole;
+    const int base = in_part ? whole : 0, nb = in_part ? ntiles - whole : whole;
+    const int q = nb >> 3, r = nb & 7, x = (id - base) & 7;
+    int wg = base + (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + ((id - base) >> 3);
+    k0 = 0;
+    kt = a.K >> 6;
+    part = nullptr;
+    if (in_part) {  // part by part: what runs together on an XCD shares the reduction range
+      const int rest = tiles - whole, split = (wg - whole) / rest;
+      part = a.part + ((size_t)(wg - whole) << 16);
+      wg -= split * rest;
+      k0 = split * a.chunk * 128;
+      kt = min(kt - split * a.chunk * 2, a.chunk * 2);
+    }
     const int per_band = TG_GROUP_M * a.tiles_n;
     const int band = wg / per_band, first = band * TG_GROUP_M;
     const int rows = min(a.tiles_m - first, TG_GROUP_M);
@@ -97,22 +133,29 @@ __global__ __launch_bounds__(512) void tgemm_tn_kernel(const TGArgs a) {
     m0 = (first + in_band % rows) * 256;
     n0 = (in_band / rows) * TN;
   };
-  const int KT = a.K >> 6;
 
   // ---- staging: thread -> row (wave * 8 + lane / 8) of a 64-row issue, physical chunk lane & 7
   const int srow = wave * 8 + (lane >> 3);
   const int schunk = (lane & 7) ^ ((srow >> 1) & 7);  // logical chunk whose data lands at physical chunk lane & 7
+  // NN: thread -> reduction row (wave * 4 + lane / 16) of a 32-row issue, physical chunk lane & 15 of its 256 bytes
+  const int wrow = wave * 4 + (lane >> 4);
+  const int wpc = ((lane & 15) ^ (((lane >> 4) << 2) | (wave & 3))) * 8;
+  const size_t stepB = NN ? (size_t)64 * a.ldb : 64;  // elements of B from K tile to K tile
   const bf16_t* srcA[2][2];  // [piece][issue]
   const bf16_t* srcB[2][2];
-  auto set_sources = [&](int m0, int n0) __attribute__((always_inline)) {
+  auto set_sources = [&](int m0, int n0, int k0) __attribute__((always_inline)) {
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
         int row = m0 + i * 128 + h * 64 + srow;
         row = row < a.M ? row : a.M - 1;
-        srcA[h][i] = a.A + (size_t)row * a.lda + schunk * 8;
+        srcA[h][i] = a.A + (size_t)row * a.lda + schunk * 8 + (NN ? k0 : 0);
         int col;
+        if (NN) {  // one pointer: N is a multiple of 256 here, pieces and issues are a fixed step apart
+          if (h == 0 && i == 0) srcB[0][0] = a.B + (size_t)(k0 + wrow) * a.ldb + n0 + (wpc >> 5) * 64 + (wpc & 31);
+          continue;
+        }
         if (EPI == 1) {  // piece h: gate (0) or up (1) rows of the tile's 128 columns, 32 per wave column
           col = n0 + (i * 2 + (wave >> 2)) * 32 + (wave & 3) * 8 + (lane >> 3);
           col = (col < a.N ? col : a.N - 1) + h * a.N;
@@ -125,10 +168,11 @@ __global__ __launch_bounds__(512) void tgemm_tn_kernel(const TGArgs a) {
   };
   auto stage = [&](int buf, int piece, int kt) __attribute__((always_inline)) {
     char* dst = smem + buf * TG_BUF + piece * TG_PIECE + wave * 1024;
-    const bf16_t* s0 = piece < 2 ? srcA[piece][0] : srcB[piece - 2][0];
-    const bf16_t* s1 = piece < 2 ? srcA[piece][1] : srcB[piece - 2][1];
-    __builtin_amdgcn_global_load_lds((gptr_t)(s0 + (size_t)kt * 64), (lptr_t)dst, 16, 0, 0);
-    __builtin_amdgcn_global_load_lds((gptr_t)(s1 + (size_t)kt * 64), (lptr_t)(dst + 8192), 16, 0, 0);
+    const bf16_t* s0 = piece < 2 ? srcA[piece][0] : NN ? srcB[0][0] + (piece - 2) * 32 : srcB[piece - 2][0];
+    const bf16_t* s1 = piece < 2 ? srcA[piece][1] : NN ? s0 + stepB / 2 : srcB[piece - 2][1];
+    const size_t at = kt * (piece < 2 ? (size_t)64 : stepB);
+    __builtin_amdgcn_global_load_lds((gptr_t)(s0 + at), (lptr_t)dst, 16, 0, 0);
+    __builtin_amdgcn_global_load_lds((gptr_t)(s1 + at), (lptr_t)(dst + 8192), 16, 0, 0);
   };
 
   // ---- fragment reads
@@ -146,7 +190,23 @@ __global__ __launch_bounds__(512) void tgemm_tn_kernel(const TGArgs a) {
       af[mt][1] = *reinterpret_cast<const bf16x8*>(p + mt * 2048 + cb1);
     }
   };
+  // NN: pieces of [64 reduction rows][128 columns]; lane (fr, fq) needs rows 8 fq .. 8 fq + 7 of column fr, two transposed reads
+  int t_adr[2][2];  // [16-column tile][row half]
+#pragma unroll
+  for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+    for (int h2 = 0; h2 < 2; ++h2)
+      t_adr[nt][h2] = (int)(tr_addr((const char*)0, 8 * fq + 4 * h2, wc * 32 + nt * 16, fr) - (const char*)0);
   auto read_b = [&](int buf, int h, tg_bfrag& bf) __attribute__((always_inline)) {
+    if (NN) {
+      const uint32_t p = (uint32_t)(uintptr_t)(lptr_t)smem + buf * TG_BUF;
+#pragma unroll
+      for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+          bf[nt][s] = cat4(tg_tr(p + t_adr[nt][0], (2 + h) * TG_PIECE + s * 8192), tg_tr(p + t_adr[nt][1], (2 + h) * TG_PIECE + s * 8192));
+      return;
+    }
     const char* p = smem + buf * TG_BUF + (2 + h) * TG_PIECE + b_off;
 #pragma unroll
     for (int nt = 0; nt < 2; ++nt) {
@@ -174,73 +234,101 @@ __global__ __launch_bounds__(512) void tgemm_tn_kernel(const TGArgs a) {
 
   // ---- result stores. Lane (row fr, column quad fq) of tile (mt, nt) holds 4 consecutive columns; the two 16-column
   // tiles of a quadrant exchange halves between neighbouring 16-lane rows (v_permlane16_swap), after which a lane holds
-  // 8 consecutive columns of one of them: 16-byte stores, the four lanes of a row write 64 contiguous bytes.
-  auto put = [&](tg_acc& acc, int m0, int n0, int mh, int nh) __attribute__((always_inline)) {
-    const int n = n0 + wc * 64 + nh * 32 + (fq & 1) * 16 + (fq >> 1) * 8;
+  // 8 consecutive columns of one of them, 16-byte chunk out_ch of the quadrant's 64 bytes.
+  const int out_ch = (fq & 1) * 2 + (fq >> 1);
+  auto pack8 = [&](const f32x4& v0, const f32x4& v1) __attribute__((always_inline)) {
+    unsigned pk[2][2];
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt) {
-      const int m = m0 + wr * 128 + mh * 64 + mt * 16 + fr;
-      unsigned pk[2][2];
+    for (int nt = 0; nt < 2; ++nt) {
+      const f32x4& v = nt ? v1 : v0;
+      bf16x2 lo = {f2bf(v[0]), f2bf(v[1])}, hi = {f2bf(v[2]), f2bf(v[3])};
+      pk[nt][0] = __builtin_bit_cast(unsigned, lo);
+      pk[nt][1] = __builtin_bit_cast(unsigned, hi);
+    }
+    const auto r0 = __builtin_amdgcn_permlane16_swap(pk[0][0], pk[1][0], false, false);
+    const auto r1 = __builtin_amdgcn_permlane16_swap(pk[0][1], pk[1][1], false, false);
+    return u32x4{r0[0], r1[0], r0[1], r1[1]};
+  };
+  auto store8 = [&](auto stream, int m, int n, u32x4 o) __attribute__((always_inline)) {
+    if (m < a.M && n < a.N) {
+      bf16_t* p = a.C + (size_t)m * a.ldc + n;
+      if (n + 8 <= a.N) {
+        if constexpr (decltype(stream)::value)
+          __builtin_nontemporal_store(o, reinterpret_cast<u32x4*>(p));
+        else
+          *reinterpret_cast<u32x4*>(p) = o;
+      } else {  // the last 4 columns of a width that is not a multiple of 8
+        *reinterpret_cast<u32x2*>(p) = (u32x2){o[0], o[1]};
+      }
+    }
+  };
+  // plain form: both column quadrants of a row half, 32 rows of 128 bytes at a time through the wave's 4 KiB
+  auto put = [&](tg_acc& c0, tg_acc& c1, int m0, int n0, float* part, int mh) __attribute__((always_inline)) {
+    char* ob = smem + TG_LDS + wave * 4096;
+    if (NN && part) {  // one part of the reduction, summed by a kernel of its own
+      float* op = part + (wr * 128 + mh * 64 + fr) * 256 + wc * 64 + fq * 4;
 #pragma unroll
-      for (int nt = 0; nt < 2; ++nt) {
-        f32x4 v = acc[mt][nt];
-        if (a.bias) {
+      for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt) {
+          *reinterpret_cast<f32x4*>(op + mt * 4096 + nt * 16) = c0[mt][nt];
+          *reinterpret_cast<f32x4*>(op + mt * 4096 + 32 + nt * 16) = c1[mt][nt];
+        }
+      return;
+    }
+    if (a.bias) {
+#pragma unroll
+      for (int nh = 0; nh < 2; ++nh)
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt) {
           const int nb = n0 + wc * 64 + nh * 32 + nt * 16 + fq * 4;
           if (nb < a.N) {
             const bf16x4 bb = *reinterpret_cast<const bf16x4*>(a.bias + nb);
 #pragma unroll
-            for (int j = 0; j < 4; ++j) v[j] += bf2f(bb[j]);
+            for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+              for (int j = 0; j < 4; ++j) (nh ? c1 : c0)[mt][nt][j] += bf2f(bb[j]);
           }
         }
-        bf16x2 lo = {f2bf(v[0]), f2bf(v[1])}, hi = {f2bf(v[2]), f2bf(v[3])};
-        pk[nt][0] = __builtin_bit_cast(unsigned, lo);
-        pk[nt][1] = __builtin_bit_cast(unsigned, hi);
+    }
+#pragma unroll
+    for (int hb = 0; hb < 2; ++hb) {
+#pragma unroll
+      for (int mi = 0; mi < 2; ++mi) {
+        const int mt = hb * 2 + mi;
+        char* row = ob + (mi * 16 + fr) * 128;
+        *reinterpret_cast<u32x4*>(row + ((out_ch ^ (fr & 7)) << 4)) = pack8(c0[mt][0], c0[mt][1]);
+        *reinterpret_cast<u32x4*>(row + (((out_ch + 4) ^ (fr & 7)) << 4)) = pack8(c1[mt][0], c1[mt][1]);
       }
-      const auto r0 = __builtin_amdgcn_permlane16_swap(pk[0][0], pk[1][0], false, false);
-      const auto r1 = __builtin_amdgcn_permlane16_swap(pk[0][1], pk[1][1], false, false);
-      const u32x4 o = {r0[0], r1[0], r0[1], r1[1]};
-      if (m < a.M && n < a.N) {
-        if (n + 8 <= a.N) {
-          *reinterpret_cast<u32x4*>(a.C + (size_t)m * a.ldc + n) = o;
-        } else {  // the last 4 columns of a width that is not a multiple of 8
-          *reinterpret_cast<u32x2*>(a.C + (size_t)m * a.ldc + n) = (u32x2){o[0], o[1]};
-        }
-      }
+      u32x4 o[4];
+      const int r8 = lane >> 3, ch = lane & 7;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[i] = *reinterpret_cast<const u32x4*>(ob + (i * 8 + r8) * 128 + ((ch ^ r8) << 4));
+#pragma unroll
+      for (int i = 0; i < 4; ++i) store8(std::true_type{}, m0 + wr * 128 + mh * 64 + hb * 32 + i * 8 + r8, n0 + wc * 64 + ch * 8, o[i]);
     }
   };
-  // gated form: `g` and `u` are the two column quadrants of one row half
+  // gated form: `g` and `u` are the two column quadrants of one row half. A wave's 32 result columns are half a line: the four
+  // waves of a wave row passing them on together through LDS was slower (1361 against 1321 us at 32768 x 8960 from 1536 deep)
+  // than storing from the registers; so was dealing the activation out over the next tile's first phases (1333).
   auto put_gated = [&](tg_acc& g, tg_acc& u, int m0, int n0, int mh) __attribute__((always_inline)) {
-    const int n = n0 + wc * 32 + (fq & 1) * 16 + (fq >> 1) * 8;
 #pragma unroll
     for (int mt = 0; mt < 4; ++mt) {
-      const int m = m0 + wr * 128 + mh * 64 + mt * 16 + fr;
-      unsigned pk[2][2];
+      f32x4 v[2];
 #pragma unroll
-      for (int nt = 0; nt < 2; ++nt) {
-        f32x4 v;
+      for (int nt = 0; nt < 2; ++nt)
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          // the unfused path carries gate|up as a bf16 tensor
+          // the unfused path carries gate|up as a bf16 tensor. v_rcp_f32 (1 ulp) for the quotient: a division is ten more
+          // instructions, 64 of them a lane and tile (1386 -> 1294 us at 32768 x 8960 from 1536 deep)
           const float gg = bf2f(f2bf(g[mt][nt][j])), uu = bf2f(f2bf(u[mt][nt][j]));
-          v[j] = gg / (1.f + __expf(-gg)) * uu;
+          v[nt][j] = gg * __builtin_amdgcn_rcpf(1.f + __expf(-gg)) * uu;
         }
-        bf16x2 lo = {f2bf(v[0]), f2bf(v[1])}, hi = {f2bf(v[2]), f2bf(v[3])};
-        pk[nt][0] = __builtin_bit_cast(unsigned, lo);
-        pk[nt][1] = __builtin_bit_cast(unsigned, hi);
-      }
-      const auto r0 = __builtin_amdgcn_permlane16_swap(pk[0][0], pk[1][0], false, false);
-      const auto r1 = __builtin_amdgcn_permlane16_swap(pk[0][1], pk[1][1], false, false);
-      const u32x4 o = {r0[0], r1[0], r0[1], r1[1]};
-      if (m < a.M && n < a.N) {
-        if (n + 8 <= a.N) {
-          *reinterpret_cast<u32x4*>(a.C + (size_t)m * a.ldc + n) = o;
-        } else {
-          *reinterpret_cast<u32x2*>(a.C + (size_t)m * a.ldc + n) = (u32x2){o[0], o[1]};
-        }
-      }
+      store8(std::false_type{}, m0 + wr * 128 + mh * 64 + mt * 16 + fr, n0 + wc * 32 + out_ch * 8, pack8(v[0], v[1]));
     }
   };
   int cm0 = 0, cn0 = 0;  // origin of the output tile being computed
+  float* cpart = nullptr;
 
   // One K tile = four phases. The K tiles of the block's successive output tiles form ONE stream: the pieces staged
   // while the last two K tiles of an output tile are computed are K tiles 0 and 1 of the NEXT output tile, so the
@@ -249,7 +337,8 @@ __global__ __launch_bounds__(512) void tgemm_tn_kernel(const TGArgs a) {
   // "t+2" is K tile 0 of the next output tile, whose source addresses replace the current ones after phase 1).
   // MODE 2: last K tile ("t+1", "t+2" are K tiles 0, 1 of the next output tile). Without a next tile nothing is staged
   // and the loads still in flight are drained.
-  int nm0 = 0, nn0 = 0;
+  int nm0 = 0, nn0 = 0, nk0 = 0, nkt = 0;
+  float* npart = nullptr;
   bool has_next = false;
   auto tile = [&](auto buf_c, int t, auto mode_c) __attribute__((always_inline)) {
     constexpr int buf = decltype(buf_c)::value, MODE = decltype(mode_c)::value;
@@ -264,21 +353,18 @@ __global__ __launch_bounds__(512) void tgemm_tn_kernel(const TGArgs a) {
     // from now, when the staggered wave group has only just passed that barrier
     asm volatile("s_waitcnt lgkmcnt(8)" ::: "memory");
     mma(acc00, bf0);
-    // last K tile: a quadrant is final once its phase is over; its stores are issued while the other wave group
-    // computes
-    if (MODE == 2 && EPI == 0) put(acc00, cm0, cn0, 0, 0);
-    if (MODE == 1 && go) set_sources(nm0, nn0);
+    if (MODE == 1 && go) set_sources(nm0, nn0, nk0);
     // phase 2: quadrant (0, 1)
     read_b(buf, 1, bf1);
     if (go) stage(buf, PB0, t2);
     mma(acc01, bf1);
-    if (MODE == 2 && EPI == 0) put(acc01, cm0, cn0, 0, 1);
+    // last K tile: a row half is final once its phases are over; it leaves while the other wave group computes
+    if (MODE == 2 && EPI == 0) put(acc00, acc01, cm0, cn0, cpart, 0);
     if (MODE == 2 && EPI == 1) put_gated(acc00, acc01, cm0, cn0, 0);
     // phase 3: quadrant (1, 1)
     read_a(buf, 1);
     if (go) stage(buf, PA0, t2);
     mma(acc11, bf1);
-    if (MODE == 2 && EPI == 0) put(acc11, cm0, cn0, 1, 1);
     // phase 4: quadrant (1, 0); the next K tile of the stream becomes readable
     if (go) {
       stage(buf, PB1, t2);
@@ -287,7 +373,7 @@ __global__ __launch_bounds__(512) void tgemm_tn_kernel(const TGArgs a) {
       tg_vmcnt<0>();
     }
     mma(acc10, bf0);
-    if (MODE == 2 && EPI == 0) put(acc10, cm0, cn0, 1, 0);
+    if (MODE == 2 && EPI == 0) put(acc10, acc11, cm0, cn0, cpart, 1);
     if (MODE == 2 && EPI == 1) put_gated(acc10, acc11, cm0, cn0, 1);
   };
   using B0 = std::integral_constant<int, 0>;
@@ -297,9 +383,10 @@ __global__ __launch_bounds__(512) void tgemm_tn_kernel(const TGArgs a) {
   using M2 = std::integral_constant<int, 2>;
 
   // ---- prologue: K tile 0 whole, B0 A0 B1 of K tile 1 (its A1 leaves in phase 1 of K tile 0)
-  int id = blockIdx.x, m0, n0;
-  tile_origin(id, m0, n0);
-  set_sources(m0, n0);
+  int id = blockIdx.x, m0, n0, k0, KT;
+  float* part;
+  tile_origin(id, m0, n0, k0, KT, part);
+  set_sources(m0, n0, k0);
   stage(0, PB0, 0);
   stage(0, PA0, 0);
   stage(0, PB1, 0);
@@ -314,9 +401,10 @@ __global__ __launch_bounds__(512) void tgemm_tn_kernel(const TGArgs a) {
   while (true) {
     const int nid = id + gridDim.x;
     has_next = nid < ntiles;
-    if (has_next) tile_origin(nid, nm0, nn0);
+    if (has_next) tile_origin(nid, nm0, nn0, nk0, nkt, npart);
     cm0 = m0;
     cn0 = n0;
+    cpart = part;
 #pragma unroll
     for (int mt = 0; mt < 4; ++mt)
 #pragma unroll
@@ -338,6 +426,8 @@ __global__ __launch_bounds__(512) void tgemm_tn_kernel(const TGArgs a) {
     id = nid;
     m0 = nm0;
     n0 = nn0;
+    KT = nkt;
+    part = npart;
   }
   if (STAGGER && wr == 0) tg_barrier();
 }
@@ -372,8 +462,6 @@ struct TWArgs {
   int splits, chunk;  // the others: workgroups per tile, pairs per workgroup (the last one of a tile may get fewer)
 };
 
-typedef f32x16 tw_acc[2];  // [32-row n tile] of one quadrant (64 n x 32 k)
-
 template <bool STAGGER>
 __global__ __launch_bounds__(512) void tgemm_wgrad_kernel(const TWArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -396,8 +484,6 @@ __global__ __launch_bounds__(512) void tgemm_wgrad_kernel(const TWArgs a) {
     b_split = (b - a.whole) - (b_tile - a.whole) * a.splits;
     b_chunk = a.chunk;
   }
-  int w = b_tile * a.pairs + b_split * b_chunk;
-  const int w_end = min(w + b_chunk, (b_tile + 1) * a.pairs);
   auto tile_origin = [&](int wg, int& n0, int& k0) __attribute__((always_inline)) {
     const int per_band = TG_GROUP_M * a.tiles_k;
     const int band = wg / per_band, first = band * TG_GROUP_M;
@@ -428,51 +514,51 @@ __global__ __launch_bounds__(512) void tgemm_wgrad_kernel(const TWArgs a) {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lptr_t)(dst + 8192), 16, v + 32 * row, 0, 0, 0);
   };
 
-  // ---- transposed fragment reads: addresses inside a piece (the same for both buffers and every 16-token slab)
-  const int gl = lane & 15, grp = lane >> 4, hf = lane >> 5, r32 = lane & 31;
-  int a_adr[2][2], b_adr[2];  // [32-row tile][token half]
+  // ---- transposed fragment reads: addresses inside a piece (the same for both buffers and every 32-token slab). Lane (fr, fq)
+  // of an operand holds tokens 8 fq .. 8 fq + 7 of column fr: two reads of four tokens
+  const int fr = lane & 15, fq = lane >> 4;
+  int a_adr[4][2], b_adr[2][2];  // [16-column tile][token half]
 #pragma unroll
   for (int h2 = 0; h2 < 2; ++h2) {
 #pragma unroll
-    for (int mi = 0; mi < 2; ++mi)
-      a_adr[mi][h2] = (int)(tr_addr((const char*)0, 8 * h2 + 4 * hf, wr * 64 + mi * 32 + 16 * (grp & 1), gl) - (const char*)0);
-    b_adr[h2] = (int)(tr_addr((const char*)0, 8 * h2 + 4 * hf, wc * 32 + 16 * (grp & 1), gl) - (const char*)0);
+    for (int mt = 0; mt < 4; ++mt)
+      a_adr[mt][h2] = (int)(tr_addr((const char*)0, 8 * fq + 4 * h2, wr * 64 + mt * 16, fr) - (const char*)0);
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt)
+      b_adr[nt][h2] = (int)(tr_addr((const char*)0, 8 * fq + 4 * h2, wc * 32 + nt * 16, fr) - (const char*)0);
   }
-  // The reads are issued from inline assembly: behind the builtin, hipcc cannot tell the transposed read from the
-  // pending LDS-DMA writes and puts s_waitcnt vmcnt(0) in front of every group of reads, draining the pipeline. The
-  // results are ordered by the explicit lgkmcnt waits of the phase.
   const uint32_t lds0 = (uint32_t)(uintptr_t)(lptr_t)smem;
-  auto trl = [&](uint32_t adr, int imm) __attribute__((always_inline)) {
-    bf16x4 v;
-    asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(v) : "v"(adr), "i"(imm));
-    return v;
-  };
-  bf16x8 af[2][4];    // [32-row tile][16-token slab]
-  bf16x8 bf0[4], bf1[4];
+  bf16x8 af[4][2];  // [16-column tile][32-token slab]
+  tg_bfrag bf0, bf1;
   auto read_a = [&](int buf, int h) __attribute__((always_inline)) {
     const uint32_t p = lds0 + buf * TG_BUF;
 #pragma unroll
-    for (int mi = 0; mi < 2; ++mi)
+    for (int mt = 0; mt < 4; ++mt)
 #pragma unroll
-      for (int s = 0; s < 4; ++s)
-        af[mi][s] = cat4(trl(p + a_adr[mi][0], h * TG_PIECE + s * 4096), trl(p + a_adr[mi][1], h * TG_PIECE + s * 4096));
+      for (int s = 0; s < 2; ++s)
+        af[mt][s] = cat4(tg_tr(p + a_adr[mt][0], h * TG_PIECE + s * 8192), tg_tr(p + a_adr[mt][1], h * TG_PIECE + s * 8192));
   };
-  auto read_b = [&](int buf, int h, bf16x8 (&bf)[4]) {
+  auto read_b = [&](int buf, int h, tg_bfrag& bf) __attribute__((always_inline)) {
     const uint32_t p = lds0 + buf * TG_BUF;
 #pragma unroll
-    for (int s = 0; s < 4; ++s)
-      bf[s] = cat4(trl(p + b_adr[0], (2 + h) * TG_PIECE + s * 4096), trl(p + b_adr[1], (2 + h) * TG_PIECE + s * 4096));
+    for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+        bf[nt][s] = cat4(tg_tr(p + b_adr[nt][0], (2 + h) * TG_PIECE + s * 8192), tg_tr(p + b_adr[nt][1], (2 + h) * TG_PIECE + s * 8192));
   };
-  tw_acc acc00, acc01, acc10, acc11;  // [n half][k half]
-  auto mma = [&](tw_acc& acc, bf16x8 (&bf)[4]) {
+  tg_acc acc00, acc01, acc10, acc11;  // [n half][k half]
+  auto mma = [&](tg_acc& acc, tg_bfrag& bf) __attribute__((always_inline)) {
     tg_barrier();
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-    for (int s = 0; s < 4; ++s)
+    for (int s = 0; s < 2; ++s)
 #pragma unroll
-      for (int mi = 0; mi < 2; ++mi) acc[mi] = mfma32(af[mi][s], bf[s], acc[mi]);
+      for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt)
+          acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[nt][s], af[mt][s], acc[mt][nt], 0, 0, 0);
     __builtin_amdgcn_s_setprio(0);
     __builtin_amdgcn_sched_barrier(0);
     tg_barrier();
@@ -503,209 +589,28 @@ __global__ __launch_bounds__(512) void tgemm_wgrad_kernel(const TWArgs a) {
   using T1 = std::integral_constant<int, 1>;
   using T2 = std::integral_constant<int, 2>;
 
-  // ---- epilogue: lane (k column r32, hf) holds rows n = (reg & 3) + 8 (reg >> 2) + 4 hf of each 32 x 32 tile
-  int n0 = 0, k0 = 0;
-  bool whole = false;
-  auto flush = [&](tw_acc& acc, int mh, int nh) __attribute__((always_inline)) {
+  // ---- one segment: pairs [p0, p1) of one output tile
+  int n0, k0;
+  const int p0 = b_split * b_chunk, p1 = min(a.pairs, p0 + b_chunk);
+  tile_origin(b_tile, n0, k0);
+  const bool whole = p0 == 0 && p1 == a.pairs;
+  const int tok0 = p0 * 128, KT = (p1 - p0) * 2;
+  tokens = a.M - tok0;
+  // N may end half way through the last tile row (N % 256 == 128): the second wave row then re-reads the first
+  // one's columns and does not write
+  const bool half_n = n0 + 128 >= a.N;
+  pA = a.dY + (size_t)tok0 * a.ldy + n0;
+  pB = a.X + (size_t)tok0 * a.ldx + k0;
+  vA = (unsigned)(srow * a.ldy + (half_n ? 0 : (pc >> 6) * 128) + (pc & 63)) * 2;
+  vB = (unsigned)(srow * a.ldx + (pc >> 5) * 64 + (pc & 31)) * 2;
 #pragma unroll
-    for (int mi = 0; mi < 2; ++mi) {
-      float* op = a.dW + (size_t)(n0 + wr * 128 + mh * 64 + mi * 32 + 4 * hf) * a.ldw + k0 + wc * 64 + nh * 32 + r32;
-      if (whole) {
-        float old[16];
+  for (int mt = 0; mt < 4; ++mt)
 #pragma unroll
-        for (int reg = 0; reg < 16; ++reg) old[reg] = op[(size_t)((reg & 3) + 8 * (reg >> 2)) * a.ldw];
-#pragma unroll
-        for (int reg = 0; reg < 16; ++reg) op[(size_t)((reg & 3) + 8 * (reg >> 2)) * a.ldw] = old[reg] + acc[mi][reg];
-      } else {
-#pragma unroll
-        for (int reg = 0; reg < 16; ++reg) unsafeAtomicAdd(op + (size_t)((reg & 3) + 8 * (reg >> 2)) * a.ldw, acc[mi][reg]);
-      }
-    }
-  };
-
-  while (w < w_end) {
-    // ---- one segment: pairs [p0, p1) of one output tile
-    const int tile_id = w / a.pairs, p0 = w - tile_id * a.pairs;
-    const int p1 = min(a.pairs, p0 + (w_end - w));
-    w += p1 - p0;
-    tile_origin(tile_id, n0, k0);
-    whole = p0 == 0 && p1 == a.pairs;
-    const int tok0 = p0 * 128, KT = (p1 - p0) * 2;
-    tokens = a.M - tok0;
-    // N may end half way through the last tile row (N % 256 == 128): the second wave row then re-reads the first
-    // one's columns and does not write
-    const bool half_n = n0 + 128 >= a.N;
-    pA = a.dY + (size_t)tok0 * a.ldy + n0;
-    pB = a.X + (size_t)tok0 * a.ldx + k0;
-    vA = (unsigned)(srow * a.ldy + (half_n ? 0 : (pc >> 6) * 128) + (pc & 63)) * 2;
-    vB = (unsigned)(srow * a.ldx + (pc >> 5) * 64 + (pc & 31)) * 2;
-#pragma unroll
-    for (int mi = 0; mi < 2; ++mi)
-#pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        acc00[mi][j] = 0.f;
-        acc01[mi][j] = 0.f;
-        acc10[mi][j] = 0.f;
-        acc11[mi][j] = 0.f;
-      }
-    stage(0, PB0, 0);
-    stage(0, PA0, 0);
-    stage(0, PB1, 0);
-    stage(0, PA1, 0);
-    stage(1, PB0, 1);
-    stage(1, PA0, 1);
-    stage(1, PB1, 1);
-    tg_vmcnt<6>();
-    tg_barrier();
-    if (STAGGER && wr == 1) tg_barrier();
-    int t = 0;
-    for (; t + 2 < KT; t += 2) {
-      tile(B0{}, t, T0{});
-      tile(B1{}, t + 1, T0{});
-    }
-    tile(B0{}, t, T1{});
-    tile(B1{}, t + 1, T2{});
-    if (STAGGER && wr == 0) tg_barrier();
-    if (!(half_n && wr == 1)) {
-      flush(acc00, 0, 0);
-      flush(acc01, 0, 1);
-      flush(acc10, 1, 0);
-      flush(acc11, 1, 1);
-    }
-  }
-}
-
-// =====================================================================================
-// Input gradient:  dX[M, C] = dY[M, R] . W[R, C]     (bf16 operands; W as it lies, no transposed copy)
-//
-// The phases of the two kernels above: dY is staged and read as the forward kernel's A operand (reduction contiguous), W as
-// the weight gradient's X (reduction slow, transposed reads). For few rows and a deep reduction: a pass over 700 tokens has 18
-// tiles of 256 x 256 for the gate|up projection's 17920 and the vocabulary's 151936 weight rows, so the reduction is split
-// until the chip is full; the parts are written as fp32 and summed by a kernel of their own (they stay in the L2 and the
-// memory-side cache).
-// =====================================================================================
-struct TNArgs {
-  const bf16_t* dY;
-  long ldy;
-  const bf16_t* W;
-  long ldw;
-  bf16_t* dX;
-  long ldx;
-  float* part;  // [splits][M][C], null for one part
-  int M, R, C;
-  int tiles_m, tiles;
-  int pairs, chunk;  // 128-deep pairs of the reduction: of all of it, of one workgroup
-};
-
-__global__ __launch_bounds__(512) void tgemm_nn_kernel(const TNArgs a) {
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wr = wave >> 2, wc = wave & 3;
-  // ids are dealt round-robin to the 8 XCDs: one XCD takes neighbouring tiles of one part, which share panels in its L2
-  const int nb = gridDim.x, xq = nb >> 3, xr = nb & 7, xx = blockIdx.x & 7;
-  const int b = (xx < xr ? xx * (xq + 1) : xr * (xq + 1) + (xx - xr) * xq) + ((int)blockIdx.x >> 3);
-  const int split = b / a.tiles, tile_id = b - split * a.tiles;
-  const int m0 = (tile_id % a.tiles_m) * 256, c0 = (tile_id / a.tiles_m) * 256;
-  const int p0 = split * a.chunk, p1 = min(a.pairs, p0 + a.chunk);
-  const int KT = (p1 - p0) * 2;
-  if (KT <= 0) return;
-
-  // ---- staging. dY piece: row (wave * 8 + lane / 8) of a 64-row issue, 16-byte chunk lane & 7. W piece: reduction row
-  // (wave * 4 + lane / 16) of a 32-row issue, chunk lane & 15. Rows of dY past M are out of the buffer's range (zeros).
-  const int arow = wave * 8 + (lane >> 3), ach = (lane & 7) ^ ((arow >> 1) & 7);
-  const int wrow = wave * 4 + (lane >> 4);
-  const int pc = ((lane & 15) ^ (((lane >> 4) << 2) | (wave & 3))) * 8;
-  const unsigned rowA = (unsigned)a.ldy * 2, rowB = (unsigned)a.ldw * 2;
-  const unsigned vA = arow * rowA + ach * 16;
-  const unsigned vB = wrow * rowB + ((pc >> 5) * 64 + (pc & 31)) * 2;
-  const unsigned rangeA = (unsigned)(min(a.M - m0, 256) - 1) * rowA + 128, rangeB = 63 * rowB + 512;
-  const bf16_t* pA = a.dY + (size_t)m0 * a.ldy + (size_t)p0 * 128;
-  const bf16_t* pB = a.W + (size_t)p0 * 128 * a.ldw + c0;
-  auto stage = [&](int buf, int piece, int kt) __attribute__((always_inline)) {
-    char* dst = smem + buf * TG_BUF + piece * TG_PIECE + wave * 1024;
-    const bool isA = piece < 2;
-    const bf16_t* base = isA ? pA + (size_t)kt * 64 : pB + (size_t)kt * 64 * a.ldw;
-    const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(base), 0, isA ? rangeA : rangeB, 0x00020000);
-    const unsigned v = isA ? vA + (piece & 1) * 64 * rowA : vB + (piece & 1) * 64;
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lptr_t)dst, 16, v, 0, 0, 0);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lptr_t)(dst + 8192), 16, v + (isA ? 128 * rowA : 32 * rowB), 0, 0, 0);
-  };
-
-  // ---- fragments: element j of lane half hf is reduction row 16 s + 8 hf + j in both operands
-  const int gl = lane & 15, grp = lane >> 4, hf = lane >> 5, r32 = lane & 31;
-  const int sw = (r32 >> 1) & 7;
-  int b_adr[2];
-#pragma unroll
-  for (int h2 = 0; h2 < 2; ++h2)
-    b_adr[h2] = (int)(tr_addr((const char*)0, 8 * hf + 4 * h2, wc * 32 + 16 * (grp & 1), gl) - (const char*)0);
-  const uint32_t lds0 = (uint32_t)(uintptr_t)(lptr_t)smem;
-  auto trl = [&](uint32_t adr, int imm) __attribute__((always_inline)) {  // see the weight gradient
-    bf16x4 v;
-    asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(v) : "v"(adr), "i"(imm));
-    return v;
-  };
-  bf16x8 af[2][4], bf0[4], bf1[4];  // [32-row tile][16-deep slab]
-  auto read_a = [&](int buf, int h) __attribute__((always_inline)) {
-    const char* p = smem + buf * TG_BUF + h * TG_PIECE + (wr * 64 + r32) * 128;
-#pragma unroll
-    for (int mi = 0; mi < 2; ++mi)
-#pragma unroll
-      for (int s = 0; s < 4; ++s) af[mi][s] = *reinterpret_cast<const bf16x8*>(p + mi * 4096 + (((2 * s + hf) ^ sw) << 4));
-  };
-  auto read_b = [&](int buf, int h, bf16x8 (&bf)[4]) __attribute__((always_inline)) {
-    const uint32_t p = lds0 + buf * TG_BUF;
-#pragma unroll
-    for (int s = 0; s < 4; ++s)
-      bf[s] = cat4(trl(p + b_adr[0], (2 + h) * TG_PIECE + s * 4096), trl(p + b_adr[1], (2 + h) * TG_PIECE + s * 4096));
-  };
-  tw_acc acc00, acc01, acc10, acc11;  // [row half][column half]
-  auto mma = [&](tw_acc& acc, bf16x8 (&bf)[4]) __attribute__((always_inline)) {
-    tg_barrier();
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-    for (int s = 0; s < 4; ++s)
-#pragma unroll
-      for (int mi = 0; mi < 2; ++mi) acc[mi] = mfma32(bf[s], af[mi][s], acc[mi]);
-    __builtin_amdgcn_s_setprio(0);
-    __builtin_amdgcn_sched_barrier(0);
-    tg_barrier();
-  };
-  // TAIL 0: tiles t+1 and t+2 exist; 1: only t+1 exists; 2: last tile
-  auto tile = [&](auto buf_c, int t, auto tail_c) __attribute__((always_inline)) {
-    constexpr int buf = decltype(buf_c)::value, TAIL = decltype(tail_c)::value;
-    read_b(buf, 0, bf0);
-    __builtin_amdgcn_sched_barrier(0);
-    read_a(buf, 0);
-    if (TAIL < 2) stage(buf ^ 1, PA1, t + 1);
-    asm volatile("s_waitcnt lgkmcnt(8)" ::: "memory");  // the eight B0 reads, issued first of 16, have returned
-    mma(acc00, bf0);
-    read_b(buf, 1, bf1);
-    if (TAIL < 1) stage(buf, PB0, t + 2);
-    mma(acc01, bf1);
-    read_a(buf, 1);
-    if (TAIL < 1) stage(buf, PA0, t + 2);
-    mma(acc11, bf1);
-    if (TAIL < 1) stage(buf, PB1, t + 2);
-    if (TAIL == 0) tg_vmcnt<6>();
-    if (TAIL == 1) tg_vmcnt<0>();
-    mma(acc10, bf0);
-  };
-  using B0 = std::integral_constant<int, 0>;
-  using B1 = std::integral_constant<int, 1>;
-  using T0 = std::integral_constant<int, 0>;
-  using T1 = std::integral_constant<int, 1>;
-  using T2 = std::integral_constant<int, 2>;
-#pragma unroll
-  for (int mi = 0; mi < 2; ++mi)
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      acc00[mi][j] = 0.f;
-      acc01[mi][j] = 0.f;
-      acc10[mi][j] = 0.f;
-      acc11[mi][j] = 0.f;
+    for (int nt = 0; nt < 2; ++nt) {
+      acc00[mt][nt] = (f32x4){0.f, 0.f, 0.f, 0.f};
+      acc01[mt][nt] = (f32x4){0.f, 0.f, 0.f, 0.f};
+      acc10[mt][nt] = (f32x4){0.f, 0.f, 0.f, 0.f};
+      acc11[mt][nt] = (f32x4){0.f, 0.f, 0.f, 0.f};
     }
   stage(0, PB0, 0);
   stage(0, PA0, 0);
@@ -716,7 +621,7 @@ __global__ __launch_bounds__(512) void tgemm_nn_kernel(const TNArgs a) {
   stage(1, PB1, 1);
   tg_vmcnt<6>();
   tg_barrier();
-  if (wr == 1) tg_barrier();  // the second wave row runs one barrier behind
+  if (STAGGER && wr == 1) tg_barrier();
   int t = 0;
   for (; t + 2 < KT; t += 2) {
     tile(B0{}, t, T0{});
@@ -724,48 +629,73 @@ __global__ __launch_bounds__(512) void tgemm_nn_kernel(const TNArgs a) {
   }
   tile(B0{}, t, T1{});
   tile(B1{}, t + 1, T2{});
-  if (wr == 0) tg_barrier();
+  if (STAGGER && wr == 0) tg_barrier();  // from here on nobody reads a staged tile: a wave has 16 KiB of LDS to itself
 
-  // ---- lane (row r32, hf) holds columns (reg & 3) + 8 (reg >> 2) + 4 hf of each 32 x 32 tile
-  auto put = [&](tw_acc& acc, int mh, int nh) __attribute__((always_inline)) {
+  // ---- lane (row fr, fq) of tile (mt, nt) holds 4 consecutive k columns. A row half (64 x 64 fp32) passes through the wave's
+  // LDS: plain adds move 256 bytes of four rows an instruction, atomic ones 256 bytes of one.
+  if (half_n && wr == 1) return;
+  char* ob = smem + wave * 16384;
+  auto flush = [&](tg_acc& c0, tg_acc& c1, int mh) __attribute__((always_inline)) {
+    float* op = a.dW + (size_t)(n0 + wr * 128 + mh * 64) * a.ldw + k0 + wc * 64;
+    typedef f32x4 __attribute__((aligned(4))) f32x4u;
 #pragma unroll
-    for (int mi = 0; mi < 2; ++mi) {
-      const int m = m0 + wr * 128 + mh * 64 + mi * 32 + r32, c = c0 + wc * 64 + nh * 32 + 4 * hf;
-      if (m >= a.M) continue;
-      if (a.part) {
-        float* op = a.part + ((size_t)split * a.M + m) * a.C + c;
+    for (int mt = 0; mt < 4; ++mt)
 #pragma unroll
-        for (int g = 0; g < 4; ++g)
-          *reinterpret_cast<f32x4*>(op + 8 * g) =
-              f32x4{acc[mi][4 * g], acc[mi][4 * g + 1], acc[mi][4 * g + 2], acc[mi][4 * g + 3]};
-      } else {
-        bf16_t* op = a.dX + (size_t)m * a.ldx + c;
+      for (int nh = 0; nh < 2; ++nh)
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          bf16x4 v;
+        for (int nt = 0; nt < 2; ++nt)
+          *reinterpret_cast<f32x4*>(ob + (mt * 16 + fr) * 256 + (((nh * 8 + nt * 4 + fq) ^ fr) << 4)) = (nh ? c1 : c0)[mt][nt];
+    if (whole) {
 #pragma unroll
-          for (int j = 0; j < 4; ++j) v[j] = f2bf(acc[mi][4 * g + j]);
-          *reinterpret_cast<bf16x4*>(op + 8 * g) = v;
+      for (int i0 = 0; i0 < 16; i0 += 8) {
+        f32x4 old[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) old[i] = *reinterpret_cast<const f32x4u*>(op + (size_t)((i0 + i) * 4 + fq) * a.ldw + fr * 4);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const int row = (i0 + i) * 4 + fq;
+          const f32x4 v = *reinterpret_cast<const f32x4*>(ob + row * 256 + ((fr ^ (row & 15)) << 4));
+          *reinterpret_cast<f32x4u*>(op + (size_t)row * a.ldw + fr * 4) = old[i] + v;
         }
+      }
+    } else {
+#pragma unroll 16
+      for (int row = 0; row < 64; ++row) {
+        const float v = *reinterpret_cast<const float*>(ob + row * 256 + (((lane >> 2) ^ (row & 15)) << 4) + (lane & 3) * 4);
+        unsafeAtomicAdd(op + (size_t)row * a.ldw + lane, v);
       }
     }
   };
-  put(acc00, 0, 0);
-  put(acc01, 0, 1);
-  put(acc10, 1, 0);
-  put(acc11, 1, 1);
+  flush(acc00, acc01, 0);
+  flush(acc10, acc11, 1);
 }
 
-// dX (rows of C numbers, C a multiple of 256) = sum of the parts, in order
-__global__ __launch_bounds__(256) void tgemm_nn_sum_kernel(const float* __restrict__ part, int splits, bf16_t* __restrict__ dX,
-                                                           long ldx, int M, int C) {
-  const size_t n = (size_t)M * C, i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
-  if (i >= n) return;
-  f32x4 v = *reinterpret_cast<const f32x4*>(part + i);
+// =====================================================================================
+// Input gradient:  dX[M, C] = dY[M, R] . W[R, C]     (bf16 operands; W as it lies, no transposed copy)
+//
+// The NN form of the forward kernel: W is staged like the weight gradient's X (reduction slow) and read transposed. Tiles that
+// would leave CUs idle in a last round (or all of them, for few rows) are split over the reduction until the chip is full; the
+// parts are written as fp32 and summed here (they stay in the L2 and the memory-side cache).
+// =====================================================================================
+// dX of the tiles from `whole` on = sum of the parts, in order. Block: 8 rows of a tile.
+__global__ __launch_bounds__(256) void tgemm_nn_sum_kernel(const TGArgs a) {
+  const int rest = a.tiles_m * a.tiles_n - a.whole, t = blockIdx.x >> 5, wg = a.whole + t;
+  const int band = wg / (TG_GROUP_M * a.tiles_n), first = band * TG_GROUP_M, rows = min(a.tiles_m - first, TG_GROUP_M);
+  const int in_band = wg - band * TG_GROUP_M * a.tiles_n;
+  const int row = (blockIdx.x & 31) * 8 + (threadIdx.x >> 5), col = (threadIdx.x & 31) * 8;
+  const int m = (first + in_band % rows) * 256 + row, n = in_band / rows * 256 + col;
+  if (m >= a.M) return;
+  const float* p = a.part + ((size_t)t << 16) + row * 256 + col;
+  f32x4 v0 = *reinterpret_cast<const f32x4*>(p), v1 = *reinterpret_cast<const f32x4*>(p + 4);
 #pragma unroll 4
-  for (int s = 1; s < splits; ++s) v += *reinterpret_cast<const f32x4*>(part + s * n + i);
-  const bf16x4 o = {f2bf(v[0]), f2bf(v[1]), f2bf(v[2]), f2bf(v[3])};
-  *reinterpret_cast<bf16x4*>(dX + i / C * ldx + i % C) = o;
+  for (int s = 1; s < a.splits; ++s) {
+    const float* q = p + ((size_t)s * rest << 16);
+    v0 += *reinterpret_cast<const f32x4*>(q);
+    v1 += *reinterpret_cast<const f32x4*>(q + 4);
+  }
+  bf16_t* op = a.C + (size_t)m * a.ldc + n;
+  *reinterpret_cast<bf16x4*>(op) = bf16x4{f2bf(v0[0]), f2bf(v0[1]), f2bf(v0[2]), f2bf(v0[3])};
+  *reinterpret_cast<bf16x4*>(op + 4) = bf16x4{f2bf(v1[0]), f2bf(v1[1]), f2bf(v1[2]), f2bf(v1[3])};
 }
 
 }  // namespace
@@ -781,12 +711,12 @@ static int tgemm_tn_launch(const void* A, long lda, const void* B, long ldb, voi
   if (((uintptr_t)A | (uintptr_t)B) % 16 != 0 || (uintptr_t)C % 8 != 0 || (bias && (uintptr_t)bias % 8 != 0)) return -1;
   if (gated && bias) return -1;
   TGArgs a{(const bf16_t*)A, lda, (const bf16_t*)B, ldb, (bf16_t*)C, ldc, (const bf16_t*)bias, M, N, K,
-           (M + 255) / 256, gated ? (N + 127) / 128 : (N + 255) / 256};
+           (M + 255) / 256, gated ? (N + 127) / 128 : (N + 255) / 256, nullptr, 0, 1, 0};
   static bool attr_set = false;  // 128 KiB of dynamic LDS: above the default limit
   if (!attr_set) {
-    HIP_RET(hipFuncSetAttribute((const void*)tgemm_tn_kernel<true, 0>, hipFuncAttributeMaxDynamicSharedMemorySize, TG_LDS));
-    HIP_RET(hipFuncSetAttribute((const void*)tgemm_tn_kernel<false, 0>, hipFuncAttributeMaxDynamicSharedMemorySize, TG_LDS));
-    HIP_RET(hipFuncSetAttribute((const void*)tgemm_tn_kernel<true, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, TG_LDS));
+    HIP_RET(hipFuncSetAttribute((const void*)tgemm_kernel<true, 0, false>, hipFuncAttributeMaxDynamicSharedMemorySize, TG_LDS + TG_OUT));
+    HIP_RET(hipFuncSetAttribute((const void*)tgemm_kernel<false, 0, false>, hipFuncAttributeMaxDynamicSharedMemorySize, TG_LDS + TG_OUT));
+    HIP_RET(hipFuncSetAttribute((const void*)tgemm_kernel<true, 1, false>, hipFuncAttributeMaxDynamicSharedMemorySize, TG_LDS));
     attr_set = true;
   }
   // max_blocks workgroups (a multiple of 8: block id mod 8 is the XCD for every tile of a block's sequence) walk the
@@ -795,11 +725,11 @@ static int tgemm_tn_launch(const void* A, long lda, const void* B, long ldb, voi
   if (max_blocks > 0 && max_blocks % 8 != 0) return -1;
   const dim3 grid(max_blocks > 0 ? std::min(ntiles, max_blocks) : ntiles), block(512);
   if (gated)
-    hipLaunchKernelGGL((tgemm_tn_kernel<true, 1>), grid, block, TG_LDS, st, a);
+    hipLaunchKernelGGL((tgemm_kernel<true, 1, false>), grid, block, TG_LDS, st, a);
   else if (stagger)
-    hipLaunchKernelGGL((tgemm_tn_kernel<true, 0>), grid, block, TG_LDS, st, a);
+    hipLaunchKernelGGL((tgemm_kernel<true, 0, false>), grid, block, TG_LDS + TG_OUT, st, a);
   else
-    hipLaunchKernelGGL((tgemm_tn_kernel<false, 0>), grid, block, TG_LDS, st, a);
+    hipLaunchKernelGGL((tgemm_kernel<false, 0, false>), grid, block, TG_LDS + TG_OUT, st, a);
   return (int)hipGetLastError();
 }
 
@@ -883,30 +813,33 @@ extern "C" int areal_tgemm_wgrad(const void* dY, long ldy, const void* X, long l
   return (int)hipGetLastError();
 }
 
-// dX[M, C] = dY[M, R] . W[R, C]; R a multiple of 128, C of 256, rows 16-byte aligned. part: splits x M x C floats, unused for
-// one part. Every part has to have work: with P = R / 128, ceil(P / ceil(P / splits)) == splits (12 pairs in 5 parts are 4).
-extern "C" int areal_tgemm_nn(const void* dY, long ldy, const void* W, long ldw, void* dX, long ldx, float* part, int splits,
-                              int M, int R, int C, hipStream_t st) {
+// dX[M, C] = dY[M, R] . W[R, C]; R a multiple of 128, C of 256, rows 16-byte aligned. The first `whole` tiles of 256 x 256 (a
+// multiple of 256, so that the parts start a round, or all of them: splits = 1) are reduced by one workgroup, the others in
+// `splits` parts. part: splits x 65536 floats for each of those. Every part has to have work: with P = R / 128,
+// ceil(P / ceil(P / splits)) == splits (12 pairs in 5 parts are 4).
+extern "C" int areal_tgemm_nn(const void* dY, long ldy, const void* W, long ldw, void* dX, long ldx, float* part, int whole,
+                              int splits, int M, int R, int C, hipStream_t st) {
   if (M <= 0 || R <= 0 || C <= 0) return R <= 0 && M > 0 && C > 0 ? -1 : 0;
   if (R % 128 != 0 || C % 256 != 0 || ldy % 8 != 0 || ldw % 8 != 0 || ldx % 4 != 0) return -1;
   if (((uintptr_t)dY | (uintptr_t)W) % 16 != 0 || (uintptr_t)dX % 8 != 0 || (uintptr_t)part % 16 != 0) return -1;
-  if (ldy < R || ldw < C || ldx < C || ldy > (1l << 22) || ldw > (1l << 24)) return -1;  // byte offsets of 256 / 64 rows: 32 bits
+  if (ldy < R || ldw < C || ldx < C || ldy > (1l << 22) || ldw > (1l << 24)) return -1;
   const int tiles_m = (M + 255) / 256, pairs = R / 128;
-  if (splits < 1 || splits > pairs || (splits > 1 && !part)) return -1;
+  const long tiles = (long)tiles_m * (C / 256);
+  if (tiles > 0x7fffffffl || splits < 1 || splits > pairs || whole < 0 || whole > tiles) return -1;
+  if (splits == 1 ? whole != tiles : whole % 256 != 0 || whole == tiles || !part) return -1;
   const int chunk = (pairs + splits - 1) / splits;
   if ((pairs + chunk - 1) / chunk != splits) return -1;  // a part without work would leave its sums unwritten
-  const long tiles = (long)tiles_m * (C / 256);
-  if (tiles * splits > 0x7fffffffl) return -1;
-  TNArgs a{(const bf16_t*)dY, ldy, (const bf16_t*)W, ldw, (bf16_t*)dX, ldx, splits > 1 ? part : nullptr, M, R, C, tiles_m,
-           (int)tiles, pairs, chunk};
+  const long items = whole + (tiles - whole) * splits;
+  if (items > 0x7fffffffl - 256) return -1;
+  TGArgs a{(const bf16_t*)dY, ldy, (const bf16_t*)W, ldw, (bf16_t*)dX, ldx, nullptr, M, C, R, tiles_m, C / 256,
+           part, whole, splits, chunk};
   static bool attr_set = false;
   if (!attr_set) {
-    HIP_RET(hipFuncSetAttribute((const void*)tgemm_nn_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, TG_LDS));
+    HIP_RET(hipFuncSetAttribute((const void*)tgemm_kernel<true, 0, true>, hipFuncAttributeMaxDynamicSharedMemorySize, TG_LDS + TG_OUT));
     attr_set = true;
   }
-  hipLaunchKernelGGL(tgemm_nn_kernel, dim3((unsigned)(tiles * splits)), dim3(512), TG_LDS, st, a);
+  hipLaunchKernelGGL((tgemm_kernel<true, 0, true>), dim3((unsigned)std::min(items, 256l)), dim3(512), TG_LDS + TG_OUT, st, a);
   if (splits > 1)
-    hipLaunchKernelGGL(tgemm_nn_sum_kernel, dim3((unsigned)(((size_t)M * C / 4 + 255) / 256)), dim3(256), 0, st, part, splits,
-                       (bf16_t*)dX, ldx, M, C);
+    hipLaunchKernelGGL(tgemm_nn_sum_kernel, dim3((unsigned)(tiles - whole) * 32), dim3(256), 0, st, a);
   return (int)hipGetLastError();
 }

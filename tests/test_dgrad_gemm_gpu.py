@@ -28,6 +28,21 @@ def test_dgrad(M, R, C, splits):
     assert bool(((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4).all())
 
 
+# full rounds of whole tiles, then the rest in parts: 264 tiles in 12 parts, 258 of 12 pairs, 520 with a ragged last row of tiles
+@pytest.mark.parametrize("M,R,C,plan", [(16641, 1536, 1024, (256, 12)), (256 * 43, 1664, 1536, (256, 13)), (33025, 384, 1024, (520, 1))])
+def test_whole_tiles_and_parts(M, R, C, plan):
+    g = torch.Generator(device=DEV).manual_seed(M)
+    dy = torch.full((M + 256, R + 8), float("nan"), device=DEV).bfloat16()[:M, :R]
+    w = torch.full((R + 64, C + 16), float("nan"), device=DEV).bfloat16()[:R, :C]
+    dy.copy_(torch.randn(M, R, device=DEV, generator=g))
+    w.copy_(torch.randn(R, C, device=DEV, generator=g) / R ** 0.5)
+    assert tg.dgrad_cost(M, R, C)[1:] == plan
+    got = tg.tgemm_nn(dy, w)
+    want = dy.double() @ w.double()
+    assert bool(((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4).all())  # one rounding, as above
+    assert torch.equal(got, tg.tgemm_nn(dy, w))
+
+
 def test_parts_have_work():
     for M in (1, 256, 700, 4096, 30000):
         for R in (128, 256, 1536, 17920, 151936):
