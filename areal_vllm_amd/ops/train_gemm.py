@@ -33,7 +33,7 @@ def supported(a: torch.Tensor, b: torch.Tensor, bias: Optional[torch.Tensor] = N
 
 
 def tgemm_tn(a: torch.Tensor, b: torch.Tensor, bias: Optional[torch.Tensor] = None,
-             out: Optional[torch.Tensor] = None, stagger: bool = True, max_blocks: int = 256) -> torch.Tensor:
+             out: Optional[torch.Tensor] = None, max_blocks: int = 256) -> torch.Tensor:
     """out[M, N] = a[M, K] @ b[N, K]^T (+ bias[N]); bf16 in, fp32 accumulation, bf16 out."""
     M, K = a.shape
     N = b.shape[0]
@@ -43,7 +43,7 @@ def tgemm_tn(a: torch.Tensor, b: torch.Tensor, bias: Optional[torch.Tensor] = No
     L.lib()
     L.check(L.lib().areal_tgemm_tn(L.ptr(a), L.c_int64(a.stride(0)), L.ptr(b), L.c_int64(b.stride(0)), L.ptr(out),
                                    L.c_int64(out.stride(0)), L.ptr(bias), L.c_int(M), L.c_int(N), L.c_int(K),
-                                   L.c_int(int(stagger)), L.c_int(int(max_blocks)), L.stream_ptr()), "tgemm_tn")
+                                   L.c_int(int(max_blocks)), L.stream_ptr()), "tgemm_tn")
     return out
 
 
@@ -70,33 +70,51 @@ def wgrad_supported(dy: torch.Tensor, x: torch.Tensor, acc: torch.Tensor) -> boo
     return dy.data_ptr() % 16 == 0 and x.data_ptr() % 16 == 0
 
 
-def tgemm_wgrad_(acc: torch.Tensor, dy: torch.Tensor, x: torch.Tensor, splits: int = 0, stagger: bool = True) -> torch.Tensor:
-    """acc[N, K] (fp32) += dy[M, N]^T @ x[M, K]: the weight gradient of ``y = x @ W^T`` summed straight into the
-    fp32 gradient buffer."""
-    assert wgrad_supported(dy, x, acc)
-    L.check(L.lib().areal_tgemm_wgrad(L.ptr(dy), L.c_int64(dy.stride(0)), L.ptr(x), L.c_int64(x.stride(0)), L.ptr(acc),
-                                      L.c_int64(acc.stride(0)), L.c_int(dy.shape[0]), L.c_int(dy.shape[1]),
-                                      L.c_int(x.shape[1]), L.c_int(int(splits)), L.c_int(int(stagger)), L.stream_ptr()),
-            "tgemm_wgrad")
-    return acc
+def _even_splits(pairs: int, splits: int) -> int:
+    """At most `splits` parts of `pairs`, none of them empty."""
+    splits = max(1, min(splits, pairs))
+    return -(-pairs // -(-pairs // splits))
 
 
 @functools.lru_cache(maxsize=1024)
-def dgrad_cost(M: int, R: int, C: int) -> Tuple[float, int, int]:
+def _tile_plan(pairs: int, tiles: int, flush: int) -> Tuple[float, int, int]:
     """(time in 128-deep pairs, 3 us each; tiles of 256 x 256 that one workgroup reduces; parts of the reduction of each of the
     others). A CU runs one workgroup: tiles beyond a multiple of 256 would leave CUs idle in a last round, so they are split
-    until the round is full. A part costs about 4 pairs more (its start, and its 256 KiB of fp32 written and read), the
-    kernel that sums the parts 2."""
-    pairs, tiles = R // 128, -(-M // 256) * (C // 256)
+    until the round is full. `flush`: pairs that writing a whole tile's result takes. A part costs 6 pairs more (its start, and
+    256 KiB of fp32 to write), a chip full of them 8 to be read and summed, the summing kernel itself 2: 48 tiles of 256 pairs in
+    5 parts take 183 us, 210 tiles in 6 parts (330 MB, more than the memory-side cache holds) 871, whole 745 (the 46 CUs that
+    idle leave their power to the others)."""
     rounds, rest = divmod(tiles, 256)
-    best = (float(-(-tiles // 256) * pairs), tiles, 1)
+    best = (float(-(-tiles // 256) * (pairs + flush)), tiles, 1)
     if rest:
         for s in range(2, min(pairs, 64) + 1):
             chunk = -(-pairs // s)
             if -(-pairs // chunk) == s:  # (every part has work)
-                cost = rounds * pairs + -(-rest * s // 256) * (chunk + 4) + 2 + 2 * s * rest / 256
+                cost = rounds * (pairs + flush) + -(-rest * s // 256) * (chunk + 6) + 2 + 8 * s * rest / 256
                 best = min(best, (cost, rounds * 256, s))
     return best
+
+
+def tgemm_wgrad_(acc: torch.Tensor, dy: torch.Tensor, x: torch.Tensor, splits: int = 0) -> torch.Tensor:
+    """acc[N, K] (fp32) += dy[M, N]^T @ x[M, K]: the weight gradient of ``y = x @ W^T`` summed straight into the
+    fp32 gradient buffer. `splits`: parts of the token range for every tile (0: chosen)."""
+    assert wgrad_supported(dy, x, acc)
+    (M, N), K = dy.shape, x.shape[1]
+    pairs, tiles = -(-M // 128), -(-N // 256) * (K // 256)
+    if splits:
+        splits = _even_splits(pairs, splits)
+        whole = 0 if splits > 1 else tiles
+    else:
+        _, whole, splits = _tile_plan(pairs, tiles, 3)
+    part = torch.empty(splits * (tiles - whole) << 16, dtype=torch.float32, device=dy.device) if splits > 1 else None
+    L.check(L.lib().areal_tgemm_wgrad(L.ptr(dy), L.c_int64(dy.stride(0)), L.ptr(x), L.c_int64(x.stride(0)), L.ptr(acc),
+                                      L.c_int64(acc.stride(0)), L.c_int(M), L.c_int(N), L.c_int(K), L.c_int(splits),
+                                      L.c_int(whole), L.ptr(part), L.stream_ptr()), "tgemm_wgrad")
+    return acc
+
+
+def dgrad_cost(M: int, R: int, C: int) -> Tuple[float, int, int]:
+    return _tile_plan(R // 128, -(-M // 256) * (C // 256), 0)
 
 
 def dgrad_splits(M: int, R: int, C: int) -> int:

@@ -18,9 +18,9 @@
 //       phase 1 -> A1 of tile t+1, phase 2 -> B0 of t+2, phase 3 -> A0 of t+2, phase 4 -> B1 of t+2.
 //     One counted wait per tile (phase 4: vmcnt(6) = the three newest pieces may still be in flight) makes tile t+1
 //     complete; it is read from the next phase on. Loads are never drained inside the loop.
-//   * raw s_barrier pairs around each MFMA cluster (s_setprio keeps hipcc from moving MFMAs across them); with
-//     STAGGER the waves of the second wave row run one barrier behind the first, so that one group's LDS reads and DMA
-//     issue overlap the other group's MFMA cluster (the two groups share every SIMD).
+//   * raw s_barrier pairs around each MFMA cluster (s_setprio keeps hipcc from moving MFMAs across them); the waves of the
+//     second wave row run one barrier behind the first, so that one group's LDS reads and DMA issue overlap the other
+//     group's MFMA cluster (the two groups share every SIMD).
 //   * LDS rows are 128 B; the XOR swizzle chunk ^ ((row >> 1) & 7) makes every 16-lane group of a ds_read_b128 hit 16
 //     different 16-byte slots. The DMA writes LDS linearly (wave base + lane x 16), so the swizzle sits on the per-lane
 //     SOURCE address and on the read address.
@@ -100,7 +100,7 @@ typedef f32x4 tg_acc[4][2];     // [m tile][n tile] of one quadrant
 // raised by the stores in flight, so that no wait stands behind one, the times are the same.
 // What is left is power: the matrix cores are busy 73 % of the time at a clock of 1.76 GHz (2.4 nominal); bare 16x16x32
 // products of random numbers run at 1.97 PFLOP/s on the whole chip, 32x32x16 ones at 1.75.
-template <bool STAGGER, int EPI, bool NN>
+template <int EPI, bool NN>
 __global__ __launch_bounds__(512) void tgemm_kernel(const TGArgs a) {
   constexpr int TN = EPI == 1 ? 128 : 256;  // output columns per tile
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -396,7 +396,7 @@ __global__ __launch_bounds__(512) void tgemm_kernel(const TGArgs a) {
   stage(1, PB1, 1);
   tg_vmcnt<6>();
   tg_barrier();
-  if (STAGGER && wr == 1) tg_barrier();
+  if (wr == 1) tg_barrier();  // the second wave row runs one barrier behind
 
   while (true) {
     const int nid = id + gridDim.x;
@@ -429,7 +429,7 @@ __global__ __launch_bounds__(512) void tgemm_kernel(const TGArgs a) {
     KT = nkt;
     part = npart;
   }
-  if (STAGGER && wr == 0) tg_barrier();
+  if (wr == 0) tg_barrier();
 }
 
 // =====================================================================================
@@ -438,15 +438,17 @@ __global__ __launch_bounds__(512) void tgemm_kernel(const TGArgs a) {
 // The same phase structure as above with the roles  rows -> n (columns of dY), columns -> k (columns of X), reduction
 // -> tokens. Both operands are stored with the REDUCTION index as the slow dimension, so the staged pieces are
 // token-major [64 tokens][128 columns] (256-byte rows, the swizzle of flash_tiles.hpp) and every MFMA operand is a pair
-// of transposed LDS reads (ds_read_b64_tr_b16: a lane receives 4 consecutive tokens of one column). 32x32x16 MFMA:
-// its transposed-read pattern (4 token rows x 64 contiguous bytes per 32 lanes) is conflict-free in that layout, and
-// a lane ends up with ONE k column per register, so a register is stored (or added) as 128 contiguous bytes per row.
+// of transposed LDS reads (ds_read_b64_tr_b16: a lane receives 4 consecutive tokens of one column; 8 rows of 32 bytes for
+// 32 lanes, which the swizzle puts on different banks).
 //   A0 / A1 = dY columns [0, 64) / [64, 128) of both wave rows; B0 / B1 = X columns [0, 32) / [32, 64) of all four
 //   wave columns - as for the forward kernel, pieces are what one phase reads.
-// grid = tiles x splits: a workgroup reduces `chunk` 128-token pairs of one output tile. A tile whose whole reduction
-// falls to one workgroup is added with a plain read-add-write; partial reductions are added with fp32 atomics (they
-// execute at the memory side, ~1.3 TB/s chip-wide), which is how a gradient of 48 tiles is reduced by four or five
-// workgroups per tile.
+// 16x16x32 products, not 32x32x16: the same rate on paper, but the kernel is limited by power and they need less of it
+// (17920 x 1536 over 32768 tokens: 1481 -> 1407 us).
+// A tile whose whole reduction falls to one workgroup is added with a plain read-add-write. The tiles that would leave CUs
+// idle in a last round are reduced by several workgroups, `chunk` 128-token pairs each, that write their sums as fp32 to
+// `part`; tgemm_wgrad_sum_kernel adds them. fp32 atomics on the gradient instead execute at the memory side, 1.3 TB/s
+// chip-wide, in any order; over 32768 tokens, us with atomics / with parts: 1536 x 1536 171 / 140, 2048 x 1536 197 / 184,
+// 17920 x 1536 1450 / 1412; over 16384: 2048 x 4096 263 / 225, 5120 x 2048 347 / 316.
 // =====================================================================================
 struct TWArgs {
   const bf16_t* dY;
@@ -460,9 +462,20 @@ struct TWArgs {
   int pairs;          // 128-token pairs of K tiles in M, the last one possibly ragged
   int whole;          // the first `whole` tiles are reduced by one workgroup each
   int splits, chunk;  // the others: workgroups per tile, pairs per workgroup (the last one of a tile may get fewer)
+  float* part;        // [tile - whole][splits][wave][m half][n half][mt][nt][lane][4]
 };
 
-template <bool STAGGER>
+typedef f32x4 __attribute__((aligned(4))) f32x4u;
+
+DEVINL void tg_wgrad_origin(const TWArgs& a, int wg, int& n0, int& k0) {
+  const int per_band = TG_GROUP_M * a.tiles_k;
+  const int band = wg / per_band, first = band * TG_GROUP_M;
+  const int rows = min(a.tiles_n - first, TG_GROUP_M);
+  const int in_band = wg - band * per_band;
+  n0 = (first + in_band % rows) * 256;
+  k0 = (in_band / rows) * 256;
+}
+
 __global__ __launch_bounds__(512) void tgemm_wgrad_kernel(const TWArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int lane = threadIdx.x & 63;
@@ -484,15 +497,6 @@ __global__ __launch_bounds__(512) void tgemm_wgrad_kernel(const TWArgs a) {
     b_split = (b - a.whole) - (b_tile - a.whole) * a.splits;
     b_chunk = a.chunk;
   }
-  auto tile_origin = [&](int wg, int& n0, int& k0) __attribute__((always_inline)) {
-    const int per_band = TG_GROUP_M * a.tiles_k;
-    const int band = wg / per_band, first = band * TG_GROUP_M;
-    const int rows = min(a.tiles_n - first, TG_GROUP_M);
-    const int in_band = wg - band * per_band;
-    n0 = (first + in_band % rows) * 256;
-    k0 = (in_band / rows) * 256;
-  };
-
   // ---- staging: thread -> token row (wave * 4 + lane / 16) of a 32-row issue, physical 16-byte chunk lane & 15
   const int srow = wave * 4 + (lane >> 4);
   const int pc = ((lane & 15) ^ (((lane >> 4) << 2) | (wave & 3))) * 8;  // piece column whose chunk lands here
@@ -592,8 +596,7 @@ __global__ __launch_bounds__(512) void tgemm_wgrad_kernel(const TWArgs a) {
   // ---- one segment: pairs [p0, p1) of one output tile
   int n0, k0;
   const int p0 = b_split * b_chunk, p1 = min(a.pairs, p0 + b_chunk);
-  tile_origin(b_tile, n0, k0);
-  const bool whole = p0 == 0 && p1 == a.pairs;
+  tg_wgrad_origin(a, b_tile, n0, k0);
   const int tok0 = p0 * 128, KT = (p1 - p0) * 2;
   tokens = a.M - tok0;
   // N may end half way through the last tile row (N % 256 == 128): the second wave row then re-reads the first
@@ -621,7 +624,7 @@ __global__ __launch_bounds__(512) void tgemm_wgrad_kernel(const TWArgs a) {
   stage(1, PB1, 1);
   tg_vmcnt<6>();
   tg_barrier();
-  if (STAGGER && wr == 1) tg_barrier();
+  if (wr == 1) tg_barrier();  // the second wave row runs one barrier behind
   int t = 0;
   for (; t + 2 < KT; t += 2) {
     tile(B0{}, t, T0{});
@@ -629,15 +632,28 @@ __global__ __launch_bounds__(512) void tgemm_wgrad_kernel(const TWArgs a) {
   }
   tile(B0{}, t, T1{});
   tile(B1{}, t + 1, T2{});
-  if (STAGGER && wr == 0) tg_barrier();  // from here on nobody reads a staged tile: a wave has 16 KiB of LDS to itself
+  if (wr == 0) tg_barrier();  // from here on nobody reads a staged tile: a wave has 16 KiB of LDS to itself
 
-  // ---- lane (row fr, fq) of tile (mt, nt) holds 4 consecutive k columns. A row half (64 x 64 fp32) passes through the wave's
-  // LDS: plain adds move 256 bytes of four rows an instruction, atomic ones 256 bytes of one.
+  // ---- lane (row fr, fq) of tile (mt, nt) holds 4 consecutive k columns
   if (half_n && wr == 1) return;
+  if (b >= a.whole) {
+    f32x4* pp = reinterpret_cast<f32x4*>(a.part + ((size_t)(b - a.whole) << 16)) + wave * 2048 + lane;
+    auto put = [&](tg_acc& acc, int q) __attribute__((always_inline)) {
+#pragma unroll
+      for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt) pp[(q * 8 + mt * 2 + nt) * 64] = acc[mt][nt];
+    };
+    put(acc00, 0);
+    put(acc01, 1);
+    put(acc10, 2);
+    put(acc11, 3);
+    return;
+  }
+  // a row half (64 x 64 fp32) passes through the wave's LDS: an instruction then moves 256 bytes of four rows
   char* ob = smem + wave * 16384;
   auto flush = [&](tg_acc& c0, tg_acc& c1, int mh) __attribute__((always_inline)) {
     float* op = a.dW + (size_t)(n0 + wr * 128 + mh * 64) * a.ldw + k0 + wc * 64;
-    typedef f32x4 __attribute__((aligned(4))) f32x4u;
 #pragma unroll
     for (int mt = 0; mt < 4; ++mt)
 #pragma unroll
@@ -645,29 +661,45 @@ __global__ __launch_bounds__(512) void tgemm_wgrad_kernel(const TWArgs a) {
 #pragma unroll
         for (int nt = 0; nt < 2; ++nt)
           *reinterpret_cast<f32x4*>(ob + (mt * 16 + fr) * 256 + (((nh * 8 + nt * 4 + fq) ^ fr) << 4)) = (nh ? c1 : c0)[mt][nt];
-    if (whole) {
 #pragma unroll
-      for (int i0 = 0; i0 < 16; i0 += 8) {
-        f32x4 old[8];
+    for (int i0 = 0; i0 < 16; i0 += 8) {
+      f32x4 old[8];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) old[i] = *reinterpret_cast<const f32x4u*>(op + (size_t)((i0 + i) * 4 + fq) * a.ldw + fr * 4);
+      for (int i = 0; i < 8; ++i) old[i] = *reinterpret_cast<const f32x4u*>(op + (size_t)((i0 + i) * 4 + fq) * a.ldw + fr * 4);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const int row = (i0 + i) * 4 + fq;
-          const f32x4 v = *reinterpret_cast<const f32x4*>(ob + row * 256 + ((fr ^ (row & 15)) << 4));
-          *reinterpret_cast<f32x4u*>(op + (size_t)row * a.ldw + fr * 4) = old[i] + v;
-        }
-      }
-    } else {
-#pragma unroll 16
-      for (int row = 0; row < 64; ++row) {
-        const float v = *reinterpret_cast<const float*>(ob + row * 256 + (((lane >> 2) ^ (row & 15)) << 4) + (lane & 3) * 4);
-        unsafeAtomicAdd(op + (size_t)row * a.ldw + lane, v);
+      for (int i = 0; i < 8; ++i) {
+        const int row = (i0 + i) * 4 + fq;
+        const f32x4 v = *reinterpret_cast<const f32x4*>(ob + row * 256 + ((fr ^ (row & 15)) << 4));
+        *reinterpret_cast<f32x4u*>(op + (size_t)row * a.ldw + fr * 4) = old[i] + v;
       }
     }
   };
   flush(acc00, acc01, 0);
   flush(acc10, acc11, 1);
+}
+
+// dW += the parts of the tiles from `whole` on, in order. Block: 32 rows x 64 columns of a tile (a wave's quarter of a row
+// half); a thread has 4 columns of 2 of the rows, 8 threads a 128-byte line.
+__global__ __launch_bounds__(256) void tgemm_wgrad_sum_kernel(const TWArgs a) {
+  const int t = blockIdx.x >> 5, wave = (blockIdx.x >> 2) & 7, mh = (blockIdx.x >> 1) & 1, mt2 = blockIdx.x & 1;
+  int n0, k0;
+  tg_wgrad_origin(a, a.whole + t, n0, k0);
+  const int fq = threadIdx.x & 3, nt = (threadIdx.x >> 2) & 1, nh = (threadIdx.x >> 3) & 1, fr = threadIdx.x >> 4;
+  if (n0 + (wave >> 2) * 128 >= a.N) return;
+  const f32x4* p = reinterpret_cast<const f32x4*>(a.part + ((size_t)t * a.splits << 16)) + wave * 2048 +
+                   ((mh * 2 + nh) * 8 + mt2 * 4 + nt) * 64 + fq * 16 + fr;
+  float* op = a.dW + (size_t)(n0 + (wave >> 2) * 128 + mh * 64 + mt2 * 32 + fr) * a.ldw + k0 + (wave & 3) * 64 + nh * 32 + nt * 16 + fq * 4;
+  f32x4u* o0 = reinterpret_cast<f32x4u*>(op);
+  f32x4u* o1 = reinterpret_cast<f32x4u*>(op + 16 * a.ldw);
+  f32x4 v0 = p[0], v1 = p[128];
+  const f32x4 d0 = *o0, d1 = *o1;
+#pragma unroll 4
+  for (int s = 1; s < a.splits; ++s) {
+    v0 += p[(size_t)s << 14];
+    v1 += p[((size_t)s << 14) + 128];
+  }
+  *o0 = d0 + v0;
+  *o1 = d1 + v1;
 }
 
 // =====================================================================================
@@ -705,7 +737,7 @@ __global__ __launch_bounds__(256) void tgemm_nn_sum_kernel(const TGArgs a) {
 // One launch = min(tiles, max_blocks) persistent workgroups (256 = one per CU).
 // gated = 1: B holds 2 N rows (gate rows, then up rows), C[M, N] = silu(A.gate^T) * (A.up^T), no bias.
 static int tgemm_tn_launch(const void* A, long lda, const void* B, long ldb, void* C, long ldc, const void* bias, int M,
-                           int N, int K, int stagger, int max_blocks, int gated, hipStream_t st) {
+                           int N, int K, int max_blocks, int gated, hipStream_t st) {
   if (M <= 0 || N <= 0) return 0;
   if (K % 128 != 0 || N % 4 != 0 || lda % 8 != 0 || ldb % 8 != 0 || ldc % 4 != 0) return -1;
   if (((uintptr_t)A | (uintptr_t)B) % 16 != 0 || (uintptr_t)C % 8 != 0 || (bias && (uintptr_t)bias % 8 != 0)) return -1;
@@ -714,9 +746,8 @@ static int tgemm_tn_launch(const void* A, long lda, const void* B, long ldb, voi
            (M + 255) / 256, gated ? (N + 127) / 128 : (N + 255) / 256, nullptr, 0, 1, 0};
   static bool attr_set = false;  // 128 KiB of dynamic LDS: above the default limit
   if (!attr_set) {
-    HIP_RET(hipFuncSetAttribute((const void*)tgemm_kernel<true, 0, false>, hipFuncAttributeMaxDynamicSharedMemorySize, TG_LDS + TG_OUT));
-    HIP_RET(hipFuncSetAttribute((const void*)tgemm_kernel<false, 0, false>, hipFuncAttributeMaxDynamicSharedMemorySize, TG_LDS + TG_OUT));
-    HIP_RET(hipFuncSetAttribute((const void*)tgemm_kernel<true, 1, false>, hipFuncAttributeMaxDynamicSharedMemorySize, TG_LDS));
+    HIP_RET(hipFuncSetAttribute((const void*)tgemm_kernel<0, false>, hipFuncAttributeMaxDynamicSharedMemorySize, TG_LDS + TG_OUT));
+    HIP_RET(hipFuncSetAttribute((const void*)tgemm_kernel<1, false>, hipFuncAttributeMaxDynamicSharedMemorySize, TG_LDS));
     attr_set = true;
   }
   // max_blocks workgroups (a multiple of 8: block id mod 8 is the XCD for every tile of a block's sequence) walk the
@@ -725,17 +756,15 @@ static int tgemm_tn_launch(const void* A, long lda, const void* B, long ldb, voi
   if (max_blocks > 0 && max_blocks % 8 != 0) return -1;
   const dim3 grid(max_blocks > 0 ? std::min(ntiles, max_blocks) : ntiles), block(512);
   if (gated)
-    hipLaunchKernelGGL((tgemm_kernel<true, 1, false>), grid, block, TG_LDS, st, a);
-  else if (stagger)
-    hipLaunchKernelGGL((tgemm_kernel<true, 0, false>), grid, block, TG_LDS + TG_OUT, st, a);
+    hipLaunchKernelGGL((tgemm_kernel<1, false>), grid, block, TG_LDS, st, a);
   else
-    hipLaunchKernelGGL((tgemm_kernel<false, 0, false>), grid, block, TG_LDS + TG_OUT, st, a);
+    hipLaunchKernelGGL((tgemm_kernel<0, false>), grid, block, TG_LDS + TG_OUT, st, a);
   return (int)hipGetLastError();
 }
 
 extern "C" int areal_tgemm_tn(const void* A, long lda, const void* B, long ldb, void* C, long ldc, const void* bias,
-                              int M, int N, int K, int stagger, int max_blocks, hipStream_t st) {
-  return tgemm_tn_launch(A, lda, B, ldb, C, ldc, bias, M, N, K, stagger, max_blocks, 0, st);
+                              int M, int N, int K, int max_blocks, hipStream_t st) {
+  return tgemm_tn_launch(A, lda, B, ldb, C, ldc, bias, M, N, K, max_blocks, 0, st);
 }
 
 // C[M, F] = silu(A . Wg^T) * (A . Wu^T) with W = [Wg; Wu] of shape [2 F, K] (the gate|up projection of a gated MLP and
@@ -743,73 +772,38 @@ extern "C" int areal_tgemm_tn(const void* A, long lda, const void* B, long ldb, 
 // activations (scoring, prefill).
 extern "C" int areal_tgemm_swiglu(const void* A, long lda, const void* W, long ldw, void* C, long ldc, int M, int F,
                                   int K, int max_blocks, hipStream_t st) {
-  return tgemm_tn_launch(A, lda, W, ldw, C, ldc, nullptr, M, F, K, 1, max_blocks, 1, st);
+  return tgemm_tn_launch(A, lda, W, ldw, C, ldc, nullptr, M, F, K, max_blocks, 1, st);
 }
 
 // dW[N, K] (fp32, leading dimension ldw) += dY[M, N]^T . X[M, K]. N a multiple of 128, K of 256, rows 16-byte aligned.
-// splits: 0 = chosen. A ragged last 128-token pair is filled up with zeros: handing its few tokens to a library GEMM
+// The first `whole` tiles of 256 x 256 (a multiple of 256, or all of them: splits = 1) are reduced by one workgroup each, the
+// others in `splits` parts; part: splits x 65536 floats for each of those. Every part has to have work, as for areal_tgemm_nn.
+// A ragged last 128-token pair is filled up with zeros: handing its few tokens to a library GEMM
 // instead reads and writes the whole fp32 gradient a second time (60 tokens: 51 us for 17920 x 1536, 507 us for the
 // 151936 x 1536 LM head, 1.4 of the 9.2 ms of a pass over 700 tokens and 7 layers).
 extern "C" int areal_tgemm_wgrad(const void* dY, long ldy, const void* X, long ldx, float* dW, long ldw, int M, int N,
-                                 int K, int splits, int stagger, hipStream_t st) {
+                                 int K, int splits, int whole, float* part, hipStream_t st) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   if (N % 128 != 0 || K % 256 != 0 || ldy % 8 != 0 || ldx % 8 != 0) return -1;
   if (ldy < N || ldx < K) return -1;  // the loads end at the last row's last byte: rows must not overlap
   if (ldy > (1l << 24) || ldx > (1l << 24)) return -1;  // byte offsets of 64 rows: 32 bits
-  if (((uintptr_t)dY | (uintptr_t)X) % 16 != 0 || (uintptr_t)dW % 4 != 0) return -1;
-  const int tiles = ((N + 255) / 256) * (K / 256), pairs = (M + 127) / 128;
-  // splits >= 1: that many workgroups per tile (1 = every tile added without atomics). splits <= 0: choose. Blocks run
-  // in rounds of 256 (one per CU); a block costs its share of the pairs (~3.1 us each) plus ~8 us of prologue and
-  // flush, ~25 us more when the tile is flushed with atomic adds (a CU retires one 256-byte atomic instruction per
-  // ~50 ns) - so splitting pays for gradients of few tiles (qkv: 48 tiles x 4) and not for 210 or 420 tiles. An even
-  // deal of ALL work over 256 workgroups (stream-K, nearly every tile partial) was measured 20-25 % slower than whole
-  // tiles for those.
-  // With more than 256 tiles the full rounds run whole tiles and only the tiles of the last, partly filled round are
-  // split (420 tiles: 256 whole + 164 x 3).
-  int whole = 0;
-  if (splits <= 0) {
-    auto block_us = [&](int s) { return ((pairs + s - 1) / s) * 3.1 + 8.0 + (s > 1 ? 25.0 : 0.0); };
-    const int full = tiles / 256 * 256, rest = tiles - full;
-    double best = 1e30;
-    for (int s = 1; s <= 16 && pairs / s >= 4; ++s) {
-      const int chunk = (pairs + s - 1) / s;
-      if ((pairs + chunk - 1) / chunk != s) continue;  // this count leaves a workgroup without work
-      // every tile split s ways
-      double t = ((tiles * s + 255) / 256) * block_us(s);
-      if (t < best - 1e-9) {
-        best = t;
-        splits = s;
-        whole = s == 1 ? tiles : 0;
-      }
-      // full rounds whole, the rest split s ways
-      if (full > 0 && rest > 0 && s > 1) {
-        t = (full / 256) * block_us(1) + ((rest * s + 255) / 256) * block_us(s);
-        if (t < best - 1e-9) {
-          best = t;
-          splits = s;
-          whole = full;
-        }
-      }
-    }
-  } else if (splits == 1) {
-    whole = tiles;
-  }
-  splits = std::max(1, std::min(splits, pairs));
+  if (((uintptr_t)dY | (uintptr_t)X) % 16 != 0 || (uintptr_t)dW % 4 != 0 || (uintptr_t)part % 16 != 0) return -1;
+  const int pairs = (M - 1) / 128 + 1;
+  const long tiles = (long)((N + 255) / 256) * (K / 256);
+  if (splits < 1 || splits > pairs || whole < 0 || whole > tiles) return -1;
+  if (splits == 1 ? whole != tiles : whole % 256 != 0 || whole == tiles || !part) return -1;
   const int chunk = (pairs + splits - 1) / splits;
-  splits = (pairs + chunk - 1) / chunk;
-  const int nblocks = whole + (tiles - whole) * splits;
-  TWArgs a{(const bf16_t*)dY, ldy, (const bf16_t*)X, ldx, dW, ldw, M, N, K, (N + 255) / 256, K / 256, pairs, whole, splits, chunk};
+  if ((pairs + chunk - 1) / chunk != splits) return -1;
+  const long nblocks = whole + (tiles - whole) * splits;
+  if (nblocks > 0x7fffffffl || (tiles - whole) > (0x7fffffffl >> 5)) return -1;
+  TWArgs a{(const bf16_t*)dY, ldy, (const bf16_t*)X, ldx, dW, ldw, M, N, K, (N + 255) / 256, K / 256, pairs, whole, splits, chunk, part};
   static bool attr_set = false;
   if (!attr_set) {
-    HIP_RET(hipFuncSetAttribute((const void*)tgemm_wgrad_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, TG_LDS));
-    HIP_RET(hipFuncSetAttribute((const void*)tgemm_wgrad_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize, TG_LDS));
+    HIP_RET(hipFuncSetAttribute((const void*)tgemm_wgrad_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, TG_LDS));
     attr_set = true;
   }
-  const dim3 grid(nblocks), block(512);
-  if (stagger)
-    hipLaunchKernelGGL(tgemm_wgrad_kernel<true>, grid, block, TG_LDS, st, a);
-  else
-    hipLaunchKernelGGL(tgemm_wgrad_kernel<false>, grid, block, TG_LDS, st, a);
+  hipLaunchKernelGGL(tgemm_wgrad_kernel, dim3((unsigned)nblocks), dim3(512), TG_LDS, st, a);
+  if (splits > 1) hipLaunchKernelGGL(tgemm_wgrad_sum_kernel, dim3((unsigned)(tiles - whole) * 32), dim3(256), 0, st, a);
   return (int)hipGetLastError();
 }
 
@@ -835,10 +829,10 @@ extern "C" int areal_tgemm_nn(const void* dY, long ldy, const void* W, long ldw,
            part, whole, splits, chunk};
   static bool attr_set = false;
   if (!attr_set) {
-    HIP_RET(hipFuncSetAttribute((const void*)tgemm_kernel<true, 0, true>, hipFuncAttributeMaxDynamicSharedMemorySize, TG_LDS + TG_OUT));
+    HIP_RET(hipFuncSetAttribute((const void*)tgemm_kernel<0, true>, hipFuncAttributeMaxDynamicSharedMemorySize, TG_LDS + TG_OUT));
     attr_set = true;
   }
-  hipLaunchKernelGGL((tgemm_kernel<true, 0, true>), dim3((unsigned)std::min(items, 256l)), dim3(512), TG_LDS + TG_OUT, st, a);
+  hipLaunchKernelGGL((tgemm_kernel<0, true>), dim3((unsigned)std::min(items, 256l)), dim3(512), TG_LDS + TG_OUT, st, a);
   if (splits > 1)
     hipLaunchKernelGGL(tgemm_nn_sum_kernel, dim3((unsigned)(tiles - whole) * 32), dim3(256), 0, st, a);
   return (int)hipGetLastError();

@@ -23,7 +23,7 @@ def test_row_strides(ldy, ldx, taken):
     if not taken:
         p = L.c_void_p(1 << 20)  # never read: the entry refuses the strides first
         assert L.lib().areal_tgemm_wgrad(p, L.c_int64(ldy), p, L.c_int64(ldx), p, L.c_int64(256), L.c_int(1024), L.c_int(128),
-                                         L.c_int(256), L.c_int(0), L.c_int(1), L.c_void_p(0)) == -1
+                                         L.c_int(256), L.c_int(1), L.c_int(1), L.c_void_p(0), L.c_void_p(0)) == -1
 
 
 @pytest.mark.parametrize("which", range(4))
