@@ -226,12 +226,20 @@ class _LMHeadLogprobFn(torch.autograd.Function):
         stats = torch.empty(4, T, dtype=torch.float32, device=hidden.device)
         need_grad = hidden.requires_grad or weight.requires_grad
         kept = []
+        whole = None
+        if need_grad and keep_logits and T > chunk and weight.dtype == hidden.dtype and weight.shape[0] % 8 == 0:
+            # one tensor for all chunks: the backward then works on all rows at once
+            whole = torch.empty(T, weight.shape[0], dtype=hidden.dtype, device=hidden.device)
+            kept.append(whole)
         for s in range(0, T, chunk):
             e = min(T, s + chunk)
-            lg = _chunk_logits(hidden[s:e], weight)
+            if whole is not None:
+                lg = torch.mm(hidden[s:e], weight.t(), out=whole[s:e])
+            else:
+                lg = _chunk_logits(hidden[s:e], weight)
+                if need_grad and keep_logits:
+                    kept.append(lg)
             logprob_stats(lg, labels[s:e], temperature, vocab_start, out=stats[:, s:e])
-            if need_grad and keep_logits:
-                kept.append(lg)
         logp, ent, lse, ez = _finalize(*merge_shard_stats(stats, group))
         ctx.save_for_backward(hidden, weight, labels, lse, ez, *kept)
         ctx.meta = (temperature, chunk, keep_logits, vocab_start, group, reduce_dh)
@@ -252,9 +260,17 @@ class _LMHeadLogprobFn(torch.autograd.Function):
         direct = mg is not None and hidden.is_cuda and mg.dtype == torch.float32 and mg.shape == weight.shape
         if direct:
             dw = None
+        whole = kept[0] if keep_logits and T > chunk and kept[0].shape[0] == T else None
+        if whole is not None and direct and train_gemm.wgrad_supported(whole, hidden, mg) and train_gemm.dgrad_supported(whole, weight):
+            # the fp32 gradient of the head is read and added to once instead of once a chunk (1.9 GB of traffic each for a
+            # 151936 x 1536 head), and the products' tiles fill whole rounds of the chip
+            chunk = T
         for i, s in enumerate(range(0, T, chunk)):
             e = min(T, s + chunk)
-            lg = kept[i] if keep_logits else _chunk_logits(hidden[s:e], weight)
+            if whole is not None:
+                lg = whole[s:e]
+            else:
+                lg = kept[i] if keep_logits else _chunk_logits(hidden[s:e], weight)
             _bwd_inplace(lg, labels[s:e], temperature, lse[s:e], ez[s:e],
                          dlogp[s:e] if dlogp is not None else None, dent[s:e] if dent is not None else None,
                          vocab_start)
