@@ -28,11 +28,45 @@ def _hip_ok(x, w) -> bool:
             and w.shape[2] % 64 == 0)
 
 
+# Rows an expert, on average, from which tiles of 256 x 256 (the trainer's dense kernels, operands by LDS-DMA) are the better
+# ones although an expert's last row tile is half empty. us of the 64 / 128-row kernels and of these, out / dx / dW:
+# 128 experts, 1536 columns, 2048 deep: 64 rows 215 / 198 / 631 and 169 / 177 / 622, 128 321 / 261 / 651 and 225 / 229 / 650,
+# 512 669 / 633 / 1037 and 425 / 494 / 862, 1024 1131 / 1123 / 1595 and 729 / 800 / 1163; 2048 columns, 768 deep: 64 99 / 128 /
+# 311 and 114 / 111 / 330, 128 134 / 201 / 322 and 134 / 119 / 307, 1024 628 / 746 / 846 and 430 / 389 / 599; 32 experts, 1024 by
+# 1024: 64 21 / 22 / 46 and 28 / 29 / 47, 128 28 / 29 / 52 and 29 / 30 / 50.
+BIG_MIN_ROWS = 128
+# dW of large experts with few rows is all reading and writing of the gradient, which the small tiles (two workgroups a CU)
+# overlap better: 8 experts, 28672 columns, 4096 deep, 256 / 1024 / 2048 rows 1569 / 3397 / 5774 and 1860 / 3655 / 4938.
+BIG_WGRAD_MAX_SIZE, BIG_WGRAD_ANY_SIZE_ROWS = 1 << 24, 2048
+
+
+def _big_tiles(T: int, E: int) -> bool:
+    return "AREAL_GROUPED_GEMM_TILE_M" not in os.environ and T >= BIG_MIN_ROWS * E
+
+
+def _big_wgrad(T: int, E: int, N: int, K: int) -> bool:
+    return _big_tiles(T, E) and K % 256 == 0 and (N * K <= BIG_WGRAD_MAX_SIZE or T >= BIG_WGRAD_ANY_SIZE_ROWS * E)
+
+
+def big_grouped(x: torch.Tensor, w: torch.Tensor, offsets: torch.Tensor, nn: bool) -> torch.Tensor:
+    """x[t] @ W[e]^T, or with `nn` x[t] @ W[e], on tiles of 256 x 256 (``csrc/hip/train_gemm.hip``)."""
+    T, K = x.shape
+    E, N = w.shape[0], w.shape[2 if nn else 1]
+    out = torch.empty(T, N, dtype=x.dtype, device=x.device)
+    table = torch.empty(4 * (T // 256 + E + 1), dtype=torch.int32, device=x.device)
+    L.check(L.lib().areal_tgemm_grouped(L.ptr(x), L.ptr(w), L.ptr(out), L.ptr(offsets), L.ptr(table), L.c_int(T), L.c_int(E),
+                                        L.c_int(N), L.c_int(K), L.c_int64(w.stride(0)), L.c_int(int(nn)), L.stream_ptr()),
+            "tgemm_grouped")
+    return out
+
+
 def _launch(x: torch.Tensor, w: torch.Tensor, offsets: torch.Tensor) -> torch.Tensor:
     T, K = x.shape
     E, N, K2 = w.shape
     assert K == K2 and offsets.numel() == E + 1 and offsets.dtype == torch.int32 and offsets.is_cuda
     assert x.is_contiguous() and w.stride(2) == 1 and w.stride(1) == K, "operands must be K-contiguous"
+    if K % 128 == 0 and w.stride(0) % 8 == 0 and _big_tiles(T, E):
+        return big_grouped(x, w, offsets, False)
     out = torch.empty(T, N, dtype=x.dtype, device=x.device)
     tile_m = int(os.environ.get("AREAL_GROUPED_GEMM_TILE_M", "0"))  # 0: chosen from the rows per expert
     tm = L.lib().areal_grouped_gemm_tile_m(L.c_int(T), L.c_int(E), L.c_int(N), L.c_int(tile_m))
@@ -70,7 +104,9 @@ class _GroupedGemmFn(torch.autograd.Function):
         dx = dw = None
         E, N, K = w.shape
         if ctx.needs_input_grad[0]:
-            if K % 128 == 0:
+            if N % 128 == 0 and K % 256 == 0 and _big_tiles(dy.shape[0], E) and w.is_contiguous():
+                dx = big_grouped(dy, w, offsets, True)
+            elif K % 128 == 0:
                 # dx[t] = dy[t] @ W[e]: the weights are read as they are (transposed LDS reads in the kernel)
                 T = dy.shape[0]
                 dx = torch.empty(T, K, dtype=dy.dtype, device=dy.device)
@@ -88,6 +124,12 @@ class _GroupedGemmFn(torch.autograd.Function):
                 # carries an fp32 `main_grad` view the kernel adds into it (no bf16 dW, no separate add kernel)
                 mg = _fold_target(w)
                 dst = mg if mg is not None else torch.empty_like(w)
+                if mg is not None and _big_wgrad(x.shape[0], E, N, K):
+                    L.check(L.lib().areal_tgemm_grouped_wgrad(L.ptr(dy), L.ptr(x), L.ptr(mg), L.ptr(offsets), L.c_int(E),
+                                                              L.c_int(N), L.c_int(K), L.c_int64(mg.stride(0)),
+                                                              L.stream_ptr()), "tgemm_grouped_wgrad")
+                    _after_fold(w)
+                    return dx, None, None, None
                 L.check(L.lib().areal_grouped_gemm_wgrad(L.ptr(dy), L.ptr(x), L.ptr(dst), L.ptr(offsets),
                                                          L.c_int(x.shape[0]), L.c_int(E), L.c_int(N), L.c_int(K),
                                                          L.c_int64(dst.stride(0)), L.c_int(int(mg is not None)),

@@ -56,7 +56,12 @@ struct TGArgs {
   // part [splits][tile - whole][256][256] fp32
   float* part;
   int whole, splits, chunk;
+  // grouped (GRP): rows sorted by expert, B [experts][..] `stride` elements apart; table[0] = row tiles of all experts, then
+  // one entry {first row, end of the expert's rows, expert} a row tile, written by tgemm_table_kernel
+  const int4* table;
+  long stride;
 };
+typedef const __attribute__((address_space(4))) int4* tg_table_t;  // scalar loads
 
 constexpr int TG_PIECE = 128 * 128;   // bytes of one staged piece
 constexpr int TG_BUF = 4 * TG_PIECE;  // A0 A1 B0 B1 of one K tile
@@ -100,7 +105,10 @@ typedef f32x4 tg_acc[4][2];     // [m tile][n tile] of one quadrant
 // raised by the stores in flight, so that no wait stands behind one, the times are the same.
 // What is left is power: the matrix cores are busy 73 % of the time at a clock of 1.76 GHz (2.4 nominal); bare 16x16x32
 // products of random numbers run at 1.97 PFLOP/s on the whole chip, 32x32x16 ones at 1.75.
-template <int EPI, bool NN>
+//
+// GRP: the same product for rows sorted by expert, each expert's with its own B (routed experts). A row tile never straddles
+// two experts; its tail rows repeat the expert's last one and are not stored.
+template <int EPI, bool NN, bool GRP>
 __global__ __launch_bounds__(512) void tgemm_kernel(const TGArgs a) {
   constexpr int TN = EPI == 1 ? 128 : 256;  // output columns per tile
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -109,29 +117,47 @@ __global__ __launch_bounds__(512) void tgemm_kernel(const TGArgs a) {
   const int wr = wave >> 2, wc = wave & 3;
 
   // ---- tile sequence number -> output tile
-  const int tiles = a.tiles_m * a.tiles_n, whole = NN ? a.whole : tiles;
-  const int ntiles = NN ? whole + (tiles - whole) * a.splits : tiles;  // work items
-  auto tile_origin = [&](int id, int& m0, int& n0, int& k0, int& kt, float*& part) __attribute__((always_inline)) {
-    const bool in_part = NN && id >= whole;
+  const tg_table_t table = (tg_table_t)a.table;
+  const int tiles_m = GRP ? table[0].x : a.tiles_m;
+  const int tiles = tiles_m * a.tiles_n, whole = NN && !GRP ? a.whole : tiles;
+  const int ntiles = NN && !GRP ? whole + (tiles - whole) * a.splits : tiles;  // work items
+  if (GRP && (int)blockIdx.x >= ntiles) return;  // (the grid is an upper bound)
+  struct Tile {
+    int m0, n0, k0, kt, mlim, e;  // origin; reduction from k0 on, K tiles; end of the rows; expert
+    float* part;
+  };
+  auto tile_origin = [&](int id) __attribute__((always_inline)) {
+    Tile t;
+    const bool in_part = NN && !GRP && id >= whole;
     const int base = in_part ? whole : 0, nb = in_part ? ntiles - whole : whole;
     const int q = nb >> 3, r = nb & 7, x = (id - base) & 7;
     int wg = base + (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + ((id - base) >> 3);
-    k0 = 0;
-    kt = a.K >> 6;
-    part = nullptr;
+    t.k0 = 0;
+    t.kt = a.K >> 6;
+    t.part = nullptr;
     if (in_part) {  // part by part: what runs together on an XCD shares the reduction range
       const int rest = tiles - whole, split = (wg - whole) / rest;
-      part = a.part + ((size_t)(wg - whole) << 16);
+      t.part = a.part + ((size_t)(wg - whole) << 16);
       wg -= split * rest;
-      k0 = split * a.chunk * 128;
-      kt = min(kt - split * a.chunk * 2, a.chunk * 2);
+      t.k0 = split * a.chunk * 128;
+      t.kt = min(t.kt - split * a.chunk * 2, a.chunk * 2);
     }
     const int per_band = TG_GROUP_M * a.tiles_n;
     const int band = wg / per_band, first = band * TG_GROUP_M;
-    const int rows = min(a.tiles_m - first, TG_GROUP_M);
+    const int rows = min(tiles_m - first, TG_GROUP_M);
     const int in_band = wg - band * per_band;
-    m0 = (first + in_band % rows) * 256;
-    n0 = (in_band / rows) * TN;
+    t.n0 = (in_band / rows) * TN;
+    const int mt = first + in_band % rows;
+    if (GRP) {
+      t.m0 = table[1 + mt].x;
+      t.mlim = table[1 + mt].y;
+      t.e = table[1 + mt].z;
+    } else {
+      t.m0 = mt * 256;
+      t.mlim = a.M;
+      t.e = 0;
+    }
+    return t;
   };
 
   // ---- staging: thread -> row (wave * 8 + lane / 8) of a 64-row issue, physical chunk lane & 7
@@ -143,17 +169,19 @@ __global__ __launch_bounds__(512) void tgemm_kernel(const TGArgs a) {
   const size_t stepB = NN ? (size_t)64 * a.ldb : 64;  // elements of B from K tile to K tile
   const bf16_t* srcA[2][2];  // [piece][issue]
   const bf16_t* srcB[2][2];
-  auto set_sources = [&](int m0, int n0, int k0) __attribute__((always_inline)) {
+  auto set_sources = [&](const Tile& t) __attribute__((always_inline)) {
+    const int m0 = t.m0, n0 = t.n0, k0 = t.k0;
+    const bf16_t* B = GRP ? a.B + t.e * a.stride : a.B;
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
         int row = m0 + i * 128 + h * 64 + srow;
-        row = row < a.M ? row : a.M - 1;
+        row = row < t.mlim ? row : t.mlim - 1;
         srcA[h][i] = a.A + (size_t)row * a.lda + schunk * 8 + (NN ? k0 : 0);
         int col;
         if (NN) {  // one pointer: N is a multiple of 256 here, pieces and issues are a fixed step apart
-          if (h == 0 && i == 0) srcB[0][0] = a.B + (size_t)(k0 + wrow) * a.ldb + n0 + (wpc >> 5) * 64 + (wpc & 31);
+          if (h == 0 && i == 0) srcB[0][0] = B + (size_t)(k0 + wrow) * a.ldb + n0 + (wpc >> 5) * 64 + (wpc & 31);
           continue;
         }
         if (EPI == 1) {  // piece h: gate (0) or up (1) rows of the tile's 128 columns, 32 per wave column
@@ -163,7 +191,7 @@ __global__ __launch_bounds__(512) void tgemm_kernel(const TGArgs a) {
           col = n0 + (i * 2 + (wave >> 2)) * 64 + h * 32 + (wave & 3) * 8 + (lane >> 3);
           col = col < a.N ? col : a.N - 1;
         }
-        srcB[h][i] = a.B + (size_t)col * a.ldb + schunk * 8;
+        srcB[h][i] = B + (size_t)col * a.ldb + schunk * 8;
       }
   };
   auto stage = [&](int buf, int piece, int kt) __attribute__((always_inline)) {
@@ -249,8 +277,9 @@ __global__ __launch_bounds__(512) void tgemm_kernel(const TGArgs a) {
     const auto r1 = __builtin_amdgcn_permlane16_swap(pk[0][1], pk[1][1], false, false);
     return u32x4{r0[0], r1[0], r0[1], r1[1]};
   };
+  Tile cur = {};  // the output tile being computed
   auto store8 = [&](auto stream, int m, int n, u32x4 o) __attribute__((always_inline)) {
-    if (m < a.M && n < a.N) {
+    if (m < cur.mlim && n < a.N) {
       bf16_t* p = a.C + (size_t)m * a.ldc + n;
       if (n + 8 <= a.N) {
         if constexpr (decltype(stream)::value)
@@ -263,9 +292,11 @@ __global__ __launch_bounds__(512) void tgemm_kernel(const TGArgs a) {
     }
   };
   // plain form: both column quadrants of a row half, 32 rows of 128 bytes at a time through the wave's 4 KiB
-  auto put = [&](tg_acc& c0, tg_acc& c1, int m0, int n0, float* part, int mh) __attribute__((always_inline)) {
+  auto put = [&](tg_acc& c0, tg_acc& c1, int mh) __attribute__((always_inline)) {
+    const int m0 = cur.m0, n0 = cur.n0;
+    float* part = cur.part;
     char* ob = smem + TG_LDS + wave * 4096;
-    if (NN && part) {  // one part of the reduction, summed by a kernel of its own
+    if (NN && !GRP && part) {  // one part of the reduction, summed by a kernel of its own
       float* op = part + (wr * 128 + mh * 64 + fr) * 256 + wc * 64 + fq * 4;
 #pragma unroll
       for (int mt = 0; mt < 4; ++mt)
@@ -276,7 +307,7 @@ __global__ __launch_bounds__(512) void tgemm_kernel(const TGArgs a) {
         }
       return;
     }
-    if (a.bias) {
+    if (!NN && !GRP && a.bias) {
 #pragma unroll
       for (int nh = 0; nh < 2; ++nh)
 #pragma unroll
@@ -311,7 +342,8 @@ __global__ __launch_bounds__(512) void tgemm_kernel(const TGArgs a) {
   // gated form: `g` and `u` are the two column quadrants of one row half. A wave's 32 result columns are half a line: the four
   // waves of a wave row passing them on together through LDS was slower (1361 against 1321 us at 32768 x 8960 from 1536 deep)
   // than storing from the registers; so was dealing the activation out over the next tile's first phases (1333).
-  auto put_gated = [&](tg_acc& g, tg_acc& u, int m0, int n0, int mh) __attribute__((always_inline)) {
+  auto put_gated = [&](tg_acc& g, tg_acc& u, int mh) __attribute__((always_inline)) {
+    const int m0 = cur.m0, n0 = cur.n0;
 #pragma unroll
     for (int mt = 0; mt < 4; ++mt) {
       f32x4 v[2];
@@ -327,8 +359,6 @@ __global__ __launch_bounds__(512) void tgemm_kernel(const TGArgs a) {
       store8(std::false_type{}, m0 + wr * 128 + mh * 64 + mt * 16 + fr, n0 + wc * 32 + out_ch * 8, pack8(v[0], v[1]));
     }
   };
-  int cm0 = 0, cn0 = 0;  // origin of the output tile being computed
-  float* cpart = nullptr;
 
   // One K tile = four phases. The K tiles of the block's successive output tiles form ONE stream: the pieces staged
   // while the last two K tiles of an output tile are computed are K tiles 0 and 1 of the NEXT output tile, so the
@@ -337,8 +367,7 @@ __global__ __launch_bounds__(512) void tgemm_kernel(const TGArgs a) {
   // "t+2" is K tile 0 of the next output tile, whose source addresses replace the current ones after phase 1).
   // MODE 2: last K tile ("t+1", "t+2" are K tiles 0, 1 of the next output tile). Without a next tile nothing is staged
   // and the loads still in flight are drained.
-  int nm0 = 0, nn0 = 0, nk0 = 0, nkt = 0;
-  float* npart = nullptr;
+  Tile next = {};
   bool has_next = false;
   auto tile = [&](auto buf_c, int t, auto mode_c) __attribute__((always_inline)) {
     constexpr int buf = decltype(buf_c)::value, MODE = decltype(mode_c)::value;
@@ -353,14 +382,14 @@ __global__ __launch_bounds__(512) void tgemm_kernel(const TGArgs a) {
     // from now, when the staggered wave group has only just passed that barrier
     asm volatile("s_waitcnt lgkmcnt(8)" ::: "memory");
     mma(acc00, bf0);
-    if (MODE == 1 && go) set_sources(nm0, nn0, nk0);
+    if (MODE == 1 && go) set_sources(next);
     // phase 2: quadrant (0, 1)
     read_b(buf, 1, bf1);
     if (go) stage(buf, PB0, t2);
     mma(acc01, bf1);
     // last K tile: a row half is final once its phases are over; it leaves while the other wave group computes
-    if (MODE == 2 && EPI == 0) put(acc00, acc01, cm0, cn0, cpart, 0);
-    if (MODE == 2 && EPI == 1) put_gated(acc00, acc01, cm0, cn0, 0);
+    if (MODE == 2 && EPI == 0) put(acc00, acc01, 0);
+    if (MODE == 2 && EPI == 1) put_gated(acc00, acc01, 0);
     // phase 3: quadrant (1, 1)
     read_a(buf, 1);
     if (go) stage(buf, PA0, t2);
@@ -373,8 +402,8 @@ __global__ __launch_bounds__(512) void tgemm_kernel(const TGArgs a) {
       tg_vmcnt<0>();
     }
     mma(acc10, bf0);
-    if (MODE == 2 && EPI == 0) put(acc10, acc11, cm0, cn0, cpart, 1);
-    if (MODE == 2 && EPI == 1) put_gated(acc10, acc11, cm0, cn0, 1);
+    if (MODE == 2 && EPI == 0) put(acc10, acc11, 1);
+    if (MODE == 2 && EPI == 1) put_gated(acc10, acc11, 1);
   };
   using B0 = std::integral_constant<int, 0>;
   using B1 = std::integral_constant<int, 1>;
@@ -383,10 +412,9 @@ __global__ __launch_bounds__(512) void tgemm_kernel(const TGArgs a) {
   using M2 = std::integral_constant<int, 2>;
 
   // ---- prologue: K tile 0 whole, B0 A0 B1 of K tile 1 (its A1 leaves in phase 1 of K tile 0)
-  int id = blockIdx.x, m0, n0, k0, KT;
-  float* part;
-  tile_origin(id, m0, n0, k0, KT, part);
-  set_sources(m0, n0, k0);
+  int id = blockIdx.x;
+  cur = tile_origin(id);
+  set_sources(cur);
   stage(0, PB0, 0);
   stage(0, PA0, 0);
   stage(0, PB1, 0);
@@ -401,10 +429,8 @@ __global__ __launch_bounds__(512) void tgemm_kernel(const TGArgs a) {
   while (true) {
     const int nid = id + gridDim.x;
     has_next = nid < ntiles;
-    if (has_next) tile_origin(nid, nm0, nn0, nk0, nkt, npart);
-    cm0 = m0;
-    cn0 = n0;
-    cpart = part;
+    if (has_next) next = tile_origin(nid);
+    const int KT = cur.kt;
 #pragma unroll
     for (int mt = 0; mt < 4; ++mt)
 #pragma unroll
@@ -424,12 +450,37 @@ __global__ __launch_bounds__(512) void tgemm_kernel(const TGArgs a) {
     tile(B1{}, t + 1, M2{});
     if (!has_next) break;
     id = nid;
-    m0 = nm0;
-    n0 = nn0;
-    KT = nkt;
-    part = npart;
+    cur = next;
   }
   if (wr == 0) tg_barrier();
+}
+
+// Row tiles of 256 of the experts' rows (offsets [E + 1]), in order: table[0].x = their number, then {first row, end of the
+// expert's rows, expert} each. One block.
+__global__ __launch_bounds__(256) void tgemm_table_kernel(const int* __restrict__ offsets, int E, int4* __restrict__ table) {
+  __shared__ int wsum[4];
+  const int t = threadIdx.x, lane = t & 63;
+  int base = 0;
+  for (int e0 = 0; e0 < E; e0 += 256) {
+    const int e = e0 + t;
+    const int lo = e < E ? offsets[e] : 0, hi = e < E ? offsets[e + 1] : 0, n = (hi - lo + 255) / 256;
+    int incl = n;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int y = __shfl_up(incl, o, 64);
+      if (lane >= o) incl += y;
+    }
+    if (lane == 63) wsum[t >> 6] = incl;
+    __syncthreads();
+    int at = base + incl - n;
+    for (int w = 0; w < 4; ++w) {
+      if (w < (t >> 6)) at += wsum[w];
+      base += wsum[w];
+    }
+    __syncthreads();
+    for (int i = 0; i < n; ++i) table[1 + at + i] = make_int4(lo + i * 256, hi, e, 0);
+  }
+  if (t == 0) table[0] = make_int4(base, 0, 0, 0);
 }
 
 // =====================================================================================
@@ -463,6 +514,9 @@ struct TWArgs {
   int whole;          // the first `whole` tiles are reduced by one workgroup each
   int splits, chunk;  // the others: workgroups per tile, pairs per workgroup (the last one of a tile may get fewer)
   float* part;        // [tile - whole][splits][wave][m half][n half][mt][nt][lane][4]
+  // grouped (GRP): rows offsets[e] .. offsets[e + 1] belong to expert e, whose gradient lies `stride` elements from the last
+  const int* offsets;
+  long stride;
 };
 
 typedef f32x4 __attribute__((aligned(4))) f32x4u;
@@ -476,6 +530,7 @@ DEVINL void tg_wgrad_origin(const TWArgs& a, int wg, int& n0, int& k0) {
   k0 = (in_band / rows) * 256;
 }
 
+template <bool GRP>
 __global__ __launch_bounds__(512) void tgemm_wgrad_kernel(const TWArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int lane = threadIdx.x & 63;
@@ -486,13 +541,22 @@ __global__ __launch_bounds__(512) void tgemm_wgrad_kernel(const TWArgs a) {
   // the 8 XCDs: the workgroups of one XCD take neighbouring tiles, which share dY / X panels in its L2.
   // (whole tiles and split tiles are renumbered separately: the hardware starts workgroups in id order, and the long
   // whole-tile workgroups have to start first; `whole` is 0, a multiple of 256, or the whole grid)
-  const bool in_whole = (int)blockIdx.x < a.whole;
+  const bool in_whole = GRP || (int)blockIdx.x < a.whole;
   const int base = in_whole ? 0 : a.whole, nb = in_whole ? a.whole : (int)gridDim.x - a.whole;
   const int id = blockIdx.x - base;
   const int xq = nb >> 3, xr = nb & 7, xx = id & 7;
   const int b = base + (xx < xr ? xx * (xq + 1) : xr * (xq + 1) + (xx - xr) * xq) + (id >> 3);
-  int b_tile = b, b_split = 0, b_chunk = a.pairs;
-  if (b >= a.whole) {
+  int b_tile = b, b_split = 0, b_chunk = a.pairs, row_lo = 0, row_hi = a.M;
+  float* dW = a.dW;
+  if (GRP) {
+    const int per = a.tiles_n * a.tiles_k, e = b / per;
+    b_tile = b - e * per;
+    row_lo = a.offsets[e];
+    row_hi = a.offsets[e + 1];
+    if (row_hi <= row_lo) return;  // an expert without rows adds nothing
+    dW += e * a.stride;
+    b_chunk = (row_hi - row_lo + 127) / 128;
+  } else if (b >= a.whole) {
     b_tile = a.whole + (b - a.whole) / a.splits;
     b_split = (b - a.whole) - (b_tile - a.whole) * a.splits;
     b_chunk = a.chunk;
@@ -595,10 +659,10 @@ __global__ __launch_bounds__(512) void tgemm_wgrad_kernel(const TWArgs a) {
 
   // ---- one segment: pairs [p0, p1) of one output tile
   int n0, k0;
-  const int p0 = b_split * b_chunk, p1 = min(a.pairs, p0 + b_chunk);
+  const int p0 = b_split * b_chunk, p1 = GRP ? b_chunk : min(a.pairs, p0 + b_chunk);
   tg_wgrad_origin(a, b_tile, n0, k0);
-  const int tok0 = p0 * 128, KT = (p1 - p0) * 2;
-  tokens = a.M - tok0;
+  const int tok0 = row_lo + p0 * 128, KT = (p1 - p0) * 2;
+  tokens = row_hi - tok0;
   // N may end half way through the last tile row (N % 256 == 128): the second wave row then re-reads the first
   // one's columns and does not write
   const bool half_n = n0 + 128 >= a.N;
@@ -636,7 +700,7 @@ __global__ __launch_bounds__(512) void tgemm_wgrad_kernel(const TWArgs a) {
 
   // ---- lane (row fr, fq) of tile (mt, nt) holds 4 consecutive k columns
   if (half_n && wr == 1) return;
-  if (b >= a.whole) {
+  if (!GRP && b >= a.whole) {
     f32x4* pp = reinterpret_cast<f32x4*>(a.part + ((size_t)(b - a.whole) << 16)) + wave * 2048 + lane;
     auto put = [&](tg_acc& acc, int q) __attribute__((always_inline)) {
 #pragma unroll
@@ -653,7 +717,7 @@ __global__ __launch_bounds__(512) void tgemm_wgrad_kernel(const TWArgs a) {
   // a row half (64 x 64 fp32) passes through the wave's LDS: an instruction then moves 256 bytes of four rows
   char* ob = smem + wave * 16384;
   auto flush = [&](tg_acc& c0, tg_acc& c1, int mh) __attribute__((always_inline)) {
-    float* op = a.dW + (size_t)(n0 + wr * 128 + mh * 64) * a.ldw + k0 + wc * 64;
+    float* op = dW + (size_t)(n0 + wr * 128 + mh * 64) * a.ldw + k0 + wc * 64;
 #pragma unroll
     for (int mt = 0; mt < 4; ++mt)
 #pragma unroll
@@ -743,11 +807,11 @@ static int tgemm_tn_launch(const void* A, long lda, const void* B, long ldb, voi
   if (((uintptr_t)A | (uintptr_t)B) % 16 != 0 || (uintptr_t)C % 8 != 0 || (bias && (uintptr_t)bias % 8 != 0)) return -1;
   if (gated && bias) return -1;
   TGArgs a{(const bf16_t*)A, lda, (const bf16_t*)B, ldb, (bf16_t*)C, ldc, (const bf16_t*)bias, M, N, K,
-           (M + 255) / 256, gated ? (N + 127) / 128 : (N + 255) / 256, nullptr, 0, 1, 0};
+           (M + 255) / 256, gated ? (N + 127) / 128 : (N + 255) / 256, nullptr, 0, 1, 0, nullptr, 0};
   static bool attr_set = false;  // 128 KiB of dynamic LDS: above the default limit
   if (!attr_set) {
-    HIP_RET(hipFuncSetAttribute((const void*)tgemm_kernel<0, false>, hipFuncAttributeMaxDynamicSharedMemorySize, TG_LDS + TG_OUT));
-    HIP_RET(hipFuncSetAttribute((const void*)tgemm_kernel<1, false>, hipFuncAttributeMaxDynamicSharedMemorySize, TG_LDS));
+    HIP_RET(hipFuncSetAttribute((const void*)tgemm_kernel<0, false, false>, hipFuncAttributeMaxDynamicSharedMemorySize, TG_LDS + TG_OUT));
+    HIP_RET(hipFuncSetAttribute((const void*)tgemm_kernel<1, false, false>, hipFuncAttributeMaxDynamicSharedMemorySize, TG_LDS));
     attr_set = true;
   }
   // max_blocks workgroups (a multiple of 8: block id mod 8 is the XCD for every tile of a block's sequence) walk the
@@ -756,9 +820,9 @@ static int tgemm_tn_launch(const void* A, long lda, const void* B, long ldb, voi
   if (max_blocks > 0 && max_blocks % 8 != 0) return -1;
   const dim3 grid(max_blocks > 0 ? std::min(ntiles, max_blocks) : ntiles), block(512);
   if (gated)
-    hipLaunchKernelGGL((tgemm_kernel<1, false>), grid, block, TG_LDS, st, a);
+    hipLaunchKernelGGL((tgemm_kernel<1, false, false>), grid, block, TG_LDS, st, a);
   else
-    hipLaunchKernelGGL((tgemm_kernel<0, false>), grid, block, TG_LDS + TG_OUT, st, a);
+    hipLaunchKernelGGL((tgemm_kernel<0, false, false>), grid, block, TG_LDS + TG_OUT, st, a);
   return (int)hipGetLastError();
 }
 
@@ -796,13 +860,13 @@ extern "C" int areal_tgemm_wgrad(const void* dY, long ldy, const void* X, long l
   if ((pairs + chunk - 1) / chunk != splits) return -1;
   const long nblocks = whole + (tiles - whole) * splits;
   if (nblocks > 0x7fffffffl || (tiles - whole) > (0x7fffffffl >> 5)) return -1;
-  TWArgs a{(const bf16_t*)dY, ldy, (const bf16_t*)X, ldx, dW, ldw, M, N, K, (N + 255) / 256, K / 256, pairs, whole, splits, chunk, part};
+  TWArgs a{(const bf16_t*)dY, ldy, (const bf16_t*)X, ldx, dW, ldw, M, N, K, (N + 255) / 256, K / 256, pairs, whole, splits, chunk, part, nullptr, 0};
   static bool attr_set = false;
   if (!attr_set) {
-    HIP_RET(hipFuncSetAttribute((const void*)tgemm_wgrad_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, TG_LDS));
+    HIP_RET(hipFuncSetAttribute((const void*)tgemm_wgrad_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize, TG_LDS));
     attr_set = true;
   }
-  hipLaunchKernelGGL(tgemm_wgrad_kernel, dim3((unsigned)nblocks), dim3(512), TG_LDS, st, a);
+  hipLaunchKernelGGL(tgemm_wgrad_kernel<false>, dim3((unsigned)nblocks), dim3(512), TG_LDS, st, a);
   if (splits > 1) hipLaunchKernelGGL(tgemm_wgrad_sum_kernel, dim3((unsigned)(tiles - whole) * 32), dim3(256), 0, st, a);
   return (int)hipGetLastError();
 }
@@ -826,14 +890,61 @@ extern "C" int areal_tgemm_nn(const void* dY, long ldy, const void* W, long ldw,
   const long items = whole + (tiles - whole) * splits;
   if (items > 0x7fffffffl - 256) return -1;
   TGArgs a{(const bf16_t*)dY, ldy, (const bf16_t*)W, ldw, (bf16_t*)dX, ldx, nullptr, M, C, R, tiles_m, C / 256,
-           part, whole, splits, chunk};
+           part, whole, splits, chunk, nullptr, 0};
   static bool attr_set = false;
   if (!attr_set) {
-    HIP_RET(hipFuncSetAttribute((const void*)tgemm_kernel<0, true>, hipFuncAttributeMaxDynamicSharedMemorySize, TG_LDS + TG_OUT));
+    HIP_RET(hipFuncSetAttribute((const void*)tgemm_kernel<0, true, false>, hipFuncAttributeMaxDynamicSharedMemorySize, TG_LDS + TG_OUT));
     attr_set = true;
   }
-  hipLaunchKernelGGL((tgemm_kernel<0, true>), dim3((unsigned)std::min(items, 256l)), dim3(512), TG_LDS + TG_OUT, st, a);
+  hipLaunchKernelGGL((tgemm_kernel<0, true, false>), dim3((unsigned)std::min(items, 256l)), dim3(512), TG_LDS + TG_OUT, st, a);
   if (splits > 1)
     hipLaunchKernelGGL(tgemm_nn_sum_kernel, dim3((unsigned)(tiles - whole) * 32), dim3(256), 0, st, a);
+  return (int)hipGetLastError();
+}
+
+// ---- routed experts: rows sorted by expert, offsets [E + 1] on the device. table: 4 (T / 256 + E + 1) ints of scratch.
+// nn = 0: C[t, N] = A[t, K] . B[e, N, K]^T, K a multiple of 128, N of 8; nn = 1: C[t, N] = A[t, K] . B[e, K, N], N of 256.
+extern "C" int areal_tgemm_grouped(const void* A, const void* B, void* C, const int* offsets, int* table, int T, int E, int N,
+                                   int K, long stride, int nn, hipStream_t st) {
+  if (T <= 0 || E <= 0) return 0;
+  if (K % 128 != 0 || N <= 0 || N % (nn ? 256 : 8) != 0 || stride % 8 != 0) return -1;
+  if (((uintptr_t)A | (uintptr_t)B | (uintptr_t)C | (uintptr_t)table) % 16 != 0) return -1;
+  const int tiles_n = (N + 255) / 256;
+  const long most = ((long)T / 256 + E) * tiles_n;  // (an expert's last tile may be partly empty)
+  if (most > 0x7fffffffl - 256) return -1;
+  hipLaunchKernelGGL(tgemm_table_kernel, dim3(1), dim3(256), 0, st, offsets, E, (int4*)table);
+  TGArgs a{(const bf16_t*)A, K, (const bf16_t*)B, nn ? N : K, (bf16_t*)C, N, nullptr, T, N, K, 0, tiles_n,
+           nullptr, 0, 1, 0, (const int4*)table, stride};
+  static bool attr_set = false;
+  if (!attr_set) {
+    HIP_RET(hipFuncSetAttribute((const void*)tgemm_kernel<0, false, true>, hipFuncAttributeMaxDynamicSharedMemorySize, TG_LDS + TG_OUT));
+    HIP_RET(hipFuncSetAttribute((const void*)tgemm_kernel<0, true, true>, hipFuncAttributeMaxDynamicSharedMemorySize, TG_LDS + TG_OUT));
+    attr_set = true;
+  }
+  const dim3 grid((unsigned)std::min(most, 256l)), block(512);
+  if (nn)
+    hipLaunchKernelGGL((tgemm_kernel<0, true, true>), grid, block, TG_LDS + TG_OUT, st, a);
+  else
+    hipLaunchKernelGGL((tgemm_kernel<0, false, true>), grid, block, TG_LDS + TG_OUT, st, a);
+  return (int)hipGetLastError();
+}
+
+// dW[e, N, K] (fp32, experts `stride` elements apart) += dY[t, N]^T . X[t, K] over each expert's rows; N a multiple of 128, K
+// of 256.
+extern "C" int areal_tgemm_grouped_wgrad(const void* dY, const void* X, float* dW, const int* offsets, int E, int N, int K,
+                                         long stride, hipStream_t st) {
+  if (E <= 0) return 0;
+  if (N <= 0 || K <= 0 || N % 128 != 0 || K % 256 != 0 || N > (1 << 24) || K > (1 << 24)) return -1;
+  if (((uintptr_t)dY | (uintptr_t)X) % 16 != 0 || (uintptr_t)dW % 4 != 0) return -1;
+  const int tiles_n = (N + 255) / 256, tiles_k = K / 256;
+  const long blocks = (long)tiles_n * tiles_k * E;
+  if (blocks > 0x7fffffffl) return -1;
+  TWArgs a{(const bf16_t*)dY, N, (const bf16_t*)X, K, dW, K, 0, N, K, tiles_n, tiles_k, 0, (int)blocks, 1, 0, nullptr, offsets, stride};
+  static bool attr_set = false;
+  if (!attr_set) {
+    HIP_RET(hipFuncSetAttribute((const void*)tgemm_wgrad_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, TG_LDS));
+    attr_set = true;
+  }
+  hipLaunchKernelGGL(tgemm_wgrad_kernel<true>, dim3((unsigned)blocks), dim3(512), TG_LDS, st, a);
   return (int)hipGetLastError();
 }
