@@ -774,7 +774,7 @@ class ModelRunner:
                 logits = self._lm_head(self._decode_layers_fused(st, h, rope_pos))
             else:
                 logits = self._decode_step_logits(st, h, rope_pos)
-            if self.keep_logits:
+            if self.keep_logits and s == self.decode_steps - 1:
                 st["logits"].copy_(logits)
             ops.sample(logits, st["temperature"], st["top_k"] if filtered else None, st["top_p"] if filtered else None,
                        self.seed, self.step_counter, bump_step=True, out_tokens=st["out_tokens"][s],

@@ -15,6 +15,9 @@ from . import _lib as L
 # unfiltered batches (no top-k / top-p) split every row over several workgroups; 0 keeps the one-workgroup-per-row
 # kernel for A/B timing
 SPLIT_UNFILTERED = os.environ.get("AREAL_SAMPLE_SPLIT", "1") != "0"
+# rows up to which the rows of a filtered batch are split over several workgroups (16 to 2 each, 512 in all)
+SPLIT_FILTERED_MAX_ROWS = 384
+SLICE_WORDS = 516  # of workspace for a row's slice (csrc/hip/sampling.hip)
 
 
 class TokenCounts:
@@ -117,14 +120,19 @@ def sample(logits: torch.Tensor, temperature: Optional[torch.Tensor], top_k: Opt
             "sample_unfiltered",
         )
         return out_tokens, out_logprobs
+    lib = L.lib()
+    ws, S = None, 0
+    if 0 < B <= SPLIT_FILTERED_MAX_ROWS:
+        S = min(16, -(-512 // B))
+        ws = torch.empty(B * S * SLICE_WORDS + 2, dtype=torch.float32, device=logits.device)
     L.check(
-        L.lib().areal_sample(L.ptr(logits), L.c_int(L.dtype_flag(logits)), L.c_int(B), L.c_int(V),
+        lib.areal_sample(L.ptr(logits), L.c_int(L.dtype_flag(logits)), L.c_int(B), L.c_int(V),
                              L.c_int64(logits.stride(0)), L.ptr(temperature), L.ptr(top_k), L.ptr(top_p),
                              L.c_uint64(int(seed) & 0xFFFFFFFFFFFFFFFF), L.ptr(step), L.c_int(int(bump_step)),
                              L.ptr(out_tokens), L.ptr(out_logprobs), L.ptr(active),
                              L.ptr(counts.table if counts is not None else None),
                              L.c_int64(counts.ld if counts is not None else 0), L.ptr(count_slot), L.ptr(freq_pen),
-                             L.ptr(pres_pen), L.stream_ptr()),
+                             L.ptr(pres_pen), L.ptr(ws), L.c_int(S), L.stream_ptr()),
         "sample",
     )
     return out_tokens, out_logprobs

@@ -205,11 +205,10 @@ DEVINL void select_bin(Select& S, E each, float lo, float hi, float scale, float
   __syncthreads();
 }
 
-// floor: entries below it do not count (the top-k threshold, or -inf); mn, mx: smallest and largest finite entry.
-// Returns floor where even all entries fall short of the target.
-template <bool MASS, typename T>
-DEVINL float select_threshold(Select& S, const Row<T>& R, int V, int V8, float floor, float mn, float mx, float target_f,
-                              float* red) {
+// row(f): f(z) for every entry, over the whole block. floor: entries below it do not count (the top-k threshold, or -inf);
+// mn, mx: smallest and largest finite entry. Returns floor where even all entries fall short of the target.
+template <bool MASS, typename E>
+DEVINL float select_threshold(Select& S, E row, float floor, float mn, float mx, float target_f, float* red) {
   if (!(mx < INFINITY) || !(mx > -INFINITY) || target_f != target_f) return floor;
   const int tid = threadIdx.x;
   const float bottom = fmaxf(floor, mn);
@@ -217,7 +216,6 @@ DEVINL float select_threshold(Select& S, const Row<T>& R, int V, int V8, float f
   const unsigned long long target = tf < 1. ? 1ull : (unsigned long long)tf;
   unsigned long long above = 0ull;
   float lo = fmaxf(bottom, mx - SEL_RANGE), hi = mx, scale = 0.f;
-  auto row = [&](auto f) __attribute__((always_inline)) { for_each_z(R, V, V8, [&](int, float z) { f(z); }); };
   int n = 0;
   for (int round = 0;; ++round) {
     if (round == 8) return lo;
@@ -311,19 +309,227 @@ DEVINL float select_threshold(Select& S, const Row<T>& R, int V, int V8, float f
   return t > -INFINITY ? t : lo;
 }
 
+// ---------------------------------------------------------------------------------------------
+// Filtered rows, first part: S workgroups a row, each with a slice of it: the slice's maximum, minimum and sum of exponentials.
+// With a small top-k what the workgroup that owns the row then still needs of its 152k entries are those that can be among the
+// k largest, so every slice also hands on a superset of its own k largest entries (the bins of its histogram from the k-th
+// largest's on): seven passes of one workgroup over the row become two of S workgroups over a slice and work on a few
+// hundred entries. us of one part and of two, 151936 bf16 entries: top-k 50 with top-p 0.95, one dominant token, 1 / 24 / 64 /
+// 320 rows 96 / 97 / 98 / 215 and 39 / 42 / 41 / 104; top-p 0.95 alone, which only gains the first pass, 49 / 50 / 50 / 110 and
+// 43 / 45 / 49 / 112.
+// ws: [B][S][SLICE_WORDS] words: {max, sum of exp(z - max), number of entries (-1: none or too many, the row's own passes find
+// the set), min}, entries, their places; behind them the step (the second part's first workgroup counts it on, so the others
+// read it here).
+constexpr int TOPK_MAX = 128, TOPK_CAP = 256, SLICE_WORDS = 4 + 2 * TOPK_CAP, SLICES = SEL_CAP / TOPK_CAP, SLICE_THREADS = 512;
+
+template <typename T>
+__global__ __launch_bounds__(SLICE_THREADS) void sample_slice_kernel(
+    const T* __restrict__ logits, int64_t ld, int V, const float* __restrict__ temperature, const int* __restrict__ top_k,
+    const float* __restrict__ top_p, const int64_t* __restrict__ step_ptr, const int* __restrict__ active,
+    const int16_t* __restrict__ counts, int64_t count_ld, const int* __restrict__ count_slot,
+    const float* __restrict__ freq_pen, const float* __restrict__ pres_pen, float* __restrict__ ws, int S) {
+  constexpr int NT = SLICE_THREADS, BINS = 1024, PER = BINS / NT;
+  __shared__ float red[16];
+  __shared__ unsigned hist[BINS], part[NT / 64];
+  __shared__ int s_bin, s_above, s_n, s_pos;
+  const int row = blockIdx.y, s = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  if (row == 0 && s == 0 && tid == 0 && step_ptr)
+    *reinterpret_cast<int64_t*>(ws + (size_t)gridDim.y * S * SLICE_WORDS) = step_ptr[0];
+  if (active && !active[row]) return;
+  const float temp = temperature ? temperature[row] : 1.f;
+  const int k = top_k ? top_k[row] : V;
+  const bool limited = k >= 1 && k < V;
+  if (temp <= 0.f || !(limited || (top_p && top_p[row] < 1.f))) return;
+  const T* p = logits + (size_t)row * ld;
+  const int V8 = (reinterpret_cast<uintptr_t>(p) & 15) == 0 ? (V & ~7) : 0;
+  const int slot = (counts && count_slot) ? count_slot[row] : -1;
+  Row<T> R;
+  R.p = p;
+  R.cnt = slot >= 0 ? counts + (size_t)slot * count_ld : nullptr;
+  R.freq = R.cnt && freq_pen ? freq_pen[row] : 0.f;
+  R.pres = R.cnt && pres_pen ? pres_pen[row] : 0.f;
+  R.inv_t = 1.f / temp;
+  const int chunks = V8 >> 3, per = (chunks + S - 1) / S;
+  const int first = min(chunks, s * per) * 8, end = min(chunks, (s + 1) * per) * 8;
+  // f8(i, z) over groups of 8 entries of the slice, f1(i, z_i) over those behind the last whole group (or over the whole row
+  // when it is not 16-byte aligned)
+  auto walk = [&](auto f8, auto f1) __attribute__((always_inline)) {
+    constexpr int PF = 4;
+    for (int base = first + tid * 8; base < end; base += NT * 8 * PF) {
+      float zz[PF][8];
+#pragma unroll
+      for (int u = 0; u < PF; ++u)
+        if (base + u * NT * 8 < end) R.z8(base + u * NT * 8, zz[u]);
+#pragma unroll
+      for (int u = 0; u < PF; ++u) {
+        const int i8 = base + u * NT * 8;
+        if (i8 >= end) break;
+        f8(i8, zz[u]);
+      }
+    }
+    if (s == S - 1)
+      for (int i = V8 + tid; i < V; i += NT) f1(i, R.z1(i));
+  };
+  auto each = [&](auto f) __attribute__((always_inline)) {
+    walk([&](int i8, const float* z) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) f(i8 + j, z[j]);
+    }, f);
+  };
+  float mx = -INFINITY, mn = INFINITY, se = 0.f;
+  auto raise = [&](float m) {
+    if (m > mx) {
+      se *= __expf(mx - m);
+      mx = m;
+    }
+  };
+  walk([&](int, const float* z) {
+    float m8 = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      m8 = fmaxf(m8, z[j]);
+      mn = fminf(mn, z[j] > -INFINITY ? z[j] : INFINITY);
+    }
+    raise(m8);
+    if (mx > -INFINITY)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) se += __expf(z[j] - mx);
+  }, [&](int, float z) {
+    mn = fminf(mn, z > -INFINITY ? z : INFINITY);
+    raise(z);
+    if (mx > -INFINITY) se += __expf(z - mx);
+  });
+  const float own = mx;  // this thread's largest entry
+  const float mx_all = block_max(mx, red);
+  mn = -block_max(-mn, red);
+  se = block_sum(mx > -INFINITY ? se * __expf(mx - mx_all) : 0.f, red);
+  mx = mx_all;
+  float* o = ws + ((size_t)row * S + s) * SLICE_WORDS;
+  // The bin of [lo, hi] from which on there are k entries, from the top down (s_bin, -1: fewer in all), their number in the bin
+  // and above it; `above` entries lie above hi. fill(f): f(z) for every entry that counts
+  float lo = mn, hi = mx, scale = 0.f;
+  int bin = 0, above = 0;
+  auto find = [&](auto fill) __attribute__((always_inline)) {
+    scale = hi > lo ? (float)BINS / (hi - lo) : 0.f;
+    if (!(scale < INFINITY)) scale = 0.f;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < PER; ++i) hist[i * NT + tid] = 0u;
+    if (tid == 0) s_bin = -1;
+    __syncthreads();
+    fill([&](float z) {
+      if (z >= lo && z <= hi) atomicAdd(&hist[sel_bin(z, lo, scale)], 1u);
+    });
+    __syncthreads();
+    unsigned c[PER], sum = 0;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) sum += c[i] = hist[BINS - 1 - (tid * PER + i)];
+    unsigned run = sum;
+#pragma unroll
+    for (int of = 1; of < 64; of <<= 1) {
+      const unsigned y = __shfl_up(run, of, 64);
+      if (lane >= of) run += y;
+    }
+    if (lane == 63) part[wid] = run;
+    __syncthreads();
+    run += above - sum;
+    for (int i = 0; i < wid; ++i) run += part[i];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      if ((int)run < k && (int)(run + c[i]) >= k) {
+        s_bin = BINS - 1 - (tid * PER + i);
+        s_above = (int)run;
+        s_n = (int)c[i];
+      }
+      run += c[i];
+    }
+    __syncthreads();
+    bin = s_bin;
+  };
+  // Hands on the entries from the bin on (of a bracket that ends at the largest entry, or one that lies in such a bin); their number
+  auto hand_on = [&]() __attribute__((always_inline)) {
+    __syncthreads();
+    if (tid == 0) s_pos = 0;
+    __syncthreads();
+    each([&](int i, float z) {
+      if (z > hi || (z >= lo && sel_bin(z, lo, scale) >= bin)) {
+        const int at = atomicAdd(&s_pos, 1);
+        if (at < TOPK_CAP) {
+          o[4 + at] = z;
+          o[4 + TOPK_CAP + at] = __int_as_float(i);
+        }
+      }
+    });
+    __syncthreads();
+    return s_pos;
+  };
+  int n = -1;  // entries handed on
+  if (limited && k <= TOPK_MAX && mx < INFINITY) {
+    if (!(mx > -INFINITY)) {
+      n = 0;
+    } else {
+      // the k-th largest of the threads' largest entries is no larger than the k-th largest entry, and for entries in no
+      // particular order not much smaller: a little over k of them reach it
+      const float low = -block_max(own > -INFINITY ? -own : -INFINITY, red);
+      lo = low;
+      find([&](auto f) { if (own > -INFINITY) f(own); });
+      if (bin < 0) {  // fewer threads than k have entries: all of them
+        lo = mn;
+        scale = 0.f;
+        bin = 0;
+      }
+      n = hand_on();
+      lo = mn;
+      hi = mx;
+      for (int round = 0; n > TOPK_CAP; ++round) {  // too many: the bin of the k-th largest entry itself
+        find([&](auto f) { each([&](int, float z) { f(z); }); });
+        if (bin < 0 || s_above + s_n <= TOPK_CAP) {
+          bin = max(bin, 0);
+          n = hand_on();
+          break;
+        }
+        if (scale == 0.f || round == 6) break;
+        above = s_above;
+        float l = INFINITY, h = -INFINITY;
+        each([&](int, float z) {
+          if (z >= lo && z <= hi && sel_bin(z, lo, scale) == bin) {
+            l = fminf(l, z);
+            h = fmaxf(h, z);
+          }
+        });
+        lo = -block_max(-l, red);
+        hi = block_max(h, red);
+      }
+    }
+  }
+  if (tid == 0) {
+    o[0] = mx;
+    o[1] = se;
+    o[2] = __int_as_float(n > TOPK_CAP ? -1 : n);
+    o[3] = mn;
+  }
+}
+
+// ws, S: what sample_slice_kernel has left (null: nothing; the rows' statistics are then a pass of this kernel's own, and step_ptr
+// is not counted on)
 template <typename T>
 __global__ __launch_bounds__(1024) void sample_kernel(
     const T* __restrict__ logits, int64_t ld, int V, const float* __restrict__ temperature,
     const int* __restrict__ top_k, const float* __restrict__ top_p, uint64_t seed,
-    const int64_t* __restrict__ step_ptr, int64_t* __restrict__ out_tok,
+    int64_t* step_ptr, int64_t* __restrict__ out_tok,
     float* __restrict__ out_logp, const int* __restrict__ active, int16_t* __restrict__ counts,
     int64_t count_ld, const int* __restrict__ count_slot, const float* __restrict__ freq_pen,
-    const float* __restrict__ pres_pen) {
+    const float* __restrict__ pres_pen, const float* __restrict__ ws, int S, int bump_step) {
   __shared__ float red[16];
   __shared__ float redv[16];
   __shared__ int redi[16];
   __shared__ Select sel;
+  __shared__ float list_z[SEL_CAP];
+  __shared__ int list_i[SEL_CAP];
   const int row = blockIdx.x;
+  const int64_t* step_at = ws ? reinterpret_cast<const int64_t*>(ws + (size_t)gridDim.x * S * SLICE_WORDS) : step_ptr;
+  const uint64_t step = step_ptr ? (uint64_t)step_at[0] : 0;
+  if (ws && step_ptr && bump_step && row == 0 && threadIdx.x == 0) step_ptr[0] = (int64_t)step + 1;
   if (active && !active[row]) {  // uniform over the block
     if (threadIdx.x == 0) {
       out_tok[row] = 0;
@@ -337,7 +543,6 @@ __global__ __launch_bounds__(1024) void sample_kernel(
   const float inv_t = greedy ? 1.f : 1.f / temp;
   const int k = top_k ? top_k[row] : V;
   const float tp = top_p ? top_p[row] : 1.f;
-  const uint64_t step = step_ptr ? (uint64_t)step_ptr[0] : 0;
   const bool filtered = !greedy && ((k < V && k >= 1) || tp < 1.f);
   // noise word of entry i: word i & 3 of the Philox block with counter ctr0 + i / 4
   const uint64_t ctr0 = step * (uint64_t)((V + 3) / 4);
@@ -351,11 +556,76 @@ __global__ __launch_bounds__(1024) void sample_kernel(
   R.pres = cnt && pres_pen ? pres_pen[row] : 0.f;
   R.inv_t = inv_t;
 
+  float mx = -INFINITY, mn = INFINITY, se = 0.f;
+  const bool sliced = ws && filtered;
+  bool listed = sliced;  // the slices have handed on all that can be drawn
+  if (sliced) {
+    const float* o = ws + (size_t)row * S * SLICE_WORDS;
+    for (int s = 0; s < S; ++s) {
+      mx = fmaxf(mx, o[(size_t)s * SLICE_WORDS]);
+      mn = fminf(mn, o[(size_t)s * SLICE_WORDS + 3]);
+      listed = listed && __float_as_int(o[(size_t)s * SLICE_WORDS + 2]) >= 0;
+    }
+    for (int s = 0; s < S; ++s) {
+      const float m = o[(size_t)s * SLICE_WORDS];
+      if (m > -INFINITY) se += o[(size_t)s * SLICE_WORDS + 1] * __expf(m - mx);
+    }
+  }
+  if (listed) {
+    const float* o = ws + (size_t)row * S * SLICE_WORDS;
+    int n = 0;
+    for (int s = 0; s < S; ++s, o += SLICE_WORDS) {
+      const int c = __float_as_int(o[2]);
+      for (int i = threadIdx.x; i < c; i += blockDim.x) {
+        list_z[n + i] = o[4 + i];
+        list_i[n + i] = __float_as_int(o[4 + TOPK_CAP + i]);
+      }
+      n += c;
+    }
+    __syncthreads();
+    auto list = [&](auto f) __attribute__((always_inline)) { for (int i = threadIdx.x; i < n; i += blockDim.x) f(list_z[i]); };
+    mn = INFINITY;
+    list([&](float z) { mn = fminf(mn, z); });
+    mn = -block_max(-mn, red);
+    float thr = select_threshold<false>(sel, list, -INFINITY, mn, mx, (float)k, red);
+    if (tp < 1.f) {  // mass of the top-k set, the nucleus's reference: an integer, for the entries come in any order
+      unsigned long long m = 0ull;
+      list([&](float z) { m += z >= thr ? sel_mass(z, mx) : 0ull; });
+#pragma unroll
+      for (int of = 32; of > 0; of >>= 1) m += __shfl_xor(m, of, 64);
+      __syncthreads();
+      if ((threadIdx.x & 63) == 0) sel.part[threadIdx.x >> 6] = m;
+      __syncthreads();
+      m = 0ull;
+      for (int w = 0; w < 16; ++w) m += sel.part[w];
+      __syncthreads();
+      thr = select_threshold<true>(sel, list, thr, mn, mx, tp * (float)((double)m / (double)SEL_FIX), red);
+    }
+    ArgMax best;
+    best.v = -INFINITY;
+    best.i = 0x7fffffff;
+    for (int i = threadIdx.x; i < n; i += blockDim.x)
+      if (list_z[i] >= thr) {
+        ArgMax c;
+        c.i = list_i[i];
+        c.v = list_z[i] + gumbel(Philox::gen(seed, (uint64_t)row, ctr0 + (uint64_t)(c.i >> 2))[c.i & 3]);
+        best = amax(best, c);
+      }
+    best = block_argmax(best, redv, redi);
+    if (threadIdx.x == 0) {
+      int tok = best.i;
+      if (tok < 0 || tok >= V) tok = 0;
+      out_tok[row] = tok;
+      if (out_logp) out_logp[row] = R.z1(tok) - (mx + __logf(se));
+      if (cnt && cnt[tok] < 32767) cnt[tok] += 1;
+    }
+    return;
+  }
+
   // pass 1: running max / sum-exp (rescaled when the max moves) and min of z. Without filtering the
   // arg-max of z (+ Gumbel noise unless greedy) is taken in the same pass, so the row is read once.
   const bool pick_now = !filtered;
   const bool noise = !greedy;
-  float mx = -INFINITY, mn = INFINITY, se = 0.f;
   ArgMax best;
   best.v = -INFINITY;
   best.i = 0x7fffffff;
@@ -363,75 +633,78 @@ __global__ __launch_bounds__(1024) void sample_kernel(
   // thread sees ~19 chunks of a 152k-entry row, and with one load in flight at a time the pass is a chain of that
   // many memory round trips (the per-entry noise and exponentials are cheap next to them).
   constexpr int PF = 4;
-  for (int base = threadIdx.x * 8; base < V8; base += blockDim.x * 8 * PF) {
-    float zz[PF][8];
+  if (!sliced) {
+    for (int base = threadIdx.x * 8; base < V8; base += blockDim.x * 8 * PF) {
+      float zz[PF][8];
 #pragma unroll
-    for (int u = 0; u < PF; ++u) {
-      const int i8 = base + u * (int)blockDim.x * 8;
-      if (i8 < V8) R.z8(i8, zz[u]);
-    }
-#pragma unroll
-    for (int u = 0; u < PF; ++u) {
-      const int i8 = base + u * (int)blockDim.x * 8;
-      if (i8 >= V8) break;
-      float* z = zz[u];
-      float m8 = -INFINITY;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        m8 = fmaxf(m8, z[j]);
-        mn = fminf(mn, z[j] > -INFINITY ? z[j] : INFINITY);
+      for (int u = 0; u < PF; ++u) {
+        const int i8 = base + u * (int)blockDim.x * 8;
+        if (i8 < V8) R.z8(i8, zz[u]);
       }
-      if (m8 > mx) {
-        se *= __expf(mx - m8);
-        mx = m8;
-      }
-      if (mx > -INFINITY) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) se += __expf(z[j] - mx);
-      }
-      if (pick_now) {
-        u32x4 r0, r1;
-        if (noise) {
-          r0 = Philox::gen(seed, (uint64_t)row, ctr0 + (uint64_t)(i8 >> 2));
-          r1 = Philox::gen(seed, (uint64_t)row, ctr0 + (uint64_t)(i8 >> 2) + 1);
-        }
+      for (int u = 0; u < PF; ++u) {
+        const int i8 = base + u * (int)blockDim.x * 8;
+        if (i8 >= V8) break;
+        float* z = zz[u];
+        float m8 = -INFINITY;
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-          ArgMax c;
-          c.v = noise ? z[j] + gumbel(j < 4 ? r0[j] : r1[j - 4]) : z[j];
-          c.i = i8 + j;
-          best = amax(best, c);
+          m8 = fmaxf(m8, z[j]);
+          mn = fminf(mn, z[j] > -INFINITY ? z[j] : INFINITY);
+        }
+        if (m8 > mx) {
+          se *= __expf(mx - m8);
+          mx = m8;
+        }
+        if (mx > -INFINITY) {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) se += __expf(z[j] - mx);
+        }
+        if (pick_now) {
+          u32x4 r0, r1;
+          if (noise) {
+            r0 = Philox::gen(seed, (uint64_t)row, ctr0 + (uint64_t)(i8 >> 2));
+            r1 = Philox::gen(seed, (uint64_t)row, ctr0 + (uint64_t)(i8 >> 2) + 1);
+          }
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            ArgMax c;
+            c.v = noise ? z[j] + gumbel(j < 4 ? r0[j] : r1[j - 4]) : z[j];
+            c.i = i8 + j;
+            best = amax(best, c);
+          }
         }
       }
     }
-  }
-  for (int i = V8 + threadIdx.x; i < V; i += blockDim.x) {
-    const float z = R.z1(i);
-    mn = fminf(mn, z > -INFINITY ? z : INFINITY);
-    if (z > mx) {
-      se *= __expf(mx - z);
-      mx = z;
+    for (int i = V8 + threadIdx.x; i < V; i += blockDim.x) {
+      const float z = R.z1(i);
+      mn = fminf(mn, z > -INFINITY ? z : INFINITY);
+      if (z > mx) {
+        se *= __expf(mx - z);
+        mx = z;
+      }
+      if (mx > -INFINITY) se += __expf(z - mx);
+      if (pick_now) {
+        ArgMax c;
+        c.v = z;
+        c.i = i;
+        if (noise) c.v += gumbel(Philox::gen(seed, (uint64_t)row, ctr0 + (uint64_t)(i >> 2))[i & 3]);
+        best = amax(best, c);
+      }
     }
-    if (mx > -INFINITY) se += __expf(z - mx);
-    if (pick_now) {
-      ArgMax c;
-      c.v = z;
-      c.i = i;
-      if (noise) c.v += gumbel(Philox::gen(seed, (uint64_t)row, ctr0 + (uint64_t)(i >> 2))[i & 3]);
-      best = amax(best, c);
-    }
+    const float mx_all = block_max(mx, red);
+    mn = -block_max(-mn, red);
+    se = block_sum(mx > -INFINITY ? se * __expf(mx - mx_all) : 0.f, red);
+    mx = mx_all;
   }
-  const float mx_all = block_max(mx, red);
-  mn = -block_max(-mn, red);
-  se = block_sum(mx > -INFINITY ? se * __expf(mx - mx_all) : 0.f, red);
-  mx = mx_all;
   const float lse = mx + __logf(se);
 
   if (filtered) {
     float thr = -INFINITY;
     float mass_k = se;  // mass (relative to exp(-mx)) of the top-k set
+    auto all = [&](auto f) __attribute__((always_inline)) { for_each_z(R, V, V8, [&](int, float z) { f(z); }); };
     if (k < V && k >= 1) {
-      thr = select_threshold<false>(sel, R, V, V8, -INFINITY, mn, mx, (float)k, red);
+      thr = select_threshold<false>(sel, all, -INFINITY, mn, mx, (float)k, red);
       if (tp < 1.f) {  // the nucleus is taken inside the top-k set: its mass is the reference
         float mk = 0.f;
         for_each_z(R, V, V8, [&](int, float z) {
@@ -440,7 +713,7 @@ __global__ __launch_bounds__(1024) void sample_kernel(
         mass_k = block_sum(mk, red);
       }
     }
-    if (tp < 1.f) thr = select_threshold<true>(sel, R, V, V8, thr, mn, mx, tp * mass_k, red);
+    if (tp < 1.f) thr = select_threshold<true>(sel, all, thr, mn, mx, tp * mass_k, red);
     // arg-max of z + Gumbel noise over the entries that survive the threshold. The noise block of four entries is made
     // once, and only where one of them survives: with a block per entry a nucleus of 100k entries took 33 us longer.
     for (int base = threadIdx.x * 8; base < V8; base += blockDim.x * 8 * PF) {
@@ -648,6 +921,8 @@ extern "C" int areal_sample_splits(int B) {
   return s > 16 ? 16 : s;
 }
 
+
+
 extern "C" int areal_sample_unfiltered(const void* logits, int dtype, int B, int V, int64_t ld,
                                        const float* temperature, uint64_t seed, int64_t* step_ptr, int bump_step,
                                        int64_t* out_tok, float* out_logp, const int* active, int16_t* counts,
@@ -683,18 +958,28 @@ extern "C" int areal_sample(const void* logits, int dtype, int B, int V, int64_t
                             uint64_t seed, int64_t* step_ptr, int bump_step, int64_t* out_tok,
                             float* out_logp, const int* active, int16_t* counts, int64_t count_ld,
                             const int* count_slot, const float* freq_pen, const float* pres_pen,
-                            hipStream_t st) {
+                            float* ws, int S, hipStream_t st) {
   if (B == 0) return 0;
   if (counts && (count_ld % 8 != 0 || count_ld < V)) return (int)hipErrorInvalidValue;
+  if (ws && (S < 1 || S > SLICES || (uintptr_t)ws % 8 != 0)) return (int)hipErrorInvalidValue;
+  if (ws) {
+    const dim3 grid(S, B), block(SLICE_THREADS);
+    if (dtype == 0)
+      hipLaunchKernelGGL(sample_slice_kernel<bf16_t>, grid, block, 0, st, (const bf16_t*)logits, ld, V, temperature, top_k, top_p,
+                         step_ptr, active, counts, count_ld, count_slot, freq_pen, pres_pen, ws, S);
+    else
+      hipLaunchKernelGGL(sample_slice_kernel<float>, grid, block, 0, st, (const float*)logits, ld, V, temperature, top_k, top_p,
+                         step_ptr, active, counts, count_ld, count_slot, freq_pen, pres_pen, ws, S);
+  }
   if (dtype == 0)
     hipLaunchKernelGGL(sample_kernel<bf16_t>, dim3(B), dim3(1024), 0, st, (const bf16_t*)logits, ld, V,
                        temperature, top_k, top_p, seed, step_ptr, out_tok, out_logp, active, counts, count_ld,
-                       count_slot, freq_pen, pres_pen);
+                       count_slot, freq_pen, pres_pen, ws, S, bump_step);
   else
     hipLaunchKernelGGL(sample_kernel<float>, dim3(B), dim3(1024), 0, st, (const float*)logits, ld, V,
                        temperature, top_k, top_p, seed, step_ptr, out_tok, out_logp, active, counts, count_ld,
-                       count_slot, freq_pen, pres_pen);
-  if (bump_step && step_ptr)
+                       count_slot, freq_pen, pres_pen, ws, S, bump_step);
+  if (bump_step && step_ptr && !ws)
     hipLaunchKernelGGL(bump_step_kernel, dim3(1), dim3(64), 0, st, step_ptr);
   return (int)hipGetLastError();
 }
