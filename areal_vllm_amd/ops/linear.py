@@ -29,13 +29,20 @@ def _accumulate_wgrad(weight: torch.Tensor, dy2: torch.Tensor, x2: torch.Tensor)
         mg.add_(torch.mm(dy2.t(), x2))
 
 
+def _product(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) -> torch.Tensor:
+    """x @ W^T (+ b) outside autograd."""
+    if bias is None and x.is_cuda and x.dim() == 2:
+        return train_gemm.forward(x, weight)
+    return F.linear(x, weight, bias)
+
+
 class _LinearMainGrad(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, weight, bias, reduce_dx_group):
         ctx.save_for_backward(x, weight)
         ctx.has_bias = bias is not None
         ctx.group = reduce_dx_group
-        return F.linear(x, weight, bias)
+        return _product(x, weight, bias)
 
     @staticmethod
     def backward(ctx, dy):
@@ -76,7 +83,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] =
     if torch.is_grad_enabled() and (reduce_dx_group is not None or (
             weight.requires_grad and getattr(weight, "main_grad", None) is not None)):
         return _LinearMainGrad.apply(x, weight, bias, reduce_dx_group)
-    return F.linear(x, weight, bias)
+    return F.linear(x, weight, bias) if torch.is_grad_enabled() else _product(x, weight, bias)
 
 
 class _EmbeddingMainGrad(torch.autograd.Function):

@@ -183,7 +183,8 @@ def _group_size(group) -> int:
 
 
 def _chunk_logits(hidden: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
-    lg = torch.matmul(hidden, weight.t())
+    own = hidden.is_cuda and not torch.is_grad_enabled()
+    lg = train_gemm.forward(hidden, weight) if own else torch.matmul(hidden, weight.t())
     if lg.is_cuda and not _is_aligned(lg):  # odd vocabulary (shard): rows must start on 16-byte boundaries
         lg = _aligned_copy(lg)
     return lg
@@ -234,7 +235,7 @@ class _LMHeadLogprobFn(torch.autograd.Function):
         for s in range(0, T, chunk):
             e = min(T, s + chunk)
             if whole is not None:
-                lg = torch.mm(hidden[s:e], weight.t(), out=whole[s:e])
+                lg = train_gemm.forward(hidden[s:e], weight, out=whole[s:e])
             else:
                 lg = _chunk_logits(hidden[s:e], weight)
                 if need_grad and keep_logits:

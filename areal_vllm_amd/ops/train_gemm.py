@@ -33,17 +33,22 @@ def supported(a: torch.Tensor, b: torch.Tensor, bias: Optional[torch.Tensor] = N
 
 
 def tgemm_tn(a: torch.Tensor, b: torch.Tensor, bias: Optional[torch.Tensor] = None,
-             out: Optional[torch.Tensor] = None, max_blocks: int = 256) -> torch.Tensor:
-    """out[M, N] = a[M, K] @ b[N, K]^T (+ bias[N]); bf16 in, fp32 accumulation, bf16 out."""
+             out: Optional[torch.Tensor] = None, max_blocks: int = 256, plan: Optional[Tuple[int, int]] = None) -> torch.Tensor:
+    """out[M, N] = a[M, K] @ b[N, K]^T (+ bias[N]); bf16 in, fp32 accumulation, bf16 out. `plan`: (tiles reduced by one
+    workgroup, parts of the others) of ``_tile_plan``, without a bias."""
     M, K = a.shape
     N = b.shape[0]
     if out is None:
         out = torch.empty(M, N, dtype=torch.bfloat16, device=a.device)
     assert supported(a, b, bias) and out.dtype == torch.bfloat16 and out.stride(1) == 1 and out.stride(0) % 4 == 0
-    L.lib()
+    whole, splits = plan or (0, 1)
+    part = None
+    if splits > 1:
+        part = torch.empty(splits * (-(-M // 256) * -(-N // 256) - whole) << 16, dtype=torch.float32, device=a.device)
     L.check(L.lib().areal_tgemm_tn(L.ptr(a), L.c_int64(a.stride(0)), L.ptr(b), L.c_int64(b.stride(0)), L.ptr(out),
                                    L.c_int64(out.stride(0)), L.ptr(bias), L.c_int(M), L.c_int(N), L.c_int(K),
-                                   L.c_int(int(max_blocks)), L.stream_ptr()), "tgemm_tn")
+                                   L.c_int(int(max_blocks)), L.ptr(part), L.c_int(whole), L.c_int(splits), L.stream_ptr()),
+            "tgemm_tn")
     return out
 
 
@@ -173,6 +178,27 @@ def dgrad(dy: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None)
         if _dgrad_own(dy.shape[0], *w.shape):
             return tgemm_nn(dy, w, out=out)
     return torch.mm(dy, w) if out is None else torch.mm(dy, w, out=out)
+
+
+# Where the own kernel is ahead of the library in y = x W^T, own / library us. Deep reductions, whose tiles it splits: 18944 deep
+# to 3584 columns, 300 / 700 / 3000 / 6000 / 12000 / 24576 rows 68 / 98, 92 / 169, 325 / 550, 564 / 1048, 1142 / 1548, 2298 /
+# 2279; 8960 to 1536, 300 / 513 / 700 / 1500 / 3000 / 6000 rows 34 / 31, 39 / 34, 40 / 45, 53 / 61, 82 / 83, 148 / 142. Wide
+# results, which it stores by whole lines: 1536 deep to 151936 columns, 300 / 700 / 1500 / 3000 / 8192 rows 192 / 187, 285 /
+# 354, 578 / 639, 1154 / 1171, 2890 / 2984. Elsewhere the two are level, or the library has the smaller tiles.
+def _forward_own(M: int, K: int, N: int) -> bool:
+    if N >= 65536:
+        return M >= 600
+    return 256 < M <= 12288 if K >= 16384 else K >= 8192 and 600 <= M <= 2048
+
+
+def forward(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """x[M, K] @ w[N, K]^T outside autograd."""
+    if (x.dim() == 2 and w.dim() == 2 and _forward_own(x.shape[0], w.shape[1], w.shape[0]) and supported(x, w)
+            and w.shape[0] % 8 == 0 and (out is None or out.dtype == torch.bfloat16 and out.stride(1) == 1
+                                         and out.stride(0) % 8 == 0 and out.data_ptr() % 16 == 0)):
+        _, whole, splits = _tile_plan(x.shape[1] // 128, -(-x.shape[0] // 256) * -(-w.shape[0] // 256), 0)
+        return tgemm_tn(x, w, out=out, plan=(whole, splits))
+    return torch.mm(x, w.t(), out=out) if out is not None else torch.nn.functional.linear(x, w)
 
 
 # rows from which the fused gate|up + SwiGLU kernel replaces library GEMM + activation kernel in no-grad forwards

@@ -52,7 +52,7 @@ struct TGArgs {
   const bf16_t* bias;
   int M, N, K;
   int tiles_m, tiles_n;
-  // NN: the tiles from `whole` on are reduced in `splits` parts of `chunk` 128-deep pairs each (the last one may get fewer);
+  // plain and NN: the tiles from `whole` on are reduced in `splits` parts of `chunk` 128-deep pairs each (the last one may get fewer);
   // part [splits][tile - whole][256][256] fp32
   float* part;
   int whole, splits, chunk;
@@ -111,6 +111,7 @@ typedef f32x4 tg_acc[4][2];     // [m tile][n tile] of one quadrant
 template <int EPI, bool NN, bool GRP>
 __global__ __launch_bounds__(512) void tgemm_kernel(const TGArgs a) {
   constexpr int TN = EPI == 1 ? 128 : 256;  // output columns per tile
+  constexpr bool PARTS = EPI == 0 && !GRP;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -119,8 +120,8 @@ __global__ __launch_bounds__(512) void tgemm_kernel(const TGArgs a) {
   // ---- tile sequence number -> output tile
   const tg_table_t table = (tg_table_t)a.table;
   const int tiles_m = GRP ? table[0].x : a.tiles_m;
-  const int tiles = tiles_m * a.tiles_n, whole = NN && !GRP ? a.whole : tiles;
-  const int ntiles = NN && !GRP ? whole + (tiles - whole) * a.splits : tiles;  // work items
+  const int tiles = tiles_m * a.tiles_n, whole = PARTS ? a.whole : tiles;
+  const int ntiles = PARTS ? whole + (tiles - whole) * a.splits : tiles;  // work items
   if (GRP && (int)blockIdx.x >= ntiles) return;  // (the grid is an upper bound)
   struct Tile {
     int m0, n0, k0, kt, mlim, e;  // origin; reduction from k0 on, K tiles; end of the rows; expert
@@ -128,7 +129,7 @@ __global__ __launch_bounds__(512) void tgemm_kernel(const TGArgs a) {
   };
   auto tile_origin = [&](int id) __attribute__((always_inline)) {
     Tile t;
-    const bool in_part = NN && !GRP && id >= whole;
+    const bool in_part = PARTS && id >= whole;
     const int base = in_part ? whole : 0, nb = in_part ? ntiles - whole : whole;
     const int q = nb >> 3, r = nb & 7, x = (id - base) & 7;
     int wg = base + (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + ((id - base) >> 3);
@@ -178,7 +179,7 @@ __global__ __launch_bounds__(512) void tgemm_kernel(const TGArgs a) {
       for (int i = 0; i < 2; ++i) {
         int row = m0 + i * 128 + h * 64 + srow;
         row = row < t.mlim ? row : t.mlim - 1;
-        srcA[h][i] = a.A + (size_t)row * a.lda + schunk * 8 + (NN ? k0 : 0);
+        srcA[h][i] = a.A + (size_t)row * a.lda + schunk * 8 + (PARTS ? k0 : 0);
         int col;
         if (NN) {  // one pointer: N is a multiple of 256 here, pieces and issues are a fixed step apart
           if (h == 0 && i == 0) srcB[0][0] = B + (size_t)(k0 + wrow) * a.ldb + n0 + (wpc >> 5) * 64 + (wpc & 31);
@@ -191,7 +192,7 @@ __global__ __launch_bounds__(512) void tgemm_kernel(const TGArgs a) {
           col = n0 + (i * 2 + (wave >> 2)) * 64 + h * 32 + (wave & 3) * 8 + (lane >> 3);
           col = col < a.N ? col : a.N - 1;
         }
-        srcB[h][i] = B + (size_t)col * a.ldb + schunk * 8;
+        srcB[h][i] = B + (size_t)col * a.ldb + schunk * 8 + (PARTS ? k0 : 0);
       }
   };
   auto stage = [&](int buf, int piece, int kt) __attribute__((always_inline)) {
@@ -296,7 +297,7 @@ __global__ __launch_bounds__(512) void tgemm_kernel(const TGArgs a) {
     const int m0 = cur.m0, n0 = cur.n0;
     float* part = cur.part;
     char* ob = smem + TG_LDS + wave * 4096;
-    if (NN && !GRP && part) {  // one part of the reduction, summed by a kernel of its own
+    if (PARTS && part) {  // one part of the reduction, summed by a kernel of its own
       float* op = part + (wr * 128 + mh * 64 + fr) * 256 + wc * 64 + fq * 4;
 #pragma unroll
       for (int mt = 0; mt < 4; ++mt)
@@ -773,14 +774,14 @@ __global__ __launch_bounds__(256) void tgemm_wgrad_sum_kernel(const TWArgs a) {
 // would leave CUs idle in a last round (or all of them, for few rows) are split over the reduction until the chip is full; the
 // parts are written as fp32 and summed here (they stay in the L2 and the memory-side cache).
 // =====================================================================================
-// dX of the tiles from `whole` on = sum of the parts, in order. Block: 8 rows of a tile.
-__global__ __launch_bounds__(256) void tgemm_nn_sum_kernel(const TGArgs a) {
+// C of the tiles from `whole` on = sum of the parts, in order. Block: 8 rows of a tile.
+__global__ __launch_bounds__(256) void tgemm_sum_kernel(const TGArgs a) {
   const int rest = a.tiles_m * a.tiles_n - a.whole, t = blockIdx.x >> 5, wg = a.whole + t;
   const int band = wg / (TG_GROUP_M * a.tiles_n), first = band * TG_GROUP_M, rows = min(a.tiles_m - first, TG_GROUP_M);
   const int in_band = wg - band * TG_GROUP_M * a.tiles_n;
   const int row = (blockIdx.x & 31) * 8 + (threadIdx.x >> 5), col = (threadIdx.x & 31) * 8;
   const int m = (first + in_band % rows) * 256 + row, n = in_band / rows * 256 + col;
-  if (m >= a.M) return;
+  if (m >= a.M || n >= a.N) return;
   const float* p = a.part + ((size_t)t << 16) + row * 256 + col;
   f32x4 v0 = *reinterpret_cast<const f32x4*>(p), v1 = *reinterpret_cast<const f32x4*>(p + 4);
 #pragma unroll 4
@@ -791,23 +792,38 @@ __global__ __launch_bounds__(256) void tgemm_nn_sum_kernel(const TGArgs a) {
   }
   bf16_t* op = a.C + (size_t)m * a.ldc + n;
   *reinterpret_cast<bf16x4*>(op) = bf16x4{f2bf(v0[0]), f2bf(v0[1]), f2bf(v0[2]), f2bf(v0[3])};
-  *reinterpret_cast<bf16x4*>(op + 4) = bf16x4{f2bf(v1[0]), f2bf(v1[1]), f2bf(v1[2]), f2bf(v1[3])};
+  if (n + 8 <= a.N) *reinterpret_cast<bf16x4*>(op + 4) = bf16x4{f2bf(v1[0]), f2bf(v1[1]), f2bf(v1[2]), f2bf(v1[3])};
 }
 
 }  // namespace
 
 // C[M, N] = A[M, K] . B[N, K]^T (+ bias). Leading dimensions in elements (multiples of 8: 16-byte rows), K a multiple
 // of 128, N a multiple of 4. Returns -1 for shapes outside that (the caller keeps its library path).
-// One launch = min(tiles, max_blocks) persistent workgroups (256 = one per CU).
+// One launch = min(tiles, max_blocks) persistent workgroups (256 = one per CU). splits > 1 (no bias): the tiles from `whole` on
+// in parts, as for areal_tgemm_nn.
 // gated = 1: B holds 2 N rows (gate rows, then up rows), C[M, N] = silu(A.gate^T) * (A.up^T), no bias.
 static int tgemm_tn_launch(const void* A, long lda, const void* B, long ldb, void* C, long ldc, const void* bias, int M,
-                           int N, int K, int max_blocks, int gated, hipStream_t st) {
+                           int N, int K, int max_blocks, int gated, float* part, int whole, int splits, hipStream_t st) {
   if (M <= 0 || N <= 0) return 0;
   if (K % 128 != 0 || N % 4 != 0 || lda % 8 != 0 || ldb % 8 != 0 || ldc % 4 != 0) return -1;
   if (((uintptr_t)A | (uintptr_t)B) % 16 != 0 || (uintptr_t)C % 8 != 0 || (bias && (uintptr_t)bias % 8 != 0)) return -1;
   if (gated && bias) return -1;
+  const long tiles = (long)((M + 255) / 256) * (gated ? (N + 127) / 128 : (N + 255) / 256);
+  const int pairs = K / 128;
+  int chunk = pairs;
+  if (splits == 1) {
+    whole = (int)tiles;
+  } else {  // (see areal_tgemm_nn)
+    if (gated || bias || splits < 1 || splits > pairs || whole < 0 || whole >= tiles || whole % 256 != 0 || !part ||
+        (uintptr_t)part % 16 != 0)
+      return -1;
+    chunk = (pairs + splits - 1) / splits;
+    if ((pairs + chunk - 1) / chunk != splits) return -1;
+  }
+  const long items = whole + (tiles - whole) * splits;
+  if (items > 0x7fffffffl - 256) return -1;
   TGArgs a{(const bf16_t*)A, lda, (const bf16_t*)B, ldb, (bf16_t*)C, ldc, (const bf16_t*)bias, M, N, K,
-           (M + 255) / 256, gated ? (N + 127) / 128 : (N + 255) / 256, nullptr, 0, 1, 0, nullptr, 0};
+           (M + 255) / 256, gated ? (N + 127) / 128 : (N + 255) / 256, part, whole, splits, chunk, nullptr, 0};
   static bool attr_set = false;  // 128 KiB of dynamic LDS: above the default limit
   if (!attr_set) {
     HIP_RET(hipFuncSetAttribute((const void*)tgemm_kernel<0, false, false>, hipFuncAttributeMaxDynamicSharedMemorySize, TG_LDS + TG_OUT));
@@ -816,19 +832,19 @@ static int tgemm_tn_launch(const void* A, long lda, const void* B, long ldb, voi
   }
   // max_blocks workgroups (a multiple of 8: block id mod 8 is the XCD for every tile of a block's sequence) walk the
   // tiles; 0 = one workgroup per tile
-  const int ntiles = a.tiles_m * a.tiles_n;
   if (max_blocks > 0 && max_blocks % 8 != 0) return -1;
-  const dim3 grid(max_blocks > 0 ? std::min(ntiles, max_blocks) : ntiles), block(512);
+  const dim3 grid((unsigned)(max_blocks > 0 ? std::min(items, (long)max_blocks) : items)), block(512);
   if (gated)
     hipLaunchKernelGGL((tgemm_kernel<1, false, false>), grid, block, TG_LDS, st, a);
   else
     hipLaunchKernelGGL((tgemm_kernel<0, false, false>), grid, block, TG_LDS + TG_OUT, st, a);
+  if (splits > 1) hipLaunchKernelGGL(tgemm_sum_kernel, dim3((unsigned)(tiles - whole) * 32), dim3(256), 0, st, a);
   return (int)hipGetLastError();
 }
 
 extern "C" int areal_tgemm_tn(const void* A, long lda, const void* B, long ldb, void* C, long ldc, const void* bias,
-                              int M, int N, int K, int max_blocks, hipStream_t st) {
-  return tgemm_tn_launch(A, lda, B, ldb, C, ldc, bias, M, N, K, max_blocks, 0, st);
+                              int M, int N, int K, int max_blocks, float* part, int whole, int splits, hipStream_t st) {
+  return tgemm_tn_launch(A, lda, B, ldb, C, ldc, bias, M, N, K, max_blocks, 0, part, whole, splits, st);
 }
 
 // C[M, F] = silu(A . Wg^T) * (A . Wu^T) with W = [Wg; Wu] of shape [2 F, K] (the gate|up projection of a gated MLP and
@@ -836,7 +852,7 @@ extern "C" int areal_tgemm_tn(const void* A, long lda, const void* B, long ldb, 
 // activations (scoring, prefill).
 extern "C" int areal_tgemm_swiglu(const void* A, long lda, const void* W, long ldw, void* C, long ldc, int M, int F,
                                   int K, int max_blocks, hipStream_t st) {
-  return tgemm_tn_launch(A, lda, W, ldw, C, ldc, nullptr, M, F, K, max_blocks, 1, st);
+  return tgemm_tn_launch(A, lda, W, ldw, C, ldc, nullptr, M, F, K, max_blocks, 1, nullptr, 0, 1, st);
 }
 
 // dW[N, K] (fp32, leading dimension ldw) += dY[M, N]^T . X[M, K]. N a multiple of 128, K of 256, rows 16-byte aligned.
@@ -898,7 +914,7 @@ extern "C" int areal_tgemm_nn(const void* dY, long ldy, const void* W, long ldw,
   }
   hipLaunchKernelGGL((tgemm_kernel<0, true, false>), dim3((unsigned)std::min(items, 256l)), dim3(512), TG_LDS + TG_OUT, st, a);
   if (splits > 1)
-    hipLaunchKernelGGL(tgemm_nn_sum_kernel, dim3((unsigned)(tiles - whole) * 32), dim3(256), 0, st, a);
+    hipLaunchKernelGGL(tgemm_sum_kernel, dim3((unsigned)(tiles - whole) * 32), dim3(256), 0, st, a);
   return (int)hipGetLastError();
 }
 
