@@ -670,10 +670,14 @@ class ModelRunner:
             if gate_up_mode == "experts":
                 # router + permutation + grouped GEMMs + weighted combine; the sum joins the residual stream in the
                 # next norm's kernel
-                mixed = blk.mlp(x, None, self.model.ep_group)
+                mixed = blk.mlp(x, None, self.model.ep_group) if tp else blk.mlp.decode_parts(x, self.model.ep_group)
                 if tp:
                     self._tp_all_reduce(mixed)
-                x, residual = ops.rmsnorm(mixed, nw, eps, residual, gemma)
+                if isinstance(mixed, tuple):
+                    ys, weights, inv = mixed
+                    x, residual = ops.moe_combine_rmsnorm(ys, weights, inv, residual, nw, eps, gemma)
+                else:
+                    x, residual = ops.rmsnorm(mixed, nw, eps, residual, gemma)
                 continue
             if gate_up_mode == "balanced":
                 act = dg.dgemm_swiglu_balanced(x, blk.mlp.gate_up, act=gate_act)

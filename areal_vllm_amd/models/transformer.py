@@ -301,8 +301,14 @@ class MoE(nn.Module):
                 break
         return torch.exp(lk + f.unsqueeze(1) + g.unsqueeze(0))
 
-    def _route(self, x, router, ep_group, n_valid: int, aux_scale: float):
-        """Route the rows of `x` (the first `n_valid` are real tokens) to their experts and combine the outputs.
+    def decode_parts(self, x, ep_group):
+        """The layer of a decode step up to the recombination: (expert outputs in expert order, weights [T, k], inverse of the
+        order) for `ops.moe_combine_rmsnorm`, or the mixed rows themselves where the layer needs another path."""
+        return self._route(x, self.router, ep_group, x.shape[0], 1.0, parts=True)
+
+    def _route(self, x, router, ep_group, n_valid: int, aux_scale: float, parts: bool = False):
+        """Route the rows of `x` (the first `n_valid` are real tokens) to their experts and combine the outputs (`parts`:
+        leave that to the caller where the layer has no host synchronisation).
         Router options: see `ModelConfig.moe_*` (reference ``realhf/impl/model/modules/moe/router.py:53-161``,
         ``realhf/impl/model/utils/moe.py:54-100,310-390``)."""
         cfg = self.cfg
@@ -312,9 +318,9 @@ class MoE(nn.Module):
         if cfg.moe_input_jitter_eps and self.training:  # the router alone sees the jittered input
             eps = float(cfg.moe_input_jitter_eps)
             xr = x * torch.empty_like(x).uniform_(1.0 - eps, 1.0 + eps)
-        raw = F.linear(xr, router)
         plain = cfg.moe_routing_type in ("aux_loss", "none")
         fused_route = plain and not torch.is_grad_enabled() and not self.training
+        raw = None if fused_route else F.linear(xr, router)
         logits = None if fused_route else raw.float()
         aux = None
         if cfg.moe_z_loss_coef > 0 and self.training and n_valid > 0:
@@ -323,7 +329,7 @@ class MoE(nn.Module):
         if fused_route:
             # scoring / serving pass: softmax (fp32 arithmetic on the projection's output), top-k and
             # re-normalisation in one launch; weights in the dtype the combine multiplies in
-            topv, topi = ops.moe_topk(raw, k, cfg.norm_topk_prob, out_dtype=x.dtype)
+            topv, topi = ops.moe_route(xr, router, k, cfg.norm_topk_prob, out_dtype=x.dtype)
         elif cfg.moe_routing_type == "sinkhorn":
             act = torch.sigmoid(logits) if k == 1 else probs
             if self.training:
@@ -370,14 +376,18 @@ class MoE(nn.Module):
         # expert-sorted position -> (token, choice) pair t*k + j (stable), its inverse, the source row of every
         # position and the experts' row ranges: one counting sort (``ops/moe.py::moe_sort``)
         order, inv, src_row, offsets = ops.moe_sort(flat_e, E, k)
-        xs = ops.moe_permute(x, order, inv, k, src_row)
         if (cfg.moe_capacity_factor is None and not torch.is_grad_enabled() and not (ep_group is not None and self.ep_size > 1)
-                and ops.grouped_gemm_offsets_ok(xs, self.gate_up) and ops.grouped_gemm_offsets_ok(xs, self.down)):
+                and ops.grouped_gemm_offsets_ok(x, self.gate_up) and ops.grouped_gemm_offsets_ok(x, self.down)):
             # inference: the experts' row ranges stay on the device (the grouped kernels read them there), so the
             # layer has no host synchronisation and can sit inside a captured decode graph
             offsets = offsets[:E + 1]
-            h = ops.swiglu(ops.grouped_gemm_offsets(xs, self.gate_up, offsets))
-            return ops.moe_combine(ops.grouped_gemm_offsets(h, self.down, offsets), topv, order, inv)
+            if ops.gate_up_rows_ok(T * k, self.gate_up):
+                h = ops.grouped_gate_up(x, src_row, self.gate_up, offsets)
+            else:
+                h = ops.swiglu(ops.grouped_gemm_offsets(ops.moe_permute(x, order, inv, k, src_row), self.gate_up, offsets))
+            ys = ops.grouped_gemm_offsets(h, self.down, offsets)
+            return (ys, topv, inv) if parts else ops.moe_combine(ys, topv, order, inv)
+        xs = ops.moe_permute(x, order, inv, k, src_row)
         counts = (offsets[1:] - offsets[:-1]).long()  # E experts + the bin of dropped pairs
         if cfg.moe_capacity_factor is not None:
             n_drop = int(counts[E])

@@ -30,5 +30,6 @@ from .sampling import TokenCounts, advance_step_, decode_advance_, decode_begin_
 from . import train_gemm  # noqa: F401
 from .linear import embedding, linear  # noqa: F401
 from .decode_gemm import dgemm, splitk_residual_rmsnorm, splitk_rope_cache_write  # noqa: F401
-from .grouped_gemm import grouped_gemm, grouped_gemm_offsets, grouped_gemm_offsets_ok, grouped_gemm_ref  # noqa: F401
-from .moe import moe_combine, moe_permute, moe_sort, moe_topk  # noqa: F401
+from .grouped_gemm import (gate_up_rows_ok, grouped_gate_up, grouped_gemm, grouped_gemm_offsets,  # noqa: F401
+                           grouped_gemm_offsets_ok, grouped_gemm_ref)
+from .moe import moe_combine, moe_combine_rmsnorm, moe_permute, moe_route, moe_sort, moe_topk  # noqa: F401

@@ -223,6 +223,29 @@ def grouped_gemm_offsets(x: torch.Tensor, w: torch.Tensor, offsets: torch.Tensor
     return _launch(x.contiguous(), w, offsets)
 
 
+def gate_up_rows_ok(n_pairs: int, w: torch.Tensor) -> bool:
+    """Whether `grouped_gate_up` is the kernel for so many rows: its tiles are the small ones, and a column tile holds 64
+    gate and 64 up columns."""
+    return (n_pairs > 0 and not _big_tiles(n_pairs, w.shape[0]) and "AREAL_GROUPED_GEMM_TILE_M" not in os.environ
+            and w.shape[1] % 128 == 0 and w.stride(0) % 8 == 0 and n_pairs // 64 + w.shape[0] <= 65535)
+
+
+def grouped_gate_up(x: torch.Tensor, src_row: torch.Tensor, w: torch.Tensor, offsets: torch.Tensor) -> torch.Tensor:
+    """silu(x[src_row] @ gate^T) * (x[src_row] @ up^T) of every row's expert, forward only, in one launch: x [T, K], src_row
+    int64 [R] = the source row of every position of the expert order, w [E, 2 F, K] = gate rows | up rows, offsets int32
+    [E + 1] on the device -> [R, F]; the roundings are those of the gather, the grouped GEMM and the activation run apart."""
+    x = x.contiguous() if x.data_ptr() % 16 == 0 else x.clone(memory_format=torch.contiguous_format)
+    R, K = src_row.numel(), x.shape[1]
+    E, N, K2 = w.shape
+    assert K == K2 and offsets.numel() == E + 1 and offsets.dtype == torch.int32 and src_row.dtype == torch.int64
+    assert w.stride(2) == 1 and w.stride(1) == K and src_row.is_contiguous()
+    out = torch.empty(R, N // 2, dtype=x.dtype, device=x.device)
+    L.check(L.lib().areal_grouped_gate_up(L.ptr(x), L.ptr(src_row), L.ptr(w), L.ptr(out), L.ptr(offsets), L.c_int(R), L.c_int(E),
+                                          L.c_int(N), L.c_int(K), L.c_int64(w.stride(0)), L.c_int(R // 64 + E), L.stream_ptr()),
+            "grouped_gate_up")
+    return out
+
+
 def grouped_gemm_rows(x: torch.Tensor, w: torch.Tensor, offsets: torch.Tensor) -> torch.Tensor:
     """Forward-only grouped GEMM for ANY operand shape and for bf16 or fp32 (fp32: true fp32 products): the MFMA
     kernel where it applies, otherwise an LDS-tiled kernel with fp32 accumulation. x [T, K] rows sorted by expert,

@@ -54,10 +54,16 @@ DEVINL int gg_off(int row, int ch) { return row * 128 + ((ch ^ ((row >> 1) & 7))
 // MFMAs instead of one (64 x 64: the K loop is bound by LDS reads and barriers, not by the matrix cores).
 // KH = number of 64-deep sub-tiles staged per step: with 2 a step holds twice the MFMA work between the barrier
 // pairs and behind every register prefetch of the next step's global loads.
-template <int TM, int TN, int KH, bool NT>
+// GATED: the rows are gathered on the way in (row p of the sorted order is x[src_row[p]]) and the weights are a gate half and
+// an up half: the W tile takes TN / 2 columns of each, a lane's accumulators ni = 0 | 1 are a token's gate and up values of the
+// same columns, and the epilogue stores silu(gate) * up (gate and up rounded to bf16 first), [T, N / 2]. For a decode step,
+// where the gather and the activation are launches of their own and little else (64 / 512 rows of 2048, 8 of 128 experts
+// of 768: 166 -> 158 us / 197 -> 167, 1 row 29 -> 25).
+template <int TM, int TN, int KH, bool NT, bool GATED>
 __global__ __launch_bounds__(256) void grouped_gemm_nt_kernel(
-    const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, bf16_t* __restrict__ out,
+    const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, bf16_t* __restrict__ out, const int64_t* __restrict__ src_row,
     const int* __restrict__ offsets, int E, int N, int K, int64_t w_expert_stride) {
+  static_assert(!GATED || TN == 128, "a wave's two column tiles are gate and up");
   constexpr int MI = TM / 64, NI = TN / 64;
   __shared__ __attribute__((aligned(16))) char smem[KH * (TM + TN) * 128];
   char* as = smem;                  // x tile  [KH][TM rows][64 k]
@@ -67,7 +73,7 @@ __global__ __launch_bounds__(256) void grouped_gemm_nt_kernel(
   int tile, e, row_lo, row_hi;
   if (!gg_find_tile<TM>(offsets, E, blockIdx.y, e, tile, row_lo, row_hi)) return;  // beyond the last tile (the grid is an upper bound)
   const int m0 = row_lo + tile * TM;
-  const int n0 = blockIdx.x * TN;
+  const int n0 = blockIdx.x * (GATED ? TN / 2 : TN);
   const bf16_t* we = w + (size_t)e * w_expert_stride;
 
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
@@ -80,17 +86,24 @@ __global__ __launch_bounds__(256) void grouped_gemm_nt_kernel(
   // the launch below).
   const int lrow = tid >> 3, lch = tid & 7;
   bf16x8 areg[KH * TM / 32] = {}, breg[KH * TN / 32];
+  int64_t arow[TM / 32];  // source row of each of this thread's tile rows
+#pragma unroll
+  for (int i = 0; i < TM / 32; ++i) {
+    const int m = m0 + lrow + 32 * i;
+    arow[i] = GATED ? (m < row_hi ? src_row[m] : 0) : m;
+  }
   auto load = [&](int k0) {
 #pragma unroll
     for (int h = 0; h < KH; ++h) {
 #pragma unroll
       for (int i = 0; i < TM / 32; ++i) {
         const int m = m0 + lrow + 32 * i;
-        if (m < row_hi) areg[h * (TM / 32) + i] = ld8(x + (size_t)m * K + k0 + 64 * h + lch * 8);
+        if (m < row_hi) areg[h * (TM / 32) + i] = ld8(x + (size_t)arow[i] * K + k0 + 64 * h + lch * 8);
       }
 #pragma unroll
       for (int i = 0; i < TN / 32; ++i) {
-        const bf16x8* p = reinterpret_cast<const bf16x8*>(we + (size_t)(n0 + lrow + 32 * i) * K + k0 + 64 * h + lch * 8);
+        const int n = GATED ? (i & 1) * (N / 2) + n0 + 32 * (i >> 1) + lrow : n0 + lrow + 32 * i;
+        const bf16x8* p = reinterpret_cast<const bf16x8*>(we + (size_t)n * K + k0 + 64 * h + lch * 8);
         breg[h * (TN / 32) + i] = NT ? __builtin_nontemporal_load(p) : *p;
       }
     }
@@ -142,7 +155,22 @@ __global__ __launch_bounds__(256) void grouped_gemm_nt_kernel(
 #pragma unroll
   for (int mi = 0; mi < MI; ++mi) {
     const int m = m0 + (TM / 2) * wm + 32 * mi + r;
-    if (m < row_hi) {
+    if constexpr (GATED) {
+      if (m < row_hi) {
+        bf16_t* op = out + (size_t)m * (N / 2) + n0 + 32 * wn;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          bf16x4 v;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const float a = bf2f(f2bf(acc[2 * mi][4 * g + j])), u = bf2f(f2bf(acc[2 * mi + 1][4 * g + j]));
+            const float sig = 1.f / (1.f + __expf(-a));
+            v[j] = f2bf(a * sig * u);
+          }
+          *reinterpret_cast<bf16x4*>(op + 8 * g + 4 * hf) = v;
+        }
+      }
+    } else if (m < row_hi) {
 #pragma unroll
       for (int ni = 0; ni < NI; ++ni) {
         bf16_t* op = out + (size_t)m * N + n0 + (TN / 2) * wn + 32 * ni;
@@ -166,6 +194,13 @@ extern "C" int areal_grouped_gemm_tile_m(int T, int E, int N, int tile_m) {
   return (E > 0 && T / E >= 256) ? 128 : 64;
 }
 
+// Weights past the caches: where most experts' rows are one tile, so that a weight is read once (up to 48 rows an expert on
+// average: at 64 half of them are two), and where there is more than a workgroup for each of the 256 CUs: fewer wait for
+// single loads, which are then slower. us from the caches / past them, cold weights: 128 experts, 1536 columns, 2048 deep,
+// 7 rows 18 / 24, 32 31 / 31, 64 59 / 52, 512 164 / 149, 48 an expert 193 / 179, 64 212 / 240, 255 465 / 642; 8 experts,
+// 14336 columns, 4096 deep, 1 row 32 / 48, 2 55 / 55, 4 87 / 77, 64 184 / 167; 16 of 704 columns, 1024 deep, 16 rows 9 / 12.
+static bool gg_stream(int T, int E, int col_tiles) { return T <= 48l * E && (long)(T < E ? T : E) * col_tiles > 256; }
+
 extern "C" int areal_grouped_gemm_nt(const void* x, const void* w, void* out, const int* offsets, int T,
                                      int E, int N, int K, int64_t w_expert_stride, int max_tiles, int tile_m,
                                      hipStream_t st) {
@@ -183,20 +218,32 @@ extern "C" int areal_grouped_gemm_nt(const void* x, const void* w, void* out, co
     const char* e = getenv("AREAL_GROUPED_GEMM_KSTEP");
     return e && atoi(e) == 128;
   }();
-  // Weights past the caches: where most experts' rows are one tile, so that a weight is read once (up to 48 rows an expert on
-  // average: at 64 half of them are two), and where there is more than a workgroup for each of the 256 CUs: fewer wait for
-  // single loads, which are then slower. us from the caches / past them, cold weights: 128 experts, 1536 columns, 2048 deep,
-  // 7 rows 18 / 24, 32 31 / 31, 64 59 / 52, 512 164 / 149, 48 an expert 193 / 179, 64 212 / 240, 255 465 / 642; 8 experts,
-  // 14336 columns, 4096 deep, 1 row 32 / 48, 2 55 / 55, 4 87 / 77, 64 184 / 167; 16 of 704 columns, 1024 deep, 16 rows 9 / 12.
-  const bool stream = T <= 48l * E && (long)(T < E ? T : E) * (N / tn) > 256;
+  const bool stream = gg_stream(T, E, N / tn);
 #define AREAL_GG_LAUNCH(TM_, TN_, KH_, NT_)                                                                    \
-  hipLaunchKernelGGL((grouped_gemm_nt_kernel<TM_, TN_, KH_, NT_>), grid, block, 0, st, (const bf16_t*)x,        \
-                     (const bf16_t*)w, (bf16_t*)out, offsets, E, N, K, w_expert_stride)
+  hipLaunchKernelGGL((grouped_gemm_nt_kernel<TM_, TN_, KH_, NT_, false>), grid, block, 0, st, (const bf16_t*)x, \
+                     (const bf16_t*)w, (bf16_t*)out, (const int64_t*)nullptr, offsets, E, N, K, w_expert_stride)
   if (tm == 128 && tn == 128) {
     if (deep && K % 128 == 0) AREAL_GG_LAUNCH(128, 128, 2, false); else AREAL_GG_LAUNCH(128, 128, 1, false);
   } else if (tm == 128) AREAL_GG_LAUNCH(128, 64, 1, false);
   else if (tn == 128) { if (stream) AREAL_GG_LAUNCH(64, 128, 1, true); else AREAL_GG_LAUNCH(64, 128, 1, false); }
   else { if (stream) AREAL_GG_LAUNCH(64, 64, 1, true); else AREAL_GG_LAUNCH(64, 64, 1, false); }
+#undef AREAL_GG_LAUNCH
+  return (int)hipGetLastError();
+}
+
+// out [T, N / 2] = silu(x[src_row] . gate^T) * (x[src_row] . up^T), W [E, N, K] with the gate rows ahead of the up rows; tiles of
+// 64 rows: max_tiles >= T / 64 + E
+extern "C" int areal_grouped_gate_up(const void* x, const int64_t* src_row, const void* w, void* out, const int* offsets, int T,
+                                     int E, int N, int K, int64_t w_expert_stride, int max_tiles, hipStream_t st) {
+  if (T == 0 || E == 0) return 0;
+  if (N % 128 != 0 || K % 64 != 0) return -1;
+  if (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) % 16 != 0 || w_expert_stride % 8 != 0) return -2;
+  if (max_tiles < T / 64 + E || max_tiles > 65535) return -3;
+  const dim3 grid(N / 128, max_tiles), block(256);
+#define AREAL_GG_LAUNCH(NT_)                                                                                      \
+  hipLaunchKernelGGL((grouped_gemm_nt_kernel<64, 128, 1, NT_, true>), grid, block, 0, st, (const bf16_t*)x,         \
+                     (const bf16_t*)w, (bf16_t*)out, src_row, offsets, E, N, K, w_expert_stride)
+  if (gg_stream(T, E, N / 128)) AREAL_GG_LAUNCH(true); else AREAL_GG_LAUNCH(false);
 #undef AREAL_GG_LAUNCH
   return (int)hipGetLastError();
 }

@@ -127,6 +127,88 @@ extern "C" int areal_moe_combine_dots(const void* g, const void* src, const int6
 }
 
 // ---------------------------------------------------------------------------------------------------------------
+
+// The weighted sum of a token's expert outputs (rounded to bf16, as above), the residual stream's sum (rounded) and its
+// RMSNorm, for a decode step: one workgroup a row, every thread 8 columns of up to MAXC chunks, a row's k expert rows
+// requested at once. As two kernels the sum made a trip through memory and a second launch (64 rows of 2048,
+// k = 8: 5.2 + 5.7 us in a decode step, 6.7 now).
+template <int KMAX, int MAXC>
+__global__ __launch_bounds__(256) void moe_combine_rmsnorm_kernel(
+    const bf16_t* __restrict__ src, const int64_t* __restrict__ inv, const bf16_t* __restrict__ w,
+    const bf16_t* __restrict__ res, const bf16_t* __restrict__ nw, bf16_t* __restrict__ res_out, bf16_t* __restrict__ y, int k,
+    int H, float eps, int gemma) {
+  __shared__ float red[16];
+  const int64_t t = blockIdx.x;
+  int64_t rows[KMAX];
+  float wt[KMAX];
+#pragma unroll
+  for (int j = 0; j < KMAX; ++j) {
+    rows[j] = j < k ? inv[t * k + j] : 0;
+    wt[j] = j < k ? bf2f(w[t * k + j]) : 0.f;
+  }
+  float v[MAXC][8];
+  bf16x8 ww[MAXC];  // requested ahead of the reduction's barriers
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < MAXC; ++i) {
+    const int c = 8 * (threadIdx.x + 256 * i);
+    if (c < H) {
+      const bf16x8 r = ld8(res + t * (int64_t)H + c);
+      ww[i] = ld8(nw + c);
+      float acc[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) acc[q] = 0.f;
+#pragma unroll
+      for (int j = 0; j < KMAX; ++j) {
+        if (j < k) {
+          const bf16x8 a = ld8(src + rows[j] * (int64_t)H + c);
+#pragma unroll
+          for (int q = 0; q < 8; ++q) acc[q] += wt[j] * bf2f(a[q]);
+        }
+      }
+      bf16x8 s;
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        s[q] = f2bf(bf2f(f2bf(acc[q])) + bf2f(r[q]));
+        v[i][q] = bf2f(s[q]);
+        ss += v[i][q] * v[i][q];
+      }
+      st8(res_out + t * (int64_t)H + c, s);
+    }
+  }
+  ss = block_sum(ss, red);
+  const float rstd = rsqrtf(ss / (float)H + eps);
+#pragma unroll
+  for (int i = 0; i < MAXC; ++i) {
+    const int c = 8 * (threadIdx.x + 256 * i);
+    if (c < H) {
+      bf16x8 o;
+#pragma unroll
+      for (int q = 0; q < 8; ++q) o[q] = f2bf(v[i][q] * rstd * (bf2f(ww[i][q]) + (gemma ? 1.f : 0.f)));
+      st8(y + t * (int64_t)H + c, o);
+    }
+  }
+}
+
+// src [T*k, H], inv [T*k], w [T, k] bf16, res / res_out / y [T, H], nw [H]; H a multiple of 8 up to 8192, k up to 16
+extern "C" int areal_moe_combine_rmsnorm(const void* src, const int64_t* inv, const void* w, const void* res, const void* nw,
+                                         void* res_out, void* y, int64_t T, int k, int H, float eps, int gemma,
+                                         hipStream_t st) {
+  if (H % 8 != 0 || H < 8 || H > 8192 || k < 1 || k > 16 || T < 0 || T > 0x7fffffff) return -1;
+  if (((uintptr_t)src | (uintptr_t)res | (uintptr_t)nw | (uintptr_t)res_out | (uintptr_t)y) % 16 != 0) return -2;
+  if (T == 0) return 0;
+#define LAUNCH(KM, MC)                                                                                                   \
+  hipLaunchKernelGGL((moe_combine_rmsnorm_kernel<KM, MC>), dim3((unsigned)T), dim3(256), 0, st, (const bf16_t*)src, inv, \
+                     (const bf16_t*)w, (const bf16_t*)res, (const bf16_t*)nw, (bf16_t*)res_out, (bf16_t*)y, k, H, eps, gemma)
+  if (k <= 8) {
+    if (H <= 2048) LAUNCH(8, 1); else if (H <= 4096) LAUNCH(8, 2); else LAUNCH(8, 4);
+  } else {
+    if (H <= 2048) LAUNCH(16, 1); else if (H <= 4096) LAUNCH(16, 2); else LAUNCH(16, 4);
+  }
+#undef LAUNCH
+  return (int)hipGetLastError();
+}
+
 // Routing: softmax + top-k of the router logits, and the expert-sorted order of the (token, choice) pairs, as a few
 // fixed launches. Done with library primitives the same work is a dozen dependent small kernels per layer (softmax,
 // top-k, sort, index-put, bincount, cumsum, floor-divide ...), about a third of a decode step of a 128-expert model.
@@ -141,12 +223,17 @@ extern "C" int areal_moe_combine_dots(const void* g, const void* src, const int6
 // Expert ids may be 0 .. E: id E is the bin of dropped pairs, sorted behind every expert.
 constexpr int RT_MAX_PER_LANE = 8;  // experts <= 512
 
+// What bounds it is the chain of k extractions: the wave's maximum through the VALU's lane exchanges and the lowest expert
+// that holds it from a ballot, where value and index used to travel through six LDS permutations an extraction (64 rows, 8 of
+// 128 experts: 7.6 us a launch in a decode step, 7.1 now with ten partial products summed on the way, whose GEMM takes 4.0
+// where the whole product took 10.5). slabs > 0: `logits` are that many fp32 partial products [slabs, T, E] of the router,
+// whose sum is rounded to bf16 as the projection's output is.
 template <typename TIN, int PER_LANE>
-__global__ __launch_bounds__(256) void moe_topk_kernel(const TIN* __restrict__ logits, int64_t T, int E, int k,
+__global__ __launch_bounds__(256) void moe_topk_kernel(const TIN* __restrict__ logits, int slabs, int64_t T, int E, int k,
                                                        int norm, int64_t* __restrict__ topi,
                                                        float* __restrict__ topv, bf16_t* __restrict__ topv_bf) {
   const int lane = threadIdx.x & 63;
-  const int64_t t = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int64_t t = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
   if (t >= T) return;
   const TIN* row = logits + t * (int64_t)E;
   float v[PER_LANE];
@@ -155,6 +242,12 @@ __global__ __launch_bounds__(256) void moe_topk_kernel(const TIN* __restrict__ l
   for (int i = 0; i < PER_LANE; ++i) {
     const int e = lane + 64 * i;
     v[i] = e < E ? (float)row[e] : -INFINITY;
+    if (sizeof(TIN) == 4 && slabs > 0 && e < E) {
+      float s = v[i];
+#pragma unroll 4
+      for (int j = 1; j < slabs; ++j) s += (float)row[(size_t)j * T * E + e];
+      v[i] = bf2f(f2bf(s));
+    }
     mx = fmaxf(mx, v[i]);
   }
   mx = wave_max(mx);
@@ -166,25 +259,18 @@ __global__ __launch_bounds__(256) void moe_topk_kernel(const TIN* __restrict__ l
   int mine_i = 0;
   float picked = 0.f;
   for (int j = 0; j < k; ++j) {
-    float bv = -INFINITY;
-    int bi = 0x7fffffff;
+    float bv = v[0];
 #pragma unroll
-    for (int i = 0; i < PER_LANE; ++i) {  // ascending expert index within the lane: first maximum wins
-      if (v[i] > bv) {
-        bv = v[i];
-        bi = lane + 64 * i;
+    for (int i = 1; i < PER_LANE; ++i) bv = fmaxf(bv, v[i]);
+    bv = wave_max(bv);
+    int bi = 0;  // also where fewer finite logits than k are left, which finite router outputs do not give
+    if (bv > -INFINITY) {
+#pragma unroll
+      for (int i = PER_LANE - 1; i >= 0; --i) {  // the lowest index of the largest value
+        const unsigned long long has = __ballot(v[i] == bv);
+        if (has) bi = 64 * i + __ffsll(has) - 1;
       }
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      const float ov = __shfl_xor(bv, o, 64);
-      const int oi = __shfl_xor(bi, o, 64);
-      if (ov > bv || (ov == bv && oi < bi)) {
-        bv = ov;
-        bi = oi;
-      }
-    }
-    if (bi >= E) bi = 0;  // fewer finite logits than k: cannot happen for finite router outputs
     const float p = __expf(bv - mx) / se;
     picked += p;
     if (lane == j) {
@@ -365,12 +451,13 @@ __global__ __launch_bounds__(1024) void moe_sort_single_kernel(const int64_t* __
 }
 
 template <typename TIN>
-static int topk_launch(const TIN* logits, int64_t T, int E, int k, int norm, int64_t* topi, float* topv,
+static int topk_launch(const TIN* logits, int slabs, int64_t T, int E, int k, int norm, int64_t* topi, float* topv,
                        bf16_t* topv_bf, hipStream_t st) {
-  const dim3 grid((unsigned)((T + 3) / 4)), block(256);
+  const int waves = T <= 1024 ? 1 : 4;  // a row a CU while there are CUs: a workgroup's rows share its load path
+  const dim3 grid((unsigned)((T + waves - 1) / waves)), block(64 * waves);
 #define TOPK_CASE(P) \
   if (E <= 64 * P) { \
-    hipLaunchKernelGGL((moe_topk_kernel<TIN, P>), grid, block, 0, st, logits, T, E, k, norm, topi, topv, topv_bf); \
+    hipLaunchKernelGGL((moe_topk_kernel<TIN, P>), grid, block, 0, st, logits, slabs, T, E, k, norm, topi, topv, topv_bf); \
     return (int)hipGetLastError(); \
   }
   TOPK_CASE(1) TOPK_CASE(2) TOPK_CASE(4) TOPK_CASE(8)
@@ -378,13 +465,14 @@ static int topk_launch(const TIN* logits, int64_t T, int E, int k, int norm, int
   return -1;
 }
 
-// logits [T, E] fp32 (dtype 1) or bf16 (dtype 0); weights are written as fp32 (topv), bf16 (topv_bf) or both.
-extern "C" int areal_moe_topk(const void* logits, int dtype, int64_t T, int E, int k, int norm, int64_t* topi,
+// logits [T, E] fp32 (dtype 1) or bf16 (dtype 0); slabs > 0: fp32 partial products [slabs, T, E]; weights are written as fp32
+// (topv), bf16 (topv_bf) or both.
+extern "C" int areal_moe_topk(const void* logits, int dtype, int slabs, int64_t T, int E, int k, int norm, int64_t* topi,
                               float* topv, void* topv_bf, hipStream_t st) {
   if (T == 0) return 0;
-  if (E < 1 || E > 64 * RT_MAX_PER_LANE || k < 1 || k > 64 || k > E) return -1;
-  if (dtype == 0) return topk_launch((const bf16_t*)logits, T, E, k, norm, topi, topv, (bf16_t*)topv_bf, st);
-  return topk_launch((const float*)logits, T, E, k, norm, topi, topv, (bf16_t*)topv_bf, st);
+  if (E < 1 || E > 64 * RT_MAX_PER_LANE || k < 1 || k > 64 || k > E || slabs < 0 || (slabs && dtype == 0)) return -1;
+  if (dtype == 0) return topk_launch((const bf16_t*)logits, 0, T, E, k, norm, topi, topv, (bf16_t*)topv_bf, st);
+  return topk_launch((const float*)logits, slabs, T, E, k, norm, topi, topv, (bf16_t*)topv_bf, st);
 }
 
 // Sigmoid scores with group-limited choice: the E experts form `n_groups` equal groups of neighbours, a group's score is
