@@ -29,6 +29,14 @@ typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 DEVINL float bf2f(bf16_t x) { return (float)x; }
 DEVINL bf16_t f2bf(float x) { return (bf16_t)x; }
 
+// Weight rows of a multiple of 4096 bytes: the workgroups of a product that streams its weights start together, and in the same
+// reduction order they all read the same 128 bytes of their rows, addresses equal modulo 4096, which meet in a few of the
+// memory's channels. Workgroup t of such a product starts at step t * k_rotation(K) instead and wraps round. us without /
+// with, cold weights: 151936 columns, 64 rows, K 2048 145 / 127 (at 1536, which spreads by itself, 100 / 100), 4096 262 / 220;
+// 28672 columns, 8 rows, 4096 51 / 38, 8192 106 / 69; 65536 columns, 64 rows, 8192 238 / 161. Between: 1024 50 / 52, 2560 123 /
+// 124, 3072 135 / 136, 3584 148 / 148, 5120 220 / 220 (100352 columns, 64 rows).
+static inline int k_rotation(int K) { return K % 2048 == 0 ? 13 : 0; }
+
 // Exchanges across 16- and 32-lane rows in the VALU (v_permlane16_swap / v_permlane32_swap of gfx950) instead of
 // through the LDS crossbar (`__shfl_xor(v, 16 | 32)` compiles to ds_bpermute_b32: an LDS-pipe round trip of ~100
 // cycles on the dependent path, and LDS traffic in kernels that otherwise use none). Fed the same register twice

@@ -40,6 +40,7 @@ struct DGArgs {
   void* Y;
   long ys;
   int M, N, K, k_per_split;
+  int rot;  // column tile t starts its reduction at step t * rot (modulo the steps) and wraps round: k_rotation (common.hpp)
   int nt;  // non-temporal weight loads (each weight byte is read once per launch)
   int act;  // gate activation of the gated-MLP epilogue (gate_act_f)
   unsigned inv_y = 0, inv_z = 0;  // ceil(2^32 / column tiles), ceil(2^32 / row blocks); 0: workgroups in launch order
@@ -157,7 +158,10 @@ __global__ __launch_bounds__(64 * (WM * WN + LW)) void dgemm_kernel(const DGArgs
       src[j] = a.X + (size_t)m * a.xs + k_begin + 8 * c;
     }
   }
+  const int rot = (ct * a.rot) % nsteps;
   auto issue = [&](int buf, int step) {
+    step += rot;
+    step -= step >= nsteps ? nsteps : 0;
     char* base = smem + buf * STAGE_BYTES + lwave * (IPW * 1024);
 #pragma unroll
     for (int j = 0; j < IPW; ++j) {
@@ -465,6 +469,8 @@ extern "C" int areal_dgemm(const void* X, long xs, const void* W, const void* bi
   DGArgs a;
   a.X = (const bf16_t*)X; a.xs = xs; a.W = (const bf16_t*)W; a.bias = (const bf16_t*)bias; a.Y = Y; a.ys = ys;
   a.M = M; a.N = N; a.K = K; a.k_per_split = kps; a.nt = nt; a.act = act;
+  // several row blocks reread the weights from the caches: 200 / 320 rows level (K 2048 213 / 314 us and 210 / 313)
+  a.rot = ksplit == 1 && M <= 128 ? k_rotation(K) : 0;
   a.pos = nullptr; a.slots = nullptr; a.cos_t = a.sin_t = nullptr; a.q_out = a.kcache = a.vcache = nullptr;
   a.Hq = a.Hkv = 0; a.D = 2; a.max_pos = 0; a.do_rope = 0;
   switch (cfg) {
@@ -497,7 +503,7 @@ extern "C" int areal_dgemm_qkv_rope(const void* X, long xs, const void* W, const
   if (cfg == 4 && (D / 2) % 64 != 0) return -2;
   DGArgs a;
   a.X = (const bf16_t*)X; a.xs = xs; a.W = (const bf16_t*)W; a.bias = (const bf16_t*)bias; a.Y = nullptr; a.ys = 0;
-  a.M = M; a.N = N; a.K = K; a.k_per_split = K; a.nt = nt; a.act = 0;
+  a.M = M; a.N = N; a.K = K; a.k_per_split = K; a.nt = nt; a.rot = 0; a.act = 0;
   a.pos = pos; a.slots = slots; a.cos_t = cos_t; a.sin_t = sin_t; a.q_out = (bf16_t*)q_out;
   a.kcache = (bf16_t*)kcache; a.vcache = (bf16_t*)vcache; a.Hq = Hq; a.Hkv = Hkv; a.D = D; a.max_pos = max_pos;
   a.do_rope = do_rope;

@@ -62,7 +62,7 @@ DEVINL int gg_off(int row, int ch) { return row * 128 + ((ch ^ ((row >> 1) & 7))
 template <int TM, int TN, int KH, bool NT, bool GATED>
 __global__ __launch_bounds__(256) void grouped_gemm_nt_kernel(
     const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, bf16_t* __restrict__ out, const int64_t* __restrict__ src_row,
-    const int* __restrict__ offsets, int E, int N, int K, int64_t w_expert_stride) {
+    const int* __restrict__ offsets, int E, int N, int K, int64_t w_expert_stride, int rot) {
   static_assert(!GATED || TN == 128, "a wave's two column tiles are gate and up");
   constexpr int MI = TM / 64, NI = TN / 64;
   __shared__ __attribute__((aligned(16))) char smem[KH * (TM + TN) * 128];
@@ -126,11 +126,15 @@ __global__ __launch_bounds__(256) void grouped_gemm_nt_kernel(
 #pragma unroll
     for (int j = 0; j < 16; ++j) acc[t][j] = 0.f;
 
-  load(0);
+  const int first = (int)(blockIdx.y * rot) % (K / (64 * KH)) * (64 * KH);  // rot: gg_rot, at the launch
+  load(first);
   for (int k0 = 0; k0 < K; k0 += 64 * KH) {
     __syncthreads();  // previous tile fully consumed
     stage();
-    if (k0 + 64 * KH < K) load(k0 + 64 * KH);
+    if (k0 + 64 * KH < K) {
+      const int next = first + k0 + 64 * KH;
+      load(next < K ? next : next - K);
+    }
     __syncthreads();
 #pragma unroll
     for (int s = 0; s < 4 * KH; ++s) {
@@ -199,6 +203,11 @@ extern "C" int areal_grouped_gemm_tile_m(int T, int E, int N, int tile_m) {
 // single loads, which are then slower. us from the caches / past them, cold weights: 128 experts, 1536 columns, 2048 deep,
 // 7 rows 18 / 24, 32 31 / 31, 64 59 / 52, 512 164 / 149, 48 an expert 193 / 179, 64 212 / 240, 255 465 / 642; 8 experts,
 // 14336 columns, 4096 deep, 1 row 32 / 48, 2 55 / 55, 4 87 / 77, 64 184 / 167; 16 of 704 columns, 1024 deep, 16 rows 9 / 12.
+// Row tile t starts its reduction at step 13 t (k_rotation, common.hpp) while the weights are read once; with more rows, whose
+// column tiles are reread from the caches, the common order is level or better. us without / with: 128 experts, 1536 columns,
+// 2048 deep, 64 rows 60 / 52, 512 157 / 127, 1600 161 / 129, 4096 169 / 138, but 8192 207 / 213, 16000 337 / 356; 64 experts, 2816
+// columns, 2048 deep, 512 rows 152 / 119; 8 experts, 4096 columns, 14336 deep, 128 rows 199 / 186.
+static int gg_rot(int T, int E, int K) { return T <= 48l * E ? k_rotation(K) : 0; }
 static bool gg_stream(int T, int E, int col_tiles) { return T <= 48l * E && (long)(T < E ? T : E) * col_tiles > 256; }
 
 extern "C" int areal_grouped_gemm_nt(const void* x, const void* w, void* out, const int* offsets, int T,
@@ -218,10 +227,11 @@ extern "C" int areal_grouped_gemm_nt(const void* x, const void* w, void* out, co
     const char* e = getenv("AREAL_GROUPED_GEMM_KSTEP");
     return e && atoi(e) == 128;
   }();
+  const int rot = gg_rot(T, E, K);
   const bool stream = gg_stream(T, E, N / tn);
 #define AREAL_GG_LAUNCH(TM_, TN_, KH_, NT_)                                                                    \
   hipLaunchKernelGGL((grouped_gemm_nt_kernel<TM_, TN_, KH_, NT_, false>), grid, block, 0, st, (const bf16_t*)x, \
-                     (const bf16_t*)w, (bf16_t*)out, (const int64_t*)nullptr, offsets, E, N, K, w_expert_stride)
+                     (const bf16_t*)w, (bf16_t*)out, (const int64_t*)nullptr, offsets, E, N, K, w_expert_stride, rot)
   if (tm == 128 && tn == 128) {
     if (deep && K % 128 == 0) AREAL_GG_LAUNCH(128, 128, 2, false); else AREAL_GG_LAUNCH(128, 128, 1, false);
   } else if (tm == 128) AREAL_GG_LAUNCH(128, 64, 1, false);
@@ -240,9 +250,10 @@ extern "C" int areal_grouped_gate_up(const void* x, const int64_t* src_row, cons
   if (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) % 16 != 0 || w_expert_stride % 8 != 0) return -2;
   if (max_tiles < T / 64 + E || max_tiles > 65535) return -3;
   const dim3 grid(N / 128, max_tiles), block(256);
+  const int rot = gg_rot(T, E, K);
 #define AREAL_GG_LAUNCH(NT_)                                                                                      \
   hipLaunchKernelGGL((grouped_gemm_nt_kernel<64, 128, 1, NT_, true>), grid, block, 0, st, (const bf16_t*)x,         \
-                     (const bf16_t*)w, (bf16_t*)out, src_row, offsets, E, N, K, w_expert_stride)
+                     (const bf16_t*)w, (bf16_t*)out, src_row, offsets, E, N, K, w_expert_stride, rot)
   if (gg_stream(T, E, N / 128)) AREAL_GG_LAUNCH(true); else AREAL_GG_LAUNCH(false);
 #undef AREAL_GG_LAUNCH
   return (int)hipGetLastError();
