@@ -207,6 +207,11 @@ def merge_shard_stats(stats: torch.Tensor, group) -> Tuple[torch.Tensor, torch.T
     return m, (allst[:, 1] * f).sum(0), (allst[:, 2] * f).sum(0), allst[:, 3].sum(0)
 
 
+# Chunks whose rows go through the head at once where the logits are not written: their statistics take 3 / 32 of the bytes
+# that one chunk's logits would.
+STATS_CHUNKS = 8
+
+
 class _LMHeadLogprobFn(torch.autograd.Function):
     """hidden [T, H] x weight [V_local, H]^T -> (logp [T], entropy [T]) in row chunks.
 
@@ -218,16 +223,28 @@ class _LMHeadLogprobFn(torch.autograd.Function):
 
     The bf16 logits of every chunk are kept for the backward (288 GB of HBM makes keeping them cheaper
     than recomputing the LM-head GEMM); the backward turns them into d(logits) in place and feeds two
-    GEMMs. With `keep_logits=False` they are recomputed instead.
+    GEMMs. With `keep_logits=False` they are recomputed instead. Without a backward pass (`grad` off: the trainer's
+    recomputation) the GEMM reduces its tiles itself and no logits are written (``train_gemm.logit_stats``).
     """
 
     @staticmethod
-    def forward(ctx, hidden, weight, labels, temperature, chunk, keep_logits, vocab_start, group, reduce_dh):
+    def forward(ctx, hidden, weight, labels, temperature, chunk, keep_logits, vocab_start, group, reduce_dh, grad):
         T = hidden.shape[0]
         stats = torch.empty(4, T, dtype=torch.float32, device=hidden.device)
-        need_grad = hidden.requires_grad or weight.requires_grad
+        need_grad = grad and (hidden.requires_grad or weight.requires_grad)
         kept = []
         whole = None
+        step = chunk * STATS_CHUNKS
+        if (not need_grad and hidden.is_cuda and labels.is_contiguous()
+                and all(train_gemm.stats_supported(hidden[s:s + step], weight, temperature) for s in range(0, T, step))):
+            # no backward pass: the logits are never written
+            for s in range(0, T, step):
+                train_gemm.logit_stats(hidden[s:s + step], weight, labels[s:s + step], temperature, vocab_start,
+                                       stats[:, s:s + step])
+            logp, ent, lse, ez = _finalize(*merge_shard_stats(stats, group))
+            ctx.save_for_backward(hidden, weight, labels, lse, ez)
+            ctx.meta = (temperature, chunk, False, vocab_start, group, reduce_dh)
+            return logp, ent
         if need_grad and keep_logits and T > chunk and weight.dtype == hidden.dtype and weight.shape[0] % 8 == 0:
             # one tensor for all chunks: the backward then works on all rows at once
             whole = torch.empty(T, weight.shape[0], dtype=hidden.dtype, device=hidden.device)
@@ -289,7 +306,7 @@ class _LMHeadLogprobFn(torch.autograd.Function):
                 done(weight)
         if reduce_dh and _group_size(group) > 1:
             dist.all_reduce(dh, group=group)
-        return dh, dw, None, None, None, None, None, None, None
+        return dh, dw, None, None, None, None, None, None, None, None
 
 
 def lm_head_logprobs(hidden: torch.Tensor, weight: torch.Tensor, labels: torch.Tensor, temperature: float = 1.0,
@@ -299,4 +316,4 @@ def lm_head_logprobs(hidden: torch.Tensor, weight: torch.Tensor, labels: torch.T
     weight [V, H], or the vocabulary rows [vocab_start, vocab_start + V_local) of a tensor-parallel shard
     whose peers are the ranks of `group`."""
     return _LMHeadLogprobFn.apply(hidden, weight, labels.long(), float(temperature), int(chunk), keep_logits,
-                                  int(vocab_start), group, bool(reduce_dh))
+                                  int(vocab_start), group, bool(reduce_dh), torch.is_grad_enabled())

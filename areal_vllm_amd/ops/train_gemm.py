@@ -201,6 +201,27 @@ def forward(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None
     return torch.mm(x, w.t(), out=out) if out is not None else torch.nn.functional.linear(x, w)
 
 
+def stats_supported(x: torch.Tensor, w: torch.Tensor, temperature: float) -> bool:
+    """Whether `logit_stats` is the kernel for these logits: where the products are its own anyway, over a vocabulary."""
+    return (0.0 < temperature < float("inf") and x.dim() == 2 and w.dim() == 2 and w.shape[0] >= 65536
+            and _forward_own(x.shape[0], w.shape[1], w.shape[0]) and supported(x, w) and w.shape[1] > 0)
+
+
+def logit_stats(x: torch.Tensor, w: torch.Tensor, labels: torch.Tensor, temperature: float, vocab_start: int,
+                out: torch.Tensor) -> None:
+    """out[4, M] (rows with unit stride) = ``ops.logprob.logprob_stats`` of the logits x[M, K] @ w[N, K]^T (in bf16), which are
+    not written."""
+    M, K = x.shape
+    N = w.shape[0]
+    assert labels.dtype == torch.int64 and labels.is_contiguous() and labels.numel() == M
+    assert out.dtype == torch.float32 and out.shape == (4, M) and out.stride(1) == 1
+    part = torch.empty(3 * ((N + 63) // 64) * M, dtype=torch.float32, device=x.device)
+    L.check(L.lib().areal_tgemm_stats(L.ptr(x), L.c_int64(x.stride(0)), L.ptr(w), L.c_int64(w.stride(0)), L.ptr(labels),
+                                      L.c_int64(vocab_start), L.c_int(M), L.c_int(N), L.c_int(K), L.c_float(1.0 / temperature),
+                                      L.ptr(part), L.ptr(out[0]), L.ptr(out[1]), L.ptr(out[2]), L.ptr(out[3]), L.stream_ptr()),
+            "tgemm_stats")
+
+
 # rows from which the fused gate|up + SwiGLU kernel replaces library GEMM + activation kernel in no-grad forwards
 GATED_MIN_ROWS = int(os.environ.get("AREAL_FUSED_MLP_MIN_ROWS", "4096"))
 

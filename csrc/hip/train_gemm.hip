@@ -60,6 +60,8 @@ struct TGArgs {
   // one entry {first row, end of the expert's rows, expert} a row tile, written by tgemm_table_kernel
   const int4* table;
   long stride;
+  // statistics (EPI 2): log2(e) / temperature; part = [maximum | sum | weighted sum][ceil(N / 64)][M]
+  float scale;
 };
 typedef const __attribute__((address_space(4))) int4* tg_table_t;  // scalar loads
 
@@ -105,6 +107,12 @@ typedef f32x4 tg_acc[4][2];     // [m tile][n tile] of one quadrant
 // raised by the stores in flight, so that no wait stands behind one, the times are the same.
 // What is left is power: the matrix cores are busy 73 % of the time at a clock of 1.76 GHz (2.4 nominal); bare 16x16x32
 // products of random numbers run at 1.97 PFLOP/s on the whole chip, 32x32x16 ones at 1.75.
+//
+// EPI 2 (LM head without a backward pass): the logits leave as three numbers a row and 64 columns - the largest logit z, the sum
+// of exp((z - largest) / temperature) and the same sum weighted with z, of logits rounded to bf16 - which tgemm_stats_kernel
+// merges: 1 / 11 of the bytes, and no pass that reads the logits again. 32768 x 151936 from 1536 deep: 11.45 ms with the logits
+// and 1.68 for the pass over them, now 11.80 + 0.21. What the exponentials cost (two bf16 logits a conversion, one fma and one
+// v_exp_f32 each, no subtraction: 11.98 -> 11.8) the other wave row waits for.
 //
 // GRP: the same product for rows sorted by expert, each expert's with its own B (routed experts). A row tile never straddles
 // two experts; its tail rows repeat the expert's last one and are not stored.
@@ -361,6 +369,63 @@ __global__ __launch_bounds__(512) void tgemm_kernel(const TGArgs a) {
     }
   };
 
+  // statistics: a wave's 64 columns of a row half. The four 16-lane rows hold 4 of every 16 columns of the same 16 result rows.
+  auto put_stats = [&](tg_acc& c0, tg_acc& c1, int mh) __attribute__((always_inline)) {
+    const int col = cur.n0 + wc * 64;
+    if (col >= a.N) return;
+    const bool edge = col + 64 > a.N;  // columns behind the last one (whole quads) repeat it in the operands: left out
+    float keep[3] = {0.f, 0.f, 0.f};   // row mt = fq of this lane's four
+#pragma unroll
+    for (int mt = 0; mt < 4; ++mt) {
+      float mx = -INFINITY, sum = 0.f, ws = 0.f;
+      float z[2][2][4];
+#pragma unroll
+      for (int nh = 0; nh < 2; ++nh)
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt) {
+          const f32x4& v = (nh ? c1 : c0)[mt][nt];
+#pragma unroll
+          for (int j = 0; j < 4; j += 2) {
+            const bf16x2 p = {f2bf(v[j]), f2bf(v[j + 1])};
+            const unsigned u = __builtin_bit_cast(unsigned, p);
+            z[nh][nt][j] = __uint_as_float(u << 16);
+            z[nh][nt][j + 1] = __uint_as_float(u & 0xffff0000u);
+          }
+          if (edge && col + nh * 32 + nt * 16 + fq * 4 >= a.N) continue;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) mx = fmaxf(mx, z[nh][nt][j]);
+        }
+      mx = max_xor16(max_xor32(mx));
+      const float ref = mx * a.scale;  // rounded: the merge takes the difference back
+#pragma unroll
+      for (int nh = 0; nh < 2; ++nh)
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt) {
+          if (edge && col + nh * 32 + nt * 16 + fq * 4 >= a.N) continue;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const float e = __builtin_amdgcn_exp2f(fmaf(z[nh][nt][j], a.scale, -ref));
+            sum += e;
+            ws = fmaf(e, z[nh][nt][j], ws);
+          }
+        }
+      sum = sum_xor16(sum_xor32(sum));
+      ws = sum_xor16(sum_xor32(ws));
+      if (fq == mt) {
+        keep[0] = mx;
+        keep[1] = sum;
+        keep[2] = ws;
+      }
+    }
+    const int m = cur.m0 + wr * 128 + mh * 64 + lane;  // = .. + fq * 16 + fr
+    if (m < a.M) {
+      const size_t cbs = (a.N + 63) >> 6;
+      float* op = a.part + (size_t)(col >> 6) * a.M + m;
+#pragma unroll
+      for (int i = 0; i < 3; ++i) op[i * cbs * a.M] = keep[i];
+    }
+  };
+
   // One K tile = four phases. The K tiles of the block's successive output tiles form ONE stream: the pieces staged
   // while the last two K tiles of an output tile are computed are K tiles 0 and 1 of the NEXT output tile, so the
   // prologue's load latency is paid once per block and the result stores run under the next tile's loads.
@@ -391,6 +456,7 @@ __global__ __launch_bounds__(512) void tgemm_kernel(const TGArgs a) {
     // last K tile: a row half is final once its phases are over; it leaves while the other wave group computes
     if (MODE == 2 && EPI == 0) put(acc00, acc01, 0);
     if (MODE == 2 && EPI == 1) put_gated(acc00, acc01, 0);
+    if (MODE == 2 && EPI == 2) put_stats(acc00, acc01, 0);
     // phase 3: quadrant (1, 1)
     read_a(buf, 1);
     if (go) stage(buf, PA0, t2);
@@ -405,6 +471,7 @@ __global__ __launch_bounds__(512) void tgemm_kernel(const TGArgs a) {
     mma(acc10, bf0);
     if (MODE == 2 && EPI == 0) put(acc10, acc11, 1);
     if (MODE == 2 && EPI == 1) put_gated(acc10, acc11, 1);
+    if (MODE == 2 && EPI == 2) put_stats(acc10, acc11, 1);
   };
   using B0 = std::integral_constant<int, 0>;
   using B1 = std::integral_constant<int, 1>;
@@ -795,6 +862,66 @@ __global__ __launch_bounds__(256) void tgemm_sum_kernel(const TGArgs a) {
   if (n + 8 <= a.N) *reinterpret_cast<bf16x4*>(op + 4) = bf16x4{f2bf(v1[0]), f2bf(v1[1]), f2bf(v1[2]), f2bf(v1[3])};
 }
 
+// The label's logit of every row, of the same products in the same order as the tiles above (and so with their bits): a wave's
+// 16 rows against their 16 label rows of B, the diagonal of the result. out[m] = bf16 logit * inv_temp, 0 for a label outside
+// [first, first + N).
+__global__ __launch_bounds__(256) void tgemm_label_kernel(const bf16_t* __restrict__ A, long lda, const bf16_t* __restrict__ B,
+                                                          long ldb, const int64_t* __restrict__ labels, int64_t first, int M,
+                                                          int N, int K, float inv_temp, float* __restrict__ out) {
+  const int lane = threadIdx.x & 63, fr = lane & 15, fq = lane >> 4;
+  const int m0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * 16;
+  if (m0 >= M) return;
+  const int m = min(m0 + fr, M - 1);
+  const int64_t lab = labels[m] - first;
+  const bool has = lab >= 0 && lab < N;
+  const bf16_t* pa = A + (size_t)m * lda + fq * 8;
+  const bf16_t* pb = B + (size_t)(has ? lab : 0) * ldb + fq * 8;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+  for (int k = 0; k < K; k += 32) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ld8(pb + k), ld8(pa + k), acc, 0, 0, 0);
+  // lane (fr, fq) holds rows 4 fq .. 4 fq + 3 (labels) of column fr (token)
+  const float v = (fr & 3) == 0 ? acc[0] : (fr & 3) == 1 ? acc[1] : (fr & 3) == 2 ? acc[2] : acc[3];
+  if (fq == fr >> 2 && m0 + fr < M) out[m0 + fr] = has ? bf2f(f2bf(v)) * inv_temp : 0.f;
+}
+
+// part [3][cbs][M] of the statistics form -> largest logit, sum of exponentials and weighted sum of a row, of logits divided by
+// the temperature. 32 rows a workgroup, the column blocks dealt to 32 threads each.
+__global__ __launch_bounds__(1024) void tgemm_stats_kernel(const float* __restrict__ part, int cbs, int M, float scale,
+                                                           float inv_temp, float* __restrict__ out_m, float* __restrict__ out_s,
+                                                           float* __restrict__ out_w) {
+#pragma clang fp contract(off)  // largest * scale is the rounded product that the tiles' sums are relative to
+  __shared__ float red[3][32][33];
+  const int r = threadIdx.x & 31, g = threadIdx.x >> 5, m = blockIdx.x * 32 + r;
+  const size_t plane = (size_t)cbs * M;
+  float mx = -INFINITY, s = 0.f, w = 0.f;
+  auto merge = [&](float m2, float s2, float w2) {  // sums relative to 2^round(largest * scale); a side without anything adds nothing
+    const float top = fmaxf(mx, m2), ref = top * scale;
+    const float f1 = s == 0.f ? 0.f : __builtin_amdgcn_exp2f(mx * scale - ref);
+    const float f2 = s2 == 0.f ? 0.f : __builtin_amdgcn_exp2f(m2 * scale - ref);
+    s = s * f1 + s2 * f2;
+    w = w * f1 + w2 * f2;
+    mx = top;
+  };
+  if (m < M) {
+#pragma unroll 4
+    for (int cb = g; cb < cbs; cb += 32) {
+      const float* p = part + (size_t)cb * M + m;
+      merge(p[0], p[plane], p[2 * plane]);
+    }
+  }
+  red[0][g][r] = mx;
+  red[1][g][r] = s;
+  red[2][g][r] = w;
+  __syncthreads();
+  if (g == 0 && m < M) {
+    for (int i = 1; i < 32; ++i) merge(red[0][i][r], red[1][i][r], red[2][i][r]);
+    const float ref = mx * scale, to = 1.f - 0.69314718f * fmaf(mx, scale, -ref);  // 2^(ref - largest * scale)
+    out_m[m] = mx * inv_temp;
+    out_s[m] = s * to;
+    out_w[m] = w * to * inv_temp;
+  }
+}
+
 }  // namespace
 
 // C[M, N] = A[M, K] . B[N, K]^T (+ bias). Leading dimensions in elements (multiples of 8: 16-byte rows), K a multiple
@@ -845,6 +972,33 @@ static int tgemm_tn_launch(const void* A, long lda, const void* B, long ldb, voi
 extern "C" int areal_tgemm_tn(const void* A, long lda, const void* B, long ldb, void* C, long ldc, const void* bias,
                               int M, int N, int K, int max_blocks, float* part, int whole, int splits, hipStream_t st) {
   return tgemm_tn_launch(A, lda, B, ldb, C, ldc, bias, M, N, K, max_blocks, 0, part, whole, splits, st);
+}
+
+// Statistics of the rows of logits A[M, K] . B[N, K]^T / temperature (rounded to bf16 before the division), which are not
+// written: out_m the largest, out_s sum exp(z - largest), out_w the same weighted with z, out_tgt the label's (0 for labels
+// outside [first, first + N)). part: 3 * ceil(N / 64) * M floats; inv_temp > 0. Returns -1 for shapes that areal_tgemm_tn
+// does not take.
+extern "C" int areal_tgemm_stats(const void* A, long lda, const void* B, long ldb, const int64_t* labels, long first, int M, int N,
+                                 int K, float inv_temp, float* part, float* out_m, float* out_s, float* out_w, float* out_tgt,
+                                 hipStream_t st) {
+  if (M <= 0 || N <= 0) return 0;
+  if (K % 128 != 0 || K < 128 || N % 4 != 0 || lda % 8 != 0 || ldb % 8 != 0 || !(inv_temp > 0.f)) return -1;
+  if (((uintptr_t)A | (uintptr_t)B) % 16 != 0 || !part) return -1;
+  const long tiles = (long)((M + 255) / 256) * ((N + 255) / 256);
+  if (tiles > 0x7fffffffl - 256) return -1;
+  TGArgs a{(const bf16_t*)A, lda, (const bf16_t*)B, ldb, nullptr, 0, nullptr, M, N, K, (M + 255) / 256, (N + 255) / 256, part,
+           (int)tiles, 1, K / 128, nullptr, 0, inv_temp * 1.4426950408889634f};
+  static bool attr_set = false;  // 128 KiB of dynamic LDS: above the default limit
+  if (!attr_set) {
+    HIP_RET(hipFuncSetAttribute((const void*)tgemm_kernel<2, false, false>, hipFuncAttributeMaxDynamicSharedMemorySize, TG_LDS));
+    attr_set = true;
+  }
+  hipLaunchKernelGGL((tgemm_kernel<2, false, false>), dim3((unsigned)std::min(tiles, 256l)), dim3(512), TG_LDS, st, a);
+  hipLaunchKernelGGL(tgemm_label_kernel, dim3((unsigned)((M + 63) / 64)), dim3(256), 0, st, (const bf16_t*)A, lda, (const bf16_t*)B,
+                     ldb, labels, (int64_t)first, M, N, K, inv_temp, out_tgt);
+  hipLaunchKernelGGL(tgemm_stats_kernel, dim3((unsigned)((M + 31) / 32)), dim3(1024), 0, st, part, (N + 63) / 64, M, a.scale, inv_temp,
+                     out_m, out_s, out_w);
+  return (int)hipGetLastError();
 }
 
 // C[M, F] = silu(A . Wg^T) * (A . Wu^T) with W = [Wg; Wu] of shape [2 F, K] (the gate|up projection of a gated MLP and
