@@ -637,26 +637,28 @@ extern "C" int areal_splitk_residual_rmsnorm(const float* slab, int S, const voi
 
 // qkv = bf16(sum_k slab[k] + bias), laid out [T, Hq + 2 Hkv, D]: rotate q and k (half-split layout), write q to
 // q_out [T, Hq, D] (bf16), k / v into the paged caches at slots[t] (K [P, Hkv, 32, D], V [P, Hkv, D, 32]).
-// One block per token (256 .. 1024 threads by row length): the summed row is staged in LDS (fp32, Nq floats), then
-// rotated / scattered from there.
+// One block per token and `heads` heads (64 .. 1024 threads): the summed columns are staged in LDS (fp32), then rotated /
+// scattered from there.
 __global__ __launch_bounds__(1024) void splitk_rope_cache_write_kernel(
     const float* __restrict__ slab, int S, const bf16_t* __restrict__ bias, const int* __restrict__ pos,
     const int64_t* __restrict__ slots, const float* __restrict__ cos_t, const float* __restrict__ sin_t,
     bf16_t* __restrict__ q_out, void* __restrict__ kcache, void* __restrict__ vcache, int T, int Hq, int Hkv,
     int D, int max_pos, int do_rope, const bf16_t* __restrict__ q_norm, const bf16_t* __restrict__ k_norm,
-    float norm_eps, int fp8) {
+    float norm_eps, int fp8, int heads) {
   extern __shared__ __attribute__((aligned(16))) float rowbuf[];
   const int t = blockIdx.x;
   const int half = D >> 1;
   const int lph = half >> 3;
   const int Nq = (Hq + 2 * Hkv) * D;
   const size_t stride = (size_t)T * Nq;
+  const int h0 = blockIdx.y * heads, h1 = min(Hq + 2 * Hkv, h0 + heads);  // this block's heads
+  const int c0 = h0 * D;
   // Position, slot and this thread's first rotary-table rows are requested before the slab sum, so that their
   // latency (a dependent pos -> table chain) runs under the slab loads instead of after the barrier.
   int p = pos[t];
   p = p < 0 ? 0 : (p >= max_pos ? max_pos - 1 : p);
   const int64_t slot = slots ? slots[t] : -1;
-  const int nrot = (Hq + Hkv) * lph;
+  const int nrot = max(0, min(Hq + Hkv, h1) - h0) * lph;
   f32x4 c_pre[2], s_pre[2];
   if (do_rope && (int)threadIdx.x < nrot) {
     const int sub0 = threadIdx.x % lph;
@@ -664,10 +666,10 @@ __global__ __launch_bounds__(1024) void splitk_rope_cache_write_kernel(
     const f32x4* sp4 = reinterpret_cast<const f32x4*>(sin_t + (size_t)p * half + sub0 * 8);
     c_pre[0] = cp4[0]; c_pre[1] = cp4[1]; s_pre[0] = sp4[0]; s_pre[1] = sp4[1];
   }
-  for (int c = threadIdx.x; c < (Nq >> 2); c += blockDim.x) {
-    f32x4 s = slab_sum4(slab + (size_t)t * Nq + c * 4, stride, S);
+  for (int c = threadIdx.x; c < ((h1 - h0) * D >> 2); c += blockDim.x) {
+    f32x4 s = slab_sum4(slab + (size_t)t * Nq + c0 + c * 4, stride, S);
     if (bias) {
-      const bf16x4 b = *reinterpret_cast<const bf16x4*>(bias + c * 4);
+      const bf16x4 b = *reinterpret_cast<const bf16x4*>(bias + c0 + c * 4);
 #pragma unroll
       for (int j = 0; j < 4; ++j) s[j] += bf2f(b[j]);
     }
@@ -680,10 +682,10 @@ __global__ __launch_bounds__(1024) void splitk_rope_cache_write_kernel(
   const int64_t page = slot >= 0 ? slot / 32 : 0;
   const int off = slot >= 0 ? (int)(slot % 32) : 0;
   for (int i = threadIdx.x; i < nrot; i += blockDim.x) {
-    const int head = i / lph, sub = i % lph;
+    const int local = i / lph, head = h0 + local, sub = i % lph;
     // 16-byte LDS / global reads: dword reads at this 32-byte lane stride would be 8-way bank conflicts
-    const f32x4* lo4 = reinterpret_cast<const f32x4*>(rowbuf + head * D + sub * 8);
-    const f32x4* hi4 = reinterpret_cast<const f32x4*>(rowbuf + head * D + sub * 8 + half);
+    const f32x4* lo4 = reinterpret_cast<const f32x4*>(rowbuf + local * D + sub * 8);
+    const f32x4* hi4 = reinterpret_cast<const f32x4*>(rowbuf + local * D + sub * 8 + half);
     // A lane's two 16-byte halves sit 32 bytes from its neighbour's: read in the same order by all lanes, the 16
     // lanes that ds_read_b128 serves together ({0-3, 12-15, 20-27}, ...) would use only every other 16-byte slot of
     // the 256-byte bank row, twice each. Lanes 16-31 and 48-63 take their halves in the opposite order instead.
@@ -746,10 +748,10 @@ __global__ __launch_bounds__(1024) void splitk_rope_cache_write_kernel(
     }
   }
   if (slot >= 0) {
-    const float* vrow = rowbuf + (Hq + Hkv) * D;
-    for (int i = threadIdx.x; i < Hkv * D; i += blockDim.x) {
-      const int vh = i / D, d = i % D;
-      st1_cache(vcache, (((size_t)page * Hkv + vh) * D + d) * 32 + off, vrow[i], fp8);
+    const int v0 = max(h0, Hq + Hkv);
+    for (int i = threadIdx.x; i < (h1 - v0) * D; i += blockDim.x) {
+      const int vh = v0 - Hq - Hkv + i / D, d = i % D;
+      st1_cache(vcache, (((size_t)page * Hkv + vh) * D + d) * 32 + off, rowbuf[(v0 - h0) * D + i], fp8);
     }
   }
 }
@@ -766,9 +768,17 @@ extern "C" int areal_splitk_rope_cache_write(const float* slab, int S, const voi
   if (q_norm && (D / 16 > 64 || ((D / 16) & (D / 16 - 1)) != 0)) return -3;  // lanes of a head: a power of two in one wave
   // one float4 chunk of the summed row per thread where the row allows it: all of a thread's slab loads are in
   // flight at once (a second pass over the row would wait for the first one's loads)
-  const int threads = std::min(1024, std::max(256, (((Hq + 2 * Hkv) * D / 4 + 63) / 64) * 64));
-  hipLaunchKernelGGL(splitk_rope_cache_write_kernel, dim3(T), dim3(threads), lds, st, slab, S, (const bf16_t*)bias, pos,
+  // Heads of 256 columns a block, of 512 for rows of more than 2048: one token's slabs through one CU's load path wait for each
+  // other. us of whole rows / so split, 8 / 24 / 64 / 128 / 320 tokens: 16 heads of 128 in 8 to 2 slabs 3.5 / 3.5 / 3.6 / 3.6 / 5.0
+  // and 2.9 / 2.9 / 3.1 / 3.3 / 4.7; 40 heads with norms, 3 to 1 slabs 4.7 / 4.8 / 5.0 / 5.3 / 8.9 and 3.4 / 3.4 / 4.0 / 4.7 / 7.6;
+  // 48 heads 4.0 / 4.1 / 4.6 / 6.4 / 10.1 and 3.0 / 3.3 / 3.8 / 5.6 / 9.2; 18 heads of 64 3.1 / 3.2 / 3.3 / 3.4 / 4.1 and 2.7 / 2.7 /
+  // 2.8 / 3.0 / 3.8.
+  const int all = Hq + 2 * Hkv;
+  const int heads = std::min(all, std::max(1, (all * D <= 2048 ? 256 : 512) / D));
+  const int threads = std::min(1024, std::max(64, ((heads * D / 4 + 63) / 64) * 64));
+  hipLaunchKernelGGL(splitk_rope_cache_write_kernel, dim3(T, (all + heads - 1) / heads), dim3(threads),
+                     (size_t)heads * D * sizeof(float), st, slab, S, (const bf16_t*)bias, pos,
                      slots, cos_t, sin_t, (bf16_t*)q_out, kcache, vcache, T, Hq, Hkv, D, max_pos,
-                     do_rope, (const bf16_t*)q_norm, (const bf16_t*)k_norm, norm_eps, fp8);
+                     do_rope, (const bf16_t*)q_norm, (const bf16_t*)k_norm, norm_eps, fp8, heads);
   return (int)hipGetLastError();
 }
