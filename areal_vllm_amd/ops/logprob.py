@@ -271,13 +271,12 @@ class _LMHeadLogprobFn(torch.autograd.Function):
         dlogp = dlogp.contiguous().float() if dlogp is not None else None
         dent = dent.contiguous().float() if dent is not None else None
         dh = torch.empty_like(hidden)
-        dw = torch.zeros_like(weight) if ctx.needs_input_grad[1] else None
+        want_dw = ctx.needs_input_grad[1]
         # With an fp32 gradient buffer behind the weight, every chunk's d(logits)^T . hidden is summed straight into it
         # (fp32 across chunks, no [V, H] bf16 temporary, no separate accumulation pass).
-        mg = getattr(weight, "main_grad", None) if dw is not None else None
+        mg = getattr(weight, "main_grad", None) if want_dw else None
         direct = mg is not None and hidden.is_cuda and mg.dtype == torch.float32 and mg.shape == weight.shape
-        if direct:
-            dw = None
+        dw = torch.zeros_like(weight) if want_dw and not direct else None
         whole = kept[0] if keep_logits and T > chunk and kept[0].shape[0] == T else None
         if whole is not None and direct and train_gemm.wgrad_supported(whole, hidden, mg) and train_gemm.dgrad_supported(whole, weight):
             # the fp32 gradient of the head is read and added to once instead of once a chunk (1.9 GB of traffic each for a
