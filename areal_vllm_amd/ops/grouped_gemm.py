@@ -1,9 +1,9 @@
 """Grouped GEMM for expert-sorted tokens (MoE): ``out[t] = x[t] @ W[expert(t)]^T``.
 
-Forward runs the MFMA kernel of ``csrc/hip/grouped_gemm.hip`` (one launch for all experts, tiles never
-straddle experts). The backward pass computes ``dx`` with a sibling kernel that reads the weights untransposed and
-``dW`` of all experts with one launch of the grouped weight-gradient kernel (expert shapes that are no multiples of
-128: per expert with library GEMMs). Counterpart of ``grouped_gemm.ops.gmm`` in the reference
+Forward, ``dx`` (on the untransposed weights) and ``dW`` of all experts are one launch each (tiles never straddle experts): the
+trainer's 256 x 256 tiles (``csrc/hip/train_gemm.hip``) from 128 rows an expert on, the kernels of ``csrc/hip/grouped_gemm.hip``
+below (dW of expert shapes that are no multiples of 128: per expert with library GEMMs). Counterpart of
+``grouped_gemm.ops.gmm`` in the reference
 (``realhf/impl/model/modules/moe/experts.py:195-210``).
 """
 import os
@@ -38,14 +38,20 @@ BIG_MIN_ROWS = 128
 # dW of large experts with few rows is all reading and writing of the gradient, which the small tiles (two workgroups a CU)
 # overlap better: 8 experts, 28672 columns, 4096 deep, 256 / 1024 / 2048 rows 1569 / 3397 / 5774 and 1860 / 3655 / 4938.
 BIG_WGRAD_MAX_SIZE, BIG_WGRAD_ANY_SIZE_ROWS = 1 << 24, 2048
+# A tile of dW is reduced by one workgroup: behind an expert with many times the mean's rows the chip waits for its few large
+# tiles. us of the small / the large ones, largest expert 2.6 / 6 / 13 / 24 / 53 means (forward and dx gain as with even rows):
+# 128 experts, 1024 rows on average, 1536 columns, 2048 deep 1552, 1565, 1549, 1579, 2001 and 1174, 1337, 1605, 1869, 3021; 64
+# experts of 768 rows, 2816 columns, 2.2 / 4.4 / 8.1 / 13.5 / 27 means 1151, 1153, 1158, 1212, 1316 and 893, 1007, 1155, 1389, 1882.
+BIG_WGRAD_CROWDED = 8
 
 
 def _big_tiles(T: int, E: int) -> bool:
     return "AREAL_GROUPED_GEMM_TILE_M" not in os.environ and T >= BIG_MIN_ROWS * E
 
 
-def _big_wgrad(T: int, E: int, N: int, K: int) -> bool:
-    return _big_tiles(T, E) and K % 256 == 0 and (N * K <= BIG_WGRAD_MAX_SIZE or T >= BIG_WGRAD_ANY_SIZE_ROWS * E)
+def _big_wgrad(T: int, E: int, N: int, K: int, largest: int) -> bool:
+    return (_big_tiles(T, E) and K % 256 == 0 and largest * E <= BIG_WGRAD_CROWDED * T
+            and (N * K <= BIG_WGRAD_MAX_SIZE or T >= BIG_WGRAD_ANY_SIZE_ROWS * E))
 
 
 def big_grouped(x: torch.Tensor, w: torch.Tensor, offsets: torch.Tensor, nn: bool) -> torch.Tensor:
@@ -124,7 +130,7 @@ class _GroupedGemmFn(torch.autograd.Function):
                 # carries an fp32 `main_grad` view the kernel adds into it (no bf16 dW, no separate add kernel)
                 mg = _fold_target(w)
                 dst = mg if mg is not None else torch.empty_like(w)
-                if mg is not None and _big_wgrad(x.shape[0], E, N, K):
+                if mg is not None and _big_wgrad(x.shape[0], E, N, K, max(ctx.counts)):
                     L.check(L.lib().areal_tgemm_grouped_wgrad(L.ptr(dy), L.ptr(x), L.ptr(mg), L.ptr(offsets), L.c_int(E),
                                                               L.c_int(N), L.c_int(K), L.c_int64(mg.stride(0)),
                                                               L.stream_ptr()), "tgemm_grouped_wgrad")
@@ -195,10 +201,12 @@ class _LibraryLoopFn(torch.autograd.Function):
         return dx, dw, None
 
 
-# Few, large experts (Mixtral: 8 experts, thousands of rows each): one library GEMM per expert runs at 0.9-1.1 PFLOP/s,
-# the grouped kernel at about half of that; many small experts (Qwen3-MoE: 128 experts, ~1000 rows each): the loop is
-# launch-bound and the grouped kernel is 2-3x faster (tools/grouped_gemm_probe.py). AREAL_GROUPED_GEMM=hip|library
-# overrides the choice.
+# Few, large experts (Mixtral: 8 experts, thousands of rows each): one library GEMM per expert, at 0.9-1.1 PFLOP/s. The grouped
+# kernels are ahead there while the experts' rows are even, and far behind where they are not: a crowded expert's gradient tiles
+# are reduced by one workgroup each. us of the library / grouped, forward and backward, 8 experts, 28672 columns, 4096 deep: 1024 rows
+# each 7350 / 6259, 2048 10588 / 9385, 1284 to 3000 rows 12061 / 11730, 34 to 9000 rows 12316 / 18765. Many small experts
+# (Qwen3-MoE: 128 experts, ~1000 rows each): the loop is launch-bound and the grouped kernel is 2-3x faster
+# (tools/grouped_gemm_probe.py). AREAL_GROUPED_GEMM=hip|library overrides the choice.
 LIBRARY_MAX_EXPERTS = 16
 LIBRARY_MIN_ROWS_PER_EXPERT = 1024
 

@@ -10,7 +10,7 @@ G = sys.modules["areal_vllm_amd.ops.grouped_gemm"]
 DEV = "cuda:0"
 pytestmark = pytest.mark.gpu
 
-COUNTS = [[0, 1, 255, 256, 257, 0, 700, 300], [5000], [0, 0, 130, 127, 900, 129], [200] * 300]
+COUNTS = [[0, 1, 255, 256, 257, 0, 700, 300], [5000], [0, 0, 130, 127, 900, 129], [200] * 300, [3000] + [100] * 23]
 
 
 @pytest.mark.parametrize("counts", COUNTS)
@@ -21,7 +21,7 @@ def test_big_tiles(counts, N, K, monkeypatch):
     E, T = len(counts), sum(counts)
     if E * N * K > 1 << 26:
         pytest.skip("one size of many experts is enough")
-    assert G._big_tiles(T, E)
+    assert G._big_tiles(T, E) and G._big_wgrad(T, E, 256, 256, max(counts)) == (counts[0] != 3000)  # dW of a crowded expert: small tiles
     g = torch.Generator(device=DEV).manual_seed(T + N + K)
     x = torch.randn(T, K, device=DEV, generator=g).bfloat16().requires_grad_(True)
     w = (torch.randn(E, N, K, device=DEV, generator=g) / K ** 0.5).bfloat16().requires_grad_(True)
