@@ -3,7 +3,7 @@
 ``y = x @ W^T (+ b)``. In the backward pass ``dW`` is not materialised in bf16 and added afterwards:
 when the weight carries a ``main_grad`` view (see ``models/transformer.py::FlatParams.alloc_main_grad``)
 the weight-gradient GEMM runs with bf16 operands, fp32 output and beta = 1 directly on that view
-(hipBLASLt through ``torch.addmm(..., out_dtype=float32, out=main_grad)``), so micro-batch gradients are
+(``train_gemm.tgemm_wgrad_``; shapes it does not take: ``torch.addmm(..., out_dtype=float32, out=main_grad)``), so micro-batch gradients are
 summed in fp32 without a rounding step and without a separate add kernel. This is the role of apex's
 ``fused_weight_gradient_mlp_cuda.wgrad_gemm_accum_fp32`` in the reference
 (``realhf/impl/model/parallelism/tensor_parallel/modules.py:242-402``).

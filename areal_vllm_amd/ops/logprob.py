@@ -4,7 +4,7 @@
 ``areal/utils/functional.py:10-80`` (``log_softmax(logits.float() / T)[label]`` and ``-sum p log p``),
 but on GPU one HIP pass per row produces (max, sum exp, sum exp*z, target) so fp32 [T, V] is never
 materialised. ``lm_head_logprobs`` additionally fuses the LM-head GEMM in row chunks: bf16 logits of a
-chunk are produced by hipBLASLt, reduced by the kernel and (for training) kept in bf16 for the backward,
+chunk are produced by a GEMM, reduced by the kernel and (for training) kept in bf16 for the backward,
 whose gradient kernel overwrites them in place with d(logits).
 
 Tensor-parallel vocab shards (reference: ``realhf/impl/model/parallelism/tensor_parallel/modules.py:

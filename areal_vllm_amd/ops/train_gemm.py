@@ -1,9 +1,11 @@
 """Hand-written dense bf16 GEMM for the trainer and for prefill (``csrc/hip/train_gemm.hip``).
 
-``tgemm_tn(a, b)`` = ``a @ b.T`` for K-contiguous operands (activations x ``nn.Linear`` weight, or output gradient
-x transposed weight copy). The kernel covers the shapes transformer layers produce (K a multiple of 128, N of 4,
-16-byte aligned rows); `supported()` tells the caller when to keep the library GEMM instead - it is a statement
-about shapes, not a fallback for a missing extension (on a GPU the extension is mandatory)."""
+``tgemm_tn(a, b)`` = ``a @ b.T`` for K-contiguous operands (activations x ``nn.Linear`` weight), ``tgemm_nn(dy, w)`` =
+``dy @ w`` on the weight as it lies in memory (input gradient), ``tgemm_wgrad_`` adds ``dy.T @ x`` to an fp32 gradient,
+``logit_stats`` reduces a vocabulary's logits without writing them. The kernels cover the shapes transformer layers produce (K a
+multiple of 128, N of 4, 16-byte aligned rows); `supported()` and the rules beside `forward` and `dgrad` tell the caller when to
+keep the library GEMM instead - statements about shapes, not a fallback for a missing extension (on a GPU the extension is
+mandatory)."""
 import functools
 import os
 from typing import Optional, Tuple

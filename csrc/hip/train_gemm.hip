@@ -2,8 +2,8 @@
 //
 //     C[M, N] = A[M, K] . B[N, K]^T (+ bias[N])          bf16 operands, fp32 accumulation, bf16 result
 //
-// Both operands are K-contiguous: A = activations, B = an nn.Linear weight (forward) or its transposed copy
-// (input gradient). Role in the reference: the cuBLAS GEMMs behind torch.nn.functional.linear in
+// Both operands are K-contiguous: A = activations, B = an nn.Linear weight; the NN form (input gradient) takes B [K, N] as the
+// weight lies in memory. Role in the reference: the cuBLAS GEMMs behind torch.nn.functional.linear in
 // realhf/impl/model/parallelism/tensor_parallel/modules.py:242-402 and the HF model code.
 //
 // Structure (one workgroup = one 256 x 256 output tile, 8 waves as 2 (M) x 4 (N), a wave owns 128 x 64):
