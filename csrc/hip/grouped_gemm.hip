@@ -126,7 +126,7 @@ __global__ __launch_bounds__(256) void grouped_gemm_nt_kernel(
 #pragma unroll
     for (int j = 0; j < 16; ++j) acc[t][j] = 0.f;
 
-  const int first = (int)(blockIdx.y * rot) % (K / (64 * KH)) * (64 * KH);  // rot: gg_rot, at the launch
+  const int first = e * rot % (K / (64 * KH)) * (64 * KH);  // rot: gg_rot, at the launch
   load(first);
   for (int k0 = 0; k0 < K; k0 += 64 * KH) {
     __syncthreads();  // previous tile fully consumed
@@ -203,10 +203,11 @@ extern "C" int areal_grouped_gemm_tile_m(int T, int E, int N, int tile_m) {
 // single loads, which are then slower. us from the caches / past them, cold weights: 128 experts, 1536 columns, 2048 deep,
 // 7 rows 18 / 24, 32 31 / 31, 64 59 / 52, 512 164 / 149, 48 an expert 193 / 179, 64 212 / 240, 255 465 / 642; 8 experts,
 // 14336 columns, 4096 deep, 1 row 32 / 48, 2 55 / 55, 4 87 / 77, 64 184 / 167; 16 of 704 columns, 1024 deep, 16 rows 9 / 12.
-// Row tile t starts its reduction at step 13 t (k_rotation, common.hpp) while the weights are read once; with more rows, whose
-// column tiles are reread from the caches, the common order is level or better. us without / with: 128 experts, 1536 columns,
-// 2048 deep, 64 rows 60 / 52, 512 157 / 127, 1600 161 / 129, 4096 169 / 138, but 8192 207 / 213, 16000 337 / 356; 64 experts, 2816
-// columns, 2048 deep, 512 rows 152 / 119; 8 experts, 4096 columns, 14336 deep, 128 rows 199 / 186.
+// Expert e's tiles start their reduction at step 13 e (k_rotation, common.hpp) while the weights are read once: by expert, so that
+// what other rows chose does not change the order of a row's sums. With more rows, whose column tiles are reread from the caches,
+// the common order is level or better. us without / with: 128 experts, 1536 columns, 2048 deep, 64 rows 57 / 53, 512 147 / 124,
+// 1600 162 / 136, 4096 173 / 150, but 8192 207 / 213, 16000 337 / 356; 64 experts, 2816 columns, 2048 deep, 512 rows 159 / 121;
+// 8 experts, 4096 columns, 14336 deep, 128 rows 191 / 186 (by row tile the same within 1 us).
 static int gg_rot(int T, int E, int K) { return T <= 48l * E ? k_rotation(K) : 0; }
 static bool gg_stream(int T, int E, int col_tiles) { return T <= 48l * E && (long)(T < E ? T : E) * col_tiles > 256; }
 

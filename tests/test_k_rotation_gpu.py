@@ -48,3 +48,21 @@ def test_grouped_gemm_takes_every_step_once(T, k, E, F, K):
     ref = torch.einsum("tk,tnk->tn", xs.float().cpu(), w.float().cpu()[topi[order].cpu()])
     assert torch.equal(out.cpu(), ref.bfloat16())
     assert torch.equal(ops.grouped_gate_up(x, src_row, w, offsets[:E + 1]), ops.swiglu(out))
+
+
+@pytest.mark.parametrize("T,k,E,F,K", [(64, 8, 128, 128, 2048), (70, 2, 8, 192, 4096)])
+def test_a_row_has_the_same_bits_whatever_the_others_choose(T, k, E, F, K):
+    torch.manual_seed(T)
+    x = torch.randn(T, K, device="cuda").bfloat16()
+    w = (torch.randn(E, 2 * F, K, device="cuda") * K ** -0.5).bfloat16()
+    topi = torch.rand(T, E, device="cuda").topk(k, -1).indices
+    crowded = topi.clone()
+    crowded[5:] = torch.arange(k, device="cuda")  # several row tiles an expert ahead of the first five rows' experts
+    rows = []
+    for choice in (topi, crowded):
+        order, inv, src_row, offsets = ops.moe_sort(choice.reshape(-1), E, k)
+        first = inv.view(T, k)[:5].reshape(-1)
+        xs = ops.moe_permute(x, order, inv, k, src_row)
+        rows.append((ops.grouped_gemm_offsets(xs, w, offsets[:E + 1])[first], ops.grouped_gate_up(x, src_row, w, offsets[:E + 1])[first]))
+    for a, b in zip(*rows):
+        assert torch.equal(a, b)
