@@ -406,7 +406,8 @@ __global__ __launch_bounds__(512) void tgemm_kernel(const TGArgs a) {
           for (int j = 0; j < 4; ++j) mx = fmaxf(mx, z[nh][nt][j]);
         }
       mx = max_xor16(max_xor32(mx));
-      const float ref = mx * a.scale;  // rounded: the merge takes the difference back
+      // rounded: the merge takes the difference back. A block of nothing but -inf (forbidden ids) adds nothing to the row's sum
+      const float ref = mx > -INFINITY ? mx * a.scale : 0.f;
 #pragma unroll
       for (int nh = 0; nh < 2; ++nh)
 #pragma unroll

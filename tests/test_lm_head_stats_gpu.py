@@ -28,6 +28,26 @@ def test_stats_are_those_of_the_written_logits(M, N, K, first, temperature):
     assert ((out[2] - ref[2]).abs() <= big * 2.0 ** -16).all()
 
 
+def test_a_block_of_forbidden_ids():
+    torch.manual_seed(3)
+    M, N, K = 600, 65536, 128
+    x = torch.randn(M, K, device="cuda").bfloat16()
+    w = (torch.randn(N, K, device="cuda") * K ** -0.5).bfloat16()
+    x[:, 0] = 1.0
+    w[39936:40064, 0] = float("-inf")  # two whole blocks of 64 columns
+    w[50000, 0] = float("-inf")
+    labels = torch.randint(0, 39936, (M,), device="cuda")
+    labels[0] = 40000
+    assert tg.stats_supported(x, w, 1.0)
+    out = torch.empty(4, M, device="cuda")
+    tg.logit_stats(x, w, labels, 1.0, 0, out)
+    ref = torch.stack(lp.logprob_stats(tg.tgemm_tn(x, w), labels))
+    assert torch.equal(out[3], ref[3]) and out[3, 0] == float("-inf")
+    assert torch.equal(out[0], ref[0])
+    assert ((out[1] - ref[1]).abs() <= ref[1] * 2.0 ** -16).all()  # as above
+    assert out[2].isnan().all() and ref[2].isnan().all()  # 0 times -inf, in either form
+
+
 def test_no_grad_head_equals_the_one_with_logits():
     torch.manual_seed(0)
     T, N, K = 1300, 65536, 256
