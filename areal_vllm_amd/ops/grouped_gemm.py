@@ -25,7 +25,7 @@ def grouped_gemm_ref(x: torch.Tensor, w: torch.Tensor, counts: List[int]) -> tor
 
 def _hip_ok(x, w) -> bool:
     return (x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and w.shape[1] % 64 == 0
-            and w.shape[2] % 64 == 0)
+            and w.shape[2] % 64 == 0 and w.shape[2] > 0)
 
 
 # Rows an expert, on average, from which tiles of 256 x 256 (the trainer's dense kernels, operands by LDS-DMA) are the better

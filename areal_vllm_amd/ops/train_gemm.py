@@ -23,7 +23,7 @@ def supported(a: torch.Tensor, b: torch.Tensor, bias: Optional[torch.Tensor] = N
         return False
     M, K = a.shape
     N = b.shape[0]
-    if b.shape[1] != K or K % 128 != 0 or N % 4 != 0 or M == 0:
+    if b.shape[1] != K or K % 128 != 0 or K == 0 or N % 4 != 0 or M == 0:
         return False
     if a.stride(1) != 1 or b.stride(1) != 1 or a.stride(0) % 8 or b.stride(0) % 8:
         return False
@@ -206,7 +206,7 @@ def forward(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None
 def stats_supported(x: torch.Tensor, w: torch.Tensor, temperature: float) -> bool:
     """Whether `logit_stats` is the kernel for these logits: where the products are its own anyway, over a vocabulary."""
     return (0.0 < temperature < float("inf") and x.dim() == 2 and w.dim() == 2 and w.shape[0] >= 65536
-            and _forward_own(x.shape[0], w.shape[1], w.shape[0]) and supported(x, w) and w.shape[1] > 0)
+            and _forward_own(x.shape[0], w.shape[1], w.shape[0]) and supported(x, w))
 
 
 def logit_stats(x: torch.Tensor, w: torch.Tensor, labels: torch.Tensor, temperature: float, vocab_start: int,
@@ -233,7 +233,7 @@ def gated_supported(x: torch.Tensor, w_gate_up: torch.Tensor) -> bool:
             and w_gate_up.dtype == torch.bfloat16):
         return False
     M, K = x.shape
-    if w_gate_up.shape[1] != K or w_gate_up.shape[0] % 2 or K % 128 or (w_gate_up.shape[0] // 2) % 4:
+    if w_gate_up.shape[1] != K or w_gate_up.shape[0] % 2 or K % 128 or K == 0 or (w_gate_up.shape[0] // 2) % 4:
         return False
     if x.stride(1) != 1 or x.stride(0) % 8 or not w_gate_up.is_contiguous():
         return False

@@ -459,7 +459,7 @@ extern "C" int areal_dgemm(const void* X, long xs, const void* W, const void* bi
     act = 1;
     epilogue = DG_SWIGLU;
   }
-  if (K % 64 != 0 || xs % 8 != 0 || N % 32 != 0) return -1;
+  if (K % 64 != 0 || K < 64 || xs % 8 != 0 || N % 32 != 0) return -1;
   if (epilogue == DG_SWIGLU && (N / 2) % 32 != 0) return -2;
   if (ksplit < 1) ksplit = 1;
   if (ksplit > 1 && epilogue != DG_SLAB) return -3;
@@ -499,7 +499,7 @@ extern "C" int areal_dgemm_qkv_rope(const void* X, long xs, const void* W, const
                                     int do_rope, int cfg, int stages, int loader_waves, int nt, hipStream_t st) {
   if (M <= 0) return 0;
   const int N = (Hq + 2 * Hkv) * D;
-  if (K % 64 != 0 || xs % 8 != 0 || D % 64 != 0) return -1;
+  if (K % 64 != 0 || K < 64 || xs % 8 != 0 || D % 64 != 0) return -1;
   if (cfg == 4 && (D / 2) % 64 != 0) return -2;
   DGArgs a;
   a.X = (const bf16_t*)X; a.xs = xs; a.W = (const bf16_t*)W; a.bias = (const bf16_t*)bias; a.Y = nullptr; a.ys = 0;

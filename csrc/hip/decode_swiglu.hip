@@ -238,7 +238,7 @@ int sg_stages(const SGArgs& a, int stages, hipStream_t st) {
 extern "C" int areal_dswiglu(const void* X, long xs, const void* W, void* Y, long ys, int M, int F, int K, int w,
                              int mblocks, int stages, int nt, int act, hipStream_t st) {
   if (M <= 0) return 0;
-  if (K % 64 != 0 || xs % 8 != 0 || F % 4 != 0 || w % 4 != 0 || w < 4 || ys % 4 != 0) return -1;
+  if (K % 64 != 0 || K < 64 || xs % 8 != 0 || F % 4 != 0 || w % 4 != 0 || w < 4 || ys % 4 != 0) return -1;
   if (mblocks < 1 || mblocks > 2) return -2;
   if (((uintptr_t)X | (uintptr_t)W) % 16 != 0 || ((uintptr_t)Y) % 8 != 0) return -3;
   SGArgs a;

@@ -215,7 +215,7 @@ extern "C" int areal_grouped_gemm_nt(const void* x, const void* w, void* out, co
                                      int E, int N, int K, int64_t w_expert_stride, int max_tiles, int tile_m,
                                      hipStream_t st) {
   if (T == 0 || E == 0) return 0;
-  if (N % 64 != 0 || K % 64 != 0) return -1;
+  if (N % 64 != 0 || K % 64 != 0 || K < 64) return -1;
   if (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) % 16 != 0) return -2;
   if (max_tiles < 1) return -3;
   const int tm = areal_grouped_gemm_tile_m(T, E, N, tile_m);
@@ -247,7 +247,7 @@ extern "C" int areal_grouped_gemm_nt(const void* x, const void* w, void* out, co
 extern "C" int areal_grouped_gate_up(const void* x, const int64_t* src_row, const void* w, void* out, const int* offsets, int T,
                                      int E, int N, int K, int64_t w_expert_stride, int max_tiles, hipStream_t st) {
   if (T == 0 || E == 0) return 0;
-  if (N % 128 != 0 || K % 64 != 0) return -1;
+  if (N % 128 != 0 || K % 64 != 0 || K < 64) return -1;
   if (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) % 16 != 0 || w_expert_stride % 8 != 0) return -2;
   if (max_tiles < T / 64 + E || max_tiles > 65535) return -3;
   const dim3 grid(N / 128, max_tiles), block(256);

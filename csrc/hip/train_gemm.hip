@@ -943,7 +943,7 @@ __global__ __launch_bounds__(1024) void tgemm_stats_kernel(const float* __restri
 static int tgemm_tn_launch(const void* A, long lda, const void* B, long ldb, void* C, long ldc, const void* bias, int M,
                            int N, int K, int max_blocks, int gated, float* part, int whole, int splits, hipStream_t st) {
   if (M <= 0 || N <= 0) return 0;
-  if (K % 128 != 0 || N % 4 != 0 || lda % 8 != 0 || ldb % 8 != 0 || ldc % 4 != 0) return -1;
+  if (K % 128 != 0 || K < 128 || N % 4 != 0 || lda % 8 != 0 || ldb % 8 != 0 || ldc % 4 != 0) return -1;
   if (((uintptr_t)A | (uintptr_t)B) % 16 != 0 || (uintptr_t)C % 8 != 0 || (bias && (uintptr_t)bias % 8 != 0)) return -1;
   if (gated && bias) return -1;
   const long tiles = (long)((M + 255) / 256) * (gated ? (N + 127) / 128 : (N + 255) / 256);
@@ -1088,7 +1088,7 @@ extern "C" int areal_tgemm_nn(const void* dY, long ldy, const void* W, long ldw,
 extern "C" int areal_tgemm_grouped(const void* A, const void* B, void* C, const int* offsets, int* table, int T, int E, int N,
                                    int K, long stride, int nn, hipStream_t st) {
   if (T <= 0 || E <= 0) return 0;
-  if (K % 128 != 0 || N <= 0 || N % (nn ? 256 : 8) != 0 || stride % 8 != 0) return -1;
+  if (K % 128 != 0 || K < 128 || N <= 0 || N % (nn ? 256 : 8) != 0 || stride % 8 != 0) return -1;
   if (((uintptr_t)A | (uintptr_t)B | (uintptr_t)C | (uintptr_t)table) % 16 != 0) return -1;
   const int tiles_n = (N + 255) / 256;
   const long most = ((long)T / 256 + E) * tiles_n;  // (an expert's last tile may be partly empty)
