@@ -11,6 +11,7 @@ import os
 from typing import Optional, Tuple
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _lib as L
 
@@ -193,9 +194,19 @@ def _forward_own(M: int, K: int, N: int) -> bool:
     return 256 < M <= 12288 if K >= 16384 else K >= 8192 and 600 <= M <= 2048
 
 
+def plain(*tensors: torch.Tensor) -> bool:
+    """Whether a kernel on raw pointers may stand in for an ATen product of these tensors: nothing rewrites or records the call
+    (vmap and its like, tracing and compilation, dispatch and function modes, autocast), and no operand is a subclass or a dual."""
+    return not (torch._C._are_functorch_transforms_active() or torch._C._len_torch_dispatch_stack()
+                or torch._C._len_torch_function_stack() or torch.jit.is_tracing() or torch.compiler.is_compiling()
+                or torch.is_autocast_enabled(tensors[0].device.type)
+                or any(type(t) not in (torch.Tensor, torch.nn.Parameter) or forward_ad.unpack_dual(t).tangent is not None
+                       for t in tensors))
+
+
 def forward(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """x[M, K] @ w[N, K]^T outside autograd."""
-    if (x.dim() == 2 and w.dim() == 2 and _forward_own(x.shape[0], w.shape[1], w.shape[0]) and supported(x, w)
+    if (x.dim() == 2 and w.dim() == 2 and _forward_own(x.shape[0], w.shape[1], w.shape[0]) and plain(x, w) and supported(x, w)
             and w.shape[0] % 8 == 0 and (out is None or out.dtype == torch.bfloat16 and out.stride(1) == 1
                                          and out.stride(0) % 8 == 0 and out.data_ptr() % 16 == 0)):
         _, whole, splits = _tile_plan(x.shape[1] // 128, -(-x.shape[0] // 256) * -(-w.shape[0] // 256), 0)
