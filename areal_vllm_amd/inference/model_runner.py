@@ -27,7 +27,7 @@ import torch.nn.functional as F
 
 from .. import ops
 from ..models.config import ModelConfig
-from ..models.transformer import Transformer
+from ..models.transformer import MoE, Transformer
 from ..ops.attention import PAGE_SIZE
 from ..utils import logging
 
@@ -670,7 +670,10 @@ class ModelRunner:
             if gate_up_mode == "experts":
                 # router + permutation + grouped GEMMs + weighted combine; the sum joins the residual stream in the
                 # next norm's kernel
-                mixed = blk.mlp(x, None, self.model.ep_group) if tp else blk.mlp.decode_parts(x, self.model.ep_group)
+                if tp or not isinstance(blk.mlp, MoE):
+                    mixed = blk.mlp(x, None, self.model.ep_group)
+                else:
+                    mixed = blk.mlp.decode_parts(x, self.model.ep_group)
                 if tp:
                     self._tp_all_reduce(mixed)
                 if isinstance(mixed, tuple):

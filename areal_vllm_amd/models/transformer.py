@@ -20,6 +20,7 @@ import torch
 import torch.distributed as dist
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.nn.modules.module import _has_any_global_hook
 
 from .. import ops
 from ..parallel import comm
@@ -303,7 +304,11 @@ class MoE(nn.Module):
 
     def decode_parts(self, x, ep_group):
         """The layer of a decode step up to the recombination: (expert outputs in expert order, weights [T, k], inverse of the
-        order) for `ops.moe_combine_rmsnorm`, or the mixed rows themselves where the layer needs another path."""
+        order) for `ops.moe_combine_rmsnorm`, or the mixed rows themselves where the layer needs another path or somebody
+        watches or replaces its call."""
+        if (self._forward_hooks or self._forward_pre_hooks or _has_any_global_hook() or "forward" in self.__dict__
+                or type(self).forward is not MoE.forward):
+            return self(x, None, ep_group)
         return self._route(x, self.router, ep_group, x.shape[0], 1.0, parts=True)
 
     def _route(self, x, router, ep_group, n_valid: int, aux_scale: float, parts: bool = False):

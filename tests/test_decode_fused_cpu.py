@@ -7,7 +7,7 @@ import torch
 
 from areal_vllm_amd.inference.model_runner import ModelRunner
 from areal_vllm_amd.models.config import preset
-from areal_vllm_amd.models.transformer import Transformer
+from areal_vllm_amd.models.transformer import MoE, Transformer
 from areal_vllm_amd.ops import decode_gemm as dg
 from areal_vllm_amd.ops.attention import PAGE_SIZE
 
@@ -62,6 +62,42 @@ def test_fused_decode_matches_plain(B, name):
     for (k0, v0), (k1, v1) in zip(kv0, kv1):
         torch.testing.assert_close(k0, k1, atol=1e-4, rtol=1e-4)
         torch.testing.assert_close(v0, v1, atol=1e-4, rtol=1e-4)
+
+
+@pytest.mark.parametrize("how", ["hook", "pre-hook", "global hook", "patched", "subclass", "module"])
+def test_routed_layers_are_called_where_somebody_watches(how):
+    """The decode step takes a routed layer apart; hooks and replaced layers see whole calls all the same."""
+    torch.manual_seed(0)
+    cfg = preset("tiny-moe")
+    model = Transformer(cfg, dtype=torch.float32, device="cpu").requires_grad_(False).eval()
+    model.flatten()
+    model.init_weights(seed=3)
+    mlp, seen, handle = model.layers[1].mlp, [], None
+
+    def whole(x, tp_group, ep_group=None):
+        seen.append(MoE.forward(mlp, x, tp_group, ep_group))
+        return seen[-1]
+
+    if how == "hook":
+        mlp.register_forward_hook(lambda m, args, out: seen.append(out))
+    elif how == "pre-hook":
+        mlp.register_forward_pre_hook(lambda m, args: seen.append(args[0]))
+    elif how == "global hook":
+        handle = torch.nn.modules.module.register_module_forward_hook(lambda m, args, out: seen.append(out) if m is mlp else None)
+    elif how == "patched":
+        mlp.forward = whole
+    elif how == "subclass":
+        mlp.__class__ = type("Watched", (MoE,), {"forward": lambda self, *a: whole(*a)})
+    else:
+        model.layers[1].mlp = type("Other", (torch.nn.Module,), {"forward": lambda self, *a: whole(*a)})()
+    B, steps, ctx = 9, 2, 40
+    r = ModelRunner(model, 64, 128, B, decode_steps=steps, use_graph=False, buckets=[B], fused_decode=True)
+    try:
+        r.decode(_plan(B, ctx, steps, cfg.vocab_size, seed=7))
+    finally:
+        if handle is not None:
+            handle.remove()
+    assert len(seen) == steps and all(s.shape == (B, cfg.hidden_size) for s in seen)
 
 
 def test_pick_config_is_launchable():
