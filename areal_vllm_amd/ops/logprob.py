@@ -234,22 +234,19 @@ class _LMHeadLogprobFn(torch.autograd.Function):
         need_grad = grad and (hidden.requires_grad or weight.requires_grad)
         kept = []
         whole = None
-        step = chunk * STATS_CHUNKS
-        if (not need_grad and hidden.is_cuda and labels.is_contiguous()
-                and all(train_gemm.stats_supported(hidden[s:s + step], weight, temperature) for s in range(0, T, step))):
-            # no backward pass: the logits are never written
-            for s in range(0, T, step):
-                train_gemm.logit_stats(hidden[s:s + step], weight, labels[s:s + step], temperature, vocab_start,
-                                       stats[:, s:s + step])
-            logp, ent, lse, ez = _finalize(*merge_shard_stats(stats, group))
-            ctx.save_for_backward(hidden, weight, labels, lse, ez)
-            ctx.meta = (temperature, chunk, False, vocab_start, group, reduce_dh)
-            return logp, ent
         if need_grad and keep_logits and T > chunk and weight.dtype == hidden.dtype and weight.shape[0] % 8 == 0:
             # one tensor for all chunks: the backward then works on all rows at once
             whole = torch.empty(T, weight.shape[0], dtype=hidden.dtype, device=hidden.device)
             kept.append(whole)
-        for s in range(0, T, chunk):
+        unwritten = not need_grad and hidden.is_cuda and labels.is_contiguous()
+        s = 0
+        while s < T:
+            e = min(T, s + chunk * STATS_CHUNKS)
+            if unwritten and train_gemm.stats_supported(hidden[s:e], weight, temperature):
+                # no backward pass: these rows' logits are never written (a last few rows' are, too few for that product)
+                train_gemm.logit_stats(hidden[s:e], weight, labels[s:e], temperature, vocab_start, stats[:, s:e])
+                s = e
+                continue
             e = min(T, s + chunk)
             if whole is not None:
                 lg = train_gemm.forward(hidden[s:e], weight, out=whole[s:e])
@@ -258,6 +255,7 @@ class _LMHeadLogprobFn(torch.autograd.Function):
                 if need_grad and keep_logits:
                     kept.append(lg)
             logprob_stats(lg, labels[s:e], temperature, vocab_start, out=stats[:, s:e])
+            s = e
         logp, ent, lse, ez = _finalize(*merge_shard_stats(stats, group))
         ctx.save_for_backward(hidden, weight, labels, lse, ez, *kept)
         ctx.meta = (temperature, chunk, keep_logits, vocab_start, group, reduce_dh)
@@ -314,5 +312,7 @@ def lm_head_logprobs(hidden: torch.Tensor, weight: torch.Tensor, labels: torch.T
     """Fused LM head + log-prob + entropy. hidden [T, H] (bf16), labels int64 [T] (global token ids);
     weight [V, H], or the vocabulary rows [vocab_start, vocab_start + V_local) of a tensor-parallel shard
     whose peers are the ranks of `group`."""
+    if int(chunk) < 1:
+        raise ValueError(f"lm_head_logprobs takes chunks of one row and more, not {chunk}")
     return _LMHeadLogprobFn.apply(hidden, weight, labels.long(), float(temperature), int(chunk), keep_logits,
                                   int(vocab_start), group, bool(reduce_dh), torch.is_grad_enabled())

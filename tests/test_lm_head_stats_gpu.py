@@ -64,3 +64,18 @@ def test_no_grad_head_equals_the_one_with_logits():
     assert glogp.requires_grad and not logp.requires_grad
     # log of a sum that agrees to 2^-16, and differences of numbers up to 30 in fp32
     assert (logp - glogp).abs().max() < 2e-5 and (ent - gent).abs().max() < 4e-5
+
+
+def test_a_last_few_rows_do_not_bring_all_logits_back(monkeypatch):
+    torch.manual_seed(1)
+    T, N, K, chunk = 860, 65536, 256, 100  # 800 rows at once, then 60
+    x = torch.randn(T, K, device="cuda").bfloat16()
+    w = torch.nn.Parameter((torch.randn(N, K, device="cuda") * 4 * K ** -0.5).bfloat16())
+    labels = torch.randint(0, N, (T,), device="cuda")
+    rows, stats = [], tg.logit_stats
+    monkeypatch.setattr(tg, "logit_stats", lambda h, *a: (rows.append(h.shape[0]), stats(h, *a)))
+    with torch.no_grad():
+        logp, ent = ops.lm_head_logprobs(x, w, labels, chunk=chunk)
+    assert rows == [800]
+    glogp, gent = ops.lm_head_logprobs(x, w, labels, chunk=chunk)
+    assert (logp - glogp).abs().max() < 2e-5 and (ent - gent).abs().max() < 4e-5  # as above

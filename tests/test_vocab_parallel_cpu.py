@@ -148,3 +148,14 @@ def test_critic_under_tensor_parallel_shards_embedding_but_not_value_head():
     assert not torch.equal(moved["model.embed_tokens.weight"], a["model.embed_tokens.weight"])  # the step did train
     for k in a:
         torch.testing.assert_close(b[k], a[k], atol=2e-5, rtol=1e-4, msg=lambda m: f"{k}: {m}")
+
+
+@pytest.mark.parametrize("grad", [False, True])
+def test_chunks_of_no_rows_are_refused(grad):
+    from areal_vllm_amd import ops
+
+    h, w = torch.randn(5, 8), torch.randn(16, 8, requires_grad=grad)
+    with pytest.raises(ValueError):
+        ops.lm_head_logprobs(h, w, torch.zeros(5, dtype=torch.long), chunk=0)
+    logp, _ = ops.lm_head_logprobs(h, w, torch.zeros(5, dtype=torch.long), chunk=2)
+    torch.testing.assert_close(logp, torch.log_softmax(h @ w.t(), -1)[:, 0], atol=1e-5, rtol=1e-5)
