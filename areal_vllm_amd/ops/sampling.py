@@ -15,8 +15,13 @@ from . import _lib as L
 # unfiltered batches (no top-k / top-p) split every row over several workgroups; 0 keeps the one-workgroup-per-row
 # kernel for A/B timing
 SPLIT_UNFILTERED = os.environ.get("AREAL_SAMPLE_SPLIT", "1") != "0"
-# rows up to which the rows of a filtered batch are split over several workgroups (16 to 2 each, 512 in all)
+# Rows up to which the rows of a filtered batch are split over several workgroups. A CU holds two of them: 512 make a round, and
+# 3 a row from 257 rows on fill two better than 2 would. More than 8, or slices below 8192 entries, cost more than they bring: top-k
+# 50 with top-p 0.95, us with 0 / 1 / 2 / 3 / 4 / 8 / 16 a row: 151936 bf16 entries, 16 rows 85 / 64 / 44 / 37 / 34 / 32 / 35, 128 rows
+# 106 / 76 / 51 / 46 / 42 / 49 / 66, 200 rows 108 / 78 / 57 / 64 / 61 / 71 / 89, 320 rows 192 / 101 / 95 / 87 / 91 / 106 / 144; 32000 of
+# them, 16 rows 35 / 31 / 27 / 26 / 25 / 27 / 32, 200 rows 36 / 31 / 29 / 35 / 36 / 46 / 69.
 SPLIT_FILTERED_MAX_ROWS = 384
+SLICE_MIN_ENTRIES = 8192
 SLICE_WORDS = 516  # of workspace for a row's slice (csrc/hip/sampling.hip)
 
 
@@ -76,6 +81,14 @@ def sample_ref(logits, temperature, top_k, top_p, generator=None, active=None, c
     return toks, lps
 
 
+def _slices(B: int, V: int) -> int:
+    """Workgroups for each of B filtered rows of V entries besides the one that owns it; 0: that one alone."""
+    most = V // SLICE_MIN_ENTRIES
+    if most < 2:
+        return 0
+    return min(8, most, 512 // B if B <= 256 else 3 if B <= 341 else 1)
+
+
 def sample(logits: torch.Tensor, temperature: Optional[torch.Tensor], top_k: Optional[torch.Tensor],
            top_p: Optional[torch.Tensor], seed: int, step: Optional[torch.Tensor] = None, bump_step: bool = True,
            out_tokens: Optional[torch.Tensor] = None, out_logprobs: Optional[torch.Tensor] = None,
@@ -122,8 +135,7 @@ def sample(logits: torch.Tensor, temperature: Optional[torch.Tensor], top_k: Opt
         return out_tokens, out_logprobs
     lib = L.lib()
     ws, S = None, 0
-    if 0 < B <= SPLIT_FILTERED_MAX_ROWS:
-        S = min(16, -(-512 // B))
+    if 0 < B <= SPLIT_FILTERED_MAX_ROWS and (S := _slices(B, V)):
         ws = torch.empty(B * S * SLICE_WORDS + 2, dtype=torch.float32, device=logits.device)
     L.check(
         lib.areal_sample(L.ptr(logits), L.c_int(L.dtype_flag(logits)), L.c_int(B), L.c_int(V),

@@ -314,13 +314,18 @@ DEVINL float select_threshold(Select& S, E row, float floor, float mn, float mx,
 // With a small top-k what the workgroup that owns the row then still needs of its 152k entries are those that can be among the
 // k largest, so every slice also hands on a superset of its own k largest entries (the bins of its histogram from the k-th
 // largest's on): seven passes of one workgroup over the row become two of S workgroups over a slice and work on a few
-// hundred entries. us of one part and of two, 151936 bf16 entries: top-k 50 with top-p 0.95, one dominant token, 1 / 24 / 64 /
-// 320 rows 96 / 97 / 98 / 215 and 39 / 42 / 41 / 104; top-p 0.95 alone, which only gains the first pass, 49 / 50 / 50 / 110 and
-// 43 / 45 / 49 / 112.
+// hundred entries. us of one part and of two, top-k 50 with top-p 0.95, 1 / 64 / 200 / 320 rows: 151936 bf16 entries 83 / 86 / 108 /
+// 191 and 31 / 35 / 57 / 87, 32000 of them 33 / 35 / 35 / 66 and 25 / 26 / 29 / 52; 50257, whose rows start off the 16-byte grid and
+// are walked entry by entry, 42 / 78 / 79 / 161 and 27 / 32 / 54 / 81.
 // ws: [B][S][SLICE_WORDS] words: {max, sum of exp(z - max), number of entries (-1: none or too many, the row's own passes find
 // the set), min}, entries, their places; behind them the step (the second part's first workgroup counts it on, so the others
 // read it here).
 constexpr int TOPK_MAX = 128, TOPK_CAP = 256, SLICE_WORDS = 4 + 2 * TOPK_CAP, SLICES = SEL_CAP / TOPK_CAP, SLICE_THREADS = 512;
+
+// Whether the row's slices do anything: with a small top-k, or where there are enough of them to shorten the first pass. us of
+// one part and of two, top-p 0.95 alone, 8 / 4 / 2 slices (64 / 128 / 256 rows): 151936 bf16 entries 127 / 138 / 140 and 124 / 132 /
+// 140, 65536 fp32 69 / 70 / 84 and 69 / 74 / 86, 32000 fp32 41 / 42 / 44 and 43 / 43 / 50.
+DEVINL bool row_sliced(int k, int V, int S) { return (k >= 1 && k < V && k <= TOPK_MAX) || S >= 8; }
 
 template <typename T>
 __global__ __launch_bounds__(SLICE_THREADS) void sample_slice_kernel(
@@ -339,7 +344,7 @@ __global__ __launch_bounds__(SLICE_THREADS) void sample_slice_kernel(
   const float temp = temperature ? temperature[row] : 1.f;
   const int k = top_k ? top_k[row] : V;
   const bool limited = k >= 1 && k < V;
-  if (temp <= 0.f || !(limited || (top_p && top_p[row] < 1.f))) return;
+  if (temp <= 0.f || !(limited || (top_p && top_p[row] < 1.f)) || !row_sliced(k, V, S)) return;
   const T* p = logits + (size_t)row * ld;
   const int V8 = (reinterpret_cast<uintptr_t>(p) & 15) == 0 ? (V & ~7) : 0;
   const int slot = (counts && count_slot) ? count_slot[row] : -1;
@@ -367,8 +372,7 @@ __global__ __launch_bounds__(SLICE_THREADS) void sample_slice_kernel(
         f8(i8, zz[u]);
       }
     }
-    if (s == S - 1)
-      for (int i = V8 + tid; i < V; i += NT) f1(i, R.z1(i));
+    for (int i = V8 + s * NT + tid; i < V; i += S * NT) f1(i, R.z1(i));
   };
   auto each = [&](auto f) __attribute__((always_inline)) {
     walk([&](int i8, const float* z) {
@@ -557,7 +561,7 @@ __global__ __launch_bounds__(1024) void sample_kernel(
   R.inv_t = inv_t;
 
   float mx = -INFINITY, mn = INFINITY, se = 0.f;
-  const bool sliced = ws && filtered;
+  const bool sliced = ws && filtered && row_sliced(k, V, S);
   bool listed = sliced;  // the slices have handed on all that can be drawn
   if (sliced) {
     const float* o = ws + (size_t)row * S * SLICE_WORDS;
@@ -920,7 +924,6 @@ extern "C" int areal_sample_splits(int B) {
   const int s = (1024 + B - 1) / B;
   return s > 16 ? 16 : s;
 }
-
 
 
 extern "C" int areal_sample_unfiltered(const void* logits, int dtype, int B, int V, int64_t ld,

@@ -41,6 +41,7 @@ def test_same_as_one_workgroup(V, B, k, p, monkeypatch):
     slot[: min(B, 3)] = torch.arange(min(B, 3), dtype=torch.int32, device=DEV)
     pen = torch.full((B,), 0.7, device=DEV)
     got = []
+    monkeypatch.setattr(S, "_slices", lambda B, V: min(16, -(-512 // B)))
     for most in (0, 384):
         monkeypatch.setattr(S, "SPLIT_FILTERED_MAX_ROWS", most)
         counts = ops.TokenCounts(3, V, torch.device(DEV))
@@ -52,3 +53,18 @@ def test_same_as_one_workgroup(V, B, k, p, monkeypatch):
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][2], got[1][2])
     # sums of V fp32 exponentials in another order
     assert torch.allclose(got[0][1], got[1][1], atol=1e-4, rtol=1e-5)
+
+
+# the rule's own counts; rows of an odd length start off the 16-byte grid and are walked entry by entry, by all slices
+@pytest.mark.parametrize("B,V,n", [(3, 50257, 6), (70, 50257, 6), (200, 50257, 2), (300, 50257, 3), (350, 50257, 1), (64, 65536, 8)])
+@pytest.mark.parametrize("k,p", [(50, 0.95), (1 << 30, 0.9), (200, 1.0)])
+def test_the_rule(B, V, n, k, p, monkeypatch):
+    assert S._slices(B, V) == n
+    torch.manual_seed(B)
+    logits = 3 * torch.randn(B, V, device=DEV)
+    t, kk, pp = torch.ones(B, device=DEV), torch.full((B,), k, dtype=torch.int32, device=DEV), torch.full((B,), p, device=DEV)
+    got = [ops.sample(logits, t, kk, pp, 5, torch.zeros(1, dtype=torch.int64, device=DEV))]
+    monkeypatch.setattr(S, "SPLIT_FILTERED_MAX_ROWS", 0)
+    got.append(ops.sample(logits, t, kk, pp, 5, torch.zeros(1, dtype=torch.int64, device=DEV)))
+    assert torch.equal(got[0][0], got[1][0])
+    assert torch.allclose(got[0][1], got[1][1], atol=1e-4, rtol=1e-5)  # as above
