@@ -6,6 +6,7 @@ below (dW of expert shapes that are no multiples of 128: per expert with library
 ``grouped_gemm.ops.gmm`` in the reference
 (``realhf/impl/model/modules/moe/experts.py:195-210``).
 """
+import math
 import os
 from typing import List
 
@@ -34,10 +35,16 @@ def _hip_ok(x, w) -> bool:
 # 512 669 / 633 / 1037 and 425 / 494 / 862, 1024 1131 / 1123 / 1595 and 729 / 800 / 1163; 2048 columns, 768 deep: 64 99 / 128 /
 # 311 and 114 / 111 / 330, 128 134 / 201 / 322 and 134 / 119 / 307, 1024 628 / 746 / 846 and 430 / 389 / 599; 32 experts, 1024 by
 # 1024: 64 21 / 22 / 46 and 28 / 29 / 47, 128 28 / 29 / 52 and 29 / 30 / 50.
-BIG_MIN_ROWS = 128
-# dW of large experts with few rows is all reading and writing of the gradient, which the small tiles (two workgroups a CU)
-# overlap better: 8 experts, 28672 columns, 4096 deep, 256 / 1024 / 2048 rows 1569 / 3397 / 5774 and 1860 / 3655 / 4938.
-BIG_WGRAD_MAX_SIZE, BIG_WGRAD_ANY_SIZE_ROWS = 1 << 24, 2048
+# They come one a CU: below 54 % of the chip's rounds filled the small ones, of which a CU holds several, are ahead. us small / these,
+# out: 4 experts of 400 rows, 2048 columns, 768 deep (33 tiles) 14 / 22; 8 of 128, 4096 columns, 1408 deep (64) 34 / 36; 16 of 400,
+# 2048 columns, 768 deep (132 and 264 in all) 21 / 25 and 40 / 44; 16 of 200, 1536 columns (123) 24 / 25; 16 of 400, 2816 columns, 512
+# deep (363) 46 / 35.
+BIG_MIN_ROWS, BIG_MIN_FILL = 128, 0.54
+# dW of experts with few rows is all reading and writing of the gradient, which the small tiles (two workgroups a CU) overlap
+# better, large experts' up to many rows. us of the small ones / of these: 16 experts, 1536 columns, 768 deep, 128 / 200 / 400 / 800 rows
+# 40, 43, 53, 79 / 50, 53, 60, 75 (288 tiles); 128 of them 250, 278, 366, 557 / 260, 280, 310, 399; 8 experts, 28672 columns, 4096
+# deep, 256 / 1024 / 2048 rows 1569 / 3397 / 5774 and 1860 / 3655 / 4938.
+BIG_WGRAD_MIN_ROWS, BIG_WGRAD_MAX_SIZE, BIG_WGRAD_ANY_SIZE_ROWS = 384, 1 << 24, 2048
 # A tile of dW is reduced by one workgroup: behind an expert with many times the mean's rows the chip waits for its few large
 # tiles. us of the small / the large ones, largest expert 2.6 / 6 / 13 / 24 / 53 means (forward and dx gain as with even rows):
 # 128 experts, 1024 rows on average, 1536 columns, 2048 deep 1552, 1565, 1549, 1579, 2001 and 1174, 1337, 1605, 1869, 3021; 64
@@ -45,13 +52,20 @@ BIG_WGRAD_MAX_SIZE, BIG_WGRAD_ANY_SIZE_ROWS = 1 << 24, 2048
 BIG_WGRAD_CROWDED = 8
 
 
-def _big_tiles(T: int, E: int) -> bool:
-    return "AREAL_GROUPED_GEMM_TILE_M" not in os.environ and T >= BIG_MIN_ROWS * E
+def _rounds_filled(tiles: float) -> bool:
+    return tiles >= BIG_MIN_FILL * 256 * math.ceil(tiles / 256)
 
 
-def _big_wgrad(T: int, E: int, N: int, K: int, largest: int) -> bool:
-    return (_big_tiles(T, E) and K % 256 == 0 and largest * E <= BIG_WGRAD_CROWDED * T
-            and (N * K <= BIG_WGRAD_MAX_SIZE or T >= BIG_WGRAD_ANY_SIZE_ROWS * E))
+def _big_tiles(T: int, E: int, N: int) -> bool:
+    """Tiles of 256 x 256 for T rows of E experts and N result columns (half a row tile an expert is empty on average)."""
+    return (T >= BIG_MIN_ROWS * E and _rounds_filled((T / 256 + E / 2) * -(-N // 256))
+            and "AREAL_GROUPED_GEMM_TILE_M" not in os.environ)
+
+
+def _big_wgrad(T: int, E: int, N: int, K: int, counts: List[int]) -> bool:
+    return (T >= BIG_WGRAD_MIN_ROWS * E and K % 256 == 0 and (N * K <= BIG_WGRAD_MAX_SIZE or T >= BIG_WGRAD_ANY_SIZE_ROWS * E)
+            and _rounds_filled(E * -(-N // 256) * (K // 256)) and max(counts) * E <= BIG_WGRAD_CROWDED * T
+            and "AREAL_GROUPED_GEMM_TILE_M" not in os.environ)
 
 
 def big_grouped(x: torch.Tensor, w: torch.Tensor, offsets: torch.Tensor, nn: bool) -> torch.Tensor:
@@ -71,7 +85,7 @@ def _launch(x: torch.Tensor, w: torch.Tensor, offsets: torch.Tensor) -> torch.Te
     E, N, K2 = w.shape
     assert K == K2 and offsets.numel() == E + 1 and offsets.dtype == torch.int32 and offsets.is_cuda
     assert x.is_contiguous() and w.stride(2) == 1 and w.stride(1) == K, "operands must be K-contiguous"
-    if K % 128 == 0 and w.stride(0) % 8 == 0 and _big_tiles(T, E):
+    if K % 128 == 0 and w.stride(0) % 8 == 0 and _big_tiles(T, E, N):
         return big_grouped(x, w, offsets, False)
     out = torch.empty(T, N, dtype=x.dtype, device=x.device)
     tile_m = int(os.environ.get("AREAL_GROUPED_GEMM_TILE_M", "0"))  # 0: chosen from the rows per expert
@@ -110,7 +124,7 @@ class _GroupedGemmFn(torch.autograd.Function):
         dx = dw = None
         E, N, K = w.shape
         if ctx.needs_input_grad[0]:
-            if N % 128 == 0 and K % 256 == 0 and _big_tiles(dy.shape[0], E) and w.is_contiguous():
+            if N % 128 == 0 and K % 256 == 0 and _big_tiles(dy.shape[0], E, K) and w.is_contiguous():
                 dx = big_grouped(dy, w, offsets, True)
             elif K % 128 == 0:
                 # dx[t] = dy[t] @ W[e]: the weights are read as they are (transposed LDS reads in the kernel)
@@ -130,7 +144,7 @@ class _GroupedGemmFn(torch.autograd.Function):
                 # carries an fp32 `main_grad` view the kernel adds into it (no bf16 dW, no separate add kernel)
                 mg = _fold_target(w)
                 dst = mg if mg is not None else torch.empty_like(w)
-                if mg is not None and _big_wgrad(x.shape[0], E, N, K, max(ctx.counts)):
+                if mg is not None and _big_wgrad(x.shape[0], E, N, K, ctx.counts):
                     L.check(L.lib().areal_tgemm_grouped_wgrad(L.ptr(dy), L.ptr(x), L.ptr(mg), L.ptr(offsets), L.c_int(E),
                                                               L.c_int(N), L.c_int(K), L.c_int64(mg.stride(0)),
                                                               L.stream_ptr()), "tgemm_grouped_wgrad")
@@ -234,7 +248,7 @@ def grouped_gemm_offsets(x: torch.Tensor, w: torch.Tensor, offsets: torch.Tensor
 def gate_up_rows_ok(n_pairs: int, w: torch.Tensor) -> bool:
     """Whether `grouped_gate_up` is the kernel for so many rows: its tiles are the small ones, and a column tile holds 64
     gate and 64 up columns."""
-    return (n_pairs > 0 and not _big_tiles(n_pairs, w.shape[0]) and "AREAL_GROUPED_GEMM_TILE_M" not in os.environ
+    return (0 < n_pairs < BIG_MIN_ROWS * w.shape[0] and "AREAL_GROUPED_GEMM_TILE_M" not in os.environ
             and w.shape[1] % 128 == 0 and w.stride(0) % 8 == 0 and n_pairs // 64 + w.shape[0] <= 65535)
 
 

