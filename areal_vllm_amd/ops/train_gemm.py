@@ -183,15 +183,33 @@ def dgrad(dy: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None)
     return torch.mm(dy, w) if out is None else torch.mm(dy, w, out=out)
 
 
-# Where the own kernel is ahead of the library in y = x W^T, own / library us. Deep reductions, whose tiles it splits: 18944 deep
-# to 3584 columns, 300 / 700 / 3000 / 6000 / 12000 / 24576 rows 68 / 98, 92 / 169, 325 / 550, 564 / 1048, 1142 / 1548, 2298 /
-# 2279; 8960 to 1536, 300 / 513 / 700 / 1500 / 3000 / 6000 rows 34 / 31, 39 / 34, 40 / 45, 53 / 61, 82 / 83, 148 / 142. Wide
-# results, which it stores by whole lines: 1536 deep to 151936 columns, 300 / 700 / 1500 / 3000 / 8192 rows 192 / 187, 285 /
-# 354, 578 / 639, 1154 / 1171, 2890 / 2984. Elsewhere the two are level, or the library has the smaller tiles.
+# Where the own kernel is ahead of the library in y = x W^T, own / library us (the library's choices jump: of 70 depths and widths
+# those below are where the own one is ahead or level but for single sizes, of which the worst is 8 % behind).
+# Deep reductions of up to 128 tiles, which it splits: 8960 deep to 1536 columns, 800 / 1500 / 2048 rows 40 / 46, 52 / 69, 61 / 70;
+# 11008 to 4096, 1100 rows 99 / 121; 18944 to 3584, 257 / 800 rows 66 / 93, 120 / 164. A few tiles of 9 to 16 thousand deep are the
+# library's (8960 to 512, 800 rows 29 / 25), so are 8192 deep ones (1536 columns, 800 rows 38 / 35) and 96 and more tiles of 8192
+# columns (11008 deep, 600 rows 134 / 126). More tiles: rounds that are not full, from 16384 deep on: 18944 to 4096, 4500 rows (288
+# tiles) 0.49 of the library's time, to 5120, 9000 rows (720) 0.76; but to 3584, 9000 rows (504) 867 / 822, and one round of more
+# than 128 (160 to 256 tiles) 4 to 19 % slower.
+# Wide results, stored by whole lines: 1536 deep to 151936 columns, 300 / 700 / 1500 / 3000 / 8192 rows 192 / 187, 285 / 354, 578 /
+# 639, 1154 / 1171, 2890 / 2984; 128256 columns, 896 / 5120 deep, 1642 rows 0.91 / 0.94 of the library's time, but 3584 and 4096 deep
+# 2500 to 8192 rows 1.01 to 1.06 of it, and 65536 columns from 2500 rows on 1.02 to 1.13.
 def _forward_own(M: int, K: int, N: int) -> bool:
-    if N >= 65536:
-        return M >= 600
-    return 256 < M <= 12288 if K >= 16384 else K >= 8192 and 600 <= M <= 2048
+    if N >= 98304:
+        return M >= 600 and (K <= 3072 or K >= 4608)
+    if K < 8704 or not 256 < M <= 12288 or N >= 65536:
+        return False
+    tiles = -(-M // 256) * -(-N // 256)
+    if tiles <= 128:
+        return K >= 16384 or 600 <= M <= 2048 and N <= 6144 and tiles * K >= 150000
+    return K >= 16384 and 256 < tiles <= 0.95 * 256 * -(-tiles // 256)
+
+
+# Logits that are reduced, not written, us of that form / of the library's product and the pass over its logits: 151936 columns, 896
+# to 5120 deep, 600 to 8192 rows 0.75 to 1.02 of its time, 65536 columns, 896 / 2048 deep 0.87 to 0.98 / 0.95 to 1.04; 3584 and 4096
+# deep 1.00 to 1.12, with 100352 columns 0.90 to 1.08.
+def _stats_own(M: int, K: int, N: int) -> bool:
+    return N >= 65536 and M >= 600 and (N >= 98304 or K <= 3072)
 
 
 def plain(*tensors: torch.Tensor) -> bool:
@@ -215,9 +233,9 @@ def forward(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None
 
 
 def stats_supported(x: torch.Tensor, w: torch.Tensor, temperature: float) -> bool:
-    """Whether `logit_stats` is the kernel for these logits: where the products are its own anyway, over a vocabulary."""
-    return (0.0 < temperature < float("inf") and x.dim() == 2 and w.dim() == 2 and w.shape[0] >= 65536
-            and _forward_own(x.shape[0], w.shape[1], w.shape[0]) and supported(x, w))
+    """Whether `logit_stats` is the kernel for these logits."""
+    return (0.0 < temperature < float("inf") and x.dim() == 2 and w.dim() == 2
+            and _stats_own(x.shape[0], w.shape[1], w.shape[0]) and supported(x, w))
 
 
 def logit_stats(x: torch.Tensor, w: torch.Tensor, labels: torch.Tensor, temperature: float, vocab_start: int,

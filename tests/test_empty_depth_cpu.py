@@ -18,8 +18,8 @@ def _operand(*shape):
 
 @pytest.mark.parametrize("K", [128, 0])
 def test_rules(K):
-    x, w = _operand(700, K), _operand(65536, K)
-    assert tg._forward_own(700, K, 65536)
+    x, w = _operand(700, K), _operand(98304, K)
+    assert tg._forward_own(700, K, 98304)
     assert tg.supported(x, w) == tg.stats_supported(x, w, 1.0) == tg.gated_supported(x, w) == (K > 0)
     assert _hip_ok(x, _operand(8, 128, K)) == dg.serves(_operand(64, K), _operand(128, K)) == (K > 0)
 

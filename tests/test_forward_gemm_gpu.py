@@ -25,9 +25,17 @@ def test_parts(M, K, N, plan):
     assert bool((out[:, N:] == 7.0).all())
 
 
-def test_rule():
-    for M, K, N, own in ((700, 8960, 1536, True), (700, 1536, 17920, False), (8192, 1536, 151936, True), (300, 1536, 151936, False),
-                         (6000, 18944, 3584, True), (20000, 18944, 3584, False)):
-        assert tg._forward_own(M, K, N) == own
-        x, w = torch.zeros(M, K, device=DEV).bfloat16(), torch.zeros(N, K, device=DEV).bfloat16()
-        assert tg.forward(x, w).shape == (M, N)
+@pytest.mark.parametrize("M,K,N,own", [(700, 8960, 1536, True), (700, 1536, 17920, False), (8192, 1536, 151936, True),
+                                       (300, 1536, 151936, False), (6000, 18944, 3584, True), (20000, 18944, 3584, False),
+                                       (1999, 11008, 4096, True), (701, 16384, 64, True), (601, 128, 98304 + 8, True)])
+def test_rule(M, K, N, own):
+    assert tg._forward_own(M, K, N) == own
+    g = torch.Generator(device=DEV).manual_seed(M + K)
+    x = torch.randn(M, K, device=DEV, generator=g).bfloat16()
+    w = (torch.randn(N, K, device=DEV, generator=g) / K ** 0.5).bfloat16()
+    got = tg.forward(x, w)
+    assert got.shape == (M, N)
+    rows = torch.cat([torch.arange(0, M, max(1, M // 500), device=DEV), torch.arange(max(0, M - 300), M, device=DEV)])
+    for at in range(0, N, 16384):  # (float64: some rows of every tile, and all of the ragged last one)
+        want = x[rows].double() @ w[at:at + 16384].double().t()
+        assert bool(((got[rows, at:at + 16384].double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4).all())  # as above
