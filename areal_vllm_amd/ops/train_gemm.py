@@ -184,7 +184,7 @@ def dgrad(dy: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None)
 
 
 # Where the own kernel is ahead of the library in y = x W^T, own / library us (the library's choices jump: of 70 depths and widths
-# those below are where the own one is ahead or level but for single sizes, of which the worst is 8 % behind).
+# those below are where the own one is ahead or level: 0.69 of its time in the mean of 273 sizes, 12 of them 3 to 16 % behind).
 # Deep reductions of up to 128 tiles, which it splits: 8960 deep to 1536 columns, 800 / 1500 / 2048 rows 40 / 46, 52 / 69, 61 / 70;
 # 11008 to 4096, 1100 rows 99 / 121; 18944 to 3584, 257 / 800 rows 66 / 93, 120 / 164. A few tiles of 9 to 16 thousand deep are the
 # library's (8960 to 512, 800 rows 29 / 25), so are 8192 deep ones (1536 columns, 800 rows 38 / 35) and 96 and more tiles of 8192
