@@ -36,6 +36,9 @@ DEVINL bf16_t f2bf(float x) { return (bf16_t)x; }
 // 28672 columns, 8 rows, 4096 51 / 38, 8192 106 / 69; 65536 columns, 64 rows, 8192 238 / 161. Between: 1024 50 / 52, 2560 123 /
 // 124, 3072 135 / 136, 3584 148 / 148, 5120 220 / 220 (100352 columns, 64 rows).
 static inline int k_rotation(int K) { return K % 2048 == 0 ? 13 : 0; }
+// First step of workgroup t. The remainder is vector arithmetic: back to a scalar register, or every address of the loop that
+// follows becomes a vector's.
+DEVINL int k_start(int t, int rot, int nsteps) { return rot == 0 ? 0 : __builtin_amdgcn_readfirstlane(t * rot % nsteps); }
 
 // Exchanges across 16- and 32-lane rows in the VALU (v_permlane16_swap / v_permlane32_swap of gfx950) instead of
 // through the LDS crossbar (`__shfl_xor(v, 16 | 32)` compiles to ds_bpermute_b32: an LDS-pipe round trip of ~100

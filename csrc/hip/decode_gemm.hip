@@ -40,7 +40,6 @@ struct DGArgs {
   void* Y;
   long ys;
   int M, N, K, k_per_split;
-  int rot;  // column tile t starts its reduction at step t * rot (modulo the steps) and wraps round: k_rotation (common.hpp)
   int nt;  // non-temporal weight loads (each weight byte is read once per launch)
   int act;  // gate activation of the gated-MLP epilogue (gate_act_f)
   unsigned inv_y = 0, inv_z = 0;  // ceil(2^32 / column tiles), ceil(2^32 / row blocks); 0: workgroups in launch order
@@ -54,6 +53,7 @@ struct DGArgs {
   bf16_t* kcache;
   bf16_t* vcache;
   int Hq, Hkv, D, max_pos, do_rope;
+  int rot = 0;  // column tile t starts its reduction at step t * rot (modulo the steps) and wraps round: k_rotation (common.hpp)
 };
 
 template <int N>
@@ -89,7 +89,7 @@ DEVINL float gate_act_f(float x, int act) {
 // LW = 0: every wave stages its share of each tile and computes. LW > 0: LW extra waves do nothing but issue the
 // LDS-DMA pieces (a piece costs a dedicated wave ~25 issue cycles, but 100-185 in a wave that is also issuing
 // ds_reads and MFMAs), the WM x WN waves only compute; both kinds meet at the one barrier per K step.
-template <int TM, int TN, int WM, int WN, int STAGES, int EPI, int LW>
+template <int TM, int TN, int WM, int WN, int STAGES, int EPI, int LW, bool ROT>
 __global__ __launch_bounds__(64 * (WM * WN + LW)) void dgemm_kernel(const DGArgs a) {
   constexpr int NW = WM * WN, BM = 32 * TM * WM, BN = 32 * TN * WN;
   constexpr int NLOAD = LW > 0 ? LW : NW;  // waves that stage
@@ -158,10 +158,12 @@ __global__ __launch_bounds__(64 * (WM * WN + LW)) void dgemm_kernel(const DGArgs
       src[j] = a.X + (size_t)m * a.xs + k_begin + 8 * c;
     }
   }
-  const int rot = (ct * a.rot) % nsteps;
+  const int rot = ROT ? k_start(ct, a.rot, nsteps) : 0;
   auto issue = [&](int buf, int step) {
-    step += rot;
-    step -= step >= nsteps ? nsteps : 0;
+    if (ROT) {
+      step += rot;
+      step -= step >= nsteps ? nsteps : 0;
+    }
     char* base = smem + buf * STAGE_BYTES + lwave * (IPW * 1024);
 #pragma unroll
     for (int j = 0; j < IPW; ++j) {
@@ -357,13 +359,13 @@ __global__ __launch_bounds__(64 * (WM * WN + LW)) void dgemm_kernel(const DGArgs
   }
 }
 
-template <int TM, int TN, int WM, int WN, int STAGES, int EPI, int LW>
-int launch_cfg(const DGArgs& a, int ksplit, hipStream_t st) {
+template <int TM, int TN, int WM, int WN, int STAGES, int EPI, int LW, bool ROT>
+int launch_as(const DGArgs& a, int ksplit, hipStream_t st) {
   constexpr int BM = 32 * TM * WM, BN = 32 * TN * WN;
   constexpr size_t lds = (size_t)STAGES * (BM + BN) * 128;
   if (lds > 160 * 1024) return -20;
   if (LW > 0 && ((BM + BN) / 8) % LW != 0) return -23;
-  auto kern = dgemm_kernel<TM, TN, WM, WN, STAGES, EPI, ((BM + BN) / 8) % (LW > 0 ? LW : 1) == 0 ? LW : 0>;
+  auto kern = dgemm_kernel<TM, TN, WM, WN, STAGES, EPI, ((BM + BN) / 8) % (LW > 0 ? LW : 1) == 0 ? LW : 0, ROT>;
   if (lds > 64 * 1024) {
     static bool attr_set = false;  // per instantiation
     if (!attr_set) {
@@ -381,6 +383,16 @@ int launch_cfg(const DGArgs& a, int ksplit, hipStream_t st) {
   }
   hipLaunchKernelGGL(kern, grid, dim3(64 * (WM * WN + LW)), lds, st, b);
   return (int)hipGetLastError();
+}
+
+// Rotated starts (areal_dgemm) for the tiles that wide layers take, split-K and paired heads without: their workgroups are few, or
+// start apart by themselves. A kernel of their own: the wrapped step costs the others up to 4 % (100 rows, 8192 by 8192 78 / 81 us).
+template <int TM, int TN, int WM, int WN, int STAGES, int EPI, int LW>
+int launch_cfg(const DGArgs& a, int ksplit, hipStream_t st) {
+  constexpr bool WIDE = (EPI == DG_BF16 || EPI == DG_SWIGLU) && LW == 4 && 32 * TN * WN == 128 && 32 * TM * WM <= 128;
+  if constexpr (WIDE)
+    if (a.rot) return launch_as<TM, TN, WM, WN, STAGES, EPI, LW, true>(a, ksplit, st);
+  return launch_as<TM, TN, WM, WN, STAGES, EPI, LW, false>(a, ksplit, st);
 }
 
 template <int TM, int TN, int WM, int WN, int STAGES, int LW>
@@ -469,8 +481,10 @@ extern "C" int areal_dgemm(const void* X, long xs, const void* W, const void* bi
   DGArgs a;
   a.X = (const bf16_t*)X; a.xs = xs; a.W = (const bf16_t*)W; a.bias = (const bf16_t*)bias; a.Y = Y; a.ys = ys;
   a.M = M; a.N = N; a.K = K; a.k_per_split = kps; a.nt = nt; a.act = act;
-  // several row blocks reread the weights from the caches: 200 / 320 rows level (K 2048 213 / 314 us and 210 / 313)
-  a.rot = ksplit == 1 && M <= 128 ? k_rotation(K) : 0;
+  // Several row blocks reread the weights from the caches: 200 / 320 rows level (K 2048 213 / 314 us and 210 / 313). Fewer columns
+  // are fewer workgroups that meet: us without / with, 4096 deep, 24 and 100 rows, 4096 columns 22.6 / 22.7, 29.0 / 29.4, 8192
+  // 29.3 / 29.2, 41.0 / 41.8, 16384 31.7 / 29.9, 42.2 / 42.5, 32768 56.9 / 41.1, 59.5 / 50.0.
+  a.rot = ksplit == 1 && N >= 16384 && M <= (N >= 32768 ? 128 : 64) ? k_rotation(K) : 0;
   a.pos = nullptr; a.slots = nullptr; a.cos_t = a.sin_t = nullptr; a.q_out = a.kcache = a.vcache = nullptr;
   a.Hq = a.Hkv = 0; a.D = 2; a.max_pos = 0; a.do_rope = 0;
   switch (cfg) {
@@ -503,7 +517,7 @@ extern "C" int areal_dgemm_qkv_rope(const void* X, long xs, const void* W, const
   if (cfg == 4 && (D / 2) % 64 != 0) return -2;
   DGArgs a;
   a.X = (const bf16_t*)X; a.xs = xs; a.W = (const bf16_t*)W; a.bias = (const bf16_t*)bias; a.Y = nullptr; a.ys = 0;
-  a.M = M; a.N = N; a.K = K; a.k_per_split = K; a.nt = nt; a.rot = 0; a.act = 0;
+  a.M = M; a.N = N; a.K = K; a.k_per_split = K; a.nt = nt; a.act = 0;
   a.pos = pos; a.slots = slots; a.cos_t = cos_t; a.sin_t = sin_t; a.q_out = (bf16_t*)q_out;
   a.kcache = (bf16_t*)kcache; a.vcache = (bf16_t*)vcache; a.Hq = Hq; a.Hkv = Hkv; a.D = D; a.max_pos = max_pos;
   a.do_rope = do_rope;

@@ -39,9 +39,9 @@ struct SGArgs {
   int w;        // columns per range (multiple of 4)
   int ntiles;   // ceil(F / w)
   int mblocks;  // row blocks (1 or 2)
-  int rot;      // range t starts its reduction at step t * rot and wraps round: k_rotation (common.hpp)
   int nt;       // non-temporal weight loads
   int act;      // gate activation: 0 SiLU (SwiGLU), 1 tanh-approximated GELU (GeGLU)
+  int rot;      // range t starts its reduction at step t * rot and wraps round: k_rotation (common.hpp)
 };
 
 template <int N>
@@ -68,7 +68,7 @@ DEVINL float sg_gate(float x, int act) {
 }
 
 // RT: 16-row activation tiles per consumer wave (block rows BM = 64 RT); TW: 16-column tiles per half (gate / up).
-template <int RT, int TW, int STAGES>
+template <int RT, int TW, int STAGES, bool ROT>
 __global__ __launch_bounds__(512) void dswiglu_kernel(const SGArgs a) {
   constexpr int BM = 64 * RT, HW = 16 * TW, WR = 2 * HW;  // weight rows of a stage: HW gate + HW up
   constexpr int NP = (WR + BM) / 8, IPW = NP / 4;          // 1-KiB pieces per stage, per loader wave
@@ -119,10 +119,12 @@ __global__ __launch_bounds__(512) void dswiglu_kernel(const SGArgs a) {
         src[j] = a.X + (size_t)m * a.xs + 8 * c;
       }
     }
-    const int rot = (tile * a.rot) % nsteps;
+    const int rot = ROT ? k_start(tile, a.rot, nsteps) : 0;
     auto issue = [&](int buf, int step) {
-      step += rot;
-      step -= step >= nsteps ? nsteps : 0;
+      if (ROT) {
+        step += rot;
+        step -= step >= nsteps ? nsteps : 0;
+      }
       char* base = smem + buf * STAGE_BYTES + lwave * (IPW * 1024);
 #pragma unroll
       for (int j = 0; j < IPW; ++j) {
@@ -203,11 +205,11 @@ __global__ __launch_bounds__(512) void dswiglu_kernel(const SGArgs a) {
   }
 }
 
-template <int RT, int TW, int STAGES>
-int sg_launch(const SGArgs& a, hipStream_t st) {
+template <int RT, int TW, int STAGES, bool ROT>
+int sg_launch_as(const SGArgs& a, hipStream_t st) {
   constexpr size_t lds = (size_t)STAGES * (32 * TW + 64 * RT) * 128;
   static_assert(lds <= 160 * 1024, "staging exceeds the LDS of a CU");
-  auto kern = dswiglu_kernel<RT, TW, STAGES>;
+  auto kern = dswiglu_kernel<RT, TW, STAGES, ROT>;
   static bool attr_set = false;  // per instantiation
   if (!attr_set) {
     HIP_RET(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
@@ -216,6 +218,11 @@ int sg_launch(const SGArgs& a, hipStream_t st) {
   const int groups = a.mblocks == 1 ? a.ntiles : ((a.ntiles + 7) / 8) * 8 * a.mblocks;
   hipLaunchKernelGGL(kern, dim3(groups), dim3(512), lds, st, a);
   return (int)hipGetLastError();
+}
+
+template <int RT, int TW, int STAGES>
+int sg_launch(const SGArgs& a, hipStream_t st) {
+  return a.rot ? sg_launch_as<RT, TW, STAGES, true>(a, st) : sg_launch_as<RT, TW, STAGES, false>(a, st);
 }
 
 template <int RT, int TW>
@@ -244,8 +251,9 @@ extern "C" int areal_dswiglu(const void* X, long xs, const void* W, void* Y, lon
   SGArgs a;
   a.X = (const bf16_t*)X; a.xs = xs; a.W = (const bf16_t*)W; a.Y = (bf16_t*)Y; a.ys = ys;
   a.M = M; a.F = F; a.K = K; a.w = w; a.ntiles = (F + w - 1) / w; a.mblocks = mblocks; a.nt = nt; a.act = act;
-  // us without / with, 14336 columns, 4096 deep, 8 / 64 / 128 / 200 rows: 46 / 41, 47 / 41, 53 / 52, 78 / 77
-  a.rot = mblocks == 1 ? k_rotation(K) : 0;
+  // us without / with, 14336 columns, 4096 deep, 8 / 64 / 128 / 200 rows: 46 / 41, 47 / 41, 53 / 52, 78 / 77; 8 / 100 rows, 8192 columns
+  // 34 / 25, 38 / 33, but 4096 columns 23.7 / 23.9, 30.1 / 31.0
+  a.rot = mblocks == 1 && F >= 8192 ? k_rotation(K) : 0;
   const int rows = (M + mblocks - 1) / mblocks;  // rows per block
   const int rt = (rows + 63) / 64;
   const int tw = (w + 15) / 16;

@@ -59,10 +59,10 @@ DEVINL int gg_off(int row, int ch) { return row * 128 + ((ch ^ ((row >> 1) & 7))
 // same columns, and the epilogue stores silu(gate) * up (gate and up rounded to bf16 first), [T, N / 2]. For a decode step,
 // where the gather and the activation are launches of their own and little else (64 / 512 rows of 2048, 8 of 128 experts
 // of 768: 166 -> 158 us / 197 -> 167, 1 row 29 -> 25).
-template <int TM, int TN, int KH, bool NT, bool GATED>
+template <int TM, int TN, int KH, bool NT, bool ROT, bool GATED>
 __global__ __launch_bounds__(256) void grouped_gemm_nt_kernel(
-    const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, bf16_t* __restrict__ out, const int64_t* __restrict__ src_row,
-    const int* __restrict__ offsets, int E, int N, int K, int64_t w_expert_stride, int rot) {
+    const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, bf16_t* __restrict__ out, const int* __restrict__ offsets, int E,
+    int N, int K, int64_t w_expert_stride, int rot, const int64_t* __restrict__ src_row) {
   static_assert(!GATED || TN == 128, "a wave's two column tiles are gate and up");
   constexpr int MI = TM / 64, NI = TN / 64;
   __shared__ __attribute__((aligned(16))) char smem[KH * (TM + TN) * 128];
@@ -86,11 +86,13 @@ __global__ __launch_bounds__(256) void grouped_gemm_nt_kernel(
   // the launch below).
   const int lrow = tid >> 3, lch = tid & 7;
   bf16x8 areg[KH * TM / 32] = {}, breg[KH * TN / 32];
-  int64_t arow[TM / 32];  // source row of each of this thread's tile rows
+  int64_t arow[TM / 32];  // GATED: source row of each of this thread's tile rows
+  if constexpr (GATED) {
 #pragma unroll
-  for (int i = 0; i < TM / 32; ++i) {
-    const int m = m0 + lrow + 32 * i;
-    arow[i] = GATED ? (m < row_hi ? src_row[m] : 0) : m;
+    for (int i = 0; i < TM / 32; ++i) {
+      const int m = m0 + lrow + 32 * i;
+      arow[i] = m < row_hi ? src_row[m] : 0;
+    }
   }
   auto load = [&](int k0) {
 #pragma unroll
@@ -98,7 +100,7 @@ __global__ __launch_bounds__(256) void grouped_gemm_nt_kernel(
 #pragma unroll
       for (int i = 0; i < TM / 32; ++i) {
         const int m = m0 + lrow + 32 * i;
-        if (m < row_hi) areg[h * (TM / 32) + i] = ld8(x + (size_t)arow[i] * K + k0 + 64 * h + lch * 8);
+        if (m < row_hi) areg[h * (TM / 32) + i] = ld8(x + (GATED ? (size_t)arow[i] : (size_t)m) * K + k0 + 64 * h + lch * 8);
       }
 #pragma unroll
       for (int i = 0; i < TN / 32; ++i) {
@@ -126,14 +128,14 @@ __global__ __launch_bounds__(256) void grouped_gemm_nt_kernel(
 #pragma unroll
     for (int j = 0; j < 16; ++j) acc[t][j] = 0.f;
 
-  const int first = e * rot % (K / (64 * KH)) * (64 * KH);  // rot: gg_rot, at the launch
+  const int first = ROT ? k_start(e, rot, K / (64 * KH)) * (64 * KH) : 0;  // rot: gg_rot, at the launch
   load(first);
   for (int k0 = 0; k0 < K; k0 += 64 * KH) {
     __syncthreads();  // previous tile fully consumed
     stage();
     if (k0 + 64 * KH < K) {
-      const int next = first + k0 + 64 * KH;
-      load(next < K ? next : next - K);
+      const int next = ROT ? first + k0 + 64 * KH : k0 + 64 * KH;
+      load(ROT && next >= K ? next - K : next);
     }
     __syncthreads();
 #pragma unroll
@@ -205,10 +207,10 @@ extern "C" int areal_grouped_gemm_tile_m(int T, int E, int N, int tile_m) {
 // 14336 columns, 4096 deep, 1 row 32 / 48, 2 55 / 55, 4 87 / 77, 64 184 / 167; 16 of 704 columns, 1024 deep, 16 rows 9 / 12.
 // Expert e's tiles start their reduction at step 13 e (k_rotation, common.hpp) while the weights are read once: by expert, so that
 // what other rows chose does not change the order of a row's sums. With more rows, whose column tiles are reread from the caches,
-// the common order is level or better. us without / with: 128 experts, 1536 columns, 2048 deep, 64 rows 57 / 53, 512 147 / 124,
+// the common order is level or better; below 16 rows a few experts' tiles stay apart by themselves (8 rows of 8 experts, 14336
+// columns, 4096 deep 75 / 87). us without / with: 128 experts, 1536 columns, 2048 deep, 64 rows 57 / 53, 512 147 / 124,
 // 1600 162 / 136, 4096 173 / 150, but 8192 207 / 213, 16000 337 / 356; 64 experts, 2816 columns, 2048 deep, 512 rows 159 / 121;
 // 8 experts, 4096 columns, 14336 deep, 128 rows 191 / 186 (by row tile the same within 1 us).
-static int gg_rot(int T, int E, int K) { return T <= 48l * E ? k_rotation(K) : 0; }
 static bool gg_stream(int T, int E, int col_tiles) { return T <= 48l * E && (long)(T < E ? T : E) * col_tiles > 256; }
 
 extern "C" int areal_grouped_gemm_nt(const void* x, const void* w, void* out, const int* offsets, int T,
@@ -228,16 +230,23 @@ extern "C" int areal_grouped_gemm_nt(const void* x, const void* w, void* out, co
     const char* e = getenv("AREAL_GROUPED_GEMM_KSTEP");
     return e && atoi(e) == 128;
   }();
-  const int rot = gg_rot(T, E, K);
   const bool stream = gg_stream(T, E, N / tn);
-#define AREAL_GG_LAUNCH(TM_, TN_, KH_, NT_)                                                                    \
-  hipLaunchKernelGGL((grouped_gemm_nt_kernel<TM_, TN_, KH_, NT_, false>), grid, block, 0, st, (const bf16_t*)x, \
-                     (const bf16_t*)w, (bf16_t*)out, (const int64_t*)nullptr, offsets, E, N, K, w_expert_stride, rot)
+  const int rot = stream && T >= 16 ? k_rotation(K) : 0;
+#define AREAL_GG_LAUNCH(TM_, TN_, KH_, NT_, ROT_)                                                              \
+  hipLaunchKernelGGL((grouped_gemm_nt_kernel<TM_, TN_, KH_, NT_, ROT_, false>), grid, block, 0, st, (const bf16_t*)x, \
+                     (const bf16_t*)w, (bf16_t*)out, offsets, E, N, K, w_expert_stride, rot, (const int64_t*)nullptr)
   if (tm == 128 && tn == 128) {
-    if (deep && K % 128 == 0) AREAL_GG_LAUNCH(128, 128, 2, false); else AREAL_GG_LAUNCH(128, 128, 1, false);
-  } else if (tm == 128) AREAL_GG_LAUNCH(128, 64, 1, false);
-  else if (tn == 128) { if (stream) AREAL_GG_LAUNCH(64, 128, 1, true); else AREAL_GG_LAUNCH(64, 128, 1, false); }
-  else { if (stream) AREAL_GG_LAUNCH(64, 64, 1, true); else AREAL_GG_LAUNCH(64, 64, 1, false); }
+    if (deep && K % 128 == 0) AREAL_GG_LAUNCH(128, 128, 2, false, false); else AREAL_GG_LAUNCH(128, 128, 1, false, false);
+  } else if (tm == 128) AREAL_GG_LAUNCH(128, 64, 1, false, false);
+  else if (tn == 128) {
+    if (rot) AREAL_GG_LAUNCH(64, 128, 1, true, true);
+    else if (stream) AREAL_GG_LAUNCH(64, 128, 1, true, false);
+    else AREAL_GG_LAUNCH(64, 128, 1, false, false);
+  } else {
+    if (rot) AREAL_GG_LAUNCH(64, 64, 1, true, true);
+    else if (stream) AREAL_GG_LAUNCH(64, 64, 1, true, false);
+    else AREAL_GG_LAUNCH(64, 64, 1, false, false);
+  }
 #undef AREAL_GG_LAUNCH
   return (int)hipGetLastError();
 }
@@ -251,11 +260,14 @@ extern "C" int areal_grouped_gate_up(const void* x, const int64_t* src_row, cons
   if (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) % 16 != 0 || w_expert_stride % 8 != 0) return -2;
   if (max_tiles < T / 64 + E || max_tiles > 65535) return -3;
   const dim3 grid(N / 128, max_tiles), block(256);
-  const int rot = gg_rot(T, E, K);
-#define AREAL_GG_LAUNCH(NT_)                                                                                      \
-  hipLaunchKernelGGL((grouped_gemm_nt_kernel<64, 128, 1, NT_, true>), grid, block, 0, st, (const bf16_t*)x,         \
-                     (const bf16_t*)w, (bf16_t*)out, src_row, offsets, E, N, K, w_expert_stride, rot)
-  if (gg_stream(T, E, N / 128)) AREAL_GG_LAUNCH(true); else AREAL_GG_LAUNCH(false);
+  const bool stream = gg_stream(T, E, N / 128);
+  const int rot = stream && T >= 16 ? k_rotation(K) : 0;
+#define AREAL_GG_LAUNCH(NT_, ROT_)                                                                                \
+  hipLaunchKernelGGL((grouped_gemm_nt_kernel<64, 128, 1, NT_, ROT_, true>), grid, block, 0, st, (const bf16_t*)x,   \
+                     (const bf16_t*)w, (bf16_t*)out, offsets, E, N, K, w_expert_stride, rot, src_row)
+  if (rot) AREAL_GG_LAUNCH(true, true);
+  else if (stream) AREAL_GG_LAUNCH(true, false);
+  else AREAL_GG_LAUNCH(false, false);
 #undef AREAL_GG_LAUNCH
   return (int)hipGetLastError();
 }

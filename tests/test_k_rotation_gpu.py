@@ -14,7 +14,8 @@ def _ints(*shape):
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 8192, 2048), (33, 8224, 4096), (64, 8192 + 96, 2048), (65, 9000 // 32 * 32, 6144),
-                                   (128, 8192, 14336), (129, 8192, 2048), (64, 8192, 1984)])
+                                   (128, 8192, 14336), (129, 8192, 2048), (64, 8192, 1984), (1, 16384, 2048), (64, 16384 + 96, 4096),
+                                   (100, 32768 + 32, 6144), (128, 32768, 2048)])
 def test_decode_gemm_takes_every_step_once(M, N, K):
     torch.manual_seed(M)
     x, w = _ints(M, K), _ints(N, K)
@@ -23,9 +24,11 @@ def test_decode_gemm_takes_every_step_once(M, N, K):
     assert dg.pick_config(M, N, K, dg.EPI_BF16)[2] == 1
     for stages in (2, 3):
         assert torch.equal(dg.dgemm(x, w, cfg=8, stages=stages), ref.bfloat16())
+        assert torch.equal(dg.dgemm(x, w, cfg=4, stages=stages, loader_waves=4), ref.bfloat16())  # (rotated where it is wide)
 
 
-@pytest.mark.parametrize("M,F,K", [(1, 512, 2048), (64, 4096, 4096), (130, 1000, 2048), (200, 1024, 2048)])
+@pytest.mark.parametrize("M,F,K", [(1, 512, 2048), (64, 4096, 4096), (130, 1000, 2048), (200, 1024, 2048),
+                                   (1, 8192, 2048), (100, 8192 + 40, 6144), (200, 8192, 2048)])
 def test_decode_swiglu_takes_every_step_once(M, F, K):
     torch.manual_seed(F)
     x, w = _ints(M, K), _ints(2 * F, K)
@@ -37,7 +40,8 @@ def test_decode_swiglu_takes_every_step_once(M, F, K):
     assert ((out.double() - ref).abs() <= ref.abs() * (3 + whole[:, :F].abs()) * 2.0 ** -8 + 1e-6).all()
 
 
-@pytest.mark.parametrize("T,k,E,F,K", [(1, 1, 4, 64, 2048), (40, 8, 128, 64, 2048), (66, 2, 4, 128, 4096), (300, 2, 4, 64, 2048)])
+@pytest.mark.parametrize("T,k,E,F,K", [(1, 1, 4, 64, 2048), (40, 8, 128, 64, 2048), (66, 2, 4, 128, 4096), (300, 2, 4, 64, 2048),
+                                         (11, 8, 128, 192, 2048)])
 def test_grouped_gemm_takes_every_step_once(T, k, E, F, K):
     torch.manual_seed(T)
     x, w = _ints(T, K), _ints(E, 2 * F, K)
@@ -50,7 +54,7 @@ def test_grouped_gemm_takes_every_step_once(T, k, E, F, K):
     assert torch.equal(ops.grouped_gate_up(x, src_row, w, offsets[:E + 1]), ops.swiglu(out))
 
 
-@pytest.mark.parametrize("T,k,E,F,K", [(64, 8, 128, 128, 2048), (70, 2, 8, 192, 4096)])
+@pytest.mark.parametrize("T,k,E,F,K", [(64, 8, 128, 192, 2048), (70, 2, 8, 2176, 4096)])
 def test_a_row_has_the_same_bits_whatever_the_others_choose(T, k, E, F, K):
     torch.manual_seed(T)
     x = torch.randn(T, K, device="cuda").bfloat16()
