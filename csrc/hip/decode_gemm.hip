@@ -651,8 +651,9 @@ extern "C" int areal_splitk_residual_rmsnorm(const float* slab, int S, const voi
 
 // qkv = bf16(sum_k slab[k] + bias), laid out [T, Hq + 2 Hkv, D]: rotate q and k (half-split layout), write q to
 // q_out [T, Hq, D] (bf16), k / v into the paged caches at slots[t] (K [P, Hkv, 32, D], V [P, Hkv, D, 32]).
-// One block per token and `heads` heads (64 .. 1024 threads): the summed columns are staged in LDS (fp32), then rotated /
+// One block per token (SPLIT: and `heads` heads; 64 .. 1024 threads): the summed columns are staged in LDS (fp32), then rotated /
 // scattered from there.
+template <bool SPLIT>
 __global__ __launch_bounds__(1024) void splitk_rope_cache_write_kernel(
     const float* __restrict__ slab, int S, const bf16_t* __restrict__ bias, const int* __restrict__ pos,
     const int64_t* __restrict__ slots, const float* __restrict__ cos_t, const float* __restrict__ sin_t,
@@ -665,14 +666,14 @@ __global__ __launch_bounds__(1024) void splitk_rope_cache_write_kernel(
   const int lph = half >> 3;
   const int Nq = (Hq + 2 * Hkv) * D;
   const size_t stride = (size_t)T * Nq;
-  const int h0 = blockIdx.y * heads, h1 = min(Hq + 2 * Hkv, h0 + heads);  // this block's heads
+  const int h0 = SPLIT ? blockIdx.y * heads : 0, h1 = SPLIT ? min(Hq + 2 * Hkv, h0 + heads) : Hq + 2 * Hkv;  // this block's heads
   const int c0 = h0 * D;
   // Position, slot and this thread's first rotary-table rows are requested before the slab sum, so that their
   // latency (a dependent pos -> table chain) runs under the slab loads instead of after the barrier.
   int p = pos[t];
   p = p < 0 ? 0 : (p >= max_pos ? max_pos - 1 : p);
   const int64_t slot = slots ? slots[t] : -1;
-  const int nrot = max(0, min(Hq + Hkv, h1) - h0) * lph;
+  const int nrot = (SPLIT ? max(0, min(Hq + Hkv, h1) - h0) : Hq + Hkv) * lph;
   f32x4 c_pre[2], s_pre[2];
   if (do_rope && (int)threadIdx.x < nrot) {
     const int sub0 = threadIdx.x % lph;
@@ -680,7 +681,7 @@ __global__ __launch_bounds__(1024) void splitk_rope_cache_write_kernel(
     const f32x4* sp4 = reinterpret_cast<const f32x4*>(sin_t + (size_t)p * half + sub0 * 8);
     c_pre[0] = cp4[0]; c_pre[1] = cp4[1]; s_pre[0] = sp4[0]; s_pre[1] = sp4[1];
   }
-  for (int c = threadIdx.x; c < ((h1 - h0) * D >> 2); c += blockDim.x) {
+  for (int c = threadIdx.x; c < ((SPLIT ? (h1 - h0) * D : Nq) >> 2); c += blockDim.x) {
     f32x4 s = slab_sum4(slab + (size_t)t * Nq + c0 + c * 4, stride, S);
     if (bias) {
       const bf16x4 b = *reinterpret_cast<const bf16x4*>(bias + c0 + c * 4);
@@ -762,10 +763,11 @@ __global__ __launch_bounds__(1024) void splitk_rope_cache_write_kernel(
     }
   }
   if (slot >= 0) {
-    const int v0 = max(h0, Hq + Hkv);
-    for (int i = threadIdx.x; i < (h1 - v0) * D; i += blockDim.x) {
-      const int vh = v0 - Hq - Hkv + i / D, d = i % D;
-      st1_cache(vcache, (((size_t)page * Hkv + vh) * D + d) * 32 + off, rowbuf[(v0 - h0) * D + i], fp8);
+    const int v0 = SPLIT ? max(h0, Hq + Hkv) : Hq + Hkv;
+    const float* vrow = rowbuf + (v0 - h0) * D;
+    for (int i = threadIdx.x; i < (SPLIT ? h1 - v0 : Hkv) * D; i += blockDim.x) {
+      const int vh = (SPLIT ? v0 - Hq - Hkv : 0) + i / D, d = i % D;
+      st1_cache(vcache, (((size_t)page * Hkv + vh) * D + d) * 32 + off, vrow[i], fp8);
     }
   }
 }
@@ -783,16 +785,17 @@ extern "C" int areal_splitk_rope_cache_write(const float* slab, int S, const voi
   // one float4 chunk of the summed row per thread where the row allows it: all of a thread's slab loads are in
   // flight at once (a second pass over the row would wait for the first one's loads)
   // Heads of 256 columns a block, of 512 for rows of more than 2048: one token's slabs through one CU's load path wait for each
-  // other. us of whole rows / so split, 8 / 24 / 64 / 128 / 320 tokens: 16 heads of 128 in 8 to 2 slabs 3.5 / 3.5 / 3.6 / 3.6 / 5.0
-  // and 2.9 / 2.9 / 3.1 / 3.3 / 4.7; 40 heads with norms, 3 to 1 slabs 4.7 / 4.8 / 5.0 / 5.3 / 8.9 and 3.4 / 3.4 / 4.0 / 4.7 / 7.6;
-  // 48 heads 4.0 / 4.1 / 4.6 / 6.4 / 10.1 and 3.0 / 3.3 / 3.8 / 5.6 / 9.2; 18 heads of 64 3.1 / 3.2 / 3.3 / 3.4 / 4.1 and 2.7 / 2.7 /
-  // 2.8 / 3.0 / 3.8.
+  // other. With more tokens (and long rows) whole rows fill the chip by themselves. us of whole rows / so split, 32 / 96 / 160 / 256 /
+  // 448 tokens: 16 heads of 128 in 8 to 2 slabs 3.8 / 3.9 / 4.1 / 4.5 / 4.9 and 3.1 / 3.4 / 3.9 / 4.3 / 5.3; 40 heads with norms, 3 to 1
+  // slabs 5.0 / 5.3 / 5.7 / 6.4 / 7.9 and 3.9 / 4.3 / 5.4 / 6.6 / 8.6; 80 heads 5.4 / 6.1 / 7.4 / 9.9 / 10.6 and 3.7 / 5.1 / 6.9 / 10.3 /
+  // 12.7; 18 heads of 64 3.9 / 4.0 / 4.1 / 4.2 / 4.6 and 3.4 / 3.6 / 3.7 / 3.9 / 4.3.
   const int all = Hq + 2 * Hkv;
-  const int heads = std::min(all, std::max(1, (all * D <= 2048 ? 256 : 512) / D));
-  const int threads = std::min(1024, std::max(64, ((heads * D / 4 + 63) / 64) * 64));
-  hipLaunchKernelGGL(splitk_rope_cache_write_kernel, dim3(T, (all + heads - 1) / heads), dim3(threads),
-                     (size_t)heads * D * sizeof(float), st, slab, S, (const bf16_t*)bias, pos,
-                     slots, cos_t, sin_t, (bf16_t*)q_out, kcache, vcache, T, Hq, Hkv, D, max_pos,
+  const bool split = T <= 160 || (long)T * all * D <= 524288;
+  const int heads = split ? std::min(all, std::max(1, (all * D <= 2048 ? 256 : 512) / D)) : all;
+  const int threads = std::min(1024, std::max(split ? 64 : 256, ((heads * D / 4 + 63) / 64) * 64));
+  const auto kern = split ? splitk_rope_cache_write_kernel<true> : splitk_rope_cache_write_kernel<false>;
+  hipLaunchKernelGGL(kern, dim3(T, (all + heads - 1) / heads), dim3(threads), (size_t)heads * D * sizeof(float), st, slab, S,
+                     (const bf16_t*)bias, pos, slots, cos_t, sin_t, (bf16_t*)q_out, kcache, vcache, T, Hq, Hkv, D, max_pos,
                      do_rope, (const bf16_t*)q_norm, (const bf16_t*)k_norm, norm_eps, fp8, heads);
   return (int)hipGetLastError();
 }

@@ -10,7 +10,10 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("T,Hq,Hkv,D,S,norm,fp8", [(1, 1, 1, 16, 1, False, False), (3, 5, 1, 128, 8, True, False),
                                                    (9, 14, 2, 64, 3, False, False), (4, 32, 8, 128, 5, True, True),
-                                                   (7, 11, 3, 80, 2, False, False), (2, 3, 2, 256, 4, False, True)])
+                                                   (7, 11, 3, 80, 2, False, False), (2, 3, 2, 256, 4, False, True),
+                                                   # many tokens of long rows: a workgroup each; the last ones that are split
+                                                   (161, 32, 8, 128, 2, True, False), (240, 64, 8, 128, 1, False, True),
+                                                   (160, 32, 8, 128, 2, True, False), (250, 12, 2, 128, 3, False, False)])
 def test_heads_dealt_to_blocks(T, Hq, Hkv, D, S, norm, fp8):
     torch.manual_seed(Hq)
     N = (Hq + 2 * Hkv) * D
