@@ -85,11 +85,12 @@ def _even_splits(pairs: int, splits: int) -> int:
 
 
 @functools.lru_cache(maxsize=1024)
-def _tile_plan(pairs: int, tiles: int, flush: int) -> Tuple[float, int, int]:
+def _tile_plan(pairs: int, tiles: int, flush: int, rows: int = 256) -> Tuple[float, int, int]:
     """(time in 128-deep pairs, 3 us each; tiles of 256 x 256 that one workgroup reduces; parts of the reduction of each of the
     others). A CU runs one workgroup: tiles beyond a multiple of 256 would leave CUs idle in a last round, so they are split
     until the round is full. `flush`: pairs that writing a whole tile's result takes. A part costs 6 pairs more (its start, and
-    256 KiB of fp32 to write), a chip full of them 8 to be read and summed, the summing kernel itself 2: 48 tiles of 256 pairs in
+    256 KiB of fp32 to write; half of it for the few `rows` of a single row tile), a chip full of them 8 to be read and summed, the
+    summing kernel itself 2 and a 24th for each part that a thread adds: 48 tiles of 256 pairs in
     5 parts take 183 us, 210 tiles in 6 parts (330 MB, more than the memory-side cache holds) 871, whole 745 (the 46 CUs that
     idle leave their power to the others)."""
     rounds, rest = divmod(tiles, 256)
@@ -98,7 +99,8 @@ def _tile_plan(pairs: int, tiles: int, flush: int) -> Tuple[float, int, int]:
         for s in range(2, min(pairs, 64) + 1):
             chunk = -(-pairs // s)
             if -(-pairs // chunk) == s:  # (every part has work)
-                cost = rounds * (pairs + flush) + -(-rest * s // 256) * (chunk + 6) + 2 + 8 * s * rest / 256
+                cost = (rounds * (pairs + flush) + -(-rest * s // 256) * (chunk + 3 + 3 * rows / 256) + 2
+                        + 8 * s * rest / 256 * rows / 256 + s / 24)
                 best = min(best, (cost, rounds * 256, s))
     return best
 
@@ -122,7 +124,7 @@ def tgemm_wgrad_(acc: torch.Tensor, dy: torch.Tensor, x: torch.Tensor, splits: i
 
 
 def dgrad_cost(M: int, R: int, C: int) -> Tuple[float, int, int]:
-    return _tile_plan(R // 128, -(-M // 256) * (C // 256), 0)
+    return _tile_plan(R // 128, -(-M // 256) * (C // 256), 0, min(256, -(-M // 32) * 32))
 
 
 def dgrad_splits(M: int, R: int, C: int) -> int:
@@ -165,13 +167,16 @@ def tgemm_nn(dy: torch.Tensor, w: torch.Tensor, splits: int = 0, out: Optional[t
 # 41 / 49, 257 / 290, 682 / 755; 2048 to 4096, 1500 / 3000 / 32768 rows 46 / 33, 48 / 49, 386 / 439; 2048 to 1536, 700 / 6000 /
 # 12000 / 32768 rows 31 / 22, 46 / 42, 78 / 100, 148 / 161. So: a deep reduction, or rounds that are
 # filled to five eighths (384 tiles 16 pairs deep: 92 / 90; 288 tiles 8 deep, two rounds for 1.1: 53 / 49; 1536 deep to 1536, 144 tiles: 35 / 33).
-DGRAD_MIN_DEPTH, DGRAD_MIN_TILES, DGRAD_MAX_LOSS = 8192, 192, 1.6
+# A deep reduction of one round of tiles that splitting does not fill is the library's: 10000 rows, 8192 deep to 1024 columns (160
+# tiles) 142 / 136, 3000 rows, 28672 deep to 4096 (192) 590 / 560; filled, it is not: 37888 deep to 3584 (168) 636 / 1057.
+DGRAD_MIN_DEPTH, DGRAD_MIN_TILES, DGRAD_MAX_LOSS, DGRAD_MAX_ROUND_LOSS = 8192, 192, 1.6, 1.25
 
 
 def _dgrad_own(M: int, R: int, C: int) -> bool:
     tiles = -(-M // 256) * (C // 256)
-    return R >= DGRAD_MIN_DEPTH or (tiles >= DGRAD_MIN_TILES
-                                    and dgrad_cost(M, R, C)[0] <= DGRAD_MAX_LOSS * M * (C // 256) * (R // 128) / 65536)
+    if R >= DGRAD_MIN_DEPTH:
+        return not 128 < tiles < 256 or dgrad_cost(M, R, C)[0] <= DGRAD_MAX_ROUND_LOSS * tiles * (R // 128) / 256
+    return tiles >= DGRAD_MIN_TILES and dgrad_cost(M, R, C)[0] <= DGRAD_MAX_LOSS * M * (C // 256) * (R // 128) / 65536
 
 
 def dgrad(dy: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:

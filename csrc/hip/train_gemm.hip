@@ -187,18 +187,31 @@ __global__ __launch_bounds__(512) void tgemm_kernel(const TGArgs a) {
   const int wrow = wave * 4 + (lane >> 4);
   const int wpc = ((lane & 15) ^ (((lane >> 4) << 2) | (wave & 3))) * 8;
   const size_t stepB = NN ? (size_t)64 * a.ldb : 64;  // elements of B from K tile to K tile
+  // NN, which takes any number of rows: rows of A past the last one are out of a buffer's range and cost the CU's load path nothing
+  // (repeating the last one instead: 2 rows from 28672 deep to 2048 columns 38 us, so 26). One descriptor per K tile; byte offsets
+  // of 256 rows fit 32 bits.
+  constexpr bool RANGE_A = NN && !GRP;
+  const unsigned rowA = (unsigned)a.lda * 2, vA = srow * rowA + schunk * 16;
+  const bf16_t* baseA = nullptr;
+  unsigned rangeA = 0;
   const bf16_t* srcA[2][2];  // [piece][issue]
   const bf16_t* srcB[2][2];
   auto set_sources = [&](const Tile& t) __attribute__((always_inline)) {
     const int m0 = t.m0, n0 = t.n0, k0 = t.k0;
     const bf16_t* B = GRP ? a.B + t.e * a.stride : a.B;
+    if (RANGE_A) {
+      baseA = a.A + (size_t)m0 * a.lda + k0;
+      rangeA = (unsigned)(min(a.M - m0, 256) - 1) * rowA + 128;
+    }
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
-        int row = m0 + i * 128 + h * 64 + srow;
-        row = row < t.mlim ? row : t.mlim - 1;
-        srcA[h][i] = a.A + (size_t)row * a.lda + schunk * 8 + (PARTS ? k0 : 0);
+        if (!RANGE_A) {
+          int row = m0 + i * 128 + h * 64 + srow;
+          row = row < t.mlim ? row : t.mlim - 1;
+          srcA[h][i] = a.A + (size_t)row * a.lda + schunk * 8 + (PARTS ? k0 : 0);
+        }
         int col;
         if (NN) {  // one pointer: N is a multiple of 256 here, pieces and issues are a fixed step apart
           if (h == 0 && i == 0) srcB[0][0] = B + (size_t)(k0 + wrow) * a.ldb + n0 + (wpc >> 5) * 64 + (wpc & 31);
@@ -216,6 +229,13 @@ __global__ __launch_bounds__(512) void tgemm_kernel(const TGArgs a) {
   };
   auto stage = [&](int buf, int piece, int kt) __attribute__((always_inline)) {
     char* dst = smem + buf * TG_BUF + piece * TG_PIECE + wave * 1024;
+    if (RANGE_A && piece < 2) {
+      const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(baseA + (size_t)kt * 64), 0, rangeA, 0x00020000);
+      const unsigned v = vA + piece * 64 * rowA;  // the whole offset in the vector operand, the one that the range check is about
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lptr_t)dst, 16, v, 0, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lptr_t)(dst + 8192), 16, v + 128 * rowA, 0, 0, 0);
+      return;
+    }
     const bf16_t* s0 = piece < 2 ? srcA[piece][0] : NN ? srcB[0][0] + (piece - 2) * 32 : srcB[piece - 2][0];
     const bf16_t* s1 = piece < 2 ? srcA[piece][1] : NN ? s0 + stepB / 2 : srcB[piece - 2][1];
     const size_t at = kt * (piece < 2 ? (size_t)64 : stepB);
@@ -318,8 +338,10 @@ __global__ __launch_bounds__(512) void tgemm_kernel(const TGArgs a) {
     char* ob = smem + TG_LDS + wave * 4096;
     if (PARTS && part) {  // one part of the reduction, summed by a kernel of its own
       float* op = part + (wr * 128 + mh * 64 + fr) * 256 + wc * 64 + fq * 4;
+      const int left = a.M - m0 - wr * 128 - mh * 64 - fr;  // rows past the last one are not read (2 rows, 28 parts: 58 MB of them)
 #pragma unroll
       for (int mt = 0; mt < 4; ++mt)
+        if (mt * 16 < left)
 #pragma unroll
         for (int nt = 0; nt < 2; ++nt) {
           *reinterpret_cast<f32x4*>(op + mt * 4096 + nt * 16) = c0[mt][nt];
@@ -852,21 +874,33 @@ __global__ __launch_bounds__(256) void tgemm_wgrad_sum_kernel(const TWArgs a) {
 // would leave CUs idle in a last round (or all of them, for few rows) are split over the reduction until the chip is full; the
 // parts are written as fp32 and summed here (they stay in the L2 and the memory-side cache).
 // =====================================================================================
-// C of the tiles from `whole` on = sum of the parts, in order. Block: 8 rows of a tile.
+// C of the tiles from `whole` on = sum of the parts, in order. Block: 8 rows of a tile, of 256 threads; 2 of 64 for a single row of
+// tiles: few rows' parts through a few CUs' load paths take longer than their products (16 rows, 19 parts of 2560 columns: 3 us).
 __global__ __launch_bounds__(256) void tgemm_sum_kernel(const TGArgs a) {
-  const int rest = a.tiles_m * a.tiles_n - a.whole, t = blockIdx.x >> 5, wg = a.whole + t;
+  const int lg = 31 - __clz(blockDim.x) - 5;  // rows of the block: 8 or 2
+  const int rest = a.tiles_m * a.tiles_n - a.whole, t = blockIdx.x >> (8 - lg), wg = a.whole + t;
   const int band = wg / (TG_GROUP_M * a.tiles_n), first = band * TG_GROUP_M, rows = min(a.tiles_m - first, TG_GROUP_M);
   const int in_band = wg - band * TG_GROUP_M * a.tiles_n;
-  const int row = (blockIdx.x & 31) * 8 + (threadIdx.x >> 5), col = (threadIdx.x & 31) * 8;
+  const int row = ((blockIdx.x & ((256 >> lg) - 1)) << lg) + (threadIdx.x >> 5), col = (threadIdx.x & 31) * 8;
   const int m = (first + in_band % rows) * 256 + row, n = in_band / rows * 256 + col;
   if (m >= a.M || n >= a.N) return;
   const float* p = a.part + ((size_t)t << 16) + row * 256 + col;
   f32x4 v0 = *reinterpret_cast<const f32x4*>(p), v1 = *reinterpret_cast<const f32x4*>(p + 4);
-#pragma unroll 4
-  for (int s = 1; s < a.splits; ++s) {
-    const float* q = p + ((size_t)s * rest << 16);
-    v0 += *reinterpret_cast<const f32x4*>(q);
-    v1 += *reinterpret_cast<const f32x4*>(q + 4);
+  for (int s = 1; s < a.splits; s += 8) {  // eight parts requested at a time, the last few too
+    f32x4 q0[8], q1[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      if (s + j < a.splits) {
+        const float* q = p + ((size_t)(s + j) * rest << 16);
+        q0[j] = *reinterpret_cast<const f32x4*>(q);
+        q1[j] = *reinterpret_cast<const f32x4*>(q + 4);
+      }
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      if (s + j < a.splits) {
+        v0 += q0[j];
+        v1 += q1[j];
+      }
   }
   bf16_t* op = a.C + (size_t)m * a.ldc + n;
   *reinterpret_cast<bf16x4*>(op) = bf16x4{f2bf(v0[0]), f2bf(v0[1]), f2bf(v0[2]), f2bf(v0[3])};
@@ -935,6 +969,11 @@ __global__ __launch_bounds__(1024) void tgemm_stats_kernel(const float* __restri
 
 }  // namespace
 
+static void tgemm_sum_launch(const TGArgs& a, long tiles, hipStream_t st) {
+  const int threads = a.tiles_m == 1 ? 64 : 256;
+  hipLaunchKernelGGL(tgemm_sum_kernel, dim3((unsigned)(tiles * (8192 / threads))), dim3(threads), 0, st, a);
+}
+
 // C[M, N] = A[M, K] . B[N, K]^T (+ bias). Leading dimensions in elements (multiples of 8: 16-byte rows), K a multiple
 // of 128, N a multiple of 4. Returns -1 for shapes outside that (the caller keeps its library path).
 // One launch = min(tiles, max_blocks) persistent workgroups (256 = one per CU). splits > 1 (no bias): the tiles from `whole` on
@@ -976,7 +1015,7 @@ static int tgemm_tn_launch(const void* A, long lda, const void* B, long ldb, voi
     hipLaunchKernelGGL((tgemm_kernel<1, false, false>), grid, block, TG_LDS, st, a);
   else
     hipLaunchKernelGGL((tgemm_kernel<0, false, false>), grid, block, TG_LDS + TG_OUT, st, a);
-  if (splits > 1) hipLaunchKernelGGL(tgemm_sum_kernel, dim3((unsigned)(tiles - whole) * 32), dim3(256), 0, st, a);
+  if (splits > 1) tgemm_sum_launch(a, tiles - whole, st);
   return (int)hipGetLastError();
 }
 
@@ -1078,8 +1117,7 @@ extern "C" int areal_tgemm_nn(const void* dY, long ldy, const void* W, long ldw,
     attr_set = true;
   }
   hipLaunchKernelGGL((tgemm_kernel<0, true, false>), dim3((unsigned)std::min(items, 256l)), dim3(512), TG_LDS + TG_OUT, st, a);
-  if (splits > 1)
-    hipLaunchKernelGGL(tgemm_sum_kernel, dim3((unsigned)(tiles - whole) * 32), dim3(256), 0, st, a);
+  if (splits > 1) tgemm_sum_launch(a, tiles - whole, st);
   return (int)hipGetLastError();
 }
 

@@ -50,3 +50,16 @@ def test_parts_have_work():
                 s = tg.dgrad_splits(M, R, C)
                 pairs = R // 128
                 assert 1 <= s <= pairs and -(-pairs // -(-pairs // s)) == s
+
+
+@pytest.mark.parametrize("M", [1, 17, 200])
+def test_parts_hold_the_rows_that_there_are(M):
+    R, C, splits = 1536, 512, 4
+    dy, w = torch.randn(M, R, device=DEV).bfloat16(), torch.randn(R, C, device=DEV).bfloat16()
+    out = torch.empty(M, C, device=DEV, dtype=torch.bfloat16)
+    part = torch.full((splits, 2, 256, 256), 7.0, device=DEV)
+    tg.L.check(tg.L.lib().areal_tgemm_nn(tg.L.ptr(dy), tg.L.c_int64(R), tg.L.ptr(w), tg.L.c_int64(C), tg.L.ptr(out), tg.L.c_int64(C),
+                                         tg.L.ptr(part), tg.L.c_int(0), tg.L.c_int(splits), tg.L.c_int(M), tg.L.c_int(R),
+                                         tg.L.c_int(C), tg.L.stream_ptr()), "tgemm_nn")
+    assert bool((part[:, :, M:] == 7.0).all())  # a few rows' parts are a few rows: the others are most of the call's bytes
+    assert torch.equal(out, part[:, :, :M].sum(0).permute(1, 0, 2).reshape(M, C).bfloat16())  # (four parts: added in order)

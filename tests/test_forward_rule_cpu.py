@@ -20,3 +20,14 @@ def test_deep(M, K, N, own):
 ])
 def test_vocabulary(M, K, N, written, reduced):
     assert tg._forward_own(M, K, N) == written and tg._stats_own(M, K, N) == reduced
+
+
+@pytest.mark.parametrize("M,R,C,own", [(2, 28672, 2048, True), (10000, 8192, 1024, False), (3000, 28672, 4096, False),
+                                       (3000, 37888, 3584, True), (32768, 17920, 1536, True), (700, 1536, 8960, False),
+                                       (12000, 1536, 8960, True)])
+def test_input_gradients(M, R, C, own):
+    assert tg._dgrad_own(M, R, C) == own
+
+
+def test_few_rows_take_more_parts():
+    assert tg.dgrad_cost(2, 17920, 1536)[2] == 35 and tg.dgrad_cost(256, 17920, 1536)[2] == 28
