@@ -207,8 +207,8 @@ def merge_shard_stats(stats: torch.Tensor, group) -> Tuple[torch.Tensor, torch.T
     return m, (allst[:, 1] * f).sum(0), (allst[:, 2] * f).sum(0), allst[:, 3].sum(0)
 
 
-# Chunks whose rows go through the head at once where the logits are not written: their statistics take 3 / 32 of the bytes
-# that one chunk's logits would.
+# Chunks whose rows go through the head at once where the logits are not written: three fp32 numbers a row and 64 columns are
+# 3 / 32 of the bytes of those rows' logits, so 3 / 4 of one chunk's.
 STATS_CHUNKS = 8
 
 

@@ -129,10 +129,6 @@ def dgrad_cost(M: int, R: int, C: int) -> Tuple[float, int, int]:
     return _tile_plan(R // 128, -(-M // 256) * (C // 256), 0, min(256, -(-M // 32) * 32))
 
 
-def dgrad_splits(M: int, R: int, C: int) -> int:
-    return dgrad_cost(M, R, C)[2]
-
-
 def dgrad_supported(dy: torch.Tensor, w: torch.Tensor) -> bool:
     if not (dy.is_cuda and dy.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and dy.dim() == 2 and w.dim() == 2):
         return False

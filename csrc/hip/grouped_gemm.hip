@@ -128,7 +128,7 @@ __global__ __launch_bounds__(256) void grouped_gemm_nt_kernel(
 #pragma unroll
     for (int j = 0; j < 16; ++j) acc[t][j] = 0.f;
 
-  const int first = ROT ? k_start(e, rot, K / (64 * KH)) * (64 * KH) : 0;  // rot: gg_rot, at the launch
+  const int first = ROT ? k_start(e, rot, K / (64 * KH)) * (64 * KH) : 0;  // rot: at the launch
   load(first);
   for (int k0 = 0; k0 < K; k0 += 64 * KH) {
     __syncthreads();  // previous tile fully consumed

@@ -25,7 +25,8 @@
 //     different 16-byte slots. The DMA writes LDS linearly (wave base + lane x 16), so the swizzle sits on the per-lane
 //     SOURCE address and on the read address.
 //   * the product is computed transposed (B rows as the MFMA A operand): a lane ends up with 4 consecutive output
-//     columns of one row and stores 8 bytes.
+//     columns of one row. Results pass through the 32 KiB of LDS that the operand tiles leave free and leave as 16-byte pieces
+//     of whole 128-byte lines; the gated form, whose wave has half a line, stores 16 bytes a lane from the registers.
 //   * block id -> tile: contiguous id ranges per XCD (ids are dealt round-robin to the 8 XCDs), walked in bands of 4
 //     tile rows so that the blocks running together on an XCD share A and B panels in its L2.
 #include <stdlib.h>
@@ -1001,7 +1002,7 @@ static int tgemm_tn_launch(const void* A, long lda, const void* B, long ldb, voi
   if (items > 0x7fffffffl - 256) return -1;
   TGArgs a{(const bf16_t*)A, lda, (const bf16_t*)B, ldb, (bf16_t*)C, ldc, (const bf16_t*)bias, M, N, K,
            (M + 255) / 256, gated ? (N + 127) / 128 : (N + 255) / 256, part, whole, splits, chunk, nullptr, 0};
-  static bool attr_set = false;  // 128 KiB of dynamic LDS: above the default limit
+  static bool attr_set = false;  // 160 KiB of dynamic LDS, 128 the gated form: above the default limit
   if (!attr_set) {
     HIP_RET(hipFuncSetAttribute((const void*)tgemm_kernel<0, false, false>, hipFuncAttributeMaxDynamicSharedMemorySize, TG_LDS + TG_OUT));
     HIP_RET(hipFuncSetAttribute((const void*)tgemm_kernel<1, false, false>, hipFuncAttributeMaxDynamicSharedMemorySize, TG_LDS));

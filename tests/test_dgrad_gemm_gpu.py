@@ -47,7 +47,7 @@ def test_parts_have_work():
     for M in (1, 256, 700, 4096, 30000):
         for R in (128, 256, 1536, 17920, 151936):
             for C in (256, 1536, 8960):
-                s = tg.dgrad_splits(M, R, C)
+                s = tg.dgrad_cost(M, R, C)[2]
                 pairs = R // 128
                 assert 1 <= s <= pairs and -(-pairs // -(-pairs // s)) == s
 

@@ -3,15 +3,18 @@ import pytest
 import torch
 
 from areal_vllm_amd import ops
+from areal_vllm_amd.ops import train_gemm as tg
 
 DEV = "cuda:0"
 pytestmark = pytest.mark.gpu
 
 
-# one launch for all rows (V a multiple of 128); chunk by chunk where the gradient kernels do not take the shape; padded rows
-@pytest.mark.parametrize("T,V,chunk", [(1300, 2176, 512), (1024, 2176, 512), (700, 2056, 256), (700, 2055, 256), (300, 2176, 512)])
+# one launch for all rows (V a multiple of 128; from 8192 on both gradients are the own kernels', split over V); chunk by chunk where
+# they do not take the shape; padded rows
+@pytest.mark.parametrize("T,V,chunk", [(1300, 8320, 512), (600, 9088, 256), (1300, 2176, 512), (1024, 2176, 512), (700, 2056, 256), (700, 2055, 256), (300, 2176, 512)])
 def test_backward_of_several_chunks(T, V, chunk):
     H = 256
+    assert tg._dgrad_own(T, V, H) == (V >= 8192)
     g = torch.Generator(device=DEV).manual_seed(T + V)
     h = torch.randn(T, H, device=DEV, generator=g).bfloat16()
     w = (torch.randn(V, H, device=DEV, generator=g) / H ** 0.5).bfloat16()
