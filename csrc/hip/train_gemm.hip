@@ -117,8 +117,8 @@ typedef f32x4 tg_acc[4][2];     // [m tile][n tile] of one quadrant
 // own 4 KiB at a time, and leaves as whole 128-byte lines: 1510 -> 1346 us, streamed past the caches (nontemporal) 1299;
 // 8192 x 151936 from 1536 deep 3287 -> 2801 us (library: 1294 and 3002). The waits of the stream do not matter: with counts
 // raised by the stores in flight, so that no wait stands behind one, the times are the same.
-// What is left is power: the matrix cores are busy 73 % of the time at a clock of 1.76 GHz (2.4 nominal); bare 16x16x32
-// products of random numbers run at 1.97 PFLOP/s on the whole chip, 32x32x16 ones at 1.75.
+// What is left is power: the matrix cores are busy 65 to 86 % of the time in the large products, at clocks of 1.3 to 1.8 GHz (2.4
+// nominal); bare products of normal numbers reach 1.7 to 1.8 PFLOP/s on the whole chip with either instruction, of zeros 2.2 to 2.5.
 //
 // EPI 2 (LM head without a backward pass): the logits leave as three numbers a row and 64 columns - the largest logit z, the sum
 // of exp((z - largest) / temperature) and the same sum weighted with z, of logits rounded to bf16 - which tgemm_stats_kernel
@@ -595,8 +595,8 @@ __global__ __launch_bounds__(256) void tgemm_table_kernel(const int* __restrict_
 // 32 lanes, which the swizzle puts on different banks).
 //   A0 / A1 = dY columns [0, 64) / [64, 128) of both wave rows; B0 / B1 = X columns [0, 32) / [32, 64) of all four
 //   wave columns - as for the forward kernel, pieces are what one phase reads.
-// 16x16x32 products, not 32x32x16: the same rate on paper, but the kernel is limited by power and they need less of it
-// (17920 x 1536 over 32768 tokens: 1481 -> 1407 us).
+// 16x16x32 products, not 32x32x16: where all CUs are busy 5 % faster (17920 x 1536 over 32768 tokens: 1481 -> 1407 us); where half of
+// them idle up to 5 % slower, for twice the transposed reads of A (2560 x 2560 over 2000 tokens, 100 tiles: 45 -> 48).
 // A tile whose whole reduction falls to one workgroup is added with a plain read-add-write. The tiles that would leave CUs
 // idle in a last round are reduced by several workgroups, `chunk` 128-token pairs each, that write their sums as fp32 to
 // `part`; tgemm_wgrad_sum_kernel adds them. fp32 atomics on the gradient instead execute at the memory side, 1.3 TB/s
