@@ -116,12 +116,23 @@ def moe_topk(logits: torch.Tensor, k: int, norm: bool, out_dtype=torch.float32):
     return topv, topi
 
 
+# Where a router's product in partial sums pays: few experts of few columns, whose tiles are few. us of the library's product / of
+# partial sums, each with the top-k, cold weights, 16 / 128 / 512 rows: 32 experts, 2048 deep 11.9 / 9.0, 12.4 / 9.4, 12.7 / 10.4; 128,
+# 2048 deep 12.6 / 10.7, 12.8 / 11.5, 13.3 / 12.8; 128, 4096 deep 15.6 / 12.1, 16.2 / 13.8, 16.5 / 17.1; 64, 7168 deep 12.2 / 10.9, 12.6 /
+# 12.4, 13.0 / 14.4; but 128, 7168 deep 12.9 / 14.0, 14.0 / 15.3, 14.6 / 20.2; 256, 2048 deep 13.8 / 14.1, 13.9 / 14.9, 14.6 / 16.9; 512,
+# 4096 deep 21.7 / 26.0, 22.0 / 27.3, 20.3 / 34.6.
+ROUTE_MAX_EXPERTS, ROUTE_MAX_SIZE, ROUTE_MAX_SIZE_MANY_ROWS = 160, 1 << 19, 9 << 15
+
+
+def _route_in_parts(T: int, E: int, H: int) -> bool:
+    return 0 < T <= dg.MAX_ROWS and E <= ROUTE_MAX_EXPERTS and E * H <= (ROUTE_MAX_SIZE if T <= 128 else ROUTE_MAX_SIZE_MANY_ROWS)
+
+
 def moe_route(x: torch.Tensor, router: torch.Tensor, k: int, norm: bool, out_dtype=torch.float32):
     """`moe_topk` of the router's projection x [T, H] @ router [E, H]^T (rounded to x's dtype). A decode batch's projection is a
-    few tiles: split over the depth to fill the chip, its fp32 partial products are summed by the top-k kernel itself (128 experts,
-    2048 deep, cold weights, 1 / 64 / 512 rows: 15.3 / 15.4 / 15.4 -> 9.2 / 11.0 / 13.0 us with the library's product before)."""
+    few tiles: split over the depth to fill the chip, its fp32 partial products are summed by the top-k kernel itself."""
     T, E = x.shape[0], router.shape[0]
-    if not (x.is_cuda and T > 0 and dg.serves(x, router) and E <= 512 and k <= min(64, E)
+    if not (x.is_cuda and _route_in_parts(T, E, x.shape[1]) and dg.serves(x, router) and k <= min(64, E)
             and out_dtype in (torch.float32, torch.bfloat16)):
         return moe_topk(F.linear(x, router), k, norm, out_dtype)
     slab = dg.dgemm(x, router, epilogue=dg.EPI_SLAB)

@@ -6,6 +6,7 @@ import pytest
 from areal_vllm_amd import ops  # noqa: F401
 
 G = sys.modules["areal_vllm_amd.ops.grouped_gemm"]
+M = sys.modules["areal_vllm_amd.ops.moe"]
 
 
 @pytest.mark.parametrize("T,E,N,K,out,dx,dw", [
@@ -25,3 +26,10 @@ def test_rule(T, E, N, K, out, dx, dw, monkeypatch):
     assert got == (out, dx, dw)
     monkeypatch.delenv("AREAL_GROUPED_GEMM_TILE_M")
     assert not G._big_wgrad(T, E, N, K, [9 * T // E])  # behind a crowded expert
+
+
+@pytest.mark.parametrize("T,E,H,parts", [(64, 128, 2048, True), (512, 128, 2048, True), (128, 128, 4096, True),
+                                         (129, 128, 4096, False), (16, 128, 7168, False), (1, 256, 1024, False),
+                                         (512, 32, 7168, True), (513, 32, 1024, False), (0, 32, 1024, False)])
+def test_router(T, E, H, parts):
+    assert M._route_in_parts(T, E, H) == parts
