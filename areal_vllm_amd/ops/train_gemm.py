@@ -170,6 +170,7 @@ def tgemm_nn(dy: torch.Tensor, w: torch.Tensor, splits: int = 0, out: Optional[t
 DGRAD_MIN_DEPTH, DGRAD_MIN_TILES, DGRAD_MAX_LOSS, DGRAD_MAX_ROUND_LOSS = 8192, 192, 1.6, 1.25
 
 
+@functools.lru_cache(maxsize=1024)
 def _dgrad_own(M: int, R: int, C: int) -> bool:
     tiles = -(-M // 256) * (C // 256)
     if R >= DGRAD_MIN_DEPTH:
@@ -210,9 +211,9 @@ def _forward_own(M: int, K: int, N: int) -> bool:
 
 # Logits that are reduced, not written, us of that form / of the library's product and the pass over its logits: 151936 columns, 896
 # to 5120 deep, 600 to 8192 rows 0.75 to 1.02 of its time, 65536 columns, 896 / 2048 deep 0.87 to 0.98 / 0.95 to 1.04; 3584 and 4096
-# deep 1.00 to 1.12, with 100352 columns 0.90 to 1.08.
+# deep 1.00 to 1.12, with 100352 columns 0.90 to 1.08; 151936 of them 4096 deep, 4000 / 8192 / 13019 rows 1.00 / 1.02 / 1.04.
 def _stats_own(M: int, K: int, N: int) -> bool:
-    return N >= 65536 and M >= 600 and (N >= 98304 or K <= 3072)
+    return N >= 65536 and M >= 600 and (K <= 3072 or N >= 98304 and (M <= 4096 or K <= 3584 or K >= 4608))
 
 
 def plain(*tensors: torch.Tensor) -> bool:
