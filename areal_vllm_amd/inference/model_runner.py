@@ -653,7 +653,7 @@ class ModelRunner:
         x, residual = ops.rmsnorm(h, layers[0].ln1, eps, None, gemma)
         for li, blk in enumerate(layers):
             kc, vc = self.kv[li]
-            if self.fused_qkv_rope and Bp >= dg.QKV_ROPE_MIN_ROWS:
+            if self.fused_qkv_rope and Bp >= dg.QKV_ROPE_MIN_ROWS and H <= dg.QKV_ROPE_MAX_DEPTH:
                 q = dg.dgemm_qkv_rope(x, blk.attn.qkv, blk.attn.qkv_bias, rope_pos, st["slots"], self.rope, kc, vc,
                                       hq, hkv, D)
             else:

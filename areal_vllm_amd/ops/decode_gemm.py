@@ -13,6 +13,7 @@ SGLang's CUDA kernels (``areal/api/cli_args.py:398-454``).
 CPU tensors take PyTorch paths with the same rounding points, so the engine's control flow is testable
 without a GPU.
 """
+from functools import lru_cache
 from typing import Optional, Tuple
 
 import torch
@@ -60,11 +61,11 @@ def valid_ksplit(K: int, ksplit: int) -> int:
 
 
 def pick_config(M: int, N: int, K: int, epilogue: int) -> Tuple[int, int, int, int, bool]:
-    """-> (cfg, stages, ksplit, loader_waves, nt), from the sweep on MI355X (``tools/dgemm_probe.py``, kept in
-    ``profiles/dgemm_probe_qwen2-1.5b_s2.log``): what a block waits for is its CU's load path (~40 GB/s per CU
-    measured), so small-N layers take small tiles and as many K splits as fill the chip once, wide layers take
-    tiles as tall as the batch; four LDS stages where they fit; dedicated loader waves and non-temporal weight
-    loads are worth 3-8 % except on the widest tiles."""
+    """-> (cfg, stages, ksplit, loader_waves, nt) of the tiled kernel, from the sweep on MI355X (``tools/dgemm_probe.py``,
+    kept in ``profiles/dgemm_probe_qwen2-1.5b_s2.log``): small-N layers take small tiles and as many K splits as fill the
+    chip once, wide layers tiles as tall as the batch; four LDS stages where they fit; dedicated loader waves and
+    non-temporal weight loads are worth 3-8 % except on the widest tiles. Partial sums take it only where their operands
+    are not 16-byte aligned (`slab_plan` otherwise)."""
     override = _OVERRIDES.get((M, N, K, epilogue))
     if override is not None:
         return override
@@ -101,6 +102,32 @@ def pick_config(M: int, N: int, K: int, epilogue: int) -> Tuple[int, int, int, i
 _OVERRIDES = {}
 
 
+@lru_cache(maxsize=4096)
+def slab_plan(M: int, N: int, K: int) -> Tuple[int, int, int]:
+    """-> (32-column tiles a workgroup, row blocks, splits of the reduction) of a product into partial sums: the least of
+    a workgroup's 64-deep steps x (46 ns for each 32 rows and each 32 columns that it stages, 5.6 for each pair of them
+    that it multiplies, 46 for the step) x rounds of 256 workgroups, and 0.45 us for each MB of partial sums, written here
+    and read by the row kernel behind (0.15 of it). Fitted to 6500 launches (13 layers of 896 to 5120 columns, 896 to
+    18944 deep, 8 to 512 rows); its choice is 1.2 % behind the best of them in the mean, 10 % at worst."""
+    steps = K // 64
+    best = None
+    for mblocks in range(-(-M // 256), -(-M // 32) + 1):
+        rt = -(-(-(-M // mblocks)) // 32)
+        if mblocks > 1 and (mblocks - 1) * rt * 32 >= M:
+            continue  # a row block of no rows
+        for ct in range(1, 6):
+            tiles = -(-N // (32 * ct)) * mblocks
+            for ksplit in range(1, max(1, min(24, N_CU // tiles, steps)) + 1):
+                per = -(-steps // ksplit)
+                if per * (ksplit - 1) >= steps:
+                    continue  # a split of no steps
+                rounds = -(-tiles * ksplit // N_CU)
+                cost = rounds * per * (46 * (rt + ct) + 5.6 * rt * ct + 46) + 450 * ksplit * M * N * 4e-6
+                if best is None or cost < best[0]:
+                    best = (cost, ct, mblocks, ksplit)
+    return best[1:]
+
+
 MAX_ROWS = 512  # rows of a decode batch the kernels are laid out for
 
 
@@ -120,7 +147,12 @@ def dgemm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,
     M, K = x.shape
     N = w.shape[0]
     assert w.shape[1] == K
-    if cfg is None:
+    plan = None
+    if (epilogue == EPI_SLAB and (cfg, stages, ksplit, loader_waves, nt) == (None,) * 5
+            and all(t is None or t.data_ptr() % 16 == 0 for t in (x, w, out))):
+        plan = slab_plan(M, N, K) if M > 0 and N > 0 and K >= 64 else (1, 1, 1)
+        cfg, ksplit = 8, plan[2]
+    elif cfg is None:
         c, s, k, lw_, nt_ = pick_config(M, N, K, epilogue)
         cfg = c
         stages = s if stages is None else stages
@@ -159,6 +191,11 @@ def dgemm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,
     if epilogue == EPI_SLAB:
         assert out.dtype == torch.float32 and out.is_contiguous() and out.numel() >= ksplit * M * N
         ys = N
+        if plan is not None:
+            L.check(L.lib().areal_dtile_slab(L.ptr(x), L.c_int64(x.stride(0)), L.ptr(w), L.ptr(out), L.c_int(M), L.c_int(N),
+                                             L.c_int(K), L.c_int(plan[0]), L.c_int(plan[1]), L.c_int(plan[2]), L.c_int(4),
+                                             L.c_int(1), L.stream_ptr()), "dgemm")
+            return out
     else:
         assert out.stride(1) == 1
         ys = out.stride(0)
@@ -168,20 +205,25 @@ def dgemm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,
     return out
 
 
+@lru_cache(maxsize=4096)
 def swiglu_plan(M: int, F: int) -> Optional[Tuple[int, int]]:
     """-> (columns per workgroup, row blocks) of the balanced gate|up kernel for M rows and F gate columns, or None
-    where it has no instantiation. A workgroup stages (rows per block + 2 x columns) rows of K elements and the launch
-    takes about 7 us + 0.065 us per staged row at K = 1536 (``profiles/swiglu_probe_s1.log``), so with row blocks x
-    column ranges fixed at the number of CUs the best split has about twice as many block rows as columns: two row
-    blocks from 129 rows on, ranges as narrow as fill the chip (a multiple of 4, at most 80 columns)."""
+    where it has no instantiation. With row blocks x column ranges fixed at the number of CUs a workgroup's time is that
+    of what it stages and multiplies (`slab_plan`): row blocks of 32-row multiples, ranges as narrow as fill the chip (a
+    multiple of 4, at most 80 columns)."""
     if M > 512 or F % 4 != 0:
         return None
-    for mblocks in ((2, 1) if 128 < M <= 256 else ((1,) if M <= 128 else (2,))):
-        target = max(1, N_CU // mblocks)
-        w = (-(-F // target) + 3) // 4 * 4
-        if w <= 80:
-            return w, mblocks
-    return None
+    M, best = max(M, 1), None
+    for mblocks in range(-(-M // 256), 5):
+        rt = -(-(-(-M // mblocks)) // 32)
+        w = (-(-F // (N_CU // mblocks)) + 3) // 4 * 4
+        if w > 80 or (mblocks > 1 and (mblocks - 1) * rt * 32 >= M):
+            continue
+        ct = -(-w // 16)
+        cost = 46 * (rt + ct) + 5.6 * rt * ct
+        if best is None or cost < best[0]:
+            best = (cost, w, mblocks)
+    return None if best is None else best[1:]
 
 
 def dgemm_swiglu_balanced(x: torch.Tensor, w_gate_up: torch.Tensor, out: Optional[torch.Tensor] = None, *,
@@ -295,11 +337,11 @@ def splitk_rope_cache_write(slab: torch.Tensor, n_split: int, bias: Optional[tor
 # (cfg, stages, loader_waves, nt) of the fused qkv projection by batch rows, from ``tools/dgemm_probe.py --layers qkv_rope``
 # (profiles/dgemm_probe_qkv_rope_s12.log): 32-row tiles up to 256 rows, 64-row tiles above; four dedicated loader waves
 QKV_ROPE_CONFIG = {"small": (9, 4, 4, True), "large": (8, 4, 4, True)}
-# Below this many rows the split-K GEMM + row kernel pair is as fast or faster: a block of the fused kernel walks
-# all of K (24 steps of ~0.4 us at K = 1536), split-K blocks an eighth of it. Stand-alone 12.1 vs 14.0 us at 256
-# rows and 13.5 vs 17.1 us at 384; inside the captured decode step the difference is within noise at 256 rows
-# and 1 % of the step at 384 (profiles/decode_probe_fused_qkv_s12.log).
-QKV_ROPE_MIN_ROWS = 320
+# From so many rows on, and up to so deep, the one launch is level with or ahead of the split-K GEMM and its row kernel (captured, cold
+# weights, us of the one / the two): a block of it walks all of K, split-K blocks a part of it. 1536 deep to 2048 columns 320 / 384 /
+# 448 / 512 rows 15.7 / 13.7, 15.7 / 14.9, 16.1 / 15.8, 16.3 / 16.4; 896 deep to 1152 11.4 / 10.1, 11.5 / 10.6, 11.6 / 11.0, 11.7 /
+# 12.0; 2048 deep to 6144 at 512 rows 61 / 37, 3584 to 4608 61 / 35, 4096 to 6144 91 / 44.
+QKV_ROPE_MIN_ROWS, QKV_ROPE_MAX_DEPTH = 512, 1536
 
 
 def dgemm_qkv_rope(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], positions, slots, table, kcache,

@@ -1,24 +1,29 @@
-// gate|up projection of a decode step with the SwiGLU activation in its epilogue, decomposed so that EVERY CU of the
-// chip gets one workgroup:   Y[M, F] = silu(X W_gate^T) * (X W_up^T),  W = [gate; up] [2F, K],  M = 64 ... 512 rows.
+// Decode-batch GEMMs for gfx950 on 16-wide tiles, with the fragments of the next half step requested while the present one is
+// multiplied: Y = X W^T for M = 1 ... 512 rows, either the gated-MLP projection with its activation in the epilogue
+//     Y[M, F] = act(X W_gate^T) * (X W_up^T),  W = [gate; up] [2F, K]
+// or fp32 partial sums of a reduction split over workgroups, Y [ksplit, M, N], summed in split order by the row kernel that follows
+// (decode_gemm.hip).
 //
-// What a workgroup of such a GEMM waits for is its CU's load path (every workgroup stages all of its activation rows
-// through L2 besides its share of the weights), so the time of the launch is the time of the busiest CU. Tiles of
-// 32-column multiples leave CUs idle for the common layer widths (Qwen2-1.5B: F = 8960 = 140 x 64 -> 140 workgroups of
-// the 256-row x 128-column kernel in decode_gemm.hip on 256 CUs). Here a workgroup owns a column range of ANY width
-// w (a multiple of 4, up to 16 TW): F / w ranges, chosen by the caller so that ranges x row blocks ~ number of CUs
-// (F = 8960: w = 36 -> 249 workgroups). The MFMA tiles are 16 columns wide (v_mfma_f32_16x16x32_bf16), so a range is
-// computed as ceil(w / 16) tiles with the surplus columns fed from clamped (repeated) weight rows and never stored:
-// matrix-pipe time is not what this shape waits for.
+// What bounds these products is, in this order:
+//   * the CU's load path. Loads return in order through a buffer of 32 to 64 KB: 23 GB/s a CU for bytes that come from HBM (all CUs
+//     together 6 TB/s), 100 to 110 for bytes that are in the XCD's L2, 42 where the two alternate one to one and 57 one to three. A
+//     workgroup stages (rows + weight rows) x K, so its rows are padded to 32 only (320 rows are two blocks of 160, not of 192) and
+//     its column range has ANY width (a multiple of 4; F = 8960: 72 of 125 ranges), which gives every CU one workgroup;
+//   * the matrix pipe, and LDS reads that block their wave's issue until the LDS has taken them. 2 x 2 waves, each on 16 RT rows
+//     and 16 CT weight rows, read RT + CT fragments for RT x CT products (a quarter of the rows and all columns, as before: 13 reads
+//     for 30 products at 192 x 72, now 10 for 25), and the reads of the next 32 deep are dealt out between the products of the
+//     present ones. 64 deep at 160 x (72 + 72): 2500 cycles before; now 1125 from LDS alone, 1590 with weights from HBM.
+// Captured, cold weights, us before / now: gate|up of 8960 columns, 1536 deep, 24 / 93 / 320 / 512 rows 12.8 / 12.0, 17.5 / 16.3, 29.1 /
+// 24.6, 35.3 / 31.2; 14336, 4096 deep, 200 rows 71.7 / 57.3; partial sums (on decode_gemm.hip's tiles before) of 1536 columns, 8960 deep,
+// 24 / 93 / 320 rows 8.2 / 7.3, 10.7 / 9.7, 21.3 / 17.4; 2048, 1536 deep 4.5 / 4.0, 5.7 / 5.2, 9.7 / 7.4; 5120, 13824 deep 29.9 / 24.9, 41.7 /
+// 30.3, 76.4 / 50.6; 6144, 4096 deep 16.0 / 10.7, 19.8 / 13.7, 44.3 / 25.1. Faster at all of 156 and 97 sizes measured.
 //
-//   * 4 consumer waves (one per SIMD): wave v owns activation rows [16 RT v, 16 RT (v + 1)) of the block and all 2 TW
-//     column tiles (TW gate tiles and the matching TW up tiles, so SwiGLU stays inside a lane);
-//   * 4 loader waves issue the LDS-DMA pieces (global_load_lds_dwordx4, 8 rows x 128 B each) of STAGES-deep staging,
-//     one raw s_barrier per 64-deep K step, counted vmcnt so that STAGES - 2 tiles stay in flight across it; the XOR
-//     swizzle that makes the ds_read_b128 fragment reads conflict-free sits on the per-lane SOURCE address;
-//   * product transposed (A = weight rows, B = activation rows): a lane ends up with 4 consecutive output columns of
-//     one row -> 8-byte bf16 stores;
-//   * with two row blocks (M > 256) the two workgroups that stream the same weight columns get block ids 8 apart, i.e.
-//     the same XCD under round-robin placement: the second reader is served by that XCD's L2 (speed only).
+//   * waves 4..7 do nothing but issue the LDS-DMA pieces (global_load_lds_dwordx4, 8 rows x 128 B each) of a ring of stages, one raw
+//     s_barrier per 64-deep step, counted vmcnt so that the later stages stay in flight across it; the XOR swizzle that makes the
+//     ds_read_b128 fragment reads conflict-free sits on the per-lane SOURCE address;
+//   * product transposed (A = weight rows, B = activation rows). A gated block's weight tiles hold two gate rows and the two matching
+//     up rows of every four, so that a lane has both factors of an output, and a pair of tiles gives it four columns in a row: an
+//     8-byte store. A wave's last tile of an odd number gives two columns.
 //
 // Role in the reference: the MLP GEMM + activation kernels of its serving engine (areal/api/cli_args.py:398-454).
 #include "common.hpp"
@@ -27,96 +32,173 @@ namespace {
 
 typedef const __attribute__((address_space(1))) void* gptr_t;
 typedef __attribute__((address_space(3))) void* lptr_t;
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
-struct SGArgs {
+enum { DT_GATED = 0, DT_SLAB = 1 };
+
+struct DTArgs {
   const bf16_t* X;
   long xs;
   const bf16_t* W;
-  bf16_t* Y;
+  void* Y;
   long ys;
-  int M, F, K;
-  int w;        // columns per range (multiple of 4)
-  int ntiles;   // ceil(F / w)
-  int mblocks;  // row blocks (1 or 2)
-  int nt;       // non-temporal weight loads
-  int act;      // gate activation: 0 SiLU (SwiGLU), 1 tanh-approximated GELU (GeGLU)
-  int rot;      // range t starts its reduction at step t * rot and wraps round: k_rotation (common.hpp)
+  int M, N, K;   // N: output columns (gated: F)
+  int w;         // columns per range (multiple of 4)
+  int ntiles;    // ceil(N / w)
+  int mblocks;   // row blocks of 32 RT rows
+  int ksplit, steps;  // workgroups a reduction, 64-deep steps of each (the last one's may be fewer, not 0)
+  int stages;    // LDS ring
+  int nt;        // non-temporal weight loads
+  int act;       // gate activation: 0 SiLU (SwiGLU), 1 tanh-approximated GELU (GeGLU)
+  int rot;       // range t starts its reduction at step t * rot and wraps round: k_rotation (common.hpp)
 };
 
 template <int N>
-DEVINL void sg_wait_vmcnt() {
+DEVINL void dt_vmcnt() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
+// Wait until at most `keep` stages (IPW pieces of this wave each) that were issued after the one needed now are in flight.
 template <int IPW>
-DEVINL void sg_wait_tiles(int keep) {
-  constexpr int C = 63;
+DEVINL void dt_wait(int keep) {
+  constexpr int C = 63;  // largest count the instruction encodes; a smaller count only waits for more
   switch (keep) {
-    case 0: sg_wait_vmcnt<0>(); break;
-    case 1: sg_wait_vmcnt<(IPW < C ? IPW : C)>(); break;
-    default: sg_wait_vmcnt<(2 * IPW < C ? 2 * IPW : C)>(); break;
+    case 0: dt_vmcnt<0>(); break;
+    case 1: dt_vmcnt<(IPW < C ? IPW : C)>(); break;
+    case 2: dt_vmcnt<(2 * IPW < C ? 2 * IPW : C)>(); break;
+    case 3: dt_vmcnt<(3 * IPW < C ? 3 * IPW : C)>(); break;
+    default: dt_vmcnt<(4 * IPW < C ? 4 * IPW : C)>(); break;
   }
 }
 
-DEVINL float sg_silu(float x) { return x / (1.f + __expf(-x)); }
-DEVINL float sg_gate(float x, int act) {
-  if (act == 0) return sg_silu(x);
+// x / (1 + exp(-x)), correctly rounded quotient (train_gemm.hip's tg_silu: a Newton step on the quotient behind v_rcp_f32).
+DEVINL float dt_silu(float g) {
+  const float a = 0.25f * g, d = fmaf(0.25f, __expf(-g), 0.25f);
+  const float y = __builtin_amdgcn_rcpf(d), q = a * y;
+  return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-d, q, a), y, q), d, a);
+}
+template <bool GELU>
+DEVINL float dt_gate(float x) {
+  if (!GELU) return dt_silu(x);
   const float inner = 0.7978845608028654f * (x + 0.044715f * x * x * x);
   const float e = __expf(-2.f * fabsf(inner));
   return 0.5f * x * (1.f + copysignf((1.f - e) / (1.f + e), inner));
 }
 
-// RT: 16-row activation tiles per consumer wave (block rows BM = 64 RT); TW: 16-column tiles per half (gate / up).
-template <int RT, int TW, int STAGES, bool ROT>
-__global__ __launch_bounds__(512) void dswiglu_kernel(const SGArgs a) {
-  constexpr int BM = 64 * RT, HW = 16 * TW, WR = 2 * HW;  // weight rows of a stage: HW gate + HW up
-  constexpr int NP = (WR + BM) / 8, IPW = NP / 4;          // 1-KiB pieces per stage, per loader wave
-  static_assert(NP % 4 == 0, "pieces divide evenly over the four loader waves");
-  constexpr int STAGE_BYTES = (WR + BM) * 128;
+// LDS reads may not cross this barrier; the builtin's wait tells the compiler that nothing is outstanding behind it (its own count
+// would merge the loop's two read groups and wait for both before the first product).
+DEVINL void dt_lds_done() { __builtin_amdgcn_s_waitcnt(0xC07F); }  // lgkmcnt(0)
+DEVINL void dt_barrier() {
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+template <int RT, int CT>
+struct DTFrag {
+  bf16x8 x[RT], w[CT];
+  DEVINL void read(const char* xp, const char* wp) {
+#pragma unroll
+    for (int r = 0; r < RT; ++r) x[r] = *reinterpret_cast<const bf16x8*>(xp + r * 2048);
+#pragma unroll
+    for (int c = 0; c < CT; ++c) w[c] = *reinterpret_cast<const bf16x8*>(wp + c * 2048);
+  }
+  DEVINL void multiply(f32x4 (&acc)[CT][RT]) const {
+#pragma unroll
+    for (int c = 0; c < CT; ++c)
+#pragma unroll
+      for (int r = 0; r < RT; ++r) acc[c][r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[c], x[r], acc[c][r], 0, 0, 0);
+  }
+};
+
+// The reads since the last sched_barrier, dealt out between the products since then.
+template <int RT, int CT, int ID>
+DEVINL void dt_deal() {
+  constexpr int PER = (CT * RT) / (CT + RT) > 0 ? (CT * RT) / (CT + RT) : 1;
+#pragma unroll
+  for (int i = 0; i < CT + RT; ++i) {
+    __builtin_amdgcn_sched_group_barrier(0x100, 1, ID);
+    __builtin_amdgcn_sched_group_barrier(0x8, PER, ID);
+  }
+  __builtin_amdgcn_sched_group_barrier(0x8, CT * RT, ID);
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// A wave's gated outputs: rows m + 16 r, columns from nb on, below c1. All of a row's values are computed before the first store: in
+// the branches of the stores, four at a time and with the compiler's division, 50 outputs a lane took 8500 cycles; now 5060.
+template <int RT, int CT, bool GELU>
+DEVINL void dt_store_gated(const DTArgs& a, const f32x4 (&acc)[CT][RT], int m, int nb, int c1, int q) {
+#pragma unroll
+  for (int r = 0; r < RT; ++r) {
+    bf16x2 o[CT];
+#pragma unroll
+    for (int c = 0; c < CT; ++c)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)  // gate / up rounded to bf16 first: the values an unfused bf16 GEMM output would carry
+        o[c][j] = f2bf(dt_gate<GELU>(bf2f(f2bf(acc[c][r][j]))) * bf2f(f2bf(acc[c][r][2 + j])));
+    if (m + 16 * r >= a.M) continue;
+    bf16_t* y = (bf16_t*)a.Y + (size_t)(m + 16 * r) * a.ys;
+#pragma unroll
+    for (int p = 0; p < CT / 2; ++p) {
+      const int n = nb + 16 * p + 4 * q;  // ranges and this wave's part start at multiples of 4: the four columns are inside together
+      if (n < c1) *reinterpret_cast<bf16x4*>(y + n) = bf16x4{o[2 * p][0], o[2 * p][1], o[2 * p + 1][0], o[2 * p + 1][1]};
+    }
+    if constexpr (CT & 1) {
+      const int n = nb + 8 * (CT - 1) + 2 * q;
+      if (n < c1) *reinterpret_cast<bf16x2*>(y + n) = o[CT - 1];
+    }
+  }
+}
+
+template <int RT, int CT, int EPI, bool ROT>
+__global__ __launch_bounds__(512) void dtile_kernel(const DTArgs a) {
+  constexpr int BM = 32 * RT, WR = 32 * CT;  // activation rows and weight rows of a stage
+  constexpr int IPW = RT + CT;               // 1-KiB pieces per stage and loader wave
+  constexpr int STAGE_BYTES = (BM + WR) * 128;
+  // both halves' fragments beside the accumulators of large tiles exceed the 256 registers of a wave
+  constexpr bool AHEAD = 4 * RT * CT + 8 * (RT + CT) <= 224;
   extern __shared__ __attribute__((aligned(16))) char smem[];
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const bool is_loader = wave >= 4;
-  const int lwave = wave - 4;
-
-  // block id -> (column range, row block); the row blocks of one range are 8 ids apart
-  int tile, mb;
+  // Ids are dealt round-robin to the 8 XCDs: each XCD takes a contiguous range, row blocks first, then column ranges, then splits, so
+  // that a weight range's row blocks meet in one L2 and a slice of X is fetched by one or two of them.
+  int tile, mb, sp;
   {
-    const int id = blockIdx.x;
-    if (a.mblocks == 1) {
-      tile = id;
-      mb = 0;
-    } else {
-      const int x = id & 7, slot = id >> 3;
-      mb = slot % a.mblocks;
-      tile = (slot / a.mblocks) * 8 + x;
-    }
+    const int nb = gridDim.x, q = nb >> 3, r = nb & 7, x = blockIdx.x & 7;
+    const int pos = (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + (blockIdx.x >> 3);
+    const int rest = pos / a.mblocks;
+    mb = pos - rest * a.mblocks;
+    sp = rest / a.ntiles;
+    tile = rest - sp * a.ntiles;
   }
-  if (tile >= a.ntiles) return;
   const int c0 = tile * a.w;
-  const int c1 = min(a.F, c0 + a.w);
+  const int c1 = min(a.N, c0 + a.w);
   const int m0 = mb * BM;
-  const int nsteps = a.K >> 6;
+  const int k0 = sp * a.steps * 64;
+  const int nsteps = min(a.steps, (a.K >> 6) - sp * a.steps);
+  const int stages = a.stages;
 
-  if (is_loader) {
-    // ---- staging: piece i of a stage = LDS rows 8i .. 8i+7 (gate rows, up rows, activation rows)
+  if (wave >= 4) {
+    // ---- staging: piece i of a stage = LDS rows 8i .. 8i+7 (weight rows, then activation rows); this wave has every fourth
+    const int lw = wave - 4;
     const bf16_t* src[IPW];
 #pragma unroll
     for (int j = 0; j < IPW; ++j) {
-      const int i = lwave * IPW + j;
-      const int row = 8 * i + (lane >> 3);
+      const int row = 8 * (lw + 4 * j) + (lane >> 3);
       const int c = (lane & 7) ^ ((row >> 1) & 7);  // logical 16-byte chunk stored at physical chunk lane&7
-      if (8 * i < WR) {
-        const int half = row >= HW ? 1 : 0;
-        int col = c0 + (row - half * HW);
-        col = col < c1 ? col : c1 - 1;  // surplus columns of the last 16-wide tile repeat the last real one
-        src[j] = a.W + ((size_t)half * a.F + col) * a.K + 8 * c;
+      if (j < CT) {
+        size_t n;  // surplus rows of the last tiles repeat the range's last column
+        if (EPI == DT_GATED) {
+          const int t = row >> 4, i = row & 3, q = (row & 15) >> 2, wn = t / CT, ct = t % CT;
+          int col = wn * CT * 8 + 8 * (ct & ~1) + (i & 1);
+          col += (CT & 1) && ct == CT - 1 ? 2 * q : 4 * q + 2 * (ct & 1);
+          n = (size_t)(i >> 1) * a.N + min(c0 + col, c1 - 1);
+        } else {
+          n = min(c0 + row, c1 - 1);
+        }
+        src[j] = a.W + n * a.K + k0 + 8 * c;
       } else {
-        int m = m0 + row - WR;
-        m = m < a.M ? m : a.M - 1;
-        src[j] = a.X + (size_t)m * a.xs + 8 * c;
+        const int m = min(m0 + row - WR, a.M - 1);
+        src[j] = a.X + (size_t)m * a.xs + k0 + 8 * c;
       }
     }
     const int rot = ROT ? k_start(tile, a.rot, nsteps) : 0;
@@ -125,143 +207,184 @@ __global__ __launch_bounds__(512) void dswiglu_kernel(const SGArgs a) {
         step += rot;
         step -= step >= nsteps ? nsteps : 0;
       }
-      char* base = smem + buf * STAGE_BYTES + lwave * (IPW * 1024);
+      char* base = smem + buf * STAGE_BYTES + lw * 1024;
 #pragma unroll
       for (int j = 0; j < IPW; ++j) {
-        if (a.nt && 8 * (lwave * IPW + j) < WR)
-          __builtin_amdgcn_global_load_lds((gptr_t)(src[j] + step * 64), (lptr_t)(base + j * 1024), 16, 0, 2);
+        if (j < CT && a.nt)
+          __builtin_amdgcn_global_load_lds((gptr_t)(src[j] + step * 64), (lptr_t)(base + j * 4096), 16, 0, 2);
         else
-          __builtin_amdgcn_global_load_lds((gptr_t)(src[j] + step * 64), (lptr_t)(base + j * 1024), 16, 0, 0);
+          __builtin_amdgcn_global_load_lds((gptr_t)(src[j] + step * 64), (lptr_t)(base + j * 4096), 16, 0, 0);
       }
     };
-#pragma unroll
-    for (int s = 0; s < STAGES - 1; ++s)
+    for (int s = 0; s < stages - 1; ++s)
       if (s < nsteps) issue(s, s);
+    int buf = stages - 1;
     for (int t = 0; t < nsteps; ++t) {
-      const int ahead = nsteps - 1 - t;
-      constexpr int KEEP = STAGES - 2 < 2 ? STAGES - 2 : 2;
-      sg_wait_tiles<IPW>(ahead < KEEP ? ahead : KEEP);
-      __builtin_amdgcn_s_barrier();
-      if (t + STAGES - 1 < nsteps) issue((t + STAGES - 1) % STAGES, t + STAGES - 1);
+      dt_wait<IPW>(min(nsteps - 1 - t, stages - 2));
+      __builtin_amdgcn_s_barrier();  // stage t is there, and every wave is done with stage t - 1
+      if (t + stages - 1 < nsteps) {
+        issue(buf, t + stages - 1);
+        buf = buf + 1 == stages ? 0 : buf + 1;
+      }
     }
     return;
   }
 
-  // ---- consumers
+  // ---- consumers: wave (wm, wn) owns rows [16 RT wm, + 16 RT) and weight rows [16 CT wn, + 16 CT) of the stage
+  const int wm = wave & 1, wn = wave >> 1;
   const int r16 = lane & 15, q = lane >> 4;
   const int key = (r16 >> 1) & 7;  // tile bases are multiples of 16 rows: the row's swizzle key is the lane's
-  int coff[2];
-#pragma unroll
-  for (int s = 0; s < 2; ++s) coff[s] = ((4 * s + q) ^ key) << 4;
-  const int wbase = r16 * 128;                                  // + tile * 2048
-  const int xbase = (WR + wave * 16 * RT + r16) * 128;           // + rt * 2048
+  const int co0 = (q ^ key) << 4, co1 = ((4 + q) ^ key) << 4;
+  const int wb = (wn * CT * 16 + r16) * 128, xb = (WR + wm * RT * 16 + r16) * 128;
 
-  f32x4_t acc[2 * TW][RT];
+  f32x4 acc[CT][RT];
 #pragma unroll
-  for (int t = 0; t < 2 * TW; ++t)
+  for (int c = 0; c < CT; ++c)
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt) acc[t][rt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int r = 0; r < RT; ++r) acc[c][r] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  for (int t = 0; t < nsteps; ++t) {
-    __builtin_amdgcn_s_barrier();
-    const char* sb = smem + (t % STAGES) * STAGE_BYTES;
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      bf16x8 wf[2 * TW], xf[RT];
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt) xf[rt] = *reinterpret_cast<const bf16x8*>(sb + xbase + rt * 2048 + coff[s]);
-#pragma unroll
-      for (int ct = 0; ct < 2 * TW; ++ct) wf[ct] = *reinterpret_cast<const bf16x8*>(sb + wbase + ct * 2048 + coff[s]);
-#pragma unroll
-      for (int ct = 0; ct < 2 * TW; ++ct)
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt)
-          acc[ct][rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[ct], xf[rt], acc[ct][rt], 0, 0, 0);
+  const char* sb = smem;
+  int buf = 0;
+  if constexpr (AHEAD) {
+    DTFrag<RT, CT> fa, fb;
+    dt_barrier();
+    fa.read(sb + xb + co0, sb + wb + co0);
+    for (int t = 0; t + 1 < nsteps; ++t) {
+      dt_lds_done();
+      fb.read(sb + xb + co1, sb + wb + co1);
+      fa.multiply(acc);
+      dt_deal<RT, CT, 0>();
+      dt_lds_done();  // every read of this stage has returned before any wave may restage it
+      dt_barrier();
+      buf = buf + 1 == stages ? 0 : buf + 1;
+      sb = smem + buf * STAGE_BYTES;
+      fa.read(sb + xb + co0, sb + wb + co0);
+      fb.multiply(acc);
+      dt_deal<RT, CT, 1>();
     }
-    // every fragment read of this buffer has returned before any wave may restage it
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    fb.read(sb + xb + co1, sb + wb + co1);
+    fa.multiply(acc);
+    fb.multiply(acc);
+  } else {
+    for (int t = 0; t < nsteps; ++t) {
+      dt_barrier();
+      DTFrag<RT, CT> f;
+      f.read(sb + xb + co0, sb + wb + co0);
+      f.multiply(acc);
+      f.read(sb + xb + co1, sb + wb + co1);
+      f.multiply(acc);
+      dt_lds_done();
+      buf = buf + 1 == stages ? 0 : buf + 1;
+      sb = smem + buf * STAGE_BYTES;
+    }
   }
 
-  // ---- epilogue. acc[ct][rt][i]: activation row m0 + (wave RT + rt) 16 + r16, column c0 + 16 (ct % TW) + 4 q + i
+  // ---- epilogue. acc[c][r][i]: activation row m, weight row 4 q + i of tile c
+  if constexpr (EPI == DT_GATED) {
+    if (a.act == 0) dt_store_gated<RT, CT, false>(a, acc, m0 + wm * RT * 16 + r16, c0 + wn * CT * 8, c1, q);
+    else dt_store_gated<RT, CT, true>(a, acc, m0 + wm * RT * 16 + r16, c0 + wn * CT * 8, c1, q);
+  } else {
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt) {
-    const int m = m0 + (wave * RT + rt) * 16 + r16;
-    if (m >= a.M) continue;
-    bf16_t* yrow = a.Y + (size_t)m * a.ys;
+    for (int r = 0; r < RT; ++r) {
+      const int m = m0 + (wm * RT + r) * 16 + r16;
+      if (m >= a.M) continue;
+      float* y = (float*)a.Y + ((size_t)sp * a.M + m) * a.ys;
 #pragma unroll
-    for (int ct = 0; ct < TW; ++ct) {
-      const int n = c0 + 16 * ct + 4 * q;
-      if (n < c1) {  // ranges are multiples of 4 wide: the four columns are inside together
-        bf16x4 o;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          // gate / up rounded to bf16 first: the values an unfused bf16 GEMM output would carry
-          const float gg = bf2f(f2bf(acc[ct][rt][j])), uu = bf2f(f2bf(acc[ct + TW][rt][j]));
-          o[j] = f2bf(sg_gate(gg, a.act) * uu);
-        }
-        *reinterpret_cast<bf16x4*>(yrow + n) = o;
+      for (int c = 0; c < CT; ++c) {
+        const int n = c0 + (wn * CT + c) * 16 + 4 * q;
+        if (n < c1) *reinterpret_cast<f32x4*>(y + n) = acc[c][r];
       }
     }
   }
 }
 
-template <int RT, int TW, int STAGES, bool ROT>
-int sg_launch_as(const SGArgs& a, hipStream_t st) {
-  constexpr size_t lds = (size_t)STAGES * (32 * TW + 64 * RT) * 128;
-  static_assert(lds <= 160 * 1024, "staging exceeds the LDS of a CU");
-  auto kern = dswiglu_kernel<RT, TW, STAGES, ROT>;
-  static bool attr_set = false;  // per instantiation
-  if (!attr_set) {
-    HIP_RET(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    attr_set = true;
+template <int RT, int CT, int EPI, bool ROT>
+int dt_launch_as(DTArgs a, hipStream_t st) {
+  constexpr int stage_bytes = 32 * (RT + CT) * 128;
+  a.stages = max(2, min(a.stages, min(6, 160 * 1024 / stage_bytes)));
+  auto kern = dtile_kernel<RT, CT, EPI, ROT>;
+  if (a.stages * stage_bytes > 64 * 1024) {
+    static bool attr_set = false;  // per instantiation
+    if (!attr_set) {
+      HIP_RET(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 / stage_bytes * stage_bytes));
+      attr_set = true;
+    }
   }
-  const int groups = a.mblocks == 1 ? a.ntiles : ((a.ntiles + 7) / 8) * 8 * a.mblocks;
-  hipLaunchKernelGGL(kern, dim3(groups), dim3(512), lds, st, a);
+  hipLaunchKernelGGL(kern, dim3(a.ntiles * a.ksplit * a.mblocks), dim3(512), a.stages * stage_bytes, st, a);
   return (int)hipGetLastError();
 }
 
-template <int RT, int TW, int STAGES>
-int sg_launch(const SGArgs& a, hipStream_t st) {
-  return a.rot ? sg_launch_as<RT, TW, STAGES, true>(a, st) : sg_launch_as<RT, TW, STAGES, false>(a, st);
+template <int RT, int CT, int EPI>
+int dt_launch(const DTArgs& a, hipStream_t st) {
+  if constexpr (EPI == DT_GATED)
+    if (a.rot) return dt_launch_as<RT, CT, EPI, true>(a, st);
+  return dt_launch_as<RT, CT, EPI, false>(a, st);
 }
 
-template <int RT, int TW>
-int sg_stages(const SGArgs& a, int stages, hipStream_t st) {
-  constexpr int stage_bytes = (32 * TW + 64 * RT) * 128;
-  if (stages >= 4 && 4 * stage_bytes <= 160 * 1024) {
-    if constexpr (4 * stage_bytes <= 160 * 1024) return sg_launch<RT, TW, 4>(a, st);
+template <int RT, int EPI>
+int dt_cols(const DTArgs& a, int ct, hipStream_t st) {
+  switch (ct) {
+    case 1: return dt_launch<RT, 1, EPI>(a, st);
+    case 2: return dt_launch<RT, 2, EPI>(a, st);
+    case 3: return dt_launch<RT, 3, EPI>(a, st);
+    case 4: return dt_launch<RT, 4, EPI>(a, st);
+    case 5: return dt_launch<RT, 5, EPI>(a, st);
   }
-  if (stages >= 3 && 3 * stage_bytes <= 160 * 1024) {
-    if constexpr (3 * stage_bytes <= 160 * 1024) return sg_launch<RT, TW, 3>(a, st);
+  return -10;
+}
+
+template <int EPI>
+int dt_rows(const DTArgs& a, int rt, int ct, hipStream_t st) {
+  switch (rt) {
+    case 1: return dt_cols<1, EPI>(a, ct, st);
+    case 2: return dt_cols<2, EPI>(a, ct, st);
+    case 3: return dt_cols<3, EPI>(a, ct, st);
+    case 4: return dt_cols<4, EPI>(a, ct, st);
+    case 5: return dt_cols<5, EPI>(a, ct, st);
+    case 6: return dt_cols<6, EPI>(a, ct, st);
+    case 7: return dt_cols<7, EPI>(a, ct, st);
+    case 8: return dt_cols<8, EPI>(a, ct, st);
   }
-  return sg_launch<RT, TW, 2>(a, st);
+  return -10;
 }
 
 }  // namespace
 
 // X [M, K] bf16 (row stride xs), W = [gate; up] [2F, K] bf16 contiguous, Y [M, F] bf16 (row stride ys).
-// K % 64 == 0, F % 4 == 0, w % 4 == 0, 4 <= w <= 80, M <= 256 mblocks, mblocks in {1, 2}. Returns -10 for a shape
+// K % 64 == 0, F % 4 == 0, w % 4 == 0, 4 <= w <= 80, M <= 256 mblocks, mblocks in {1 .. 4}. Returns -10 for a shape
 // no instantiation covers (the caller then takes another kernel).
 extern "C" int areal_dswiglu(const void* X, long xs, const void* W, void* Y, long ys, int M, int F, int K, int w,
                              int mblocks, int stages, int nt, int act, hipStream_t st) {
   if (M <= 0) return 0;
   if (K % 64 != 0 || K < 64 || xs % 8 != 0 || F % 4 != 0 || w % 4 != 0 || w < 4 || ys % 4 != 0) return -1;
-  if (mblocks < 1 || mblocks > 2) return -2;
+  if (mblocks < 1 || mblocks > 4) return -2;
   if (((uintptr_t)X | (uintptr_t)W) % 16 != 0 || ((uintptr_t)Y) % 8 != 0) return -3;
-  SGArgs a;
-  a.X = (const bf16_t*)X; a.xs = xs; a.W = (const bf16_t*)W; a.Y = (bf16_t*)Y; a.ys = ys;
-  a.M = M; a.F = F; a.K = K; a.w = w; a.ntiles = (F + w - 1) / w; a.mblocks = mblocks; a.nt = nt; a.act = act;
+  DTArgs a;
+  a.X = (const bf16_t*)X; a.xs = xs; a.W = (const bf16_t*)W; a.Y = Y; a.ys = ys;
+  a.M = M; a.N = F; a.K = K; a.w = w; a.ntiles = (F + w - 1) / w; a.mblocks = mblocks; a.ksplit = 1; a.steps = K / 64;
+  a.stages = stages; a.nt = nt; a.act = act;
   // us without / with, 14336 columns, 4096 deep, 8 / 64 / 128 / 200 rows: 46 / 41, 47 / 41, 53 / 52, 78 / 77; 8 / 100 rows, 8192 columns
   // 34 / 25, 38 / 33, but 4096 columns 23.7 / 23.9, 30.1 / 31.0
   a.rot = mblocks == 1 && F >= 8192 ? k_rotation(K) : 0;
   const int rows = (M + mblocks - 1) / mblocks;  // rows per block
-  const int rt = (rows + 63) / 64;
-  const int tw = (w + 15) / 16;
-  if (rt < 1 || rt > 4) return -10;
-#define SG_CASE(R, T) \
-  if (rt == R && tw <= T) return sg_stages<R, T>(a, stages, st)
-  SG_CASE(1, 3); SG_CASE(2, 3); SG_CASE(3, 3); SG_CASE(4, 3);
-  SG_CASE(1, 5); SG_CASE(2, 5); SG_CASE(3, 5); SG_CASE(4, 5);
-#undef SG_CASE
-  return -10;
+  return dt_rows<DT_GATED>(a, (rows + 31) / 32, (w + 15) / 16, st);
+}
+
+// X [M, K] bf16 (row stride xs), W [N, K] bf16 contiguous, Y fp32 [ksplit, M, N]: partial sums of 64-deep steps [s, s + 1) * steps,
+// steps = ceil(K / 64 / ksplit), none of them empty. K % 64 == 0, N % 4 == 0; 32 rt rows (1 <= rt <= 8) and 32 ct columns (1 <= ct <=
+// 5) a workgroup, rt >= ceil(M / 32 / mblocks).
+extern "C" int areal_dtile_slab(const void* X, long xs, const void* W, void* Y, int M, int N, int K, int ct, int mblocks, int ksplit,
+                                int stages, int nt, hipStream_t st) {
+  if (M <= 0) return 0;
+  if (K % 64 != 0 || K < 64 || xs % 8 != 0 || N % 4 != 0 || N < 4 || ksplit < 1 || mblocks < 1) return -1;
+  if (((uintptr_t)X | (uintptr_t)W | (uintptr_t)Y) % 16 != 0) return -3;
+  DTArgs a;
+  a.X = (const bf16_t*)X; a.xs = xs; a.W = (const bf16_t*)W; a.Y = Y; a.ys = N;
+  a.M = M; a.N = N; a.K = K; a.w = 32 * ct; a.mblocks = mblocks; a.ksplit = ksplit; a.steps = (K / 64 + ksplit - 1) / ksplit;
+  if ((long)a.steps * (ksplit - 1) >= K / 64) return -4;  // an empty split
+  if (ct < 1 || ct > 5) return -10;
+  a.ntiles = (N + a.w - 1) / a.w;
+  a.stages = stages; a.nt = nt; a.act = 0; a.rot = 0;
+  const int rows = (M + mblocks - 1) / mblocks;
+  return dt_rows<DT_SLAB>(a, (rows + 31) / 32, ct, st);
 }

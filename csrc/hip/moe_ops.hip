@@ -239,17 +239,26 @@ __global__ __launch_bounds__(256) void moe_topk_kernel(const TIN* __restrict__ l
   float v[PER_LANE];
   float mx = -INFINITY;
 #pragma unroll
-  for (int i = 0; i < PER_LANE; ++i) {
-    const int e = lane + 64 * i;
-    v[i] = e < E ? (float)row[e] : -INFINITY;
-    if (sizeof(TIN) == 4 && slabs > 0 && e < E) {
-      float s = v[i];
-#pragma unroll 4
-      for (int j = 1; j < slabs; ++j) s += (float)row[(size_t)j * T * E + e];
-      v[i] = bf2f(f2bf(s));
+  for (int i = 0; i < PER_LANE; ++i) v[i] = lane + 64 * i < E ? (float)row[lane + 64 * i] : -INFINITY;
+  if (sizeof(TIN) == 4 && slabs > 0) {
+    constexpr int U = PER_LANE <= 2 ? 8 : 4;  // slabs in flight for all of a lane's experts together
+    for (int j = 1; j < slabs; j += U) {
+      float u[U][PER_LANE];
+#pragma unroll
+      for (int b = 0; b < U; ++b)
+#pragma unroll
+        for (int i = 0; i < PER_LANE; ++i)
+          u[b][i] = j + b < slabs && lane + 64 * i < E ? (float)row[(size_t)(j + b) * T * E + lane + 64 * i] : 0.f;
+#pragma unroll
+      for (int b = 0; b < U; ++b)
+#pragma unroll
+        for (int i = 0; i < PER_LANE; ++i) v[i] += u[b][i];
     }
-    mx = fmaxf(mx, v[i]);
+#pragma unroll
+    for (int i = 0; i < PER_LANE; ++i) v[i] = bf2f(f2bf(v[i]));
   }
+#pragma unroll
+  for (int i = 0; i < PER_LANE; ++i) mx = fmaxf(mx, v[i]);
   mx = wave_max(mx);
   float se = 0.f;
 #pragma unroll
