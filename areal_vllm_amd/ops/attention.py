@@ -8,6 +8,7 @@ Counterparts in the reference: ``flash_attn_varlen_func`` / ``flash_attn_with_kv
 ``areal/engine/base_hf_engine.py:291-406``.
 """
 import math
+from functools import lru_cache
 from typing import Optional, Tuple
 
 import torch
@@ -380,22 +381,32 @@ def context_slots(block_tables: torch.Tensor, cu_k: torch.Tensor) -> torch.Tenso
     return block_tables.long()[seq, t // PAGE_SIZE] * PAGE_SIZE + t % PAGE_SIZE
 
 
-# Workgroups that a prefill against the cache should start, and the fewest keys of one of them
-PAGED_PREFILL_WORKGROUPS, PAGED_PREFILL_KEYS = 256, 128
+# Most workgroups of a prefill against the cache whose keys are split, and the fewest keys of one of them
+PAGED_PREFILL_WORKGROUPS, PAGED_PREFILL_KEYS = 1024, 64
 
 
 def paged_prefill_splits(batch: int, n_q_heads: int, max_q: int, max_k: int, total_q: Optional[int] = None) -> int:
-    """Ranges into which the keys of a query tile are split: one workgroup walks 64 keys in 2.4 us, so the few tiles of a
-    short turn behind a long context wait for one another while most of the chip idles. One range where the walk that is saved
-    is shorter than the second launch and the partial results (4 us, and 0.35 us for every 1000 rows of them). us unsplit /
-    split, over 623 shapes of 1 to 12 requests: 93 tokens behind 811, 12 heads, 37 / 21 in 7 ranges; 512 behind 8000 277 / 92;
-    512 alone, 32 heads, 23 / 28 in 2; 2 x 256 alone, 64 tiles, 16 / 20; 5 x 256 behind 64, 120 tiles, 18 / 27: the rule takes
-    0.3 % more than the better of the two, always splitting 3 % more."""
-    tiles = max(1, batch * n_q_heads * ((max_q + 127) // 128))
-    splits = max(1, min(PAGED_PREFILL_WORKGROUPS // tiles, max_k // PAGED_PREFILL_KEYS, 32))
+    """Ranges into which the keys of a query tile are split (at most 32): one workgroup walks 64 keys in 2.1 us, two that
+    share a CU in 2.7, so the few tiles of a short turn behind a long context wait for one another while most of the chip
+    idles. The least of that walk (in rounds of two workgroups a CU) and, with more than one range, of the second launch and
+    the partial results (4 us, and 0.35 us for every 1000 rows of them). us in 1 / 5 / 7 / 8 / 10 / 20 ranges, the rule's in
+    brackets: 93 tokens behind 811, 12 heads 37 / 17.0 / 17.4 / [15.8] / 16.3 / -; 512 behind 8000 273 / 67 / 67 / 63 / [56] /
+    67; 300 behind 4000 142 / 43 / [37] / 40 / 37 / 43; 40 behind 20000 618 / 134 / 98 / 88 / 73 / [46]; 2000 behind 500 in 1
+    / 2 / 3 / 4 86 / 61 / [53] / 58; 8 x 500 behind 700 [52] / 92 / 107 / 113 / 140 / -; 2 x 256 alone, 32 heads [15.5] / 27."""
+    return _ranges(max(1, batch * n_q_heads * ((max_q + 127) // 128)), n_q_heads * (batch * max_q if total_q is None else total_q),
+                   max_k, PAGED_PREFILL_WORKGROUPS, PAGED_PREFILL_KEYS)
+
+
+@lru_cache(maxsize=4096)
+def _ranges(tiles: int, rows: int, max_k: int, workgroups: int, keys: int) -> int:
     walk = -(-max_k // 64)  # tiles of 64 keys
-    rows = splits * n_q_heads * (batch * max_q if total_q is None else total_q)
-    return splits if 2.4 * (walk - -(-walk // splits)) > 4 + 3.5e-4 * rows else 1
+
+    def cost(splits):
+        groups = tiles * splits
+        return (-(-walk // splits) * (2.1 if groups <= 256 else 2.7) * max(1.0, groups / 512)
+                + (4 + 3.5e-4 * rows * splits if splits > 1 else 0))
+
+    return min(range(1, max(1, min(workgroups // tiles, max_k // keys, 32)) + 1), key=cost)
 
 
 def flash_attn_paged_prefill(q, kcache, vcache, block_tables, cu_q, cu_k, max_q: int, scale: Optional[float] = None,

@@ -108,7 +108,8 @@ def slab_plan(M: int, N: int, K: int) -> Tuple[int, int, int]:
     a workgroup's 64-deep steps x (46 ns for each 32 rows and each 32 columns that it stages, 5.6 for each pair of them
     that it multiplies, 46 for the step) x rounds of 256 workgroups, and 0.45 us for each MB of partial sums, written here
     and read by the row kernel behind (0.15 of it). Fitted to 6500 launches (13 layers of 896 to 5120 columns, 896 to
-    18944 deep, 8 to 512 rows); its choice is 1.2 % behind the best of them in the mean, 10 % at worst."""
+    18944 deep, 8 to 512 rows); its choice is 1.2 % behind the best of them in the mean, 10 % at worst. No split of less than
+    192 deep: a ring that is never full, and products of few columns need no more parts than their readers sum at once."""
     steps = K // 64
     best = None
     for mblocks in range(-(-M // 256), -(-M // 32) + 1):
@@ -117,7 +118,7 @@ def slab_plan(M: int, N: int, K: int) -> Tuple[int, int, int]:
             continue  # a row block of no rows
         for ct in range(1, 6):
             tiles = -(-N // (32 * ct)) * mblocks
-            for ksplit in range(1, max(1, min(24, N_CU // tiles, steps)) + 1):
+            for ksplit in range(1, max(1, min(24, N_CU // tiles, K // 192)) + 1):
                 per = -(-steps // ksplit)
                 if per * (ksplit - 1) >= steps:
                     continue  # a split of no steps

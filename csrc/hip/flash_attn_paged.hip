@@ -38,7 +38,7 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_paged_kernel(
     const bf16_t* __restrict__ q, const void* __restrict__ kcache, const void* __restrict__ vcache,
     const int* __restrict__ block_tables, int max_pages, bf16_t* __restrict__ o, float* __restrict__ lse,
     const int* __restrict__ cu_q, const int* __restrict__ cu_k, int64_t q_stride, int64_t o_stride, int Hq, int Hkv,
-    int nbatch, int total_q, float scale_log2, int causal, int window = 0, int keep = 0,
+    int nbatch, int total_q, int n_rank, int splits, float scale_log2, int causal, int window = 0, int keep = 0,
     const bf16_t* __restrict__ r1 = nullptr, const bf16_t* __restrict__ r2 = nullptr,
     const bf16_t* __restrict__ gate = nullptr, int64_t gate_stride = 0, int chunk = 0,
     const bf16_t* __restrict__ sink = nullptr, const KVStrides str = KVStrides{}, float* __restrict__ part = nullptr) {
@@ -47,15 +47,31 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_paged_kernel(
   char* ks = smem;             // K tile  [64 keys][256 B], 16-byte chunks swizzled (flash_tiles.hpp)
   char* vs = smem + 64 * 256;  // V^T tile [128 channels][128 B = 64 keys], 8-byte chunks swizzled
 
-  // grid order: see flash_fwd_kernel (heaviest query tiles first, query heads of one kv group on one XCD)
-  const int G = Hq / Hkv;
-  const int n_g = Hkv * nbatch, n_g_pad = (n_g + 7) & ~7;
-  const int per_rank = G * n_g_pad;
-  const int rank = blockIdx.x / per_rank, rem = blockIdx.x - rank * per_rank;
-  const int hj = rem / n_g_pad, slot = rem - hj * n_g_pad;
-  int g = slot - rank % n_g_pad;
-  g += g < 0 ? n_g_pad : 0;
-  if (g >= n_g) return;
+  // grid order: see flash_fwd_kernel (heaviest query tiles first, query heads of one kv group on one XCD). Fewer groups than XCDs:
+  // the XCDs take turns in (query tile, range of keys, group), without idle workgroups between the others: a lone request with
+  // two key heads had all its workgroups on two XCDs (us, 12 heads on 2, 300 tokens behind 4000 in 7 / 10 ranges 63 /
+  // 61, now 37 / 37; 93 behind 811 in 8 19.3, now 15.8; 512 behind 8000 in 10 96, now 56).
+  const int G = Hq / Hkv, n_g = Hkv * nbatch;
+  int rank, range, hj, g;
+  if (n_g < 8) {
+    const int slot = blockIdx.x >> 3;
+    hj = slot % G;
+    int rest = slot / G * 8 + (blockIdx.x & 7);
+    g = rest % n_g;
+    rest /= n_g;
+    range = rest % splits;
+    rank = rest / splits;
+  } else {
+    const int n_g_pad = (n_g + 7) & ~7, per_rank = G * n_g_pad, per_range = per_rank * n_rank;
+    range = blockIdx.x / per_range;
+    int rem = blockIdx.x - range * per_range;
+    rank = rem / per_rank;
+    rem -= rank * per_rank;
+    hj = rem / n_g_pad;
+    g = rem - hj * n_g_pad - rank % n_g_pad;
+    g += g < 0 ? n_g_pad : 0;
+    if (g >= n_g) return;
+  }
   const int b = g / Hkv, kvh = g - b * Hkv, head = kvh * G + hj;
   const int q_beg = cu_q[b], q_len = cu_q[b + 1] - q_beg;
   const int k_len = cu_k[b + 1] - cu_k[b];
@@ -117,29 +133,37 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_paged_kernel(
   auto tile_of = [&](int it) { return it < n_keep ? it : t_lo + it - n_keep; };
   int it_lo = 0, it_hi = n_iter;
   if (!WIN && part) {
-    const int per = (n_iter + (int)gridDim.y - 1) / (int)gridDim.y;
-    it_lo = min((int)blockIdx.y * per, n_iter);
+    const int per = (n_iter + splits - 1) / splits;
+    it_lo = min(range * per, n_iter);
     it_hi = min(it_lo + per, n_iter);
   }
 
   // K: thread -> (key row = tid>>4 + 16 i, 16-byte chunk tid&15). V^T: piece id = tid + 256 i ->
-  // (page half = id>>9, channel = (id>>2)&127, 8-token chunk = id&3): a wave reads 1 KiB of contiguous cache.
+  // (page half = id>>9, channel = (id>>2)&127, 8-token chunk = id&3): a wave reads 1 KiB of contiguous cache. The page ids of 32
+  // steps are fetched at once, one a lane: with a load of its own ahead of every tile's rows a step of a lone workgroup waited
+  // for two memory latencies (15 tiles in 38.2 us, now 36.3). Rows past the context are read where the cache has them (masked
+  // scores, zeroed V), at given strides the last row instead.
   const int lrow = tid >> 4, lch = tid & 15;
   bf16x8 kreg[4], vreg[4];
-  auto load_tile = [&](int t) {
+  int ids = 0;
+  auto load_tile = [&](int it) {
+    const int t = tile_of(it), j = (it - it_lo) & 31;
+    if (j == 0) {
+      const int step = it + (lane >> 1);
+      ids = bt[min(2 * tile_of(min(step, it_hi - 1)) + (lane & 1), last_page)];
+    }
+    const int page[2] = {__builtin_amdgcn_readlane(ids, 2 * j), __builtin_amdgcn_readlane(ids, 2 * j + 1)};
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      int key = t * 64 + lrow + 16 * i;
-      key = key < k_len ? key : k_len - 1;
-      const int page = bt[key >> 5];
-      kreg[i] = ld8_cache<FP8>(kcache, (STR ? page * str.k_page + kvh * str.k_head + (key & 31) * str.k_key
-                                            : (((size_t)page * Hkv + kvh) * 32 + (key & 31)) * D) + lch * 8);
+      const int key = t * 64 + lrow + 16 * i;
+      const int row = STR ? min(key, k_len - 1) & 31 : lrow + 16 * (i & 1);
+      const int64_t pg = page[i >> 1];
+      kreg[i] = ld8_cache<FP8>(kcache, (STR ? pg * str.k_page + kvh * str.k_head + row * str.k_key
+                                            : ((size_t)pg * Hkv + kvh) * 32 * D + row * D) + lch * 8);
       const int id = tid + 256 * i;
-      const int half = id >> 9, ch = (id >> 2) & 127, c16 = id & 3;
-      int pg = t * 2 + half;
-      pg = pg < last_page ? pg : last_page;
-      vreg[i] = ld8_cache<FP8>(vcache, (STR ? bt[pg] * str.v_page + kvh * str.v_head + ch * str.v_ch
-                                            : (((size_t)bt[pg] * Hkv + kvh) * D + ch) * 32) + c16 * 8);
+      const int ch = (id >> 2) & 127, c16 = id & 3;
+      vreg[i] = ld8_cache<FP8>(vcache, (STR ? pg * str.v_page + kvh * str.v_head + ch * str.v_ch
+                                            : ((size_t)pg * Hkv + kvh) * D * 32 + ch * 32) + c16 * 8);
     }
   };
   auto store_tile = [&](int t) {
@@ -164,7 +188,7 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_paged_kernel(
     }
   };
   if (it_lo < it_hi) {
-    load_tile(tile_of(it_lo));
+    load_tile(it_lo);
     store_tile(tile_of(it_lo));
   }
   __syncthreads();
@@ -173,7 +197,7 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_paged_kernel(
   const int vsw = (r >> 1) & 15;  // swizzle key of this lane's V^T rows (32 db + r)
   for (int it = it_lo; it < it_hi; ++it) {
     const int t = tile_of(it);
-    if (it + 1 < it_hi) load_tile(tile_of(it + 1));
+    if (it + 1 < it_hi) load_tile(it + 1);
     f32x16 sacc[2];
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb) {
@@ -258,7 +282,7 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_paged_kernel(
   if (!WIN && part) {  // this range of keys: O not divided by l, then (m, l) behind the O of all ranges
     if (my_q < q_len) {
       const size_t rows = (size_t)total_q * Hq, row = (size_t)(q_beg + my_q) * Hq + head;
-      float* op = part + (blockIdx.y * rows + row) * D + 4 * hf;
+      float* op = part + (range * rows + row) * D + 4 * hf;
 #pragma unroll
       for (int db = 0; db < 4; ++db)
 #pragma unroll
@@ -266,7 +290,7 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_paged_kernel(
           *reinterpret_cast<f32x4*>(op + 32 * db + 8 * gq) =
               f32x4{oacc[db][4 * gq], oacc[db][4 * gq + 1], oacc[db][4 * gq + 2], oacc[db][4 * gq + 3]};
       if (hf == 0) {
-        float* ml = part + gridDim.y * rows * D + (blockIdx.y * rows + row) * 2;
+        float* ml = part + splits * rows * D + (range * rows + row) * 2;
         ml[0] = m;
         ml[1] = l;
       }
@@ -325,6 +349,11 @@ __global__ __launch_bounds__(256) void flash_paged_combine_kernel(const float* _
   *reinterpret_cast<bf16x2*>(o + row / Hq * o_stride + row % Hq * 128 + lane * 2) = r;
 }
 
+static dim3 paged_grid(int B, int Hq, int Hkv, int n_rank, int splits) {
+  const int64_t n_g = (int64_t)Hkv * B, n = n_g < 8 ? (n_rank * splits * n_g + 7) / 8 * 8 : n_rank * splits * ((n_g + 7) & ~7);
+  return dim3((unsigned)(n * (Hq / Hkv)));
+}
+
 // q [total_q, Hq, 128] (row stride q_stride), K cache [P, Hkv, 32, 128], V cache [P, Hkv, 128, 32], block_tables
 // [B, max_pages] int32 (page of tokens 32 i .. 32 i + 31 of request b), cu_q / cu_k [B + 1]: query rows and context
 // lengths (the context of request b INCLUDES its query rows: they are in the cache already). Every request needs
@@ -344,12 +373,12 @@ extern "C" int areal_flash_fwd_paged(const void* q, const void* kcache, const vo
   if ((q_stride | o_stride) % 8 != 0) return -3;
   if (((uintptr_t)q | (uintptr_t)kcache | (uintptr_t)vcache | (uintptr_t)o) % 16 != 0) return -4;
   const float scale_log2 = softmax_scale * 1.4426950408889634f;
-  const int n_g_pad = (Hkv * B + 7) & ~7;
-  dim3 grid((unsigned)(((max_q + 127) / 128) * (Hq / Hkv) * n_g_pad)), block(256);
-  grid.y = (unsigned)splits;
+  const int n_rank = (max_q + 127) / 128;
+  dim3 grid = paged_grid(B, Hq, Hkv, n_rank, splits), block(256);
 #define AREAL_PAGED_LAUNCH(FP8_)                                                                                            \
   hipLaunchKernelGGL(flash_fwd_paged_kernel<FP8_>, grid, block, 0, st, (const bf16_t*)q, kcache, vcache, block_tables,      \
-                     max_pages, (bf16_t*)o, lse, cu_q, cu_k, q_stride, o_stride, Hq, Hkv, B, total_q, scale_log2, causal,   \
+                     max_pages, (bf16_t*)o, lse, cu_q, cu_k, q_stride, o_stride, Hq, Hkv, B, total_q, n_rank, splits,       \
+                     scale_log2, causal,                                                                                    \
                      0, 0, (const bf16_t*)nullptr, (const bf16_t*)nullptr, (const bf16_t*)nullptr, (int64_t)0, 0,           \
                      (const bf16_t*)nullptr, KVStrides{}, part)
   if (fp8) AREAL_PAGED_LAUNCH(true); else AREAL_PAGED_LAUNCH(false);
@@ -377,11 +406,11 @@ extern "C" int areal_flash_fwd_paged_window(const void* q, const void* kcache, c
   if (((uintptr_t)q | (uintptr_t)kcache | (uintptr_t)vcache | (uintptr_t)o) % 16 != 0) return -4;
   if (gate && (gate_stride % 4 != 0 || (uintptr_t)gate % 8 != 0)) return -5;
   const float scale_log2 = softmax_scale * 1.4426950408889634f;
-  const int n_g_pad = (Hkv * B + 7) & ~7;
-  dim3 grid((unsigned)(((max_q + 127) / 128) * (Hq / Hkv) * n_g_pad)), block(256);
+  const int n_rank = (max_q + 127) / 128;
+  dim3 grid = paged_grid(B, Hq, Hkv, n_rank, 1), block(256);
   hipLaunchKernelGGL((flash_fwd_paged_kernel<false, true>), grid, block, 0, st, (const bf16_t*)q, kcache, vcache,
                      block_tables, max_pages, (bf16_t*)o, (float*)nullptr, cu_q, cu_k, q_stride, o_stride, Hq, Hkv, B,
-                     total_q, scale_log2, 1, window, keep, (const bf16_t*)r1, (const bf16_t*)r2, (const bf16_t*)gate,
+                     total_q, n_rank, 1, scale_log2, 1, window, keep, (const bf16_t*)r1, (const bf16_t*)r2, (const bf16_t*)gate,
                      gate_stride, chunk);
   return (int)hipGetLastError();
 }
@@ -399,11 +428,11 @@ extern "C" int areal_flash_fwd_strided(const void* q, const void* k, const void*
   if ((q_stride | o_stride | k_page | k_head | k_key | v_page | v_head | v_ch) % 8 != 0) return -3;
   if (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)o) % 16 != 0) return -4;
   const float scale_log2 = softmax_scale * 1.4426950408889634f;
-  const int n_g_pad = (Hkv * B + 7) & ~7;
-  dim3 grid((unsigned)(((max_q + 127) / 128) * (Hq / Hkv) * n_g_pad)), block(256);
+  const int n_rank = (max_q + 127) / 128;
+  dim3 grid = paged_grid(B, Hq, Hkv, n_rank, 1), block(256);
   hipLaunchKernelGGL((flash_fwd_paged_kernel<false, true, true>), grid, block, 0, st, (const bf16_t*)q, k, v, block_tables,
                      max_pages, (bf16_t*)o, (float*)nullptr, cu_q, cu_k, q_stride, o_stride, Hq, Hkv, B, total_q,
-                     scale_log2, 1, 0, 0, (const bf16_t*)nullptr, (const bf16_t*)nullptr, (const bf16_t*)nullptr,
+                     n_rank, 1, scale_log2, 1, 0, 0, (const bf16_t*)nullptr, (const bf16_t*)nullptr, (const bf16_t*)nullptr,
                      (int64_t)0, 0, (const bf16_t*)sink, KVStrides{k_page, k_head, k_key, v_page, v_head, v_ch});
   return (int)hipGetLastError();
 }
