@@ -300,18 +300,44 @@ class ModelRunner:
         return F.linear(x.float(), w.float())
 
     # ----------------------------------------------------------------------------- prefill
+    def _upload(self, arrays: Dict[str, np.ndarray]) -> Dict[str, torch.Tensor]:
+        """Host arrays -> device tensors of their shapes and types, by one copy that the host does not wait for (torch keeps
+        the pinned buffer until it is done)."""
+        arrays = {k: np.ascontiguousarray(v) for k, v in arrays.items()}
+        at, total = {}, 0
+        for k, v in arrays.items():
+            at[k] = total
+            total += -(-v.nbytes // 16) * 16
+        host = torch.empty(total, dtype=torch.uint8, pin_memory=self.device.type == "cuda")
+        raw = host.numpy()
+        for k, v in arrays.items():
+            raw[at[k]:at[k] + v.nbytes] = v.reshape(-1).view(np.uint8)
+        flat = host.to(self.device, non_blocking=True)
+        return {k: flat[at[k]:at[k] + v.nbytes].view(torch.from_numpy(v).dtype).view(v.shape) for k, v in arrays.items()}
+
     @torch.no_grad()
     def prefill(self, plan: Dict[str, Any]) -> Tuple[np.ndarray, np.ndarray]:
         dev = self.device
-        ids = torch.from_numpy(plan["input_ids"]).to(dev, non_blocking=True).long()
-        pos = torch.from_numpy(plan["positions"]).to(dev, non_blocking=True)
-        slots = torch.from_numpy(plan["slot_mapping"]).to(dev, non_blocking=True)
-        cu_q = torch.from_numpy(plan["cu_q"]).to(dev, non_blocking=True)
-        cu_k = torch.from_numpy(plan["cu_k"]).to(dev, non_blocking=True)
-        has_prefix = bool(plan["has_prefix"])
-        bt = torch.from_numpy(plan["block_tables"]).to(dev, non_blocking=True) if has_prefix else None
-        max_q = int(plan["max_q"])
         B = len(plan["req_ids"])
+        max_q = int(plan["max_q"])
+        has_prefix = bool(plan["has_prefix"])
+        score = plan.get("logit_rows") is not None
+        pen = {}
+        # one upload of everything ahead of the first launch: a copy behind the layers would wait for them
+        up = dict(ids=plan["input_ids"], pos=plan["positions"], slots=plan["slot_mapping"], cu_q=plan["cu_q"], cu_k=plan["cu_k"])
+        draws = not score or bool(np.any(plan["sample"]))  # (otherwise a plan that only scores)
+        if draws:
+            up.update(temp=plan["temperature"], top_p=plan["top_p"], top_k=np.minimum(plan["top_k"], self.V).astype(np.int32))
+        if has_prefix:
+            up["bt"] = plan["block_tables"]
+        if score:
+            up["rows"] = np.asarray(plan["logit_rows"], dtype=np.int64)
+        if draws and "penalty_slot" in plan and (plan["penalty_slot"] >= 0).any():  # chunks that do not sample carry slot -1
+            up.update(slot=plan["penalty_slot"], freq=plan["frequency_penalty"], pres=plan["presence_penalty"])
+        up = self._upload(up)
+        ids, pos, slots, cu_q, cu_k, bt = up["ids"].long(), up["pos"], up["slots"], up["cu_q"], up["cu_k"], up.get("bt")
+        if "slot" in up:
+            pen = dict(counts=self.token_counts(), count_slot=up["slot"], freq_pen=up["freq"], pres_pen=up["pres"])
         T = ids.numel()
         self.n_prefill_tokens += T
 
@@ -325,24 +351,16 @@ class ModelRunner:
         if self.cfg.pos_embed != "rope":
             pos = torch.zeros_like(pos) if not self.keeps_positions else pos  # the only row of the angle-zero table
         h, residual = self._prefill_layers(plan, h, pos, slots, rope, cu_q, cu_k, bt, max_q)
-        if plan.get("logit_rows") is not None:  # scoring: fp32 logits at chosen tokens of the packed batch
-            rows = torch.from_numpy(np.asarray(plan["logit_rows"], dtype=np.int64)).to(dev)
+        if score:  # fp32 logits at chosen tokens of the packed batch
+            rows = up["rows"]
             self.kept_logits = self._final_logits(h[rows], None if residual is None else residual[rows],
                                                   fp32=True).float()
-            if not np.any(plan["sample"]):  # nothing to draw: a plan that only scores
+            if not draws:
                 return np.zeros(B, np.int64), np.zeros(B, np.float32)
         last = (cu_q[1:] - 1).long()
         logits = self._final_logits(h[last], None if residual is None else residual[last])
-        temp = torch.from_numpy(plan["temperature"]).to(dev)
-        top_p = torch.from_numpy(plan["top_p"]).to(dev)
-        top_k = torch.from_numpy(np.minimum(plan["top_k"], self.V).astype(np.int32)).to(dev)
         filt = bool((plan["top_k"] < self.V).any() or (plan["top_p"] < 1.0).any())
-        pen = {}
-        if "penalty_slot" in plan and (plan["penalty_slot"] >= 0).any():  # chunks that do not sample carry slot -1
-            pen = dict(counts=self.token_counts(), count_slot=torch.from_numpy(plan["penalty_slot"]).to(dev),
-                       freq_pen=torch.from_numpy(plan["frequency_penalty"]).to(dev),
-                       pres_pen=torch.from_numpy(plan["presence_penalty"]).to(dev))
-        tok, lp = ops.sample(logits, temp, top_k if filt else None, top_p if filt else None, self.seed,
+        tok, lp = ops.sample(logits, up["temp"], up["top_k"] if filt else None, up["top_p"] if filt else None, self.seed,
                              self.step_counter, **pen)
         self._sync_tokens(tok, lp)
         tok_h, lp_h = tok.cpu().numpy(), lp.cpu().numpy()
@@ -421,6 +439,14 @@ class ModelRunner:
             return (x, s) if weight is not None else (s, None)
 
         x, residual = ops.rmsnorm(h, layers[0].ln1, eps, None, gemma)
+        if bt is not None and not tp and balanced and D == 128:  # all launches from one native call
+            norms = [blk.ln1 for blk in layers[1:]] + [None]
+            out = ops.prefill_layers.run(
+                [(b.attn.qkv, b.attn.qkv_bias, b.attn.q_norm if cfg.qk_norm else None, b.attn.k_norm if cfg.qk_norm else None,
+                  b.attn.o, b.ln2, b.mlp.gate_up, b.mlp.down, nw) for b, nw in zip(layers, norms)],
+                self.kv, x, residual, pos, slots, rope, cu_q, cu_k, bt, max_q, hq, hkv, D, eps, gemma, act)
+            if out is not None:
+                return out, None
         for li, blk in enumerate(layers):
             kc, vc = self.kv[li]
             if bt is not None:  # some row has context in the cache: attention reads the pages directly

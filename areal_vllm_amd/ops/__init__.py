@@ -27,7 +27,7 @@ from .norm_act import RotaryTable, apply_rope, qk_norm, rmsnorm, rope_inplace_, 
 from .optim import adam_prepare_, adamw_, fold_grad_, scale_, sumsq_  # noqa: F401
 from .rl import gae_1d_packed, gae_2d, gae_padded, merge_intervals, set_intervals, slice_intervals  # noqa: F401
 from .sampling import TokenCounts, advance_step_, decode_advance_, decode_begin_, sample  # noqa: F401
-from . import train_gemm  # noqa: F401
+from . import prefill_layers, train_gemm  # noqa: F401
 from .linear import embedding, linear  # noqa: F401
 from .decode_gemm import dgemm, splitk_residual_rmsnorm, splitk_rope_cache_write  # noqa: F401
 from .grouped_gemm import (gate_up_rows_ok, grouped_gate_up, grouped_gemm, grouped_gemm_offsets,  # noqa: F401
