@@ -787,12 +787,100 @@ __global__ __launch_bounds__(256) void rope_cache_write_kernel(
   }
 }
 
+// The same for many tokens: 32 of them a workgroup. Tokens that follow each other in a prompt follow each other in a page, and
+// eight of them from a multiple of eight on are one 16-byte store of a V channel instead of eight 2-byte stores to eight places of a
+// 64-byte line (what bounded the kernel above, beside its idle threads). A workgroup writes the eights that start with one of its
+// tokens; tokens of no whole eight (ends of prompts, rows in any order) go one by one. us of the two, prompts of 64 to 1216 tokens, 12
+// heads on 2 of 128, 2048 / 4096 / 15600 / 32768 tokens: 8.9 / 12.9 / 46 / 91 and 11.4 / 12.5 / 36 / 68 (on an fp8 cache 7.7 / 11.1 / 38 /
+// 72 and 11.9 / 12.9 / 34 / 66); 32 on 4 14 / 31 / 99 / 206 and 20 / 33 / 77 / 153; 14 on 2 of 64 6.3 / 8.9 / 27 / 58 and 7.7 / 9.0 / 21 / 41.
+constexpr int RC_TOK = 32, RC_MIN_TOKENS = 8192, RC_THREADS = 1024;
+__global__ __launch_bounds__(RC_THREADS) void rope_cache_write_many_kernel(
+    bf16_t* __restrict__ qkv, const int* __restrict__ pos, const int64_t* __restrict__ slots,
+    const float* __restrict__ cos_t, const float* __restrict__ sin_t, void* __restrict__ kcache,
+    void* __restrict__ vcache, int T, int Hq, int Hkv, int D, int max_pos, int do_rope, int fp8) {
+  extern __shared__ __attribute__((aligned(16))) bf16_t vbuf[];  // [RC_TOK + 7][Hkv D]: values of the tokens and of the seven behind
+  __shared__ int64_t slot_of[RC_TOK + 14];                       // of tokens t0 - 7 ... ; -1: none
+  __shared__ int run_at[RC_TOK / 8 + 1], n_runs;                 // first tokens (from t0) of the whole eights
+  __shared__ int lone[RC_TOK], n_lone;
+  const int t0 = blockIdx.x * RC_TOK, n = min(RC_TOK, T - t0), half = D >> 1, lph = half >> 3, W = Hkv * D, row_len = (Hq + 2 * Hkv) * D;
+  if (threadIdx.x < RC_TOK + 14) {
+    const int t = t0 - 7 + (int)threadIdx.x;
+    slot_of[threadIdx.x] = t >= 0 && t < T ? slots[t] : -1;
+  }
+  if (threadIdx.x == 0) n_runs = n_lone = 0;
+  for (int i = threadIdx.x; i < (RC_TOK + 7) * (W >> 3); i += RC_THREADS) {
+    const int r = i / (W >> 3), ch = i - r * (W >> 3);
+    if (t0 + r < T) st8(vbuf + r * W + ch * 8, ld8(qkv + (size_t)(t0 + r) * row_len + (Hq + Hkv) * D + ch * 8));
+  }
+  __syncthreads();
+  if ((int)threadIdx.x < n) {  // whole eight that token `threadIdx.x` belongs to
+    const int64_t s = slot_of[threadIdx.x + 7];
+    if (s >= 0) {
+      const int64_t first = s & ~7ll;
+      const int at = (int)threadIdx.x + 7 - (int)(s - first);  // its place in slot_of, if the tokens before it are its neighbours
+      bool whole = true;
+      for (int j = 0; j < 8; ++j) whole = whole && slot_of[at + j] == first + j;
+      if (!whole) lone[atomicAdd(&n_lone, 1)] = threadIdx.x;
+      else if (s == first) run_at[atomicAdd(&n_runs, 1)] = threadIdx.x;
+    }
+  }
+  const int heads = Hq + Hkv;
+  for (int i = threadIdx.x; i < n * heads * lph; i += RC_THREADS) {
+    const int sub = i % lph, rest = i / lph, head = rest % heads, r = rest / heads;
+    const int64_t slot = slot_of[r + 7];
+    bf16_t* base = qkv + (size_t)(t0 + r) * row_len + (size_t)head * D + sub * 8;
+    bf16x8 lo = ld8(base), hi = ld8(base + half);
+    if (do_rope) {
+      int p = pos[t0 + r];
+      p = p < 0 ? 0 : (p >= max_pos ? max_pos - 1 : p);
+      const f32x4* cp = reinterpret_cast<const f32x4*>(cos_t + (size_t)p * half + sub * 8);
+      const f32x4* sp = reinterpret_cast<const f32x4*>(sin_t + (size_t)p * half + sub * 8);
+      bf16x8 olo, ohi;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float a = bf2f(lo[j]), bb = bf2f(hi[j]), c = cp[j >> 2][j & 3], sn = sp[j >> 2][j & 3];
+        olo[j] = f2bf(a * c - bb * sn);
+        ohi[j] = f2bf(bb * c + a * sn);
+      }
+      lo = olo; hi = ohi;
+      st8(base, lo);
+      st8(base + half, hi);
+    }
+    if (head >= Hq && slot >= 0) {
+      const size_t kd = (((size_t)(slot / PAGE) * Hkv + head - Hq) * PAGE + slot % PAGE) * D + sub * 8;
+      st8_cache(kcache, kd, lo, fp8);
+      st8_cache(kcache, kd + half, hi, fp8);
+    }
+  }
+  __syncthreads();
+  // eights of one page beside each other: neighbouring lanes fill a channel's 64 bytes
+  for (int i = threadIdx.x; i < n_runs * W; i += RC_THREADS) {
+    const int r = run_at[i % n_runs], ch = i / n_runs, vh = ch / D, d = ch - vh * D;
+    const int64_t slot = slot_of[r + 7];
+    bf16x8 v;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = vbuf[(r + j) * W + ch];
+    st8_cache(vcache, (((size_t)(slot / PAGE) * Hkv + vh) * D + d) * PAGE + slot % PAGE, v, fp8);
+  }
+  for (int i = threadIdx.x; i < n_lone * W; i += RC_THREADS) {
+    const int r = lone[i / W], ch = i % W, vh = ch / D, d = ch - vh * D;
+    const int64_t slot = slot_of[r + 7];
+    st1_cache(vcache, (((size_t)(slot / PAGE) * Hkv + vh) * D + d) * PAGE + slot % PAGE, bf2f(vbuf[r * W + ch]), fp8);
+  }
+}
+
 extern "C" int areal_rope_cache_write(void* qkv, const int* pos, const int64_t* slots,
                                       const float* cos_t, const float* sin_t, void* kcache,
                                       void* vcache, int T, int Hq, int Hkv, int D, int max_pos,
                                       int do_rope, int fp8, hipStream_t st) {
   if (T == 0) return 0;
   if (D % 16 != 0) return -1;
+  const size_t lds = (size_t)(RC_TOK + 7) * Hkv * D * sizeof(bf16_t);
+  if (slots && T >= RC_MIN_TOKENS && lds <= 60 * 1024) {
+    hipLaunchKernelGGL(rope_cache_write_many_kernel, dim3((T + RC_TOK - 1) / RC_TOK), dim3(RC_THREADS), lds, st, (bf16_t*)qkv, pos, slots,
+                       cos_t, sin_t, kcache, vcache, T, Hq, Hkv, D, max_pos, do_rope, fp8);
+    return (int)hipGetLastError();
+  }
   hipLaunchKernelGGL(rope_cache_write_kernel, dim3(T), dim3(256), 0, st, (bf16_t*)qkv, pos, slots,
                      cos_t, sin_t, kcache, vcache, Hq, Hkv, D, max_pos, do_rope, fp8);
   return (int)hipGetLastError();
