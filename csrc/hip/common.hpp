@@ -104,9 +104,9 @@ DEVINL u32x2 bf16x8_to_fp8(bf16x8 v) {
                  pack_fp8x4(bf2f(v[4]), bf2f(v[5]), bf2f(v[6]), bf2f(v[7]))};
 }
 DEVINL bf16x8 fp8x8_to_bf16(u32x2 w) {
-  const f32x2 a = __builtin_amdgcn_cvt_pk_f32_fp8((int)w[0], false), b = __builtin_amdgcn_cvt_pk_f32_fp8((int)w[0], true);
-  const f32x2 c = __builtin_amdgcn_cvt_pk_f32_fp8((int)w[1], false), d = __builtin_amdgcn_cvt_pk_f32_fp8((int)w[1], true);
-  return (bf16x8){f2bf(a[0]), f2bf(a[1]), f2bf(b[0]), f2bf(b[1]), f2bf(c[0]), f2bf(c[1]), f2bf(d[0]), f2bf(d[1])};
+  const bf16x2 a = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w[0], 1.f, false), b = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w[0], 1.f, true);
+  const bf16x2 c = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w[1], 1.f, false), d = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w[1], 1.f, true);
+  return (bf16x8){a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
 }
 DEVINL float fp82f(fp8_t x) { return __builtin_amdgcn_cvt_pk_f32_fp8((int)x, false)[0]; }
 // 8 cache elements at element offset `i` of a cache of bf16 (FP8 = false) or fp8 (true) values, as bf16

@@ -461,6 +461,12 @@ DEVINL float ld_agent(const float* p) {
 // block: NW waves, page by page in turn. part_o: [n_items, Hq, D], part_ml: [n_items, Hq, 2],
 // arrived: [B, Hkv] zeros, zeros again afterwards. The last workgroup of a row to arrive combines its partial results
 // in the order of the items: the result does not depend on the order of arrival.
+// A wave is never without requests: the next page's K is asked for as soon as this page's scores have used up its registers, the
+// next V behind the second product; Q, whose registers that takes, is read from LDS. us a layer, page after page -> this, 12 query
+// heads on 2 of 128: 1 x 640 7.2 -> 6.9, 24 x 200-4096 16.0 -> 15.7, 256 x 640 32.1 -> 31.7, 320 x 128-1152 43.3 -> 43.2, 16 x 12000
+// 40.8 -> 38.8, 384 x 8-64 8.2 -> 7.5, fp8 48 x 6000-24000 81.0 -> 81.8, 128 x 1000 15.3 -> 14.9; 14 on 2 of 64, 300 x 100-1200 23.8 ->
+// 22.6; 8 on 1 of 256, 64 x 1000 22.1 -> 21.4, fp8 32 x 8000 34.9 -> 33.4, 1 x 640 12.5 -> 12.8: 4.8 to 5.6 of the 6 TB/s that the
+// chip reads, less where a launch is over in 10 us.
 // LDS holds the G real query rows only. Two workgroups of 8 waves a CU (128 registers a lane; heads of 64 three, of 256 one
 // of 4 waves): the register file sets that, a GQA group of 6 heads of 128 takes 26 KB of LDS.
 template <int D, bool FP8, int NW>
@@ -483,69 +489,84 @@ __global__ __launch_bounds__(64 * NW, (D > 128 ? 1 : 4)) void paged_decode_walk_
   const int mine = it.p_end - it.p_beg > wid ? (it.p_end - it.p_beg - wid + NW - 1) / NW : 0;
   int ids = lane < mine ? bt[it.p_beg + wid + NW * lane] : 0;
   const int ctx = context_lens[b];
-  // Q as the B operand of S^T = K.Q^T. fp8: a lane's 16 loaded bytes of K are the operand of two k-steps, so lane c
-  // holds Q[64 (ks / 2) + 16 c + 8 (ks % 2) + j] there and Q[32 ks + 8 c + j] otherwise
-  bf16x8 qf[KS];
+  // Q is the B operand of S^T = K.Q^T and waits in the LDS that the wave's result goes to at the end: its registers hold the next
+  // page instead. fp8: a lane's 16 loaded bytes of K are the operand of two k-steps, so lane c takes Q[64 (ks / 2) + 16 c +
+  // 8 (ks % 2) + j] there and Q[32 ks + 8 c + j] otherwise. Columns from G on repeat the last one and are not stored.
+  constexpr int QP = D + 8;  // row pitch: 16-byte reads of 16 rows on different banks
+  bf16_t* qs = reinterpret_cast<bf16_t*>(smem + wid * G * DP);
+  if (mine > 0) {
+    const int chunks = G * (D / 8);
+    const bf16_t* qp = q + (size_t)b * q_stride + (size_t)h * G * D;
+    bf16x8 qv[D / 32];
 #pragma unroll
-  for (int ks = 0; ks < KS; ++ks) {
-    const int k0 = FP8 ? (ks >> 1) * 64 + c * 16 + (ks & 1) * 8 : ks * 32 + c * 8;
-    if (col < G) qf[ks] = ld8(q + (size_t)b * q_stride + (size_t)(h * G + col) * D + k0);
-    else
+    for (int j = 0; j < D / 32; ++j) qv[j] = ld8(qp + min(lane + 64 * j, chunks - 1) * 8);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) qf[ks][j] = (bf16_t)0.f;
+    for (int j = 0; j < D / 32; ++j) {
+      const int i = min(lane + 64 * j, chunks - 1);  // (the last piece more than once)
+      st8(qs + i / (D / 8) * QP + i % (D / 8) * 8, qv[j]);
+    }
   }
+  const bf16_t* qrow = qs + min(col, G - 1) * QP + c * (FP8 ? 16 : 8);
+  auto qf = [&](int ks) __attribute__((always_inline)) { return ld8(qrow + (FP8 ? (ks >> 1) * 64 + (ks & 1) * 8 : ks * 32)); };
   f32x4 o[DB];
 #pragma unroll
   for (int i = 0; i < DB; ++i) o[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
   float m = -INFINITY, l = 0.f;  // running max (log2 units) is shared by the 4 lanes of a q
   const int key_a = 8 * (col >> 2) + (col & 3);  // row `col` of tile a; tile b: 4 rows further
 
-  for (int i = 0; i < mine; ++i) {
-    if (i > 0 && (i & 63) == 0) ids = lane + i < mine ? bt[it.p_beg + wid + NW * (lane + i)] : 0;
-    const int p = it.p_beg + wid + NW * i;
-    const int page = __builtin_amdgcn_readlane(ids, i & 63);
-    const size_t kp = ((size_t)page * Hkv + h) * PAGE * D;  // element offset of this page's K / V block
-    // all loads of the page up front (16 KiB, fp8: 8 KiB a wave in flight)
-    bf16x8 ka[KS], kb[KS], vt[DB];
-    if (FP8) {
-      const fp8_t* kc = reinterpret_cast<const fp8_t*>(kcache) + kp + key_a * D + c * 16;
-      const fp8_t* vc = reinterpret_cast<const fp8_t*>(vcache) + kp + col * PAGE + c * 8;
-      u32x4 ra[KS / 2], rb[KS / 2];
-      u32x2 rv[DB];
+  // Element offset of the K / V block of this wave's page i. The wait belongs to the fetch: behind the branch it would hold
+  // every page's loads.
+  auto block_of = [&](int i) __attribute__((always_inline)) {
+    if (i > 0 && (i & 63) == 0) {
+      ids = lane + i < mine ? bt[it.p_beg + wid + NW * (lane + i)] : 0;
+      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+    }
+    return ((size_t)__builtin_amdgcn_readlane(ids, i & 63) * Hkv + h) * PAGE * D;
+  };
+  // K and V of a page as loaded, 16 KiB (fp8: 8 KiB) a wave
+  using kraw = std::conditional_t<FP8, u32x4, bf16x8>;
+  using vraw = std::conditional_t<FP8, u32x2, bf16x8>;
+  constexpr int KL = FP8 ? KS / 2 : KS;
+  kraw ra[KL], rb[KL];
+  vraw rv[DB];
+  // a page's base is the same for all lanes, a lane's offset is the same for all pages: scalar base + 32-bit offset
+  constexpr int EB = FP8 ? 1 : 2;
+  const unsigned k_off = key_a * D * EB + c * 16, v_off = (col * PAGE + c * 8) * EB;
+  auto load_k = [&](size_t kp) __attribute__((always_inline)) {
+    const char* base = reinterpret_cast<const char*>(kcache) + kp * EB;
 #pragma unroll
-      for (int k2 = 0; k2 < KS / 2; ++k2) {
-        ra[k2] = *reinterpret_cast<const u32x4*>(kc + k2 * 64);
-        rb[k2] = *reinterpret_cast<const u32x4*>(kc + 4 * D + k2 * 64);
+    for (int k2 = 0; k2 < KL; ++k2) {
+      ra[k2] = *reinterpret_cast<const kraw*>(base + k_off + k2 * 64);
+      rb[k2] = *reinterpret_cast<const kraw*>(base + k_off + 4 * D * EB + k2 * 64);
+    }
+  };
+  auto load_v = [&](size_t kp) __attribute__((always_inline)) {
+    const char* base = reinterpret_cast<const char*>(vcache) + kp * EB;
+#pragma unroll
+    for (int j = 0; j < DB; ++j) rv[j] = *reinterpret_cast<const vraw*>(base + (j * 16 * PAGE * EB & ~4095) + v_off + (j * 16 * PAGE * EB & 4095));
+  };
+  auto page_step = [&](int p, size_t next, auto more_c) __attribute__((always_inline)) {
+    constexpr bool MORE = decltype(more_c)::value;  // another page follows
+    f32x4 sa = {0.f, 0.f, 0.f, 0.f}, sb = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (FP8) {
+#pragma unroll
+      for (int k2 = 0; k2 < KL; ++k2) {
+        sa = mfma16(fp8x8_to_bf16((u32x2){ra[k2][0], ra[k2][1]}), qf(2 * k2), sa);
+        sb = mfma16(fp8x8_to_bf16((u32x2){rb[k2][0], rb[k2][1]}), qf(2 * k2), sb);
+        sa = mfma16(fp8x8_to_bf16((u32x2){ra[k2][2], ra[k2][3]}), qf(2 * k2 + 1), sa);
+        sb = mfma16(fp8x8_to_bf16((u32x2){rb[k2][2], rb[k2][3]}), qf(2 * k2 + 1), sb);
       }
-#pragma unroll
-      for (int j = 0; j < DB; ++j) rv[j] = *reinterpret_cast<const u32x2*>(vc + j * 16 * PAGE);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int k2 = 0; k2 < KS / 2; ++k2) {
-        ka[2 * k2] = fp8x8_to_bf16((u32x2){ra[k2][0], ra[k2][1]});
-        ka[2 * k2 + 1] = fp8x8_to_bf16((u32x2){ra[k2][2], ra[k2][3]});
-        kb[2 * k2] = fp8x8_to_bf16((u32x2){rb[k2][0], rb[k2][1]});
-        kb[2 * k2 + 1] = fp8x8_to_bf16((u32x2){rb[k2][2], rb[k2][3]});
-      }
-#pragma unroll
-      for (int j = 0; j < DB; ++j) vt[j] = fp8x8_to_bf16(rv[j]);
     } else {
-      const bf16_t* kc = reinterpret_cast<const bf16_t*>(kcache) + kp + key_a * D + c * 8;
-      const bf16_t* vc = reinterpret_cast<const bf16_t*>(vcache) + kp + col * PAGE + c * 8;
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
-        ka[ks] = ld8(kc + ks * 32);
-        kb[ks] = ld8(kc + 4 * D + ks * 32);
+        sa = mfma16(ra[ks], qf(ks), sa);
+        sb = mfma16(rb[ks], qf(ks), sb);
       }
-#pragma unroll
-      for (int j = 0; j < DB; ++j) vt[j] = ld8(vc + j * 16 * PAGE);
-      __builtin_amdgcn_sched_barrier(0);
     }
-    f32x4 sa = {0.f, 0.f, 0.f, 0.f}, sb = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      sa = mfma16(ka[ks], qf[ks], sa);
-      sb = mfma16(kb[ks], qf[ks], sb);
+    if (MORE) {
+      __builtin_amdgcn_sched_barrier(0);
+      load_k(next);
+      __builtin_amdgcn_sched_barrier(0);
     }
     // lane (q = col, c): sa[r] = S[key 8c + r], sb[r] = S[key 8c + 4 + r]
     float s[8];
@@ -578,7 +599,27 @@ __global__ __launch_bounds__(64 * NW, (D > 128 ? 1 : 4)) void paged_decode_walk_
     l += ls;
     // O^T[d, q] += V^T[d, keys] . P^T[keys, q]
 #pragma unroll
-    for (int j = 0; j < DB; ++j) o[j] = mfma16(vt[j], pf, o[j]);
+    for (int j = 0; j < DB; ++j) {
+      if constexpr (FP8) o[j] = mfma16(fp8x8_to_bf16(rv[j]), pf, o[j]);
+      else o[j] = mfma16(rv[j], pf, o[j]);
+    }
+    if (MORE) {
+      __builtin_amdgcn_sched_barrier(0);
+      load_v(next);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  if (mine > 0) {
+    size_t kp = block_of(0);
+    load_k(kp);
+    load_v(kp);
+    __builtin_amdgcn_sched_barrier(0);
+    const int p0 = it.p_beg + wid;
+    for (int i = 0; i + 1 < mine; ++i) {
+      kp = block_of(i + 1);
+      page_step(p0 + NW * i, kp, std::true_type{});
+    }
+    page_step(p0 + NW * (mine - 1), 0, std::false_type{});
   }
   l = sum_xor16(l);  // l is a per-lane partial over this lane's keys: sum the 4 lanes that share a q
   l = sum_xor32(l);
