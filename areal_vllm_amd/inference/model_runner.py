@@ -647,12 +647,14 @@ class ModelRunner:
     def _decode_layers_fused(self, st: Dict[str, torch.Tensor], h: torch.Tensor, rope_pos: torch.Tensor):
         """All decoder layers of one decode step on the fused path -> final-normed hidden states [Bp, H].
 
-        Per layer: qkv GEMM with bias + RoPE + KV-cache write in its epilogue (smaller batches: split-K slabs ->
-        slab sum + bias + RoPE + KV-cache write) -> paged attention ->
+        Per layer: qkv GEMM with bias + RoPE + KV-cache write in its epilogue (between the few rows of ``decode_skinny.
+        qkv_row_tiles`` and the many of ``decode_gemm.QKV_ROPE_MIN_ROWS``: split-K slabs -> slab sum + bias + RoPE +
+        KV-cache write) -> paged attention ->
         o GEMM (slabs) -> slab sum + residual + RMSNorm -> gate|up GEMM with SwiGLU epilogue -> down GEMM
         (slabs) -> slab sum + residual + the NEXT layer's RMSNorm. Mixture-of-experts layers keep the attention
         half and run router and experts through the grouped kernels, then residual + the next norm."""
         from ..ops import decode_gemm as dg
+        from ..ops import decode_skinny as sk
 
         if self._skinny(h.shape[0]):
             return self._decode_layers_skinny(st, h, rope_pos)
@@ -677,9 +679,12 @@ class ModelRunner:
             return ops.rmsnorm(part, weight, eps, residual, gemma)
 
         x, residual = ops.rmsnorm(h, layers[0].ln1, eps, None, gemma)
+        qkv_tiles = sk.qkv_row_tiles(Bp, H, (hq + 2 * hkv) * D, D) if self.fused_qkv_rope else 0
         for li, blk in enumerate(layers):
             kc, vc = self.kv[li]
-            if self.fused_qkv_rope and Bp >= dg.QKV_ROPE_MIN_ROWS and H <= dg.QKV_ROPE_MAX_DEPTH:
+            if qkv_tiles:
+                q = sk.qkv_rope(x, blk.attn.qkv, blk.attn.qkv_bias, rope_pos, st["slots"], self.rope, kc, vc, hq, hkv, D, qkv_tiles)
+            elif self.fused_qkv_rope and Bp >= dg.QKV_ROPE_MIN_ROWS and H <= dg.QKV_ROPE_MAX_DEPTH:
                 q = dg.dgemm_qkv_rope(x, blk.attn.qkv, blk.attn.qkv_bias, rope_pos, st["slots"], self.rope, kc, vc,
                                       hq, hkv, D)
             else:

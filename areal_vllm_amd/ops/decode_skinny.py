@@ -90,3 +90,41 @@ def norm_qkv_rope(h: torch.Tensor, norm: torch.Tensor, w: torch.Tensor, bias: Op
         L.c_int(Hkv), L.c_int(D), L.c_int(table.max_pos), L.c_int(int(do_rope)), L.c_float(eps), L.c_int(int(gemma)),
         L.c_int(int(kcache.dtype == torch.float8_e4m3fn)), L.stream_ptr()), "skinny_norm_qkv")
     return q
+
+
+# One round of the chip's CUs, and as deep as the kernel is ahead of the split-K GEMM and its row kernel (figures at qkv_rows_kernel): with
+# 16 rows a workgroup up to 2304 deep (2304 to 4096 columns 9.0 / 8.1 us at 16 rows, 3584 to 4608 12.4 / 16.8), with 32 up to 1536
+# (2048 to 2560 columns at 64 rows 10.6 / 15.5); a second round is not (2048 to 3072 columns at 24 rows 8.7 / 10.7).
+QKV_ROWS_DEPTH = (2304, 1536)
+
+
+def qkv_row_tiles(M: int, K: int, N: int, head_dim: int) -> int:
+    """16-row tiles of a workgroup of `qkv_rope`, 0 where the split-K GEMM and its row kernel are the faster pair."""
+    if K % 64 == 0 and head_dim % 16 == 0:
+        for rt in (1, 2):
+            if K <= QKV_ROWS_DEPTH[rt - 1] and -(-M // (16 * rt)) * (N // 16) <= 256:
+                return rt
+    return 0
+
+
+def qkv_rope(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], positions, slots, table, kcache, vcache,
+             n_q_heads: int, n_kv_heads: int, head_dim: int, row_tiles: int, *, do_rope: bool = True) -> torch.Tensor:
+    """The packed q|k|v projection of `x` (normalised rows, any number of them) with bias; q and k rotated, k and v written into
+    the paged caches at ``slots`` (negative: not written); returns the rotated q ``[M, Hq, D]``."""
+    M, K = x.shape
+    Hq, Hkv, D = n_q_heads, n_kv_heads, head_dim
+    if not L.use_hip(x):
+        from .attention import rope_and_cache_write_
+
+        y = F.linear(x.float(), w.float(), None if bias is None else bias.float())
+        qkv = y.to(x.dtype).view(M, Hq + 2 * Hkv, D).contiguous()
+        return rope_and_cache_write_(qkv, positions, slots, table, kcache, vcache, Hq, Hkv, do_rope)[:, :Hq].contiguous()
+    assert x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.stride(1) == 1
+    assert w.is_contiguous() and w.shape == ((Hq + 2 * Hkv) * D, K) and (bias is None or bias.dtype == torch.bfloat16 and bias.is_contiguous())
+    assert positions.dtype == torch.int32 and slots.dtype == torch.int64 and positions.numel() >= M and slots.numel() >= M
+    q = torch.empty(M, Hq, D, dtype=x.dtype, device=x.device)
+    L.check(L.lib().areal_qkv_rows(
+        L.ptr(x), L.c_int64(x.stride(0)), L.ptr(w), L.ptr(bias), L.ptr(positions), L.ptr(slots), L.ptr(table.cos), L.ptr(table.sin),
+        L.ptr(q), L.ptr(kcache), L.ptr(vcache), L.c_int(M), L.c_int(K), L.c_int(Hq), L.c_int(Hkv), L.c_int(D), L.c_int(table.max_pos),
+        L.c_int(int(do_rope)), L.c_int(int(kcache.dtype == torch.float8_e4m3fn)), L.c_int(row_tiles), L.stream_ptr()), "qkv_rows")
+    return q

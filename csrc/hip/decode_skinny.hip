@@ -95,6 +95,38 @@ DEVINL float dot8(bf16x8 a, bf16x8 b, float c) {
   return c;
 }
 
+// Members d and d + D / 2 of a head of row m: bias (0: none), rotation (c = 1, s = 0 where none is wanted; V heads have none), q to
+// a.Y, k and v to their page.
+DEVINL void put_pair(const SKArgs& a, int head, int d, int m, float lo, float hi, float bias_lo, float bias_hi, float c, float s,
+                     int64_t slot) {
+  const int half = a.D >> 1;
+  lo = bf2f(f2bf(lo + bias_lo));  // the unfused path carries the projection as a bf16 tensor
+  hi = bf2f(f2bf(hi + bias_hi));
+  if (a.do_rope && head < a.Hq + a.Hkv) {
+    const float x = lo;
+    lo = x * c - hi * s;
+    hi = hi * c + x * s;
+  }
+  if (head < a.Hq) {
+    bf16_t* q = a.Y + ((size_t)m * a.Hq + head) * a.D + d;
+    q[0] = f2bf(lo);
+    q[half] = f2bf(hi);
+    return;
+  }
+  if (slot < 0) return;
+  const int64_t page = slot / 32;
+  const int off = (int)(slot % 32);
+  if (head < a.Hq + a.Hkv) {
+    const size_t at = (((size_t)page * a.Hkv + head - a.Hq) * 32 + off) * a.D + d;
+    st1_cache(a.kcache, at, bf2f(f2bf(lo)), a.fp8);  // fp8: from the bf16 value, as the other writers
+    st1_cache(a.kcache, at + half, bf2f(f2bf(hi)), a.fp8);
+  } else {
+    const size_t at = (((size_t)page * a.Hkv + head - a.Hq - a.Hkv) * a.D + d) * 32 + off;
+    st1_cache(a.vcache, at, lo, a.fp8);
+    st1_cache(a.vcache, at + (size_t)half * 32, hi, a.fp8);
+  }
+}
+
 // What follows the projection; sum(j, h, m): the fp32 sum of column j (SK_GATED: of half h; SK_QKV: member h of pair j) of
 // row m, read from LDS.
 template <int MODE, typename Sum>
@@ -121,40 +153,15 @@ DEVINL void finish(const SKArgs& a, Sum sum) {
     const int head = blockIdx.x / per, d0 = (blockIdx.x % per) * a.cols;
     for (int i = threadIdx.x; i < a.cols * a.M; i += THREADS) {
       const int j = i % a.cols, m = i / a.cols, d = d0 + j;
-      float lo = sum(j, 0, m), hi = sum(j, 1, m);
-      if (a.bias) {
-        lo += bf2f(a.bias[head * a.D + d]);
-        hi += bf2f(a.bias[head * a.D + d + half]);
-      }
-      lo = bf2f(f2bf(lo));  // the unfused path carries the projection as a bf16 tensor
-      hi = bf2f(f2bf(hi));
+      float c = 1.f, s = 0.f;
       if (a.do_rope && head < a.Hq + a.Hkv) {
         int p = a.pos[m];
         p = p < 0 ? 0 : (p >= a.max_pos ? a.max_pos - 1 : p);
-        const float c = a.cos_t[(size_t)p * half + d], s = a.sin_t[(size_t)p * half + d];
-        const float x = lo;
-        lo = x * c - hi * s;
-        hi = hi * c + x * s;
+        c = a.cos_t[(size_t)p * half + d];
+        s = a.sin_t[(size_t)p * half + d];
       }
-      if (head < a.Hq) {
-        bf16_t* q = a.Y + ((size_t)m * a.Hq + head) * a.D + d;
-        q[0] = f2bf(lo);
-        q[half] = f2bf(hi);
-        continue;
-      }
-      const int64_t slot = a.slots[m];
-      if (slot < 0) continue;
-      const int64_t page = slot / 32;
-      const int off = (int)(slot % 32);
-      if (head < a.Hq + a.Hkv) {
-        const size_t at = (((size_t)page * a.Hkv + head - a.Hq) * 32 + off) * a.D + d;
-        st1_cache(a.kcache, at, bf2f(f2bf(lo)), a.fp8);  // fp8: from the bf16 value, as the other writers
-        st1_cache(a.kcache, at + half, bf2f(f2bf(hi)), a.fp8);
-      } else {
-        const size_t at = (((size_t)page * a.Hkv + head - a.Hq - a.Hkv) * a.D + d) * 32 + off;
-        st1_cache(a.vcache, at, lo, a.fp8);
-        st1_cache(a.vcache, at + (size_t)half * 32, hi, a.fp8);
-      }
+      put_pair(a, head, d, m, sum(j, 0, m), sum(j, 1, m), a.bias ? bf2f(a.bias[head * a.D + d]) : 0.f,
+               a.bias ? bf2f(a.bias[head * a.D + d + half]) : 0.f, c, s, head < a.Hq ? -1 : a.slots[m]);
     }
   }
 }
@@ -442,6 +449,120 @@ __global__ __launch_bounds__(THREADS) void skinny_mfma_kernel(const SKArgs a) {
   });
 }
 
+// The packed q|k|v projection of rows that are normalised already, with bias, rotation and KV-cache write: a workgroup owns 16 RT
+// rows and 8 rotated pairs over all of K, its 8 waves deal the 64-deep chunks of K among themselves, every operand goes from memory
+// to the registers of the one wave that multiplies it (up to 1536 deep all of them at once), and the partial sums meet in LDS.
+// What bounds it: one round trip to memory and the load path of a CU, 32 K (1 + RT) bytes a workgroup; the split-K GEMM and the row
+// kernel behind it that this replaces are two launches and a round trip of fp32 slabs. Captured, cold weights, us of the two / this:
+// 1536 deep to 2048 columns 9 / 16 / 24 / 32 / 48 / 64 rows 7.2 / 5.3, 7.4 / 5.8, 7.5 / 5.9, 7.5 / 6.1, 8.2 / 7.8, 8.5 / 8.2; 896 to
+// 1152 9 / 48 / 96 rows 6.3 / 4.3, 7.5 / 4.8, 7.9 / 6.2; 1024 to 4096 16 / 32 rows 7.4 / 5.1, 8.5 / 7.1; 2048 to 2560 16 rows 8.6 / 7.6.
+// 32 columns a workgroup or 64 rows (fewer loads of the other operand) were slower wherever one round of workgroups is enough
+// (24 rows of the first: 7.4 to 8.7), and beyond that the split-K GEMM is ahead (128 rows 10.2 / 11.1).
+template <int RT>
+__global__ __launch_bounds__(THREADS, 4) void qkv_rows_kernel(const SKArgs a) {
+  constexpr int PAIRS = 8, ITEMS = 16 * RT * PAIRS, NI = (ITEMS + THREADS - 1) / THREADS, U = 3;
+  __shared__ f32x4 red[WAVES * RT * 64];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & 15, kq = lane >> 4;
+  const int half = a.D >> 1, per = half / PAIRS, nrb = (a.M + 16 * RT - 1) / (16 * RT), ncb = (a.N >> 1) / PAIRS;
+  // the blocks of an XCD: a range of columns, all rows of it one after the other
+  const int q8 = gridDim.x >> 3, id = (blockIdx.x & 7) * q8 + (blockIdx.x >> 3);
+  const int cb = id / nrb, m0 = (id - cb * nrb) * 16 * RT;
+  if (cb >= ncb) return;
+  const int head = cb / per, d0 = (cb - head * per) * PAIRS;
+  const int nchunk = a.K >> 6;
+  const int mine = wave < nchunk ? (nchunk - wave + WAVES - 1) / WAVES : 0;
+  const bool rot = a.do_rope && head < a.Hq + a.Hkv;
+
+  // what the results need: on its way ahead of the operands
+  int pos[NI];
+  int64_t slot[NI];
+  float blo[NI], bhi[NI];
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int idx = threadIdx.x + i * THREADS, m = min(m0 + idx / PAIRS, a.M - 1), d = d0 + idx % PAIRS;
+    pos[i] = rot ? a.pos[m] : 0;
+    slot[i] = head < a.Hq ? -1 : a.slots[m];
+    blo[i] = a.bias ? bf2f(a.bias[head * a.D + d]) : 0.f;
+    bhi[i] = a.bias ? bf2f(a.bias[head * a.D + d + half]) : 0.f;
+  }
+  const bf16_t* wp = a.W + (size_t)(head * a.D + d0 + (r & 7) + (r >> 3) * half) * a.K + 8 * kq;  // pair j: rows j and j + 8 of the tile
+  const bf16_t* xp[RT];
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) xp[rt] = a.X + (size_t)min(m0 + rt * 16 + r, a.M - 1) * a.xs + 8 * kq;  // (rows past the last repeat it)
+  __builtin_amdgcn_sched_barrier(0);
+
+  bf16x8 wf[U][2], xf[U][2][RT];
+  auto load = [&](int u, int i) __attribute__((always_inline)) {
+    const int k = (wave + WAVES * i) * 64;
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      wf[u][s] = ld8(wp + k + 32 * s);
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) xf[u][s][rt] = ld8(xp[rt] + k + 32 * s);
+    }
+  };
+  f32x4 acc[RT];
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) acc[rt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto multiply = [&](int u) __attribute__((always_inline)) {
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) acc[rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[u][s], xf[u][s][rt], acc[rt], 0, 0, 0);
+  };
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (u < mine) load(u, u);
+  __builtin_amdgcn_sched_barrier(0);
+  float c[NI], s[NI];
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int p = pos[i] < 0 ? 0 : (pos[i] >= a.max_pos ? a.max_pos - 1 : pos[i]), d = d0 + (threadIdx.x + i * THREADS) % PAIRS;
+    c[i] = rot ? a.cos_t[(size_t)p * half + d] : 1.f;
+    s[i] = rot ? a.sin_t[(size_t)p * half + d] : 0.f;
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  int i = 0;
+  for (; i + 2 * U <= mine; i += U)
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      multiply(u);
+      __builtin_amdgcn_sched_barrier(0);
+      load(u, i + U + u);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (i + u < mine) {
+      multiply(u);
+      if (i + U + u < mine) load(u, i + U + u);
+    }
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (i + U + u < mine) multiply(u);
+
+  // partial sums: [wave][row tile][lane] of 4 (weight row 4 kq + e, row r)
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) red[(wave * RT + rt) * 64 + lane] = acc[rt];
+  __syncthreads();
+  const float* rf = reinterpret_cast<const float*>(red);
+#pragma unroll
+  for (int n = 0; n < NI; ++n) {
+    const int idx = threadIdx.x + n * THREADS, m = idx / PAIRS, j = idx % PAIRS;
+    if (idx >= ITEMS || m0 + m >= a.M) continue;
+    float v[2] = {0.f, 0.f};
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int row = j + 8 * h, at = (m >> 4) * 256 + ((row >> 2) * 16 + (m & 15)) * 4 + (row & 3);
+#pragma unroll
+      for (int w = 0; w < WAVES; ++w) v[h] += rf[w * RT * 256 + at];
+    }
+    put_pair(a, head, d0 + j, m0 + m, v[0], v[1], blo[n], bhi[n], c[n], s[n], slot[n]);
+  }
+}
+
 template <int MT, int RB, bool NORM, int MODE>
 int sk_dot(SKArgs& a, int blocks, hipStream_t st) {
   a.wk = 1;
@@ -527,4 +648,22 @@ extern "C" int areal_skinny_norm_qkv(const void* X, int64_t xs, const void* nw, 
   if (M == 1) return sk_dot<1, 1, true, SK_QKV>(a, blocks, st);
   if (M == 2) return sk_dot<2, 1, true, SK_QKV>(a, blocks, st);
   return sk_mfma<1, 3, true, true, SK_QKV>(a, blocks, st);
+}
+
+// The same of rows that are normalised already, any number of them: 16 rt rows (rt 1 or 2) and 8 pairs a workgroup. D a multiple of 16.
+extern "C" int areal_qkv_rows(const void* X, int64_t xs, const void* W, const void* bias, const int* pos, const int64_t* slots,
+                              const float* cos_t, const float* sin_t, void* Y, void* kcache, void* vcache, int M, int K, int Hq,
+                              int Hkv, int D, int max_pos, int do_rope, int fp8, int rt, hipStream_t st) {
+  if (M < 1 || K < 64 || K % 64 != 0 || xs % 8 != 0 || D < 16 || D % 16 != 0 || (rt != 1 && rt != 2)) return -1;
+  if (((uintptr_t)X | (uintptr_t)W) % 16 != 0) return -2;
+  SKArgs a = {};
+  a.X = (const bf16_t*)X; a.xs = xs; a.W = (const bf16_t*)W; a.bias = (const bf16_t*)bias; a.Y = (bf16_t*)Y; a.M = M;
+  a.N = (Hq + 2 * Hkv) * D; a.K = K; a.pos = pos; a.slots = slots; a.cos_t = cos_t; a.sin_t = sin_t; a.kcache = kcache;
+  a.vcache = vcache; a.Hq = Hq; a.Hkv = Hkv; a.D = D; a.max_pos = max_pos; a.do_rope = do_rope; a.fp8 = fp8;
+  const long blocks = (long)((M + 16 * rt - 1) / (16 * rt)) * (a.N / 16);
+  if (blocks > 0x7ffffff0l) return -1;
+  const dim3 grid((unsigned)((blocks + 7) / 8 * 8));
+  if (rt == 1) hipLaunchKernelGGL(qkv_rows_kernel<1>, grid, dim3(THREADS), 0, st, a);
+  else hipLaunchKernelGGL(qkv_rows_kernel<2>, grid, dim3(THREADS), 0, st, a);
+  return (int)hipGetLastError();
 }
