@@ -2,8 +2,8 @@
 
 Forward, ``dx`` (on the untransposed weights) and ``dW`` of all experts are one launch each (tiles never straddle experts): the
 trainer's 256 x 256 tiles (``csrc/hip/train_gemm.hip``) from 128 rows an expert on, the kernels of ``csrc/hip/grouped_gemm.hip``
-below (dW of expert shapes that are no multiples of 128: per expert with library GEMMs). Counterpart of
-``grouped_gemm.ops.gmm`` in the reference
+below (dW into an fp32 gradient: tiles of 128 x 128 of ``train_gemm.hip``; dW of expert shapes that are no multiples of 128: per
+expert with library GEMMs). Counterpart of ``grouped_gemm.ops.gmm`` in the reference
 (``realhf/impl/model/modules/moe/experts.py:195-210``).
 """
 import math
@@ -40,15 +40,17 @@ def _hip_ok(x, w) -> bool:
 # 2048 columns, 768 deep (132 and 264 in all) 21 / 25 and 40 / 44; 16 of 200, 1536 columns (123) 24 / 25; 16 of 400, 2816 columns, 512
 # deep (363) 46 / 35.
 BIG_MIN_ROWS, BIG_MIN_FILL = 128, 0.54
-# dW of experts with few rows is all reading and writing of the gradient, which the small tiles (two workgroups a CU) overlap
-# better, large experts' up to many rows. us of the small ones / of these: 16 experts, 1536 columns, 768 deep, 128 / 200 / 400 / 800 rows
-# 40, 43, 53, 79 / 50, 53, 60, 75 (288 tiles); 128 of them 250, 278, 366, 557 / 260, 280, 310, 399; 8 experts, 28672 columns, 4096
-# deep, 256 / 1024 / 2048 rows 1569 / 3397 / 5774 and 1860 / 3655 / 4938.
+# dW in fp32, tiles of 256 x 256 / of 128 x 128 (several on a CU, whose products run beside one another's gradients), us: 128 experts of
+# 1536 columns, 2048 deep, 128 / 400 / 700 / 1024 / 2048 rows 647 / 548, 840 / 680, 1006 / 863, 1147 / 1076, 1684 / 1833 (the large ones streamed
+# past the caches 553, 810, 949, 1092, 1624); 2048 columns, 768 deep 341 / 285, 420 / 349, 492 / 449, 574 / 562, 871 / 991; 8 of 28672 columns, 4096
+# deep, 400 / 1024 / 2048 rows 1929 / 1352, 2694 / 2285, 3847 / 4074; 16 of 1536 columns, 768 deep, 1024 rows 69 / 56.
+FEW_WGRAD_ROWS = 1024
+# What else the large ones ask for; their experts may be large from many rows on only.
 BIG_WGRAD_MIN_ROWS, BIG_WGRAD_MAX_SIZE, BIG_WGRAD_ANY_SIZE_ROWS = 384, 1 << 24, 2048
 # A tile of dW is reduced by one workgroup: behind an expert with many times the mean's rows the chip waits for its few large
-# tiles. us of the small / the large ones, largest expert 2.6 / 6 / 13 / 24 / 53 means (forward and dx gain as with even rows):
-# 128 experts, 1024 rows on average, 1536 columns, 2048 deep 1552, 1565, 1549, 1579, 2001 and 1174, 1337, 1605, 1869, 3021; 64
-# experts of 768 rows, 2816 columns, 2.2 / 4.4 / 8.1 / 13.5 / 27 means 1151, 1153, 1158, 1212, 1316 and 893, 1007, 1155, 1389, 1882.
+# tiles. us of tiles of 128 x 128 (each expert's on all XCDs) / the large ones, largest expert 4 / 8 / 16 / 53 means: 128 experts, 1400
+# rows on average, 1536 columns, 2048 deep 1473, 1476, 1483, 1745 and 1412, 1603, 1845, 3032; 2048 columns, 768 deep 874, 878, 930, 1443 and
+# 712, 801, 899, 1455; 64 of 2816 columns, 2048 deep 1233, 1266, 1317, 1481 and 1340, 1542, 1939, 3174.
 BIG_WGRAD_CROWDED = 8
 
 
@@ -66,6 +68,16 @@ def _big_wgrad(T: int, E: int, N: int, K: int, counts: List[int]) -> bool:
     return (T >= BIG_WGRAD_MIN_ROWS * E and K % 256 == 0 and (N * K <= BIG_WGRAD_MAX_SIZE or T >= BIG_WGRAD_ANY_SIZE_ROWS * E)
             and _rounds_filled(E * -(-N // 256) * (K // 256)) and max(counts) * E <= BIG_WGRAD_CROWDED * T
             and "AREAL_GROUPED_GEMM_TILE_M" not in os.environ)
+
+
+def _spread_experts(T: int, E: int, N: int, K: int, counts: List[int]) -> bool:
+    """Whether each expert's tiles of 128 x 128 are dealt to all XCDs, not several experts to one. The other XCDs wait for that of a
+    crowded expert; its operands pass through eight L2s instead. us dealt by experts / over all, largest expert 1 / 4 / 8 / 16 means:
+    128 experts of 500 rows, 1536 columns, 2048 deep (192 tiles) 744 / 725, 786 / 728, 854 / 722, 966 / 729; 2048 columns, 768 deep
+    (96) 387 / 424, 410 / 422, 444 / 422, 511 / 424; 8 of 500, 4096 columns, 14336 deep 769 / 796, 1319 / 837, 1756 / 897; 32 of 500,
+    1024 by 1024 (64 tiles) 63 / 82, 70 / 83, 89 / 98, 116 / 122."""
+    tiles = N // 128 * (K // 128)
+    return tiles >= 80 and max(counts) * E > (6 if tiles < 128 else 3 if tiles < 1024 else 1.5) * T
 
 
 def big_grouped(x: torch.Tensor, w: torch.Tensor, offsets: torch.Tensor, nn: bool) -> torch.Tensor:
@@ -141,23 +153,25 @@ class _GroupedGemmFn(torch.autograd.Function):
         if ctx.needs_input_grad[1]:
             if N % 128 == 0 and K % 128 == 0 and x.shape[0] > 0:
                 # dW[e] = dy_e^T . x_e for all experts in one launch (csrc/hip/grouped_gemm.hip); when the weight
-                # carries an fp32 `main_grad` view the kernel adds into it (no bf16 dW, no separate add kernel)
+                # carries an fp32 `main_grad` view the kernel (csrc/hip/train_gemm.hip) adds into it (no bf16 dW, no separate
+                # add kernel)
                 mg = _fold_target(w)
-                dst = mg if mg is not None else torch.empty_like(w)
-                if mg is not None and _big_wgrad(x.shape[0], E, N, K, ctx.counts):
-                    L.check(L.lib().areal_tgemm_grouped_wgrad(L.ptr(dy), L.ptr(x), L.ptr(mg), L.ptr(offsets), L.c_int(E),
-                                                              L.c_int(N), L.c_int(K), L.c_int64(mg.stride(0)),
-                                                              L.stream_ptr()), "tgemm_grouped_wgrad")
-                    _after_fold(w)
-                    return dx, None, None, None
-                L.check(L.lib().areal_grouped_gemm_wgrad(L.ptr(dy), L.ptr(x), L.ptr(dst), L.ptr(offsets),
-                                                         L.c_int(x.shape[0]), L.c_int(E), L.c_int(N), L.c_int(K),
-                                                         L.c_int64(dst.stride(0)), L.c_int(int(mg is not None)),
-                                                         L.stream_ptr()), "grouped_gemm_wgrad")
                 if mg is not None:
+                    T = x.shape[0]
+                    if T >= FEW_WGRAD_ROWS * E and _big_wgrad(T, E, N, K, ctx.counts):
+                        L.check(L.lib().areal_tgemm_grouped_wgrad(L.ptr(dy), L.ptr(x), L.ptr(mg), L.ptr(offsets), L.c_int(E),
+                                                                  L.c_int(N), L.c_int(K), L.c_int64(mg.stride(0)),
+                                                                  L.stream_ptr()), "tgemm_grouped_wgrad")
+                    else:
+                        L.check(L.lib().areal_tgemm_grouped_wgrad_few(
+                            L.ptr(dy), L.ptr(x), L.ptr(mg), L.ptr(offsets), L.c_int(E), L.c_int(N), L.c_int(K), L.c_int64(mg.stride(0)),
+                            L.c_int(int(_spread_experts(T, E, N, K, ctx.counts))), L.stream_ptr()), "tgemm_grouped_wgrad_few")
                     _after_fold(w)
                 else:
-                    dw = dst
+                    dw = torch.empty_like(w)
+                    L.check(L.lib().areal_grouped_gemm_wgrad(L.ptr(dy), L.ptr(x), L.ptr(dw), L.ptr(offsets),
+                                                             L.c_int(x.shape[0]), L.c_int(E), L.c_int(N), L.c_int(K),
+                                                             L.c_int64(dw.stride(0)), L.stream_ptr()), "grouped_gemm_wgrad")
             else:
                 dw = torch.zeros_like(w)
                 s = 0

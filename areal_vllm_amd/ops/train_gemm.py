@@ -105,11 +105,30 @@ def _tile_plan(pairs: int, tiles: int, flush: int, rows: int = 256) -> Tuple[flo
     return best
 
 
+def _wgrad_few(M: int, tiles: int) -> bool:
+    """Whether `tiles` of 128 x 128, several on a CU, are the better ones over M tokens; us of the tiles of 256 x 256 / of these, the
+    gradient not in the caches. Up to three tiles a CU, where the large ones would need parts: 2 tiles, 600 / 1024 tokens 10.5 /
+    9.6, 11.7 / 14; 16 tiles, 600 / 1024 / 1500 13.5 / 10, 16.4 / 14.6, 17.1 / 19.7; 64, 1500 / 2048 23.2 / 20.3, 23.4 / 25.7; 144, 2048 /
+    3000 31 / 27, 35.7 / 37.1; 256, 2048 / 3072 40 / 29, 45 / 39; 456, 3000 65 / 49; 768, 3072 / 78 / 76. Not where they fill most of
+    one round: 840, 700 / 1024 38.3 / 37, 43.4 / 44.5, and with the gradient in the memory-side cache 34 / 37. More: 1200, 1500 88 / 73;
+    1680, 700 / 1500 / 2048 78 / 61, 107 / 93, 127 / 117; 5504, 1024 / 1500 / 2048 270 / 211, 330 / 293, 394 / 392; but full rounds,
+    1008, 1024 / 1500 51 / 47, 61 / 59; 14244, 1024 / 1500 637 / 599, 789 / 798."""
+    if tiles <= 768:
+        return M <= min(3072, 600 + 11 * tiles)
+    filled = tiles / 1024 / -(-tiles // 1024)
+    return tiles >= 960 and M <= (1536 if filled <= 0.92 else 1024)
+
+
 def tgemm_wgrad_(acc: torch.Tensor, dy: torch.Tensor, x: torch.Tensor, splits: int = 0) -> torch.Tensor:
     """acc[N, K] (fp32) += dy[M, N]^T @ x[M, K]: the weight gradient of ``y = x @ W^T`` summed straight into the
     fp32 gradient buffer. `splits`: parts of the token range for every tile (0: chosen)."""
     assert wgrad_supported(dy, x, acc)
     (M, N), K = dy.shape, x.shape[1]
+    if not splits and _wgrad_few(M, N // 128 * (K // 128)):
+        L.check(L.lib().areal_tgemm_wgrad_few(L.ptr(dy), L.c_int64(dy.stride(0)), L.ptr(x), L.c_int64(x.stride(0)), L.ptr(acc),
+                                              L.c_int64(acc.stride(0)), L.c_int(M), L.c_int(N), L.c_int(K), L.stream_ptr()),
+                "tgemm_wgrad_few")
+        return acc
     pairs, tiles = -(-M // 128), -(-N // 256) * (K // 256)
     if splits:
         splits = _even_splits(pairs, splits)

@@ -622,6 +622,7 @@ struct TWArgs {
 };
 
 typedef f32x4 __attribute__((aligned(4))) f32x4u;
+constexpr long TG_STREAM = 1l << 26;  // elements of an fp32 gradient that the memory-side cache cannot hold
 
 DEVINL void tg_wgrad_origin(const TWArgs& a, int wg, int& n0, int& k0) {
   const int per_band = TG_GROUP_M * a.tiles_k;
@@ -632,7 +633,10 @@ DEVINL void tg_wgrad_origin(const TWArgs& a, int wg, int& n0, int& k0) {
   k0 = (in_band / rows) * 256;
 }
 
-template <bool GRP>
+// NT: a gradient larger than the 256 MB of the memory-side cache is streamed past the caches (us, 151936 x 1536, 1024 / 2048 / 4096 / 16384
+// tokens 637 / 594, 949 / 925, 1662 / 1605, 5726 / 5728; 128 experts of 1536 x 2048, 1024 rows each 1131 / 1076). A smaller one may be
+// there still, from its clearing or the last pass: 17920 x 1536, 1024 tokens 74 us, streamed 86.
+template <bool GRP, bool NT>
 __global__ __launch_bounds__(512) void tgemm_wgrad_kernel(const TWArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int lane = threadIdx.x & 63;
@@ -831,12 +835,22 @@ __global__ __launch_bounds__(512) void tgemm_wgrad_kernel(const TWArgs a) {
     for (int i0 = 0; i0 < 16; i0 += 8) {
       f32x4 old[8];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) old[i] = *reinterpret_cast<const f32x4u*>(op + (size_t)((i0 + i) * 4 + fq) * a.ldw + fr * 4);
+      for (int i = 0; i < 8; ++i) {
+        const f32x4u* p = reinterpret_cast<const f32x4u*>(op + (size_t)((i0 + i) * 4 + fq) * a.ldw + fr * 4);
+        if constexpr (NT)
+          old[i] = __builtin_nontemporal_load(p);
+        else
+          old[i] = *p;
+      }
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         const int row = (i0 + i) * 4 + fq;
         const f32x4 v = *reinterpret_cast<const f32x4*>(ob + row * 256 + ((fr ^ (row & 15)) << 4));
-        *reinterpret_cast<f32x4u*>(op + (size_t)row * a.ldw + fr * 4) = old[i] + v;
+        f32x4u* p = reinterpret_cast<f32x4u*>(op + (size_t)row * a.ldw + fr * 4);
+        if constexpr (NT)
+          __builtin_nontemporal_store(old[i] + v, p);
+        else
+          *p = old[i] + v;
       }
     }
   };
@@ -866,6 +880,143 @@ __global__ __launch_bounds__(256) void tgemm_wgrad_sum_kernel(const TWArgs a) {
   }
   *o0 = d0 + v0;
   *o1 = d1 + v1;
+}
+
+// =====================================================================================
+// Weight gradient over few tokens: tiles of 128 x 128, a workgroup of 4 waves (2 x 2, 64 x 64 each), three or four of them on a CU.
+//
+// Over few tokens the fp32 gradient is what moves: it is read and written once, 5 to 50 times the operands' bytes. The kernel above has
+// one workgroup a CU, whose gradient passes behind its products, not beside them, and few tiles need parts and a second launch. Here
+// one workgroup's products run beside another's gradient. A ring of S stages of 32 tokens, one barrier a stage; the gradient is
+// streamed past the L2 (nontemporal: nothing reads it again soon, and the operands' panels stay there). What bounds it: the
+// memory up to some 700 tokens, above that the LDS (32 KiB read and 16 KiB written a stage for 256 cycles of products: 6 us a tile
+// and 1024 tokens with the CU full). us, gradient not in the caches, kernel above / this one: 17920 x 1536, 256 / 700 / 1500 tokens
+// 59 / 48, 78 / 61, 107 / 93; 2048 x 1536 19 / 9.3, 28 / 14, 31 / 22; 151936 x 1536 425 / 340, 572 / 436, 789 / 798. Without
+// streaming 700 tokens take 68, 15 and 514 us. S: 2 stages leave room for four workgroups, 3 for three, better where there are no
+// more than three a CU (2048 x 1536, 1500 tokens 26 / 22; 22016 x 4096, 700 tokens 164 / 175; 4 stages 206).
+// Sums are taken over all tokens in their order, as in a whole tile above.
+//
+// GRP: routed experts' gradients, rows sorted by expert. us, 128 experts of 1536 x 2048, 64 / 256 / 512 / 700 rows an expert, kernel
+// above / this one: 618 / 550, 710 / 561, 862 / 746, 992 / 871.
+// =====================================================================================
+constexpr int TWF_STAGE = 16 * 1024;  // 32 tokens x 128 columns of both operands
+
+template <bool GRP, int S>
+__global__ __launch_bounds__(256, S == 2 ? 4 : 3) void tgemm_wgrad_few_kernel(const TWArgs a) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wr = wave >> 1, wc = wave & 1, fr = lane & 15, fq = lane >> 4;
+
+  // ---- id -> tile: contiguous ranges per XCD, walked in bands of 8 tile rows. Ranges of all experts' tiles (an expert's operands then
+  // pass through one L2), or, where an expert alone has many, of each expert's: a crowded expert would keep one XCD busy
+  int nb = gridDim.x, id = blockIdx.x, e = 0;
+  if (GRP && a.chunk) {
+    nb = a.tiles_n * a.tiles_k;
+    e = id / nb;
+    id -= e * nb;
+  }
+  const int xq = nb >> 3, xr = nb & 7, xx = id & 7;
+  int b = (xx < xr ? xx * (xq + 1) : xr * (xq + 1) + (xx - xr) * xq) + (id >> 3);
+  int row_lo = 0, row_hi = a.M;
+  float* dW = a.dW;
+  if (GRP) {
+    if (!a.chunk) {
+      const int per = a.tiles_n * a.tiles_k;
+      e = b / per;
+      b -= e * per;
+    }
+    row_lo = a.offsets[e];
+    row_hi = a.offsets[e + 1];
+    if (row_hi <= row_lo) return;  // an expert without rows adds nothing
+    dW += e * a.stride;
+  }
+  const int per_band = 8 * a.tiles_k, band = b / per_band, in_band = b - band * per_band;
+  const int band_rows = min(a.tiles_n - band * 8, 8);
+  const int n0 = (band * 8 + in_band % band_rows) * 128, k0 = in_band / band_rows * 128;
+
+  // ---- staging: thread -> token row (wave * 4 + lane / 16) of a 16-row issue; rows past the last token are out of the buffer's
+  // range and write zeros (as in tgemm_wgrad_kernel)
+  const int srow = wave * 4 + fq, pc = (fr ^ ((fq << 2) | wave)) * 8;
+  const int tokens = row_hi - row_lo;
+  const bf16_t* pA = a.dY + (size_t)row_lo * a.ldy + n0;
+  const bf16_t* pB = a.X + (size_t)row_lo * a.ldx + k0;
+  const unsigned rowA = (unsigned)a.ldy * 2, rowB = (unsigned)a.ldx * 2;  // bytes
+  const unsigned vA = srow * rowA + pc * 2, vB = srow * rowB + pc * 2;
+  auto stage = [&](int slot, int t) __attribute__((always_inline)) {
+    char* dst = smem + slot * TWF_STAGE + wave * 1024;
+    const int rows = min(tokens - t * 32, 32);
+    const unsigned ra = rows > 0 ? (rows - 1) * rowA + 256 : 0u, rb = rows > 0 ? (rows - 1) * rowB + 256 : 0u;
+    const auto sa = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(pA + (size_t)t * 16 * rowA), 0, ra, 0x00020000);
+    const auto sb = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(pB + (size_t)t * 16 * rowB), 0, rb, 0x00020000);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(sa, (lptr_t)dst, 16, vA, 0, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(sa, (lptr_t)(dst + 4096), 16, vA + 16 * rowA, 0, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(sb, (lptr_t)(dst + 8192), 16, vB, 0, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(sb, (lptr_t)(dst + 12288), 16, vB + 16 * rowB, 0, 0, 0);
+  };
+
+  int a_adr[4][2], b_adr[4][2];  // [16-column tile][token half]
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int h2 = 0; h2 < 2; ++h2) {
+      a_adr[i][h2] = (int)(tr_addr((const char*)0, 8 * fq + 4 * h2, wr * 64 + i * 16, fr) - (const char*)0);
+      b_adr[i][h2] = (int)(tr_addr((const char*)0, 8 * fq + 4 * h2, wc * 64 + i * 16, fr) - (const char*)0);
+    }
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(lptr_t)smem;
+  f32x4 acc[4][4] = {};  // [n tile][k tile]
+
+  const int KT = (tokens + 31) >> 5;
+#pragma unroll
+  for (int i = 0; i < S - 1; ++i) stage(i, i);
+  int slot = 0;
+  for (int t = 0; t < KT; ++t) {
+    tg_vmcnt<4 * (S - 2)>();
+    tg_barrier();  // stage t is complete; everyone has read stage t - 1, which the next request overwrites
+    const int next = slot == 0 ? S - 1 : slot - 1;
+    stage(next, t + S - 1);
+    const uint32_t p = lds0 + slot * TWF_STAGE;
+    bf16x8 af[4], bf[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) bf[i] = cat4(tg_tr(p + b_adr[i][0], 8192), tg_tr(p + b_adr[i][1], 8192));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) af[i] = cat4(tg_tr(p + a_adr[i][0], 0), tg_tr(p + a_adr[i][1], 0));
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+      for (int nt = 0; nt < 4; ++nt) acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[nt], af[mt], acc[mt][nt], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    slot = slot == S - 1 ? 0 : slot + 1;
+  }
+  tg_vmcnt<0>();
+
+  // ---- lane (fr, fq) of tile (mt, nt) holds 4 consecutive k columns of row fr; 32 rows at a time pass through 8 KiB of LDS, after
+  // which an instruction moves 256 bytes of four rows
+  float* op = dW + (size_t)(n0 + wr * 64 + fq) * a.ldw + k0 + wc * 64 + fr * 4;
+  f32x4 old[16];
+  auto fetch = [&](int i0, int i1) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = i0; i < i1; ++i) old[i] = __builtin_nontemporal_load(reinterpret_cast<const f32x4u*>(op + (size_t)i * 4 * a.ldw));
+  };
+  fetch(0, S == 2 ? 8 : 16);  // (four workgroups a CU: 128 registers)
+  tg_barrier();               // from here on nobody reads a stage
+  char* ob = smem + wave * 8192;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    if (S == 2 && h == 1) fetch(8, 16);
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+      for (int nt = 0; nt < 4; ++nt) *reinterpret_cast<f32x4*>(ob + (m * 16 + fr) * 256 + (((nt * 4 + fq) ^ fr) << 4)) = acc[h * 2 + m][nt];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int row = i * 4 + fq;
+      const f32x4 v = *reinterpret_cast<const f32x4*>(ob + row * 256 + ((fr ^ (row & 15)) << 4));
+      __builtin_nontemporal_store(old[h * 8 + i] + v, reinterpret_cast<f32x4u*>(op + (size_t)(h * 8 + i) * 4 * a.ldw));
+    }
+  }
 }
 
 // =====================================================================================
@@ -1084,11 +1235,32 @@ extern "C" int areal_tgemm_wgrad(const void* dY, long ldy, const void* X, long l
   TWArgs a{(const bf16_t*)dY, ldy, (const bf16_t*)X, ldx, dW, ldw, M, N, K, (N + 255) / 256, K / 256, pairs, whole, splits, chunk, part, nullptr, 0};
   static bool attr_set = false;
   if (!attr_set) {
-    HIP_RET(hipFuncSetAttribute((const void*)tgemm_wgrad_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize, TG_LDS));
+    HIP_RET(hipFuncSetAttribute((const void*)tgemm_wgrad_kernel<false, false>, hipFuncAttributeMaxDynamicSharedMemorySize, TG_LDS));
+    HIP_RET(hipFuncSetAttribute((const void*)tgemm_wgrad_kernel<false, true>, hipFuncAttributeMaxDynamicSharedMemorySize, TG_LDS));
     attr_set = true;
   }
-  hipLaunchKernelGGL(tgemm_wgrad_kernel<false>, dim3((unsigned)nblocks), dim3(512), TG_LDS, st, a);
+  if ((long)N * K >= TG_STREAM)
+    hipLaunchKernelGGL((tgemm_wgrad_kernel<false, true>), dim3((unsigned)nblocks), dim3(512), TG_LDS, st, a);
+  else
+    hipLaunchKernelGGL((tgemm_wgrad_kernel<false, false>), dim3((unsigned)nblocks), dim3(512), TG_LDS, st, a);
   if (splits > 1) hipLaunchKernelGGL(tgemm_wgrad_sum_kernel, dim3((unsigned)(tiles - whole) * 32), dim3(256), 0, st, a);
+  return (int)hipGetLastError();
+}
+
+// The same for few tokens (tiles of 128 x 128, no parts); K a multiple of 128.
+extern "C" int areal_tgemm_wgrad_few(const void* dY, long ldy, const void* X, long ldx, float* dW, long ldw, int M, int N, int K,
+                                     hipStream_t st) {
+  if (M <= 0 || N <= 0 || K <= 0) return 0;
+  if (N % 128 != 0 || K % 128 != 0 || ldy % 8 != 0 || ldx % 8 != 0) return -1;
+  if (ldy < N || ldx < K || ldy > (1l << 24) || ldx > (1l << 24)) return -1;  // (as above)
+  if (((uintptr_t)dY | (uintptr_t)X) % 16 != 0 || (uintptr_t)dW % 4 != 0) return -1;
+  const long tiles = (long)(N / 128) * (K / 128);
+  if (tiles > 0x7fffffffl) return -1;
+  const TWArgs a{(const bf16_t*)dY, ldy, (const bf16_t*)X, ldx, dW, ldw, M, N, K, N / 128, K / 128, 0, 0, 1, 0, nullptr, nullptr, 0};
+  if (tiles <= 768)  // three a CU
+    hipLaunchKernelGGL((tgemm_wgrad_few_kernel<false, 3>), dim3((unsigned)tiles), dim3(256), 3 * TWF_STAGE, st, a);
+  else
+    hipLaunchKernelGGL((tgemm_wgrad_few_kernel<false, 2>), dim3((unsigned)tiles), dim3(256), 2 * TWF_STAGE, st, a);
   return (int)hipGetLastError();
 }
 
@@ -1162,9 +1334,27 @@ extern "C" int areal_tgemm_grouped_wgrad(const void* dY, const void* X, float* d
   TWArgs a{(const bf16_t*)dY, N, (const bf16_t*)X, K, dW, K, 0, N, K, tiles_n, tiles_k, 0, (int)blocks, 1, 0, nullptr, offsets, stride};
   static bool attr_set = false;
   if (!attr_set) {
-    HIP_RET(hipFuncSetAttribute((const void*)tgemm_wgrad_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, TG_LDS));
+    HIP_RET(hipFuncSetAttribute((const void*)tgemm_wgrad_kernel<true, false>, hipFuncAttributeMaxDynamicSharedMemorySize, TG_LDS));
+    HIP_RET(hipFuncSetAttribute((const void*)tgemm_wgrad_kernel<true, true>, hipFuncAttributeMaxDynamicSharedMemorySize, TG_LDS));
     attr_set = true;
   }
-  hipLaunchKernelGGL(tgemm_wgrad_kernel<true>, dim3((unsigned)blocks), dim3(512), TG_LDS, st, a);
+  if ((long)E * N * K >= TG_STREAM)
+    hipLaunchKernelGGL((tgemm_wgrad_kernel<true, true>), dim3((unsigned)blocks), dim3(512), TG_LDS, st, a);
+  else
+    hipLaunchKernelGGL((tgemm_wgrad_kernel<true, false>), dim3((unsigned)blocks), dim3(512), TG_LDS, st, a);
+  return (int)hipGetLastError();
+}
+
+// The same for few rows an expert (tiles of 128 x 128); K a multiple of 128.
+extern "C" int areal_tgemm_grouped_wgrad_few(const void* dY, const void* X, float* dW, const int* offsets, int E, int N, int K,
+                                             long stride, int spread, hipStream_t st) {
+  if (E <= 0) return 0;
+  if (N <= 0 || K <= 0 || N % 128 != 0 || K % 128 != 0 || N > (1 << 24) || K > (1 << 24)) return -1;
+  if (((uintptr_t)dY | (uintptr_t)X) % 16 != 0 || (uintptr_t)dW % 4 != 0) return -1;
+  const long per = (long)(N / 128) * (K / 128), tiles = per * E;
+  if (tiles > 0x7fffffffl) return -1;
+  // (an expert's tiles over all XCDs: from 4 tiles a CU on, where each XCD's share of them still uses its operands several times)
+  const TWArgs a{(const bf16_t*)dY, N, (const bf16_t*)X, K, dW, K, 0, N, K, N / 128, K / 128, 0, 0, 1, spread, nullptr, offsets, stride};
+  hipLaunchKernelGGL((tgemm_wgrad_few_kernel<true, 2>), dim3((unsigned)tiles), dim3(256), 2 * TWF_STAGE, st, a);
   return (int)hipGetLastError();
 }

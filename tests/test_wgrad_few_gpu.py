@@ -1,0 +1,62 @@
+"""Weight gradients over few tokens (tiles of 128 x 128): around the edges of a stage of 32 tokens, few and many tiles, experts."""
+import sys
+
+import pytest
+import torch
+
+from areal_vllm_amd import ops
+from areal_vllm_amd.ops import _lib as L, train_gemm as tg
+
+G = sys.modules["areal_vllm_amd.ops.grouped_gemm"]
+DEV = "cuda:0"
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("M", [1, 31, 32, 33, 65, 256, 287, 700])
+@pytest.mark.parametrize("N,K", [(128, 128), (1152, 384), (4096, 4096)])
+def test_dense(M, N, K):
+    g = torch.Generator(device=DEV).manual_seed(M + N)
+    # what lies past the last token and beside the columns must not be read: operands and gradient are cut out of larger ones
+    dy, x = torch.full((M + 40, N + 8), float("nan"), device=DEV).bfloat16(), torch.full((M + 40, K + 8), float("inf"), device=DEV).bfloat16()
+    dy[:M, :N] = torch.randn(M, N, device=DEV, generator=g).bfloat16()
+    x[:M, :K] = torch.randn(M, K, device=DEV, generator=g).bfloat16()
+    dy, x = dy[:M, :N], x[:M, :K]
+    whole = torch.randn(N, K + 1, device=DEV, generator=g)
+    want = whole.double()
+    want[:, :K] += dy.double().t() @ x.double()
+    L.check(L.lib().areal_tgemm_wgrad_few(L.ptr(dy), L.c_int64(N + 8), L.ptr(x), L.c_int64(K + 8), L.ptr(whole), L.c_int64(K + 1),
+                                          L.c_int(M), L.c_int(N), L.c_int(K), L.stream_ptr()), "tgemm_wgrad_few")
+    # fp32 sums of M products of size one
+    assert float((whole.double() - want).abs().max()) < 1e-3 * max(1.0, M ** 0.5 / 16)
+    assert torch.equal(whole[:, K].double(), want[:, K])
+
+
+@pytest.mark.parametrize("counts", [[0, 1, 255, 256, 257, 0, 700, 300], [5000], [3000] + [100] * 23, [31, 32, 33, 0]])
+@pytest.mark.parametrize("N,K", [(128, 128), (256, 512), (1536, 768)])
+@pytest.mark.parametrize("form", ["by expert", "over all XCDs", "large"])
+def test_grouped(counts, N, K, form, monkeypatch):
+    monkeypatch.setenv("AREAL_GROUPED_GEMM", "hip")
+    monkeypatch.delenv("AREAL_GROUPED_GEMM_TILE_M", raising=False)
+    if form == "large" and K % 256:
+        pytest.skip("tiles of 256 columns")
+    monkeypatch.setattr(G, "FEW_WGRAD_ROWS", 0)
+    monkeypatch.setattr(G, "_big_wgrad", lambda *a: form == "large")
+    monkeypatch.setattr(G, "_spread_experts", lambda *a: form == "over all XCDs")
+    E, T = len(counts), sum(counts)
+    g = torch.Generator(device=DEV).manual_seed(T + N + K)
+    x = torch.randn(T, K, device=DEV, generator=g).bfloat16()
+    w = (torch.randn(E, N, K, device=DEV, generator=g) / K ** 0.5).bfloat16().requires_grad_(True)
+    w.main_grad = torch.ones(E, N, K, device=DEV)
+    dy = (torch.randn(T, N, device=DEV, generator=g) / N ** 0.5).bfloat16()
+    ops.grouped_gemm(x, w, counts).backward(dy)
+    at = 0
+    for e, n in enumerate(counts):
+        want = dy[at:at + n].double().t() @ x[at:at + n].double()
+        # fp32 sums of up to 5000 products of size N ** -0.5
+        assert float((w.main_grad[e].double() - 1.0 - want).abs().max()) < 1e-4
+        at += n
+
+
+def test_rule_takes_both():
+    assert tg._wgrad_few(700, 192) and tg._wgrad_few(1500, 1680) and tg._wgrad_few(1024, 14244)
+    assert not tg._wgrad_few(32768, 192) and not tg._wgrad_few(700, 840) and not tg._wgrad_few(1500, 14244)
