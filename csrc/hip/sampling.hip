@@ -120,7 +120,14 @@ DEVINL void for_each_z(const Row<T>& r, int V, int V8, F f) {
   for (int i = V8 + threadIdx.x; i < V; i += blockDim.x) f(i, r.z1(i));
 }
 
-DEVINL float gumbel(uint32_t bits) { return -__logf(-__logf(u32_to_unit(bits) * 0.99999994f)); }
+// __logf of a positive, normal, finite number: the same bits without the scaling of subnormals and the test for infinities, 5
+// instructions for 14. Both arguments below are such: 2^-24 .. 1 - 2^-24 and the negated logarithms of these. (sample_partial_kernel,
+// 320 rows of 151936 at temperature 1: 84 -> 66 us, with the largest of eight keys found before their index is compared.)
+DEVINL float log_normal(float x) {
+  const float l = __builtin_amdgcn_logf(x), hi = 0x1.62e42ep-1f, lo = 0x1.efa39ep-25f;
+  return fmaf(l, hi, fmaf(l, lo, fmaf(l, hi, -(l * hi))));
+}
+DEVINL float gumbel(uint32_t bits) { return -log_normal(-log_normal(u32_to_unit(bits) * 0.99999994f)); }
 
 // ---------------------------------------------------------------------------------------------
 // Thresholds of top-k and top-p: the largest entry t of a row with F(t) >= target, F(t) = number (MASS = false) or
@@ -835,13 +842,18 @@ __global__ __launch_bounds__(256) void sample_partial_kernel(
         r0 = Philox::gen(seed, (uint64_t)row, ctr0 + (uint64_t)(i8 >> 2));
         r1 = Philox::gen(seed, (uint64_t)row, ctr0 + (uint64_t)(i8 >> 2) + 1);
       }
+      ArgMax c;  // of these eight: the first of the largest
+      c.v = -INFINITY;
+      c.i = i8;
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        ArgMax c;
-        c.v = noise ? z[j] + gumbel(j < 4 ? r0[j] : r1[j - 4]) : z[j];
-        c.i = i8 + j;
-        best = amax(best, c);
+        const float key = noise ? z[j] + gumbel(j < 4 ? r0[j] : r1[j - 4]) : z[j];
+        if (key > c.v) {
+          c.v = key;
+          c.i = i8 + j;
+        }
       }
+      best = amax(best, c);
     }
   }
   if (s == S - 1) {  // the entries behind the last whole group of 8 (or the whole row when it is not 16-byte aligned)
