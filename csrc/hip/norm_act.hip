@@ -23,11 +23,15 @@ __global__ __launch_bounds__(256) void rmsnorm_fwd_kernel(
   const bf16_t* xr = x + (size_t)row * H;
   const bf16_t* rr = res ? res + (size_t)row * H : nullptr;
   float v[MAXV][8];
+  // requested with the row, not behind its reduction (us, 1 / 700 / 32768 x 1536 3.14 / 4.38 / 77.5 -> 3.04 / 4.12 / 75.3, 16384 x 2048
+  // 47.6 -> 44.4; rows of more than 4096 have no registers left)
+  bf16x8 wv[MAXV];
   float ss = 0.f;
 #pragma unroll
   for (int i = 0; i < MAXV; ++i) {
     const int c = lane + i * 64;
     if (c < nvec) {
+      if (MAXV <= 8) wv[i] = ld8(w + c * 8);
       bf16x8 a = ld8(xr + c * 8);
       if (rr) {
         bf16x8 b = ld8(rr + c * 8);
@@ -55,11 +59,11 @@ __global__ __launch_bounds__(256) void rmsnorm_fwd_kernel(
   for (int i = 0; i < MAXV; ++i) {
     const int c = lane + i * 64;
     if (c < nvec) {
-      bf16x8 ww = ld8(w + c * 8);
       bf16x8 o;
+      if (MAXV > 8) wv[i] = ld8(w + c * 8);
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        float wf = bf2f(ww[j]) + (gemma ? 1.f : 0.f);
+        float wf = bf2f(wv[i][j]) + (gemma ? 1.f : 0.f);
         o[j] = f2bf(v[i][j] * rstd * wf);
       }
       st8(y + (size_t)row * H + c * 8, o);
@@ -71,7 +75,10 @@ __global__ __launch_bounds__(256) void rmsnorm_fwd_kernel(
 // dw partials: each block accumulates its rows' dy*xhat per column in registers,
 // reduces its 4 waves through LDS and writes one partial row; a second kernel sums
 // the partial rows (no atomics: every block would hit the same H floats).
-template <int MAXV>
+// EARLY: the residual gradient is requested with the row, not behind the row's reduction. A wave of many rows waits once less for each
+// (us, 32768 x 1536 99 -> 92, 16384 x 2048 66 -> 59); over few rows there is nothing to gain (700 x 1536 9.9 / 10.1), rows of more
+// than 2048 have no registers left.
+template <int MAXV, bool EARLY>
 __global__ __launch_bounds__(256) void rmsnorm_bwd_kernel(
     const bf16_t* __restrict__ dy, const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
     const float* __restrict__ rstd, const bf16_t* __restrict__ dres, bf16_t* __restrict__ dx,
@@ -89,6 +96,7 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_kernel(
   for (int row = blockIdx.x * nw + wid; row < T; row += gridDim.x * nw) {
     const float rs = rstd[row];
     float g[MAXV][8], xh[MAXV][8];
+    bf16x8 dr[EARLY ? MAXV : 1];
     float dot = 0.f;
 #pragma unroll
     for (int i = 0; i < MAXV; ++i) {
@@ -97,6 +105,9 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_kernel(
         bf16x8 a = ld8(dy + (size_t)row * H + c * 8);
         bf16x8 b = ld8(x + (size_t)row * H + c * 8);
         bf16x8 ww = ld8(w + c * 8);
+        if constexpr (EARLY) {
+          if (dres) dr[i] = ld8(dres + (size_t)row * H + c * 8);
+        }
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
           const float dyf = bf2f(a[j]);
@@ -113,12 +124,13 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_kernel(
       const int c = lane + i * 64;
       if (c < nvec) {
         bf16x8 o;
-        bf16x8 dr;
-        if (dres) dr = ld8(dres + (size_t)row * H + c * 8);
+        if constexpr (!EARLY) {
+          if (dres) dr[0] = ld8(dres + (size_t)row * H + c * 8);
+        }
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
           float d = rs * (g[i][j] - xh[i][j] * dot);
-          if (dres) d += bf2f(dr[j]);
+          if (dres) d += bf2f(dr[EARLY ? i : 0][j]);
           o[j] = f2bf(d);
         }
         st8(dx + (size_t)row * H + c * 8, o);
@@ -210,19 +222,22 @@ extern "C" int areal_rmsnorm_bwd(const void* dy, const void* x, const void* w, c
   if (lds > 160 * 1024) return -2;
   dim3 grid(G), block(256);
   const int maxv = (H / 8 + 63) / 64;
-#define LAUNCH(MV)                                                                             \
+#define LAUNCH(MV, EARLY)                                                                      \
   do {                                                                                         \
     if (lds > 64 * 1024)                                                                       \
-      HIP_RET(hipFuncSetAttribute((const void*)rmsnorm_bwd_kernel<MV>,                         \
+      HIP_RET(hipFuncSetAttribute((const void*)rmsnorm_bwd_kernel<MV, EARLY>,                  \
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));      \
-    hipLaunchKernelGGL(rmsnorm_bwd_kernel<MV>, grid, block, lds, st, (const bf16_t*)dy,        \
+    hipLaunchKernelGGL((rmsnorm_bwd_kernel<MV, EARLY>), grid, block, lds, st, (const bf16_t*)dy, \
                        (const bf16_t*)x, (const bf16_t*)w, rstd, (const bf16_t*)dres,          \
                        (bf16_t*)dx, workspace, T, H, gemma);                                   \
   } while (0)
-  if (maxv <= 2) LAUNCH(2);
-  else if (maxv <= 4) LAUNCH(4);
-  else if (maxv <= 8) LAUNCH(8);
-  else LAUNCH(16);
+  const bool many = T > 4096;  // rows a wave: more than two
+  if (maxv <= 2 && many) LAUNCH(2, true);
+  else if (maxv <= 2) LAUNCH(2, false);
+  else if (maxv <= 4 && many) LAUNCH(4, true);
+  else if (maxv <= 4) LAUNCH(4, false);
+  else if (maxv <= 8) LAUNCH(8, false);
+  else LAUNCH(16, false);
 #undef LAUNCH
   hipLaunchKernelGGL(colsum_partial_kernel, dim3((H + 31) / 32), dim3(256), 0, st, workspace,
                      (bf16_t*)dw_bf16, dw_f32, G, H);
