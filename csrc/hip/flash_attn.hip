@@ -36,7 +36,7 @@
 // norm's gradient, elements of some 300 times the overall rms, by 0.7 %.)
 // Measured (12 query heads on 2 key heads), register-staged tiles, one workgroup's waves in step -> this: 25 sequences of 1133
 // tokens 177 -> 151 us, 2 of 300 15.0 -> 11.5 us, 24576 tokens 2.13 -> 1.86 ms (873 -> 998 TFLOP/s); 3 x 8192 (28 on 4
-// heads) 1.94 -> 1.62 ms.
+// heads) 1.94 -> 1.62 ms; since the next tile's DMA is no longer waited for at once (dma16) 143 us, 1.78 ms (1030 TFLOP/s), 1.60 ms.
 // =====================================================================================
 __global__ __launch_bounds__(256, 2) void flash_fwd_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf16_t* __restrict__ v,
@@ -194,6 +194,7 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_kernel(
   if (causal) n_full = min(n_full, max(0, (q0 + shift + 1) / 64));
   n_full = min(n_full, ntile_k);
   if (ntile_k > 0) issue(0);
+  dma_pin(qf);
   int t = 0;
   for (; t < n_full; ++t) {
     dma_arrive();
@@ -342,8 +343,8 @@ __global__ __launch_bounds__(256, 2) void flash_bwd_dq_kernel(
     for (int s = 0; s < 8; ++s) { qf[s] = ld8(qp + s * 16); dof[s] = ld8(dp + s * 16); }
   }
   // rows past the end: lse = +inf makes every probability zero
-  const float lse2 = q_ok ? delta[(size_t)(Hq + head) * total_q + q_beg + my_q] : INFINITY;
-  const float dlt = q_ok ? delta[(size_t)head * total_q + q_beg + my_q] : 0.f;
+  float lse2 = q_ok ? delta[(size_t)(Hq + head) * total_q + q_beg + my_q] : INFINITY;
+  float dlt = q_ok ? delta[(size_t)head * total_q + q_beg + my_q] : 0.f;
   f32x16 dqacc[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i)
@@ -419,6 +420,9 @@ __global__ __launch_bounds__(256, 2) void flash_bwd_dq_kernel(
   if (causal) n_full = min(n_full, max(0, (q0 + shift + 1) / 64));
   n_full = min(n_full, ntile_k);
   if (ntile_k > 0) issue(0);
+  dma_pin(qf);
+  dma_pin(dof);
+  asm volatile("" : "+v"(lse2), "+v"(dlt));
   int t = 0;
   for (; t < n_full; ++t) {
     dma_arrive();
@@ -521,6 +525,7 @@ __global__ __launch_bounds__(256, 2) void flash_bwd_dkv_kernel(
   dma_offsets32(dooff, wid, lane, do_stride);
   const int nwork = nh > 0 ? nh * nslice : 0;
   float rc_next = 0.f;  // wave 0: lane -> lse2 (first half) or delta of the next slice's rows
+  bool rc_ok = false;   // a row of the sequence
   int it = 0, n_head = h0, n_slice = 0;  // issued so far; the next slice's head and index
   auto issue = [&]() {
     char* buf = qds + (it & 1) * 16384;
@@ -530,14 +535,14 @@ __global__ __launch_bounds__(256, 2) void flash_bwd_dkv_kernel(
                lane);
     if (wid == 0) {
       const int qi = qs0 + r;
-      const float x = delta[(size_t)((hf ? 0 : Hq) + n_head) * total_q + q_beg + (qi < q_len ? qi : q_len - 1)];
-      rc_next = qi < q_len ? x : hf ? 0.f : INFINITY;
+      rc_next = delta[(size_t)((hf ? 0 : Hq) + n_head) * total_q + q_beg + (qi < q_len ? qi : q_len - 1)];
+      rc_ok = qi < q_len;  // (chosen by when the value is stored: a choice here would wait for it, and for the slice)
     }
     if (++n_slice == nslice) { n_slice = 0; ++n_head; }
   };
   // slice `it` is complete in LDS; the one after it is on its way
   auto advance = [&]() {
-    if (wid == 0) rc[(it & 1) * 64 + lane] = rc_next;  // waits for the value, and with it for the slice's DMA
+    if (wid == 0) rc[(it & 1) * 64 + lane] = rc_ok ? rc_next : hf ? 0.f : INFINITY;  // waits for the value, and with it for the slice's DMA
     dma_arrive();
     ++it;
     if (it < nwork) issue();
@@ -598,7 +603,11 @@ __global__ __launch_bounds__(256, 2) void flash_bwd_dkv_kernel(
       }
     }
   };
-  if (nwork > 0) issue();
+  if (nwork > 0)
+    issue();
+  else
+    dma_arrive();  // (V is on its way)
+  dma_pin(kf);
   for (int h = 0; h < nh; ++h) {
     int sl = 0;
     for (; sl < n_diag; ++sl) {

@@ -64,10 +64,21 @@ DEVINL void flash_zero_uncovered(const FlashGrads& g, int64_t t, int h, int D, i
 
 // ---- staging of 64-row tiles by LDS-DMA. One wave instruction (16 bytes a lane) fills four consecutive 256-byte rows of a
 // tile linearly; the swizzle sits on the source address: lane -> row (lane >> 4) of the four, physical chunk lane & 15.
-typedef const __attribute__((address_space(1))) void* dma_gptr_t;
 typedef __attribute__((address_space(3))) void* dma_lptr_t;
-DEVINL void dma16(const void* src, void* lds) {
-  __builtin_amdgcn_global_load_lds((dma_gptr_t)src, (dma_lptr_t)lds, 16, 0, 0);
+// In assembly, because behind the builtin the compiler cannot tell the reads of one buffer from the pending writes of the other and
+// puts a wait for all of them in front of the first read: the tile after this one was waited for before this one was computed.
+// Nothing comes back into registers; what waits is `dma_arrive`, in front of every read of a tile. With `dma_pin` and the row
+// statistics of a slice chosen behind its arrival, us, forward / backward, 12 query heads on 2: 25 sequences of up to 1133 tokens 154 -> 143 /
+// 580 -> 514, one of 24576 1842 -> 1784 / 6307 -> 5853; 16 heads, 8 of 2048 206 -> 177 / 671 -> 604; short ones level.
+DEVINL void dma16(const char* base, unsigned off, const void* lds) {
+  const unsigned at = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(dma_lptr_t)lds);
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(at), "v"(off), "s"(base) : "memory", "m0");
+}
+// Registers that were loaded ahead of a loop of tiles are waited for here, once, not at their first use in every round of it
+template <int N>
+DEVINL void dma_pin(bf16x8 (&f)[N]) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) asm volatile("" : "+v"(f[i]));
 }
 // Rows 16 w + 4 i + (lane >> 4), i = 0..3, of a tile of 64 rows go through wave w of four. `off`: this lane's byte offsets of
 // the four pieces for rows `stride` elements apart.
@@ -87,13 +98,13 @@ DEVINL void dma_tile(const bf16_t* base, const unsigned (&off)[4], int64_t strid
   asm volatile("" : "+s"(b));
   if (rows >= 64) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) dma16(b + off[i], dst + i * 1024);
+    for (int i = 0; i < 4; ++i) dma16(b, off[i], dst + i * 1024);
   } else {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int row = 16 * wave + 4 * i + (lane >> 4), over = row < rows ? 0 : row - (rows - 1);
       // (same chunk order as row `row` would have: the swizzle belongs to the place in the tile)
-      dma16(b + (off[i] - (unsigned)(over * stride) * 2), dst + i * 1024);
+      dma16(b, off[i] - (unsigned)(over * stride) * 2, dst + i * 1024);
     }
   }
 }
@@ -118,12 +129,12 @@ DEVINL void dma_tile32(const bf16_t* base, const unsigned (&off)[2], int64_t str
   asm volatile("" : "+s"(b));
   if (rows >= 32) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i) dma16(b + off[i], dst + i * 1024);
+    for (int i = 0; i < 2; ++i) dma16(b, off[i], dst + i * 1024);
   } else {
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const int row = 8 * wave + 4 * i + (lane >> 4), over = row < rows ? 0 : row - (rows - 1);
-      dma16(b + (off[i] - (unsigned)(over * stride) * 2), dst + i * 1024);
+      dma16(b, off[i] - (unsigned)(over * stride) * 2, dst + i * 1024);
     }
   }
 }
