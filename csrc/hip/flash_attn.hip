@@ -553,26 +553,35 @@ __global__ __launch_bounds__(256, 2) void flash_bwd_dkv_kernel(
     const char* dos = qs + 8192;
     const float* rcs = rc + (cur & 1) * 64;
     const int qu = (first + slice) * 32;
-    // ---- S = Q.K^T, dP = dO.V^T (rows = q in registers, col = key on the lane)
+    // ---- S = Q.K^T, dP = dO.V^T (rows = q in registers, col = key on the lane). Fragments are requested ahead of the products in
+    // front of theirs, as many as there are registers for (backward pass, us, read next to their use / so: 24576 tokens, 12 heads on 2,
+    // 5723 / 5617, 16384, 32 on 4, 6879 / 6707; the same in the two other kernels gives nothing).
     f32x16 sacc, pacc;
+    bf16x8 qa[2][2], da[2], vf[2];
+    auto read_q = [&](int g) __attribute__((always_inline)) {
 #pragma unroll
-    for (int s0 = 0; s0 < 8; s0 += 2) {
-      bf16x8 qa[2];
+      for (int s = 0; s < 2; ++s) qa[g & 1][s] = *reinterpret_cast<const bf16x8*>(qs + fo.row(2 * g + s));
+    };
+    auto read_d = [&](int s) __attribute__((always_inline)) {
+      da[s & 1] = *reinterpret_cast<const bf16x8*>(dos + fo.row(s));
+      vf[s & 1] = *reinterpret_cast<const bf16x8*>(vs + (fo.row(s) + 8192 * wid));
+    };
+    read_q(0);
 #pragma unroll
-      for (int s = 0; s < 2; ++s) qa[s] = *reinterpret_cast<const bf16x8*>(qs + fo.row(s0 + s));
+    for (int g = 0; g < 4; ++g) {
+      if (g < 3)
+        read_q(g + 1);
+      else
+        read_d(0);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int s = 0; s < 2; ++s) sacc = mfma32(qa[s], kf[s0 + s], s0 + s ? sacc : f32x16{});
+      for (int s = 0; s < 2; ++s) sacc = mfma32(qa[g & 1][s], kf[2 * g + s], g + s ? sacc : f32x16{});
     }
 #pragma unroll
-    for (int s0 = 0; s0 < 8; s0 += 2) {
-      bf16x8 da[2], vf[2];
-#pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        da[s] = *reinterpret_cast<const bf16x8*>(dos + fo.row(s0 + s));
-        vf[s] = *reinterpret_cast<const bf16x8*>(vs + (fo.row(s0 + s) + 8192 * wid));
-      }
-#pragma unroll
-      for (int s = 0; s < 2; ++s) pacc = mfma32(da[s], vf[s], s0 + s ? pacc : f32x16{});
+    for (int s = 0; s < 8; ++s) {
+      if (s < 7) read_d(s + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      pacc = mfma32(da[s & 1], vf[s & 1], s ? pacc : f32x16{});
     }
     // ---- P = exp2(S c - lse), dS = P (dP - delta)
     bf16x8 pfr[2], dsfr[2];
