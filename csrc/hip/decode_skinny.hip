@@ -103,9 +103,9 @@ DEVINL void put_pair(const SKArgs& a, int head, int d, int m, float lo, float hi
   lo = bf2f(f2bf(lo + bias_lo));  // the unfused path carries the projection as a bf16 tensor
   hi = bf2f(f2bf(hi + bias_hi));
   if (a.do_rope && head < a.Hq + a.Hkv) {
-    const float x = lo;
-    lo = x * c - hi * s;
-    hi = hi * c + x * s;
+    const float x = lo;  // (which product is rounded by itself is written out: left to the compiler it changes with the code around it)
+    lo = fmaf(x, c, -(hi * s));
+    hi = fmaf(hi, c, x * s);
   }
   if (head < a.Hq) {
     bf16_t* q = a.Y + ((size_t)m * a.Hq + head) * a.D + d;

@@ -144,3 +144,23 @@ def test_layer_inside_the_runner(rows, hidden, inner, heads, extra, fp8):
     step = 2.0 ** -3 if fp8 else 2.0 ** -6  # a step of the cache's type, a few roundings apart
     for x, y in zip(ca, cb):
         assert bool(((x - y).abs() <= 0.05 + step * x.abs()).all())
+
+
+@pytest.mark.parametrize("M", [1, 2, 5])
+def test_rotation_roundings(M):
+    """Which product of a rotated value is rounded by itself: lo c - r(hi s), hi c + r(lo s), bit for bit, and so the results of every decode
+    step. The projection is exact: rows of +-1 with a mean square of one, weights in sixteenths."""
+    Hq, Hkv, D, K = 60, 2, 128, 512
+    ones, tab = torch.ones(K, device=DEV).bfloat16(), ops.RotaryTable(D, 4096, 1e6, DEV)
+    for seed in range(40):
+        g = torch.Generator(device=DEV).manual_seed(seed * 8 + M)
+        x = (torch.randint(0, 2, (M, K), device=DEV, generator=g) * 2 - 1).bfloat16()
+        w = (torch.randint(-9, 10, ((Hq + 2 * Hkv) * D, K), device=DEV, generator=g) / 16).bfloat16()
+        pos = torch.randint(0, 4096, (M,), device=DEV, generator=g, dtype=torch.int32)
+        kc, vc = ops.alloc_kv_cache(1, Hkv, D, torch.bfloat16, DEV)
+        q = sk.norm_qkv_rope(x, ones, w, None, pos, torch.full((M,), -1, device=DEV).long(), tab, kc, vc, Hq, Hkv, D, eps=0.0)
+        y = (x.float() @ w.float().t()).bfloat16().float()[:, :Hq * D].view(M, Hq, 2, D // 2)
+        lo, hi = y[:, :, 0], y[:, :, 1]
+        c, s = (t[pos.long()][:, None] for t in (tab.cos, tab.sin))
+        want = torch.cat([lo.double() * c.double() - (hi * s).double(), hi.double() * c.double() + (lo * s).double()], -1)
+        assert torch.equal(q, want.float().bfloat16()), int((q != want.float().bfloat16()).sum())
