@@ -106,13 +106,15 @@ def _tile_plan(pairs: int, tiles: int, flush: int, rows: int = 256) -> Tuple[flo
 
 
 def _wgrad_few(M: int, tiles: int) -> bool:
-    """Whether `tiles` of 128 x 128, several on a CU, are the better ones over M tokens; us of the tiles of 256 x 256 / of these, the
-    gradient not in the caches. Up to three tiles a CU, where the large ones would need parts: 2 tiles, 600 / 1024 tokens 10.5 /
-    9.6, 11.7 / 14; 16 tiles, 600 / 1024 / 1500 13.5 / 10, 16.4 / 14.6, 17.1 / 19.7; 64, 1500 / 2048 23.2 / 20.3, 23.4 / 25.7; 144, 2048 /
-    3000 31 / 27, 35.7 / 37.1; 256, 2048 / 3072 40 / 29, 45 / 39; 456, 3000 65 / 49; 768, 3072 / 78 / 76. Not where they fill most of
-    one round: 840, 700 / 1024 38.3 / 37, 43.4 / 44.5, and with the gradient in the memory-side cache 34 / 37. More: 1200, 1500 88 / 73;
-    1680, 700 / 1500 / 2048 78 / 61, 107 / 93, 127 / 117; 5504, 1024 / 1500 / 2048 270 / 211, 330 / 293, 394 / 392; but full rounds,
-    1008, 1024 / 1500 51 / 47, 61 / 59; 14244, 1024 / 1500 637 / 599, 789 / 798."""
+    """Whether `tiles` of 128 x 128, several on a CU, are the better ones over M tokens where the large ones are not split; us of the
+    tiles of 256 x 256 / of these, the gradient not in the caches. Up to three tiles a CU 2 tiles, 600 tokens 10.5 / 9.6; 16 tiles, 600
+    13.5 / 10; 768, 256 / 700 / 1280 / 3072 29.5 / 23.2, 37.6 / 30.3, 47.3 / 40.9, 78 / 76. Not where they fill most of one round, for
+    what they lose with the gradient in the memory-side cache is more than they gain without: 780 tiles, 256 / 700 / 1024 29.6 / 26.5,
+    38.7 / 37.1, 43.5 / 44.9 and 23.6 / 25.7, 32.9 / 38.5, 37.9 / 45.7; 840 29.9 / 27.1, 39.3 / 37.6, 45.5 / 45.3 and 25.0 / 26.0, 34.5 /
+    38.3, 39.4 / 45.9; 900 31.1 / 27.9, 41.0 / 38.6, 47.0 / 46.3 and 26.0 / 27.2, 36.0 / 39.6, 41.2 / 47.2; from 960 on 33.2 / 27.2, 43.5 /
+    37.7, 49.0 / 46.2 and 28.3 / 27.1, 38.7 / 38.6, 44.0 / 46.7. More: 1200, 1500 88 / 73; 1680, 700 / 1500 / 2048 78 / 61, 107 / 93, 127 /
+    117; 5504, 1024 / 1500 / 2048 270 / 211, 330 / 293, 394 / 392; but full rounds, 1008, 1024 / 1500 51 / 47, 61 / 59; 14244, 1024 / 1500
+    637 / 599, 789 / 798."""
     if tiles <= 768:
         return M <= min(3072, 600 + 11 * tiles)
     filled = tiles / 1024 / -(-tiles // 1024)
@@ -124,11 +126,6 @@ def tgemm_wgrad_(acc: torch.Tensor, dy: torch.Tensor, x: torch.Tensor, splits: i
     fp32 gradient buffer. `splits`: parts of the token range for every tile (0: chosen)."""
     assert wgrad_supported(dy, x, acc)
     (M, N), K = dy.shape, x.shape[1]
-    if not splits and _wgrad_few(M, N // 128 * (K // 128)):
-        L.check(L.lib().areal_tgemm_wgrad_few(L.ptr(dy), L.c_int64(dy.stride(0)), L.ptr(x), L.c_int64(x.stride(0)), L.ptr(acc),
-                                              L.c_int64(acc.stride(0)), L.c_int(M), L.c_int(N), L.c_int(K), L.stream_ptr()),
-                "tgemm_wgrad_few")
-        return acc
     pairs, tiles = -(-M // 128), -(-N // 256) * (K // 256)
     if splits:
         splits = _even_splits(pairs, splits)
@@ -137,6 +134,13 @@ def tgemm_wgrad_(acc: torch.Tensor, dy: torch.Tensor, x: torch.Tensor, splits: i
         # (reading, adding to and writing a tile's gradient: 1500 tokens, 1536 x 1536, 36 tiles whole / in 3 parts 37 / 28 us, 48
         # tiles 38 / 31, 100 tiles 40 / 58)
         _, whole, splits = _tile_plan(pairs, tiles, 5)
+        # Parts sum in shorter chains: in place of whole tiles only the small ones give the same bits. Relative error against 64 bits in
+        # parts / in one chain, 512 x 512, 700 tokens 7.7e-8 / 1.5e-7, 2048 x 1536, 1500 1.3e-7 / 2.3e-7 (31 / 22 us).
+        if splits == 1 and _wgrad_few(M, N // 128 * (K // 128)):
+            L.check(L.lib().areal_tgemm_wgrad_few(L.ptr(dy), L.c_int64(dy.stride(0)), L.ptr(x), L.c_int64(x.stride(0)), L.ptr(acc),
+                                                  L.c_int64(acc.stride(0)), L.c_int(M), L.c_int(N), L.c_int(K), L.stream_ptr()),
+                    "tgemm_wgrad_few")
+            return acc
     part = torch.empty(splits * (tiles - whole) << 16, dtype=torch.float32, device=dy.device) if splits > 1 else None
     L.check(L.lib().areal_tgemm_wgrad(L.ptr(dy), L.c_int64(dy.stride(0)), L.ptr(x), L.c_int64(x.stride(0)), L.ptr(acc),
                                       L.c_int64(acc.stride(0)), L.c_int(M), L.c_int(N), L.c_int(K), L.c_int(splits),

@@ -894,7 +894,8 @@ __global__ __launch_bounds__(256) void tgemm_wgrad_sum_kernel(const TWArgs a) {
 // 59 / 48, 78 / 61, 107 / 93; 2048 x 1536 19 / 9.3, 28 / 14, 31 / 22; 151936 x 1536 425 / 340, 572 / 436, 789 / 798. Without
 // streaming 700 tokens take 68, 15 and 514 us. S: 2 stages leave room for four workgroups, 3 for three, better where there are no
 // more than three a CU (2048 x 1536, 1500 tokens 26 / 22; 22016 x 4096, 700 tokens 164 / 175; 4 stages 206).
-// Sums are taken over all tokens in their order, as in a whole tile above.
+// Sums are taken over all tokens in their order, as in a whole tile above and bit for bit as there; tiles that are split there stay
+// there (1500 tokens of 2048 x 1536), for parts sum in shorter chains.
 //
 // GRP: routed experts' gradients, rows sorted by expert. us, 128 experts of 1536 x 2048, 64 / 256 / 512 / 700 rows an expert, kernel
 // above / this one: 618 / 550, 710 / 561, 862 / 746, 992 / 871.

@@ -60,3 +60,14 @@ def test_grouped(counts, N, K, form, monkeypatch):
 def test_rule_takes_both():
     assert tg._wgrad_few(700, 192) and tg._wgrad_few(1500, 1680) and tg._wgrad_few(1024, 14244)
     assert not tg._wgrad_few(32768, 192) and not tg._wgrad_few(700, 840) and not tg._wgrad_few(1500, 14244)
+
+
+@pytest.mark.parametrize("M,N,K", [(700, 512, 512), (1024, 512, 512), (1500, 2048, 1536), (2048, 1536, 1536), (700, 2048, 1536), (1031, 6144, 2048)])
+def test_no_less_precise_than_large_tiles(M, N, K):
+    """The chosen form's error against 64 bits beside that of the large tiles with the parts that they would take."""
+    g = torch.Generator(device=DEV).manual_seed(M + N)
+    dy, x = torch.randn(M, N, device=DEV, generator=g).bfloat16(), torch.randn(M, K, device=DEV, generator=g).bfloat16()
+    want = dy.double().t() @ x.double()
+    parts = tg._tile_plan(-(-M // 128), -(-N // 256) * (K // 256), 5)[2]
+    err = [float((tg.tgemm_wgrad_(torch.zeros(N, K, device=DEV), dy, x, splits=s).double() - want).norm() / want.norm()) for s in (parts, 0)]
+    assert err[1] <= 1.02 * err[0], err  # (the mean over a quarter of a million roundings and more)
