@@ -75,9 +75,10 @@ def _spread_experts(T: int, E: int, N: int, K: int, counts: List[int]) -> bool:
     crowded expert; its operands pass through eight L2s instead. us dealt by experts / over all, largest expert 1 / 4 / 8 / 16 means:
     128 experts of 500 rows, 1536 columns, 2048 deep (192 tiles) 744 / 725, 786 / 728, 854 / 722, 966 / 729; 2048 columns, 768 deep
     (96) 387 / 424, 410 / 422, 444 / 422, 511 / 424; 8 of 500, 4096 columns, 14336 deep 769 / 796, 1319 / 837, 1756 / 897; 32 of 500,
-    1024 by 1024 (64 tiles) 63 / 82, 70 / 83, 89 / 98, 116 / 122."""
-    tiles = N // 128 * (K // 128)
-    return tiles >= 80 and max(counts) * E > (6 if tiles < 128 else 3 if tiles < 1024 else 1.5) * T
+    1024 by 1024 (64 tiles) 63 / 82, 70 / 83, 89 / 98, 116 / 122; nearly all rows with one expert, 16 of 16 / 64 / 128, 1536 columns, 768 deep
+    (72) 14.6 / 10.2, 37.4 / 36.6, 53.0 / 50.1."""
+    tiles, most = N // 128 * (K // 128), max(counts)
+    return 2 * most > T or tiles >= 80 and most * E > (6 if tiles < 128 else 3 if tiles < 1024 else 1.5) * T
 
 
 def big_grouped(x: torch.Tensor, w: torch.Tensor, offsets: torch.Tensor, nn: bool) -> torch.Tensor:
@@ -164,8 +165,8 @@ class _GroupedGemmFn(torch.autograd.Function):
                                                                   L.stream_ptr()), "tgemm_grouped_wgrad")
                     else:
                         L.check(L.lib().areal_tgemm_grouped_wgrad_few(
-                            L.ptr(dy), L.ptr(x), L.ptr(mg), L.ptr(offsets), L.c_int(E), L.c_int(N), L.c_int(K), L.c_int64(mg.stride(0)),
-                            L.c_int(int(_spread_experts(T, E, N, K, ctx.counts))), L.stream_ptr()), "tgemm_grouped_wgrad_few")
+                            L.ptr(dy), L.ptr(x), L.ptr(mg), L.ptr(offsets), L.c_int(max(ctx.counts)), L.c_int(E), L.c_int(N), L.c_int(K),
+                            L.c_int64(mg.stride(0)), L.c_int(int(_spread_experts(T, E, N, K, ctx.counts))), L.stream_ptr()), "tgemm_grouped_wgrad_few")
                     _after_fold(w)
                 else:
                     dw = torch.empty_like(w)

@@ -619,6 +619,7 @@ struct TWArgs {
   // grouped (GRP): rows offsets[e] .. offsets[e + 1] belong to expert e, whose gradient lies `stride` elements from the last
   const int* offsets;
   long stride;
+  int band = 8;  // tgemm_wgrad_few_kernel: tile rows that are walked together
 };
 
 typedef f32x4 __attribute__((aligned(4))) f32x4u;
@@ -909,7 +910,7 @@ __global__ __launch_bounds__(256, S == 2 ? 4 : 3) void tgemm_wgrad_few_kernel(co
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wr = wave >> 1, wc = wave & 1, fr = lane & 15, fq = lane >> 4;
 
-  // ---- id -> tile: contiguous ranges per XCD, walked in bands of 8 tile rows. Ranges of all experts' tiles (an expert's operands then
+  // ---- id -> tile: contiguous ranges per XCD, walked in bands of tile rows. Ranges of all experts' tiles (an expert's operands then
   // pass through one L2), or, where an expert alone has many, of each expert's: a crowded expert would keep one XCD busy
   int nb = gridDim.x, id = blockIdx.x, e = 0;
   if (GRP && a.chunk) {
@@ -932,9 +933,9 @@ __global__ __launch_bounds__(256, S == 2 ? 4 : 3) void tgemm_wgrad_few_kernel(co
     if (row_hi <= row_lo) return;  // an expert without rows adds nothing
     dW += e * a.stride;
   }
-  const int per_band = 8 * a.tiles_k, band = b / per_band, in_band = b - band * per_band;
-  const int band_rows = min(a.tiles_n - band * 8, 8);
-  const int n0 = (band * 8 + in_band % band_rows) * 128, k0 = in_band / band_rows * 128;
+  const int per_band = a.band * a.tiles_k, band = b / per_band, in_band = b - band * per_band;
+  const int band_rows = min(a.tiles_n - band * a.band, a.band);
+  const int n0 = (band * a.band + in_band % band_rows) * 128, k0 = in_band / band_rows * 128;
 
   // ---- staging: thread -> token row (wave * 4 + lane / 16) of a 16-row issue; rows past the last token are out of the buffer's
   // range and write zeros (as in tgemm_wgrad_kernel)
@@ -1346,16 +1347,20 @@ extern "C" int areal_tgemm_grouped_wgrad(const void* dY, const void* X, float* d
   return (int)hipGetLastError();
 }
 
-// The same for few rows an expert (tiles of 128 x 128); K a multiple of 128.
-extern "C" int areal_tgemm_grouped_wgrad_few(const void* dY, const void* X, float* dW, const int* offsets, int E, int N, int K,
+// The same for few rows an expert (tiles of 128 x 128), `most` at most; K a multiple of 128. `spread`: each expert's tiles are dealt to all XCDs.
+extern "C" int areal_tgemm_grouped_wgrad_few(const void* dY, const void* X, float* dW, const int* offsets, int most, int E, int N, int K,
                                              long stride, int spread, hipStream_t st) {
   if (E <= 0) return 0;
   if (N <= 0 || K <= 0 || N % 128 != 0 || K % 128 != 0 || N > (1 << 24) || K > (1 << 24)) return -1;
   if (((uintptr_t)dY | (uintptr_t)X) % 16 != 0 || (uintptr_t)dW % 4 != 0) return -1;
   const long per = (long)(N / 128) * (K / 128), tiles = per * E;
   if (tiles > 0x7fffffffl) return -1;
-  // (an expert's tiles over all XCDs: from 4 tiles a CU on, where each XCD's share of them still uses its operands several times)
-  const TWArgs a{(const bf16_t*)dY, N, (const bf16_t*)X, K, dW, K, 0, N, K, N / 128, K / 128, 0, 0, 1, spread, nullptr, offsets, stride};
+  // Few rows' operands fit the L2 in any order, and tile after tile along the gradient's rows the memory is read and written in
+  // longer pieces: us in bands of 1 / 8 tile rows, 8 experts of 4096 x 14336, 16 / 64 / 128 / 200 / 400 rows 695 / 723, 696 / 727, 696 / 724, 730
+  // / 725, 911 / 747; 128 of 1536 x 2048 525 / 559, 521 / 546, 517 / 540, 523 / 552, 641 / 687; 16 of 2048 x 7168 343 / 361, 341 / 361,
+  // 342 / 360, 344 / 360, 449 / 377; all of 254 / 508 / 1016 rows with one of the first 193 / 194, 221 / 203, 786 / 760.
+  const int band = most <= 256 ? 1 : 8;
+  const TWArgs a{(const bf16_t*)dY, N, (const bf16_t*)X, K, dW, K, 0, N, K, N / 128, K / 128, 0, 0, 1, spread, nullptr, offsets, stride, band};
   hipLaunchKernelGGL((tgemm_wgrad_few_kernel<true, 2>), dim3((unsigned)tiles), dim3(256), 2 * TWF_STAGE, st, a);
   return (int)hipGetLastError();
 }

@@ -28,6 +28,23 @@ def test_rule(T, E, N, K, out, dx, dw, monkeypatch):
     assert not G._big_wgrad(T, E, N, K, [9 * T // E])  # behind a crowded expert
 
 
+@pytest.mark.parametrize("E,N,K,rows,crowd,spread", [  # `crowd`: the largest expert's rows, of the mean's
+    (128, 1536, 2048, 500, 1, False), (128, 1536, 2048, 500, 2.9, False), (128, 1536, 2048, 500, 3.1, True),  # 192 tiles
+    (128, 2048, 768, 500, 5.9, False), (128, 2048, 768, 500, 6.1, True),  # 96
+    (8, 4096, 14336, 500, 2.9, False), (8, 4096, 14336, 500, 3.1, True),  # 3584: 1.5 from 1024 tiles on
+    (32, 1024, 1024, 500, 15, False), (32, 1024, 1024, 500, 17, True),  # 64: only behind an expert with more than half of all rows
+    (16, 1536, 768, 16, 8, False), (16, 1536, 768, 16, 8.1, True),  # 72
+])
+def test_spread(E, N, K, rows, crowd, spread):
+    most, T = int(rows * crowd), rows * E
+    if N // 128 * (K // 128) >= 1024:
+        most = int(rows * crowd / 2)
+    counts = [(T - most) // (E - 1)] * E
+    counts[E // 2] = most
+    counts[0] += T - sum(counts)
+    assert max(counts) == most and G._spread_experts(T, E, N, K, counts) == spread
+
+
 @pytest.mark.parametrize("T,E,H,parts", [(64, 128, 2048, True), (512, 128, 2048, True), (128, 128, 4096, True),
                                          (129, 128, 4096, False), (16, 128, 7168, False), (1, 256, 1024, False),
                                          (512, 32, 7168, True), (513, 32, 1024, False), (0, 32, 1024, False)])
