@@ -8,12 +8,16 @@ Counterparts in the reference: ``flash_attn_varlen_func`` / ``flash_attn_with_kv
 ``areal/engine/base_hf_engine.py:291-406``.
 """
 import math
-from functools import lru_cache
 from typing import Optional, Tuple
 
 import torch
 
 from . import _lib as L
+
+try:
+    from areal_vllm_amd._C import _runtime as _rt
+except ImportError:  # extension not built
+    _rt = None
 
 PAGE_SIZE = 32  # tokens per KV page; fixed by the decode kernel's MFMA operand layout
 
@@ -397,8 +401,7 @@ def paged_prefill_splits(batch: int, n_q_heads: int, max_q: int, max_k: int, tot
                    max_k, PAGED_PREFILL_WORKGROUPS, PAGED_PREFILL_KEYS)
 
 
-@lru_cache(maxsize=4096)
-def _ranges(tiles: int, rows: int, max_k: int, workgroups: int, keys: int) -> int:
+def _ranges_py(tiles: int, rows: int, max_k: int, workgroups: int, keys: int) -> int:
     walk = -(-max_k // 64)  # tiles of 64 keys
 
     def cost(splits):
@@ -407,6 +410,9 @@ def _ranges(tiles: int, rows: int, max_k: int, workgroups: int, keys: int) -> in
                 + (4 + 3.5e-4 * rows * splits if splits > 1 else 0))
 
     return min(range(1, max(1, min(workgroups // tiles, max_k // keys, 32)) + 1), key=cost)
+
+
+_ranges = _ranges_py if _rt is None else _rt.key_ranges  # (0.7 us for 8)
 
 
 def flash_attn_paged_prefill(q, kcache, vcache, block_tables, cu_q, cu_k, max_q: int, scale: Optional[float] = None,

@@ -21,6 +21,11 @@ import torch.nn.functional as F
 
 from . import _lib as L
 
+try:
+    from areal_vllm_amd._C import _runtime as _rt
+except ImportError:  # extension not built
+    _rt = None
+
 EPI_BF16, EPI_SLAB, EPI_SWIGLU, EPI_GEGLU = 0, 1, 2, 3  # GEGLU: the SwiGLU epilogue with a tanh-GELU gate
 GATED = (EPI_SWIGLU, EPI_GEGLU)
 
@@ -102,14 +107,7 @@ def pick_config(M: int, N: int, K: int, epilogue: int) -> Tuple[int, int, int, i
 _OVERRIDES = {}
 
 
-@lru_cache(maxsize=4096)
-def slab_plan(M: int, N: int, K: int) -> Tuple[int, int, int]:
-    """-> (32-column tiles a workgroup, row blocks, splits of the reduction) of a product into partial sums: the least of
-    a workgroup's 64-deep steps x (46 ns for each 32 rows and each 32 columns that it stages, 5.6 for each pair of them
-    that it multiplies, 46 for the step) x rounds of 256 workgroups, and 0.45 us for each MB of partial sums, written here
-    and read by the row kernel behind (0.15 of it). Fitted to 6500 launches (13 layers of 896 to 5120 columns, 896 to
-    18944 deep, 8 to 512 rows); its choice is 1.2 % behind the best of them in the mean, 10 % at worst. No split of less than
-    192 deep: a ring that is never full, and products of few columns need no more parts than their readers sum at once."""
+def _slab_plan_py(M: int, N: int, K: int) -> Tuple[int, int, int]:
     steps = K // 64
     best = None
     for mblocks in range(-(-M // 256), -(-M // 32) + 1):
@@ -127,6 +125,20 @@ def slab_plan(M: int, N: int, K: int) -> Tuple[int, int, int]:
                 if best is None or cost < best[0]:
                     best = (cost, ct, mblocks, ksplit)
     return best[1:]
+
+
+@lru_cache(maxsize=4096)
+def slab_plan(M: int, N: int, K: int) -> Tuple[int, int, int]:
+    """-> (32-column tiles a workgroup, row blocks, splits of the reduction) of a product into partial sums: the least of
+    a workgroup's 64-deep steps x (46 ns for each 32 rows and each 32 columns that it stages, 5.6 for each pair of them
+    that it multiplies, 46 for the step) x rounds of 256 workgroups, and 0.45 us for each MB of partial sums, written here
+    and read by the row kernel behind (0.15 of it). Fitted to 6500 launches (13 layers of 896 to 5120 columns, 896 to
+    18944 deep, 8 to 512 rows); its choice is 1.2 % behind the best of them in the mean, 10 % at worst. No split of less than
+    192 deep in the mean: a ring that is never full, and products of few columns need no more parts than their readers sum at once
+    (what is left for the last split may be less: 832 deep in four are 256, 256, 256 and 64).
+    The search is native: a prefill's row count is seldom one that was there before, and nothing is launched until its three products
+    have their plans (us for a new count, 1536 to 2048 and 1536, 8960 to 1536 42, 50 and 180 in Python, 0.8 each now)."""
+    return _slab_plan_py(M, N, K) if _rt is None else _rt.slab_plan(M, N, K)
 
 
 MAX_ROWS = 512  # rows of a decode batch the kernels are laid out for

@@ -6,6 +6,7 @@
 //                                 (the numba routine the reference uses for DP sequence balancing)
 //   * merge_intervals           - sort + merge of [start, end) intervals
 //                                 (csrc/interval_op/interval_op.cpp:1-29 in the reference)
+//   * slab_plan, key_ranges     - launch plans of a prefill's row count (launch_plans.hpp)
 #include <pybind11/numpy.h>
 #include <pybind11/pybind11.h>
 #include <pybind11/stl.h>
@@ -13,6 +14,7 @@
 #include <numeric>
 #include <set>
 
+#include "launch_plans.hpp"
 #include "scheduler.hpp"
 
 namespace py = pybind11;
@@ -308,4 +310,6 @@ PYBIND11_MODULE(_runtime, m) {
   m.def("ffd_allocate", &ffd_allocate, py::arg("values"), py::arg("capacity"), py::arg("min_groups"));
   m.def("partition_balanced", &partition_balanced, py::arg("lens"), py::arg("k"), py::arg("min_size") = 1);
   m.def("merge_intervals", &merge_intervals);
+  m.def("slab_plan", &slab_plan);
+  m.def("key_ranges", &key_ranges);
 }
