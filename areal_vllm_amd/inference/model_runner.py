@@ -679,7 +679,9 @@ class ModelRunner:
             return ops.rmsnorm(part, weight, eps, residual, gemma)
 
         x, residual = ops.rmsnorm(h, layers[0].ln1, eps, None, gemma)
-        qkv_tiles = sk.qkv_row_tiles(Bp, H, (hq + 2 * hkv) * D, D) if self.fused_qkv_rope else 0
+        qkv_tiles = 0
+        if self.fused_qkv_rope and all(b.attn.qkv.data_ptr() % 16 == 0 for b in layers):  # (its lanes load 16 bytes)
+            qkv_tiles = sk.qkv_row_tiles(Bp, H, (hq + 2 * hkv) * D, D)
         for li, blk in enumerate(layers):
             kc, vc = self.kv[li]
             if qkv_tiles:

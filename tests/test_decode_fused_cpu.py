@@ -9,6 +9,7 @@ from areal_vllm_amd.inference.model_runner import ModelRunner
 from areal_vllm_amd.models.config import preset
 from areal_vllm_amd.models.transformer import MoE, Transformer
 from areal_vllm_amd.ops import decode_gemm as dg
+from areal_vllm_amd.ops import decode_skinny as sk
 from areal_vllm_amd.ops.attention import PAGE_SIZE
 
 
@@ -62,6 +63,27 @@ def test_fused_decode_matches_plain(B, name):
     for (k0, v0), (k1, v1) in zip(kv0, kv1):
         torch.testing.assert_close(k0, k1, atol=1e-4, rtol=1e-4)
         torch.testing.assert_close(v0, v1, atol=1e-4, rtol=1e-4)
+
+
+@pytest.mark.parametrize("offset", [0, 2])
+def test_unaligned_qkv_weights_take_the_split_product(offset, monkeypatch):
+    """The one-launch projection loads 16 bytes a lane and refuses other weights; the split-K product takes them."""
+    torch.manual_seed(0)
+    cfg = preset("tiny")
+    model = Transformer(cfg, dtype=torch.float32, device="cpu").requires_grad_(False).eval()
+    model.flatten()
+    model.init_weights(seed=3)
+    w = model.layers[-1].attn.qkv
+    w.data = torch.cat([torch.zeros(offset), w.data.flatten()])[offset:].view(w.shape)
+    calls = []
+    whole = sk.qkv_rope
+    monkeypatch.setattr(sk, "qkv_rope", lambda *a, **k: calls.append(a[1].data_ptr() % 16) or whole(*a, **k))
+    B, steps, ctx = 9, 2, 40
+    r = ModelRunner(model, 64, 128, B, decode_steps=steps, use_graph=False, buckets=[B], fused_decode=True)
+    assert not r._skinny(B) and sk.qkv_row_tiles(B, cfg.hidden_size, w.shape[0], cfg.head_dim)
+    r.decode(_plan(B, ctx, steps, cfg.vocab_size, seed=7))
+    assert calls == ([0] * steps * cfg.n_layers if w.data_ptr() % 16 == 0 else [])
+    assert (offset == 0) == bool(calls)
 
 
 @pytest.mark.parametrize("how", ["hook", "pre-hook", "global hook", "patched", "subclass", "module"])
