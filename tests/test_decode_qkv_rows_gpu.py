@@ -51,6 +51,30 @@ def test_qkv_rope(M, row_tiles, Hq, Hkv, D, K, fp8, bias):
             assert not written.float().transpose(1, 2).reshape(40 * 32, -1)[untouched].any()
 
 
+@pytest.mark.parametrize("M,row_tiles", [(1, 1), (16, 1), (17, 2), (33, 1), (100, 2)])
+@pytest.mark.parametrize("Hq,Hkv,D,K,fp8,bias", [(12, 2, 128, 1536, False, True), (12, 2, 128, 1536, True, True), (8, 1, 256, 2304, True, False),
+                                                 (3, 3, 16, 64, False, False), (1, 1, 128, 5120, False, True)])
+def test_every_rounding(M, row_tiles, Hq, Hkv, D, K, fp8, bias):
+    """Products in sixteenths are exact in fp32, in any order: bit for bit the bf16 projection, lo c - r(hi s) and hi c + r(lo s) rounded to
+    bf16, and on an fp8 cache those of them that it holds."""
+    g = torch.Generator(device=DEV).manual_seed(M * 7 + K)
+    sixteenths = lambda n, *shape: torch.randint(-n, n + 1, shape, device=DEV, generator=g).float() / 16
+    x, N = sixteenths(5, M, K).bfloat16(), (Hq + 2 * Hkv) * D
+    w, b = sixteenths(2, N, K).bfloat16(), sixteenths(9, N).bfloat16() if bias else None
+    pos, slots = torch.randint(0, 500, (M,), device=DEV, generator=g, dtype=torch.int32), torch.randperm(8 * 32, device=DEV, generator=g)[:M].long()
+    tab = ops.RotaryTable(D, 512, 1e4, DEV)
+    kc, vc = ops.alloc_kv_cache(8, Hkv, D, torch.float8_e4m3fn if fp8 else torch.bfloat16, DEV)
+    q = sk.qkv_rope(x, w, b, pos, slots, tab, kc, vc, Hq, Hkv, D, row_tiles)
+    y = x.float() @ w.float().t() + (b.float() if bias else 0.0)
+    y = y.bfloat16().float().view(M, Hq + 2 * Hkv, 2, D // 2)
+    lo, hi, (c, s) = y[:, :Hq + Hkv, 0], y[:, :Hq + Hkv, 1], (t[pos.long()][:, None] for t in (tab.cos, tab.sin))
+    rot = torch.cat([lo.double() * c.double() - (hi * s).double(), hi.double() * c.double() + (lo * s).double()], -1).float().bfloat16()
+    assert torch.equal(q, rot[:, :Hq])
+    v = y[:, Hq + Hkv:].reshape(M, Hkv, D).bfloat16()
+    assert torch.equal(kc.float()[slots // 32, :, slots % 32], rot[:, Hq:].to(kc.dtype).float())
+    assert torch.equal(vc.float()[slots // 32, :, :, slots % 32], v.to(vc.dtype).float())
+
+
 def test_rule():
     assert sk.qkv_row_tiles(24, 1536, 2048, 128) == 1 and sk.qkv_row_tiles(32, 1536, 2048, 128) == 1
     assert sk.qkv_row_tiles(33, 1536, 2048, 128) == 2 and sk.qkv_row_tiles(64, 1536, 2048, 128) == 2

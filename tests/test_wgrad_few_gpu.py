@@ -71,3 +71,41 @@ def test_no_less_precise_than_large_tiles(M, N, K):
     parts = tg._tile_plan(-(-M // 128), -(-N // 256) * (K // 256), 5)[2]
     err = [float((tg.tgemm_wgrad_(torch.zeros(N, K, device=DEV), dy, x, splits=s).double() - want).norm() / want.norm()) for s in (parts, 0)]
     assert err[1] <= 1.02 * err[0], err  # (the mean over a quarter of a million roundings and more)
+
+
+@pytest.mark.parametrize("splits", [0, 1, 2])
+def test_large_gradients_are_streamed(splits):
+    """Gradients from 2^26 elements on pass the caches by: the large tiles' other form."""
+    M, N, K = 1700, 65536 + 128, 1024
+    assert not tg._wgrad_few(M, N // 128 * (K // 128))
+    g = torch.Generator(device=DEV).manual_seed(splits)
+    dy, x = torch.randn(M, N, device=DEV, generator=g).bfloat16(), torch.randn(M, K, device=DEV, generator=g).bfloat16()
+    whole = torch.randn(N, K + 1, device=DEV, generator=g)
+    before = whole.clone()
+    tg.tgemm_wgrad_(whole[:, :K], dy, x, splits=splits)
+    for lo, hi in ((0, 300), (32700, 33100), (N - 400, N)):
+        want = before[lo:hi, :K].double() + dy[:, lo:hi].double().t() @ x.double()
+        # fp32 sums of 1700 products of size one
+        assert float((whole[lo:hi, :K].double() - want).abs().max()) < 1e-3 * M ** 0.5 / 16
+    assert torch.equal(whole[:, K], before[:, K])
+
+
+def test_large_grouped_gradients_are_streamed(monkeypatch):
+    monkeypatch.setenv("AREAL_GROUPED_GEMM", "hip")
+    monkeypatch.delenv("AREAL_GROUPED_GEMM_TILE_M", raising=False)
+    monkeypatch.setattr(G, "FEW_WGRAD_ROWS", 0)
+    monkeypatch.setattr(G, "_big_wgrad", lambda *a: True)
+    counts, N, K = [0, 1, 300, 257, 64, 0, 700, 129], 4096 + 128, 2048
+    g = torch.Generator(device=DEV).manual_seed(1)
+    x = torch.randn(sum(counts), K, device=DEV, generator=g).bfloat16()
+    w = torch.empty(len(counts), N, K, device=DEV, dtype=torch.bfloat16).normal_(0, K ** -0.5, generator=g).requires_grad_(True)
+    w.main_grad = torch.ones(len(counts), N, K, device=DEV)
+    assert w.numel() >= 1 << 26
+    dy = (torch.randn(sum(counts), N, device=DEV, generator=g) / N ** 0.5).bfloat16()
+    ops.grouped_gemm(x, w, counts).backward(dy)
+    at = 0
+    for e, n in enumerate(counts):
+        want = dy[at:at + n].double().t() @ x[at:at + n].double()
+        # fp32 sums of up to 700 products of size N ** -0.5
+        assert float((w.main_grad[e].double() - 1.0 - want).abs().max()) < 1e-4
+        at += n
