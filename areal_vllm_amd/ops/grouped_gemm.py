@@ -45,8 +45,8 @@ BIG_MIN_ROWS, BIG_MIN_FILL = 128, 0.54
 # past the caches 553, 810, 949, 1092, 1624); 2048 columns, 768 deep 341 / 285, 420 / 349, 492 / 449, 574 / 562, 871 / 991; 8 of 28672 columns, 4096
 # deep, 400 / 1024 / 2048 rows 1929 / 1352, 2694 / 2285, 3847 / 4074; 16 of 1536 columns, 768 deep, 1024 rows 69 / 56.
 FEW_WGRAD_ROWS = 1024
-# What else the large ones ask for; their experts may be large from many rows on only.
-BIG_WGRAD_MIN_ROWS, BIG_WGRAD_MAX_SIZE, BIG_WGRAD_ANY_SIZE_ROWS = 384, 1 << 24, 2048
+# Their experts may be large from many rows on only.
+BIG_WGRAD_MAX_SIZE, BIG_WGRAD_ANY_SIZE_ROWS = 1 << 24, 2048
 # A tile of dW is reduced by one workgroup: behind an expert with many times the mean's rows the chip waits for its few large
 # tiles. us of tiles of 128 x 128 (each expert's on all XCDs) / the large ones, largest expert 4 / 8 / 16 / 53 means: 128 experts, 1400
 # rows on average, 1536 columns, 2048 deep 1473, 1476, 1483, 1745 and 1412, 1603, 1845, 3032; 2048 columns, 768 deep 874, 878, 930, 1443 and
@@ -65,7 +65,8 @@ def _big_tiles(T: int, E: int, N: int) -> bool:
 
 
 def _big_wgrad(T: int, E: int, N: int, K: int, counts: List[int]) -> bool:
-    return (T >= BIG_WGRAD_MIN_ROWS * E and K % 256 == 0 and (N * K <= BIG_WGRAD_MAX_SIZE or T >= BIG_WGRAD_ANY_SIZE_ROWS * E)
+    """Tiles of 256 x 256 for an fp32 dW (not where AREAL_GROUPED_GEMM_TILE_M asks for the small kernels, as for out and dx)."""
+    return (T >= FEW_WGRAD_ROWS * E and K % 256 == 0 and (N * K <= BIG_WGRAD_MAX_SIZE or T >= BIG_WGRAD_ANY_SIZE_ROWS * E)
             and _rounds_filled(E * -(-N // 256) * (K // 256)) and max(counts) * E <= BIG_WGRAD_CROWDED * T
             and "AREAL_GROUPED_GEMM_TILE_M" not in os.environ)
 
@@ -159,7 +160,7 @@ class _GroupedGemmFn(torch.autograd.Function):
                 mg = _fold_target(w)
                 if mg is not None:
                     T = x.shape[0]
-                    if T >= FEW_WGRAD_ROWS * E and _big_wgrad(T, E, N, K, ctx.counts):
+                    if _big_wgrad(T, E, N, K, ctx.counts):
                         L.check(L.lib().areal_tgemm_grouped_wgrad(L.ptr(dy), L.ptr(x), L.ptr(mg), L.ptr(offsets), L.c_int(E),
                                                                   L.c_int(N), L.c_int(K), L.c_int64(mg.stride(0)),
                                                                   L.stream_ptr()), "tgemm_grouped_wgrad")

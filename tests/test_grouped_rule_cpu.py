@@ -11,9 +11,15 @@ M = sys.modules["areal_vllm_amd.ops.moe"]
 
 @pytest.mark.parametrize("T,E,N,K,out,dx,dw", [
     (4 * 400, 4, 2048, 768, False, False, False),  # 66 tiles; 25; 96
-    (8 * 400, 8, 2816, 512, True, False, True),  # 182 tiles, 33, 176
-    (16 * 400, 16, 2048, 768, False, False, True),  # 264 (a second round for 8), 99, 384
-    (16 * 1000, 16, 2816, 2048, True, True, True),
+    (8 * 400, 8, 2816, 512, True, False, False),  # 182 tiles, 33, 176
+    (16 * 400, 16, 2048, 768, False, False, False),  # 264 (a second round for 8), 99, 384
+    (16 * 1000, 16, 2816, 2048, True, True, False),
+    (16 * 1023, 16, 2048, 768, True, True, False),  # gradients of 1024 rows an expert and more
+    (16 * 1024, 16, 2048, 768, True, True, True),  # 384
+    (4 * 1024, 4, 2048, 768, True, False, False),  # 96 in one round
+    (8 * 1024, 8, 2816, 512, True, False, True),  # 176
+    (8 * 2047, 8, 28672, 4096, True, True, False),  # large experts
+    (8 * 2048, 8, 28672, 4096, True, True, True),
     (128 * 200, 128, 1536, 2048, True, True, False),  # gradients of few rows
     (128 * 1024, 128, 1536, 2048, True, True, True),
     (128 * 127, 128, 1536, 2048, False, False, False),
