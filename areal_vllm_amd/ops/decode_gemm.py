@@ -70,7 +70,7 @@ def pick_config(M: int, N: int, K: int, epilogue: int) -> Tuple[int, int, int, i
     kept in ``profiles/dgemm_probe_qwen2-1.5b_s2.log``): small-N layers take small tiles and as many K splits as fill the
     chip once, wide layers tiles as tall as the batch; four LDS stages where they fit; dedicated loader waves and
     non-temporal weight loads are worth 3-8 % except on the widest tiles. Partial sums take it only where their operands
-    are not 16-byte aligned (`slab_plan` otherwise)."""
+    are not 16-byte aligned or a configuration is given (`slab_plan` otherwise)."""
     override = _OVERRIDES.get((M, N, K, epilogue))
     if override is not None:
         return override
@@ -349,6 +349,7 @@ def splitk_rope_cache_write(slab: torch.Tensor, n_split: int, bias: Optional[tor
 
 # (cfg, stages, loader_waves, nt) of the fused qkv projection by batch rows, from ``tools/dgemm_probe.py --layers qkv_rope``
 # (profiles/dgemm_probe_qkv_rope_s12.log): 32-row tiles up to 256 rows, 64-row tiles above; four dedicated loader waves
+# (the decode step calls it with 512 rows only, see below; fewer are for callers of `dgemm_qkv_rope` itself)
 QKV_ROPE_CONFIG = {"small": (9, 4, 4, True), "large": (8, 4, 4, True)}
 # From so many rows on, and up to so deep, the one launch is level with or ahead of the split-K GEMM and its row kernel (captured, cold
 # weights, us of the one / the two): a block of it walks all of K, split-K blocks a part of it. 1536 deep to 2048 columns 320 / 384 /

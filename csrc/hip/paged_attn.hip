@@ -917,6 +917,8 @@ extern "C" int areal_rope_cache_write(void* qkv, const int* pos, const int64_t* 
   if (T == 0) return 0;
   if (D % 16 != 0) return -1;
   const size_t lds = (size_t)(RC_TOK + 7) * Hkv * D * sizeof(bf16_t);
+  // (60 KB beside the lists: what a launch may take without asking, two workgroups of 1024 threads a CU. V rows of more than 768 values, such as
+  // 8 heads of 128, would leave one workgroup a CU, which was not measured: they keep a workgroup a token.)
   if (slots && T >= RC_MIN_TOKENS && lds <= 60 * 1024) {
     hipLaunchKernelGGL(rope_cache_write_many_kernel, dim3((T + RC_TOK - 1) / RC_TOK), dim3(RC_THREADS), lds, st, (bf16_t*)qkv, pos, slots,
                        cos_t, sin_t, kcache, vcache, T, Hq, Hkv, D, max_pos, do_rope, fp8);
