@@ -2,13 +2,14 @@
 
 One decoder layer of a decode step becomes six launches instead of ten:
 
-    x1 (normalised)  --dgemm_qkv_rope (bias + RoPE + KV-cache write in the epilogue)-->  q (rotated), paged K/V
+    x1 (normalised)  --decode_skinny.qkv_rope (bias + RoPE + KV-cache write)-->  q (rotated), paged K/V
     paged attention  --dgemm split-K-->  o slabs    --splitk_residual_rmsnorm-->  residual, x2
     x2  --dgemm + SwiGLU epilogue-->  act  --dgemm split-K-->  down slabs  --splitk_residual_rmsnorm--> residual, x1'
 
-The split-K partial sums are plain fp32 slabs ``[split, M, N]`` summed in split order by the row kernel that
-follows anyway (no atomics: replays of a captured graph are bit-identical). The reference gets this path from
-SGLang's CUDA kernels (``areal/api/cli_args.py:398-454``).
+That first launch serves few rows (``decode_skinny.qkv_row_tiles``); more of them take split-K partial sums and ``splitk_rope_cache_write``,
+one launch more, and 512 rows of up to 1536 deep ``dgemm_qkv_rope``. The split-K partial sums are plain fp32 slabs
+``[split, M, N]`` summed in split order by the row kernel that follows anyway (no atomics: replays of a captured graph are
+bit-identical). The reference gets this path from SGLang's CUDA kernels (``areal/api/cli_args.py:398-454``).
 
 CPU tensors take PyTorch paths with the same rounding points, so the engine's control flow is testable
 without a GPU.

@@ -1113,7 +1113,7 @@ def test_paged_prefill_attention_matches_fp32(prefix, chunk, Hq, Hkv):
 ])
 def test_balanced_swiglu_gemm_matches_fp32(M, Fc, K, cols, mblocks):
     """gate|up GEMM + SwiGLU with one column range of arbitrary width per workgroup (decode_swiglu.hip) against
-    fp32, with the rounding points of the unfused bf16 path, for every instantiated row-tile / column-tile count."""
+    fp32, with the rounding points of the unfused bf16 path, at layers' shapes (every instantiated tile: test_decode_gated_tiles_gpu.py)."""
     from areal_vllm_amd.ops import decode_gemm as DG
 
     torch.manual_seed(M + Fc)
