@@ -28,8 +28,8 @@
 // sum in bf16, sums in fp32.
 //
 // Measured (Qwen2-1.5B, 640-token contexts, captured decode step of 28 layers), split-K path -> this: 1 row 1.44 -> 1.17 ms,
-// 2 rows 1.44 -> 1.24, 4 rows 1.47 -> 1.36, 6 rows 1.58 -> 1.45, 8 rows level. One row: gate|up 13.1 us, down 8.5, o 3.9,
-// qkv 5.2 (8.0 + 4.4, 4.6 + 4.4, 12.5, 4.6 + 4.4 before).
+// 2 rows 1.44 -> 1.24, 4 rows 1.47 -> 1.36, 6 rows 1.58 -> 1.45, 8 rows level (one row is 1.08 ms by now). One row: gate|up 11.8 us,
+// down 7.3, o 3.2, qkv 4.4 (8.0 + 4.4, 4.6 + 4.4, 12.5, 4.6 + 4.4 on the split-K path).
 #include "common.hpp"
 
 namespace {
@@ -45,7 +45,6 @@ struct SKArgs {
   bf16_t* Y;         // SK_RES: [M, N]; SK_GATED: [M, N / 2]; SK_QKV: rotated q [M, Hq, D]
   int64_t xs;
   int M, N, K, cols; // cols: columns of a workgroup (SK_GATED: of either half; SK_QKV: rotated pairs)
-  int wk;            // waves along K: 1, 2, 4 or 8
   float eps;
   int gemma, act;
   const bf16_t* bias;
@@ -128,17 +127,15 @@ DEVINL void put_pair(const SKArgs& a, int head, int d, int m, float lo, float hi
 }
 
 // What follows the projection; sum(j, h, m): the fp32 sum of column j (SK_GATED: of half h; SK_QKV: member h of pair j) of
-// row m, read from LDS.
+// row m, read from LDS. SK_RES: one result a thread, of column rj and row rm, and its residual.
 template <int MODE, typename Sum>
-DEVINL void finish(const SKArgs& a, Sum sum) {
+DEVINL void finish(const SKArgs& a, int rj, int rm, float res, Sum sum) {
   if (MODE == SK_RES) {
-    for (int i = threadIdx.x; i < a.cols * a.M; i += THREADS) {
-      const int j = i % a.cols, m = i / a.cols, n = blockIdx.x * a.cols + j;
-      if (n >= a.N) continue;
-      float s = sum(j, 0, m);
-      if (a.res) s = bf2f(f2bf(s)) + bf2f(a.res[(size_t)m * a.N + n]);
-      a.Y[(size_t)m * a.N + n] = f2bf(s);
-    }
+    const int n = blockIdx.x * a.cols + rj;
+    if (rm >= a.M || n >= a.N) return;
+    float s = sum(rj, 0, rm);
+    if (a.res) s = bf2f(f2bf(s)) + res;
+    a.Y[(size_t)rm * a.N + n] = f2bf(s);
   } else if (MODE == SK_GATED) {
     const int F = a.N >> 1;
     for (int i = threadIdx.x; i < a.cols * a.M; i += THREADS) {
@@ -166,153 +163,199 @@ DEVINL void finish(const SKArgs& a, Sum sum) {
   }
 }
 
-// One and two rows. MT: rows of X (a.M <= MT); RB: weight rows of a register set; NORM: X is normalised first
-// (K <= WK P 512: one turn)
-template <int MT, int RB, bool NORM, int MODE>
+// One and two rows. MT: rows of X (a.M = MT); RB: weight rows of a register set; WK: waves along K; NORM: X is normalised first;
+// TURNS: K > WK P 512, the waves go over their share more than once (not with NORM). Grid: workgroups (SK_QKV: of a head, heads).
+// A launch is a few microseconds long, so what stands ahead of its first load counts: the waves' split is a template parameter and a
+// wave's weight rows are one pointer and a step (rows of a pair, gate | up or the members of a rotation, belong to neighbouring
+// rows j of the workgroup). With both worked out from arguments it was 270 (o) to 500 (gate|up) instructions, 30 to 60 now. What the
+// results need besides the sums is asked for with the operands. Captured, cold weights, 1536 wide, us a launch before / now, one
+// row: qkv 5.24 / 4.40, o 3.82 / 3.16, gate|up 12.86 / 11.81 (a bare stream of these 55 MB: 10.4), down 8.02 / 7.28; two rows: 5.74 /
+// 5.24, 4.18 / 3.44, 13.8 / 12.9, 8.55 / 7.95. 8 steps of 28 layers at one row 9.50 -> 8.76 ms.
+template <int MT, int RB, int WK, bool NORM, int MODE, bool TURNS>
 __global__ __launch_bounds__(THREADS) void skinny_dot_kernel(const SKArgs a) {
+  constexpr int NWR = WAVES / WK;
+  constexpr bool PAIRED = MODE != SK_RES;
   extern __shared__ __attribute__((aligned(16))) float rf[];  // [WK][rows of the workgroup][MT]
   __shared__ float sq[WAVES][MT];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wk = wave & (a.wk - 1), wr = wave / a.wk, nwr = WAVES / a.wk;
-  const int pieces = a.K >> 3;                                 // 16-byte pieces of a row
-  const int seg = (pieces + a.wk - 1) / a.wk;                  // of a wave's share
-  const int nrows = MODE == SK_RES ? a.cols : 2 * a.cols;
+  const int wk = wave & (WK - 1), wr = wave / WK;
+  const int nrows = PAIRED ? 2 * a.cols : a.cols;
+  // row j of the workgroup: row b0 + j of W, PAIRED: b0 + j / 2 + (j % 2) second; `have` of them exist
+  int b0, second = 0, have = nrows;
+  if (MODE == SK_QKV) {
+    second = a.D >> 1;
+    b0 = blockIdx.y * a.D + blockIdx.x * a.cols;
+  } else {
+    const int F = MODE == SK_GATED ? a.N >> 1 : a.N;
+    if (MODE == SK_GATED) second = F;
+    b0 = blockIdx.x * a.cols;
+    have = min(a.cols, F - b0) * (PAIRED ? 2 : 1);
+  }
+  const int pieces = a.K >> 3;                // 16-byte pieces of a row
+  const int seg = (pieces + WK - 1) / WK;     // of a wave's share
+  const size_t pitch = (size_t)a.K * sizeof(bf16_t);
+  const char* row = reinterpret_cast<const char*>(a.W) + (size_t)(b0 + (PAIRED ? wr / 2 + (wr & 1) * second : wr)) * pitch;
 
-  // a row of the workgroup -> row of W, or -1
-  auto weight_row = [&](int j) -> int {
-    if (MODE == SK_RES) {
-      const int n = blockIdx.x * a.cols + j;
-      return j < nrows && n < a.N ? n : -1;
-    }
-    const int up = j >= a.cols, i = up ? j - a.cols : j;
-    if (MODE == SK_GATED) {
-      const int F = a.N >> 1, col = blockIdx.x * a.cols + i;
-      return j < nrows && col < F ? col + up * F : -1;
-    }
-    const int half = a.D >> 1, per = half / a.cols;  // workgroups of a head
-    return j < nrows ? (blockIdx.x / per) * a.D + (blockIdx.x % per) * a.cols + i + up * half : -1;
-  };
+  // this thread's result: column (SK_QKV: pair) j of row m
+  const int m = MT == 2 && (int)threadIdx.x >= a.cols ? 1 : 0, j = threadIdx.x - (m ? a.cols : 0);
+  const int jc = min(j, (PAIRED ? have >> 1 : have) - 1);
+  float res = 0.f, blo = 0.f, bhi = 0.f, c = 1.f, s = 0.f;
+  int64_t slot = -1;
 
-  for (int s0 = 0; s0 < seg; s0 += 64 * P) {  // one turn unless K is very long
-    int at[P];   // this lane's pieces
+  for (int s0 = 0; s0 < (TURNS ? seg : 1); s0 += 64 * P) {
+    unsigned at[P];  // this lane's pieces, in bytes
     bool ok[P];
 #pragma unroll
     for (int p = 0; p < P; ++p) {
       const int in = s0 + 64 * p + lane;
       ok[p] = in < seg && wk * seg + in < pieces;
-      at[p] = (ok[p] ? wk * seg + in : 0) * 8;
+      at[p] = (ok[p] ? wk * seg + in : 0) * 16;
     }
     bf16x8 xv[MT][P], nv[NORM ? P : 1];
 #pragma unroll
-    for (int m = 0; m < MT; ++m)
+    for (int i = 0; i < MT; ++i)
 #pragma unroll
-      for (int p = 0; p < P; ++p) xv[m][p] = ld8(a.X + (size_t)(m < a.M ? m : 0) * a.xs + at[p]);
+      for (int p = 0; p < P; ++p)
+        xv[i][p] = *reinterpret_cast<const bf16x8*>(reinterpret_cast<const char*>(a.X + (i ? a.xs : 0)) + at[p]);
     if (NORM)
 #pragma unroll
-      for (int p = 0; p < P; ++p) nv[p] = ld8(a.nw + at[p]);
+      for (int p = 0; p < P; ++p) nv[p] = *reinterpret_cast<const bf16x8*>(reinterpret_cast<const char*>(a.nw) + at[p]);
     __builtin_amdgcn_sched_barrier(0);  // ahead of the weights: loads return in order
 
     bf16x8 wv[2][RB][P];
-    auto load = [&](int set, int first) {
+    const char* next = row;
+    auto load = [&](int set, int first) __attribute__((always_inline)) {  // the rows behind those of the last call
 #pragma unroll
       for (int i = 0; i < RB; ++i) {
-        const int row = weight_row(wr + nwr * (first + i));  // the same for all lanes
-        if (row >= 0)
+        if (wr + NWR * (first + i) < have)  // the same for all lanes
 #pragma unroll
-          for (int p = 0; p < P; ++p)
-            wv[set][i][p] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(a.W + (size_t)row * a.K + at[p]));
+          for (int p = 0; p < P; ++p) wv[set][i][p] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(next + at[p]));
+        if (!PAIRED) next += NWR * pitch;
+        else if (NWR > 1) next += NWR / 2 * pitch;
+        else next += (set * RB + i) & 1 ? pitch - second * pitch : second * pitch;
       }
     };
     load(0, 0);
     load(1, RB);
+    __builtin_amdgcn_sched_barrier(0);
+    if (s0 == 0) {
+      if (MODE == SK_RES && a.res) res = bf2f(a.res[(size_t)m * a.N + b0 + jc]);
+      if (MODE == SK_QKV) {
+        const int head = blockIdx.y, half = a.D >> 1, d = blockIdx.x * a.cols + jc;
+        if (a.bias) {
+          blo = bf2f(a.bias[head * a.D + d]);
+          bhi = bf2f(a.bias[head * a.D + d + half]);
+        }
+        if (head >= a.Hq) slot = a.slots[m];
+        if (a.do_rope && head < a.Hq + a.Hkv) {
+          int p = a.pos[m];
+          p = p < 0 ? 0 : (p >= a.max_pos ? a.max_pos - 1 : p);
+          c = a.cos_t[(size_t)p * half + d];
+          s = a.sin_t[(size_t)p * half + d];
+        }
+      }
+    }
     __builtin_amdgcn_sched_barrier(0);
 
     // pieces beyond the wave's share count as zeros
 #pragma unroll
     for (int p = 0; p < P; ++p)
 #pragma unroll
-      for (int m = 0; m < MT; ++m)
-        if (!ok[p]) xv[m][p] = bf16x8{};
+      for (int i = 0; i < MT; ++i)
+        if (!ok[p]) xv[i][p] = bf16x8{};
     if (NORM) {  // every wave normalises its share for itself; with one wave along K no other is asked
       float ss[MT], fold[(MT + 3) / 4];
 #pragma unroll
-      for (int m = 0; m < MT; ++m) {
-        ss[m] = 0.f;
+      for (int i = 0; i < MT; ++i) {
+        ss[i] = 0.f;
 #pragma unroll
         for (int p = 0; p < P; ++p)
 #pragma unroll
-          for (int e = 0; e < 8; ++e) ss[m] += bf2f(xv[m][p][e]) * bf2f(xv[m][p][e]);
+          for (int e = 0; e < 8; ++e) ss[i] += bf2f(xv[i][p][e]) * bf2f(xv[i][p][e]);
       }
       lane_sums<MT>(ss, fold);
 #pragma unroll
-      for (int m = 0; m < MT; ++m) {  // value m sits in the lanes of row {0, 2, 1, 3}[m % 4]
+      for (int i = 0; i < MT; ++i) {  // value i sits in the lanes of row {0, 2, 1, 3}[i % 4]
         constexpr int row_of[4] = {0, 2, 1, 3};
-        ss[m] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(fold[m >> 2]), 16 * row_of[m & 3]));
+        ss[i] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(fold[i >> 2]), 16 * row_of[i & 3]));
       }
-      if (a.wk > 1) {
+      if (WK > 1) {
 #pragma unroll
-        for (int m = 0; m < MT; ++m)
-          if (lane == m) sq[wave][m] = ss[m];
+        for (int i = 0; i < MT; ++i)
+          if (lane == i) sq[wave][i] = ss[i];
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
 #pragma unroll
-        for (int m = 0; m < MT; ++m) {
+        for (int i = 0; i < MT; ++i) {
           float t = 0.f;
-          for (int w = 0; w < a.wk; ++w) t += sq[wave - wk + w][m];
-          ss[m] = t;
+          for (int w = 0; w < WK; ++w) t += sq[wave - wk + w][i];
+          ss[i] = t;
         }
       }
 #pragma unroll
-      for (int m = 0; m < MT; ++m) {
-        const float rstd = rsqrtf(ss[m] / (float)a.K + a.eps);
+      for (int i = 0; i < MT; ++i) {
+        const float rstd = rsqrtf(ss[i] / (float)a.K + a.eps);
 #pragma unroll
         for (int p = 0; p < P; ++p)
 #pragma unroll
           for (int e = 0; e < 8; ++e)
-            xv[m][p][e] = f2bf(bf2f(xv[m][p][e]) * rstd * (bf2f(nv[p][e]) + (a.gemma ? 1.f : 0.f)));
+            xv[i][p][e] = f2bf(bf2f(xv[i][p][e]) * rstd * (bf2f(nv[p][e]) + (a.gemma ? 1.f : 0.f)));
       }
     }
 
-    auto multiply = [&](int set, int first) {
+    auto multiply = [&](int set, int first) __attribute__((always_inline)) {
       float acc[RB * MT], fold[(RB * MT + 3) / 4];
 #pragma unroll
       for (int i = 0; i < RB; ++i)
 #pragma unroll
-        for (int m = 0; m < MT; ++m) {
-          acc[i * MT + m] = 0.f;
+        for (int k = 0; k < MT; ++k) {
+          acc[i * MT + k] = 0.f;
 #pragma unroll
-          for (int p = 0; p < P; ++p) acc[i * MT + m] = dot8(wv[set][i][p], xv[m][p], acc[i * MT + m]);
+          for (int p = 0; p < P; ++p) acc[i * MT + k] = dot8(wv[set][i][p], xv[k][p], acc[i * MT + k]);
         }
       lane_sums<RB * MT>(acc, fold);
       if ((lane & 15) == 0) {
         const int g = lane >> 4, in4 = g == 1 ? 2 : g == 2 ? 1 : g;  // which of four values this row of lanes holds
 #pragma unroll
-        for (int j = 0; j < (RB * MT + 3) / 4; ++j) {
-          const int v = 4 * j + in4, row = wr + nwr * (first + v / MT);
-          if (v < RB * MT && row < nrows) {
-            float* d = rf + ((size_t)wk * nrows + row) * MT + v % MT;
-            *d = s0 == 0 ? fold[j] : *d + fold[j];
+        for (int f = 0; f < (RB * MT + 3) / 4; ++f) {
+          const int v = 4 * f + in4, r = wr + NWR * (first + v / MT);
+          if (v < RB * MT && r < nrows) {
+            float* d = rf + ((size_t)wk * nrows + r) * MT + v % MT;
+            *d = !TURNS || s0 == 0 ? fold[f] : *d + fold[f];
           }
         }
       }
     };
-    for (int first = 0; wr + nwr * first < nrows; first += 2 * RB) {
+    for (int first = 0; wr + NWR * first < nrows; first += 2 * RB) {
 #pragma unroll
       for (int set = 0; set < 2; ++set) {
-        if (wr + nwr * (first + set * RB) < nrows) {
+        if (wr + NWR * (first + set * RB) < nrows) {
           multiply(set, first + set * RB);
-          if (wr + nwr * (first + (set + 2) * RB) < nrows) load(set, first + (set + 2) * RB);
+          if (wr + NWR * (first + (set + 2) * RB) < nrows) load(set, first + (set + 2) * RB);
         }
       }
     }
   }
   __syncthreads();
-  finish<MODE>(a, [&](int j, int h, int m) {
-    float s = 0.f;
-    for (int w = 0; w < a.wk; ++w) s += rf[((size_t)w * nrows + j + h * a.cols) * MT + m];
-    return s;
-  });
+  if ((int)threadIdx.x >= MT * a.cols || j != jc) return;
+  auto sum = [&](int h) __attribute__((always_inline)) {
+    float t = 0.f;
+#pragma unroll
+    for (int w = 0; w < WK; ++w) t += rf[((size_t)w * nrows + (PAIRED ? 2 * j + h : j)) * MT + m];
+    return t;
+  };
+  if (MODE == SK_RES) {
+    float t = sum(0);
+    if (a.res) t = bf2f(f2bf(t)) + res;
+    a.Y[(size_t)m * a.N + b0 + j] = f2bf(t);
+  } else if (MODE == SK_GATED) {
+    // gate / up rounded to bf16 first: the values an unfused bf16 GEMM output would carry
+    const float g = bf2f(f2bf(sum(0))), u = bf2f(f2bf(sum(1)));
+    a.Y[(size_t)m * (a.N >> 1) + b0 + j] = f2bf(sk_gate(g, a.act) * u);
+  } else {
+    put_pair(a, blockIdx.y, blockIdx.x * a.cols + j, m, sum(0), sum(1), blo, bhi, c, s, slot);
+  }
 }
 
 // Three to eight rows, on the matrix cores: CT 16-row weight tiles of a workgroup (SK_GATED: gate tiles, then as many up
@@ -380,6 +423,14 @@ __global__ __launch_bounds__(THREADS) void skinny_mfma_kernel(const SKArgs a) {
   };
   load(0, 0);
   __builtin_amdgcn_sched_barrier(0);
+  int rj = 0, rrow = 0;  // SK_RES: this thread's result, cols x M <= THREADS of them
+  float res = 0.f;
+  if (MODE == SK_RES) {
+    rrow = threadIdx.x / a.cols;
+    rj = threadIdx.x - rrow * a.cols;
+    if (a.res) res = bf2f(a.res[(size_t)min(rrow, a.M - 1) * a.N + min((int)blockIdx.x * a.cols + rj, a.N - 1)]);
+    __builtin_amdgcn_sched_barrier(0);
+  }
 
   if (NORM) {
     if (wave < a.M) {
@@ -438,7 +489,7 @@ __global__ __launch_bounds__(THREADS) void skinny_mfma_kernel(const SKArgs a) {
   for (int ct = 0; ct < CT; ++ct) red[(wave * CT + ct) * 64 + lane] = acc[ct];
   __syncthreads();
   const float* rf = reinterpret_cast<const float*>(red);
-  finish<MODE>(a, [&](int j, int h, int m) {
+  finish<MODE>(a, rj, rrow, res, [&](int j, int h, int m) {
     const int row = MODE == SK_QKV ? j + h * a.cols : j & 15;  // of the tile
     const int ct = MODE == SK_QKV ? 0 : (j >> 4) + h * (CT / 2);
     const int at = ct * 256 + ((row >> 2) * 16 + m) * 4 + (row & 3);
@@ -563,14 +614,29 @@ __global__ __launch_bounds__(THREADS, 4) void qkv_rows_kernel(const SKArgs a) {
   }
 }
 
-template <int MT, int RB, bool NORM, int MODE>
-int sk_dot(SKArgs& a, int blocks, hipStream_t st) {
-  a.wk = 1;
-  while (a.wk < WAVES && a.K > a.wk * P * 512) a.wk *= 2;
-  if (NORM && a.K > a.wk * P * 512) return -4;
-  const size_t lds = (size_t)a.wk * (MODE == SK_RES ? a.cols : 2 * a.cols) * MT * sizeof(float);
-  hipLaunchKernelGGL((skinny_dot_kernel<MT, RB, NORM, MODE>), dim3(blocks), dim3(THREADS), lds, st, a);
+template <int MT, int RB, int WK, bool NORM, int MODE, bool TURNS = false>
+int sk_dot_as(const SKArgs& a, dim3 grid, hipStream_t st) {
+  const size_t lds = (size_t)WK * (MODE == SK_RES ? a.cols : 2 * a.cols) * MT * sizeof(float);
+  hipLaunchKernelGGL((skinny_dot_kernel<MT, RB, WK, NORM, MODE, TURNS>), grid, dim3(THREADS), lds, st, a);
   return (int)hipGetLastError();
+}
+
+// A wave with one or two rows (o, qkv) takes sets of one: sums of rows that it does not have are not worked out.
+template <int MT, int RB, int WK, bool NORM, int MODE>
+int sk_dot_rows(const SKArgs& a, dim3 grid, hipStream_t st) {
+  if constexpr (MODE != SK_GATED)
+    if ((MODE == SK_RES ? a.cols : 2 * a.cols) <= 2 * (WAVES / WK)) return sk_dot_as<MT, 1, WK, NORM, MODE>(a, grid, st);
+  return sk_dot_as<MT, RB, WK, NORM, MODE>(a, grid, st);
+}
+
+template <int MT, int RB, bool NORM, int MODE>
+int sk_dot(const SKArgs& a, dim3 grid, hipStream_t st) {
+  if (a.K <= P * 512) return sk_dot_rows<MT, RB, 1, NORM, MODE>(a, grid, st);
+  if (a.K <= 2 * P * 512) return sk_dot_rows<MT, RB, 2, NORM, MODE>(a, grid, st);
+  if (a.K <= 4 * P * 512) return sk_dot_rows<MT, RB, 4, NORM, MODE>(a, grid, st);
+  if (a.K <= WAVES * P * 512) return sk_dot_rows<MT, RB, WAVES, NORM, MODE>(a, grid, st);
+  if constexpr (!NORM) return sk_dot_as<MT, RB, WAVES, NORM, MODE, true>(a, grid, st);
+  return -4;
 }
 
 template <int CT, int U, bool PRE, bool NORM, int MODE>
@@ -604,8 +670,8 @@ extern "C" int areal_skinny_residual(const void* X, int64_t xs, const void* W, c
   a.M = M; a.N = N; a.K = K;
   a.cols = (N + CUS - 1) / CUS < 16 ? (N + CUS - 1) / CUS : 16;
   const int blocks = (N + a.cols - 1) / a.cols;
-  if (M == 1) return sk_dot<1, 3, false, SK_RES>(a, blocks, st);
-  if (M == 2) return sk_dot<2, 3, false, SK_RES>(a, blocks, st);
+  if (M == 1) return sk_dot<1, 3, false, SK_RES>(a, dim3(blocks), st);
+  if (M == 2) return sk_dot<2, 3, false, SK_RES>(a, dim3(blocks), st);
   if (K <= 64 * WAVES * 6) return sk_mfma<1, 6, false, false, SK_RES>(a, blocks, st);
   return sk_mfma<1, 6, true, false, SK_RES>(a, blocks, st);
 }
@@ -622,8 +688,8 @@ extern "C" int areal_skinny_norm_gated(const void* X, int64_t xs, const void* nw
   while ((F + CUS * rounds - 1) / (CUS * rounds) > 48) ++rounds;
   a.cols = (F + CUS * rounds - 1) / (CUS * rounds);
   const int blocks = (F + a.cols - 1) / a.cols;
-  if (M == 1) return sk_dot<1, 5, true, SK_GATED>(a, blocks, st);
-  if (M == 2) return sk_dot<2, 5, true, SK_GATED>(a, blocks, st);
+  if (M == 1) return sk_dot<1, 5, true, SK_GATED>(a, dim3(blocks), st);
+  if (M == 2) return sk_dot<2, 5, true, SK_GATED>(a, dim3(blocks), st);
   if (a.cols <= 16) return sk_mfma<2, 3, true, true, SK_GATED>(a, blocks, st);
   if (a.cols <= 32) return sk_mfma<4, 3, false, true, SK_GATED>(a, blocks, st);
   return sk_mfma<6, 3, false, true, SK_GATED>(a, blocks, st);
@@ -645,8 +711,9 @@ extern "C" int areal_skinny_norm_qkv(const void* X, int64_t xs, const void* nw, 
   a.do_rope = do_rope; a.fp8 = fp8;
   a.cols = N / 8 <= CUS ? 4 : 8;  // rotated pairs of a workgroup
   const int blocks = N / (2 * a.cols);
-  if (M == 1) return sk_dot<1, 1, true, SK_QKV>(a, blocks, st);
-  if (M == 2) return sk_dot<2, 1, true, SK_QKV>(a, blocks, st);
+  const dim3 of_head(D / 2 / a.cols, Hq + 2 * Hkv);
+  if (M == 1) return sk_dot<1, 3, true, SK_QKV>(a, of_head, st);
+  if (M == 2) return sk_dot<2, 3, true, SK_QKV>(a, of_head, st);
   return sk_mfma<1, 3, true, true, SK_QKV>(a, blocks, st);
 }
 

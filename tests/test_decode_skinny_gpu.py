@@ -82,6 +82,19 @@ def test_norm_qkv_rope(M, Hq, Hkv, D, K, fp8, with_bias):
         assert torch.equal(a.float() != 0, b.float() != 0) or float(((a.float() != 0) != (b.float() != 0)).sum()) < 3
 
 
+@pytest.mark.parametrize("M", [1, 2])
+@pytest.mark.parametrize("N,K", [(2000, 1600), (256, 3072), (5000, 3136), (1536, 6144), (260, 12288), (7, 12352)])
+def test_linear_residual_of_every_split_of_the_waves(M, N, K):
+    """Two, four and eight waves along K, first and last depth of each; one weight row a wave and many; a last workgroup of few."""
+    test_linear_residual(M, N, K)
+
+
+@pytest.mark.parametrize("M", [1, 2])
+@pytest.mark.parametrize("Hq,Hkv,D,K", [(40, 8, 128, 2048), (2, 1, 128, 8192), (6, 2, 48, 3136), (2, 2, 16, 12288)])
+def test_norm_qkv_rope_of_every_split_of_the_waves(M, Hq, Hkv, D, K):
+    test_norm_qkv_rope(M, Hq, Hkv, D, K, False, True)
+
+
 @pytest.mark.parametrize("rows,hidden,inner,heads,extra", [
     (1, 256, 512, (4, 2, 64), dict(family="qwen2", qkv_bias=True)), (2, 1536, 1024, (12, 2, 128), dict(family="qwen2", qkv_bias=True)),
     (3, 256, 576, (4, 2, 128), dict(family="llama")), (6, 1536, 1024, (12, 2, 128), dict(family="qwen2", qkv_bias=True)),
