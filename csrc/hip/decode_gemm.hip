@@ -551,6 +551,22 @@ DEVINL f32x4 slab_sum4(const float* __restrict__ p, size_t stride, int S) {
   return (a0 + a1) + (a2 + a3);
 }
 
+// The same sums in the same order with the number of slabs known: all of them are asked for before the first is added.
+template <int S>
+struct SlabChunk {
+  f32x4 v[S];
+  DEVINL void load(const float* __restrict__ p, size_t stride) {
+#pragma unroll
+    for (int k = 0; k < S; ++k) v[k] = *reinterpret_cast<const f32x4*>(p + (size_t)k * stride);
+  }
+  DEVINL f32x4 sum() const {
+    f32x4 a[4] = {};
+#pragma unroll
+    for (int k = 0; k < S; ++k) a[k < S / 4 * 4 ? k % 4 : 0] += v[k];
+    return (a[0] + a[1]) + (a[2] + a[3]);
+  }
+};
+
 // s = bf16(sum_k slab[k] [+ bias] [+ res]); res_out = s; y = rmsnorm(s) * w (when w != null, else y = s).
 // One block of THREADS threads per row (M blocks in flight, every thread owns up to MAXC float4 chunks of the row:
 // rows of up to 2048 elements get one chunk per thread, so that all of a thread's loads are in flight at once);
@@ -629,6 +645,62 @@ __global__ __launch_bounds__(THREADS) void splitk_residual_rmsnorm_kernel(
   }
 }
 
+// Rows of up to 4 THREADS columns with residual and weight, of S slabs. A launch of this kind is its start, one round trip to memory (the
+// slabs come from other XCDs) and the block's reduction; with the slabs counted at run time it was a round trip for every four of them,
+// the residual behind them, and 80 instructions ahead of the first. Everything a row needs is asked for at once; one barrier. Captured,
+// 1536 columns, us before / now: 24 rows of 5 / 16 slabs 3.29 / 2.71, 4.31 / 3.62; 93 rows of 3 / 10 3.70 / 2.81, 4.50 / 3.60; 320 rows of 2 /
+// 8 3.88 / 3.38, 6.45 / 6.10. Up to 24 slabs (a plan's most) and one chunk a thread; other rows take the kernel above.
+template <int THREADS, int S>
+__global__ __launch_bounds__(THREADS) void splitk_residual_rmsnorm_row_kernel(
+    const float* __restrict__ slab, const bf16_t* __restrict__ res, const bf16_t* __restrict__ w, bf16_t* __restrict__ res_out,
+    bf16_t* __restrict__ y, int M, int N, float eps, int gemma) {
+  __shared__ __attribute__((aligned(16))) float red[8];
+  const int c = threadIdx.x * 4;
+  const bool in = c < N;
+  const unsigned at = blockIdx.x * (unsigned)N + (in ? c : 0);
+  SlabChunk<S> chunk;
+  chunk.load(slab + at, (size_t)M * N);
+  const bf16x4 rr = *reinterpret_cast<const bf16x4*>(res + at);
+  const bf16x4 ww = *reinterpret_cast<const bf16x4*>(w + (in ? c : 0));
+  __builtin_amdgcn_sched_barrier(0);
+  const f32x4 s = chunk.sum();
+  bf16x4 o;
+  float ss = 0.f;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    o[j] = f2bf(bf2f(f2bf(s[j])) + bf2f(rr[j]));
+    ss += bf2f(o[j]) * bf2f(o[j]);
+  }
+  if (in) *reinterpret_cast<bf16x4*>(res_out + at) = o;
+  ss = wave_sum(in ? ss : 0.f);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
+  __syncthreads();
+  {  // the order of block_sum
+    const f32x4 lo = *reinterpret_cast<const f32x4*>(red), hi = *reinterpret_cast<const f32x4*>(red + 4);
+    float t[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) t[i] = i + 4 < THREADS / 64 ? lo[i] + hi[i] : lo[i];
+    ss = (t[0] + t[2]) + (t[1] + t[3]);
+  }
+  const float rstd = rsqrtf(ss / (float)N + eps);
+  bf16x4 q;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) q[j] = f2bf(bf2f(o[j]) * rstd * (bf2f(ww[j]) + (gemma ? 1.f : 0.f)));
+  if (in) *reinterpret_cast<bf16x4*>(y + at) = q;
+}
+
+template <int THREADS, int S>
+static bool launch_row(const float* slab, int n, const void* res, const void* w, void* res_out, void* y, int M, int N, float eps,
+                       int gemma, hipStream_t st) {
+  if constexpr (S > 0) {
+    if (n != S) return launch_row<THREADS, S - 1>(slab, n, res, w, res_out, y, M, N, eps, gemma, st);
+    hipLaunchKernelGGL((splitk_residual_rmsnorm_row_kernel<THREADS, S>), dim3(M), dim3(THREADS), 0, st, slab, (const bf16_t*)res,
+                       (const bf16_t*)w, (bf16_t*)res_out, (bf16_t*)y, M, N, eps, gemma);
+    return true;
+  }
+  return false;
+}
+
 extern "C" int areal_splitk_residual_rmsnorm(const float* slab, int S, const void* bias, const void* res,
                                              const void* w, void* res_out, void* y, int M, int N, float eps,
                                              int gemma, hipStream_t st) {
@@ -636,6 +708,11 @@ extern "C" int areal_splitk_residual_rmsnorm(const float* slab, int S, const voi
   if (N % 4 != 0 || N > 4 * 256 * 16 || S < 1) return -1;
   const int nchunk = N / 4;
   dim3 grid(M);
+  if (res && w && res_out && y && !bias && S <= 24 && (size_t)M * N < (1u << 31)) {
+    if (nchunk <= 256 && launch_row<256, 24>(slab, S, res, w, res_out, y, M, N, eps, gemma, st)) return (int)hipGetLastError();
+    if (nchunk <= 384 && launch_row<384, 24>(slab, S, res, w, res_out, y, M, N, eps, gemma, st)) return (int)hipGetLastError();
+    if (nchunk <= 512 && launch_row<512, 24>(slab, S, res, w, res_out, y, M, N, eps, gemma, st)) return (int)hipGetLastError();
+  }
 #define LAUNCH(MC, TH)                                                                                          \
   hipLaunchKernelGGL((splitk_residual_rmsnorm_kernel<MC, TH>), grid, dim3(TH), 0, st, slab, S, (const bf16_t*)bias, \
                      (const bf16_t*)res, (const bf16_t*)w, (bf16_t*)res_out, (bf16_t*)y, M, N, eps, gemma)
@@ -651,25 +728,33 @@ extern "C" int areal_splitk_residual_rmsnorm(const float* slab, int S, const voi
 
 // qkv = bf16(sum_k slab[k] + bias), laid out [T, Hq + 2 Hkv, D]: rotate q and k (half-split layout), write q to
 // q_out [T, Hq, D] (bf16), k / v into the paged caches at slots[t] (K [P, Hkv, 32, D], V [P, Hkv, D, 32]).
-// One block per token (SPLIT: and `heads` heads; 64 .. 1024 threads): the summed columns are staged in LDS (fp32), then rotated /
+// DC: D (0: any), SC: S (0: any). One block per token (SPLIT: and `heads` heads; 64 .. 1024 threads): the summed columns are staged in LDS (fp32), then rotated /
 // scattered from there.
-template <bool SPLIT>
+template <bool SPLIT, int DC, int SC>
 __global__ __launch_bounds__(1024) void splitk_rope_cache_write_kernel(
     const float* __restrict__ slab, int S, const bf16_t* __restrict__ bias, const int* __restrict__ pos,
     const int64_t* __restrict__ slots, const float* __restrict__ cos_t, const float* __restrict__ sin_t,
     bf16_t* __restrict__ q_out, void* __restrict__ kcache, void* __restrict__ vcache, int T, int Hq, int Hkv,
-    int D, int max_pos, int do_rope, const bf16_t* __restrict__ q_norm, const bf16_t* __restrict__ k_norm,
+    int D_, int max_pos, int do_rope, const bf16_t* __restrict__ q_norm, const bf16_t* __restrict__ k_norm,
     float norm_eps, int fp8, int heads) {
   extern __shared__ __attribute__((aligned(16))) float rowbuf[];
   const int t = blockIdx.x;
+  const int D = DC ? DC : D_;
   const int half = D >> 1;
   const int lph = half >> 3;
   const int Nq = (Hq + 2 * Hkv) * D;
   const size_t stride = (size_t)T * Nq;
   const int h0 = SPLIT ? blockIdx.y * heads : 0, h1 = SPLIT ? min(Hq + 2 * Hkv, h0 + heads) : Hq + 2 * Hkv;  // this block's heads
   const int c0 = h0 * D;
-  // Position, slot and this thread's first rotary-table rows are requested before the slab sum, so that their
-  // latency (a dependent pos -> table chain) runs under the slab loads instead of after the barrier.
+  // The first columns' slabs and bias are requested, then position and slot, then this thread's first rotary-table rows (a dependent
+  // pos -> table chain): all of it is on its way before the first value is used.
+  const int ncol = (SPLIT ? (h1 - h0) * D : Nq) >> 2;
+  const float* row = slab + (size_t)t * Nq + c0;
+  SlabChunk<SC ? SC : 1> chunk;
+  bf16x4 b_pre = {};
+  const int first_col = min((int)threadIdx.x, ncol - 1) * 4;
+  if (SC) chunk.load(row + first_col, stride);
+  if (bias) b_pre = *reinterpret_cast<const bf16x4*>(bias + c0 + first_col);
   int p = pos[t];
   p = p < 0 ? 0 : (p >= max_pos ? max_pos - 1 : p);
   const int64_t slot = slots ? slots[t] : -1;
@@ -681,10 +766,13 @@ __global__ __launch_bounds__(1024) void splitk_rope_cache_write_kernel(
     const f32x4* sp4 = reinterpret_cast<const f32x4*>(sin_t + (size_t)p * half + sub0 * 8);
     c_pre[0] = cp4[0]; c_pre[1] = cp4[1]; s_pre[0] = sp4[0]; s_pre[1] = sp4[1];
   }
-  for (int c = threadIdx.x; c < ((SPLIT ? (h1 - h0) * D : Nq) >> 2); c += blockDim.x) {
-    f32x4 s = slab_sum4(slab + (size_t)t * Nq + c0 + c * 4, stride, S);
+  for (int c = threadIdx.x; c < ncol; c += blockDim.x) {
+    const bool first = c == (int)threadIdx.x;
+    f32x4 s;
+    if (SC && first) s = chunk.sum();
+    else s = slab_sum4(row + c * 4, stride, S);
     if (bias) {
-      const bf16x4 b = *reinterpret_cast<const bf16x4*>(bias + c0 + c * 4);
+      const bf16x4 b = first ? b_pre : *reinterpret_cast<const bf16x4*>(bias + c0 + c * 4);
 #pragma unroll
       for (int j = 0; j < 4; ++j) s[j] += bf2f(b[j]);
     }
@@ -772,6 +860,16 @@ __global__ __launch_bounds__(1024) void splitk_rope_cache_write_kernel(
   }
 }
 
+// The kernel for heads of DC and S slabs (more than SC of them: counted at run time). With both known the slabs are asked for at once,
+// ahead of the position that the angles wait for, and places in a head are shifts: 12 heads of 128 on 2, 93 / 160 / 320 tokens of 3 / 2 / 2
+// slabs 3.86 / 4.40 / 5.34 -> 3.36 / 3.51 / 4.66 us. Heads of other sizes keep one form.
+template <int DC, int SC>
+static auto rope_row_kernel(bool split, int S) {
+  if constexpr (SC > 0)
+    if (S != SC) return rope_row_kernel<DC, SC - 1>(split, S);
+  return split ? splitk_rope_cache_write_kernel<true, DC, SC> : splitk_rope_cache_write_kernel<false, DC, SC>;
+}
+
 extern "C" int areal_splitk_rope_cache_write(const float* slab, int S, const void* bias, const int* pos,
                                              const int64_t* slots, const float* cos_t, const float* sin_t,
                                              void* q_out, void* kcache, void* vcache, int T, int Hq, int Hkv, int D,
@@ -793,7 +891,8 @@ extern "C" int areal_splitk_rope_cache_write(const float* slab, int S, const voi
   const bool split = T <= 160 || (long)T * all * D <= 524288;
   const int heads = split ? std::min(all, std::max(1, (all * D <= 2048 ? 256 : 512) / D)) : all;
   const int threads = std::min(1024, std::max(split ? 64 : 256, ((heads * D / 4 + 63) / 64) * 64));
-  const auto kern = split ? splitk_rope_cache_write_kernel<true> : splitk_rope_cache_write_kernel<false>;
+  const auto kern = D == 128 ? rope_row_kernel<128, 8>(split, S) : split ? splitk_rope_cache_write_kernel<true, 0, 0>
+                                                                         : splitk_rope_cache_write_kernel<false, 0, 0>;
   hipLaunchKernelGGL(kern, dim3(T, (all + heads - 1) / heads), dim3(threads), (size_t)heads * D * sizeof(float), st, slab, S,
                      (const bf16_t*)bias, pos, slots, cos_t, sin_t, (bf16_t*)q_out, kcache, vcache, T, Hq, Hkv, D, max_pos,
                      do_rope, (const bf16_t*)q_norm, (const bf16_t*)k_norm, norm_eps, fp8, heads);
