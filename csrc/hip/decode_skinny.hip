@@ -55,6 +55,7 @@ struct SKArgs {
   void* kcache;
   void* vcache;
   int Hq, Hkv, D, max_pos, do_rope, fp8;
+  unsigned per_inv;  // qkv_rows: reciprocal of the column blocks of a head
 };
 
 DEVINL float sk_gate(float x, int act) {
@@ -508,7 +509,9 @@ __global__ __launch_bounds__(THREADS) void skinny_mfma_kernel(const SKArgs a) {
 // 1536 deep to 2048 columns 9 / 16 / 24 / 32 / 48 / 64 rows 7.2 / 5.3, 7.4 / 5.8, 7.5 / 5.9, 7.5 / 6.1, 8.2 / 7.8, 8.5 / 8.2; 896 to
 // 1152 9 / 48 / 96 rows 6.3 / 4.3, 7.5 / 4.8, 7.9 / 6.2; 1024 to 4096 16 / 32 rows 7.4 / 5.1, 8.5 / 7.1; 2048 to 2560 16 rows 8.6 / 7.6.
 // 32 columns a workgroup or 64 rows (fewer loads of the other operand) were slower wherever one round of workgroups is enough
-// (24 rows of the first: 7.4 to 8.7), and beyond that the split-K GEMM is ahead (128 rows 10.2 / 11.1).
+// (24 rows of the first: 7.4 to 8.7), and beyond that the split-K GEMM is ahead (128 rows 10.2 / 11.1). Since then without a division
+// and without a wait ahead of the operands (a bias that was widened where it was loaded held them back): 12 / 24 / 48 rows of the first
+// 6.00 -> 5.43, 6.38 -> 5.84, 8.22 -> 7.77.
 template <int RT>
 __global__ __launch_bounds__(THREADS, 4) void qkv_rows_kernel(const SKArgs a) {
   constexpr int PAIRS = 8, ITEMS = 16 * RT * PAIRS, NI = (ITEMS + THREADS - 1) / THREADS, U = 3;
@@ -516,27 +519,27 @@ __global__ __launch_bounds__(THREADS, 4) void qkv_rows_kernel(const SKArgs a) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, kq = lane >> 4;
-  const int half = a.D >> 1, per = half / PAIRS, nrb = (a.M + 16 * RT - 1) / (16 * RT), ncb = (a.N >> 1) / PAIRS;
-  // the blocks of an XCD: a range of columns, all rows of it one after the other
-  const int q8 = gridDim.x >> 3, id = (blockIdx.x & 7) * q8 + (blockIdx.x >> 3);
-  const int cb = id / nrb, m0 = (id - cb * nrb) * 16 * RT;
-  if (cb >= ncb) return;
-  const int head = cb / per, d0 = (cb - head * per) * PAIRS;
+  // grid: (8 XCDs, row blocks, column blocks of an XCD): a range of columns, all rows of it one after the other
+  const int half = a.D >> 1, ncb = (a.N >> 1) / PAIRS;
+  const int cb0 = blockIdx.x * gridDim.z + blockIdx.z, cb = min(cb0, ncb - 1), m0 = blockIdx.y * 16 * RT;
+  const int head = quotient(cb, half / PAIRS, a.per_inv), d0 = (cb - head * (half / PAIRS)) * PAIRS;
   const int nchunk = a.K >> 6;
   const int mine = wave < nchunk ? (nchunk - wave + WAVES - 1) / WAVES : 0;
   const bool rot = a.do_rope && head < a.Hq + a.Hkv;
 
-  // what the results need: on its way ahead of the operands
+  // what the results need: on its way ahead of the operands, and not looked at before them
   int pos[NI];
   int64_t slot[NI];
-  float blo[NI], bhi[NI];
+  bf16_t blo[NI], bhi[NI];
+  const bf16_t* bias = (a.bias ? a.bias : a.W) + head * a.D + d0;  // (without one: values that are not used)
+  const int* positions = a.pos;
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
-    const int idx = threadIdx.x + i * THREADS, m = min(m0 + idx / PAIRS, a.M - 1), d = d0 + idx % PAIRS;
-    pos[i] = rot ? a.pos[m] : 0;
-    slot[i] = head < a.Hq ? -1 : a.slots[m];
-    blo[i] = a.bias ? bf2f(a.bias[head * a.D + d]) : 0.f;
-    bhi[i] = a.bias ? bf2f(a.bias[head * a.D + d + half]) : 0.f;
+    const int idx = threadIdx.x + i * THREADS, m = min(m0 + idx / PAIRS, a.M - 1);
+    pos[i] = positions[m];
+    slot[i] = a.slots[m];
+    blo[i] = bias[idx % PAIRS];
+    bhi[i] = bias[idx % PAIRS + half];
   }
   const bf16_t* wp = a.W + (size_t)(head * a.D + d0 + (r & 7) + (r >> 3) * half) * a.K + 8 * kq;  // pair j: rows j and j + 8 of the tile
   const bf16_t* xp[RT];
@@ -570,9 +573,9 @@ __global__ __launch_bounds__(THREADS, 4) void qkv_rows_kernel(const SKArgs a) {
   float c[NI], s[NI];
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
-    const int p = pos[i] < 0 ? 0 : (pos[i] >= a.max_pos ? a.max_pos - 1 : pos[i]), d = d0 + (threadIdx.x + i * THREADS) % PAIRS;
-    c[i] = rot ? a.cos_t[(size_t)p * half + d] : 1.f;
-    s[i] = rot ? a.sin_t[(size_t)p * half + d] : 0.f;
+    const int p = max(0, min(pos[i], a.max_pos - 1)), d = d0 + (threadIdx.x + i * THREADS) % PAIRS;
+    c[i] = a.cos_t[(size_t)p * half + d];
+    s[i] = a.sin_t[(size_t)p * half + d];
   }
   __builtin_amdgcn_sched_barrier(0);
   int i = 0;
@@ -610,7 +613,9 @@ __global__ __launch_bounds__(THREADS, 4) void qkv_rows_kernel(const SKArgs a) {
 #pragma unroll
       for (int w = 0; w < WAVES; ++w) v[h] += rf[w * RT * 256 + at];
     }
-    put_pair(a, head, d0 + j, m0 + m, v[0], v[1], blo[n], bhi[n], c[n], s[n], slot[n]);
+    if (cb0 < ncb)
+      put_pair(a, head, d0 + j, m0 + m, v[0], v[1], a.bias ? bf2f(blo[n]) : 0.f, a.bias ? bf2f(bhi[n]) : 0.f, rot ? c[n] : 1.f,
+               rot ? s[n] : 0.f, head < a.Hq ? -1 : slot[n]);
   }
 }
 
@@ -727,10 +732,15 @@ extern "C" int areal_qkv_rows(const void* X, int64_t xs, const void* W, const vo
   a.X = (const bf16_t*)X; a.xs = xs; a.W = (const bf16_t*)W; a.bias = (const bf16_t*)bias; a.Y = (bf16_t*)Y; a.M = M;
   a.N = (Hq + 2 * Hkv) * D; a.K = K; a.pos = pos; a.slots = slots; a.cos_t = cos_t; a.sin_t = sin_t; a.kcache = kcache;
   a.vcache = vcache; a.Hq = Hq; a.Hkv = Hkv; a.D = D; a.max_pos = max_pos; a.do_rope = do_rope; a.fp8 = fp8;
-  const long blocks = (long)((M + 16 * rt - 1) / (16 * rt)) * (a.N / 16);
-  if (blocks > 0x7ffffff0l) return -1;
-  const dim3 grid((unsigned)((blocks + 7) / 8 * 8));
-  if (rt == 1) hipLaunchKernelGGL(qkv_rows_kernel<1>, grid, dim3(THREADS), 0, st, a);
-  else hipLaunchKernelGGL(qkv_rows_kernel<2>, grid, dim3(THREADS), 0, st, a);
+  const int cols = a.N / 16, per = D / 16, most = 65535 * 16 * rt;  // rows of a launch
+  if ((cols + 7) / 8 > 65535) return -1;
+  a.per_inv = reciprocal(cols, per);
+  for (int m = 0; m < M; m += most) {
+    a.M = M - m < most ? M - m : most;
+    const dim3 grid(8, (a.M + 16 * rt - 1) / (16 * rt), (cols + 7) / 8);
+    if (rt == 1) hipLaunchKernelGGL(qkv_rows_kernel<1>, grid, dim3(THREADS), 0, st, a);
+    else hipLaunchKernelGGL(qkv_rows_kernel<2>, grid, dim3(THREADS), 0, st, a);
+    a.X += (size_t)most * xs; a.Y += (size_t)most * Hq * D; a.pos += most; a.slots += most;
+  }
   return (int)hipGetLastError();
 }
