@@ -21,6 +21,8 @@
 //   * waves 4..7 do nothing but issue the LDS-DMA pieces (global_load_lds_dwordx4, 8 rows x 128 B each) of a ring of stages, one raw
 //     s_barrier per 64-deep step, counted vmcnt so that the later stages stay in flight across it; the XOR swizzle that makes the
 //     ds_read_b128 fragment reads conflict-free sits on the per-lane SOURCE address;
+//   * a workgroup's place by reciprocals of the host and 32-bit row products, ahead of the first load: 0.1 us a launch (24 rows, 1536 deep
+//     to 1536 columns 3.81 -> 3.68, 8960 deep 7.30 -> 7.19; gate|up of 320 rows 26.1 -> 25.7).
 //   * product transposed (A = weight rows, B = activation rows). A gated block's weight tiles hold two gate rows and the two matching
 //     up rows of every four, so that a lane has both factors of an output, and a pair of tiles gives it four columns in a row: an
 //     8-byte store. A wave's last tile of an odd number gives two columns.
@@ -49,6 +51,7 @@ struct DTArgs {
   int stages;    // LDS ring
   int nt;        // non-temporal weight loads
   int act;       // gate activation: 0 SiLU (SwiGLU), 1 tanh-approximated GELU (GeGLU)
+  unsigned inv_m, inv_t;  // reciprocals of mblocks and ntiles (quotient)
   int rot;       // range t starts its reduction at step t * rot and wraps round: k_rotation (common.hpp)
 };
 
@@ -165,9 +168,9 @@ __global__ __launch_bounds__(512) void dtile_kernel(const DTArgs a) {
   {
     const int nb = gridDim.x, q = nb >> 3, r = nb & 7, x = blockIdx.x & 7;
     const int pos = (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + (blockIdx.x >> 3);
-    const int rest = pos / a.mblocks;
+    const int rest = quotient(pos, a.mblocks, a.inv_m);
     mb = pos - rest * a.mblocks;
-    sp = rest / a.ntiles;
+    sp = quotient(rest, a.ntiles, a.inv_t);
     tile = rest - sp * a.ntiles;
   }
   const int c0 = tile * a.w;
@@ -197,8 +200,10 @@ __global__ __launch_bounds__(512) void dtile_kernel(const DTArgs a) {
         }
         src[j] = a.W + n * a.K + k0 + 8 * c;
       } else {
-        const int m = min(m0 + row - WR, a.M - 1);
-        src[j] = a.X + (size_t)m * a.xs + k0 + 8 * c;
+        const unsigned m = min(m0 + row - WR, a.M - 1);
+        size_t at = (size_t)m * (unsigned)a.xs;  // (32 by 32 bits: a 64-bit product is four slow instructions a piece)
+        if (a.xs >> 32) at += (size_t)(m * (unsigned)(a.xs >> 32)) << 32;
+        src[j] = a.X + at + k0 + 8 * c;
       }
     }
     const int rot = ROT ? k_start(tile, a.rot, nsteps) : 0;
@@ -310,6 +315,8 @@ int dt_launch_as(DTArgs a, hipStream_t st) {
       attr_set = true;
     }
   }
+  a.inv_m = reciprocal((long)a.ntiles * a.ksplit * a.mblocks, a.mblocks);
+  a.inv_t = reciprocal((long)a.ntiles * a.ksplit, a.ntiles);
   hipLaunchKernelGGL(kern, dim3(a.ntiles * a.ksplit * a.mblocks), dim3(512), a.stages * stage_bytes, st, a);
   return (int)hipGetLastError();
 }
