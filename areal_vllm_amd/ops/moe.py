@@ -75,6 +75,12 @@ class _CombineFn(torch.autograd.Function):
         T, k = w.shape
         dout = dout.contiguous()
         dys = dw = None
+        if all(ctx.needs_input_grad[:2]) and k <= 16 and _hip_rows(ys) and _hip_rows(dout) and T > 0:
+            ys = ys.contiguous()
+            dys, dw = torch.empty_like(ys), torch.empty(T, k, dtype=ys.dtype, device=ys.device)
+            L.check(L.lib().areal_moe_combine_bwd(L.ptr(dout), L.ptr(ys), L.ptr(inv), L.ptr(w), L.ptr(dys), L.ptr(dw), L.c_int64(T),
+                                                  L.c_int(k), L.c_int(ys.shape[1]), L.stream_ptr()), "moe_combine_bwd")
+            return dys, dw.to(ctx.w_dtype), None, None
         if ctx.needs_input_grad[0]:  # dys[p] = w[pair at p] * dout[token at p]
             dys = _gather_rows(dout, order // k, w.reshape(-1)[order].contiguous())
         if ctx.needs_input_grad[1]:  # dw[t, j] = <dout[t], ys[inv[t*k + j]]>

@@ -84,6 +84,55 @@ __global__ __launch_bounds__(256) void moe_combine_dots_kernel(const bf16_t* __r
   }
 }
 
+// Backward of the combine in one pass over the token's rows: dys[inv[t, j], :] = w[t, j] g[t, :] and dw[t, j] = <g[t, :], ys[inv[t, j], :]>,
+// with the roundings and the order of sums of gather_rows (scaled) and combine_dots. Memory bounds it, 2 k + 1 rows a token; the two apart
+// read g twice and reduced the k products one after the other: 16384 tokens of 2048, k = 8, 318 us apart and 231 in one.
+template <int KMAX>
+__global__ __launch_bounds__(256) void moe_combine_bwd_kernel(const bf16_t* __restrict__ g, const bf16_t* __restrict__ ys,
+                                                              const int64_t* __restrict__ inv, const bf16_t* __restrict__ w,
+                                                              bf16_t* __restrict__ dys, bf16_t* __restrict__ dw, int k, int H) {
+  __shared__ float red[4][KMAX];
+  const int64_t t = blockIdx.x;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int64_t rows[KMAX];
+  float wt[KMAX], acc[KMAX];
+#pragma unroll
+  for (int j = 0; j < KMAX; ++j) {
+    rows[j] = j < k ? inv[t * k + j] : 0;
+    wt[j] = j < k ? bf2f(w[t * k + j]) : 0.f;
+    acc[j] = 0.f;
+  }
+  for (int c = threadIdx.x * 8; c < H; c += 256 * 8) {
+    const bf16x8 a = ld8(g + t * (int64_t)H + c);
+    bf16x8 b[KMAX];
+#pragma unroll
+    for (int j = 0; j < KMAX; ++j)
+      if (j < k) b[j] = ld8(ys + rows[j] * (int64_t)H + c);
+#pragma unroll
+    for (int j = 0; j < KMAX; ++j) {
+      if (j < k) {
+        bf16x8 o;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          acc[j] += bf2f(a[i]) * bf2f(b[j][i]);
+          o[i] = f2bf(bf2f(a[i]) * wt[j]);
+        }
+        st8(dys + rows[j] * (int64_t)H + c, o);
+      }
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < KMAX; ++j) {
+    const float v = wave_sum(acc[j]);
+    if (lane == 0) red[wave][j] = v;
+  }
+  __syncthreads();
+  if ((int)threadIdx.x < k) {
+    const int j = threadIdx.x;
+    dw[t * k + j] = f2bf((red[0][j] + red[2][j]) + (red[1][j] + red[3][j]));
+  }
+}
+
 static int check_rows(const void* a, const void* b, int H) {
   if (H % 8 != 0) return -1;
   if (((uintptr_t)a | (uintptr_t)b) % 16 != 0) return -2;
@@ -123,6 +172,20 @@ extern "C" int areal_moe_combine_dots(const void* g, const void* src, const int6
   if (int e = check_rows(g, src, H)) return e;
   hipLaunchKernelGGL(moe_combine_dots_kernel, dim3((unsigned)T), dim3(256), 0, st, (const bf16_t*)g,
                      (const bf16_t*)src, inv, (bf16_t*)dw, T, k, H);
+  return (int)hipGetLastError();
+}
+
+extern "C" int areal_moe_combine_bwd(const void* g, const void* ys, const int64_t* inv, const void* w, void* dys, void* dw, int64_t T,
+                                     int k, int H, hipStream_t st) {
+  if (T == 0) return 0;
+  if (int e = check_rows(g, ys, H)) return e;
+  if ((uintptr_t)dys % 16 != 0) return -2;
+  if (k < 1 || k > 16 || T < 0 || T > 0x7fffffff) return -3;
+#define LAUNCH(KM)                                                                                                              \
+  hipLaunchKernelGGL(moe_combine_bwd_kernel<KM>, dim3((unsigned)T), dim3(256), 0, st, (const bf16_t*)g, (const bf16_t*)ys, inv, \
+                     (const bf16_t*)w, (bf16_t*)dys, (bf16_t*)dw, k, H)
+  if (k <= 2) LAUNCH(2); else if (k <= 4) LAUNCH(4); else if (k <= 8) LAUNCH(8); else LAUNCH(16);
+#undef LAUNCH
   return (int)hipGetLastError();
 }
 
