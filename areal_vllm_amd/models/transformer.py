@@ -326,12 +326,17 @@ class MoE(nn.Module):
         plain = cfg.moe_routing_type in ("aux_loss", "none")
         fused_route = plain and not torch.is_grad_enabled() and not self.training
         raw = None if fused_route else F.linear(xr, router)
-        logits = None if fused_route else raw.float()
+        # no loss looks at the router's logits or probabilities: softmax, top-k and their gradient are one launch each way
+        alone = plain and not (self.training and (cfg.moe_z_loss_coef > 0 or cfg.moe_routing_type == "aux_loss"
+                                                  and cfg.router_aux_loss_coef > 0))
+        logits = None if fused_route or alone else raw.float()
         aux = None
         if cfg.moe_z_loss_coef > 0 and self.training and n_valid > 0:
             aux = aux_scale * cfg.moe_z_loss_coef * torch.logsumexp(logits[:n_valid], -1).square().mean()
-        probs = None if fused_route else torch.softmax(logits, -1)
-        if fused_route:
+        probs = None if fused_route or alone else torch.softmax(logits, -1)
+        if alone and not fused_route:
+            topv, topi = ops.moe_topk_grad(raw, k, cfg.norm_topk_prob)
+        elif fused_route:
             # scoring / serving pass: softmax (fp32 arithmetic on the projection's output), top-k and
             # re-normalisation in one launch; weights in the dtype the combine multiplies in
             topv, topi = ops.moe_route(xr, router, k, cfg.norm_topk_prob, out_dtype=x.dtype)

@@ -9,8 +9,11 @@ k-row gathers: each output row is written once, in a fixed order."""
 import torch
 import torch.nn.functional as F
 
+from torch.autograd.function import once_differentiable
+
 from . import _lib as L
 from . import decode_gemm as dg
+from . import train_gemm
 from .norm_act import rmsnorm
 
 
@@ -120,6 +123,39 @@ def moe_topk(logits: torch.Tensor, k: int, norm: bool, out_dtype=torch.float32):
                                    L.c_int(k), L.c_int(int(bool(norm))), L.ptr(topi), L.ptr(topv) if f32 else None,
                                    None if f32 else L.ptr(topv), L.stream_ptr()), "moe_topk")
     return topv, topi
+
+
+class _TopkFn(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, logits, k, norm):
+        logits = logits.contiguous()
+        topv, topi = moe_topk(logits, k, norm)
+        ctx.save_for_backward(logits, topi)
+        ctx.norm = norm
+        ctx.mark_non_differentiable(topi)
+        return topv, topi
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, dv, _):
+        logits, topi = ctx.saved_tensors
+        (T, E), k = logits.shape, topi.shape[1]
+        out = torch.empty_like(logits)
+        dv = dv.float().contiguous()
+        L.check(L.lib().areal_moe_topk_bwd(L.ptr(logits), L.c_int(L.dtype_flag(logits)), L.c_int64(T), L.c_int(E), L.c_int(k),
+                                           L.c_int(int(bool(ctx.norm))), L.ptr(topi), L.ptr(dv), L.ptr(out), L.stream_ptr()),
+                "moe_topk_bwd")
+        return out, None, None
+
+
+def moe_topk_grad(logits: torch.Tensor, k: int, norm: bool):
+    """`moe_topk` with fp32 weights that a gradient flows through: one launch each way on the GPU (its kernels serve up to 512
+    experts and 64 choices of plain tensors), library operations elsewhere."""
+    if (L.use_hip(logits) and logits.dtype in (torch.float32, torch.bfloat16) and logits.shape[1] <= 512 and k <= min(64, logits.shape[1])
+            and logits.shape[0] > 0 and train_gemm.plain(logits)):
+        return _TopkFn.apply(logits, k, norm)
+    topv, topi = torch.topk(torch.softmax(logits.float(), -1), k, -1)
+    return (topv / topv.sum(-1, keepdim=True) if norm else topv), topi
 
 
 # Where a router's product in partial sums pays: few experts of few columns, whose tiles are few. us of the library's product / of

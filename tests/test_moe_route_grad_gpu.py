@@ -1,11 +1,45 @@
-"""Gradients of a routed layer's glue."""
+"""Gradients of a routed layer's glue: the weights of the choices and the recombination, one launch each."""
 import pytest
 import torch
 
 from areal_vllm_amd import ops
+from areal_vllm_amd.ops import moe
 
 DEV = "cuda:0"
 pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("T,E,k", [(1, 1, 1), (3, 2, 2), (5, 63, 7), (4, 64, 64), (1025, 65, 8), (300, 128, 8), (9, 257, 33), (2, 512, 64)])
+@pytest.mark.parametrize("norm", [True, False])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_weights_of_the_choices(T, E, k, norm, dtype):
+    g = torch.Generator(device=DEV).manual_seed(T + E)
+    z = (torch.randn(T, E, device=DEV, generator=g) * 2).to(dtype).requires_grad_(True)
+    v, i = moe.moe_topk_grad(z, k, norm)
+    assert v.dtype == torch.float32 and not i.requires_grad
+    gv = torch.randn(T, k, device=DEV, generator=g)
+    (dz,) = torch.autograd.grad(v, z, gv)
+    z64 = z.detach().double().requires_grad_(True)
+    want = torch.softmax(z64, -1).gather(1, i)
+    want = want / want.sum(-1, keepdim=True) if norm else want
+    (d64,) = torch.autograd.grad(want, z64, gv.double())
+    # an exponential is off by a few 2^-24, a sum of 512 of them and the quotients by some more; the terms of a gradient cancel
+    # down from the size of g p, 16-bit results are rounded once
+    assert float((v.double() - want).detach().abs().max()) < 2.0 ** -19
+    err = (dz.double() - d64).abs()
+    assert float((err - (2.0 ** -8 * d64.abs() if dtype == torch.bfloat16 else 0.0)).max()) < 2.0 ** -18 * max(1.0, float(gv.abs().max()))
+
+
+def test_choices_next_to_infinities():
+    z = torch.full((2, 70), -float("inf"), device=DEV)
+    z[:, 3], z[:, 69] = 1.0, 2.0
+    z.requires_grad_(True)
+    v, i = moe.moe_topk_grad(z, 2, True)
+    assert i.tolist() == [[69, 3]] * 2
+    (dz,) = torch.autograd.grad(v, z, torch.tensor([[1.0, 0.0], [0.0, 1.0]], device=DEV))
+    p = float(torch.sigmoid(torch.tensor(1.0))) * (1 - float(torch.sigmoid(torch.tensor(1.0))))
+    assert torch.allclose(dz[:, 69].cpu(), torch.tensor([p, -p]), atol=1e-6) and torch.allclose(dz[:, 3].cpu(), torch.tensor([-p, p]), atol=1e-6)
+    assert int((dz != 0).sum()) == 4
 
 
 @pytest.mark.parametrize("T,k,H", [(1, 1, 8), (3, 2, 2040), (5, 3, 2048), (2, 4, 2056), (64, 8, 2048), (7, 9, 4104), (3, 16, 64)])
