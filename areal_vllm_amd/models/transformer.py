@@ -260,12 +260,13 @@ class MoE(nn.Module):
         self.down = nn.Parameter(torch.empty(self.n_local, cfg.hidden_size, f, dtype=dtype, device=device))
         self.aux_loss = None
 
-    def _experts(self, xs, counts):
-        """All local experts on their expert-sorted token slabs: two grouped GEMMs around SwiGLU."""
+    def _experts(self, xs, counts, offsets=None):
+        """All local experts on their expert-sorted token slabs: two grouped GEMMs around SwiGLU. `offsets`: the slabs' row
+        ranges on the device."""
         if xs.shape[0] == 0:
             return xs.new_zeros(0, self.cfg.hidden_size)
-        h = ops.swiglu(ops.grouped_gemm(xs, self.gate_up, counts))
-        return ops.grouped_gemm(h, self.down, counts)
+        h = ops.swiglu(ops.grouped_gemm(xs, self.gate_up, counts, offsets))
+        return ops.grouped_gemm(h, self.down, counts, offsets)
 
     def forward(self, x, tp_group, ep_group=None):
         if not self.token_shard:
@@ -325,7 +326,10 @@ class MoE(nn.Module):
             xr = x * torch.empty_like(x).uniform_(1.0 - eps, 1.0 + eps)
         plain = cfg.moe_routing_type in ("aux_loss", "none")
         fused_route = plain and not torch.is_grad_enabled() and not self.training
-        raw = None if fused_route else F.linear(xr, router)
+        # whole 128 x 256 tiles: the router's gradient is summed into its fp32 buffer by the split weight-gradient product (16384 tokens,
+        # 128 experts of 2048: 33 us; the library, whose tiles are not split, 135 to 171)
+        own_dw = router.shape[0] % 128 == 0 and router.shape[1] % 256 == 0
+        raw = None if fused_route else (ops.linear if own_dw else F.linear)(xr, router)
         # no loss looks at the router's logits or probabilities: softmax, top-k and their gradient are one launch each way
         alone = plain and not (self.training and (cfg.moe_z_loss_coef > 0 or cfg.moe_routing_type == "aux_loss"
                                                   and cfg.router_aux_loss_coef > 0))
@@ -363,7 +367,6 @@ class MoE(nn.Module):
         if self.training:
             self.aux_loss = aux
         flat_e = topi.reshape(-1)
-        n_drop = 0
         if cfg.moe_capacity_factor is not None:
             # at most `cap` (token, choice) pairs per expert; the rest are dropped: they get weight zero and the
             # sentinel expert E, which sorts them behind every real expert's slab, where no expert touches them
@@ -397,18 +400,20 @@ class MoE(nn.Module):
                 h = ops.swiglu(ops.grouped_gemm_offsets(ops.moe_permute(x, order, inv, k, src_row), self.gate_up, offsets))
             ys = ops.grouped_gemm_offsets(h, self.down, offsets)
             return (ys, topv, inv) if parts else ops.moe_combine(ys, topv, order, inv)
+        ep = ep_group is not None and self.ep_size > 1
+        # E experts + the bin of dropped pairs, on their way to the host while the rows are gathered
+        fetch = None if ep and cfg.moe_capacity_factor is None else ops.host_list(offsets)
         xs = ops.moe_permute(x, order, inv, k, src_row)
-        counts = (offsets[1:] - offsets[:-1]).long()  # E experts + the bin of dropped pairs
-        if cfg.moe_capacity_factor is not None:
-            n_drop = int(counts[E])
-        counts = counts[:E]
-        n_keep = T * k - n_drop
-        if ep_group is not None and self.ep_size > 1:
+        ranges = None if fetch is None else fetch()
+        n_drop = 0 if cfg.moe_capacity_factor is None else ranges[E + 1] - ranges[E]
+        if n_drop:  # (a slice of everything would still cost a fill and a copy of all rows on the way back)
+            xs = xs[:T * k - n_drop]
+        if ep:
             from ..parallel.expert_parallel import ep_dispatch_combine
 
-            ys = ep_dispatch_combine(self, xs[:n_keep], counts, ep_group)
+            ys = ep_dispatch_combine(self, xs, (offsets[1:E + 1] - offsets[:E]).long(), ep_group)
         else:
-            ys = self._experts(xs[:n_keep], counts.tolist())
+            ys = self._experts(xs, [ranges[e + 1] - ranges[e] for e in range(E)], offsets[:E + 1])
         if n_drop:
             ys = torch.cat([ys, ys.new_zeros(n_drop, ys.shape[1])])
         # every token gathers its k expert outputs (no scatter-add: each output row is written once)

@@ -6,9 +6,10 @@ below (dW into an fp32 gradient: tiles of 128 x 128 of ``train_gemm.hip``; dW of
 expert with library GEMMs). Counterpart of ``grouped_gemm.ops.gmm`` in the reference
 (``realhf/impl/model/modules/moe/experts.py:195-210``).
 """
+import itertools
 import math
 import os
-from typing import List
+from typing import List, Optional
 
 import torch
 
@@ -306,8 +307,9 @@ def grouped_gemm_rows(x: torch.Tensor, w: torch.Tensor, offsets: torch.Tensor) -
     return grouped_gemm_ref(x, w, [off[e + 1] - off[e] for e in range(E)])
 
 
-def grouped_gemm(x: torch.Tensor, w: torch.Tensor, counts: List[int]) -> torch.Tensor:
-    """x [T, K] rows sorted by expert, w [E, N, K], counts[e] rows per expert (host ints, sum = T)."""
+def grouped_gemm(x: torch.Tensor, w: torch.Tensor, counts: List[int], offsets: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """x [T, K] rows sorted by expert, w [E, N, K], counts[e] rows per expert (host ints, sum = T). `offsets`: the same as int32 row
+    ranges [E + 1] on x's device, where the caller has them."""
     if _hip_ok(x, w) and x.shape[0] > 0 and _prefer_library(x.shape[0], w.shape[0]):
         L.lib()  # on a GPU box the kernel library must exist even when a shape goes to the GEMM library
         return _LibraryLoopFn.apply(x.contiguous(), w, list(counts))
@@ -315,5 +317,7 @@ def grouped_gemm(x: torch.Tensor, w: torch.Tensor, counts: List[int]) -> torch.T
         if x.is_cuda and x.dtype == torch.bfloat16:
             L.lib()  # on a GPU box the library must exist even when a shape falls back
         return grouped_gemm_ref(x, w, counts)
-    offsets = torch.tensor([0] + list(torch.tensor(counts).cumsum(0)), dtype=torch.int32).to(x.device, non_blocking=True)
+    if offsets is None:
+        offsets = torch.tensor([0] + list(itertools.accumulate(counts)), dtype=torch.int32).to(x.device, non_blocking=True)
+    assert offsets.dtype == torch.int32 and offsets.numel() == w.shape[0] + 1
     return _GroupedGemmFn.apply(x.contiguous(), w, offsets, list(counts))

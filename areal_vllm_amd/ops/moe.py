@@ -278,6 +278,23 @@ def moe_sort(flat_e: torch.Tensor, n_experts: int, k: int):
     return order, inv, src_row, offsets
 
 
+def host_list(t: torch.Tensor):
+    """``t.tolist()`` in two halves: starts the copy and returns a function that waits for it (not for what the caller has
+    launched in between)."""
+    if not t.is_cuda:
+        return t.tolist
+    host = torch.empty(t.shape, dtype=t.dtype, pin_memory=True)
+    host.copy_(t, non_blocking=True)
+    done = torch.cuda.Event()
+    done.record(torch.cuda.current_stream(t.device))
+
+    def wait():
+        done.synchronize()
+        return host.tolist()
+
+    return wait
+
+
 def moe_combine(ys: torch.Tensor, w: torch.Tensor, order: torch.Tensor, inv: torch.Tensor) -> torch.Tensor:
     """Expert outputs in expert order ys [T*k, H], routing weights w [T, k] -> [T, H]."""
     return _CombineFn.apply(ys, w, order, inv)
