@@ -439,11 +439,11 @@ class ModelRunner:
             return (x, s) if weight is not None else (s, None)
 
         x, residual = ops.rmsnorm(h, layers[0].ln1, eps, None, gemma)
-        if bt is not None and not tp and balanced and D == 128:  # all launches from one native call
-            norms = [blk.ln1 for blk in layers[1:]] + [None]
+        if bt is not None and not tp and balanced and D == 128:  # the launches of many layers from one native call
+            n = len(layers)
             out = ops.prefill_layers.run(
-                [(b.attn.qkv, b.attn.qkv_bias, b.attn.q_norm if cfg.qk_norm else None, b.attn.k_norm if cfg.qk_norm else None,
-                  b.attn.o, b.ln2, b.mlp.gate_up, b.mlp.down, nw) for b, nw in zip(layers, norms)],
+                ((b.attn.qkv, b.attn.qkv_bias, b.attn.q_norm if cfg.qk_norm else None, b.attn.k_norm if cfg.qk_norm else None,
+                  b.attn.o, b.ln2, b.mlp.gate_up, b.mlp.down, layers[i + 1].ln1 if i + 1 < n else None) for i, b in enumerate(layers)),
                 self.kv, x, residual, pos, slots, rope, cu_q, cu_k, bt, max_q, hq, hkv, D, eps, gemma, act)
             if out is not None:
                 return out, None

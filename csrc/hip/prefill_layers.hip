@@ -3,8 +3,8 @@
 // activation, the down product and its row kernel. Host code only: the kernels are those of decode_swiglu.hip, decode_gemm.hip and
 // flash_attn_paged.hip through their own entries, and every check is theirs.
 //
-// What bounds such a prefill is the host: 252 launches of 28 layers took 2250 us to queue from Python, of 2640 in all, where the
-// kernels take 1950 (93 tokens behind 811); from here 900 to 1000.
+// What bounded such a prefill is the host: 252 launches of 28 layers took 2250 us to queue from Python, of 2640 in all, where the
+// kernels took 1950 (93 tokens behind 811); from here 650, in a few calls that the caller prepares one ahead of the other.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -32,7 +32,8 @@ struct PrefillLayer {
 };
 struct PrefillPass {
   const PrefillLayer* layers;
-  void* x;            // [T, H] bf16: the first layer's normalised input, overwritten
+  const void* first;  // [T, H] bf16: the first layer's normalised input, kept (or x itself: behind the layers of an earlier call)
+  void* x;            // [T, H] bf16: the layers' normalised inputs
   const void* stream;  // [T, H] bf16: the residual stream ahead of the first layer, kept
   void* res[2];       // [T, H] bf16 each: written in turn, res[1] by the last layer
   float* slab;       // the largest of the products' partial sums
@@ -61,7 +62,7 @@ extern "C" int areal_prefill_layers(const PrefillPass* p, hipStream_t st) {
   };
   for (int i = 0; i < p->n_layers; ++i) {
     const PrefillLayer& l = p->layers[i];
-    RUN(product(p->x, l.qkv, N, H, p->qkv_plan));
+    RUN(product(i == 0 ? p->first : p->x, l.qkv, N, H, p->qkv_plan));
     RUN(areal_splitk_rope_cache_write(p->slab, p->qkv_plan[2], l.qkv_bias, p->pos, p->slots, p->cos_t, p->sin_t, p->q, l.kcache,
                                       l.vcache, T, p->Hq, p->Hkv, p->D, p->max_pos, 1, l.q_norm, l.k_norm, p->eps, p->fp8, st));
     RUN(areal_flash_fwd_paged(p->q, l.kcache, l.vcache, p->block_tables, p->max_pages, p->attn, nullptr, p->cu_q, p->cu_k, p->B,

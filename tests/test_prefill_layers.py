@@ -68,3 +68,41 @@ def test_upload():
     got = ModelRunner._upload(SimpleNamespace(device=torch.device("cpu")), arrays)
     for k, v in arrays.items():
         assert got[k].numpy().dtype == v.dtype and np.array_equal(got[k].numpy(), v) and got[k].shape == v.shape
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layers,odd", [(1, None), (2, None), (3, None), (8, None), (9, None), (3, 0), (3, 1), (9, 2), (9, 8)])
+def test_layers_in_several_calls(layers, odd):
+    """Every number of layers around those of the first calls, and a layer whose weight is off the 16-byte grid in each of them: the
+    numbers of the single launches, which take over from the start."""
+    torch.manual_seed(1)
+    cfg = ModelConfig(family="qwen2", vocab_size=512, hidden_size=128, n_layers=layers, n_q_heads=2, n_kv_heads=1, head_dim=128,
+                      intermediate_size=192, max_position_embeddings=512, qkv_bias=True)
+    m = Transformer(cfg, dtype=torch.bfloat16, device=torch.device("cuda"))
+    m.requires_grad_(False)
+    m.flatten()
+    for n, p in m.named_parameters():
+        p.copy_(torch.randn_like(p) * (0.05 if p.dim() > 1 else 0.1) + (p.dim() == 1 and "bias" not in n))
+    plan = dict(input_ids=np.arange(5, dtype=np.int32), positions=np.arange(40, 45, dtype=np.int32), slot_mapping=np.arange(40, 45),
+                cu_q=np.array([0, 5], np.int32), cu_k=np.array([0, 45], np.int32), max_q=5, has_prefix=True,
+                block_tables=np.arange(2, dtype=np.int32)[None], req_ids=np.arange(1), temperature=np.zeros(1, np.float32),
+                top_p=np.ones(1, np.float32), top_k=np.full(1, 1 << 30), sample=np.ones(1, np.int32), logit_rows=np.arange(5))
+    out = []
+    for single in (False, True):
+        if odd is not None:
+            w = m.layers[odd].mlp.down if odd % 2 else m.layers[odd].ln2
+            moved = torch.empty(w.numel() + 4, dtype=w.dtype, device="cuda")[4:].view_as(w)  # 8 bytes past the grid
+            w.data = moved.copy_(w)
+        r = ModelRunner(m, num_pages=2, max_context=64, max_batch=1)
+        if single:
+            r._prefill_fused = lambda rows: False
+        for pair in r.kv:
+            for t in pair:
+                t.copy_(torch.linspace(-1, 1, t.numel(), device="cuda").view_as(t))
+        r.prefill(plan)
+        out.append((r.kept_logits.clone(), [t.clone() for kv in r.kv for t in kv]))
+    (la, ca), (lb, cb) = out
+    # 16-bit roundings of the layers' products (library against split sums) add up over the layers: some steps of 2^-8
+    assert float((la - lb).norm() / lb.norm()) < 2.0 ** -8 * (2 + layers)
+    for a, b in zip(ca, cb):
+        assert float((a.float() - b.float()).norm() / b.float().norm()) < 2.0 ** -8 * (2 + layers)
