@@ -753,13 +753,16 @@ class ModelRunner:
         eps, gemma = cfg.rms_norm_eps, cfg.gemma_norm
         act = "silu" if cfg.hidden_act == "silu" else "gelu_tanh"
         residual = h
+        # one row: the o projection combines the attention's partial results itself
+        parts = st["items"] is not None and h.is_cuda and Bp == 1 and hq * D <= sk.PARTS_MAX_WIDTH and D in (64, 128, 256)
         for li, blk in enumerate(self.model.layers):
             kc, vc = self.kv[li]
             q = sk.norm_qkv_rope(residual, blk.ln1, blk.attn.qkv, blk.attn.qkv_bias, rope_pos, st["slots"], self.rope, kc,
                                  vc, hq, hkv, D, eps=eps, gemma=gemma)
             attn = ops.paged_attention_decode(q, kc, vc, st["block_tables"], st["context_lens"], nsplit=st["nsplit"],
-                                              workspace=st["ws"], items=st["items"])
-            residual = sk.linear_residual(attn.view(Bp, hq * D), blk.attn.o, residual)
+                                              workspace=st["ws"], items=st["items"], combine=not parts)
+            attn = attn.view(Bp, hq * D)
+            residual = sk.parts_residual(attn, st["items"], blk.attn.o, residual) if parts else sk.linear_residual(attn, blk.attn.o, residual)
             a = sk.norm_gated(residual, blk.ln2, blk.mlp.gate_up, eps=eps, gemma=gemma, act=act)
             residual = sk.linear_residual(a, blk.mlp.down, residual)
         return ops.rmsnorm(residual, self.model.norm, eps, None, gemma)[0]

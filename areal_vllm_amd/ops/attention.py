@@ -517,6 +517,7 @@ class DecodeItems:
         if pages is not None:  # a row of n pages is at most sqrt(3 n) items
             self.n_items = min(self.n_items, batch * (math.isqrt(3 * pages) + 1))
         self.items = torch.zeros(self.n_items, 8, dtype=torch.int32, device=device)
+        self.rows = torch.zeros(batch, 2, dtype=torch.int32, device=device)  # first partial result and number of each row's items
         self.part_o = torch.empty(self.n_items, n_q_heads, head_dim, dtype=torch.float32, device=device)
         self.part_ml = torch.empty(self.n_items, n_q_heads, 2, dtype=torch.float32, device=device)
         self.arrived = torch.zeros(batch, n_kv_heads, dtype=torch.int32, device=device)
@@ -525,7 +526,7 @@ class DecodeItems:
         """Lay the items out for these context lengths; every layer of the step then uses them."""
         if L.use_hip(context_lens):
             assert context_lens.dtype == torch.int32 and context_lens.is_contiguous() and context_lens.numel() == self.batch
-            L.check(L.lib().areal_paged_decode_items(L.ptr(context_lens), L.ptr(self.items), L.c_int(self.batch),
+            L.check(L.lib().areal_paged_decode_items(L.ptr(context_lens), L.ptr(self.items), L.ptr(self.rows), L.c_int(self.batch),
                                                      L.c_int(self.target), L.c_int(self.n_items), L.c_int(int(self.finer)),
                                                      L.stream_ptr()),
                     "paged_decode_items")
@@ -534,10 +535,12 @@ class DecodeItems:
 
 def paged_attention_decode(q, kcache, vcache, block_tables, context_lens, scale=None, nsplit=1,
                            workspace: Optional[DecodeWorkspace] = None, out=None, q_row_stride=None,
-                           items: Optional[DecodeItems] = None):
+                           items: Optional[DecodeItems] = None, combine: bool = True):
     """q [B, Hq, D] (may be the q slice of a fused qkv row, pass q_row_stride in elements).
     block_tables int32 [B, max_pages]; context_lens int32 [B] (including the current token). `items`: the work items of
-    these context lengths (`nsplit` and `workspace` are not used then)."""
+    these context lengths (`nsplit` and `workspace` are not used then). Without `combine` the partial results of rows that have
+    several stay in `items.part_o` and `items.part_ml` for a kernel that combines them itself (``decode_skinny.parts_residual``),
+    and the result holds the other rows only."""
     B, Hq, D = q.shape
     Hkv = kcache.shape[1]
     if scale is None:
@@ -545,6 +548,7 @@ def paged_attention_decode(q, kcache, vcache, block_tables, context_lens, scale=
     if not L.use_hip(q):
         return paged_decode_ref(q, kcache, vcache, block_tables, context_lens, scale)
     assert q.dtype == torch.bfloat16 and block_tables.dtype == torch.int32 and context_lens.dtype == torch.int32
+    assert combine or items is not None
     if out is None:
         out = torch.empty(B, Hq, D, dtype=q.dtype, device=q.device)
     if q_row_stride is None:
@@ -554,7 +558,7 @@ def paged_attention_decode(q, kcache, vcache, block_tables, context_lens, scale=
         L.check(
             L.lib().areal_paged_decode_walk(
                 L.ptr(q), L.ptr(kcache), L.ptr(vcache), L.ptr(block_tables), L.ptr(context_lens), L.ptr(items.items),
-                L.c_int(items.n_items), L.ptr(out), L.ptr(items.part_o), L.ptr(items.part_ml), L.ptr(items.arrived),
+                L.c_int(items.n_items), L.ptr(out), L.ptr(items.part_o), L.ptr(items.part_ml), L.ptr(items.arrived if combine else None),
                 L.c_int(Hq), L.c_int(Hkv), L.c_int(D), L.c_int(block_tables.shape[1]), L.c_float(scale),
                 L.c_int(q_row_stride), L.c_int(int(is_fp8(kcache))), L.stream_ptr(),
             ),

@@ -50,6 +50,25 @@ def linear_residual(x: torch.Tensor, w: torch.Tensor, residual: Optional[torch.T
     return y
 
 
+# One row: with two, whose partial results every workgroup would have to combine, the two launches apart are as fast (12 heads of 128 on 2,
+# 640 tokens 10.9 / 11.0 us), and the matrix-core form of more rows reads its operand from memory.
+PARTS_MAX_WIDTH = 8192  # values of the row, in LDS
+
+
+def parts_residual(x: torch.Tensor, items, w: torch.Tensor, residual: torch.Tensor) -> torch.Tensor:
+    """`linear_residual` of one row of attention output as ``paged_attention_decode(.., items=items, combine=False)`` leaves it: `x`
+    or its partial results in `items` (GPU only)."""
+    K, N = items.n_q_heads * items.head_dim, w.shape[0]
+    assert items.batch == 1 and x.numel() == K <= PARTS_MAX_WIDTH and x.dtype == torch.bfloat16 and x.is_contiguous()
+    assert w.dtype == torch.bfloat16 and w.is_contiguous() and w.shape[1] == K
+    assert residual.dtype == w.dtype and residual.shape == (1, N) and residual.is_contiguous()
+    y = torch.empty(1, N, dtype=w.dtype, device=w.device)
+    L.check(L.lib().areal_skinny_parts_residual(L.ptr(x), L.ptr(items.part_o), L.ptr(items.part_ml), L.ptr(items.rows), L.ptr(w),
+                                                L.ptr(residual), L.ptr(y), L.c_int(N), L.c_int(items.n_q_heads), L.c_int(items.head_dim),
+                                                L.stream_ptr()), "skinny_parts_residual")
+    return y
+
+
 def norm_gated(h: torch.Tensor, norm: torch.Tensor, w_gate_up: torch.Tensor, *, eps: float, gemma: bool = False,
                act: str = "silu") -> torch.Tensor:
     """``act(x @ gate.T) * (x @ up.T)`` of ``x = rmsnorm(h) * norm`` with ``w_gate_up = [gate; up]`` -> bf16 [M, F]."""

@@ -55,6 +55,10 @@ struct SKArgs {
   void* kcache;
   void* vcache;
   int Hq, Hkv, D, max_pos, do_rope, fp8;
+  // PARTS: what the decode attention has left of X: partial results rows[0].x .. + rows[0].y, or X itself where that is one
+  const float *part_o, *part_ml;
+  const int2* rows;
+  int d_shift;       // log2 of the head size
   unsigned per_inv;  // qkv_rows: reciprocal of the column blocks of a head
 };
 
@@ -172,7 +176,12 @@ DEVINL void finish(const SKArgs& a, int rj, int rm, float res, Sum sum) {
 // results need besides the sums is asked for with the operands. Captured, cold weights, 1536 wide, us a launch before / now, one
 // row: qkv 5.24 / 4.40, o 3.82 / 3.16, gate|up 12.86 / 11.81 (a bare stream of these 55 MB: 10.4), down 8.02 / 7.28; two rows: 5.74 /
 // 5.24, 4.18 / 3.44, 13.8 / 12.9, 8.55 / 7.95. 8 steps of 28 layers at one row 9.50 -> 8.76 ms.
-template <int MT, int RB, int WK, bool NORM, int MODE, bool TURNS>
+// PARTS (o): X is combined here from the partial results of the decode attention, in the order and with the roundings that it would
+// combine them with itself: every workgroup reads all of them (30 KB at 640 tokens) ahead of its weights, where the attention's
+// last workgroup of a row waits for its stores, a counter, the sums and the results, one trip past the L2 after the other. A row with a
+// single partial result is read as the attention has written it. Captured, attention and o, 12 heads of 128 on 2, us apart / so: 100 / 300 /
+// 640 / 1900 / 6000 / 20000 tokens 7.7 / 7.8, 10.2 / 8.5, 10.3 / 8.9, 12.1 / 10.9, 14.5 / 13.1, 20.5 / 18.8.
+template <int MT, int RB, int WK, bool NORM, int MODE, bool TURNS, bool PARTS>
 __global__ __launch_bounds__(THREADS) void skinny_dot_kernel(const SKArgs a) {
   constexpr int NWR = WAVES / WK;
   constexpr bool PAIRED = MODE != SK_RES;
@@ -204,6 +213,31 @@ __global__ __launch_bounds__(THREADS) void skinny_dot_kernel(const SKArgs a) {
   float res = 0.f, blo = 0.f, bhi = 0.f, c = 1.f, s = 0.f;
   int64_t slot = -1;
 
+  // PARTS: four values a thread and turn, the first eight partial results of the first turn on their way ahead of the weights
+  constexpr int PT = 4 * THREADS;
+  f32x4 po[8];
+  float2 pml[8];
+  int first_part = 0, nparts = 0;
+  auto fetch_parts = [&](int col, int k0) __attribute__((always_inline)) {
+    const float* o = a.part_o + (size_t)(first_part + k0) * a.K + col;
+    const float* ml = a.part_ml + ((size_t)(first_part + k0) * (a.K >> a.d_shift) + (col >> a.d_shift)) * 2;
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+      if (k0 + k < nparts) {  // the same for all lanes
+        po[k] = *reinterpret_cast<const f32x4*>(o + (size_t)k * a.K);
+        pml[k] = *reinterpret_cast<const float2*>(ml + (size_t)k * (a.K >> a.d_shift) * 2);
+      }
+  };
+  bf16_t* xs = reinterpret_cast<bf16_t*>(rf + (WK * nrows * MT + 3) / 4 * 4);  // [K]
+  if constexpr (PARTS) {
+    static_assert(MT == 1);
+    const int2 r = a.rows[0];
+    first_part = r.x;
+    nparts = r.y;
+    if (nparts > 1 && (int)threadIdx.x * 4 < a.K) fetch_parts(threadIdx.x * 4, 0);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+
   for (int s0 = 0; s0 < (TURNS ? seg : 1); s0 += 64 * P) {
     unsigned at[P];  // this lane's pieces, in bytes
     bool ok[P];
@@ -214,6 +248,7 @@ __global__ __launch_bounds__(THREADS) void skinny_dot_kernel(const SKArgs a) {
       at[p] = (ok[p] ? wk * seg + in : 0) * 16;
     }
     bf16x8 xv[MT][P], nv[NORM ? P : 1];
+    if (!PARTS || nparts <= 1)
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
@@ -258,6 +293,45 @@ __global__ __launch_bounds__(THREADS) void skinny_dot_kernel(const SKArgs a) {
       }
     }
     __builtin_amdgcn_sched_barrier(0);
+
+    if (PARTS && nparts > 1) {
+      if (s0 == 0) {
+        for (int col = threadIdx.x * 4; col < a.K; col += PT) {
+          float mm = -INFINITY, ll = 0.f;
+          f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+          for (int k0 = 0; k0 < nparts; k0 += 8) {
+            if (k0 > 0 || col >= PT) fetch_parts(col, k0);
+            float mn = mm;
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+              if (k0 + k < nparts) mn = fmaxf(mn, pml[k].x);
+            const float f0 = mm == -INFINITY ? 0.f : fast_exp2(mm - mn);
+            if (k0 > 0) {
+              acc *= f0;
+              ll *= f0;
+            }
+            mm = mn;
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+              if (k0 + k < nparts) {
+                const float f = pml[k].x == -INFINITY ? 0.f : fast_exp2(pml[k].x - mn);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[e] += po[k][e] * f;
+                ll += pml[k].y * f;
+              }
+          }
+          bf16x4 o;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[e] = f2bf(ll > 0.f ? acc[e] / ll : 0.f);
+          *reinterpret_cast<bf16x4*>(xs + col) = o;
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+      }
+#pragma unroll
+      for (int p = 0; p < P; ++p) xv[0][p] = *reinterpret_cast<const bf16x8*>(reinterpret_cast<const char*>(xs) + at[p]);
+    }
 
     // pieces beyond the wave's share count as zeros
 #pragma unroll
@@ -619,28 +693,30 @@ __global__ __launch_bounds__(THREADS, 4) void qkv_rows_kernel(const SKArgs a) {
   }
 }
 
-template <int MT, int RB, int WK, bool NORM, int MODE, bool TURNS = false>
+template <int MT, int RB, int WK, bool NORM, int MODE, bool PARTS, bool TURNS = false>
 int sk_dot_as(const SKArgs& a, dim3 grid, hipStream_t st) {
-  const size_t lds = (size_t)WK * (MODE == SK_RES ? a.cols : 2 * a.cols) * MT * sizeof(float);
-  hipLaunchKernelGGL((skinny_dot_kernel<MT, RB, WK, NORM, MODE, TURNS>), grid, dim3(THREADS), lds, st, a);
+  size_t lds = (size_t)WK * (MODE == SK_RES ? a.cols : 2 * a.cols) * MT * sizeof(float);
+  if (PARTS) lds = (lds + 15) / 16 * 16 + (size_t)a.K * sizeof(bf16_t);
+  if (lds > 64 * 1024) return -4;
+  hipLaunchKernelGGL((skinny_dot_kernel<MT, RB, WK, NORM, MODE, TURNS, PARTS>), grid, dim3(THREADS), lds, st, a);
   return (int)hipGetLastError();
 }
 
 // A wave with one or two rows (o, qkv) takes sets of one: sums of rows that it does not have are not worked out.
-template <int MT, int RB, int WK, bool NORM, int MODE>
+template <int MT, int RB, int WK, bool NORM, int MODE, bool PARTS>
 int sk_dot_rows(const SKArgs& a, dim3 grid, hipStream_t st) {
   if constexpr (MODE != SK_GATED)
-    if ((MODE == SK_RES ? a.cols : 2 * a.cols) <= 2 * (WAVES / WK)) return sk_dot_as<MT, 1, WK, NORM, MODE>(a, grid, st);
-  return sk_dot_as<MT, RB, WK, NORM, MODE>(a, grid, st);
+    if ((MODE == SK_RES ? a.cols : 2 * a.cols) <= 2 * (WAVES / WK)) return sk_dot_as<MT, 1, WK, NORM, MODE, PARTS>(a, grid, st);
+  return sk_dot_as<MT, RB, WK, NORM, MODE, PARTS>(a, grid, st);
 }
 
-template <int MT, int RB, bool NORM, int MODE>
+template <int MT, int RB, bool NORM, int MODE, bool PARTS = false>
 int sk_dot(const SKArgs& a, dim3 grid, hipStream_t st) {
-  if (a.K <= P * 512) return sk_dot_rows<MT, RB, 1, NORM, MODE>(a, grid, st);
-  if (a.K <= 2 * P * 512) return sk_dot_rows<MT, RB, 2, NORM, MODE>(a, grid, st);
-  if (a.K <= 4 * P * 512) return sk_dot_rows<MT, RB, 4, NORM, MODE>(a, grid, st);
-  if (a.K <= WAVES * P * 512) return sk_dot_rows<MT, RB, WAVES, NORM, MODE>(a, grid, st);
-  if constexpr (!NORM) return sk_dot_as<MT, RB, WAVES, NORM, MODE, true>(a, grid, st);
+  if (a.K <= P * 512) return sk_dot_rows<MT, RB, 1, NORM, MODE, PARTS>(a, grid, st);
+  if (a.K <= 2 * P * 512) return sk_dot_rows<MT, RB, 2, NORM, MODE, PARTS>(a, grid, st);
+  if (a.K <= 4 * P * 512) return sk_dot_rows<MT, RB, 4, NORM, MODE, PARTS>(a, grid, st);
+  if (a.K <= WAVES * P * 512) return sk_dot_rows<MT, RB, WAVES, NORM, MODE, PARTS>(a, grid, st);
+  if constexpr (!NORM) return sk_dot_as<MT, RB, WAVES, NORM, MODE, PARTS, true>(a, grid, st);
   return -4;
 }
 
@@ -679,6 +755,20 @@ extern "C" int areal_skinny_residual(const void* X, int64_t xs, const void* W, c
   if (M == 2) return sk_dot<2, 3, false, SK_RES>(a, dim3(blocks), st);
   if (K <= 64 * WAVES * 6) return sk_mfma<1, 6, false, false, SK_RES>(a, blocks, st);
   return sk_mfma<1, 6, true, false, SK_RES>(a, blocks, st);
+}
+
+// The same of one row of the decode attention's output, K = Hq heads of D (64, 128 or 256), that it has left as rows[0].y > 1 partial
+// results from rows[0].x on, part_o [.., Hq, D] and part_ml [.., Hq, 2], or written to X.
+extern "C" int areal_skinny_parts_residual(const void* X, const float* part_o, const float* part_ml, const void* rows, const void* W,
+                                           const void* res, void* Y, int N, int Hq, int D, hipStream_t st) {
+  if (Hq < 1 || (D != 64 && D != 128 && D != 256)) return -1;
+  if (int rc = sk_check(X, 0, W, 1, N, Hq * D)) return rc;
+  if ((uintptr_t)part_o % 16 != 0 || ((uintptr_t)part_ml | (uintptr_t)rows) % 8 != 0) return -2;
+  SKArgs a = {};
+  a.X = (const bf16_t*)X; a.W = (const bf16_t*)W; a.res = (const bf16_t*)res; a.Y = (bf16_t*)Y; a.M = 1; a.N = N; a.K = Hq * D;
+  a.part_o = part_o; a.part_ml = part_ml; a.rows = (const int2*)rows; a.d_shift = D == 64 ? 6 : D == 128 ? 7 : 8;
+  a.cols = (N + CUS - 1) / CUS < 16 ? (N + CUS - 1) / CUS : 16;
+  return sk_dot<1, 3, false, SK_RES, true>(a, dim3((N + a.cols - 1) / a.cols), st);
 }
 
 // Y [M, F] = gate(h W_gate^T) * (h W_up^T), h = RMSNorm(X) nw, W = [gate; up] [2F, K]. K <= 8192.

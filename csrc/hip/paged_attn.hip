@@ -357,8 +357,8 @@ DEVINL int pages_per_item(int np, int even) {
 // grid 1, block 1024. n_items >= min(target + B, the rows' largest number of items x B),
 // with `finer` 2 target + B. Pages per item: the whole batch over `target` items.
 __global__ __launch_bounds__(1024) void paged_decode_items_kernel(const int* __restrict__ context_lens,
-                                                                  DecodeItem* __restrict__ items, int B, int target,
-                                                                  int n_items, int finer) {
+                                                                  DecodeItem* __restrict__ items, int2* __restrict__ rows,
+                                                                  int B, int target, int n_items, int finer) {
   constexpr int NB = 64;  // size classes of the sort
   __shared__ int red[16], red_n[16], hist[NB];
   const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
@@ -438,6 +438,7 @@ __global__ __launch_bounds__(1024) void paged_decode_items_kernel(const int* __r
       at += red[w];
     }
     const int base = before + incl - n;
+    if (n > 0 && rows) rows[b] = base + n <= n_items ? make_int2(base, n) : make_int2(0, 0);
     for (int i = 0; i < n; ++i) {
       const int lo = i * per, hi = min(np, lo + per);
       const int place = atomicAdd(&hist[size_class(hi - lo)], 1);
@@ -659,7 +660,7 @@ __global__ __launch_bounds__(64 * NW, (D > 128 ? 1 : 4)) void paged_decode_walk_
       }
     }
   }
-  if (it.n == 1) return;
+  if (it.n == 1 || !arrived) return;
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // every wave's stores have arrived ...
   __syncthreads();
   if (threadIdx.x == 0) {                           // ... before the workgroup is counted
@@ -723,12 +724,12 @@ __global__ __launch_bounds__(64 * NW, (D > 128 ? 1 : 4)) void paged_decode_walk_
   combine(std::integral_constant<int, 2>{});
 }
 
-// Items of the batch's decode attention; `items`: n_items x 8 ints, at least min(target + B, B x most items of a row); with finer 2 target + B.
-extern "C" int areal_paged_decode_items(const int* context_lens, void* items, int B, int target, int n_items, int finer,
+// Items of the batch's decode attention; rows [B] (or null): first partial result and number of a row's items; `items`: n_items x 8 ints, at least min(target + B, B x most items of a row); with finer 2 target + B.
+extern "C" int areal_paged_decode_items(const int* context_lens, void* items, void* rows, int B, int target, int n_items, int finer,
                                         hipStream_t st) {
   if (B < 1 || target < 1 || n_items < B) return -1;
-  hipLaunchKernelGGL(paged_decode_items_kernel, dim3(1), dim3(1024), 0, st, context_lens, (DecodeItem*)items, B, target,
-                     n_items, finer);
+  hipLaunchKernelGGL(paged_decode_items_kernel, dim3(1), dim3(1024), 0, st, context_lens, (DecodeItem*)items, (int2*)rows, B,
+                     target, n_items, finer);
   return (int)hipGetLastError();
 }
 
@@ -753,7 +754,8 @@ static int launch_paged_decode_walk(const void* q, const void* kcache, const voi
   return (int)hipGetLastError();
 }
 
-// Decode attention over the items that areal_paged_decode_items made of the same context lengths.
+// Decode attention over the items that areal_paged_decode_items made of the same context lengths. arrived null: the partial results of
+// rows with several are left in part_o and part_ml for the kernel that follows, and `out` is written for the others only.
 extern "C" int areal_paged_decode_walk(const void* q, const void* kcache, const void* vcache, const int* block_tables,
                                        const int* context_lens, const void* items, int n_items, void* out, float* part_o,
                                        float* part_ml, int* arrived, int Hq, int Hkv, int D, int max_pages,
