@@ -168,7 +168,7 @@ DEVINL void finish(const SKArgs& a, int rj, int rm, float res, Sum sum) {
   }
 }
 
-// One and two rows. MT: rows of X (a.M = MT); RB: weight rows of a register set; WK: waves along K; NORM: X is normalised first;
+// One and two rows, with SK_RES up to eight. MT: rows of X (a.M = MT); RB: weight rows of a register set; WK: waves along K; NORM: X is normalised first;
 // TURNS: K > WK P 512, the waves go over their share more than once (not with NORM). Grid: workgroups (SK_QKV: of a head, heads).
 // A launch is a few microseconds long, so what stands ahead of its first load counts: the waves' split is a template parameter and a
 // wave's weight rows are one pointer and a step (rows of a pair, gate | up or the members of a rotation, belong to neighbouring
@@ -208,7 +208,10 @@ __global__ __launch_bounds__(THREADS) void skinny_dot_kernel(const SKArgs a) {
   const char* row = reinterpret_cast<const char*>(a.W) + (size_t)(b0 + (PAIRED ? wr / 2 + (wr & 1) * second : wr)) * pitch;
 
   // this thread's result: column (SK_QKV: pair) j of row m
-  const int m = MT == 2 && (int)threadIdx.x >= a.cols ? 1 : 0, j = threadIdx.x - (m ? a.cols : 0);
+  int m = 0;
+#pragma unroll
+  for (int i = 1; i < MT; ++i) m += (int)threadIdx.x >= i * a.cols;
+  const int j = threadIdx.x - m * a.cols;
   const int jc = min(j, (PAIRED ? have >> 1 : have) - 1);
   float res = 0.f, blo = 0.f, bhi = 0.f, c = 1.f, s = 0.f;
   int64_t slot = -1;
@@ -253,7 +256,7 @@ __global__ __launch_bounds__(THREADS) void skinny_dot_kernel(const SKArgs a) {
     for (int i = 0; i < MT; ++i)
 #pragma unroll
       for (int p = 0; p < P; ++p)
-        xv[i][p] = *reinterpret_cast<const bf16x8*>(reinterpret_cast<const char*>(a.X + (i ? a.xs : 0)) + at[p]);
+        xv[i][p] = *reinterpret_cast<const bf16x8*>(reinterpret_cast<const char*>(a.X + i * a.xs) + at[p]);
     if (NORM)
 #pragma unroll
       for (int p = 0; p < P; ++p) nv[p] = *reinterpret_cast<const bf16x8*>(reinterpret_cast<const char*>(a.nw) + at[p]);
@@ -712,8 +715,10 @@ int sk_dot_rows(const SKArgs& a, dim3 grid, hipStream_t st) {
 
 template <int MT, int RB, bool NORM, int MODE, bool PARTS = false>
 int sk_dot(const SKArgs& a, dim3 grid, hipStream_t st) {
-  if (a.K <= P * 512) return sk_dot_rows<MT, RB, 1, NORM, MODE, PARTS>(a, grid, st);
-  if (a.K <= 2 * P * 512) return sk_dot_rows<MT, RB, 2, NORM, MODE, PARTS>(a, grid, st);
+  if constexpr (MT <= 2) {
+    if (a.K <= P * 512) return sk_dot_rows<MT, RB, 1, NORM, MODE, PARTS>(a, grid, st);
+    if (a.K <= 2 * P * 512) return sk_dot_rows<MT, RB, 2, NORM, MODE, PARTS>(a, grid, st);
+  }
   if (a.K <= 4 * P * 512) return sk_dot_rows<MT, RB, 4, NORM, MODE, PARTS>(a, grid, st);
   if (a.K <= WAVES * P * 512) return sk_dot_rows<MT, RB, WAVES, NORM, MODE, PARTS>(a, grid, st);
   if constexpr (!NORM) return sk_dot_as<MT, RB, WAVES, NORM, MODE, PARTS, true>(a, grid, st);
@@ -753,8 +758,21 @@ extern "C" int areal_skinny_residual(const void* X, int64_t xs, const void* W, c
   const int blocks = (N + a.cols - 1) / a.cols;
   if (M == 1) return sk_dot<1, 3, false, SK_RES>(a, dim3(blocks), st);
   if (M == 2) return sk_dot<2, 3, false, SK_RES>(a, dim3(blocks), st);
-  if (K <= 64 * WAVES * 6) return sk_mfma<1, 6, false, false, SK_RES>(a, blocks, st);
-  return sk_mfma<1, 6, true, false, SK_RES>(a, blocks, st);
+  // Three rows and more: a tile of 16 weight rows holds only cols of its own, so with few of them the dot products are faster where rows
+  // are long (us, 3 / 4 / 6 / 8 rows, matrix cores and dot products: 1536 columns 8960 deep, 6 a workgroup, 12.3 / 12.5 / 12.9 / 13.5 and
+  // 8.5 / 8.7 / 9.8 / 10.4, 4096 deep 6.8 / 6.9 / 7.0 / 7.2 and 5.3 / 5.4 / 6.1 / 6.6, 2048 deep 4.8 / 4.7 / 5.0 / 5.1 and 4.1 / 4.2 / 4.9 / 5.2;
+  // 2048 columns 6144 deep, 8 each, 10.4 / 10.6 / 9.4 / 9.8 and 7.8 / 8.0 / 9.2 / 9.4; 3584 x 3584, 14 each, 8.0 / 8.1 / 8.7 / 8.3 and 8.4 /
+  // 8.6 / 10.2 / 10.7), and fewer of their values are rounded the other way than 64-bit sums (8960 deep 1e-4 and 2e-4).
+  const bool deep = K > 64 * WAVES * 6;
+  if (a.cols <= 8 && deep) switch (M) {
+    case 3: return sk_dot<3, 3, false, SK_RES>(a, dim3(blocks), st);
+    case 4: return sk_dot<4, 3, false, SK_RES>(a, dim3(blocks), st);
+    case 5: return sk_dot<5, 3, false, SK_RES>(a, dim3(blocks), st);
+    case 6: return sk_dot<6, 3, false, SK_RES>(a, dim3(blocks), st);
+    case 7: return sk_dot<7, 3, false, SK_RES>(a, dim3(blocks), st);
+    case 8: return sk_dot<8, 3, false, SK_RES>(a, dim3(blocks), st);
+  }
+  return deep ? sk_mfma<1, 6, true, false, SK_RES>(a, blocks, st) : sk_mfma<1, 6, false, false, SK_RES>(a, blocks, st);
 }
 
 // The same of one row of the decode attention's output, K = Hq heads of D (64, 128 or 256), that it has left as rows[0].y > 1 partial

@@ -89,6 +89,13 @@ def test_linear_residual_of_every_split_of_the_waves(M, N, K):
     test_linear_residual(M, N, K)
 
 
+@pytest.mark.parametrize("M", [3, 4, 5, 6, 7, 8])
+@pytest.mark.parametrize("N,K", [(2048, 3136), (2049, 3136), (1025, 6144), (9, 6208), (2048, 12288), (7, 12352), (896, 3072)])
+def test_linear_residual_of_more_rows_by_dot_products(M, N, K):
+    """Either side of the columns and depths that they are taken for; four and eight waves along K and more than one turn of them."""
+    test_linear_residual(M, N, K)
+
+
 @pytest.mark.parametrize("M", [1, 2])
 @pytest.mark.parametrize("Hq,Hkv,D,K", [(40, 8, 128, 2048), (2, 1, 128, 8192), (6, 2, 48, 3136), (2, 2, 16, 12288)])
 def test_norm_qkv_rope_of_every_split_of_the_waves(M, Hq, Hkv, D, K):
