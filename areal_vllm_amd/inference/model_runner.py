@@ -725,22 +725,25 @@ class ModelRunner:
             x, residual = finish(slab, residual, nw)
         return x
 
-    # Rows up to which the five-launch layer is faster than split-K GEMMs with row kernels, for hidden sizes up to 1536 and
-    # above. 28 layers of Qwen2-1.5B at 1 / 2 / 4 / 6 / 8 rows: 1.17 / 1.24 / 1.36 / 1.45 / 1.50 ms a step against 1.44 / 1.44 /
-    # 1.47 / 1.58 / 1.48; 12 layers of Llama-3-8B at 1 / 2 / 4: 1.47 / 1.55 / 1.65 against 1.66 / 1.66 / 1.58 (a row's weights
-    # no longer fit the registers at once, and the matrix-core form does not load ahead there). Other sizes, hidden 896 (24 layers),
-    # 1 / 2 / 3 / 6 rows: 0.70 / 0.76 / 0.79 / 0.83 against 0.94 / 0.97 / 0.97 / 0.99; 2048 (10 layers) 0.58 / 0.61 / 0.67 / 0.71
-    # against 0.67 / 0.68 / 0.68 / 0.69; 1 / 2 rows of 3072 0.52 / 0.55 against 0.62 / 0.63, 3584 0.70 / 0.74 against 0.74 / 0.73, 5120
-    # (13824 inner) 0.70 / 0.74 against 0.76 / 0.73, 8192 0.75 / 0.77 against 0.89 / 0.87.
-    SKINNY_MAX_ROWS, SKINNY_MAX_ROWS_WIDE = 6, 2
+    # Rows up to which the five-launch layer is faster than split-K GEMMs with row kernels: hidden sizes up to 1536, of those the ones whose
+    # MLP is wider than 4096 (gate and up then go over the chip in one uneven round of wide workgroups), and above 1536. 28 layers of
+    # Qwen2-1.5B (1536, 8960 inner) at 2 / 3 / 4 / 5 / 6 / 8 rows: 1.17 / 1.26 / 1.27 / 1.34 / 1.38 / 1.43 ms a step against 1.24 / 1.26 / 1.29 /
+    # 1.30 / 1.31 / 1.35; 24 layers of 1536 at 6 rows, 1024 / 2048 / 4096 / 6144 inner: 0.86 / 0.89 / 0.98 / 1.06 against 0.93 / 0.98 / 1.02 / 1.04; of
+    # 896 at 4 / 5 / 6 rows, 1024 inner 0.66 / 0.68 / 0.71 against 0.77 / 0.76 / 0.78, 4864 0.79 / 0.81 / 0.83 against 0.82 / 0.82 / 0.82.
+    # 12 layers of Llama-3-8B at 1 / 2 / 4: 1.47 / 1.55 / 1.65 against 1.66 / 1.66 / 1.58 (a row's weights no longer fit the registers at once).
+    # 2048 (10 layers) at 1 / 2 / 3 / 6: 0.58 / 0.61 / 0.67 / 0.71 against 0.67 / 0.68 / 0.68 / 0.69; 1 / 2 rows of 3072 0.52 / 0.55 against 0.62 /
+    # 0.63, 3584 0.70 / 0.74 against 0.74 / 0.73, 5120 (13824 inner) 0.70 / 0.74 against 0.76 / 0.73, 8192 0.75 / 0.77 against 0.89 / 0.87.
+    SKINNY_MAX_ROWS, SKINNY_MAX_ROWS_LONG, SKINNY_MAX_ROWS_WIDE = 6, 4, 2
 
     def _skinny(self, rows: int) -> bool:
         """Whether a decode step of so many rows runs the five-launch layer of ``ops/decode_skinny.py``."""
         from ..ops import decode_skinny as sk
 
         cfg = self.cfg
-        return (rows <= (self.SKINNY_MAX_ROWS if cfg.hidden_size <= 1536 else self.SKINNY_MAX_ROWS_WIDE) and self.fused_decode and not self.tp_comm and not cfg.qk_norm
-                and cfg.n_experts == 0 and self.dtype == torch.bfloat16
+        most = self.SKINNY_MAX_ROWS if cfg.hidden_size <= 1536 else self.SKINNY_MAX_ROWS_WIDE
+        if cfg.intermediate_size > 4096:
+            most = min(most, self.SKINNY_MAX_ROWS_LONG)
+        return (rows <= most and self.fused_decode and not self.tp_comm and not cfg.qk_norm and cfg.n_experts == 0 and self.dtype == torch.bfloat16
                 and sk.serves(cfg.hidden_size, cfg.intermediate_size, self.hq * cfg.head_dim, cfg.head_dim))
 
     def _decode_layers_skinny(self, st: Dict[str, torch.Tensor], h: torch.Tensor, rope_pos: torch.Tensor):
