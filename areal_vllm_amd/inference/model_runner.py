@@ -810,7 +810,7 @@ class ModelRunner:
                           st["block_tables"])
         for s in range(self.decode_steps):
             if st["items"] is not None:
-                st["items"].fill_(st["context_lens"])
+                st["items"].fill_(st["context_lens"], st["block_tables"])
             h = self._embed(st["input_ids"], st["positions"])
             rope_pos = st["positions"] if self.cfg.pos_embed == "rope" else st["zero_pos"]
             if self.is_vl:  # generated tokens of a request with images sit `delta` away from their index

@@ -522,12 +522,16 @@ class DecodeItems:
         self.part_ml = torch.empty(self.n_items, n_q_heads, 2, dtype=torch.float32, device=device)
         self.arrived = torch.zeros(batch, n_kv_heads, dtype=torch.int32, device=device)
 
-    def fill_(self, context_lens: torch.Tensor) -> "DecodeItems":
-        """Lay the items out for these context lengths; every layer of the step then uses them."""
+    def fill_(self, context_lens: torch.Tensor, block_tables: Optional[torch.Tensor] = None) -> "DecodeItems":
+        """Lay the items out for these context lengths; every layer of the step then uses them. With the rows' block tables, pages that
+        no other row shares are read past the caches (results are the same)."""
         if L.use_hip(context_lens):
             assert context_lens.dtype == torch.int32 and context_lens.is_contiguous() and context_lens.numel() == self.batch
+            assert block_tables is None or (block_tables.dtype == torch.int32 and block_tables.is_contiguous()
+                                            and block_tables.shape[0] == self.batch)
             L.check(L.lib().areal_paged_decode_items(L.ptr(context_lens), L.ptr(self.items), L.ptr(self.rows), L.c_int(self.batch),
                                                      L.c_int(self.target), L.c_int(self.n_items), L.c_int(int(self.finer)),
+                                                     L.ptr(block_tables), L.c_int(0 if block_tables is None else block_tables.shape[1]),
                                                      L.stream_ptr()),
                     "paged_decode_items")
         return self

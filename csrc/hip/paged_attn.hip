@@ -325,12 +325,12 @@ extern "C" int areal_paged_decode_window(const void* q, const void* kcache, cons
 //   fp8: 48 x 6000-24000 101 -> 77 (3.6 -> 4.7 TB/s), 24 x 200-4096 17.7 -> 11.0, 128 x 1000 21.4 -> 16.1.
 // More, smaller items cost more in combining than they even out (24 x 200-4096: 15.4 us with 256 items, 18.2 with 384;
 // 320 x 128-1152, every row divided by its length over the item's rounded up: 42 with 256, 46 with 768-1024).
-// The list depends on the context lengths alone: one launch per decode step serves every layer.
+// The list depends on the context lengths alone (`stream` on the block tables): one launch per decode step serves every layer.
 //
 // Item: {row, first page, end page, first partial result of the row, number of the row's items, this item's partial
-// result} in 8 ints; count 0: none. Longest first: a workgroup that ends early takes the next item, and the short ones
-// fill the gaps at the end.
-struct DecodeItem { int b, p_beg, p_end, base, n, part, pad0, pad1; };
+// result, whether its pages are read past the caches} in 8 ints; count 0: none. Longest first: a workgroup that ends early takes the
+// next item, and the short ones fill the gaps at the end.
+struct DecodeItem { int b, p_beg, p_end, base, n, part, stream, pad; };
 
 // Pages per item of a row of np pages: the row evenly divided into items of about `even` pages (half as much again at
 // most: splitting a row that is a little longer than an item costs more than it evens out), a multiple of STEP; and so
@@ -358,10 +358,21 @@ DEVINL int pages_per_item(int np, int even) {
 // with `finer` 2 target + B. Pages per item: the whole batch over `target` items.
 __global__ __launch_bounds__(1024) void paged_decode_items_kernel(const int* __restrict__ context_lens,
                                                                   DecodeItem* __restrict__ items, int2* __restrict__ rows,
-                                                                  int B, int target, int n_items, int finer) {
+                                                                  int B, int target, int n_items, int finer,
+                                                                  const int* __restrict__ block_tables, int max_pages) {
   constexpr int NB = 64;  // size classes of the sort
+  // Rows with the same first page (requests of one prompt), for the items' `stream`: the first row that came with it, and the last of
+  // the others. 1024 rows at most; a row that finds no place in 8 counts as alone.
+  constexpr int SLOTS = 2048, PROBES = 8;
+  __shared__ int first_page[SLOTS], leader[SLOTS], other[SLOTS];
+  const bool shared_pages = block_tables && B > 1 && B <= 1024;
   __shared__ int red[16], red_n[16], hist[NB];
   const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
+  int own_first = 0, own_slot = -1;
+  if (shared_pages) {
+    own_first = block_tables[(size_t)min(t, B - 1) * max_pages];
+    for (int i = t; i < SLOTS; i += 1024) { first_page[i] = -1; other[i] = -1; }
+  }
   int pages = 0;
   for (int b = t; b < B; b += 1024) pages += (max(context_lens[b], 0) + PAGE - 1) / PAGE;
 #pragma unroll
@@ -372,6 +383,16 @@ __global__ __launch_bounds__(1024) void paged_decode_items_kernel(const int* __r
   int total = 0;
 #pragma unroll
   for (int w = 0; w < 16; ++w) total += red[w];
+  if (shared_pages && t < B) {
+    unsigned at = (unsigned)own_first * 2654435761u >> 21;
+    for (int i = 0; i < PROBES && own_slot < 0; ++i, at = (at + 1) & (SLOTS - 1)) {
+      const int had = atomicCAS(&first_page[at], -1, own_first);
+      if (had == -1) leader[at] = t;
+      else if (had == own_first) atomicMax(&other[at], t);
+      else continue;
+      own_slot = (int)at;
+    }
+  }
   int even = max(STEP, (total + target - 1) / target);
   if (finer && even >= FINER_EVEN) {
     int longest = 0, count = 0;
@@ -439,10 +460,14 @@ __global__ __launch_bounds__(1024) void paged_decode_items_kernel(const int* __r
     }
     const int base = before + incl - n;
     if (n > 0 && rows) rows[b] = base + n <= n_items ? make_int2(base, n) : make_int2(0, 0);
+    int mate = -1;  // (behind the barriers that follow the rows' entries above)
+    if (own_slot >= 0) mate = leader[own_slot] == t ? other[own_slot] : leader[own_slot];
     for (int i = 0; i < n; ++i) {
-      const int lo = i * per, hi = min(np, lo + per);
+      const int lo = i * per, hi = min(np, lo + per), mid = min((lo + hi) / 2, max_pages - 1);
+      int stream = B == 1 || shared_pages;
+      if (mate >= 0) stream = block_tables[(size_t)b * max_pages + mid] != block_tables[(size_t)mate * max_pages + mid];
       const int place = atomicAdd(&hist[size_class(hi - lo)], 1);
-      if (place < n_items && base + n <= n_items) items[place] = DecodeItem{b, lo, hi, base, n, base + i, 0, 0};
+      if (place < n_items && base + n <= n_items) items[place] = DecodeItem{b, lo, hi, base, n, base + i, stream, 0};
     }
   }
   for (int i = at + t; i < n_items; i += 1024) items[i] = DecodeItem{0, 0, 0, 0, 0, 0, 0, 0};
@@ -468,6 +493,13 @@ DEVINL float ld_agent(const float* p) {
 // 40.8 -> 38.8, 384 x 8-64 8.2 -> 7.5, fp8 48 x 6000-24000 81.0 -> 81.8, 128 x 1000 15.3 -> 14.9; 14 on 2 of 64, 300 x 100-1200 23.8 ->
 // 22.6; 8 on 1 of 256, 64 x 1000 22.1 -> 21.4, fp8 32 x 8000 34.9 -> 33.4, 1 x 640 12.5 -> 12.8: 4.8 to 5.6 of the 6 TB/s that the
 // chip reads, less where a launch is over in 10 us.
+// Pages are asked for in whole 128-byte lines, and where no other row reads them too, past the caches (nontemporal): lines alone gain nothing,
+// the second alone 0 to 8 %, both 7 to 12: 320 x 128-1152 44.0 -> 39.6, 256 x 640 33.1 -> 29.9 (5.6 TB/s), 64 x 4000 52.0 -> 47.0, 24 x 200-4096
+// 16.6 -> 15.3, 16 x 12000 40.9 -> 37.2, fp8 48 x 6000-24000 74.0 -> 67.0, 128 x 1000 15.7 -> 14.2; 300 x 100-1200 14 on 2 of 64 22.8 -> 20.4; 64 x 1000 8
+// on 1 of 256 21.5 -> 20.2, fp8 32 x 8000 33.5 -> 30.7; 1 x 640 7.3 -> 7.0, 320 x 8-64 8.1. Pages of a common prompt come out of the caches for
+// all rows but the first; past them, 320 x 1100-1152 with 1024 tokens common to 16 rows each took 51.4 instead of 44.0, 64 x 4150 with 4096
+// common to 8 rows 40.6 instead of 31.2. The page loop is there twice; a wave's number is a scalar, so that both fit the registers. What
+// stands ahead of the first request is on every launch's path: without a division and with the item read at once, 0.2 us less.
 // LDS holds the G real query rows only. Two workgroups of 8 waves a CU (128 registers a lane; heads of 64 three, of 256 one
 // of 4 waves): the register file sets that, a GQA group of 6 heads of 128 takes 26 KB of LDS.
 template <int D, bool FP8, int NW>
@@ -475,20 +507,24 @@ __global__ __launch_bounds__(64 * NW, (D > 128 ? 1 : 4)) void paged_decode_walk_
     const bf16_t* __restrict__ q, const void* __restrict__ kcache, const void* __restrict__ vcache,
     const int* __restrict__ block_tables, const int* __restrict__ context_lens, const DecodeItem* __restrict__ items,
     bf16_t* __restrict__ out, float* __restrict__ part_o, float* __restrict__ part_ml, int* __restrict__ arrived, int Hq,
-    int Hkv, int max_pages, float scale_log2, int q_stride) {
+    int Hkv, int G, unsigned hkv_inv, int max_pages, float scale_log2, int q_stride) {
   constexpr int KS = D / 32, DB = D / 16, DP = D + 4;
   extern __shared__ __attribute__((aligned(16))) float smem[];
   __shared__ int last;
-  const DecodeItem it = items[blockIdx.x / Hkv];
-  if (it.n == 0) return;
-  const int b = it.b, h = blockIdx.x % Hkv;
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  const int G = Hq / Hkv;
+  const int item = quotient(blockIdx.x, Hkv, hkv_inv);
+  const DecodeItem it = items[item];
+  // the whole item and the arguments at once, not each where it is first used: every wait is a trip to the scalar cache or past it
+  int count = it.n;
+  asm("" : "+s"(count) : "s"(it.b), "s"(it.p_beg), "s"(it.p_end), "s"(it.base), "s"(it.part), "s"(it.stream), "s"(q), "s"(kcache), "s"(vcache),
+      "s"(block_tables), "s"(context_lens), "s"(G), "s"(q_stride));
+  if (count == 0) return;
+  const int b = it.b, h = blockIdx.x - item * Hkv;
+  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, c = lane >> 4;
   const int* bt = block_tables + (size_t)b * max_pages;
   // this wave's pages: p_beg + wid + NW i; 64 page ids are fetched at once, one a lane
   const int mine = it.p_end - it.p_beg > wid ? (it.p_end - it.p_beg - wid + NW - 1) / NW : 0;
-  int ids = lane < mine ? bt[it.p_beg + wid + NW * lane] : 0;
+  int ids = 0;
   const int ctx = context_lens[b];
   // Q is the B operand of S^T = K.Q^T and waits in the LDS that the wave's result goes to at the end: its registers hold the next
   // page instead. fp8: a lane's 16 loaded bytes of K are the operand of two k-steps, so lane c takes Q[64 (ks / 2) + 16 c +
@@ -496,14 +532,15 @@ __global__ __launch_bounds__(64 * NW, (D > 128 ? 1 : 4)) void paged_decode_walk_
   constexpr int QP = D + 8;  // row pitch: 16-byte reads of 16 rows on different banks
   bf16_t* qs = reinterpret_cast<bf16_t*>(smem + wid * G * DP);
   if (mine > 0) {
-    const int chunks = G * (D / 8);
+    ids = bt[it.p_beg + wid + NW * min(lane, mine - 1)];
+    const unsigned chunks = G * (D / 8);
     const bf16_t* qp = q + (size_t)b * q_stride + (size_t)h * G * D;
     bf16x8 qv[D / 32];
 #pragma unroll
-    for (int j = 0; j < D / 32; ++j) qv[j] = ld8(qp + min(lane + 64 * j, chunks - 1) * 8);
+    for (int j = 0; j < D / 32; ++j) qv[j] = ld8(qp + min(lane + 64u * j, chunks - 1) * 8);
 #pragma unroll
     for (int j = 0; j < D / 32; ++j) {
-      const int i = min(lane + 64 * j, chunks - 1);  // (the last piece more than once)
+      const unsigned i = min(lane + 64u * j, chunks - 1);  // (the last piece more than once)
       st8(qs + i / (D / 8) * QP + i % (D / 8) * 8, qv[j]);
     }
   }
@@ -513,7 +550,6 @@ __global__ __launch_bounds__(64 * NW, (D > 128 ? 1 : 4)) void paged_decode_walk_
 #pragma unroll
   for (int i = 0; i < DB; ++i) o[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
   float m = -INFINITY, l = 0.f;  // running max (log2 units) is shared by the 4 lanes of a q
-  const int key_a = 8 * (col >> 2) + (col & 3);  // row `col` of tile a; tile b: 4 rows further
 
   // Element offset of the K / V block of this wave's page i. The wait belongs to the fetch: behind the branch it would hold
   // every page's loads.
@@ -532,23 +568,53 @@ __global__ __launch_bounds__(64 * NW, (D > 128 ? 1 : 4)) void paged_decode_walk_
   vraw rv[DB];
   // a page's base is the same for all lanes, a lane's offset is the same for all pages: scalar base + 32-bit offset
   constexpr int EB = FP8 ? 1 : 2;
-  const unsigned k_off = key_a * D * EB + c * 16, v_off = (col * PAGE + c * 8) * EB;
-  auto load_k = [&](size_t kp) __attribute__((always_inline)) {
+  // Row r of score tile a is key 8 (r / 4) + r % 4, of tile b the key 4 further. A request asks for whole 128-byte lines: of eight rows, lanes
+  // with col >= 8 the second 64 bytes of what an operand would take of sixteen, and `sort` puts the halves of two requests in order.
+  constexpr bool LINES = KL > 1;
+  const int krow = LINES ? col & 7 : col;
+  const unsigned k_off = (8 * (krow >> 2) + (krow & 3)) * D * EB + (LINES ? (col >> 3) * 64 : 0) + c * 16, v_off = (col * PAGE + c * 8) * EB;
+  auto load_k = [&](size_t kp, auto stream_c) __attribute__((always_inline)) {
+    constexpr bool STREAM = decltype(stream_c)::value;
     const char* base = reinterpret_cast<const char*>(kcache) + kp * EB;
 #pragma unroll
     for (int k2 = 0; k2 < KL; ++k2) {
-      ra[k2] = *reinterpret_cast<const kraw*>(base + k_off + k2 * 64);
-      rb[k2] = *reinterpret_cast<const kraw*>(base + k_off + 4 * D * EB + k2 * 64);
+      const char* rows = base + (k2 & 1) * 16 * D * EB;  // rows 8 to 15 of the tiles
+      const kraw* pa = reinterpret_cast<const kraw*>(rows + k_off + (k2 >> 1) * 128);
+      const kraw* pb = reinterpret_cast<const kraw*>(rows + k_off + 4 * D * EB + (k2 >> 1) * 128);
+      ra[k2] = STREAM ? __builtin_nontemporal_load(pa) : *pa;
+      rb[k2] = STREAM ? __builtin_nontemporal_load(pb) : *pb;
     }
   };
-  auto load_v = [&](size_t kp) __attribute__((always_inline)) {
+  // a: the halves of rows 0 to 7 (lanes below and from col 8), b: of rows 8 to 15 -> the first halves of all rows, the second halves
+  auto sort = [&](kraw& a, kraw& b) __attribute__((always_inline)) {
+    u32x4 x = __builtin_bit_cast(u32x4, a), y = __builtin_bit_cast(u32x4, b);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      constexpr int ROTATE_8 = 0x128;  // within 16 lanes; the last arguments: of which groups of four lanes
+      const unsigned first = __builtin_amdgcn_update_dpp(x[i], y[i], ROTATE_8, 0xF, 0xC, false);
+      y[i] = __builtin_amdgcn_update_dpp(y[i], x[i], ROTATE_8, 0xF, 0x3, false);
+      x[i] = first;
+    }
+    a = __builtin_bit_cast(kraw, x);
+    b = __builtin_bit_cast(kraw, y);
+  };
+  auto load_v = [&](size_t kp, auto stream_c) __attribute__((always_inline)) {
+    constexpr bool STREAM = decltype(stream_c)::value;
     const char* base = reinterpret_cast<const char*>(vcache) + kp * EB;
 #pragma unroll
-    for (int j = 0; j < DB; ++j) rv[j] = *reinterpret_cast<const vraw*>(base + (j * 16 * PAGE * EB & ~4095) + v_off + (j * 16 * PAGE * EB & 4095));
+    for (int j = 0; j < DB; ++j) {
+      const vraw* p = reinterpret_cast<const vraw*>(base + (j * 16 * PAGE * EB & ~4095) + v_off + (j * 16 * PAGE * EB & 4095));
+      rv[j] = STREAM ? __builtin_nontemporal_load(p) : *p;
+    }
   };
-  auto page_step = [&](int p, size_t next, auto more_c) __attribute__((always_inline)) {
+  auto page_step = [&](int p, size_t next, auto more_c, auto stream_c) __attribute__((always_inline)) {
     constexpr bool MORE = decltype(more_c)::value;  // another page follows
     f32x4 sa = {0.f, 0.f, 0.f, 0.f}, sb = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k2 = 0; k2 + 1 < KL; k2 += 2) {
+      sort(ra[k2], ra[k2 + 1]);
+      sort(rb[k2], rb[k2 + 1]);
+    }
     if constexpr (FP8) {
 #pragma unroll
       for (int k2 = 0; k2 < KL; ++k2) {
@@ -566,7 +632,7 @@ __global__ __launch_bounds__(64 * NW, (D > 128 ? 1 : 4)) void paged_decode_walk_
     }
     if (MORE) {
       __builtin_amdgcn_sched_barrier(0);
-      load_k(next);
+      load_k(next, stream_c);
       __builtin_amdgcn_sched_barrier(0);
     }
     // lane (q = col, c): sa[r] = S[key 8c + r], sb[r] = S[key 8c + 4 + r]
@@ -606,21 +672,25 @@ __global__ __launch_bounds__(64 * NW, (D > 128 ? 1 : 4)) void paged_decode_walk_
     }
     if (MORE) {
       __builtin_amdgcn_sched_barrier(0);
-      load_v(next);
+      load_v(next, stream_c);
       __builtin_amdgcn_sched_barrier(0);
     }
   };
-  if (mine > 0) {
+  auto walk = [&](auto stream_c) __attribute__((always_inline)) {
     size_t kp = block_of(0);
-    load_k(kp);
-    load_v(kp);
+    load_k(kp, stream_c);
+    load_v(kp, stream_c);
     __builtin_amdgcn_sched_barrier(0);
     const int p0 = it.p_beg + wid;
     for (int i = 0; i + 1 < mine; ++i) {
       kp = block_of(i + 1);
-      page_step(p0 + NW * i, kp, std::true_type{});
+      page_step(p0 + NW * i, kp, std::true_type{}, stream_c);
     }
-    page_step(p0 + NW * (mine - 1), 0, std::false_type{});
+    page_step(p0 + NW * (mine - 1), 0, std::false_type{}, stream_c);
+  };
+  if (mine > 0) {
+    if (__builtin_expect(it.stream != 0, 1)) walk(std::true_type{});
+    else walk(std::false_type{});
   }
   l = sum_xor16(l);  // l is a per-lane partial over this lane's keys: sum the 4 lanes that share a q
   l = sum_xor32(l);
@@ -725,11 +795,12 @@ __global__ __launch_bounds__(64 * NW, (D > 128 ? 1 : 4)) void paged_decode_walk_
 }
 
 // Items of the batch's decode attention; rows [B] (or null): first partial result and number of a row's items; `items`: n_items x 8 ints, at least min(target + B, B x most items of a row); with finer 2 target + B.
+// block_tables [B, max_pages] (or null): pages that no other row reads are then read past the caches.
 extern "C" int areal_paged_decode_items(const int* context_lens, void* items, void* rows, int B, int target, int n_items, int finer,
-                                        hipStream_t st) {
-  if (B < 1 || target < 1 || n_items < B) return -1;
+                                        const int* block_tables, int max_pages, hipStream_t st) {
+  if (B < 1 || target < 1 || n_items < B || (block_tables && max_pages < 1)) return -1;
   hipLaunchKernelGGL(paged_decode_items_kernel, dim3(1), dim3(1024), 0, st, context_lens, (DecodeItem*)items, (int2*)rows, B,
-                     target, n_items, finer);
+                     target, n_items, finer, block_tables, max_pages);
   return (int)hipGetLastError();
 }
 
@@ -750,7 +821,7 @@ static int launch_paged_decode_walk(const void* q, const void* kcache, const voi
   }
   hipLaunchKernelGGL((paged_decode_walk_kernel<D, FP8, NW>), dim3(n_items * Hkv), dim3(64 * NW), lds, st, (const bf16_t*)q, kcache,
                      vcache, block_tables, context_lens, (const DecodeItem*)items, (bf16_t*)out, part_o, part_ml, arrived,
-                     Hq, Hkv, max_pages, scale_log2, q_stride);
+                     Hq, Hkv, Hq / Hkv, reciprocal((long)n_items * Hkv, Hkv), max_pages, scale_log2, q_stride);
   return (int)hipGetLastError();
 }
 

@@ -91,3 +91,28 @@ def test_runner_chooses_items_by_values_a_key_head(Hq, Hkv, head_dim, kv, rows, 
     got = ops.paged_attention_decode(*d, nsplit=st["nsplit"], workspace=st["ws"], items=st["items"]).float().cpu()
     ref = A.paged_decode_ref(q[:, :Hq], kc, vc, bt, cl, 1 / math.sqrt(head_dim)).float()
     assert (got - ref).abs().max() < 2e-2
+
+
+@pytest.mark.parametrize("rows,group,common", [(1, 1, 0), (2, 2, 40), (7, 3, 33), (320, 16, 20), (1024, 1024, 8), (1025, 5, 8)])
+@pytest.mark.parametrize("D,fp8", [(128, False), (128, True), (64, False), (64, True), (256, False), (256, True)])
+def test_pages_that_no_other_row_reads_go_past_the_caches(rows, group, common, D, fp8):
+    """Which items are marked: none of those that lie in pages common to a group, all of those behind them (and all results the same)."""
+    g = torch.Generator().manual_seed(rows + D)
+    ctx = [int(x) for x in torch.randint(32 * common + 1, 32 * common + 700, (rows,), generator=g)]
+    q, kc, vc, bt, cl = _setup(ctx, 4, 1, D, fp8, 4)
+    order = torch.randperm(rows, generator=g)  # rows of a group are not neighbours
+    for i in range(rows):
+        bt[order[i], :common] = bt[order[i // group * group], :common]
+    d = [t.to(DEV) for t in (q, kc, vc, bt, cl)]
+    plain = ops.DecodeItems(rows, 4, 1, D, torch.device(DEV)).fill_(d[4])
+    marked = ops.DecodeItems(rows, 4, 1, D, torch.device(DEV)).fill_(d[4], d[3])
+    size = {int(r): min(group, rows - i // group * group) for i, r in enumerate(order)}  # rows of its group
+    table = {(b, lo): (hi, stream) for b, lo, hi, _, n, _, stream, _ in marked.items.tolist() if n}
+    assert len(table) == int((plain.items[:, 4] > 0).sum())
+    for (b, lo), (hi, stream) in table.items():
+        alone = rows == 1 or (rows <= 1024 and (size[b] == 1 or (lo + hi) // 2 >= common))
+        assert stream == int(alone), (b, lo, hi, stream)
+    outs = [ops.paged_attention_decode(d[0][:, :4], *d[1:], q_row_stride=5 * D, items=i) for i in (plain, marked)]
+    assert torch.equal(*outs)
+    ref = A.paged_decode_ref(q[:, :4], kc, vc, bt, cl, 1 / math.sqrt(D)).float()
+    assert (outs[0].float().cpu() - ref).abs().max() < 2e-2  # as above
