@@ -171,9 +171,9 @@ struct Philox {
     mulhilo(0xD2511F53u, c[0], h0, l0);
     mulhilo(0xCD9E8D57u, c[2], h1, l1);
     u32x4 r;
-    r[0] = h1 ^ c[1] ^ k0;
+    r[0] = __builtin_amdgcn_bitop3_b32(h1, c[1], k0, 0x96);  // the three-way exclusive or, which the compiler makes two of
     r[1] = l1;
-    r[2] = h0 ^ c[3] ^ k1;
+    r[2] = __builtin_amdgcn_bitop3_b32(h0, c[3], k1, 0x96);
     r[3] = l0;
     return r;
   }

@@ -1,4 +1,5 @@
 """Filtered sampling with the rows split over workgroups against one workgroup a row: the same tokens and counts."""
+import math
 import sys
 
 import pytest
@@ -68,3 +69,16 @@ def test_the_rule(B, V, n, k, p, monkeypatch):
     got.append(ops.sample(logits, t, kk, pp, 5, torch.zeros(1, dtype=torch.int64, device=DEV)))
     assert torch.equal(got[0][0], got[1][0])
     assert torch.allclose(got[0][1], got[1][1], atol=1e-4, rtol=1e-5)  # as above
+
+
+@pytest.mark.parametrize("B,V", [(1, 8), (3, 517), (64, 4097), (65, 40000), (1100, 300)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_unfiltered_rows_whose_slices_are_mostly_masked(B, V, dtype):
+    """Slices of one row without a finite entry, and rows with a single one (its log-prob is zero) in any of them."""
+    g = torch.Generator(device="cuda").manual_seed(B)
+    logits = torch.full((B, V), -math.inf, dtype=dtype, device="cuda")
+    at = torch.randint(V, (B,), generator=g, device="cuda")
+    logits[torch.arange(B, device="cuda"), at] = 3.0
+    step = torch.zeros(1, dtype=torch.int64, device="cuda")
+    tok, lp = ops.sample(logits, torch.full((B,), 0.9, device="cuda"), None, None, seed=5, step=step)
+    assert torch.equal(tok, at) and float(lp.abs().max()) < 1e-6 and step.item() == 1
