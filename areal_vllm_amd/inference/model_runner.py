@@ -779,15 +779,17 @@ class ModelRunner:
                 and x.stride(1) == 1)
 
     def _lm_head(self, x: torch.Tensor, fp32: bool = False) -> torch.Tensor:
-        """Final-normed hidden states [Bp, H] -> logits [Bp, V]. Up to ~100 rows the projection is a pure weight
-        stream (467 MB for Qwen2's vocabulary) and the decode GEMM on 64-row x 128-column tiles reads it at
-        5.4-6.1 TB/s (77 / 86 / 99 us at 8 / 32 / 64 rows against 163 / 106 / 114 us for the library); from 128 rows
-        on the two are level and the library stays."""
+        """Final-normed hidden states [Bp, H] -> logits [Bp, V]. Up to 64 rows the projection is a pure weight stream (467 MB for
+        Qwen2's vocabulary), which the decode GEMM reads on 64-row x 128-column tiles at 5 to 6 TB/s (76 / 85 / 97 us at 8 / 32 / 64 rows against
+        162 / 104 / 112 us for the library); to 160 rows it goes over column ranges that hold all rows (188 us in two of those
+        row blocks, 120 in the library and 103 at 96 rows); above, the library is ahead."""
         w = self.model.head_weight
-        if not self._lm_head_own(x):
-            return F.linear(x, w)
         from ..ops import decode_gemm as dg
 
+        if not fp32 and dg.serves_wide(x, w):
+            return dg.dgemm_wide(x, w)
+        if not self._lm_head_own(x):
+            return F.linear(x, w)
         kw = dict(cfg=4, stages=3, loader_waves=4, nt=True)
         if not fp32:
             return dg.dgemm(x, w, epilogue=dg.EPI_BF16, ksplit=1, **kw)

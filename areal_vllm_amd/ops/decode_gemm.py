@@ -219,6 +219,40 @@ def dgemm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,
     return out
 
 
+# Up to 64 rows a decode step is as long on ``dgemm``'s tiles of 64 rows (14 layers of Qwen2-1.5B, 24 / 48 / 64 rows 0.76 / 0.89 / 0.94 ms in
+# both forms, 80 / 128 / 160 rows 1.14 / 1.21 / 1.38 with the tiles or the library and 1.06 / 1.18 / 1.36 with this); above 160 rows there are two row
+# blocks, and mostly the library is ahead.
+WIDE_MIN_COLUMNS, WIDE_MIN_ROWS, WIDE_MAX_ROWS = 16384, 65, 160
+
+
+def takes_wide(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether `dgemm_wide` takes the product: all rows in one block (GPU only)."""
+    M, K = x.shape
+    return (WIDE_MIN_ROWS <= M <= WIDE_MAX_ROWS and w.shape[0] % 4 == 0 and K % 64 == 0 and K > 0 and x.is_cuda
+            and x.dtype == w.dtype == torch.bfloat16 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and w.is_contiguous()
+            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
+
+
+def serves_wide(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether it is the fastest, too: enough columns for a range a CU."""
+    return w.shape[0] >= WIDE_MIN_COLUMNS and takes_wide(x, w)
+
+
+def dgemm_wide(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """``x [M, K] @ w[N, K].T`` -> bf16 [M, N] for a wide N (the LM head): one workgroup a CU that walks several column ranges."""
+    M, K = x.shape
+    N = w.shape[0]
+    if not L.use_hip(x):
+        return F.linear(x, w)
+    assert takes_wide(x, w)
+    rounds = -(-N // (160 * N_CU))  # ranges a workgroup; as narrow as that number allows, a multiple of 4
+    cols = (-(-N // (rounds * N_CU)) + 3) // 4 * 4
+    out = torch.empty(M, N, dtype=x.dtype, device=x.device)
+    L.check(L.lib().areal_dtile_rows(L.ptr(x), L.c_int64(x.stride(0)), L.ptr(w), L.ptr(out), L.c_int64(N), L.c_int(M), L.c_int(N),
+                                     L.c_int(K), L.c_int(cols), L.c_int(1), L.c_int(N_CU), L.c_int(1), L.stream_ptr()), "dgemm_wide")
+    return out
+
+
 @lru_cache(maxsize=4096)
 def swiglu_plan(M: int, F: int) -> Optional[Tuple[int, int]]:
     """-> (columns per workgroup, row blocks) of the balanced gate|up kernel for M rows and F gate columns, or None

@@ -303,6 +303,146 @@ __global__ __launch_bounds__(512) void dtile_kernel(const DTArgs a) {
   }
 }
 
+// Y [M, N] bf16 = X W^T for so many columns that every CU has several ranges (the LM head): as above, with a workgroup a CU that goes
+// from range to range. The loader waves ask for the next range's first stages while the last ones of the present are multiplied and its
+// outputs stored: with a workgroup a range the ring is empty at the start of each and drains at its end.
+// us, cold weights, decode_gemm.hip's tiles / library / this: 151936 columns, 1536 deep, 8 / 24 / 48 / 64 / 96 / 128 / 160 rows 76 / 81 / 92 / 97 /
+// 188 / 198 / -, 162 / 103 / 120 / 112 / 120 / 128 / 138, 73 / 79 / 89 / 94 / 103 / 111 / 119; 2048 deep 24 / 64 / 96 / 160 rows 108 / 124 / 238 /
+// -, 147 / 153 / 161 / 181, 103 / 118 / 128 / 150; 128256, 4096 deep 24 / 64 / 160 rows 163 / 181 / -, 195 / 210 / 249, 162 / 186 / 229; 32000,
+// 2048 deep 26 / 27 / -, 36 / 36 / 38, 25 / 27 / 38. Two row blocks: 224 rows of the first 152 (library) / 186, 320 rows 188 / 187. What
+// bounds it: the load path at 24 rows (6.0 TB/s of weights), with more rows the X that every range stages again.
+template <int RT, int CT>
+__global__ __launch_bounds__(512) void dtile_walk_kernel(const DTArgs a) {
+  constexpr int BM = 32 * RT, WR = 32 * CT, IPW = RT + CT;
+  constexpr int STAGE_BYTES = (BM + WR) * 128;
+  static_assert(4 * RT * CT + 8 * (RT + CT) <= 224, "accumulators and two sets of fragments in 256 registers");
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // tile p: row block p % mblocks of range p / mblocks. In every round an XCD has neighbouring tiles: row blocks of a range share its L2
+  const int nwg = gridDim.x, all = a.ntiles * a.mblocks;
+  const int first = (blockIdx.x & 7) * (nwg >> 3) + (blockIdx.x >> 3);  // (the grid is a multiple of 8)
+  const int nsteps = a.K >> 6, stages = a.stages;
+  const int mine = first < all ? (all - first + nwg - 1) / nwg : 0, total = mine * nsteps;
+
+  if (wave >= 4) {
+    const int lw = wave - 4;
+    const bf16_t* src[IPW];
+    int tile = first - nwg, step = nsteps, k = 0;
+    auto issue = [&](int buf) {
+      if (step == nsteps) {
+        tile += nwg;
+        step = 0;
+        const int range = quotient(tile, a.mblocks, a.inv_m), m0 = (tile - range * a.mblocks) * BM;
+        const int c0 = range * a.w, c1 = min(a.N, c0 + a.w);
+        k = k_start(range, a.rot, nsteps);
+#pragma unroll
+        for (int j = 0; j < IPW; ++j) {
+          const int row = 8 * (lw + 4 * j) + (lane >> 3);
+          const int c = (lane & 7) ^ ((row >> 1) & 7);
+          src[j] = j < CT ? a.W + (size_t)min(c0 + row, c1 - 1) * a.K + 8 * c
+                          : a.X + (size_t)min(m0 + row - WR, a.M - 1) * a.xs + 8 * c;
+        }
+      }
+      char* base = smem + buf * STAGE_BYTES + lw * 1024;
+#pragma unroll
+      for (int j = 0; j < IPW; ++j) {
+        if (j < CT && a.nt)
+          __builtin_amdgcn_global_load_lds((gptr_t)(src[j] + k * 64), (lptr_t)(base + j * 4096), 16, 0, 2);
+        else
+          __builtin_amdgcn_global_load_lds((gptr_t)(src[j] + k * 64), (lptr_t)(base + j * 4096), 16, 0, 0);
+      }
+      ++step;
+      k = k + 1 == nsteps ? 0 : k + 1;
+    };
+    for (int s = 0; s < stages - 1; ++s)
+      if (s < total) issue(s);
+    int buf = stages - 1;
+    for (int t = 0; t < total; ++t) {
+      dt_wait<IPW>(min(total - 1 - t, stages - 2));
+      __builtin_amdgcn_s_barrier();  // stage t is there, and every wave is done with stage t - 1
+      if (t + stages - 1 < total) {
+        issue(buf);
+        buf = buf + 1 == stages ? 0 : buf + 1;
+      }
+    }
+    return;
+  }
+
+  const int wm = wave & 1, wn = wave >> 1;
+  const int r16 = lane & 15, q = lane >> 4;
+  const int key = (r16 >> 1) & 7;
+  const int co0 = (q ^ key) << 4, co1 = ((4 + q) ^ key) << 4;
+  const int wb = (wn * CT * 16 + r16) * 128, xb = (WR + wm * RT * 16 + r16) * 128;
+
+  const char* sb = smem;
+  int buf = 0;
+  DTFrag<RT, CT> fa, fb;
+  if (mine > 0) {
+    dt_barrier();
+    fa.read(sb + xb + co0, sb + wb + co0);
+  }
+  for (int i = 0, tile = first; i < mine; ++i, tile += nwg) {
+    f32x4 acc[CT][RT];
+#pragma unroll
+    for (int c = 0; c < CT; ++c)
+#pragma unroll
+      for (int r = 0; r < RT; ++r) acc[c][r] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t + 1 < nsteps; ++t) {
+      dt_lds_done();
+      fb.read(sb + xb + co1, sb + wb + co1);
+      fa.multiply(acc);
+      dt_deal<RT, CT, 0>();
+      dt_lds_done();
+      dt_barrier();
+      buf = buf + 1 == stages ? 0 : buf + 1;
+      sb = smem + buf * STAGE_BYTES;
+      fa.read(sb + xb + co0, sb + wb + co0);
+      fb.multiply(acc);
+      dt_deal<RT, CT, 1>();
+    }
+    dt_lds_done();
+    fb.read(sb + xb + co1, sb + wb + co1);
+    fa.multiply(acc);
+    dt_deal<RT, CT, 2>();
+    dt_lds_done();
+    if (i + 1 < mine) {  // on to the next range's first stage: the loaders go on while this one's outputs are stored
+      dt_barrier();
+      buf = buf + 1 == stages ? 0 : buf + 1;
+      sb = smem + buf * STAGE_BYTES;
+      fa.read(sb + xb + co0, sb + wb + co0);
+    }
+    fb.multiply(acc);
+    const int range = quotient(tile, a.mblocks, a.inv_m), m0 = (tile - range * a.mblocks) * BM + wm * RT * 16 + r16;
+    const int n0 = range * a.w + wn * CT * 16 + 4 * q, c1 = min(a.N, range * a.w + a.w);
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+      if (m0 + 16 * r >= a.M) continue;
+      bf16_t* y = (bf16_t*)a.Y + (size_t)(m0 + 16 * r) * a.ys;
+#pragma unroll
+      for (int c = 0; c < CT; ++c)
+        if (n0 + 16 * c < c1)
+          *reinterpret_cast<bf16x4*>(y + n0 + 16 * c) = bf16x4{f2bf(acc[c][r][0]), f2bf(acc[c][r][1]), f2bf(acc[c][r][2]), f2bf(acc[c][r][3])};
+    }
+  }
+}
+
+template <int RT, int CT>
+int dt_walk(DTArgs a, int workgroups, hipStream_t st) {
+  constexpr int stage_bytes = 32 * (RT + CT) * 128;
+  a.stages = min(6, 160 * 1024 / stage_bytes);
+  auto kern = dtile_walk_kernel<RT, CT>;
+  static bool attr_set = false;  // per instantiation
+  if (!attr_set) {
+    HIP_RET(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 / stage_bytes * stage_bytes));
+    attr_set = true;
+  }
+  a.inv_m = reciprocal((long)a.ntiles * a.mblocks, a.mblocks);
+  hipLaunchKernelGGL(kern, dim3(workgroups), dim3(512), a.stages * stage_bytes, st, a);
+  return (int)hipGetLastError();
+}
+
 template <int RT, int CT, int EPI, bool ROT>
 int dt_launch_as(DTArgs a, hipStream_t st) {
   constexpr int stage_bytes = 32 * (RT + CT) * 128;
@@ -394,4 +534,25 @@ extern "C" int areal_dtile_slab(const void* X, long xs, const void* W, void* Y, 
   a.stages = stages; a.nt = nt; a.act = 0; a.rot = 0;
   const int rows = (M + mblocks - 1) / mblocks;
   return dt_rows<DT_SLAB>(a, (rows + 31) / 32, ct, st);
+}
+
+// X [M, K] bf16 (row stride xs), W [N, K] bf16 contiguous, Y [M, N] bf16 (row stride ys): K % 64 == 0, N % 4 == 0, 4 <= w <= 160 columns
+// a range (a multiple of 4), row blocks of 32 rt rows, rt = ceil(M / mblocks / 32) of 3 to 5.
+extern "C" int areal_dtile_rows(const void* X, long xs, const void* W, void* Y, long ys, int M, int N, int K, int w, int mblocks,
+                                int workgroups, int nt, hipStream_t st) {
+  if (M <= 0) return 0;
+  if (K % 64 != 0 || K < 64 || xs % 8 != 0 || N % 4 != 0 || N < 4 || w % 4 != 0 || w < 4 || w > 160 || ys % 4 != 0) return -1;
+  if (mblocks < 1 || workgroups < 8 || workgroups % 8 != 0) return -2;
+  if (((uintptr_t)X | (uintptr_t)W) % 16 != 0 || (uintptr_t)Y % 8 != 0) return -3;
+  DTArgs a = {};
+  a.X = (const bf16_t*)X; a.xs = xs; a.W = (const bf16_t*)W; a.Y = Y; a.ys = ys;
+  a.M = M; a.N = N; a.K = K; a.w = w; a.ntiles = (N + w - 1) / w; a.mblocks = mblocks; a.nt = nt; a.rot = k_rotation(K);
+  if ((long)a.ntiles * mblocks * (K / 64) >= (1l << 31)) return -4;
+  const int rt = ((M + mblocks - 1) / mblocks + 31) / 32;
+  switch (rt) {
+    case 3: return dt_walk<3, 5>(a, workgroups, st);
+    case 4: return dt_walk<4, 5>(a, workgroups, st);
+    case 5: return dt_walk<5, 5>(a, workgroups, st);
+  }
+  return -10;
 }
