@@ -570,26 +570,37 @@ __global__ __launch_bounds__(1024) void sample_kernel(
   float mx = -INFINITY, mn = INFINITY, se = 0.f;
   const bool sliced = ws && filtered && row_sliced(k, V, S);
   bool listed = sliced;  // the slices have handed on all that can be drawn
+  // A lane reads a slice's words and a wave copies its entries: one slice after the other they were a chain of up to 16 trips to
+  // memory (24 rows of 151936 entries in 8 slices, top-k 50 with top-p 0.95: 34.0 us for both kernels, 30.8 now).
+  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int handed = 0;
   if (sliced) {
-    const float* o = ws + (size_t)row * S * SLICE_WORDS;
-    for (int s = 0; s < S; ++s) {
-      mx = fmaxf(mx, o[(size_t)s * SLICE_WORDS]);
-      mn = fminf(mn, o[(size_t)s * SLICE_WORDS + 3]);
-      listed = listed && __float_as_int(o[(size_t)s * SLICE_WORDS + 2]) >= 0;
+    f32x4 o = {-INFINITY, 0.f, 0.f, INFINITY};
+    if (lane < S) o = *reinterpret_cast<const f32x4*>(ws + ((size_t)row * S + lane) * SLICE_WORDS);
+    mx = o[0];
+    mn = o[3];
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) {
+      mx = fmaxf(mx, __shfl_xor(mx, d, 64));
+      mn = fminf(mn, __shfl_xor(mn, d, 64));
     }
-    for (int s = 0; s < S; ++s) {
-      const float m = o[(size_t)s * SLICE_WORDS];
-      if (m > -INFINITY) se += o[(size_t)s * SLICE_WORDS + 1] * __expf(m - mx);
-    }
+    handed = __float_as_int(o[2]);
+    listed = !__any(handed < 0);
+    const float scale = o[0] > -INFINITY ? __expf(o[0] - mx) : 0.f;
+    for (int s = 0; s < S; ++s)  // in the order of the slices
+      se += __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(o[1]), s)) *
+            __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(scale), s));
   }
   if (listed) {
-    const float* o = ws + (size_t)row * S * SLICE_WORDS;
     int n = 0;
-    for (int s = 0; s < S; ++s, o += SLICE_WORDS) {
-      const int c = __float_as_int(o[2]);
-      for (int i = threadIdx.x; i < c; i += blockDim.x) {
-        list_z[n + i] = o[4 + i];
-        list_i[n + i] = __float_as_int(o[4 + TOPK_CAP + i]);
+    for (int s = 0; s < S; ++s) {
+      const int c = __builtin_amdgcn_readlane(handed, s);
+      if ((s & 15) == wid) {  // one of the block's 16 waves
+        const float* o = ws + ((size_t)row * S + s) * SLICE_WORDS + 4;
+        for (int i = lane; i < c; i += 64) {
+          list_z[n + i] = o[i];
+          list_i[n + i] = __float_as_int(o[TOPK_CAP + i]);
+        }
       }
       n += c;
     }
