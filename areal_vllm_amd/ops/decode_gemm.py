@@ -228,7 +228,7 @@ WIDE_MIN_COLUMNS, WIDE_MIN_ROWS, WIDE_MAX_ROWS = 16384, 65, 160
 def takes_wide(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether `dgemm_wide` takes the product: all rows in one block (GPU only)."""
     M, K = x.shape
-    return (WIDE_MIN_ROWS <= M <= WIDE_MAX_ROWS and w.shape[0] % 4 == 0 and K % 64 == 0 and K > 0 and x.is_cuda
+    return (WIDE_MIN_ROWS <= M <= WIDE_MAX_ROWS and w.dim() == 2 and w.shape[1] == K and w.shape[0] % 4 == 0 and K % 64 == 0 and K > 0 and x.is_cuda
             and x.dtype == w.dtype == torch.bfloat16 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and w.is_contiguous()
             and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 

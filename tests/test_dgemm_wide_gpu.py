@@ -30,3 +30,12 @@ def test_what_it_does_not_take():
     assert dg.serves_wide(x, w) and not dg.serves_wide(x, w[:16380]) and dg.takes_wide(x, w[:16380]) and not dg.takes_wide(x, w[:16382])
     assert not dg.takes_wide(x.float(), w) and not dg.takes_wide(x[:, ::2], half) and not dg.takes_wide(x[:, 4:68], half)
     assert not dg.takes_wide(x[:64], w) and not dg.takes_wide(torch.randn(161, 128, device=DEV).bfloat16(), w)
+
+
+@pytest.mark.parametrize("depth", [64, 192])
+def test_weights_of_another_depth_are_refused(depth):
+    """The kernel steps through the weight in rows as deep as x: on the host, before anything is launched."""
+    x, w = torch.randn(65, 128, device=DEV).bfloat16(), torch.randn(16384, depth, device=DEV).bfloat16()
+    assert not dg.takes_wide(x, w) and not dg.serves_wide(x, w) and not dg.takes_wide(x, w.view(-1))
+    with pytest.raises(AssertionError):
+        dg.dgemm_wide(x, w)
