@@ -115,12 +115,16 @@ def moe_topk(logits: torch.Tensor, k: int, norm: bool, out_dtype=torch.float32):
         if norm:
             topv = topv / topv.sum(-1, keepdim=True)
         return topv.to(out_dtype), topi
-    logits = logits.contiguous()
+    return _topk(logits.contiguous(), k, norm, out_dtype, False)
+
+
+def _topk(logits: torch.Tensor, k: int, norm: bool, out_dtype, train: bool):
+    T, E = logits.shape
     topi = torch.empty(T, k, dtype=torch.int64, device=logits.device)
     topv = torch.empty(T, k, dtype=out_dtype, device=logits.device)
     f32 = out_dtype == torch.float32
     L.check(L.lib().areal_moe_topk(L.ptr(logits), L.c_int(L.dtype_flag(logits)), L.c_int(0), L.c_int64(T), L.c_int(E),
-                                   L.c_int(k), L.c_int(int(bool(norm))), L.ptr(topi), L.ptr(topv) if f32 else None,
+                                   L.c_int(k), L.c_int(int(bool(norm))), L.c_int(int(train)), L.ptr(topi), L.ptr(topv) if f32 else None,
                                    None if f32 else L.ptr(topv), L.stream_ptr()), "moe_topk")
     return topv, topi
 
@@ -129,7 +133,7 @@ class _TopkFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, logits, k, norm):
         logits = logits.contiguous()
-        topv, topi = moe_topk(logits, k, norm)
+        topv, topi = _topk(logits, k, norm, torch.float32, True)
         ctx.save_for_backward(logits, topi)
         ctx.norm = norm
         ctx.mark_non_differentiable(topi)
@@ -182,7 +186,7 @@ def moe_route(x: torch.Tensor, router: torch.Tensor, k: int, norm: bool, out_dty
     topv = torch.empty(T, k, dtype=out_dtype, device=x.device)
     f32 = out_dtype == torch.float32
     L.check(L.lib().areal_moe_topk(L.ptr(slab), L.c_int(L.dtype_flag(slab)), L.c_int(slab.shape[0]), L.c_int64(T), L.c_int(E),
-                                   L.c_int(k), L.c_int(int(bool(norm))), L.ptr(topi), L.ptr(topv) if f32 else None,
+                                   L.c_int(k), L.c_int(int(bool(norm))), L.c_int(0), L.ptr(topi), L.ptr(topv) if f32 else None,
                                    None if f32 else L.ptr(topv), L.stream_ptr()), "moe_topk")
     return topv, topi
 

@@ -291,7 +291,11 @@ constexpr int RT_MAX_PER_LANE = 8;  // experts <= 512
 // 128 experts: 7.6 us a launch in a decode step, 7.1 now with ten partial products summed on the way, whose GEMM takes 4.0
 // where the whole product took 10.5). slabs > 0: `logits` are that many fp32 partial products [slabs, T, E] of the router,
 // whose sum is rounded to bf16 as the projection's output is.
-template <typename TIN, int PER_LANE>
+// TRAIN: weights that a gradient flows through, with the exponential that is right to a unit in the last place, as the library's softmax
+// takes it: __expf is off by |v - mx| 2^-24 more (probabilities of 1e-24: 25 units).
+DEVINL float route_exp(float x, bool train) { return train ? expf(x) : __expf(x); }
+
+template <typename TIN, int PER_LANE, bool TRAIN>
 __global__ __launch_bounds__(256) void moe_topk_kernel(const TIN* __restrict__ logits, int slabs, int64_t T, int E, int k,
                                                        int norm, int64_t* __restrict__ topi,
                                                        float* __restrict__ topv, bf16_t* __restrict__ topv_bf) {
@@ -325,7 +329,7 @@ __global__ __launch_bounds__(256) void moe_topk_kernel(const TIN* __restrict__ l
   mx = wave_max(mx);
   float se = 0.f;
 #pragma unroll
-  for (int i = 0; i < PER_LANE; ++i) se += v[i] > -INFINITY ? __expf(v[i] - mx) : 0.f;
+  for (int i = 0; i < PER_LANE; ++i) se += v[i] > -INFINITY ? route_exp(v[i] - mx, TRAIN) : 0.f;
   se = wave_sum(se);
   float mine_v = 0.f;  // lane j keeps choice j
   int mine_i = 0;
@@ -343,7 +347,7 @@ __global__ __launch_bounds__(256) void moe_topk_kernel(const TIN* __restrict__ l
         if (has) bi = 64 * i + __ffsll(has) - 1;
       }
     }
-    const float p = __expf(bv - mx) / se;
+    const float p = route_exp(bv - mx, TRAIN) / se;
     picked += p;
     if (lane == j) {
       mine_v = p;
@@ -522,14 +526,14 @@ __global__ __launch_bounds__(1024) void moe_sort_single_kernel(const int64_t* __
   }
 }
 
-template <typename TIN>
+template <bool TRAIN, typename TIN>
 static int topk_launch(const TIN* logits, int slabs, int64_t T, int E, int k, int norm, int64_t* topi, float* topv,
                        bf16_t* topv_bf, hipStream_t st) {
   const int waves = T <= 1024 ? 1 : 4;  // a row a CU while there are CUs: a workgroup's rows share its load path
   const dim3 grid((unsigned)((T + waves - 1) / waves)), block(64 * waves);
 #define TOPK_CASE(P) \
   if (E <= 64 * P) { \
-    hipLaunchKernelGGL((moe_topk_kernel<TIN, P>), grid, block, 0, st, logits, slabs, T, E, k, norm, topi, topv, topv_bf); \
+    hipLaunchKernelGGL((moe_topk_kernel<TIN, P, TRAIN>), grid, block, 0, st, logits, slabs, T, E, k, norm, topi, topv, topv_bf); \
     return (int)hipGetLastError(); \
   }
   TOPK_CASE(1) TOPK_CASE(2) TOPK_CASE(4) TOPK_CASE(8)
@@ -538,13 +542,18 @@ static int topk_launch(const TIN* logits, int slabs, int64_t T, int E, int k, in
 }
 
 // logits [T, E] fp32 (dtype 1) or bf16 (dtype 0); slabs > 0: fp32 partial products [slabs, T, E]; weights are written as fp32
-// (topv), bf16 (topv_bf) or both.
-extern "C" int areal_moe_topk(const void* logits, int dtype, int slabs, int64_t T, int E, int k, int norm, int64_t* topi,
+// (topv), bf16 (topv_bf) or both. train: of whole logits, weights that a gradient flows through (areal_moe_topk_bwd).
+extern "C" int areal_moe_topk(const void* logits, int dtype, int slabs, int64_t T, int E, int k, int norm, int train, int64_t* topi,
                               float* topv, void* topv_bf, hipStream_t st) {
   if (T == 0) return 0;
   if (E < 1 || E > 64 * RT_MAX_PER_LANE || k < 1 || k > 64 || k > E || slabs < 0 || (slabs && dtype == 0)) return -1;
-  if (dtype == 0) return topk_launch((const bf16_t*)logits, 0, T, E, k, norm, topi, topv, (bf16_t*)topv_bf, st);
-  return topk_launch((const float*)logits, slabs, T, E, k, norm, topi, topv, (bf16_t*)topv_bf, st);
+  if (train && slabs) return -2;
+  if (dtype == 0) {
+    if (train) return topk_launch<true>((const bf16_t*)logits, 0, T, E, k, norm, topi, topv, (bf16_t*)topv_bf, st);
+    return topk_launch<false>((const bf16_t*)logits, 0, T, E, k, norm, topi, topv, (bf16_t*)topv_bf, st);
+  }
+  if (train) return topk_launch<true>((const float*)logits, 0, T, E, k, norm, topi, topv, (bf16_t*)topv_bf, st);
+  return topk_launch<false>((const float*)logits, slabs, T, E, k, norm, topi, topv, (bf16_t*)topv_bf, st);
 }
 
 // Gradient of topk's weights in its logits: with p the softmax, e_j the choices, S the sum of their p (not `norm`: 1) and g the gradient
@@ -574,7 +583,7 @@ __global__ __launch_bounds__(256) void moe_topk_bwd_kernel(const TIN* __restrict
   mx = wave_max(mx);
 #pragma unroll
   for (int i = 0; i < PER_LANE; ++i) {
-    v[i] = v[i] > -INFINITY ? __expf(v[i] - mx) : 0.f;
+    v[i] = v[i] > -INFINITY ? route_exp(v[i] - mx, true) : 0.f;
     se += v[i];
   }
   se = wave_sum(se);

@@ -30,6 +30,27 @@ def test_weights_of_the_choices(T, E, k, norm, dtype):
     assert float((err - (2.0 ** -8 * d64.abs() if dtype == torch.bfloat16 else 0.0)).max()) < 2.0 ** -18 * max(1.0, float(gv.abs().max()))
 
 
+@pytest.mark.parametrize("E,k,dtype", [(8, 8, torch.float32), (64, 64, torch.float32), (64, 64, torch.bfloat16), (512, 64, torch.float32)])
+def test_small_probabilities_are_as_exact_as_large_ones(E, k, dtype):
+    """Logits that are multiples of 1/2 down to -80 below one that is far above all others: differences and sums are exact but for the
+    last bits. The exponential is off by a unit in the last place (2^-23), the sum (terms of e^-8 and less beside 1) and the quotient by
+    less: below 2^-21 together. The exponential of a rounded product would be off by |logit - max| 2^-24, up to 2^-18."""
+    g = torch.Generator(device=DEV).manual_seed(E)
+    z = (-8.0 - torch.randint(0, 145, (200, E), device=DEV, generator=g) / 2.0).to(dtype)
+    z[:, E // 3] = 0.0
+    z.requires_grad_(True)
+    v, i = moe.moe_topk_grad(z, k, False)
+    z64 = z.detach().double().requires_grad_(True)
+    want = torch.softmax(z64, -1).gather(1, i)
+    assert float(((v.double() - want) / want).detach().abs().max()) < 2.0 ** -21
+    gv = torch.rand(200, k, device=DEV, generator=g) + 0.5
+    (dz,) = torch.autograd.grad(v, z, gv)
+    (d64,) = torch.autograd.grad(want, z64, gv.double())
+    # p (g - sum of p g), the bracket at most 1.5: p's error, and some 2^-24 of the bracket; 16-bit results are rounded once
+    err = ((dz.double() - d64).abs() / torch.softmax(z64.detach(), -1)).max()
+    assert float(err) < (2.0 ** -20 if dtype == torch.float32 else 2.0 ** -8)
+
+
 def test_choices_next_to_infinities():
     z = torch.full((2, 70), -float("inf"), device=DEV)
     z[:, 3], z[:, 69] = 1.0, 2.0
