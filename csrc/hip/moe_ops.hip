@@ -329,7 +329,11 @@ __global__ __launch_bounds__(256) void moe_topk_kernel(const TIN* __restrict__ l
   mx = wave_max(mx);
   float se = 0.f;
 #pragma unroll
-  for (int i = 0; i < PER_LANE; ++i) se += v[i] > -INFINITY ? route_exp(v[i] - mx, TRAIN) : 0.f;
+  for (int i = 0; i < PER_LANE; ++i) {
+    // TRAIN: a NaN or +inf among the logits, or nothing but -inf, makes the row's weights NaN, as softmax does
+    const bool counts = TRAIN ? lane + 64 * i < E : v[i] > -INFINITY;
+    se += counts ? route_exp(v[i] - mx, TRAIN) : 0.f;
+  }
   se = wave_sum(se);
   float mine_v = 0.f;  // lane j keeps choice j
   int mine_i = 0;
@@ -583,7 +587,7 @@ __global__ __launch_bounds__(256) void moe_topk_bwd_kernel(const TIN* __restrict
   mx = wave_max(mx);
 #pragma unroll
   for (int i = 0; i < PER_LANE; ++i) {
-    v[i] = v[i] > -INFINITY ? route_exp(v[i] - mx, true) : 0.f;
+    v[i] = lane + 64 * i < E ? route_exp(v[i] - mx, true) : 0.f;  // (NaN where the softmax is)
     se += v[i];
   }
   se = wave_sum(se);

@@ -63,6 +63,25 @@ def test_choices_next_to_infinities():
     assert int((dz != 0).sum()) == 4
 
 
+@pytest.mark.parametrize("E,k", [(5, 2), (64, 8), (130, 3)])
+@pytest.mark.parametrize("norm", [True, False])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), None])
+def test_a_row_that_softmax_makes_nan_is_nan(E, k, norm, bad):
+    """None: a row of nothing but -inf. Weights and gradients of that row, and of no other; choices that exist."""
+    g = torch.Generator(device=DEV).manual_seed(E)
+    z = torch.randn(3, E, device=DEV, generator=g)
+    z[1] = -float("inf") if bad is None else z[1]
+    if bad is not None:
+        z[1, E - 2] = bad
+    assert bool(torch.softmax(z, -1)[1].isnan().all())
+    z.requires_grad_(True)
+    v, i = moe.moe_topk_grad(z, k, norm)
+    (dz,) = torch.autograd.grad(v, z, torch.ones_like(v) + torch.arange(k, device=DEV))
+    for t in (v, dz):
+        assert bool(t[1].isnan().all()) and bool(torch.isfinite(t[[0, 2]]).all())
+    assert int(i.min()) >= 0 and int(i.max()) < E
+
+
 @pytest.mark.parametrize("T,k,H", [(1, 1, 8), (3, 2, 2040), (5, 3, 2048), (2, 4, 2056), (64, 8, 2048), (7, 9, 4104), (3, 16, 64)])
 def test_recombination_backward_is_that_of_the_two_passes(T, k, H):
     """Rows bit for bit; a weight's gradient against 64 bits: H products summed in fp32, rounded once."""
