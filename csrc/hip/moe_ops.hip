@@ -338,6 +338,9 @@ __global__ __launch_bounds__(256) void moe_topk_kernel(const TIN* __restrict__ l
   float mine_v = 0.f;  // lane j keeps choice j
   int mine_i = 0;
   float picked = 0.f;
+  unsigned open = 0;  // TRAIN: which of this lane's experts are not chosen yet
+#pragma unroll
+  for (int i = 0; i < PER_LANE; ++i) open |= (lane + 64 * i < E ? 1u : 0u) << i;
   for (int j = 0; j < k; ++j) {
     float bv = v[0];
 #pragma unroll
@@ -348,6 +351,12 @@ __global__ __launch_bounds__(256) void moe_topk_kernel(const TIN* __restrict__ l
 #pragma unroll
       for (int i = PER_LANE - 1; i >= 0; --i) {  // the lowest index of the largest value
         const unsigned long long has = __ballot(v[i] == bv);
+        if (has) bi = 64 * i + __ffsll(has) - 1;
+      }
+    } else if (TRAIN) {  // choices of weight 0 (or NaN) are experts of their own: the gradient looks their probabilities up
+#pragma unroll
+      for (int i = PER_LANE - 1; i >= 0; --i) {
+        const unsigned long long has = __ballot(open >> i & 1);
         if (has) bi = 64 * i + __ffsll(has) - 1;
       }
     }
@@ -361,6 +370,7 @@ __global__ __launch_bounds__(256) void moe_topk_kernel(const TIN* __restrict__ l
 #pragma unroll
       for (int i = 0; i < PER_LANE; ++i)
         if (i == (bi >> 6)) v[i] = -INFINITY;
+      if (TRAIN) open &= ~(1u << (bi >> 6));
     }
   }
   if (lane < k) {

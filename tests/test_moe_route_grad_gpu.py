@@ -63,6 +63,29 @@ def test_choices_next_to_infinities():
     assert int((dz != 0).sum()) == 4
 
 
+@pytest.mark.parametrize("E,k,finite", [(2, 2, [0]), (70, 5, [0, 69]), (70, 64, [66, 0, 3]), (512, 9, [511]), (64, 64, [0])])
+@pytest.mark.parametrize("norm", [True, False])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_more_choices_than_finite_logits(E, k, finite, norm, dtype):
+    """Every choice is another expert, those of weight 0 the first ones that are left, and the gradient is softmax's of these choices."""
+    z = torch.full((3, E), -float("inf"), device=DEV)
+    z[:, finite] = torch.tensor([[0.5 * j for j in range(len(finite))]] * 3, device=DEV)
+    z = z.to(dtype).requires_grad_(True)
+    v, i = moe.moe_topk_grad(z, k, norm)
+    rest = [e for e in range(E) if e not in finite]
+    assert i.tolist() == [(finite[::-1] + rest)[:k]] * 3
+    gv = torch.arange(3 * k, device=DEV).view(3, k) / 8.0
+    (dz,) = torch.autograd.grad(v, z, gv)
+    z64 = z.detach().double().requires_grad_(True)
+    want = torch.softmax(z64, -1).gather(1, i)
+    want = want / want.sum(-1, keepdim=True) if norm else want
+    (d64,) = torch.autograd.grad(want, z64, gv.double())
+    assert float((v.double() - want).detach().abs().max()) < 2.0 ** -21  # as of small probabilities
+    # terms of up to max(gv), a few 2^-24 each; 16-bit results are rounded once
+    top = float(gv.max())
+    assert float(((dz.double() - d64).abs() - (2.0 ** -8 * d64.abs() if dtype == torch.bfloat16 else 0.0)).max()) < 2.0 ** -20 * top
+
+
 @pytest.mark.parametrize("E,k", [(5, 2), (64, 8), (130, 3)])
 @pytest.mark.parametrize("norm", [True, False])
 @pytest.mark.parametrize("bad", [float("nan"), float("inf"), None])
