@@ -14,9 +14,7 @@ import torch
 import torch.distributed as dist
 import torch.nn.functional as F
 
-from . import _lib as L
 from . import train_gemm
-from .optim import after_fold, fold_target
 
 
 def _accumulate_wgrad(weight: torch.Tensor, dy2: torch.Tensor, x2: torch.Tensor) -> None:
@@ -31,21 +29,6 @@ def _accumulate_wgrad(weight: torch.Tensor, dy2: torch.Tensor, x2: torch.Tensor)
         mg.add_(torch.mm(dy2.t(), x2))
 
 
-def _accumulate_bias(bias: torch.Tensor, dy2: torch.Tensor) -> bool:
-    """Adds the bias' gradient to its fp32 buffer, where there is one and the rows are the kernel's."""
-    acc = fold_target(bias)
-    if (acc is None or not L.use_hip(dy2) or dy2.dtype != torch.bfloat16 or dy2.stride(1) != 1 or dy2.shape[1] % 8
-            or dy2.stride(0) % 8 or dy2.data_ptr() % 16 or not dy2.shape[0]):
-        return False
-    M, N = dy2.shape
-    blocks = L.lib().areal_colsum_blocks(L.c_int(M))
-    part = torch.empty(blocks * N, dtype=torch.float32, device=dy2.device) if blocks > 1 else None
-    L.check(L.lib().areal_colsum_add(L.ptr(dy2), L.c_int64(dy2.stride(0)), L.c_int(M), L.c_int(N), L.ptr(acc), L.ptr(part), L.stream_ptr()),
-            "colsum_add")
-    after_fold(bias)
-    return True
-
-
 def _product(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) -> torch.Tensor:
     """x @ W^T (+ b) outside autograd."""
     s = weight.shape
@@ -58,13 +41,14 @@ def _product(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]
 class _LinearMainGrad(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, weight, bias, reduce_dx_group):
-        ctx.save_for_backward(x, weight, bias)
+        ctx.save_for_backward(x, weight)
+        ctx.has_bias = bias is not None
         ctx.group = reduce_dx_group
         return _product(x, weight, bias)
 
     @staticmethod
     def backward(ctx, dy):
-        x, weight, bias = ctx.saved_tensors
+        x, weight = ctx.saved_tensors
         dy2 = dy.reshape(-1, dy.shape[-1])
         dx, work = None, None
         if ctx.needs_input_grad[0]:
@@ -84,9 +68,7 @@ class _LinearMainGrad(torch.autograd.Function):
                     done(weight)
             else:
                 dw = torch.mm(dy2.t(), x.reshape(-1, x.shape[-1]))
-        db = None
-        if bias is not None and ctx.needs_input_grad[2] and not _accumulate_bias(bias, dy2):
-            db = dy2.sum(0)
+        db = dy2.sum(0) if ctx.has_bias and ctx.needs_input_grad[2] else None
         if work is not None:
             work.wait()
         return dx, dw, db, None

@@ -10,7 +10,6 @@ from typing import Optional, Tuple
 import torch
 
 from . import _lib as L
-from .optim import after_fold, fold_target
 
 
 # ------------------------------------------------------------------------------- RMSNorm
@@ -80,20 +79,16 @@ class _RMSNormFn(torch.autograd.Function):
         ds2 = ds.reshape(-1, H).contiguous() if ds is not None else None
         if L.use_hip(s):
             dx = torch.empty_like(s)
-            # an fp32 gradient buffer behind the weight is added to by the reduction itself (a launch and a 16-bit rounding less)
-            acc = fold_target(weight) if ctx.needs_input_grad[2] else None
-            dw = torch.empty_like(weight) if acc is None else None
+            dw = torch.empty_like(weight)
             G = L.lib().areal_rmsnorm_bwd_nblocks(L.c_int(T))
             ws = torch.empty(G * H, dtype=torch.float32, device=s.device)
             L.check(
                 L.lib().areal_rmsnorm_bwd(
                     L.ptr(dy2), L.ptr(s), L.ptr(weight), L.ptr(rstd), L.ptr(ds2), L.ptr(dx), L.ptr(dw),
-                    L.ptr(acc), L.ptr(ws), L.c_int(T), L.c_int(H), L.c_int(int(ctx.gemma)), L.stream_ptr(),
+                    L.ptr(None), L.ptr(ws), L.c_int(T), L.c_int(H), L.c_int(int(ctx.gemma)), L.stream_ptr(),
                 ),
                 "rmsnorm_bwd",
             )
-            if acc is not None:
-                after_fold(weight)
         else:
             dx, dw = _rmsnorm_bwd_ref(dy2, s, weight, rstd, ds2, ctx.gemma)
         dx = dx.view(ctx.shape)

@@ -6,7 +6,6 @@ on device so that a step (norm -> clip coefficient -> skip-if-nonfinite -> AdamW
 with the host: [sumsq, norm, clip_coef, applied, step, bias_corr1, bias_corr2, pad].
 """
 import math
-from typing import Optional
 
 import torch
 
@@ -32,20 +31,6 @@ def fold_grad_(acc: torch.Tensor, grad: torch.Tensor) -> None:
         L.check(L.lib().areal_fold_grad(L.ptr(acc), L.ptr(grad), L.c_int64(acc.numel()), L.stream_ptr()), "fold_grad")
     else:
         acc.add_(grad)
-
-
-def fold_target(p: torch.Tensor) -> Optional[torch.Tensor]:
-    """The fp32 buffer behind a parameter that a kernel may add its gradient to, None where the gradient goes back through autograd."""
-    mg = getattr(p, "main_grad", None)
-    ok = mg is not None and mg.is_cuda and mg.dtype == torch.float32 and mg.is_contiguous() and mg.shape == p.shape
-    return mg if ok else None
-
-
-def after_fold(p: torch.Tensor) -> None:
-    """A kernel has added the parameter's gradient to that buffer: the accumulation hook, which reports it otherwise, is passed by."""
-    done = getattr(p, "_after_fold", None)
-    if done is not None:
-        done(p)
 
 
 def scale_(x: torch.Tensor, scale: float, scale_tensor: torch.Tensor = None) -> None:

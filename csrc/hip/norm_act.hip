@@ -4,8 +4,6 @@
 // and each row is handled by one 64-lane wave with in-wave shuffles for reductions.
 // These replace the TransformerEngine/apex/flash-attn-Triton ops the reference leans
 // on (realhf/impl/model/modules/mlp.py:319-341, realhf/impl/model/modules/rotary.py).
-#include <algorithm>
-
 #include "common.hpp"
 
 // ----------------------------------------------------------------------------------
@@ -184,61 +182,8 @@ __global__ __launch_bounds__(256) void colsum_partial_kernel(const float* __rest
 #pragma unroll
     for (int i = 0; i < 8; ++i) s += red[i][cx];
     if (out_bf16) out_bf16[c] = f2bf(s);
-    if (out_f32) out_f32[c] += s;
+    if (out_f32) out_f32[c] = s;
   }
-}
-
-// Column sums of rows [blockIdx.y * chunk, + chunk) of x [M, N]: added to out (part null) or written to part [gridDim.y, N]. A block
-// covers 64 columns, 8 lanes of 8 columns beside each other and 32 rows at a time, eight of them in flight a thread.
-__global__ __launch_bounds__(256) void colsum_rows_kernel(const bf16_t* __restrict__ x, int64_t ld, int M, int N, int chunk,
-                                                          float* __restrict__ out, float* __restrict__ part) {
-  __shared__ __attribute__((aligned(16))) float red[32][64 + 4];
-  const int cl = (threadIdx.x & 7) * 8, c = blockIdx.x * 64 + cl, r = threadIdx.x >> 3;
-  const int lo = blockIdx.y * chunk, hi = min(M, lo + chunk);
-  float s[8] = {};
-  if (c < N) {
-    for (int i0 = lo + r; i0 < hi; i0 += 32 * 8) {
-      bf16x8 v[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) v[u] = ld8(x + (int64_t)min(i0 + 32 * u, hi - 1) * ld + c);
-#pragma unroll
-      for (int u = 0; u < 8; ++u)
-        if (i0 + 32 * u < hi)
-#pragma unroll
-          for (int j = 0; j < 8; ++j) s[j] += bf2f(v[u][j]);
-    }
-  }
-  *reinterpret_cast<f32x4*>(&red[r][cl]) = f32x4{s[0], s[1], s[2], s[3]};
-  *reinterpret_cast<f32x4*>(&red[r][cl + 4]) = f32x4{s[4], s[5], s[6], s[7]};
-  __syncthreads();
-  const int k = threadIdx.x, col = blockIdx.x * 64 + k;
-  if (k < 64 && col < N) {
-    float t[4] = {};
-#pragma unroll
-    for (int i = 0; i < 32; ++i) t[i & 3] += red[i][k];
-    const float sum = (t[0] + t[1]) + (t[2] + t[3]);
-    if (part) part[(size_t)blockIdx.y * N + col] = sum;
-    else out[col] += sum;
-  }
-}
-
-// Row blocks of areal_colsum_add: one up to 1024 rows, else of 512 rows and more (2048 rows in one / two 8.7 / 6.5 us).
-extern "C" int areal_colsum_blocks(int M) { return M <= 1024 ? 1 : std::min(64, (M + 511) / 512); }
-
-// out[N] (fp32) += column sums of x [M, N] (bf16, row stride ld): the gradient of a bias, into its fp32 buffer. N and ld multiples of
-// 8, x on 16 bytes; part: areal_colsum_blocks(M) * N floats where that is more than one. Memory bounds many rows, two launches of
-// latency few: us of the library's sum, its clearing and the fold of its 16-bit result / of this, 2048 columns, 700 / 4096 / 32768 rows
-// 12.2 / 18.9 / 40.0 and 4.6 / 6.0 / 25.2; relative error 1.6e-3 and 2e-8 to 7e-8.
-extern "C" int areal_colsum_add(const void* x, int64_t ld, int M, int N, float* out, float* part, hipStream_t st) {
-  if (M <= 0 || N <= 0) return 0;
-  if (N % 8 != 0 || ld % 8 != 0 || (uintptr_t)x % 16 != 0) return -1;
-  const int blocks = areal_colsum_blocks(M), chunk = (M + blocks - 1) / blocks;
-  if (blocks > 1 && !part) return -2;
-  hipLaunchKernelGGL(colsum_rows_kernel, dim3((N + 63) / 64, blocks), dim3(256), 0, st, (const bf16_t*)x, ld, M, N, chunk, out,
-                     blocks > 1 ? part : nullptr);
-  if (blocks > 1)
-    hipLaunchKernelGGL(colsum_partial_kernel, dim3((N + 31) / 32), dim3(256), 0, st, part, (bf16_t*)nullptr, out, blocks, N);
-  return (int)hipGetLastError();
 }
 
 extern "C" int areal_rmsnorm_fwd(const void* x, const void* res, const void* w, void* y, void* res_out,
@@ -267,7 +212,6 @@ extern "C" int areal_rmsnorm_bwd_nblocks(int T) {
   return g < 1 ? 1 : (g > 512 ? 512 : g);
 }
 
-// The weight's gradient is written to dw_bf16 or added to dw_f32.
 extern "C" int areal_rmsnorm_bwd(const void* dy, const void* x, const void* w, const float* rstd,
                                  const void* dres, void* dx, void* dw_bf16, float* dw_f32,
                                  float* workspace, int T, int H, int gemma, hipStream_t st) {
