@@ -326,10 +326,7 @@ class MoE(nn.Module):
             xr = x * torch.empty_like(x).uniform_(1.0 - eps, 1.0 + eps)
         plain = cfg.moe_routing_type in ("aux_loss", "none")
         fused_route = plain and not torch.is_grad_enabled() and not self.training
-        # whole 128 x 256 tiles: the router's gradient is summed into its fp32 buffer by the split weight-gradient product (16384 tokens,
-        # 128 experts of 2048: 33 us; the library, whose tiles are not split, 135 to 171)
-        own_dw = router.shape[0] % 128 == 0 and router.shape[1] % 256 == 0
-        raw = None if fused_route else (ops.linear if own_dw else F.linear)(xr, router)
+        raw = None if fused_route else ops.router_logits(xr, router)
         # no loss looks at the router's logits or probabilities: softmax, top-k and their gradient are one launch each way
         alone = plain and not (self.training and (cfg.moe_z_loss_coef > 0 or cfg.moe_routing_type == "aux_loss"
                                                   and cfg.router_aux_loss_coef > 0))

@@ -32,4 +32,4 @@ from .linear import embedding, linear  # noqa: F401
 from .decode_gemm import dgemm, splitk_residual_rmsnorm, splitk_rope_cache_write  # noqa: F401
 from .grouped_gemm import (gate_up_rows_ok, grouped_gate_up, grouped_gemm, grouped_gemm_offsets,  # noqa: F401
                            grouped_gemm_offsets_ok, grouped_gemm_ref)
-from .moe import host_list, moe_combine, moe_combine_rmsnorm, moe_permute, moe_route, moe_sort, moe_topk, moe_topk_grad  # noqa: F401
+from .moe import host_list, moe_combine, moe_combine_rmsnorm, moe_permute, moe_route, moe_sort, moe_topk, moe_topk_grad, router_logits  # noqa: F401

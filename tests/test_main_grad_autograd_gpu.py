@@ -1,9 +1,11 @@
-"""Gradients of biases and norm weights go through autograd, also where an fp32 buffer stands behind the parameter: what hangs on the
+"""Gradients of biases, norm weights and routers go through autograd, also where an fp32 buffer stands behind the parameter: what hangs on the
 parameter sees them, and one backward pass reports each once."""
 import pytest
 import torch
 
 from areal_vllm_amd import ops
+from areal_vllm_amd.models.config import ModelConfig
+from areal_vllm_amd.models.transformer import MoE
 
 DEV = "cuda:0"
 pytestmark = pytest.mark.gpu
@@ -56,3 +58,41 @@ def test_a_parameter_used_twice_is_reported_once(case):
     y = f() + f()
     y.backward(torch.ones_like(y))
     assert calls == [1] and p.told == 0 and torch.equal(p.grad.float(), torch.full_like(p, 2 * want).float())
+
+
+@pytest.mark.parametrize("tokens", [5, 256, 1000])
+def test_router(tokens):
+    """The whole layer, of a size that the split weight-gradient product takes (from 256 tokens on)."""
+    cfg = ModelConfig(family="qwen3_moe", vocab_size=64, hidden_size=256, n_layers=1, n_q_heads=2, n_kv_heads=1, head_dim=64,
+                      intermediate_size=64, n_experts=128, n_experts_per_tok=2, moe_intermediate_size=64)
+    layer = MoE(cfg, 1, torch.bfloat16, DEV)
+    g = torch.Generator(device=DEV).manual_seed(tokens)
+    with torch.no_grad():
+        for p in layer.parameters():
+            p.normal_(0.0, 0.05, generator=g)
+    p = layer.router
+    p.main_grad, p.told, seen, calls = torch.zeros(p.shape, device=DEV), 0, [], []
+    p._after_fold = lambda q: setattr(q, "told", q.told + 1)
+    p.register_hook(lambda t: seen.append(t.clone()))
+    p.register_post_accumulate_grad_hook(lambda q: calls.append(1))
+    x = torch.randn(tokens, 256, device=DEV, generator=g).bfloat16()
+    dy = torch.randn(tokens, 256, device=DEV, generator=g).bfloat16()
+    layer(x, None).backward(dy)
+    assert calls == [1] and p.told == 0 and not p.main_grad.any() and torch.equal(p.grad, seen[0]) and bool(p.grad.any())
+    (again,) = torch.autograd.grad(layer(x, None), p, dy)
+    assert torch.equal(again, p.grad)
+
+
+@pytest.mark.parametrize("T,E,H", [(255, 128, 256), (256, 128, 256), (1000, 256, 512), (4099, 128, 2048)])
+@pytest.mark.parametrize("strided", [False, True])
+def test_router_logits(T, E, H, strided):
+    g = torch.Generator(device=DEV).manual_seed(T)
+    x = torch.randn(T, H + 8 * strided, device=DEV, generator=g).bfloat16()[:, :H].requires_grad_(True)
+    w = torch.nn.Parameter((torch.randn(E, H, device=DEV, generator=g) * 0.1).bfloat16())
+    dy = torch.randn(T, E, device=DEV, generator=g).bfloat16()
+    y = ops.router_logits(x, w)
+    assert torch.equal(y, torch.nn.functional.linear(x, w))
+    dx, dw = torch.autograd.grad(y, (x, w), dy)
+    # fp32 sums of up to 4099 products of values of order one, rounded to 16 bits once
+    for got, want in ((dw, dy.double().t() @ x.detach().double()), (dx, dy.double() @ w.detach().double())):
+        assert float(((got.double() - want).abs() - 2.0 ** -8 * want.abs()).max()) < 2.0 ** -20 * T ** 0.5 * 8
