@@ -523,8 +523,8 @@ class DecodeItems:
         self.arrived = torch.zeros(batch, n_kv_heads, dtype=torch.int32, device=device)
 
     def fill_(self, context_lens: torch.Tensor, block_tables: Optional[torch.Tensor] = None) -> "DecodeItems":
-        """Lay the items out for these context lengths; every layer of the step then uses them. With the rows' block tables, pages that
-        no other row shares are read past the caches (results are the same)."""
+        """Lay the items out for these context lengths; every layer of the step then uses them. With the rows' block tables, items
+        whose middle page no other row has are read past the caches (results are the same)."""
         if L.use_hip(context_lens):
             assert context_lens.dtype == torch.int32 and context_lens.is_contiguous() and context_lens.numel() == self.batch
             assert block_tables is None or (block_tables.dtype == torch.int32 and block_tables.is_contiguous()

@@ -116,3 +116,33 @@ def test_pages_that_no_other_row_reads_go_past_the_caches(rows, group, common, D
     assert torch.equal(*outs)
     ref = A.paged_decode_ref(q[:, :4], kc, vc, bt, cl, 1 / math.sqrt(D)).float()
     assert (outs[0].float().cpu() - ref).abs().max() < 2e-2  # as above
+
+
+@pytest.mark.parametrize("rows,system,own,per", [(3, 5, 9, 2), (24, 4, 16, 4), (320, 2, 20, 16), (1024, 1, 6, 8), (64, 70, 40, 8)])
+@pytest.mark.parametrize("extra", [0, 300])
+def test_pages_of_a_prompt_behind_a_common_one(rows, system, own, per, extra):
+    """All rows share a system prompt of `system` pages, `per` of them a question of `own` pages behind it: what the rows of one question
+    read is theirs in common whichever row of another question came first. Idle rows with one page, all the same, are at the end."""
+    g = torch.Generator().manual_seed(rows)
+    ctx = [int(x) for x in torch.randint(32 * (system + own) + 1, 32 * (system + own) + 700, (rows,), generator=g)] + [1] * min(extra, 1024 - rows)
+    n = len(ctx)
+    q, kc, vc, bt, cl = _setup(ctx, 4, 1, 128, False, 4)
+    bt[rows:, 0] = 0
+    order = torch.randperm(rows, generator=g)
+    for i in range(rows):
+        bt[order[i], :system] = bt[order[0], :system]
+        bt[order[i], system:system + own] = bt[order[i // per * per], system:system + own]
+    d = [t.to(DEV) for t in (q, kc, vc, bt, cl)]
+    plain = ops.DecodeItems(n, 4, 1, 128, torch.device(DEV)).fill_(d[4])
+    marked = ops.DecodeItems(n, 4, 1, 128, torch.device(DEV)).fill_(d[4], d[3])
+    pages = [set(bt[b, :(c + 31) // 32].tolist()) for b, c in enumerate(ctx[:rows])]
+    readers = {}
+    for p in pages:
+        for x in p:
+            readers[x] = readers.get(x, 0) + 1
+    got = [(b, (lo + hi) // 2, stream) for b, lo, hi, _, k, _, stream, _ in marked.items.tolist() if k]
+    assert len(got) == int((plain.items[:, 4] > 0).sum())
+    for b, mid, stream in got:
+        assert stream == int(b >= rows or readers[int(bt[b, mid])] == 1), (b, mid, stream)
+    outs = [ops.paged_attention_decode(d[0][:, :4], *d[1:], q_row_stride=5 * 128, items=i) for i in (plain, marked)]
+    assert torch.equal(*outs)
