@@ -840,6 +840,10 @@ extern "C" int areal_qkv_rows(const void* X, int64_t xs, const void* W, const vo
   a.X = (const bf16_t*)X; a.xs = xs; a.W = (const bf16_t*)W; a.bias = (const bf16_t*)bias; a.Y = (bf16_t*)Y; a.M = M;
   a.N = (Hq + 2 * Hkv) * D; a.K = K; a.pos = pos; a.slots = slots; a.cos_t = cos_t; a.sin_t = sin_t; a.kcache = kcache;
   a.vcache = vcache; a.Hq = Hq; a.Hkv = Hkv; a.D = D; a.max_pos = max_pos; a.do_rope = do_rope; a.fp8 = fp8;
+  if (!do_rope) {  // no angles are used: what is read in their place, D / 2 floats, is the weight's first bytes, whatever the tables hold
+    a.cos_t = a.sin_t = (const float*)W;
+    a.max_pos = 1;
+  }
   const int cols = a.N / 16, per = D / 16, most = 65535 * 16 * rt;  // rows of a launch
   if ((cols + 7) / 8 > 65535) return -1;
   a.per_inv = reciprocal(cols, per);

@@ -81,3 +81,18 @@ def test_rule():
     assert sk.qkv_row_tiles(65, 1536, 2048, 128) == 0 and sk.qkv_row_tiles(24, 2048, 2560, 128) == 0
     assert sk.qkv_row_tiles(16, 2304, 4096, 256) == 1 and sk.qkv_row_tiles(9, 3584, 4608, 128) == 0
     assert sk.qkv_row_tiles(9, 1536 + 32, 2048, 128) == 0
+
+
+@pytest.mark.parametrize("row_tiles", [1, 2])
+def test_without_rotation_the_table_is_not_needed(row_tiles):
+    """Positions far out and a table of one position of smaller heads: nothing of it is read. Sums are exact, as above."""
+    g = torch.Generator(device=DEV).manual_seed(row_tiles)
+    sixteenths = lambda n, *shape: torch.randint(-n, n + 1, shape, device=DEV, generator=g).float() / 16
+    M, Hq, Hkv, D, K = 19, 3, 2, 128, 256
+    x, w, b = sixteenths(5, M, K).bfloat16(), sixteenths(2, (Hq + 2 * Hkv) * D, K).bfloat16(), sixteenths(9, (Hq + 2 * Hkv) * D).bfloat16()
+    pos, slots = torch.full((M,), 1 << 30, device=DEV, dtype=torch.int32), torch.arange(M, device=DEV)
+    kc, vc = ops.alloc_kv_cache(1, Hkv, D, torch.bfloat16, DEV)
+    q = sk.qkv_rope(x, w, b, pos, slots, ops.RotaryTable(16, 1, 1e4, DEV), kc, vc, Hq, Hkv, D, row_tiles, do_rope=False)
+    y = (x.float() @ w.float().t() + b.float()).bfloat16().view(M, Hq + 2 * Hkv, D)
+    assert torch.equal(q, y[:, :Hq]) and torch.equal(kc[0, :, :M].transpose(0, 1), y[:, Hq:Hq + Hkv])
+    assert torch.equal(vc[0, :, :, :M].permute(2, 0, 1), y[:, Hq + Hkv:])
