@@ -249,7 +249,7 @@ def dgemm_wide(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     cols = (-(-N // (rounds * N_CU)) + 3) // 4 * 4
     out = torch.empty(M, N, dtype=x.dtype, device=x.device)
     L.check(L.lib().areal_dtile_rows(L.ptr(x), L.c_int64(x.stride(0)), L.ptr(w), L.ptr(out), L.c_int64(N), L.c_int(M), L.c_int(N),
-                                     L.c_int(K), L.c_int(cols), L.c_int(1), L.c_int(N_CU), L.c_int(1), L.stream_ptr()), "dgemm_wide")
+                                     L.c_int(K), L.c_int(cols), L.c_int(N_CU), L.stream_ptr()), "dgemm_wide")
     return out
 
 

@@ -306,11 +306,10 @@ __global__ __launch_bounds__(512) void dtile_kernel(const DTArgs a) {
 // Y [M, N] bf16 = X W^T for so many columns that every CU has several ranges (the LM head): as above, with a workgroup a CU that goes
 // from range to range. The loader waves ask for the next range's first stages while the last ones of the present are multiplied and its
 // outputs stored: with a workgroup a range the ring is empty at the start of each and drains at its end.
-// us, cold weights, decode_gemm.hip's tiles / library / this: 151936 columns, 1536 deep, 8 / 24 / 48 / 64 / 96 / 128 / 160 rows 76 / 81 / 92 / 97 /
-// 188 / 198 / -, 162 / 103 / 120 / 112 / 120 / 128 / 138, 73 / 79 / 89 / 94 / 103 / 111 / 119; 2048 deep 24 / 64 / 96 / 160 rows 108 / 124 / 238 /
-// -, 147 / 153 / 161 / 181, 103 / 118 / 128 / 150; 128256, 4096 deep 24 / 64 / 160 rows 163 / 181 / -, 195 / 210 / 249, 162 / 186 / 229; 32000,
-// 2048 deep 26 / 27 / -, 36 / 36 / 38, 25 / 27 / 38. Two row blocks: 224 rows of the first 152 (library) / 186, 320 rows 188 / 187. What
-// bounds it: the load path at 24 rows (6.0 TB/s of weights), with more rows the X that every range stages again.
+// us, cold weights, decode_gemm.hip's tiles / library / this: 151936 columns, 1536 deep, 96 / 128 / 160 rows 188 / 198 / -, 120 / 128 / 138, 103 /
+// 111 / 119; 2048 deep 96 / 160 rows 238 / -, 161 / 181, 128 / 150; 128256, 4096 deep, 160 rows - / 249 / 229; 32000, 2048 deep, 160 rows
+// - / 38 / 38. What bounds it: the X that every range stages again. All rows are one block: in two blocks (each range twice) 224 rows of the
+// first took 186 where the library takes 152, 320 rows 187 / 188. Up to 64 rows a step was as long on decode_gemm.hip's tiles.
 template <int RT, int CT>
 __global__ __launch_bounds__(512) void dtile_walk_kernel(const DTArgs a) {
   constexpr int BM = 32 * RT, WR = 32 * CT, IPW = RT + CT;
@@ -320,8 +319,8 @@ __global__ __launch_bounds__(512) void dtile_walk_kernel(const DTArgs a) {
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  // tile p: row block p % mblocks of range p / mblocks. In every round an XCD has neighbouring tiles: row blocks of a range share its L2
-  const int nwg = gridDim.x, all = a.ntiles * a.mblocks;
+  // in every round an XCD has neighbouring ranges
+  const int nwg = gridDim.x, all = a.ntiles;
   const int first = (blockIdx.x & 7) * (nwg >> 3) + (blockIdx.x >> 3);  // (the grid is a multiple of 8)
   const int nsteps = a.K >> 6, stages = a.stages;
   const int mine = first < all ? (all - first + nwg - 1) / nwg : 0, total = mine * nsteps;
@@ -334,21 +333,20 @@ __global__ __launch_bounds__(512) void dtile_walk_kernel(const DTArgs a) {
       if (step == nsteps) {
         tile += nwg;
         step = 0;
-        const int range = quotient(tile, a.mblocks, a.inv_m), m0 = (tile - range * a.mblocks) * BM;
-        const int c0 = range * a.w, c1 = min(a.N, c0 + a.w);
-        k = k_start(range, a.rot, nsteps);
+        const int c0 = tile * a.w, c1 = min(a.N, c0 + a.w);
+        k = k_start(tile, a.rot, nsteps);
 #pragma unroll
         for (int j = 0; j < IPW; ++j) {
           const int row = 8 * (lw + 4 * j) + (lane >> 3);
           const int c = (lane & 7) ^ ((row >> 1) & 7);
           src[j] = j < CT ? a.W + (size_t)min(c0 + row, c1 - 1) * a.K + 8 * c
-                          : a.X + (size_t)min(m0 + row - WR, a.M - 1) * a.xs + 8 * c;
+                          : a.X + (size_t)min(row - WR, a.M - 1) * a.xs + 8 * c;
         }
       }
       char* base = smem + buf * STAGE_BYTES + lw * 1024;
 #pragma unroll
       for (int j = 0; j < IPW; ++j) {
-        if (j < CT && a.nt)
+        if (j < CT)  // weights past the caches
           __builtin_amdgcn_global_load_lds((gptr_t)(src[j] + k * 64), (lptr_t)(base + j * 4096), 16, 0, 2);
         else
           __builtin_amdgcn_global_load_lds((gptr_t)(src[j] + k * 64), (lptr_t)(base + j * 4096), 16, 0, 0);
@@ -414,8 +412,7 @@ __global__ __launch_bounds__(512) void dtile_walk_kernel(const DTArgs a) {
       fa.read(sb + xb + co0, sb + wb + co0);
     }
     fb.multiply(acc);
-    const int range = quotient(tile, a.mblocks, a.inv_m), m0 = (tile - range * a.mblocks) * BM + wm * RT * 16 + r16;
-    const int n0 = range * a.w + wn * CT * 16 + 4 * q, c1 = min(a.N, range * a.w + a.w);
+    const int m0 = wm * RT * 16 + r16, n0 = tile * a.w + wn * CT * 16 + 4 * q, c1 = min(a.N, tile * a.w + a.w);
 #pragma unroll
     for (int r = 0; r < RT; ++r) {
       if (m0 + 16 * r >= a.M) continue;
@@ -438,7 +435,6 @@ int dt_walk(DTArgs a, int workgroups, hipStream_t st) {
     HIP_RET(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 / stage_bytes * stage_bytes));
     attr_set = true;
   }
-  a.inv_m = reciprocal((long)a.ntiles * a.mblocks, a.mblocks);
   hipLaunchKernelGGL(kern, dim3(workgroups), dim3(512), a.stages * stage_bytes, st, a);
   return (int)hipGetLastError();
 }
@@ -537,19 +533,18 @@ extern "C" int areal_dtile_slab(const void* X, long xs, const void* W, void* Y, 
 }
 
 // X [M, K] bf16 (row stride xs), W [N, K] bf16 contiguous, Y [M, N] bf16 (row stride ys): K % 64 == 0, N % 4 == 0, 4 <= w <= 160 columns
-// a range (a multiple of 4), row blocks of 32 rt rows, rt = ceil(M / mblocks / 32) of 3 to 5.
-extern "C" int areal_dtile_rows(const void* X, long xs, const void* W, void* Y, long ys, int M, int N, int K, int w, int mblocks,
-                                int workgroups, int nt, hipStream_t st) {
+// a range (a multiple of 4), 65 to 160 rows.
+extern "C" int areal_dtile_rows(const void* X, long xs, const void* W, void* Y, long ys, int M, int N, int K, int w, int workgroups,
+                                hipStream_t st) {
   if (M <= 0) return 0;
   if (K % 64 != 0 || K < 64 || xs % 8 != 0 || N % 4 != 0 || N < 4 || w % 4 != 0 || w < 4 || w > 160 || ys % 4 != 0) return -1;
-  if (mblocks < 1 || workgroups < 8 || workgroups % 8 != 0) return -2;
+  if (workgroups < 8 || workgroups % 8 != 0) return -2;
   if (((uintptr_t)X | (uintptr_t)W) % 16 != 0 || (uintptr_t)Y % 8 != 0) return -3;
   DTArgs a = {};
   a.X = (const bf16_t*)X; a.xs = xs; a.W = (const bf16_t*)W; a.Y = Y; a.ys = ys;
-  a.M = M; a.N = N; a.K = K; a.w = w; a.ntiles = (N + w - 1) / w; a.mblocks = mblocks; a.nt = nt; a.rot = k_rotation(K);
-  if ((long)a.ntiles * mblocks * (K / 64) >= (1l << 31)) return -4;
-  const int rt = ((M + mblocks - 1) / mblocks + 31) / 32;
-  switch (rt) {
+  a.M = M; a.N = N; a.K = K; a.w = w; a.ntiles = (N + w - 1) / w; a.rot = k_rotation(K);
+  if ((long)a.ntiles * (K / 64) >= (1l << 31)) return -4;
+  switch ((M + 31) / 32) {
     case 3: return dt_walk<3, 5>(a, workgroups, st);
     case 4: return dt_walk<4, 5>(a, workgroups, st);
     case 5: return dt_walk<5, 5>(a, workgroups, st);
