@@ -71,10 +71,10 @@ def test_upload():
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("layers,odd", [(1, None), (2, None), (3, None), (8, None), (9, None), (3, 0), (3, 1), (9, 2), (9, 8)])
-def test_layers_in_several_calls(layers, odd):
-    """Every number of layers around those of the first calls, and a layer whose weight is off the 16-byte grid in each of them: the
-    numbers of the single launches, which take over from the start."""
+@pytest.mark.parametrize("layers,odd", [(1, None), (2, None), (3, None), (8, None), (9, None), (13, None), (3, 0), (3, 1), (9, 2), (9, 8)])
+def test_layers_in_several_calls(layers, odd, monkeypatch):
+    """Every number of layers around those of the first calls, and a layer whose weight is off the 16-byte grid in each of them, for which
+    the single launches take over from the start: their bits, and near the numbers of the layers' other path."""
     torch.manual_seed(1)
     cfg = ModelConfig(family="qwen2", vocab_size=512, hidden_size=128, n_layers=layers, n_q_heads=2, n_kv_heads=1, head_dim=128,
                       intermediate_size=192, max_position_embeddings=512, qkv_bias=True)
@@ -87,21 +87,30 @@ def test_layers_in_several_calls(layers, odd):
                 cu_q=np.array([0, 5], np.int32), cu_k=np.array([0, 45], np.int32), max_q=5, has_prefix=True,
                 block_tables=np.arange(2, dtype=np.int32)[None], req_ids=np.arange(1), temperature=np.zeros(1, np.float32),
                 top_p=np.ones(1, np.float32), top_k=np.full(1, 1 << 30), sample=np.ones(1, np.int32), logit_rows=np.arange(5))
-    out = []
-    for single in (False, True):
-        if odd is not None:
-            w = m.layers[odd].mlp.down if odd % 2 else m.layers[odd].ln2
-            moved = torch.empty(w.numel() + 4, dtype=w.dtype, device="cuda")[4:].view_as(w)  # 8 bytes past the grid
-            w.data = moved.copy_(w)
+    native, calls, out = ops.prefill_layers.run, [], []
+
+    def counted(*a):
+        r = native(*a)
+        calls.append(r is not None)
+        return r
+
+    if odd is not None:
+        w = m.layers[odd].mlp.down if odd % 2 else m.layers[odd].ln2
+        moved = torch.empty(w.numel() + 4, dtype=w.dtype, device="cuda")[4:].view_as(w)  # 8 bytes past the grid
+        w.data = moved.copy_(w)
+    for run, fused in ((counted, True), (lambda *a: None, True), (None, False)):
+        monkeypatch.setattr(ops.prefill_layers, "run", run)
         r = ModelRunner(m, num_pages=2, max_context=64, max_batch=1)
-        if single:
+        if not fused:
             r._prefill_fused = lambda rows: False
         for pair in r.kv:
             for t in pair:
                 t.copy_(torch.linspace(-1, 1, t.numel(), device="cuda").view_as(t))
         r.prefill(plan)
         out.append((r.kept_logits.clone(), [t.clone() for kv in r.kv for t in kv]))
-    (la, ca), (lb, cb) = out
+    assert calls == [odd is None]
+    (la, ca), (ls, cs), (lb, cb) = out
+    assert torch.equal(la, ls) and all(torch.equal(a, b) for a, b in zip(ca, cs))
     # 16-bit roundings of the layers' products (library against split sums) add up over the layers: some steps of 2^-8
     assert float((la - lb).norm() / lb.norm()) < 2.0 ** -8 * (2 + layers)
     for a, b in zip(ca, cb):
