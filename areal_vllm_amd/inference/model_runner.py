@@ -725,14 +725,15 @@ class ModelRunner:
             x, residual = finish(slab, residual, nw)
         return x
 
-    # Rows up to which the five-launch layer is faster than split-K GEMMs with row kernels: hidden sizes up to 1536, of those the ones whose
-    # MLP is wider than 4096 (gate and up then go over the chip in one uneven round of wide workgroups), and above 1536. 28 layers of
-    # Qwen2-1.5B (1536, 8960 inner) at 2 / 3 / 4 / 5 / 6 / 8 rows: 1.17 / 1.26 / 1.27 / 1.34 / 1.38 / 1.43 ms a step against 1.24 / 1.26 / 1.29 /
-    # 1.30 / 1.31 / 1.35; 24 layers of 1536 at 6 rows, 1024 / 2048 / 4096 / 6144 inner: 0.86 / 0.89 / 0.98 / 1.06 against 0.93 / 0.98 / 1.02 / 1.04; of
-    # 896 at 4 / 5 / 6 rows, 1024 inner 0.66 / 0.68 / 0.71 against 0.77 / 0.76 / 0.78, 4864 0.79 / 0.81 / 0.83 against 0.82 / 0.82 / 0.82.
-    # 12 layers of Llama-3-8B at 1 / 2 / 4: 1.47 / 1.55 / 1.65 against 1.66 / 1.66 / 1.58 (a row's weights no longer fit the registers at once).
-    # 2048 (10 layers) at 1 / 2 / 3 / 6: 0.58 / 0.61 / 0.67 / 0.71 against 0.67 / 0.68 / 0.68 / 0.69; 1 / 2 rows of 3072 0.52 / 0.55 against 0.62 /
-    # 0.63, 3584 0.70 / 0.74 against 0.74 / 0.73, 5120 (13824 inner) 0.70 / 0.74 against 0.76 / 0.73, 8192 0.75 / 0.77 against 0.89 / 0.87.
+    # Rows up to which the five-launch layer is faster than split-K GEMMs with row kernels, or level with them: hidden sizes up to 1536, of
+    # those the ones whose MLP is wider than 4096 (gate and up then go over the chip in one uneven round of wide workgroups), and above 1536.
+    # ms a step, 640-token contexts, five launches / split-K: 28 layers of Qwen2-1.5B (1536, 8960 inner), 1 / 2 / 3 / 4 / 5 / 6 rows 1.07 / 1.19 / 1.26 /
+    # 1.27 / 1.36 / 1.38 and 1.24 / 1.26 / 1.27 / 1.28 / 1.27 / 1.29; 24 layers of 1536 at 6 rows, 1024 / 2048 / 4096 / 6144 inner, 0.80 / 0.83 / 0.91 /
+    # 0.99 and 0.87 / 0.89 / 0.94 / 0.97; of 896 at 4 / 5 / 6 rows, 1024 inner 0.61 / 0.63 / 0.63 and 0.72 / 0.74 / 0.73, 4864 0.75 / 0.77 / 0.78 and 0.79 /
+    # 0.80 / 0.80. Above (a row's weights no longer fit the registers at once) a third row is level at best: 10 layers of 2048 at 2 / 3 / 4 rows, 4096
+    # inner 0.43 / 0.46 / 0.47 and 0.46 / 0.47 / 0.47, 8192 0.51 / 0.55 / 0.56 and 0.52 / 0.52 / 0.53; 8 of 3072, 8192 inner, 1 / 2 / 3 rows 0.51 / 0.58 / 0.62 and
+    # 0.58 / 0.60 / 0.61. A second one is not everywhere ahead, nor the first: 1 / 2 rows of 4096 (12 layers, 14336 inner) 1.24 / 1.34 and 1.28 / 1.29,
+    # 3584 (8, 18944) 0.88 / 0.95 and 0.92 / 0.93, 5120 (6, 13824) 0.84 / 0.88 and 0.81 / 0.82, 8192 (4, 28672) 1.32 / 1.35 and 1.39 / 1.39.
     SKINNY_MAX_ROWS, SKINNY_MAX_ROWS_LONG, SKINNY_MAX_ROWS_WIDE = 6, 4, 2
 
     def _skinny(self, rows: int) -> bool:

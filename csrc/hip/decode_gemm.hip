@@ -649,7 +649,8 @@ __global__ __launch_bounds__(THREADS) void splitk_residual_rmsnorm_kernel(
 // slabs come from other XCDs) and the block's reduction; with the slabs counted at run time it was a round trip for every four of them,
 // the residual behind them, and 80 instructions ahead of the first. Everything a row needs is asked for at once; one barrier. Captured,
 // 1536 columns, us before / now: 24 rows of 5 / 16 slabs 3.29 / 2.71, 4.31 / 3.62; 93 rows of 3 / 10 3.70 / 2.81, 4.50 / 3.60; 320 rows of 2 /
-// 8 3.88 / 3.38, 6.45 / 6.10. Up to 24 slabs (a plan's most) and one chunk a thread; other rows take the kernel above.
+// 8 3.88 / 3.38, 6.45 / 6.10; between the other kernels of a step 24 rows 4.7 -> 4.3 and 4.5, 93 rows
+// 4.3 -> 3.1 and 4.0. Up to 24 slabs (a plan's most) and one chunk a thread; other rows take the kernel above.
 template <int THREADS, int S>
 __global__ __launch_bounds__(THREADS) void splitk_residual_rmsnorm_row_kernel(
     const float* __restrict__ slab, const bf16_t* __restrict__ res, const bf16_t* __restrict__ w, bf16_t* __restrict__ res_out,

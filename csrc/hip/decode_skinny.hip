@@ -17,7 +17,8 @@
 //     pair of weights and row keeps up with memory, and a wave reads 1 KiB of ONE weight row per load instruction; as
 //     matrix operands (16 rows x 64 bytes a load) the same bytes take 10.8 instead of 9.2 us to load;
 //   * three to eight rows: matrix cores (with three rows the dot products take as long as the loads, with eight twice as
-//     long: 2.3 ms a step); from nine rows on the split-K path is as fast;
+//     long: 2.3 ms a step), but the long rows of a narrow down projection (areal_skinny_residual); from nine rows on the split-K path is
+//     as fast;
 //   * 8 waves: WK along K, 8 / WK along the rows, WK so that a wave's share of K is at most 3 x 64 pieces of 16 bytes
 //     (K = 1536: WK = 1, K = 8960: WK = 8); the wave's share of the activations stays in registers for all its rows;
 //   * two sets of RB weight rows in registers: all loads of gate|up, o and down of Qwen2-1.5B are in flight at once;
@@ -27,9 +28,9 @@
 // Rounding points are those of the split-K path (csrc/hip/decode_gemm.hip): normalised rows, projection and residual
 // sum in bf16, sums in fp32.
 //
-// Measured (Qwen2-1.5B, 640-token contexts, captured decode step of 28 layers), split-K path -> this: 1 row 1.44 -> 1.17 ms,
-// 2 rows 1.44 -> 1.24, 4 rows 1.47 -> 1.36, 6 rows 1.58 -> 1.45, 8 rows level (one row is 1.08 ms by now). One row: gate|up 11.8 us,
-// down 7.3, o 3.2, qkv 4.4 (8.0 + 4.4, 4.6 + 4.4, 12.5, 4.6 + 4.4 on the split-K path).
+// Measured (Qwen2-1.5B, 640-token contexts, captured decode step of 28 layers), split-K path / this: 1 row 1.24 / 1.07 ms, 2 rows 1.26 /
+// 1.19, 3 rows 1.27 / 1.26, 4 rows 1.28 / 1.27, 6 rows 1.29 / 1.38 (which rows take it: ModelRunner). One row: gate|up 11.8 us, down 7.3, o 3.2,
+// qkv 4.4.
 #include "common.hpp"
 
 namespace {

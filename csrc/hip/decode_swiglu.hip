@@ -21,8 +21,9 @@
 //   * waves 4..7 do nothing but issue the LDS-DMA pieces (global_load_lds_dwordx4, 8 rows x 128 B each) of a ring of stages, one raw
 //     s_barrier per 64-deep step, counted vmcnt so that the later stages stay in flight across it; the XOR swizzle that makes the
 //     ds_read_b128 fragment reads conflict-free sits on the per-lane SOURCE address;
-//   * a workgroup's place by reciprocals of the host and 32-bit row products, ahead of the first load: 0.1 us a launch (24 rows, 1536 deep
-//     to 1536 columns 3.81 -> 3.68, 8960 deep 7.30 -> 7.19; gate|up of 320 rows 26.1 -> 25.7).
+//   * a workgroup's place by reciprocals of the host and 32-bit row products, ahead of the first load: launches of one kernel behind another
+//     0.1 us each (24 rows, 1536 deep to 1536 columns 3.81 -> 3.68, 8960 deep 7.30 -> 7.19; gate|up of 320 rows 26.1 -> 25.7). Between the
+//     other kernels of a step 0.2 to 0.6 at 320 rows (down 17.7 -> 17.4, gate|up 25.2 -> 24.6) and nothing at 24 (4.71 / 4.73, 7.34 / 7.60).
 //   * product transposed (A = weight rows, B = activation rows). A gated block's weight tiles hold two gate rows and the two matching
 //     up rows of every four, so that a lane has both factors of an output, and a pair of tiles gives it four columns in a row: an
 //     8-byte store. A wave's last tile of an odd number gives two columns.
