@@ -96,3 +96,38 @@ def test_router_logits(T, E, H, strided):
     # fp32 sums of up to 4099 products of values of order one, rounded to 16 bits once
     for got, want in ((dw, dy.double().t() @ x.detach().double()), (dx, dy.double() @ w.detach().double())):
         assert float(((got.double() - want).abs() - 2.0 ** -8 * want.abs()).max()) < 2.0 ** -20 * T ** 0.5 * 8
+
+
+@pytest.mark.parametrize("M", [1, 31, 32, 33, 256, 257, 1024, 1025, 1536, 40000])
+@pytest.mark.parametrize("N", [8, 12, 64, 72, 2048])
+@pytest.mark.parametrize("strided", [False, True])
+def test_bias_values(M, N, strided):
+    g = torch.Generator(device=DEV).manual_seed(M + N)
+    x = torch.randn(M, 64, device=DEV, generator=g).bfloat16().requires_grad_(True)
+    w, b = _parameter(torch.randn(N, 64, device=DEV, generator=g)), _parameter(torch.randn(N, device=DEV, generator=g))
+    dy = torch.randn(M, N + (8 if strided else 0), device=DEV, generator=g).bfloat16()[:, :N]
+    ops.linear(x, w, b).backward(dy)
+    assert w.told == 1 and b.told == 0 and not b.main_grad.any()
+    want = dy.double().sum(0)
+    # fp32 sums of M values of order one, rounded to 16 bits once
+    assert float(((b.grad.double() - want).abs() - 2.0 ** -8 * want.abs()).max()) < 2.0 ** -20 * M ** 0.5 * 8
+
+
+@pytest.mark.parametrize("T,H", [(1, 8), (5, 1536), (700, 1536), (4097, 256), (3000, 8192)])
+@pytest.mark.parametrize("residual,gemma", [(False, False), (True, True)])
+def test_norm_weight_values(T, H, residual, gemma):
+    g = torch.Generator(device=DEV).manual_seed(T + H)
+    x = torch.randn(T, H, device=DEV, generator=g).bfloat16().requires_grad_(True)
+    r = torch.randn(T, H, device=DEV, generator=g).bfloat16().requires_grad_(True) if residual else None
+    w = _parameter(torch.rand(H, device=DEV, generator=g) + 0.5)
+    plain = torch.nn.Parameter(w.detach().clone())
+    dy = torch.randn(T, H, device=DEV, generator=g).bfloat16()
+    dx = []
+    for p in (w, plain):
+        x.grad = None
+        ops.rmsnorm(x, p, 1e-6, r, gemma)[0].backward(dy)
+        dx.append(x.grad.clone())
+    assert torch.equal(*dx) and torch.equal(w.grad, plain.grad) and w.told == 0 and not w.main_grad.any()
+    s = x.detach().double() if r is None else (x.detach().float() + r.detach().float()).bfloat16().double()
+    want = (dy.double() * s * torch.rsqrt(s.pow(2).mean(-1, keepdim=True) + 1e-6)).sum(0)
+    assert float(((w.grad.double() - want).abs() - 2.0 ** -8 * want.abs()).max()) < 2.0 ** -20 * (4.0 + T ** 0.5 * 8)
